@@ -228,6 +228,28 @@ int sq_stream_build_books(const int32_t* tags_host, int32_t R, int32_t W, int32_
 int sq_codebook_balance_books(const int32_t* tags_host, int32_t R, int32_t W, int32_t C, int32_t d, int32_t bits, int32_t G,
                               const uint8_t* row_book_host, uint16_t* remap_out);
 
+/* The load-time layouts built on the GPU, from tags that are already there: the same bytes as the host routines above
+ * (which stay for tags in host memory), in milliseconds instead of a fraction of a second per matrix.  tags, row_book,
+ * counts, out, scratch and remap are DEVICE pointers, row_mask_host and remap_out_host HOST pointers; the plan and balance calls
+ * and sq_stream_fill_device synchronise the stream (they are for load time and never run under graph capture).
+ *   sq_stream_plan_device   makes the plan of the buffer sq_stream_build_books would write (its layout, and for the d = 4
+ *                           formats the tile-major copy): *plan_out, the bytes of the buffer and of the scratch the fill
+ *                           needs, and runs_out / groups_out as there.  counts: sq_stream_counts_bytes bytes (0 for d = 4).
+ *   sq_stream_fill_device   writes the buffer (16-byte aligned, of that size) from the same tags.
+ *   sq_stream_plan_free     ends the plan.
+ *   sq_codebook_balance_device  sq_codebook_balance_books; counts: (G << bits) * 4 bytes.
+ *   sq_codebook_relabel_device  rewrites the tags through remap (G << bits entries) in place. */
+size_t sq_stream_counts_bytes(int32_t R, int32_t C, int32_t d, int32_t bits, int32_t G);
+int sq_stream_plan_device(const int32_t* tags, int32_t R, int32_t W, int32_t C, int32_t d, int32_t bits, int32_t G, const uint8_t* row_book,
+                          const uint8_t* row_mask_host, int32_t runs, void* counts, void** plan_out, size_t* bytes_out, size_t* scratch_out,
+                          int32_t* runs_out, int32_t* groups_out, void* stream);
+int sq_stream_fill_device(const void* plan, const int32_t* tags, const uint8_t* row_book, void* out, void* scratch, void* stream);
+void sq_stream_plan_free(void* plan);
+int sq_codebook_balance_device(const int32_t* tags, int32_t R, int32_t W, int32_t C, int32_t d, int32_t bits, int32_t G, const uint8_t* row_book,
+                               uint32_t* counts, uint16_t* remap_out_host, void* stream);
+int sq_codebook_relabel_device(int32_t* tags, int32_t R, int32_t W, int32_t C, int32_t d, int32_t bits, int32_t G, const uint8_t* row_book,
+                               const uint16_t* remap, void* stream);
+
 /* ---- The packed file's block-32 side formats (reference shapequant/packed.py:30-40): the 8-bit output head
  * `aux.lm_head` (q int8 [V, C], scale fp16 [V, C/32], w = q * scale of the row's 32-column block) and the 4-bit
  * embedding `aux.embed` (q uint8 [V, C/2] with column 2k in the low and 2k+1 in the high nibble of byte k, each

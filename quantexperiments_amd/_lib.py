@@ -95,6 +95,19 @@ def lib() -> ctypes.CDLL:
         L.sq_stream_build_books.restype = ctypes.c_int
         L.sq_codebook_balance_books.argtypes = [vp, i32, i32, i32, i32, i32, i32, vp, vp]
         L.sq_codebook_balance_books.restype = ctypes.c_int
+        pp, zp = ctypes.POINTER(ctypes.c_void_p), ctypes.POINTER(ctypes.c_size_t)
+        L.sq_stream_counts_bytes.argtypes = [i32, i32, i32, i32, i32]
+        L.sq_stream_counts_bytes.restype = sz
+        L.sq_stream_plan_device.argtypes = [vp, i32, i32, i32, i32, i32, i32, vp, vp, i32, vp, pp, zp, zp, ip, ip, vp]
+        L.sq_stream_plan_device.restype = ctypes.c_int
+        L.sq_stream_fill_device.argtypes = [vp, vp, vp, vp, vp, vp]
+        L.sq_stream_fill_device.restype = ctypes.c_int
+        L.sq_stream_plan_free.argtypes = [vp]
+        L.sq_stream_plan_free.restype = None
+        L.sq_codebook_balance_device.argtypes = [vp, i32, i32, i32, i32, i32, i32, vp, vp, vp, vp]
+        L.sq_codebook_balance_device.restype = ctypes.c_int
+        L.sq_codebook_relabel_device.argtypes = [vp, i32, i32, i32, i32, i32, i32, vp, vp, vp]
+        L.sq_codebook_relabel_device.restype = ctypes.c_int
         L.sq_q8_linear.argtypes = [vp, vp, i32, i32, vp, ctypes.c_int, i64, vp, ctypes.c_int, i64, i32, vp, sz, vp]
         L.sq_q8_workspace_bytes.argtypes = [i32, i32, i32]
         L.sq_q8_workspace_bytes.restype = sz
@@ -118,7 +131,8 @@ EXPORTS = ("sq_version", "sq_last_error", "sq_dequant", "sq_linear_small", "sq_l
            "sq_q8_dequant", "sq_q4_embed", "sq_addnorm", "sq_silu_mul",
            "sq_linear_small_from", "sq_linear_small_silu", "sq_gemm_dense_ws", "sq_gemm_dense_workspace_bytes", "sq_linear_small_noalloc",
            "sq_workspace_status", "sq_workspace_reset", "sq_noalloc_reset", "sq_stream_spin_limit", "sq_codebook_balance",
-           "sq_stream_bytes_books", "sq_stream_build_books", "sq_codebook_balance_books")
+           "sq_stream_bytes_books", "sq_stream_build_books", "sq_codebook_balance_books", "sq_stream_counts_bytes", "sq_stream_plan_device",
+           "sq_stream_fill_device", "sq_stream_plan_free", "sq_codebook_balance_device", "sq_codebook_relabel_device")
 
 
 def check(rc: int) -> None:

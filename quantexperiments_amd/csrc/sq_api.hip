@@ -402,6 +402,57 @@ int sq_codebook_balance_books(const int32_t* tags_host, int32_t R, int32_t W, in
     return SQ_OK;
 }
 
+// ---- the same from tags that are already in device memory
+static int device_build_check(const char* who, const void* tags, int32_t R, int32_t W, int32_t C, int32_t d, int32_t bits, int32_t G,
+                              const void* row_book) {
+    if (!tags) return fail(SQ_EINVAL, "%s: null pointer", who);
+    if (G < 1 || G > 256 || (G & (G - 1)) != 0) return fail(SQ_EUNSUPPORTED, "%s: %d codebooks (a power of two is needed)", who, G);
+    if (G > 1 && !row_book) return fail(SQ_EINVAL, "%s: G %d needs row_book", who, G);
+    if (d <= 0 || !stream_format_ok(R, C, d, bits, G)) return fail(SQ_EUNSUPPORTED, "%s: d %d bits %d G %d R %d not covered", who, d, bits, G, R);
+    if ((int64_t)W * 32 < (int64_t)(C / d) * bits) return fail(SQ_EINVAL, "%s: W %d too small", who, W);
+    return SQ_OK;
+}
+
+size_t sq_stream_counts_bytes(int32_t R, int32_t C, int32_t d, int32_t bits, int32_t G) {
+    return d > 0 && stream_format_ok(R, C, d, bits, G) ? stream_counts_bytes(R, C, d, bits, G) : 0;
+}
+
+int sq_stream_plan_device(const int32_t* tags, int32_t R, int32_t W, int32_t C, int32_t d, int32_t bits, int32_t G, const uint8_t* row_book,
+                          const uint8_t* row_mask_host, int32_t runs, void* counts, void** plan_out, size_t* bytes_out, size_t* scratch_out,
+                          int32_t* runs_out, int32_t* groups_out, void* stream) {
+    const char* who = "sq_stream_plan_device";
+    if (!plan_out || !bytes_out || !scratch_out || !runs_out || !groups_out) return fail(SQ_EINVAL, "%s: null pointer", who);
+    *plan_out = nullptr;
+    if (!(tags && d > 0 && !stream_format_ok(R, C, d, bits, G) && !row_mask_host && tiled_format_ok(R, W, C, d, bits))) {
+        if (int rc = device_build_check(who, tags, R, W, C, d, bits, G, row_book)) return rc;
+        if (!counts) return fail(SQ_EINVAL, "%s: null counts", who);
+    }
+    return stream_plan_device((const uint32_t*)tags, R, W, C, d, bits, G, G > 1 ? row_book : nullptr, row_mask_host, runs, counts,
+                              (StreamDevicePlan**)plan_out, bytes_out, scratch_out, runs_out, groups_out, (hipStream_t)stream);
+}
+
+int sq_stream_fill_device(const void* plan, const int32_t* tags, const uint8_t* row_book, void* out, void* scratch, void* stream) {
+    if (!plan || !tags || !out) return fail(SQ_EINVAL, "sq_stream_fill_device: null pointer");
+    if (((uintptr_t)out & 15) || ((uintptr_t)scratch & 15)) return fail(SQ_EINVAL, "sq_stream_fill_device: out and scratch must be 16-byte aligned");
+    return stream_fill_device(*(const StreamDevicePlan*)plan, (const uint32_t*)tags, row_book, (unsigned char*)out, (unsigned char*)scratch, (hipStream_t)stream);
+}
+
+void sq_stream_plan_free(void* plan) { stream_plan_free((StreamDevicePlan*)plan); }
+
+int sq_codebook_balance_device(const int32_t* tags, int32_t R, int32_t W, int32_t C, int32_t d, int32_t bits, int32_t G, const uint8_t* row_book,
+                               uint32_t* counts, uint16_t* remap_out_host, void* stream) {
+    if (int rc = device_build_check("sq_codebook_balance_device", tags, R, W, C, d, bits, G, row_book)) return rc;
+    if (!counts || !remap_out_host) return fail(SQ_EINVAL, "sq_codebook_balance_device: null pointer");
+    return stream_balance_device((const uint32_t*)tags, R, W, C, d, bits, counts, remap_out_host, G, G > 1 ? row_book : nullptr, (hipStream_t)stream);
+}
+
+int sq_codebook_relabel_device(int32_t* tags, int32_t R, int32_t W, int32_t C, int32_t d, int32_t bits, int32_t G, const uint8_t* row_book,
+                               const uint16_t* remap, void* stream) {
+    if (int rc = device_build_check("sq_codebook_relabel_device", tags, R, W, C, d, bits, G, row_book)) return rc;
+    if (!remap) return fail(SQ_EINVAL, "sq_codebook_relabel_device: null pointer");
+    return stream_relabel_device((uint32_t*)tags, R, W, C, d, bits, G > 1 ? row_book : nullptr, remap, (hipStream_t)stream);
+}
+
 size_t sq_stream_bytes(const int32_t* tags_host, int32_t R, int32_t W, int32_t C, int32_t d, int32_t bits,
                        const uint8_t* row_mask_host, int32_t runs) {
     return sq_stream_bytes_balanced(tags_host, R, W, C, d, bits, row_mask_host, runs, nullptr);

@@ -84,6 +84,18 @@ int stream_build_host(const uint32_t* tags, int R, int W, int C, int d, int bits
 // applies, by itself; every codebook is balanced over its own slices (one of at most 4096 codewords keeps its labels)
 void stream_balance_host(const uint32_t* tags, int R, int W, int C, int d, int bits, uint16_t* remap_out, int G = 1,
                          const uint8_t* row_book = nullptr);
+// The same from tags in device memory (sq_stream_plan_device and the calls beside it in sqhip.h): counts is a device scratch
+// of stream_counts_bytes, row_mask is on the host; the tile-major copies of the d = 4 formats go through the same calls.
+struct StreamDevicePlan;
+size_t stream_counts_bytes(int R, int C, int d, int bits, int G);
+int stream_plan_device(const uint32_t* tags, int R, int W, int C, int d, int bits, int G, const uint8_t* row_book, const uint8_t* row_mask_host,
+                       int runs, void* counts, StreamDevicePlan** out, size_t* bytes, size_t* scratch, int* runs_out, int* groups_out, hipStream_t s);
+int stream_fill_device(const StreamDevicePlan& D, const uint32_t* tags, const uint8_t* row_book, unsigned char* out, unsigned char* scratch,
+                       hipStream_t s);
+void stream_plan_free(StreamDevicePlan* D);
+int stream_balance_device(const uint32_t* tags, int R, int W, int C, int d, int bits, uint32_t* counts, uint16_t* remap_out, int G,
+                          const uint8_t* row_book, hipStream_t s);
+int stream_relabel_device(uint32_t* tags, int R, int W, int C, int d, int bits, const uint8_t* row_book, const uint16_t* remap, hipStream_t s);
 // sq_matrix.stream_runs is sq_stream_build's runs_out: the run count in the low 16 bits, the groups of the longest run
 // in the next 8, the most column orders in one run (less one) in bits 24-26, the steps per unit of the first-steps region
 // (less one) in bits 27-28, bit 30 = the stream carries a relabelled codebook

@@ -42,595 +42,8 @@
 #include <vector>
 #include "sq_stream.h"
 
-constexpr int STREAM_CLIMB = 1;      // hill-climbing passes of the entry ordering (load time against LDS collisions)
 
 namespace sq {
-
-// A run: groups g0 .. g0 + ng - 1 of every bucket.  Its rows belong to `norders` column orders (one without row orders);
-// the groups of order[i] begin at group bound[i] of the run (bound[0] = 0), and the kernel keeps copy i of x, gathered
-// through that order, in LDS for them.
-// u0: the index of the run's first unit (units are counted run after run).
-struct StreamRun { int32_t g0, ng, norders, u0; uint8_t bound[STREAM_RUN_ORDERS]; uint8_t order[STREAM_RUN_ORDERS]; };
-static_assert(sizeof(StreamRun) == 32, "run records are read as 8 dwords");
-
-StreamGeom stream_geom(int C, int d, int bits, int groups, int runs, bool balanced, int fs) {
-    StreamGeom g;
-    g.U = C / d;
-    g.NS = 1 << (bits - STREAM_SLICE_BITS);
-    g.KP = (g.U + STREAM_PART_MAX - 1) / STREAM_PART_MAX;
-    g.PC = (g.U + g.KP - 1) / g.KP;
-    g.NV = g.NS * g.KP;
-    g.NG = groups;
-    g.runs = runs;
-    g.fmt = stream_fmt(g.PC);
-    g.fs = fs < 1 ? g.fmt.pf : fs < g.fmt.pf ? fs : g.fmt.pf;
-    g.off_slots = ((size_t)g.NV * g.NG * 16 + 255) & ~(size_t)255;          // four words per (bucket, group)
-    g.off_runs = (g.off_slots + (size_t)g.NV * g.NG * 64 * 2 + 255) & ~(size_t)255;
-    g.off_rows = (g.off_runs + (size_t)runs * sizeof(StreamRun) + 255) & ~(size_t)255;
-    size_t end = (g.off_rows + (size_t)g.NG * 64 * 4 + 255) & ~(size_t)255;
-    g.off_table = g.off_unmap = 0;
-    if (balanced) {
-        g.off_table = end;
-        g.off_unmap = end + ((size_t)d * 2 << bits);
-        end = (g.off_unmap + ((size_t)2 << bits) + 255) & ~(size_t)255;
-    }
-    g.off_steps = end;
-    g.total_steps = 0;
-    return g;
-}
-
-// (R + 64 * 256 bounds the places: every column order can leave one group short)
-bool stream_format_ok(int R, int C, int d, int bits, int G) {
-    if (G < 1 || (G & (G - 1)) != 0 || bits < 1 || bits > 16) return false;
-    const int lb = stream_label_bits(bits, G);
-    return d == 8 && lb > STREAM_SLICE_BITS && (1 << (lb - STREAM_SLICE_BITS)) <= (G > 1 ? STREAM_SLICES_MAX : 16) && C % d == 0 &&
-           R > 0 && R + 64 * 256 < (int)STREAM_NO_ROW;
-}
-
-static inline uint32_t host_tag(const uint32_t* row, int W, int bits, int j) {
-    const int64_t p = (int64_t)j * bits;
-    const int w = (int)(p >> 5), s = (int)(p & 31);
-    uint64_t v = row[w];
-    if (s + bits > 32 && w + 1 < W) v |= (uint64_t)row[w + 1] << 32;
-    return (uint32_t)(v >> s) & ((1u << bits) - 1u);
-}
-
-static void parallel_rows(int R, const std::function<void(int, int)>& fn) {
-    unsigned nt = std::thread::hardware_concurrency();
-    if (nt < 1) nt = 1;
-    if (nt > 16) nt = 16;
-    if ((unsigned)R < nt * 64) nt = 1;
-    if (nt == 1) { fn(0, R); return; }
-    std::vector<std::thread> th;
-    const int per = (R + (int)nt - 1) / (int)nt;
-    for (unsigned t = 0; t < nt; ++t) {
-        const int a = (int)t * per, b = std::min(R, a + per);
-        if (a < b) th.emplace_back(fn, a, b);
-    }
-    for (auto& t : th) t.join();
-}
-
-
-struct StreamPlan {
-    StreamGeom g;
-    int GR;                          // groups in the longest run
-    int orders_max;                  // most column orders in one run
-    std::vector<StreamRun> runs;
-    std::vector<uint32_t> base;      // [NG * 64]: rows ordered by column order, STREAM_NO_ROW where a group is short
-    std::vector<uint16_t> cnt;       // [NV][R]
-    std::vector<uint32_t> pos;       // [NV][R]: lane position (group * 64 + lane) of row r in bucket v
-    std::vector<uint32_t> goff;      // [NV * NG + 1]: the groups' steps counted bucket after bucket, group after group (how the
-                                     // builder lays them out before they move to their places)
-    uint64_t logical_steps;          // goff[NV * NG]
-    int NU;                          // units of one bucket
-    std::vector<uint32_t> slot32;    // [NV * NG * 64]: place | count << STREAM_ROW_BITS per lane (STREAM_NO_ROW: no row), the
-                                     // builder's own form of the slots
-    std::vector<uint32_t> run_of;    // [NG]: the run of a group
-    std::vector<uint32_t> head4;     // [NV * NG][4]: {rest, nst, unit0, split}, what the buffer holds per (bucket, group)
-    std::vector<uint16_t> remap;     // balanced streams: file id -> new id (empty: identity)
-};
-
-// Relabelling of the codewords for a stream with a codebook of its own: the codewords are dealt, most used first, to
-// whichever slice of 4096 carries the fewest tags so far and still has room, so every slice ends up with the same
-// share of the tags (a slice is one workgroup's work) whatever the distribution of the tags is, and a slice's popular
-// codewords get consecutive places, i.e. different LDS bank groups.
-// With several codebooks (row_book names a row's) every codebook is relabelled by itself, over its own slices:
-// remap[book << bits | label] is the new label within the book; a codebook of at most one slice keeps its labels.
-static void balance_codewords(const uint32_t* tags, int R, int W, int U, int bits, std::vector<uint16_t>& remap, int G = 1,
-                              const uint8_t* row_book = nullptr) {
-    const int K = 1 << bits, NS = K >> STREAM_SLICE_BITS, SL = 1 << STREAM_SLICE_BITS;
-    remap.assign((size_t)G * K, 0);
-    if (NS < 2) {
-        for (size_t k = 0; k < remap.size(); ++k) remap[k] = (uint16_t)(k & (size_t)(K - 1));
-        return;
-    }
-    std::vector<uint64_t> count((size_t)G * K, 0);
-    for (int r = 0; r < R; ++r) {
-        const uint32_t* row = tags + (size_t)r * W;
-        uint64_t* cb = count.data() + (size_t)(row_book ? row_book[r] & (G - 1) : 0) * K;
-        for (int j = 0; j < U; ++j) ++cb[host_tag(row, W, bits, j)];
-    }
-    std::vector<uint32_t> ids(K);
-    std::vector<uint64_t> load(NS);
-    std::vector<int> fill(NS);
-    for (int b = 0; b < G; ++b) {
-        const uint64_t* cb = count.data() + (size_t)b * K;
-        for (int k = 0; k < K; ++k) ids[k] = (uint32_t)k;
-        std::stable_sort(ids.begin(), ids.end(), [cb](uint32_t x, uint32_t y) { return cb[x] > cb[y]; });
-        std::fill(load.begin(), load.end(), 0);
-        std::fill(fill.begin(), fill.end(), 0);
-        for (int k = 0; k < K; ++k) {
-            int best = -1;
-            for (int sl = 0; sl < NS; ++sl)
-                if (fill[sl] < SL && (best < 0 || load[sl] < load[best])) best = sl;
-            remap[(size_t)b * K + ids[k]] = (uint16_t)(best * SL + fill[best]);
-            ++fill[best];
-            load[best] += cb[ids[k]];
-        }
-    }
-}
-
-// (G > 1: the labels a row's tags become are book << bits | tag, see sq_stream.h; `balanced` is for one codebook only)
-static void plan_stream(const uint32_t* tags, int R, int W, int C, int d, int bits, const uint8_t* row_mask, int runs,
-                        StreamPlan& P, bool balanced, int G, const uint8_t* row_book) {
-    const int lbits = stream_label_bits(bits, G);
-    P.remap.clear();
-    if (balanced) balance_codewords(tags, R, W, C / d, bits, P.remap);
-    const uint16_t* remap = balanced ? P.remap.data() : nullptr;
-    // rows by column order, groups and runs
-    std::vector<uint32_t> order(R);
-    for (int r = 0; r < R; ++r) order[r] = (uint32_t)r;
-    if (row_mask)
-        std::stable_sort(order.begin(), order.end(), [row_mask](uint32_t a, uint32_t b) { return row_mask[a] < row_mask[b]; });
-    StreamGeom g0 = stream_geom(C, d, lbits, 0, 0);
-    if (runs <= 0) runs = (STREAM_DEFAULT_WGS + g0.NV / 2) / g0.NV;
-    if (runs < 1) runs = 1;
-    // Groups per column order.  A run takes the groups of one order, GR at a time, or, when orders are small, the whole
-    // groups of up to `cap` orders that follow each other (a masked k projection has 64 rows per order: one run per order
-    // would be 16 workgroups of one group each per bucket).  cap: as many gathered copies of x as fit LDS beside the slice
-    // and the run's partial sums, and as the staging loop covers with four chunks per thread.
-    std::vector<int> first, ngm;
-    for (int a = 0; a < R;) {
-        int b = a;
-        const int m = row_mask ? row_mask[order[a]] : 0;
-        while (b < R && (row_mask ? row_mask[order[b]] : 0) == m) ++b;
-        first.push_back(a);
-        ngm.push_back((b - a + 63) / 64);
-        a = b;
-    }
-    first.push_back(R);
-    int total_groups = 0;
-    for (int q : ngm) total_groups += q;
-    const int xs_bytes = g0.fmt.narrow ? 8192 : (g0.PC + 16) * 16;     // (stream_xs)
-    int cap = (160 * 1024 - 65536 - STREAM_RUN_MAX * 256 - 1024) / xs_bytes;
-    cap = std::min(cap, std::min(4, 4096 / g0.PC));            // (4: two activation rows per pass still fit LDS at C = 5120)
-    if (cap < 1 || !row_mask) cap = 1;
-    // the runs for a run length GR (into `out` if given): returns their number
-    auto pack = [&](int GR, std::vector<StreamRun>* out, int* longest) {
-        int64_t n = 0;
-        StreamRun cur{0, 0, 0, 0, {0}, {0}};
-        int gbase = 0, lg = 1;
-        auto flush = [&]() {
-            if (cur.ng > 0) { ++n; lg = std::max(lg, cur.ng); if (out) out->push_back(cur); }
-            cur = StreamRun{0, 0, 0, 0, {0}, {0}};
-        };
-        for (size_t i = 0; i < ngm.size(); ++i) {
-            const int q = ngm[i], m = row_mask ? row_mask[order[first[i]]] : 0;
-            if (q > GR) {                                        // an order longer than a run: runs of its own
-                flush();
-                for (int p0 = 0; p0 < q; p0 += GR) {
-                    cur = StreamRun{gbase + p0, std::min(GR, q - p0), 1, 0, {0}, {(uint8_t)m}};
-                    flush();
-                }
-            } else if (cur.ng > 0 && cur.ng + q <= GR && cur.norders < cap) {
-                cur.bound[cur.norders] = (uint8_t)cur.ng;
-                cur.order[cur.norders] = (uint8_t)m;
-                ++cur.norders;
-                cur.ng += q;
-            } else {
-                flush();
-                cur = StreamRun{gbase, q, 1, 0, {0}, {(uint8_t)m}};
-            }
-            gbase += q;
-        }
-        flush();
-        if (longest) *longest = lg;
-        return n;
-    };
-    // GR = the fewest groups per run that keep the run count within the request.  A run's partial sums are staged in
-    // LDS: no run longer than STREAM_RUN_MAX groups (more runs than asked for then).
-    int GR = 1;
-    while (GR < STREAM_RUN_MAX && GR < total_groups && pack(GR, nullptr, nullptr) > runs) ++GR;
-    // With one column order the kernel derives the cut from the run count alone, as ceil(groups / runs) per run: settle
-    // on a run length that this formula gives back.
-    if (ngm.size() == 1)
-        for (;;) {
-            const int n = (ngm[0] + GR - 1) / GR, g2 = (ngm[0] + n - 1) / n;
-            if (g2 == GR) break;
-            GR = g2;
-        }
-    P.runs.clear();
-    P.base.clear();
-    pack(GR, &P.runs, &P.GR);
-    P.orders_max = 1;
-    for (const StreamRun& run : P.runs) P.orders_max = std::max(P.orders_max, (int)run.norders);
-    for (size_t i = 0; i < ngm.size(); ++i) {
-        const int a = first[i], b = first[i + 1];
-        for (int k = 0; k < ngm[i] * 64; ++k) P.base.push_back(a + k < b ? order[a + k] : STREAM_NO_ROW);
-    }
-    P.g = stream_geom(C, d, lbits, (int)(P.base.size() / 64), (int)P.runs.size(), balanced);
-    const StreamGeom& g = P.g;
-    P.cnt.assign((size_t)g.NV * R, 0);
-    P.pos.assign((size_t)g.NV * R, 0);
-    P.goff.assign((size_t)g.NV * g.NG + 1, 0);
-    parallel_rows(R, [&](int a, int b) {
-        for (int r = a; r < b; ++r) {
-            const uint32_t* row = tags + (size_t)r * W;
-            const uint32_t book = row_book ? (uint32_t)(row_book[r] & (G - 1)) << bits : 0u;
-            for (int j = 0; j < g.U; ++j) {
-                uint32_t t = host_tag(row, W, bits, j);
-                if (remap) t = remap[t];
-                t |= book;
-                const int v = (j / g.PC) * g.NS + (int)(t >> STREAM_SLICE_BITS);
-                ++P.cnt[(size_t)v * R + r];
-            }
-        }
-    });
-    std::vector<uint32_t> steps((size_t)g.NV * g.NG, 0);
-    parallel_rows(g.NV, [&](int a, int b) {
-        std::vector<uint32_t> rows;
-        for (int v = a; v < b; ++v) {
-            const uint16_t* c = &P.cnt[(size_t)v * R];
-            for (const StreamRun& run : P.runs) {
-                // rows move between the groups of one column order only: a group reads one copy of x
-                for (int oi = 0; oi < run.norders; ++oi) {
-                    const int ga = run.g0 + run.bound[oi], gb = run.g0 + (oi + 1 < run.norders ? run.bound[oi + 1] : run.ng);
-                    rows.clear();
-                    for (int k = ga * 64; k < gb * 64; ++k)
-                        if (P.base[k] != STREAM_NO_ROW) rows.push_back(P.base[k]);
-                    std::stable_sort(rows.begin(), rows.end(), [c](uint32_t x, uint32_t y) { return c[x] > c[y]; });
-                    for (size_t k = 0; k < rows.size(); ++k) P.pos[(size_t)v * R + rows[k]] = (uint32_t)(ga * 64 + k);
-                    for (size_t k = 0; k < rows.size(); k += 64)
-                        steps[(size_t)v * g.NG + ga + k / 64] = (c[rows[k]] + (uint32_t)g.fmt.eps - 1u) / (uint32_t)g.fmt.eps;
-                }
-            }
-        }
-    });
-    uint64_t tot = 0;
-    for (size_t k = 0; k < steps.size(); ++k) { P.goff[k] = (uint32_t)tot; tot += steps[k]; }
-    P.goff[steps.size()] = (uint32_t)tot;
-    P.logical_steps = tot;
-    // Units and places: the first-steps region (NU units x NV buckets x FS steps) comes first, the groups'
-    // remaining steps follow bucket after bucket, group after group.
-    P.NU = 0;
-    P.run_of.assign(g.NG, 0);
-    for (size_t ri = 0; ri < P.runs.size(); ++ri) {
-        StreamRun& run = P.runs[ri];
-        run.u0 = P.NU;
-        P.NU += run.ng * stream_split_of(run.ng);
-        for (int k = 0; k < run.ng; ++k) P.run_of[run.g0 + k] = (uint32_t)ri;
-    }
-    // FS: the longest unit's step count, at most the prefetch depth
-    const uint32_t PF = (uint32_t)g.fmt.pf;
-    uint32_t fs = 1;
-    for (int v = 0; v < g.NV; ++v)
-        for (int gi = 0; gi < g.NG; ++gi) {
-            const uint32_t split = (uint32_t)stream_split_of(P.runs[P.run_of[gi]].ng), nst = steps[(size_t)v * g.NG + gi];
-            fs = std::max(fs, std::min(PF, (nst + split - 1) / split));
-        }
-    P.g.fs = (int)fs;
-    P.head4.assign((size_t)g.NV * g.NG * 4, 0);
-    uint64_t at = (uint64_t)P.NU * g.NV * fs;
-    for (int v = 0; v < g.NV; ++v)
-        for (int gi = 0; gi < g.NG; ++gi) {
-            const StreamRun& run = P.runs[P.run_of[gi]];
-            const uint32_t split = (uint32_t)stream_split_of(run.ng), nst = steps[(size_t)v * g.NG + gi];
-            uint32_t* h = &P.head4[((size_t)v * g.NG + gi) * 4];
-            h[0] = (uint32_t)at;
-            h[1] = nst;
-            h[2] = (uint32_t)run.u0 + (uint32_t)(gi - run.g0) * split;
-            h[3] = split | ((uint32_t)run.g0 << 8);
-            if (nst / split >= PF) at += nst - split * PF;
-        }
-    P.g.total_steps = at;
-}
-
-void stream_balance_host(const uint32_t* tags, int R, int W, int C, int d, int bits, uint16_t* remap_out, int G,
-                         const uint8_t* row_book) {
-    std::vector<uint16_t> remap;
-    balance_codewords(tags, R, W, C / d, bits, remap, G, row_book);
-    memcpy(remap_out, remap.data(), remap.size() * sizeof(uint16_t));
-}
-
-size_t stream_bytes_host(const uint32_t* tags, int R, int W, int C, int d, int bits, const uint8_t* row_mask, int runs,
-                         const uint16_t* table, int G, const uint8_t* row_book) {
-    StreamPlan P;
-    plan_stream(tags, R, W, C, d, bits, row_mask, runs, P, table != nullptr, G, row_book);
-    return P.g.off_steps + (size_t)P.g.total_steps * P.g.fmt.step_bytes;
-}
-
-// The lanes of a wave that one clock of a 16-byte LDS read serves.  A ds_read_b128 takes four clocks; measured on
-// gfx950 (two lanes reading different rows of one bank group while every other lane reads a third address: one extra
-// clock exactly for the pairs listed together here; 256 random address patterns then fit "sum over the four sets of
-// the most distinct addresses in one group of four banks" to within 1 percent), the sets are not 16 consecutive lanes:
-static const int LDS_CLOCK_LANES[4][16] = {
-    {0, 1, 2, 3, 12, 13, 14, 15, 20, 21, 22, 23, 24, 25, 26, 27},
-    {4, 5, 6, 7, 8, 9, 10, 11, 16, 17, 18, 19, 28, 29, 30, 31},
-    {32, 33, 34, 35, 44, 45, 46, 47, 52, 53, 54, 55, 56, 57, 58, 59},
-    {36, 37, 38, 39, 40, 41, 42, 43, 48, 49, 50, 51, 60, 61, 62, 63}};
-
-// Orders the entries of the 16 lanes of one LDS clock (see the second pass of stream_build_host): every entry slot
-// should hold, over the 16 lanes, 16 different codeword bank groups (tag mod 16) and 16 different bank groups of x
-// (chunk mod 16).  A greedy fill (each lane takes the entry that collides least with the lanes before it) followed by
-// hill climbing over the whole group: a lane that collides in a slot swaps that entry with one of its other slots when
-// the two slots together get cheaper.
-struct BankMatch {
-    static constexpr uint32_t NONE = 0xFFFFFFFFu;
-    std::vector<uint32_t> ent[16];           // [lane][slot]: the lane's real entries in slot order
-    std::vector<uint8_t> ha, hb;             // [slot][16]: lanes per codeword / x bank group
-    std::vector<uint8_t> mx;                 // [slot][4]: fullest codeword group, groups that full; the same for x
-    uint32_t cnt[16];
-    uint32_t eps = 4;                        // entries per lane and step (StreamFmt.eps)
-
-    // entry n of a lane in a group whose steps begin at base: entries are kept one per word, [step][lane][eps], until
-    // they are moved to their places
-    uint32_t* rec_of(uint32_t* base, int lane, uint32_t n) const { return base + ((size_t)(n / eps) * 64 + lane) * eps + n % eps; }
-    static int ga(uint32_t e) { return (int)(e & 15u); }
-    static int gb(uint32_t e) { return (int)((e >> STREAM_SLICE_BITS) & 15u); }
-    void add(uint32_t n, uint32_t e, int d) { ha[n * 16 + ga(e)] += d; hb[n * 16 + gb(e)] += d; }
-
-    // zero_chunk: the first of the 16 chunks of x that the kernel keeps at zero
-    void order_lanes(uint32_t* base, const uint32_t* sl, const int* lanes, uint32_t ns, uint32_t zero_chunk) {
-        uint32_t most = 0;
-        for (int l = 0; l < 16; ++l) {
-            const uint32_t s0 = sl[lanes[l]];
-            cnt[l] = (s0 & STREAM_NO_ROW) == STREAM_NO_ROW ? 0u : s0 >> STREAM_ROW_BITS;
-            ent[l].resize(cnt[l]);
-            for (uint32_t n = 0; n < cnt[l]; ++n) ent[l][n] = *rec_of(base, lanes[l], n);
-            most = std::max(most, cnt[l]);
-        }
-        if (most == 0) return;
-        ha.assign((size_t)ns * 16, 0);
-        hb.assign((size_t)ns * 16, 0);
-        // greedy fill, slot by slot; the lanes with the fewest entries left choose first
-        int order[16];
-        for (int l = 0; l < 16; ++l) order[l] = l;
-        std::sort(order, order + 16, [this](int x, int y) { return cnt[x] != cnt[y] ? cnt[x] < cnt[y] : x < y; });
-        for (uint32_t n = 0; n < most; ++n)
-            for (int d = 0; d < 16; ++d) {
-                const int l = order[d];
-                if (cnt[l] <= n) continue;
-                uint32_t bi = n;
-                int bc = 1 << 30;
-                for (uint32_t i = n; i < cnt[l]; ++i) {
-                    const int c = ha[n * 16 + ga(ent[l][i])] + hb[n * 16 + gb(ent[l][i])];
-                    if (c < bc) { bc = c; bi = i; if (c == 0) break; }
-                }
-                std::swap(ent[l][n], ent[l][bi]);
-                add(n, ent[l][n], 1);
-            }
-        // Hill climbing.  What a slot costs is the fullest bank group of its codeword reads plus that of its x reads
-        // (clocks); with 16 lanes on 16 bank groups some collisions are forced, and they are cheapest when they share
-        // slots.  A lane in a fullest group swaps that entry with one of its other slots when the clocks of the two
-        // slots together go down (ties: when the sum of squared group counts does).  The fullest group's count after
-        // moving one lane from group p to group q follows from the count, the current maximum and how many groups hold
-        // it, so a candidate costs a few operations.
-        mx.assign((size_t)most * 4, 0);
-        auto rescan = [&](uint32_t n) {
-            uint8_t* m4 = &mx[n * 4];
-            m4[0] = m4[1] = m4[2] = m4[3] = 0;
-            for (int k = 0; k < 16; ++k) {
-                const uint8_t a = ha[n * 16 + k], b = hb[n * 16 + k];
-                if (a > m4[0]) { m4[0] = a; m4[1] = 1; } else if (a == m4[0]) ++m4[1];
-                if (b > m4[2]) { m4[2] = b; m4[3] = 1; } else if (b == m4[2]) ++m4[3];
-            }
-        };
-        // fullest count of histogram h (maximum M held by `at` groups) once a lane leaves group p and joins group q
-        auto moved = [](const uint8_t* h, int M, int at, int p, int q) {
-            if (p == q) return M;
-            if (h[q] + 1 > M) return h[q] + 1;
-            return (h[p] == M && at == 1 && h[q] + 1 < M) ? M - 1 : M;
-        };
-        for (uint32_t n = 0; n < most; ++n) rescan(n);
-        for (int pass = 0; pass < STREAM_CLIMB; ++pass) {
-            bool improved = false;
-            for (uint32_t n = 0; n < most; ++n) {
-                const uint8_t* an = &ha[n * 16];
-                const uint8_t* bn = &hb[n * 16];
-                const uint8_t* xn = &mx[n * 4];
-                if (xn[0] + xn[2] <= 2) continue;
-                for (int l = 0; l < 16; ++l) {
-                    if (cnt[l] <= n) continue;
-                    const uint32_t e = ent[l][n];
-                    const int ae = ga(e), be = gb(e);
-                    if (!((an[ae] == xn[0] && xn[0] > 1) || (bn[be] == xn[2] && xn[2] > 1))) continue;
-                    int best = 0;
-                    uint32_t bm = n;
-                    for (uint32_t m = 0; m < cnt[l]; ++m) {
-                        if (m == n) continue;
-                        const uint32_t f = ent[l][m];
-                        const int af = ga(f), bf = gb(f);
-                        const uint8_t* am = &ha[m * 16];
-                        const uint8_t* bq = &hb[m * 16];
-                        const uint8_t* xm = &mx[m * 4];
-                        const int clocks = moved(an, xn[0], xn[1], ae, af) + moved(bn, xn[2], xn[3], be, bf) +
-                                           moved(am, xm[0], xm[1], af, ae) + moved(bq, xm[2], xm[3], bf, be) -
-                                           (xn[0] + xn[2] + xm[0] + xm[2]);
-                        if (clocks > 0) continue;
-                        int sq = 0;
-                        if (af != ae) sq += 4 + 2 * ((int)an[af] - an[ae] + am[ae] - am[af]);
-                        if (bf != be) sq += 4 + 2 * ((int)bn[bf] - bn[be] + bq[be] - bq[bf]);
-                        const int delta = clocks * 1024 + sq;
-                        if (delta < best) { best = delta; bm = m; }
-                    }
-                    if (bm != n) {
-                        const uint32_t f = ent[l][bm];
-                        add(n, e, -1); add(bm, f, -1); add(n, f, 1); add(bm, e, 1);
-                        std::swap(ent[l][n], ent[l][bm]);
-                        rescan(n);
-                        rescan(bm);
-                        improved = true;
-                        if (xn[0] + xn[2] <= 2) break;
-                    }
-                }
-            }
-            if (!improved) break;
-        }
-        // Write the slots back.  A lane that has run out repeats one of its own codewords (from the least used bank
-        // group) against one of the 16 chunks of x that are kept at zero (one per bank group).  A lane without a row,
-        // or whose row has no entry here, reads what a neighbour reads (the same addresses are one broadcast read); the
-        // kernel drops its sum.
-        for (uint32_t n = 0; n < ns; ++n) {
-            uint32_t chosen[16];
-            int donor = -1;
-            for (int l = 0; l < 16; ++l)
-                if (cnt[l] > n) { chosen[l] = ent[l][n]; if (donor < 0) donor = l; }
-            for (int l = 0; l < 16; ++l) {
-                if (cnt[l] > n || cnt[l] == 0) continue;
-                uint32_t bi = 0;
-                for (uint32_t i = 1; i < cnt[l]; ++i)
-                    if (ha[n * 16 + ga(ent[l][i])] < ha[n * 16 + ga(ent[l][bi])]) bi = i;
-                int kb = 0;
-                for (int k = 1; k < 16; ++k)
-                    if (hb[n * 16 + k] < hb[n * 16 + kb]) kb = k;
-                chosen[l] = (ent[l][bi] & ((1u << STREAM_SLICE_BITS) - 1u)) | ((uint32_t)(zero_chunk + kb) << STREAM_SLICE_BITS);
-                add(n, chosen[l], 1);
-                if (donor < 0) donor = l;
-            }
-            for (int l = 0; l < 16; ++l) {
-                if (cnt[l] == 0) chosen[l] = donor >= 0 ? chosen[donor] : 0u;
-                *rec_of(base, lanes[l], n) = chosen[l];
-            }
-        }
-    }
-};
-
-// One step of 64 lanes x eps entries (one per word) into its bytes: 3 bytes per entry (wide), or the three 21-bit
-// entries of a lane in one 64-bit word (narrow).
-static void encode_step(const uint32_t* e, const StreamFmt& f, unsigned char* out) {
-    for (int lane = 0; lane < 64; ++lane) {
-        const uint32_t* r = e + (size_t)lane * f.eps;
-        unsigned char* o = out + (size_t)lane * f.lane_bytes;
-        if (f.narrow) {
-            const uint64_t w = (uint64_t)r[0] | (uint64_t)r[1] << 21 | (uint64_t)r[2] << 42;
-            for (int b = 0; b < 8; ++b) o[b] = (unsigned char)(w >> (8 * b));
-        } else {
-            for (int k = 0; k < 4; ++k) { o[3 * k] = (unsigned char)r[k]; o[3 * k + 1] = (unsigned char)(r[k] >> 8); o[3 * k + 2] = (unsigned char)(r[k] >> 16); }
-        }
-    }
-}
-
-int stream_build_host(const uint32_t* tags, int R, int W, int C, int d, int bits, const uint8_t* row_mask, int runs,
-                      unsigned char* out, size_t bytes, int* runs_out, int* groups_out, const uint16_t* table, int G,
-                      const uint8_t* row_book) {
-    StreamPlan P;
-    plan_stream(tags, R, W, C, d, bits, row_mask, runs, P, table != nullptr, G, row_book);
-    const uint16_t* remap = table ? P.remap.data() : nullptr;
-    const StreamGeom& g = P.g;
-    const StreamFmt f = g.fmt;
-    const uint32_t EPS = (uint32_t)f.eps, PF = (uint32_t)f.pf, FS = (uint32_t)g.fs;
-    const size_t need = g.off_steps + (size_t)g.total_steps * f.step_bytes;
-    if (g.total_steps >= ((uint64_t)1 << 32) || g.runs >= (1 << 16)) return fail(SQ_EUNSUPPORTED, "sq_stream_build: matrix too large");
-    if (bytes < need) return fail(SQ_EINVAL, "sq_stream_build: buffer %zu < %zu", bytes, need);
-    memset(out, 0, need);
-    memcpy(out, P.head4.data(), P.head4.size() * 4);
-    memcpy(out + g.off_runs, P.runs.data(), P.runs.size() * sizeof(StreamRun));
-    memcpy(out + g.off_rows, P.base.data(), P.base.size() * 4);
-    if (table) {
-        uint16_t* tab = (uint16_t*)(out + g.off_table);
-        uint16_t* unmap = (uint16_t*)(out + g.off_unmap);
-        for (int k = 0; k < (1 << bits); ++k) {
-            memcpy(tab + (size_t)remap[k] * d, table + (size_t)k * d, (size_t)d * 2);
-            unmap[remap[k]] = (uint16_t)k;
-        }
-    }
-    std::vector<uint32_t> place(R);
-    for (size_t k = 0; k < P.base.size(); ++k)
-        if (P.base[k] != STREAM_NO_ROW) place[P.base[k]] = (uint32_t)k;
-    P.slot32.assign((size_t)g.NV * g.NG * 64, STREAM_NO_ROW);
-    uint32_t* slots = P.slot32.data();
-    // the steps are made group after group (P.goff), one entry per word, and moved to their places at the end
-    std::vector<uint32_t> laid((size_t)P.logical_steps * 64 * EPS, 0);
-    uint32_t* steps = laid.data();
-    auto rec = [&](size_t step0, uint32_t lane, uint32_t n) { return steps + ((step0 + n / EPS) * 64 + lane) * EPS + n % EPS; };
-    parallel_rows(R, [&](int a, int b) {
-        std::vector<uint32_t> q(g.NV), last(g.NV);
-        for (int r = a; r < b; ++r) {
-            const uint32_t* row = tags + (size_t)r * W;
-            const uint32_t book = row_book ? (uint32_t)(row_book[r] & (G - 1)) << bits : 0u;
-            std::fill(q.begin(), q.end(), 0u);
-            std::fill(last.begin(), last.end(), 0u);
-            for (int v = 0; v < g.NV; ++v) {
-                const uint32_t k = P.pos[(size_t)v * R + r];
-                slots[(size_t)v * g.NG * 64 + k] = place[r] | ((uint32_t)P.cnt[(size_t)v * R + r] << STREAM_ROW_BITS);
-            }
-            for (int j = 0; j < g.U; ++j) {
-                uint32_t t = host_tag(row, W, bits, j);
-                if (remap) t = remap[t];
-                t |= book;
-                const int kp = j / g.PC, v = kp * g.NS + (int)(t >> STREAM_SLICE_BITS);
-                const uint32_t k = P.pos[(size_t)v * R + r], n = q[v]++;
-                const uint32_t e = (t & ((1u << STREAM_SLICE_BITS) - 1u)) | ((uint32_t)(j - kp * g.PC) << STREAM_SLICE_BITS);
-                *rec(P.goff[(size_t)v * g.NG + (k >> 6)], k & 63, n) = e;
-                last[v] = e & ((1u << STREAM_SLICE_BITS) - 1u);
-            }
-            // Padding up to the group's longest row: the row's last codeword of the bucket again, at the chunk of x
-            // that the kernel keeps at zero, so padding adds exactly nothing and needs no test in the inner loop
-            // (a codeword that is not finite is already part of the row's sum; a row without entries in the
-            // bucket is dropped by its slot).
-            for (int v = 0; v < g.NV; ++v) {
-                const uint32_t k = P.pos[(size_t)v * R + r];
-                const size_t gi = (size_t)v * g.NG + (k >> 6);
-                const uint32_t cap = (P.goff[gi + 1] - P.goff[gi]) * EPS;
-                const uint32_t e = last[v] | ((uint32_t)g.PC << STREAM_SLICE_BITS);
-                for (uint32_t n = q[v]; n < cap; ++n) *rec(P.goff[gi], k & 63, n) = e;
-            }
-        }
-    });
-    // Second pass, group by group: the order of a lane's entries is free (padding stays behind them), so it is
-    // chosen to keep the LDS gathers apart.  A 16-byte LDS read of a wave takes four clocks of 16 lanes each
-    // (LDS_CLOCK_LANES), and two lanes of a clock collide when their addresses differ but fall into the same group
-    // of four banks (address / 16 mod 16): BankMatch arranges the entries of each clock's lanes.
-    parallel_rows(g.NV * g.NG, [&](int a, int b) {
-        BankMatch bm;
-        bm.eps = EPS;
-        for (int vg = a; vg < b; ++vg) {
-            const uint32_t st0 = P.goff[vg], ns = (P.goff[vg + 1] - st0) * EPS;
-            if (ns == 0) continue;
-            const uint32_t* sl = slots + (size_t)vg * 64;
-            uint32_t* base = steps + (size_t)st0 * 64 * EPS;
-            for (int q = 0; q < 4; ++q) bm.order_lanes(base, sl, LDS_CLOCK_LANES[q], ns, (uint32_t)g.PC);
-        }
-    });
-    // to their places: the first FS steps of every unit into the first-steps region, the rest behind each other; and
-    // the slots in their 16-bit form (place counted from the run's first place, entries or none)
-    uint16_t* slot16 = (uint16_t*)(out + g.off_slots);
-    parallel_rows(g.NV * g.NG, [&](int a, int b) {
-        for (int vg = a; vg < b; ++vg) {
-            const uint32_t* h = &P.head4[(size_t)vg * 4];
-            const int v = vg / g.NG, nst = (int)h[1], split = (int)(h[3] & 0xFFu);
-            const uint32_t p0 = (h[3] >> 8) * 64u;
-            for (int lane = 0; lane < 64; ++lane) {
-                const uint32_t s32 = slots[(size_t)vg * 64 + lane];
-                slot16[(size_t)vg * 64 + lane] = (s32 & STREAM_NO_ROW) == STREAM_NO_ROW
-                    ? (uint16_t)STREAM_SLOT_NONE
-                    : (uint16_t)(((s32 & STREAM_NO_ROW) - p0) | ((s32 >> STREAM_ROW_BITS) ? STREAM_SLOT_HAS : 0u));
-            }
-            const uint32_t* src = steps + (size_t)P.goff[vg] * 64 * EPS;
-            for (int j = 0; j < split; ++j) {
-                const int s0 = nst * j / split, s1 = nst * (j + 1) / split;
-                for (int t = s0; t < s1; ++t) {
-                    const uint64_t to = (uint32_t)(t - s0) < PF ? ((uint64_t)(h[2] + j) * g.NV + v) * FS + (t - s0)
-                                                                 : (uint64_t)h[0] + t - (uint64_t)PF * (j + 1);
-                    encode_step(src + (size_t)t * 64 * EPS, f, out + g.off_steps + to * f.step_bytes);
-                }
-            }
-        }
-    });
-    if (runs_out) *runs_out = g.runs | (P.GR << 16) | ((P.orders_max - 1) << 24) | ((g.fs - 1) << 27) | (table ? STREAM_BALANCED : 0);
-    if (groups_out) *groups_out = g.NG;
-    return SQ_OK;
-}
 
 // ---------------------------------------------------------------------------------------- device
 

@@ -1,0 +1,1085 @@
+// Load-time builder of the bucketed tag stream (layout: sq_stream.hip and sq_stream.h), on the host and on the GPU.
+#include <algorithm>
+#include <atomic>
+#include <memory>
+#include <new>
+#include <string.h>
+#include <thread>
+#include <vector>
+#include "sq_stream.h"
+
+constexpr int STREAM_CLIMB = 1;      // hill-climbing passes of the entry ordering (load time against LDS collisions)
+
+namespace sq {
+
+// A run: groups g0 .. g0 + ng - 1 of every bucket.  Its rows belong to `norders` column orders (one without row orders);
+// the groups of order[i] begin at group bound[i] of the run (bound[0] = 0), and the kernel keeps copy i of x, gathered
+// through that order, in LDS for them.
+// u0: the index of the run's first unit (units are counted run after run).
+struct StreamRun { int32_t g0, ng, norders, u0; uint8_t bound[STREAM_RUN_ORDERS]; uint8_t order[STREAM_RUN_ORDERS]; };
+static_assert(sizeof(StreamRun) == 32, "run records are read as 8 dwords");
+
+StreamGeom stream_geom(int C, int d, int bits, int groups, int runs, bool balanced, int fs) {
+    StreamGeom g;
+    g.U = C / d;
+    g.NS = 1 << (bits - STREAM_SLICE_BITS);
+    g.KP = (g.U + STREAM_PART_MAX - 1) / STREAM_PART_MAX;
+    g.PC = (g.U + g.KP - 1) / g.KP;
+    g.NV = g.NS * g.KP;
+    g.NG = groups;
+    g.runs = runs;
+    g.fmt = stream_fmt(g.PC);
+    g.fs = fs < 1 ? g.fmt.pf : fs < g.fmt.pf ? fs : g.fmt.pf;
+    g.off_slots = ((size_t)g.NV * g.NG * 16 + 255) & ~(size_t)255;          // four words per (bucket, group)
+    g.off_runs = (g.off_slots + (size_t)g.NV * g.NG * 64 * 2 + 255) & ~(size_t)255;
+    g.off_rows = (g.off_runs + (size_t)runs * sizeof(StreamRun) + 255) & ~(size_t)255;
+    size_t end = (g.off_rows + (size_t)g.NG * 64 * 4 + 255) & ~(size_t)255;
+    g.off_table = g.off_unmap = 0;
+    if (balanced) {
+        g.off_table = end;
+        g.off_unmap = end + ((size_t)d * 2 << bits);
+        end = (g.off_unmap + ((size_t)2 << bits) + 255) & ~(size_t)255;
+    }
+    g.off_steps = end;
+    g.total_steps = 0;
+    return g;
+}
+
+// (R + 64 * 256 bounds the places: every column order can leave one group short)
+bool stream_format_ok(int R, int C, int d, int bits, int G) {
+    if (G < 1 || (G & (G - 1)) != 0 || bits < 1 || bits > 16) return false;
+    const int lb = stream_label_bits(bits, G);
+    return d == 8 && lb > STREAM_SLICE_BITS && (1 << (lb - STREAM_SLICE_BITS)) <= (G > 1 ? STREAM_SLICES_MAX : 16) && C % d == 0 &&
+           R > 0 && R + 64 * 256 < (int)STREAM_NO_ROW;
+}
+
+static inline uint32_t host_tag(const uint32_t* row, int W, int bits, int j) {
+    const int64_t p = (int64_t)j * bits;
+    const int w = (int)(p >> 5), s = (int)(p & 31);
+    uint64_t v = row[w];
+    if (s + bits > 32 && w + 1 < W) v |= (uint64_t)row[w + 1] << 32;
+    return (uint32_t)(v >> s) & ((1u << bits) - 1u);
+}
+
+// fn(a, b) over blocks of `grain` of the indices 0 .. n - 1, on up to 16 threads that take the next block as they get to
+// it.  `grain` is what makes a block worth a thread: one group's entry ordering takes milliseconds (with a fixed minimum of
+// 64 indices per thread the 896 groups of a 3584-row matrix ran on one).
+static void parallel_blocks(int n, int grain, const std::function<void(int, int)>& fn) {
+    const int blocks = (n + grain - 1) / grain;
+    const int nt = std::min({(int)std::max(1u, std::thread::hardware_concurrency()), 16, blocks});
+    if (nt <= 1) { if (n > 0) fn(0, n); return; }
+    std::atomic<int> next{0};
+    auto work = [&]() {
+        for (int k; (k = next.fetch_add(1, std::memory_order_relaxed)) < blocks;) fn(k * grain, std::min(n, (k + 1) * grain));
+    };
+    std::vector<std::thread> th;
+    for (int t = 1; t < nt; ++t) th.emplace_back(work);
+    work();
+    for (auto& t : th) t.join();
+}
+
+struct StreamPlan {
+    StreamGeom g;
+    int GR;                          // groups in the longest run
+    int orders_max;                  // most column orders in one run
+    std::vector<StreamRun> runs;
+    std::vector<uint32_t> base;      // [NG * 64]: rows ordered by column order, STREAM_NO_ROW where a group is short
+    std::vector<uint16_t> cnt;       // [NV][R]
+    std::vector<uint32_t> pos;       // [NV][R]: lane position (group * 64 + lane) of row r in bucket v
+    std::vector<uint32_t> goff;      // [NV * NG + 1]: the groups' steps counted bucket after bucket, group after group (how the
+                                     // builder lays them out before they move to their places)
+    uint64_t logical_steps;          // goff[NV * NG]
+    int NU;                          // units of one bucket
+    std::vector<uint32_t> slot32;    // [NV * NG * 64]: place | count << STREAM_ROW_BITS per lane (STREAM_NO_ROW: no row), the
+                                     // builder's own form of the slots
+    std::vector<uint32_t> run_of;    // [NG]: the run of a group
+    std::vector<uint32_t> head4;     // [NV * NG][4]: {rest, nst, unit0, split}, what the buffer holds per (bucket, group)
+    std::vector<uint16_t> remap;     // balanced streams: file id -> new id (empty: identity)
+};
+
+// Relabelling of the codewords for a stream with a codebook of its own: the codewords are dealt, most used first, to
+// whichever slice of 4096 carries the fewest tags so far and still has room, so every slice ends up with the same
+// share of the tags (a slice is one workgroup's work) whatever the distribution of the tags is, and a slice's popular
+// codewords get consecutive places, i.e. different LDS bank groups.
+// With several codebooks (row_book names a row's) every codebook is relabelled by itself, over its own slices:
+// remap[book << bits | label] is the new label within the book; a codebook of at most one slice keeps its labels.
+// count[book << bits | label]: how many tags name each codeword.
+static void deal_codewords(const uint32_t* count, int bits, std::vector<uint16_t>& remap, int G) {
+    const int K = 1 << bits, NS = K >> STREAM_SLICE_BITS, SL = 1 << STREAM_SLICE_BITS;
+    remap.assign((size_t)G * K, 0);
+    if (NS < 2) {
+        for (size_t k = 0; k < remap.size(); ++k) remap[k] = (uint16_t)(k & (size_t)(K - 1));
+        return;
+    }
+    std::vector<uint32_t> ids(K), first;
+    std::vector<uint64_t> load(NS);
+    std::vector<int> fill(NS);
+    for (int b = 0; b < G; ++b) {
+        const uint32_t* cb = count + (size_t)b * K;
+        // ids by count, most used first, equal counts by id: a counting sort (counts are small when the tags spread)
+        const uint32_t most = *std::max_element(cb, cb + K);
+        if (most < (1u << 20)) {
+            first.assign((size_t)most + 2, 0);
+            for (int k = 0; k < K; ++k) ++first[most - cb[k] + 1];
+            for (size_t c = 1; c < first.size(); ++c) first[c] += first[c - 1];
+            for (int k = 0; k < K; ++k) ids[first[most - cb[k]]++] = (uint32_t)k;
+        } else {
+            for (int k = 0; k < K; ++k) ids[k] = (uint32_t)k;
+            std::stable_sort(ids.begin(), ids.end(), [cb](uint32_t x, uint32_t y) { return cb[x] > cb[y]; });
+        }
+        std::fill(load.begin(), load.end(), 0);
+        std::fill(fill.begin(), fill.end(), 0);
+        for (int k = 0; k < K; ++k) {
+            int best = -1;
+            for (int sl = 0; sl < NS; ++sl)
+                if (fill[sl] < SL && (best < 0 || load[sl] < load[best])) best = sl;
+            remap[(size_t)b * K + ids[k]] = (uint16_t)(best * SL + fill[best]);
+            ++fill[best];
+            load[best] += cb[ids[k]];
+        }
+    }
+}
+
+static void balance_codewords(const uint32_t* tags, int R, int W, int U, int bits, std::vector<uint16_t>& remap, int G = 1,
+                              const uint8_t* row_book = nullptr) {
+    std::vector<uint32_t> count((size_t)G << bits, 0);
+    if ((1 << bits) >> STREAM_SLICE_BITS >= 2)
+        for (int r = 0; r < R; ++r) {
+            const uint32_t* row = tags + (size_t)r * W;
+            uint32_t* cb = count.data() + ((size_t)(row_book ? row_book[r] & (G - 1) : 0) << bits);
+            for (int j = 0; j < U; ++j) ++cb[host_tag(row, W, bits, j)];
+        }
+    deal_codewords(count.data(), bits, remap, G);
+}
+
+// Three steps: the rows' order, groups and runs; how many entries every row has in every bucket; and from those counts the
+// lanes' places, the groups' lengths and where their steps go.  The counts come from the host's or the device's tags.
+static void plan_rows(int R, int C, int d, int lbits, const uint8_t* row_mask, int runs, StreamPlan& P, bool balanced) {
+    // rows by column order, groups and runs
+    std::vector<uint32_t> order(R);
+    for (int r = 0; r < R; ++r) order[r] = (uint32_t)r;
+    if (row_mask)
+        std::stable_sort(order.begin(), order.end(), [row_mask](uint32_t a, uint32_t b) { return row_mask[a] < row_mask[b]; });
+    StreamGeom g0 = stream_geom(C, d, lbits, 0, 0);
+    if (runs <= 0) runs = (STREAM_DEFAULT_WGS + g0.NV / 2) / g0.NV;
+    if (runs < 1) runs = 1;
+    // Groups per column order.  A run takes the groups of one order, GR at a time, or, when orders are small, the whole
+    // groups of up to `cap` orders that follow each other (a masked k projection has 64 rows per order: one run per order
+    // would be 16 workgroups of one group each per bucket).  cap: as many gathered copies of x as fit LDS beside the slice
+    // and the run's partial sums, and as the staging loop covers with four chunks per thread.
+    std::vector<int> first, ngm;
+    for (int a = 0; a < R;) {
+        int b = a;
+        const int m = row_mask ? row_mask[order[a]] : 0;
+        while (b < R && (row_mask ? row_mask[order[b]] : 0) == m) ++b;
+        first.push_back(a);
+        ngm.push_back((b - a + 63) / 64);
+        a = b;
+    }
+    first.push_back(R);
+    int total_groups = 0;
+    for (int q : ngm) total_groups += q;
+    const int xs_bytes = g0.fmt.narrow ? 8192 : (g0.PC + 16) * 16;     // (stream_xs)
+    int cap = (160 * 1024 - 65536 - STREAM_RUN_MAX * 256 - 1024) / xs_bytes;
+    cap = std::min(cap, std::min(4, 4096 / g0.PC));            // (4: two activation rows per pass still fit LDS at C = 5120)
+    if (cap < 1 || !row_mask) cap = 1;
+    // the runs for a run length GR (into `out` if given): returns their number
+    auto pack = [&](int GR, std::vector<StreamRun>* out, int* longest) {
+        int64_t n = 0;
+        StreamRun cur{0, 0, 0, 0, {0}, {0}};
+        int gbase = 0, lg = 1;
+        auto flush = [&]() {
+            if (cur.ng > 0) { ++n; lg = std::max(lg, cur.ng); if (out) out->push_back(cur); }
+            cur = StreamRun{0, 0, 0, 0, {0}, {0}};
+        };
+        for (size_t i = 0; i < ngm.size(); ++i) {
+            const int q = ngm[i], m = row_mask ? row_mask[order[first[i]]] : 0;
+            if (q > GR) {                                        // an order longer than a run: runs of its own
+                flush();
+                for (int p0 = 0; p0 < q; p0 += GR) {
+                    cur = StreamRun{gbase + p0, std::min(GR, q - p0), 1, 0, {0}, {(uint8_t)m}};
+                    flush();
+                }
+            } else if (cur.ng > 0 && cur.ng + q <= GR && cur.norders < cap) {
+                cur.bound[cur.norders] = (uint8_t)cur.ng;
+                cur.order[cur.norders] = (uint8_t)m;
+                ++cur.norders;
+                cur.ng += q;
+            } else {
+                flush();
+                cur = StreamRun{gbase, q, 1, 0, {0}, {(uint8_t)m}};
+            }
+            gbase += q;
+        }
+        flush();
+        if (longest) *longest = lg;
+        return n;
+    };
+    // GR = the fewest groups per run that keep the run count within the request.  A run's partial sums are staged in
+    // LDS: no run longer than STREAM_RUN_MAX groups (more runs than asked for then).
+    int GR = 1;
+    while (GR < STREAM_RUN_MAX && GR < total_groups && pack(GR, nullptr, nullptr) > runs) ++GR;
+    // With one column order the kernel derives the cut from the run count alone, as ceil(groups / runs) per run: settle
+    // on a run length that this formula gives back.
+    if (ngm.size() == 1)
+        for (;;) {
+            const int n = (ngm[0] + GR - 1) / GR, g2 = (ngm[0] + n - 1) / n;
+            if (g2 == GR) break;
+            GR = g2;
+        }
+    P.runs.clear();
+    P.base.clear();
+    pack(GR, &P.runs, &P.GR);
+    P.orders_max = 1;
+    for (const StreamRun& run : P.runs) P.orders_max = std::max(P.orders_max, (int)run.norders);
+    for (size_t i = 0; i < ngm.size(); ++i) {
+        const int a = first[i], b = first[i + 1];
+        for (int k = 0; k < ngm[i] * 64; ++k) P.base.push_back(a + k < b ? order[a + k] : STREAM_NO_ROW);
+    }
+    P.g = stream_geom(C, d, lbits, (int)(P.base.size() / 64), (int)P.runs.size(), balanced);
+}
+
+static void plan_counts(const uint32_t* tags, int R, int W, int bits, const uint16_t* remap, int G, const uint8_t* row_book, StreamPlan& P) {
+    const StreamGeom& g = P.g;
+    P.cnt.assign((size_t)g.NV * R, 0);
+    parallel_blocks(R, 64, [&](int a, int b) {
+        for (int r = a; r < b; ++r) {
+            const uint32_t* row = tags + (size_t)r * W;
+            const uint32_t book = row_book ? (uint32_t)(row_book[r] & (G - 1)) << bits : 0u;
+            for (int j = 0; j < g.U; ++j) {
+                uint32_t t = host_tag(row, W, bits, j);
+                if (remap) t = remap[t];
+                t |= book;
+                const int v = (j / g.PC) * g.NS + (int)(t >> STREAM_SLICE_BITS);
+                ++P.cnt[(size_t)v * R + r];
+            }
+        }
+    });
+}
+
+static void plan_places(int R, StreamPlan& P) {
+    const StreamGeom& g = P.g;
+    P.pos.assign((size_t)g.NV * R, 0);
+    P.goff.assign((size_t)g.NV * g.NG + 1, 0);
+    std::vector<uint32_t> steps((size_t)g.NV * g.NG, 0);
+    parallel_blocks(g.NV, 1, [&](int a, int b) {
+        std::vector<uint32_t> rows;
+        for (int v = a; v < b; ++v) {
+            const uint16_t* c = &P.cnt[(size_t)v * R];
+            for (const StreamRun& run : P.runs) {
+                // rows move between the groups of one column order only: a group reads one copy of x
+                for (int oi = 0; oi < run.norders; ++oi) {
+                    const int ga = run.g0 + run.bound[oi], gb = run.g0 + (oi + 1 < run.norders ? run.bound[oi + 1] : run.ng);
+                    rows.clear();
+                    for (int k = ga * 64; k < gb * 64; ++k)
+                        if (P.base[k] != STREAM_NO_ROW) rows.push_back(P.base[k]);
+                    std::stable_sort(rows.begin(), rows.end(), [c](uint32_t x, uint32_t y) { return c[x] > c[y]; });
+                    for (size_t k = 0; k < rows.size(); ++k) P.pos[(size_t)v * R + rows[k]] = (uint32_t)(ga * 64 + k);
+                    for (size_t k = 0; k < rows.size(); k += 64)
+                        steps[(size_t)v * g.NG + ga + k / 64] = (c[rows[k]] + (uint32_t)g.fmt.eps - 1u) / (uint32_t)g.fmt.eps;
+                }
+            }
+        }
+    });
+    uint64_t tot = 0;
+    for (size_t k = 0; k < steps.size(); ++k) { P.goff[k] = (uint32_t)tot; tot += steps[k]; }
+    P.goff[steps.size()] = (uint32_t)tot;
+    P.logical_steps = tot;
+    // Units and places: the first-steps region (NU units x NV buckets x FS steps) comes first, the groups'
+    // remaining steps follow bucket after bucket, group after group.
+    P.NU = 0;
+    P.run_of.assign(g.NG, 0);
+    for (size_t ri = 0; ri < P.runs.size(); ++ri) {
+        StreamRun& run = P.runs[ri];
+        run.u0 = P.NU;
+        P.NU += run.ng * stream_split_of(run.ng);
+        for (int k = 0; k < run.ng; ++k) P.run_of[run.g0 + k] = (uint32_t)ri;
+    }
+    // FS: the longest unit's step count, at most the prefetch depth
+    const uint32_t PF = (uint32_t)g.fmt.pf;
+    uint32_t fs = 1;
+    for (int v = 0; v < g.NV; ++v)
+        for (int gi = 0; gi < g.NG; ++gi) {
+            const uint32_t split = (uint32_t)stream_split_of(P.runs[P.run_of[gi]].ng), nst = steps[(size_t)v * g.NG + gi];
+            fs = std::max(fs, std::min(PF, (nst + split - 1) / split));
+        }
+    P.g.fs = (int)fs;
+    P.head4.assign((size_t)g.NV * g.NG * 4, 0);
+    uint64_t at = (uint64_t)P.NU * g.NV * fs;
+    for (int v = 0; v < g.NV; ++v)
+        for (int gi = 0; gi < g.NG; ++gi) {
+            const StreamRun& run = P.runs[P.run_of[gi]];
+            const uint32_t split = (uint32_t)stream_split_of(run.ng), nst = steps[(size_t)v * g.NG + gi];
+            uint32_t* h = &P.head4[((size_t)v * g.NG + gi) * 4];
+            h[0] = (uint32_t)at;
+            h[1] = nst;
+            h[2] = (uint32_t)run.u0 + (uint32_t)(gi - run.g0) * split;
+            h[3] = split | ((uint32_t)run.g0 << 8);
+            if (nst / split >= PF) at += nst - split * PF;
+        }
+    P.g.total_steps = at;
+}
+
+static int runs_word(const StreamPlan& P) { return P.g.runs | (P.GR << 16) | ((P.orders_max - 1) << 24) | ((P.g.fs - 1) << 27); }
+
+// every lane's place and entry count (slot32), and the slots in the buffer's 16-bit form (place counted from the run's
+// first place, entries or none)
+static void plan_slots(int R, StreamPlan& P) {
+    const StreamGeom& g = P.g;
+    std::vector<uint32_t> place(R);
+    for (size_t k = 0; k < P.base.size(); ++k)
+        if (P.base[k] != STREAM_NO_ROW) place[P.base[k]] = (uint32_t)k;
+    P.slot32.assign((size_t)g.NV * g.NG * 64, STREAM_NO_ROW);
+    parallel_blocks(g.NV, 1, [&](int a, int b) {
+        for (int v = a; v < b; ++v)
+            for (int r = 0; r < R; ++r)
+                P.slot32[(size_t)v * g.NG * 64 + P.pos[(size_t)v * R + r]] = place[r] | ((uint32_t)P.cnt[(size_t)v * R + r] << STREAM_ROW_BITS);
+    });
+}
+
+static void encode_slots(const StreamPlan& P, uint16_t* slot16) {
+    parallel_blocks(P.g.NV * P.g.NG, 256, [&](int a, int b) {
+        for (int vg = a; vg < b; ++vg) {
+            const uint32_t p0 = (P.head4[(size_t)vg * 4 + 3] >> 8) * 64u;
+            for (int lane = 0; lane < 64; ++lane) {
+                const uint32_t s32 = P.slot32[(size_t)vg * 64 + lane];
+                slot16[(size_t)vg * 64 + lane] = (s32 & STREAM_NO_ROW) == STREAM_NO_ROW
+                    ? (uint16_t)STREAM_SLOT_NONE
+                    : (uint16_t)(((s32 & STREAM_NO_ROW) - p0) | ((s32 >> STREAM_ROW_BITS) ? STREAM_SLOT_HAS : 0u));
+            }
+        }
+    });
+}
+
+// (G > 1: the labels a row's tags become are book << bits | tag, see sq_stream.h; `balanced` is for one codebook only)
+static void plan_stream(const uint32_t* tags, int R, int W, int C, int d, int bits, const uint8_t* row_mask, int runs,
+                        StreamPlan& P, bool balanced, int G, const uint8_t* row_book) {
+    P.remap.clear();
+    if (balanced) balance_codewords(tags, R, W, C / d, bits, P.remap);
+    plan_rows(R, C, d, stream_label_bits(bits, G), row_mask, runs, P, balanced);
+    plan_counts(tags, R, W, bits, balanced ? P.remap.data() : nullptr, G, row_book, P);
+    plan_places(R, P);
+}
+
+void stream_balance_host(const uint32_t* tags, int R, int W, int C, int d, int bits, uint16_t* remap_out, int G,
+                         const uint8_t* row_book) {
+    std::vector<uint16_t> remap;
+    balance_codewords(tags, R, W, C / d, bits, remap, G, row_book);
+    memcpy(remap_out, remap.data(), remap.size() * sizeof(uint16_t));
+}
+
+size_t stream_bytes_host(const uint32_t* tags, int R, int W, int C, int d, int bits, const uint8_t* row_mask, int runs,
+                         const uint16_t* table, int G, const uint8_t* row_book) {
+    StreamPlan P;
+    plan_stream(tags, R, W, C, d, bits, row_mask, runs, P, table != nullptr, G, row_book);
+    return P.g.off_steps + (size_t)P.g.total_steps * P.g.fmt.step_bytes;
+}
+
+// The lanes of a wave that one clock of a 16-byte LDS read serves.  A ds_read_b128 takes four clocks; measured on
+// gfx950 (two lanes reading different rows of one bank group while every other lane reads a third address: one extra
+// clock exactly for the pairs listed together here; 256 random address patterns then fit "sum over the four sets of
+// the most distinct addresses in one group of four banks" to within 1 percent), the sets are not 16 consecutive lanes:
+static const int LDS_CLOCK_LANES[4][16] = {
+    {0, 1, 2, 3, 12, 13, 14, 15, 20, 21, 22, 23, 24, 25, 26, 27},
+    {4, 5, 6, 7, 8, 9, 10, 11, 16, 17, 18, 19, 28, 29, 30, 31},
+    {32, 33, 34, 35, 44, 45, 46, 47, 52, 53, 54, 55, 56, 57, 58, 59},
+    {36, 37, 38, 39, 40, 41, 42, 43, 48, 49, 50, 51, 60, 61, 62, 63}};
+
+// Orders the entries of the 16 lanes of one LDS clock (see the second pass of stream_build_host): every entry slot
+// should hold, over the 16 lanes, 16 different codeword bank groups (tag mod 16) and 16 different bank groups of x
+// (chunk mod 16).  A greedy fill (each lane takes the entry that collides least with the lanes before it) followed by
+// hill climbing over the whole group: a lane that collides in a slot swaps that entry with one of its other slots when
+// the two slots together get cheaper.
+struct BankMatch {
+    static constexpr uint32_t NONE = 0xFFFFFFFFu;
+    std::vector<uint32_t> ent[16];           // [lane][slot]: the lane's real entries in slot order
+    std::vector<uint8_t> ha, hb;             // [slot][16]: lanes per codeword / x bank group
+    std::vector<uint8_t> mx;                 // [slot][4]: fullest codeword group, groups that full; the same for x
+    uint32_t cnt[16];
+    uint32_t eps = 4;                        // entries per lane and step (StreamFmt.eps)
+
+    // entry n of a lane in a group whose steps begin at base: entries are kept one per word, [step][lane][eps], until
+    // they are moved to their places
+    uint32_t* rec_of(uint32_t* base, int lane, uint32_t n) const { return base + ((size_t)(n / eps) * 64 + lane) * eps + n % eps; }
+    static int ga(uint32_t e) { return (int)(e & 15u); }
+    static int gb(uint32_t e) { return (int)((e >> STREAM_SLICE_BITS) & 15u); }
+    void add(uint32_t n, uint32_t e, int d) { ha[n * 16 + ga(e)] += d; hb[n * 16 + gb(e)] += d; }
+
+    // zero_chunk: the first of the 16 chunks of x that the kernel keeps at zero
+    void order_lanes(uint32_t* base, const uint32_t* sl, const int* lanes, uint32_t ns, uint32_t zero_chunk) {
+        uint32_t most = 0;
+        for (int l = 0; l < 16; ++l) {
+            const uint32_t s0 = sl[lanes[l]];
+            cnt[l] = (s0 & STREAM_NO_ROW) == STREAM_NO_ROW ? 0u : s0 >> STREAM_ROW_BITS;
+            ent[l].resize(cnt[l]);
+            for (uint32_t n = 0; n < cnt[l]; ++n) ent[l][n] = *rec_of(base, lanes[l], n);
+            most = std::max(most, cnt[l]);
+        }
+        if (most == 0) return;
+        ha.assign((size_t)ns * 16, 0);
+        hb.assign((size_t)ns * 16, 0);
+        // greedy fill, slot by slot; the lanes with the fewest entries left choose first
+        int order[16];
+        for (int l = 0; l < 16; ++l) order[l] = l;
+        std::sort(order, order + 16, [this](int x, int y) { return cnt[x] != cnt[y] ? cnt[x] < cnt[y] : x < y; });
+        for (uint32_t n = 0; n < most; ++n)
+            for (int d = 0; d < 16; ++d) {
+                const int l = order[d];
+                if (cnt[l] <= n) continue;
+                uint32_t bi = n;
+                int bc = 1 << 30;
+                for (uint32_t i = n; i < cnt[l]; ++i) {
+                    const int c = ha[n * 16 + ga(ent[l][i])] + hb[n * 16 + gb(ent[l][i])];
+                    if (c < bc) { bc = c; bi = i; if (c == 0) break; }
+                }
+                std::swap(ent[l][n], ent[l][bi]);
+                add(n, ent[l][n], 1);
+            }
+        // Hill climbing.  What a slot costs is the fullest bank group of its codeword reads plus that of its x reads
+        // (clocks); with 16 lanes on 16 bank groups some collisions are forced, and they are cheapest when they share
+        // slots.  A lane in a fullest group swaps that entry with one of its other slots when the clocks of the two
+        // slots together go down (ties: when the sum of squared group counts does).  The fullest group's count after
+        // moving one lane from group p to group q follows from the count, the current maximum and how many groups hold
+        // it, so a candidate costs a few operations.
+        mx.assign((size_t)most * 4, 0);
+        auto rescan = [&](uint32_t n) {
+            uint8_t* m4 = &mx[n * 4];
+            m4[0] = m4[1] = m4[2] = m4[3] = 0;
+            for (int k = 0; k < 16; ++k) {
+                const uint8_t a = ha[n * 16 + k], b = hb[n * 16 + k];
+                if (a > m4[0]) { m4[0] = a; m4[1] = 1; } else if (a == m4[0]) ++m4[1];
+                if (b > m4[2]) { m4[2] = b; m4[3] = 1; } else if (b == m4[2]) ++m4[3];
+            }
+        };
+        // fullest count of histogram h (maximum M held by `at` groups) once a lane leaves group p and joins group q
+        auto moved = [](const uint8_t* h, int M, int at, int p, int q) {
+            if (p == q) return M;
+            if (h[q] + 1 > M) return h[q] + 1;
+            return (h[p] == M && at == 1 && h[q] + 1 < M) ? M - 1 : M;
+        };
+        for (uint32_t n = 0; n < most; ++n) rescan(n);
+        for (int pass = 0; pass < STREAM_CLIMB; ++pass) {
+            bool improved = false;
+            for (uint32_t n = 0; n < most; ++n) {
+                const uint8_t* an = &ha[n * 16];
+                const uint8_t* bn = &hb[n * 16];
+                const uint8_t* xn = &mx[n * 4];
+                if (xn[0] + xn[2] <= 2) continue;
+                for (int l = 0; l < 16; ++l) {
+                    if (cnt[l] <= n) continue;
+                    const uint32_t e = ent[l][n];
+                    const int ae = ga(e), be = gb(e);
+                    if (!((an[ae] == xn[0] && xn[0] > 1) || (bn[be] == xn[2] && xn[2] > 1))) continue;
+                    int best = 0;
+                    uint32_t bm = n;
+                    for (uint32_t m = 0; m < cnt[l]; ++m) {
+                        if (m == n) continue;
+                        const uint32_t f = ent[l][m];
+                        const int af = ga(f), bf = gb(f);
+                        const uint8_t* am = &ha[m * 16];
+                        const uint8_t* bq = &hb[m * 16];
+                        const uint8_t* xm = &mx[m * 4];
+                        const int clocks = moved(an, xn[0], xn[1], ae, af) + moved(bn, xn[2], xn[3], be, bf) +
+                                           moved(am, xm[0], xm[1], af, ae) + moved(bq, xm[2], xm[3], bf, be) -
+                                           (xn[0] + xn[2] + xm[0] + xm[2]);
+                        if (clocks > 0) continue;
+                        int sq = 0;
+                        if (af != ae) sq += 4 + 2 * ((int)an[af] - an[ae] + am[ae] - am[af]);
+                        if (bf != be) sq += 4 + 2 * ((int)bn[bf] - bn[be] + bq[be] - bq[bf]);
+                        const int delta = clocks * 1024 + sq;
+                        if (delta < best) { best = delta; bm = m; }
+                    }
+                    if (bm != n) {
+                        const uint32_t f = ent[l][bm];
+                        add(n, e, -1); add(bm, f, -1); add(n, f, 1); add(bm, e, 1);
+                        std::swap(ent[l][n], ent[l][bm]);
+                        rescan(n);
+                        rescan(bm);
+                        improved = true;
+                        if (xn[0] + xn[2] <= 2) break;
+                    }
+                }
+            }
+            if (!improved) break;
+        }
+        // Write the slots back.  A lane that has run out repeats one of its own codewords (from the least used bank
+        // group) against one of the 16 chunks of x that are kept at zero (one per bank group).  A lane without a row,
+        // or whose row has no entry here, reads what a neighbour reads (the same addresses are one broadcast read); the
+        // kernel drops its sum.
+        for (uint32_t n = 0; n < ns; ++n) {
+            uint32_t chosen[16];
+            int donor = -1;
+            for (int l = 0; l < 16; ++l)
+                if (cnt[l] > n) { chosen[l] = ent[l][n]; if (donor < 0) donor = l; }
+            for (int l = 0; l < 16; ++l) {
+                if (cnt[l] > n || cnt[l] == 0) continue;
+                uint32_t bi = 0;
+                for (uint32_t i = 1; i < cnt[l]; ++i)
+                    if (ha[n * 16 + ga(ent[l][i])] < ha[n * 16 + ga(ent[l][bi])]) bi = i;
+                int kb = 0;
+                for (int k = 1; k < 16; ++k)
+                    if (hb[n * 16 + k] < hb[n * 16 + kb]) kb = k;
+                chosen[l] = (ent[l][bi] & ((1u << STREAM_SLICE_BITS) - 1u)) | ((uint32_t)(zero_chunk + kb) << STREAM_SLICE_BITS);
+                add(n, chosen[l], 1);
+                if (donor < 0) donor = l;
+            }
+            for (int l = 0; l < 16; ++l) {
+                if (cnt[l] == 0) chosen[l] = donor >= 0 ? chosen[donor] : 0u;
+                *rec_of(base, lanes[l], n) = chosen[l];
+            }
+        }
+    }
+};
+
+// One step of 64 lanes x eps entries (one per word) into its bytes: 3 bytes per entry (wide), or the three 21-bit
+// entries of a lane in one 64-bit word (narrow).
+static void encode_step(const uint32_t* e, const StreamFmt& f, unsigned char* out) {
+    for (int lane = 0; lane < 64; ++lane) {
+        const uint32_t* r = e + (size_t)lane * f.eps;
+        unsigned char* o = out + (size_t)lane * f.lane_bytes;
+        if (f.narrow) {
+            const uint64_t w = (uint64_t)r[0] | (uint64_t)r[1] << 21 | (uint64_t)r[2] << 42;
+            for (int b = 0; b < 8; ++b) o[b] = (unsigned char)(w >> (8 * b));
+        } else {
+            for (int k = 0; k < 4; ++k) { o[3 * k] = (unsigned char)r[k]; o[3 * k + 1] = (unsigned char)(r[k] >> 8); o[3 * k + 2] = (unsigned char)(r[k] >> 16); }
+        }
+    }
+}
+
+int stream_build_host(const uint32_t* tags, int R, int W, int C, int d, int bits, const uint8_t* row_mask, int runs,
+                      unsigned char* out, size_t bytes, int* runs_out, int* groups_out, const uint16_t* table, int G,
+                      const uint8_t* row_book) {
+    StreamPlan P;
+    plan_stream(tags, R, W, C, d, bits, row_mask, runs, P, table != nullptr, G, row_book);
+    const uint16_t* remap = table ? P.remap.data() : nullptr;
+    const StreamGeom& g = P.g;
+    const StreamFmt f = g.fmt;
+    const uint32_t EPS = (uint32_t)f.eps, PF = (uint32_t)f.pf, FS = (uint32_t)g.fs;
+    const size_t need = g.off_steps + (size_t)g.total_steps * f.step_bytes;
+    if (g.total_steps >= ((uint64_t)1 << 32) || g.runs >= (1 << 16)) return fail(SQ_EUNSUPPORTED, "sq_stream_build: matrix too large");
+    if (bytes < need) return fail(SQ_EINVAL, "sq_stream_build: buffer %zu < %zu", bytes, need);
+    memset(out, 0, need);
+    memcpy(out, P.head4.data(), P.head4.size() * 4);
+    memcpy(out + g.off_runs, P.runs.data(), P.runs.size() * sizeof(StreamRun));
+    memcpy(out + g.off_rows, P.base.data(), P.base.size() * 4);
+    if (table) {
+        uint16_t* tab = (uint16_t*)(out + g.off_table);
+        uint16_t* unmap = (uint16_t*)(out + g.off_unmap);
+        for (int k = 0; k < (1 << bits); ++k) {
+            memcpy(tab + (size_t)remap[k] * d, table + (size_t)k * d, (size_t)d * 2);
+            unmap[remap[k]] = (uint16_t)k;
+        }
+    }
+    plan_slots(R, P);
+    uint32_t* slots = P.slot32.data();
+    // the steps are made group after group (P.goff), one entry per word, and moved to their places at the end
+    std::vector<uint32_t> laid((size_t)P.logical_steps * 64 * EPS, 0);
+    uint32_t* steps = laid.data();
+    auto rec = [&](size_t step0, uint32_t lane, uint32_t n) { return steps + ((step0 + n / EPS) * 64 + lane) * EPS + n % EPS; };
+    parallel_blocks(R, 64, [&](int a, int b) {
+        std::vector<uint32_t> q(g.NV), last(g.NV);
+        for (int r = a; r < b; ++r) {
+            const uint32_t* row = tags + (size_t)r * W;
+            const uint32_t book = row_book ? (uint32_t)(row_book[r] & (G - 1)) << bits : 0u;
+            std::fill(q.begin(), q.end(), 0u);
+            std::fill(last.begin(), last.end(), 0u);
+            for (int j = 0; j < g.U; ++j) {
+                uint32_t t = host_tag(row, W, bits, j);
+                if (remap) t = remap[t];
+                t |= book;
+                const int kp = j / g.PC, v = kp * g.NS + (int)(t >> STREAM_SLICE_BITS);
+                const uint32_t k = P.pos[(size_t)v * R + r], n = q[v]++;
+                const uint32_t e = (t & ((1u << STREAM_SLICE_BITS) - 1u)) | ((uint32_t)(j - kp * g.PC) << STREAM_SLICE_BITS);
+                *rec(P.goff[(size_t)v * g.NG + (k >> 6)], k & 63, n) = e;
+                last[v] = e & ((1u << STREAM_SLICE_BITS) - 1u);
+            }
+            // Padding up to the group's longest row: the row's last codeword of the bucket again, at the chunk of x
+            // that the kernel keeps at zero, so padding adds exactly nothing and needs no test in the inner loop
+            // (a codeword that is not finite is already part of the row's sum; a row without entries in the
+            // bucket is dropped by its slot).
+            for (int v = 0; v < g.NV; ++v) {
+                const uint32_t k = P.pos[(size_t)v * R + r];
+                const size_t gi = (size_t)v * g.NG + (k >> 6);
+                const uint32_t cap = (P.goff[gi + 1] - P.goff[gi]) * EPS;
+                const uint32_t e = last[v] | ((uint32_t)g.PC << STREAM_SLICE_BITS);
+                for (uint32_t n = q[v]; n < cap; ++n) *rec(P.goff[gi], k & 63, n) = e;
+            }
+        }
+    });
+    // Second pass, group by group: the order of a lane's entries is free (padding stays behind them), so it is
+    // chosen to keep the LDS gathers apart.  A 16-byte LDS read of a wave takes four clocks of 16 lanes each
+    // (LDS_CLOCK_LANES), and two lanes of a clock collide when their addresses differ but fall into the same group
+    // of four banks (address / 16 mod 16): BankMatch arranges the entries of each clock's lanes.
+    parallel_blocks(g.NV * g.NG, 4, [&](int a, int b) {
+        BankMatch bm;
+        bm.eps = EPS;
+        for (int vg = a; vg < b; ++vg) {
+            const uint32_t st0 = P.goff[vg], ns = (P.goff[vg + 1] - st0) * EPS;
+            if (ns == 0) continue;
+            const uint32_t* sl = slots + (size_t)vg * 64;
+            uint32_t* base = steps + (size_t)st0 * 64 * EPS;
+            for (int q = 0; q < 4; ++q) bm.order_lanes(base, sl, LDS_CLOCK_LANES[q], ns, (uint32_t)g.PC);
+        }
+    });
+    // to their places: the first FS steps of every unit into the first-steps region, the rest behind each other
+    encode_slots(P, (uint16_t*)(out + g.off_slots));
+    parallel_blocks(g.NV * g.NG, 64, [&](int a, int b) {
+        for (int vg = a; vg < b; ++vg) {
+            const uint32_t* h = &P.head4[(size_t)vg * 4];
+            const int v = vg / g.NG, nst = (int)h[1], split = (int)(h[3] & 0xFFu);
+            const uint32_t* src = steps + (size_t)P.goff[vg] * 64 * EPS;
+            for (int j = 0; j < split; ++j) {
+                const int s0 = nst * j / split, s1 = nst * (j + 1) / split;
+                for (int t = s0; t < s1; ++t) {
+                    const uint64_t to = (uint32_t)(t - s0) < PF ? ((uint64_t)(h[2] + j) * g.NV + v) * FS + (t - s0)
+                                                                 : (uint64_t)h[0] + t - (uint64_t)PF * (j + 1);
+                    encode_step(src + (size_t)t * 64 * EPS, f, out + g.off_steps + to * f.step_bytes);
+                }
+            }
+        }
+    });
+    if (runs_out) *runs_out = runs_word(P) | (table ? STREAM_BALANCED : 0);
+    if (groups_out) *groups_out = g.NG;
+    return SQ_OK;
+}
+
+
+// ------------------------------------------------------------------------------------------ on the GPU
+//
+// The same buffer, byte for byte, from tags that are already in device memory.  What is serial and small stays on the host
+// (the rows' order and runs, the sort of the rows of a run by entry count, the places); what walks the tags runs here:
+// counting, collecting every lane's entries, ordering them for the LDS banks, encoding.  The ordering is what the host
+// spends its time on (16 cores: 150 ms for 18944 x 3584, 2.5 s for 3584 x 18944 on one).  Whole load of a matrix, tags on
+// the GPU to stream on the GPU, before / now: 3584 x 3584 363 / 2.7 ms, 18944 x 3584 155 / 6.0, 3584 x 18944 2525 / 12.9.
+
+// count[book << bits | label] += 1 for every tag (one wave per row)
+__global__ __launch_bounds__(256) void stream_codeword_count_kernel(const uint32_t* __restrict__ tags, int R, int W, int U, int bits,
+                                                                    const uint8_t* __restrict__ row_book, uint32_t* __restrict__ count) {
+    const int r = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    if (r >= R) return;
+    const uint32_t* row = tags + (int64_t)r * W;
+    const uint32_t book = row_book ? (uint32_t)row_book[r] << bits : 0u;
+    for (int j = lane; j < U; j += 64) atomicAdd(count + (book | tag_at(row, W, bits, j)), 1u);
+}
+
+__global__ __launch_bounds__(256) void stream_clear_kernel(uint32_t* __restrict__ p, int64_t n) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) p[i] = 0u;
+}
+
+// rewrites the tags of a matrix through remap[book << bits | label] in place; a thread owns 32 tags, which are whole words
+__global__ __launch_bounds__(256) void stream_relabel_kernel(uint32_t* __restrict__ tags, int R, int W, int U, int bits,
+                                                             const uint8_t* __restrict__ row_book, const uint16_t* __restrict__ remap) {
+    const int units = (U + 31) / 32;
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (int64_t)R * units) return;
+    const int r = (int)(i / units), u = (int)(i - (int64_t)r * units);
+    uint32_t* w = tags + (int64_t)r * W + u * bits;
+    const int nw = min(bits, W - u * bits), n = min(32, U - u * 32);
+    const uint16_t* map = remap + ((row_book ? (size_t)row_book[r] : 0) << bits);
+    const uint32_t mask = (1u << bits) - 1u;
+    uint64_t in = 0, out = 0;
+    int have = 0, held = 0, rd = 0, wr = 0;
+    for (int k = 0; k < n; ++k) {
+        if (have < bits) { in |= (uint64_t)(rd < nw ? w[rd] : 0u) << have; ++rd; have += 32; }
+        out |= (uint64_t)map[(uint32_t)in & mask] << held;
+        in >>= bits; have -= bits; held += bits;
+        if (held >= 32) { w[wr++] = (uint32_t)out; out >>= 32; held -= 32; }
+    }
+    // the bits behind a row's last tag are zero, as pack_bits leaves them
+    if (held > 0) w[wr++] = (uint32_t)out;
+}
+
+// cnt[v * R + r]: entries of row r in bucket v (one wave per row; its counters in LDS)
+__global__ __launch_bounds__(64) void stream_count_kernel(const uint32_t* __restrict__ tags, int R, int W, int U, int bits, int PC, int NS, int NV,
+                                                          const uint8_t* __restrict__ row_book, uint16_t* __restrict__ cnt) {
+    extern __shared__ uint32_t stream_count_lds[];
+    const int r = (int)blockIdx.x, lane = (int)threadIdx.x;
+    for (int v = lane; v < NV; v += 64) stream_count_lds[v] = 0u;
+    __syncthreads();
+    const uint32_t* row = tags + (int64_t)r * W;
+    const uint32_t book = row_book ? (uint32_t)row_book[r] << bits : 0u;
+    for (int j = lane; j < U; j += 64)
+        atomicAdd(&stream_count_lds[(j / PC) * NS + (int)((book | tag_at(row, W, bits, j)) >> STREAM_SLICE_BITS)], 1u);
+    __syncthreads();
+    for (int v = lane; v < NV; v += 64) cnt[(int64_t)v * R + r] = (uint16_t)stream_count_lds[v];
+}
+
+struct StreamFillArgs {
+    const uint32_t* tags;
+    const uint8_t* row_book;
+    const uint32_t* heads;      // [NV * NG][4], in the stream buffer
+    const uint32_t* rows;       // [NV * NG * 64]: the row of every lane (STREAM_NO_ROW: none)
+    const uint32_t* goff;       // [NV * NG + 1]: the groups' steps counted one behind the other
+    unsigned char* steps;       // the stream buffer's steps
+    unsigned char* work;        // groups that LDS does not hold: STREAM_FILL_BYTES per entry slot of every group
+    int W, U, bits, PC, NS, NV, NG, fs;
+};
+
+// Bytes one entry slot (64 lanes) of a group takes: 65 words of entries (the odd pitch spreads one lane's entries over the
+// banks), 16 + 16 bank-group counts for each of the four clocks, and their maxima.
+constexpr int STREAM_FILL_BYTES = 65 * 4 + 4 * 32 + 4 * 4;
+constexpr int STREAM_FILL_LDS = 156 * 1024;
+
+__constant__ uint8_t STREAM_CLOCK_LANES_DEV[4][16] = {
+    {0, 1, 2, 3, 12, 13, 14, 15, 20, 21, 22, 23, 24, 25, 26, 27},
+    {4, 5, 6, 7, 8, 9, 10, 11, 16, 17, 18, 19, 28, 29, 30, 31},
+    {32, 33, 34, 35, 44, 45, 46, 47, 52, 53, 54, 55, 56, 57, 58, 59},
+    {36, 37, 38, 39, 40, 41, 42, 43, 48, 49, 50, 51, 60, 61, 62, 63}};
+
+// over the 16 threads of a DPP row: four rotations of a few cycles each; and over the wave, the four rows' results as scalars
+template <int N> __device__ __forceinline__ int row_ror(int v) { return __builtin_amdgcn_update_dpp(v, v, 0x120 + N, 0xF, 0xF, false); }
+__device__ __forceinline__ int min16(int v) {
+    v = min(v, row_ror<8>(v)); v = min(v, row_ror<4>(v)); v = min(v, row_ror<2>(v));
+    return min(v, row_ror<1>(v));
+}
+__device__ __forceinline__ int max16(int v) {
+    v = max(v, row_ror<8>(v)); v = max(v, row_ror<4>(v)); v = max(v, row_ror<2>(v));
+    return max(v, row_ror<1>(v));
+}
+__device__ __forceinline__ int add16(int v) {
+    v += row_ror<8>(v); v += row_ror<4>(v); v += row_ror<2>(v);
+    return v + row_ror<1>(v);
+}
+__device__ __forceinline__ int min64(int v) {
+    v = min16(v);
+    return min(min(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+               min(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+}
+__device__ __forceinline__ int stream_ga(uint32_t e) { return (int)(e & 15u); }
+__device__ __forceinline__ int stream_gb(uint32_t e) { return (int)((e >> STREAM_SLICE_BITS) & 15u); }
+// fullest group of a histogram (maximum M, held by `at` groups) once a lane leaves a group of hp and joins another of hq
+__device__ __forceinline__ int stream_moved(int hp, int hq, int M, int at, bool same) {
+    if (same) return M;
+    return hq + 1 > M ? hq + 1 : (hp == M && at == 1 && hq + 1 < M) ? M - 1 : M;
+}
+
+// One workgroup per (bucket, group), one wave per clock of the group: it collects its 16 rows' entries (four threads per
+// row), orders them (the steps of BankMatch::order_lanes with ties resolved the same way; the 64 threads search a lane's
+// candidates together), and the four waves write the encoded steps to their places.  The search is a serial chain of
+// LDS reads, so what counts is its length: with the four clocks on one wave, 16 threads each, their branches took turns
+// (3584 x 18944: 49 ms against 10; 3584 x 3584: 1.7 against 0.8).
+template <bool LDS>
+__global__ __launch_bounds__(256) void stream_fill_kernel(StreamFillArgs a) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char stream_fill_lds[];
+    const int vg = (int)blockIdx.x, v = vg / a.NG, q = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), t = (int)threadIdx.x & 63, sub = t & 15;
+    const StreamFmt f = stream_fmt(a.PC);
+    const int nst = (int)a.heads[(size_t)vg * 4 + 1], ns = nst * f.eps;
+    if (ns == 0) return;
+    unsigned char* mem = LDS ? stream_fill_lds : a.work + (size_t)a.goff[vg] * f.eps * STREAM_FILL_BYTES;
+    uint32_t* ent = reinterpret_cast<uint32_t*>(mem);                        // [slot][65]
+    uint8_t* h = mem + (size_t)ns * (260 + 32 * q);                          // this clock's [slot][32]: codeword groups, x groups
+    uint8_t* mx = mem + (size_t)ns * (260 + 128 + 4 * q);                    // and [slot][4]: their maxima
+
+    // entries of the clock's rows in this bucket, in chunk order: thread t counts, then writes a quarter of row t / 4
+    const int crow = STREAM_CLOCK_LANES_DEV[q][t >> 2];
+    const uint32_t row_id = a.rows[(size_t)vg * 64 + crow];
+    int total = 0;
+    if (row_id != STREAM_NO_ROW) {
+        const uint32_t* row = a.tags + (int64_t)row_id * a.W;
+        const uint32_t book = a.row_book ? (uint32_t)a.row_book[row_id] << a.bits : 0u;
+        const int kp = v / a.NS, sl = v - kp * a.NS, p0 = kp * a.PC, len = min(a.PC, a.U - p0);
+        const int j0 = p0 + len * (t & 3) / 4, j1 = p0 + len * ((t & 3) + 1) / 4;
+        int n = 0;
+        for (int j = j0; j < j1; ++j) n += (int)((book | tag_at(row, a.W, a.bits, j)) >> STREAM_SLICE_BITS) == sl;
+        int before = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int c = __shfl(n, (t & ~3) + k, 64);
+            before += k < (t & 3) ? c : 0;
+            total += c;
+        }
+        for (int j = j0; j < j1; ++j) {
+            const uint32_t g = book | tag_at(row, a.W, a.bits, j);
+            if ((int)(g >> STREAM_SLICE_BITS) == sl && before < ns) {
+                ent[before * 65 + crow] = (g & ((1u << STREAM_SLICE_BITS) - 1u)) | ((uint32_t)(j - p0) << STREAM_SLICE_BITS);
+                ++before;
+            }
+        }
+    }
+    for (int i = t; i < ns * 8; i += 64) reinterpret_cast<uint32_t*>(h)[i] = 0u;
+    __syncthreads();
+
+    const int cnt = __shfl(total, sub * 4, 64), my_lane = STREAM_CLOCK_LANES_DEV[q][sub];   // thread `sub`: its lane of this clock
+    const bool has_row = __shfl((int)(row_id != STREAM_NO_ROW), sub * 4, 64) != 0;
+    const int packed = cnt << 6 | my_lane;
+    auto packed_of = [&](int l) { return __builtin_amdgcn_readlane(packed, l); };
+    const int most = __builtin_amdgcn_readfirstlane(max16(cnt));
+    // greedy fill: the lanes with the fewest entries choose first
+    int rank = 0;
+    for (int l = 0; l < 16; ++l) {
+        const int c = packed_of(l) >> 6;
+        rank += c < cnt || (c == cnt && l < sub);
+    }
+    int at_rank = 0;                                                         // thread d: the lane of rank d
+    for (int l = 0; l < 16; ++l)
+        if (__builtin_amdgcn_readlane(rank, l) == sub) at_rank = l;
+    const int ranked = __shfl(packed, at_rank, 64);
+    for (int n = 0; n < most; ++n)
+        for (int d = 0; d < 16; ++d) {
+            const int pk = __builtin_amdgcn_readlane(ranked, d), cl = pk >> 6, ln = pk & 63;
+            if (cl <= n) continue;
+            int key = 0x7FFFFFFF;                                            // cost << 16 | slot: the first cheapest
+            for (int i = n + t; i < cl; i += 64) {
+                const uint32_t e = ent[i * 65 + ln];
+                key = min(key, ((int)h[n * 32 + stream_ga(e)] + (int)h[n * 32 + 16 + stream_gb(e)]) << 16 | i);
+            }
+            const int bi = min64(key) & 0xFFFF;
+            const uint32_t en = ent[n * 65 + ln], eb = ent[bi * 65 + ln];
+            if (t == 0) {
+                ent[n * 65 + ln] = eb;
+                ent[bi * 65 + ln] = en;
+                ++h[n * 32 + stream_ga(eb)];
+                ++h[n * 32 + 16 + stream_gb(eb)];
+            }
+            __threadfence_block();
+        }
+    auto rescan = [&](int n) {
+        const int ca = h[n * 32 + sub], cb = h[n * 32 + 16 + sub];
+        const int ma = max16(ca), mb = max16(cb);
+        const int na = add16(ma > 0 && ca == ma), nb = add16(mb > 0 && cb == mb);
+        if (t == 0) *reinterpret_cast<uint32_t*>(mx + n * 4) = (uint32_t)ma | (uint32_t)na << 8 | (uint32_t)mb << 16 | (uint32_t)nb << 24;
+    };
+    for (int n = 0; n < most; ++n) rescan(n);
+    __threadfence_block();
+    for (int pass = 0; pass < STREAM_CLIMB; ++pass)
+        for (int n = 0; n < most; ++n) {
+            const uint8_t* an = h + n * 32;
+            const uint8_t* bn = an + 16;
+            uint32_t xw = *reinterpret_cast<const uint32_t*>(mx + n * 4);    // maximum and how many groups hold it, twice
+            xw = (uint32_t)__builtin_amdgcn_readfirstlane((int)xw);
+            if ((int)(xw & 0xFF) + (int)(xw >> 16 & 0xFF) <= 2) continue;
+            for (int l = 0; l < 16; ++l) {
+                const int pk = packed_of(l), cl = pk >> 6, ln = pk & 63;
+                if (cl <= n) continue;
+                const int x0 = (int)(xw & 0xFF), x1 = (int)(xw >> 8 & 0xFF), x2 = (int)(xw >> 16 & 0xFF), x3 = (int)(xw >> 24);
+                const uint32_t e = ent[n * 65 + ln];
+                const int ae = stream_ga(e), be = stream_gb(e), ane = an[ae], bne = bn[be];
+                if (!((ane == x0 && x0 > 1) || (bne == x2 && x2 > 1))) continue;
+                constexpr int NO_MOVE = 1 << 30;                             // (delta + 2^17) << 13 | slot, delta < 0
+                int key = NO_MOVE;
+                for (int m = t; m < cl; m += 64) {
+                    const uint32_t fm = ent[m * 65 + ln];
+                    const int af = stream_ga(fm), bf = stream_gb(fm);
+                    const uint8_t* am = h + m * 32;
+                    const uint8_t* bq = am + 16;
+                    const uint32_t xm = *reinterpret_cast<const uint32_t*>(mx + m * 4);
+                    const int y0 = (int)(xm & 0xFF), y1 = (int)(xm >> 8 & 0xFF), y2 = (int)(xm >> 16 & 0xFF), y3 = (int)(xm >> 24);
+                    const int anf = an[af], bnf = bn[bf], ame = am[ae], amf = am[af], bqe = bq[be], bqf = bq[bf];
+                    const int clocks = stream_moved(ane, anf, x0, x1, ae == af) + stream_moved(bne, bnf, x2, x3, be == bf) +
+                                       stream_moved(amf, ame, y0, y1, ae == af) + stream_moved(bqf, bqe, y2, y3, be == bf) - (x0 + x2 + y0 + y2);
+                    const int sq = (af != ae ? 4 + 2 * (anf - ane + ame - amf) : 0) + (bf != be ? 4 + 2 * (bnf - bne + bqe - bqf) : 0);
+                    const int delta = clocks * 1024 + sq;
+                    if (m != n && clocks <= 0 && delta < 0) key = min(key, (delta + (1 << 17)) << 13 | m);
+                }
+                key = min64(key);
+                if (key == NO_MOVE) continue;
+                const int bm = key & 0x1FFF;
+                const uint32_t fm = ent[bm * 65 + ln];
+                if (t == 0) {
+                    const int af = stream_ga(fm), bf = stream_gb(fm);
+                    --h[n * 32 + ae]; --h[n * 32 + 16 + be]; --h[bm * 32 + af]; --h[bm * 32 + 16 + bf];
+                    ++h[n * 32 + af]; ++h[n * 32 + 16 + bf]; ++h[bm * 32 + ae]; ++h[bm * 32 + 16 + be];
+                    ent[n * 65 + ln] = fm;
+                    ent[bm * 65 + ln] = e;
+                }
+                __threadfence_block();
+                rescan(n);
+                rescan(bm);
+                __threadfence_block();
+                xw = (uint32_t)__builtin_amdgcn_readfirstlane((int)*reinterpret_cast<const uint32_t*>(mx + n * 4));
+                if ((int)(xw & 0xFF) + (int)(xw >> 16 & 0xFF) <= 2) break;
+            }
+        }
+    // padding: a lane that has run out repeats one of its codewords (least used bank group) against a zero chunk of x; a
+    // lane without entries reads what a neighbour reads (in a clock without any entry: codeword 0 against a zero chunk)
+    for (int n = 0; n < ns; ++n) {
+        int donor = __builtin_amdgcn_readfirstlane(min16(cnt > n ? sub : 16));
+        for (int l = 0; l < 16; ++l) {
+            const int pk = packed_of(l), cl = pk >> 6, ln = pk & 63;
+            if (cl > n || cl == 0) continue;
+            int key = 0x7FFFFFFF;
+            for (int i = t; i < cl; i += 64) key = min(key, (int)h[n * 32 + stream_ga(ent[i * 65 + ln])] << 16 | i);
+            const int bi = min64(key) & 0xFFFF;
+            const int kb = min16((int)h[n * 32 + 16 + sub] << 4 | sub) & 15;
+            const uint32_t c = (ent[bi * 65 + ln] & ((1u << STREAM_SLICE_BITS) - 1u)) | ((uint32_t)(a.PC + kb) << STREAM_SLICE_BITS);
+            if (t == 0) {
+                ent[n * 65 + ln] = c;
+                ++h[n * 32 + stream_ga(c)];
+                ++h[n * 32 + 16 + stream_gb(c)];
+            }
+            __threadfence_block();
+            if (donor == 16) donor = l;
+        }
+        const int dl = packed_of(donor & 15) & 63;
+        if (cnt == 0 && t < 16) ent[n * 65 + my_lane] = donor < 16 ? ent[n * 65 + dl] : has_row ? (uint32_t)a.PC << STREAM_SLICE_BITS : 0u;
+    }
+    __syncthreads();
+
+    const uint32_t* hd = a.heads + (size_t)vg * 4;
+    const int split = (int)(hd[3] & 0xFFu);
+    for (int j = 0; j < split; ++j) {
+        const int s0 = nst * j / split, s1 = nst * (j + 1) / split;
+        for (int st = s0 + q; st < s1; st += 4) {
+            const uint64_t to = st - s0 < f.pf ? ((uint64_t)(hd[2] + j) * a.NV + v) * a.fs + (st - s0) : (uint64_t)hd[0] + st - (uint64_t)f.pf * (j + 1);
+            unsigned char* o = a.steps + to * f.step_bytes + t * f.lane_bytes;
+            const uint32_t* e = ent + st * f.eps * 65 + t;
+            if (f.narrow) {
+                const uint64_t w = (uint64_t)e[0] | (uint64_t)e[65] << 21 | (uint64_t)e[130] << 42;
+                *reinterpret_cast<u32x2*>(o) = u32x2{(uint32_t)w, (uint32_t)(w >> 32)};
+            } else {
+                const uint32_t e0 = e[0] & 0xFFFFFFu, e1 = e[65] & 0xFFFFFFu, e2 = e[130] & 0xFFFFFFu, e3 = e[195] & 0xFFFFFFu;
+                uint32_t* o4 = reinterpret_cast<uint32_t*>(o);
+                o4[0] = e0 | e1 << 24;
+                o4[1] = e1 >> 8 | e2 << 16;
+                o4[2] = e2 >> 16 | e3 << 8;
+            }
+        }
+    }
+}
+
+// the tile-major copy of the tags (tiled_build) from tags in device memory: a thread moves one unit of a row
+__global__ __launch_bounds__(256) void tiled_build_kernel(const uint32_t* __restrict__ tags, int R, int W, int ud, uint32_t* __restrict__ out) {
+    const int U = W / ud;
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;          // (tile, unit, row of the tile)
+    if (i >= (int64_t)((R + 15) / 16) * 16 * U) return;
+    const int k = (int)(i & 15);
+    const int64_t tu = i >> 4;
+    const int u = (int)(tu % U), r = (int)(tu / U) * 16 + k;
+    uint32_t* dst = out + i * ud;
+    const uint32_t* src = tags + (int64_t)r * W + u * ud;
+    for (int w = 0; w < ud; ++w) dst[w] = r < R ? src[w] : 0u;
+}
+
+int stream_balance_device(const uint32_t* tags, int R, int W, int C, int d, int bits, uint32_t* counts, uint16_t* remap_out, int G,
+                          const uint8_t* row_book, hipStream_t s) {
+    const int64_t n = (int64_t)G << bits;
+    hipLaunchKernelGGL(stream_clear_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, counts, n);
+    hipLaunchKernelGGL(stream_codeword_count_kernel, dim3((unsigned)((R + 3) / 4)), dim3(256), 0, s, tags, R, W, C / d, bits, row_book, counts);
+    int rc = check_launch("sq_codebook_balance_device");
+    if (rc) return rc;
+    std::vector<uint32_t> host((size_t)n);
+    hipError_t e = hipMemcpyAsync(host.data(), counts, (size_t)n * 4, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e != hipSuccess) return fail(SQ_ELAUNCH, "sq_codebook_balance_device: %s", hipGetErrorString(e));
+    std::vector<uint16_t> remap;
+    deal_codewords(host.data(), bits, remap, G);
+    memcpy(remap_out, remap.data(), remap.size() * sizeof(uint16_t));
+    return SQ_OK;
+}
+
+int stream_relabel_device(uint32_t* tags, int R, int W, int C, int d, int bits, const uint8_t* row_book, const uint16_t* remap, hipStream_t s) {
+    const int64_t n = (int64_t)R * ((C / d + 31) / 32);
+    if (n == 0) return SQ_OK;
+    hipLaunchKernelGGL(stream_relabel_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, tags, R, W, C / d, bits, row_book, remap);
+    return check_launch("sq_codebook_relabel_device");
+}
+
+size_t stream_counts_bytes(int R, int C, int d, int bits, int G) {
+    return (size_t)stream_geom(C, d, stream_label_bits(bits, G), 0, 0).NV * R * 2;
+}
+
+// A plan on its way from stream_plan_device to stream_fill_device.
+struct StreamDevicePlan {
+    StreamPlan P;
+    int R, W, C, d, bits, G;
+    bool tiled, in_lds;
+    size_t bytes, scratch;
+};
+
+int stream_plan_device(const uint32_t* tags, int R, int W, int C, int d, int bits, int G, const uint8_t* row_book, const uint8_t* row_mask_host,
+                       int runs, void* counts, StreamDevicePlan** out, size_t* bytes, size_t* scratch, int* runs_out, int* groups_out, hipStream_t s) {
+    std::unique_ptr<StreamDevicePlan> D(new StreamDevicePlan);
+    D->R = R; D->W = W; D->C = C; D->d = d; D->bits = bits; D->G = G;
+    D->tiled = !stream_format_ok(R, C, d, bits, G);
+    D->in_lds = false;
+    if (D->tiled) {
+        D->bytes = tiled_bytes(R, W);
+        D->scratch = 0;
+        *runs_out = *groups_out = 0;
+    } else {
+        StreamPlan& P = D->P;
+        plan_rows(R, C, d, stream_label_bits(bits, G), row_mask_host, runs, P, false);
+        const StreamGeom& g = P.g;
+        hipLaunchKernelGGL(stream_count_kernel, dim3((unsigned)R), dim3(64), (size_t)g.NV * 4, s, tags, R, W, g.U, bits, g.PC, g.NS, g.NV, row_book,
+                           (uint16_t*)counts);
+        int rc = check_launch("sq_stream_plan_device");
+        if (rc) return rc;
+        P.cnt.resize((size_t)g.NV * R);
+        hipError_t e = hipMemcpyAsync(P.cnt.data(), counts, P.cnt.size() * 2, hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        if (e != hipSuccess) return fail(SQ_ELAUNCH, "sq_stream_plan_device: %s", hipGetErrorString(e));
+        plan_places(R, P);
+        plan_slots(R, P);
+        if (g.total_steps >= ((uint64_t)1 << 32) || g.runs >= (1 << 16)) return fail(SQ_EUNSUPPORTED, "sq_stream_plan_device: matrix too large");
+        D->bytes = g.off_steps + (size_t)g.total_steps * g.fmt.step_bytes;
+        uint32_t longest = 0;
+        for (size_t k = 0; k + 1 < P.goff.size(); ++k) longest = std::max(longest, P.goff[k + 1] - P.goff[k]);
+        D->in_lds = (size_t)longest * g.fmt.eps * STREAM_FILL_BYTES <= STREAM_FILL_LDS;
+        // scratch: the rows of the lanes and the groups' offsets, and the groups themselves when one is too long for LDS
+        const size_t lists = (((size_t)g.NV * g.NG * 65 + 1) * 4 + 255) & ~(size_t)255;
+        D->scratch = lists + (D->in_lds ? 0 : (size_t)P.logical_steps * g.fmt.eps * STREAM_FILL_BYTES);
+        *runs_out = runs_word(P);
+        *groups_out = g.NG;
+    }
+    *bytes = D->bytes;
+    *scratch = D->scratch;
+    *out = D.release();
+    return SQ_OK;
+}
+
+int stream_fill_device(const StreamDevicePlan& D, const uint32_t* tags, const uint8_t* row_book, unsigned char* out, unsigned char* scratch, hipStream_t s) {
+    if (D.tiled) {
+        const int ud = D.bits == 12 ? 3 : D.bits == 10 ? 5 : 4;
+        const int64_t n = (int64_t)((D.R + 15) / 16) * 16 * (D.W / ud);
+        if (n == 0) return SQ_OK;
+        hipLaunchKernelGGL(tiled_build_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, tags, D.R, D.W, ud, (uint32_t*)out);
+        return check_launch("sq_stream_fill_device");
+    }
+    const StreamPlan& P = D.P;
+    const StreamGeom& g = P.g;
+    const size_t nvg = (size_t)g.NV * g.NG;
+    // everything before the steps is assembled on the host; the rest starts as zeros
+    std::vector<unsigned char> front(g.off_steps, 0);
+    memcpy(front.data(), P.head4.data(), P.head4.size() * 4);
+    memcpy(front.data() + g.off_runs, P.runs.data(), P.runs.size() * sizeof(StreamRun));
+    memcpy(front.data() + g.off_rows, P.base.data(), P.base.size() * 4);
+    encode_slots(P, (uint16_t*)(front.data() + g.off_slots));
+    std::vector<uint32_t> lists(nvg * 65 + 1);
+    for (size_t k = 0; k < nvg * 64; ++k) {
+        const uint32_t place = P.slot32[k] & STREAM_NO_ROW;
+        lists[k] = place == STREAM_NO_ROW ? STREAM_NO_ROW : P.base[place];
+    }
+    memcpy(lists.data() + nvg * 64, P.goff.data(), (nvg + 1) * 4);
+    hipError_t e = hipMemcpyAsync(out, front.data(), front.size(), hipMemcpyHostToDevice, s);
+    if (e == hipSuccess) e = hipMemcpyAsync(scratch, lists.data(), lists.size() * 4, hipMemcpyHostToDevice, s);
+    if (e != hipSuccess) return fail(SQ_ELAUNCH, "sq_stream_fill_device: %s", hipGetErrorString(e));
+    const int64_t words = (int64_t)((D.bytes - g.off_steps) / 4);
+    hipLaunchKernelGGL(stream_clear_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, s, (uint32_t*)(out + g.off_steps), words);
+    uint32_t longest = 0;
+    for (size_t k = 0; k < nvg; ++k) longest = std::max(longest, P.goff[k + 1] - P.goff[k]);
+    StreamFillArgs a;
+    a.tags = tags; a.row_book = row_book;
+    a.heads = (const uint32_t*)out;
+    a.rows = (const uint32_t*)scratch;
+    a.goff = a.rows + nvg * 64;
+    a.steps = out + g.off_steps;
+    a.work = scratch + ((lists.size() * 4 + 255) & ~(size_t)255);
+    a.W = D.W; a.U = g.U; a.bits = D.bits; a.PC = g.PC; a.NS = g.NS; a.NV = g.NV; a.NG = g.NG; a.fs = g.fs;
+    if (D.in_lds) {
+        const size_t lds = (size_t)longest * g.fmt.eps * STREAM_FILL_BYTES;
+        (void)hipFuncSetAttribute((const void*)stream_fill_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, STREAM_FILL_LDS);
+        (void)hipGetLastError();
+        hipLaunchKernelGGL((stream_fill_kernel<true>), dim3((unsigned)nvg), dim3(256), lds, s, a);
+    } else {
+        hipLaunchKernelGGL((stream_fill_kernel<false>), dim3((unsigned)nvg), dim3(256), 0, s, a);
+    }
+    int rc = check_launch("sq_stream_fill_device");
+    if (rc) return rc;
+    e = hipStreamSynchronize(s);                                 // the host lists are read until here
+    return e == hipSuccess ? SQ_OK : fail(SQ_ELAUNCH, "sq_stream_fill_device: %s", hipGetErrorString(e));
+}
+
+void stream_plan_free(StreamDevicePlan* D) { delete D; }
+
+}  // namespace sq

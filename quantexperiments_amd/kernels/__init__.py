@@ -155,29 +155,24 @@ class PackedLinear(torch.nn.Module):
         whatever the distribution of the tags, and the matrix keeps ONE codebook (a stream that carries its own
         relabelled copy, sq_stream_build_balanced, costs another 1.1 MiB per matrix).  With several codebooks each is
         relabelled by itself, over its own slices (sq_codebook_balance_books)."""
-        from ..packed import pack_bits, unpack_bits
-        host = self.words.detach().to("cpu", torch.int32).contiguous()
+        dev, L = self.words.device, _lib.lib()
         remap = torch.empty(self.G << self.bits, dtype=torch.int16)
-        book = None if self.row_book is None else self.row_book.detach().to("cpu", torch.uint8).contiguous()
-        rc = _lib.lib().sq_codebook_balance_books(host.data_ptr(), self.R, self.W, self.C, self.d, self.bits, self.G,
-                                                  None if book is None else book.data_ptr(), remap.data_ptr())
-        if rc == _lib.SQ_EUNSUPPORTED:                  # a shape the slice stream does not cover: nothing to balance
-            self.relabelled = True
-            return
-        _lib.check(rc)
-        new_of = (remap.to(torch.int32) & 0xFFFF).to(torch.int64)            # book * K + file label -> new label in the book
-        dev = self.words.device
-        if self.bits == 16 and self.G == 1:
-            old = (self.words.view(torch.int16).to(torch.int32) & 0xFFFF).to(torch.int64)
-            self.words = remap.to(dev)[old].view(torch.int32).reshape(self.R, self.W).contiguous()
-        else:
-            old = unpack_bits(host, self.bits, self.nch).to(torch.int64)
-            if book is not None:
-                old = old + (book.to(torch.int64) << self.bits)[:, None]
-            self.words = pack_bits(new_of[old], self.bits).to(dev)
+        counts = torch.empty(self.G << self.bits, dtype=torch.int32, device=dev)
+        args = (self.R, self.W, self.C, self.d, self.bits, self.G, None if self.row_book is None else self.row_book.data_ptr())
+        with torch.cuda.device(dev):
+            rc = L.sq_codebook_balance_device(self.words.data_ptr(), *args, counts.data_ptr(), remap.data_ptr(), _lib.stream_ptr(dev))
+            if rc == _lib.SQ_EUNSUPPORTED:              # a shape the slice stream does not cover: nothing to balance
+                self.relabelled = True
+                return
+            _lib.check(rc)
+            remap = remap.to(dev)
+            self.words = self.words.clone()             # (the caller's tensor keeps the file's labels)
+            _lib.check(L.sq_codebook_relabel_device(self.words.data_ptr(), *args, remap.data_ptr(), _lib.stream_ptr(dev)))
+        # row of the table a codeword moves to: book << bits | new label
+        at = torch.arange(self.G << self.bits, device=dev)
+        at = (at & -(1 << self.bits)) + (remap.to(torch.int64) & 0xFFFF)
         table = torch.empty_like(self.table)
-        at = new_of + ((torch.arange(self.G << self.bits) >> self.bits) << self.bits)      # row of the table a codeword moves to
-        table[at.to(dev)] = self.table
+        table[at] = self.table
         self.table = table
         self.relabelled = True
 
@@ -270,6 +265,8 @@ def build_stream(words: torch.Tensor, C: int, d: int, bits: int, row_mask=None, 
     below a power of two G = its maximum rounded up; or a (row_book, G) pair): the matrix has G codebooks behind each
     other in its table (sq_stream_build_books; not together with `table`)."""
     L = _lib.lib()
+    if words.is_cuda and table is None:
+        return _build_stream_device(words, C, d, bits, row_mask, runs, row_book)
     host = words.detach().to("cpu", torch.int32).contiguous()
     mask = None if row_mask is None else row_mask.detach().to("cpu", torch.uint8).contiguous()
     mp = None if mask is None else mask.data_ptr()
@@ -300,6 +297,42 @@ def build_stream(words: torch.Tensor, C: int, d: int, bits: int, row_mask=None, 
     _lib.check(L.sq_stream_build_balanced(host.data_ptr(), R, W, C, d, bits, mp, runs, tp, out.data_ptr(), n, ctypes.byref(r),
                                           ctypes.byref(g)))
     return out.to(words.device), r.value, g.value
+
+
+def _build_stream_device(words: torch.Tensor, C: int, d: int, bits: int, row_mask, runs: int, row_book):
+    """build_stream for tags on the GPU: the library plans on the host from counts taken there and writes the buffer on the
+    GPU (sq_stream_plan_device, sq_stream_fill_device); the tags never leave the device."""
+    L, dev = _lib.lib(), words.device
+    words = words.detach().to(torch.int32).contiguous()
+    mask = None if row_mask is None else row_mask.detach().to("cpu", torch.uint8).contiguous()
+    R, W = words.shape
+    book, G = None, 1
+    if row_book is not None:
+        book, G = row_book if isinstance(row_book, tuple) else (row_book, None)
+        book = book.detach().to(dev, torch.uint8).contiguous()
+        top = int(book.max()) if R else 0
+        if G is None:
+            G = 1 << top.bit_length()
+        if top >= G:
+            raise ValueError(f"row_book names codebook {top} of {G}")
+    new = lambda n: torch.empty(max(n, 1), dtype=torch.uint8, device=dev)
+    counts = new(L.sq_stream_counts_bytes(R, C, d, bits, G))
+    plan, nbytes, nscratch = ctypes.c_void_p(), ctypes.c_size_t(), ctypes.c_size_t()
+    r, g = ctypes.c_int32(), ctypes.c_int32()
+    bp = None if book is None else book.data_ptr()
+    with torch.cuda.device(dev):
+        rc = L.sq_stream_plan_device(words.data_ptr(), R, W, C, d, bits, G, bp, None if mask is None else mask.data_ptr(), runs,
+                                     counts.data_ptr(), ctypes.byref(plan), ctypes.byref(nbytes), ctypes.byref(nscratch), ctypes.byref(r),
+                                     ctypes.byref(g), _lib.stream_ptr(dev))
+        if rc in (_lib.SQ_EUNSUPPORTED, _lib.SQ_EINVAL):          # a format the load-time layouts do not cover
+            return None, 0, 0
+        _lib.check(rc)
+        try:
+            out, scratch = new(nbytes.value), new(nscratch.value)
+            _lib.check(L.sq_stream_fill_device(plan, words.data_ptr(), bp, out.data_ptr(), scratch.data_ptr(), _lib.stream_ptr(dev)))
+        finally:
+            L.sq_stream_plan_free(plan)
+    return out, r.value, g.value
 
 
 STREAM_PART_MAX = 4064      # chunks per column part of the tag stream (sq_stream.h)

@@ -1,0 +1,59 @@
+"""The load-time layouts built on the GPU are the host builder's, byte for byte, and so is the relabelling."""
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from quantexperiments_amd import _lib
+from quantexperiments_amd.kernels import build_stream
+from quantexperiments_amd.packed import pack_bits
+
+pytestmark = pytest.mark.gpu
+
+# R, C, d, bits, G, M, runs, tags
+CASES = [(1, 64, 8, 16, 1, 1, 0, "any"), (65, 3584, 8, 16, 1, 1, 2, "any"), (200, 3976, 8, 13, 1, 1, 0, "any"), (64, 3968, 8, 14, 1, 1, 1, "any"),
+         (300, 5120, 8, 16, 1, 16, 3, "any"), (130, 8 * 4100, 8, 16, 1, 1, 1, "any"), (70, 8 * 4064, 8, 13, 1, 1, 1, "one"), (90, 1024, 8, 12, 4, 1, 2, "any"),
+         (40, 512, 8, 15, 2, 3, 0, "low"), (129, 17408, 8, 16, 1, 1, 0, "low"), (17, 640, 4, 10, 1, 1, 0, "any"), (16, 384, 4, 12, 1, 1, 0, "any"),
+         (31, 896, 4, 8, 2, 1, 0, "any")]
+
+
+@pytest.mark.parametrize("R,C,d,bits,G,M,runs,how", CASES)
+def test_device_builder_writes_the_host_builders_bytes(R, C, d, bits, G, M, runs, how):
+    g = torch.Generator().manual_seed(R * 7 + C)
+    n = C // d
+    top = {"any": 1 << bits, "low": 1 << (bits - 2), "one": 1}[how]
+    words = pack_bits(torch.randint(0, top, (R, n), generator=g), bits)
+    mask = torch.randint(0, M, (R,), generator=g).to(torch.uint8) if M > 1 else None
+    book = (torch.randint(0, G, (R,), generator=g).to(torch.uint8), G) if G > 1 else None
+    want, r0, g0 = build_stream(words, C, d, bits, mask, runs, row_book=book)
+    got, r1, g1 = build_stream(words.cuda(), C, d, bits, mask, runs, row_book=None if book is None else (book[0].cuda(), G))
+    assert (r0, g0) == (r1, g1) and want is not None
+    assert torch.equal(got.cpu(), want)
+
+
+@pytest.mark.parametrize("R,C,bits,G", [(3, 64, 16, 1), (70, 1000, 13, 1), (65, 3584, 16, 1), (90, 1032, 14, 4), (33, 264, 12, 2)])
+def test_device_relabelling(R, C, bits, G):
+    L = _lib.lib()
+    g = torch.Generator().manual_seed(bits)
+    n = C // 8
+    tags = (torch.rand(R, n, generator=g) ** 3 * (1 << bits)).long().clamp_(max=(1 << bits) - 1)
+    words = pack_bits(tags, bits)
+    book = torch.randint(0, G, (R,), generator=g).to(torch.uint8)
+    bp = book.data_ptr() if G > 1 else None
+    want = np.zeros(G << bits, np.uint16)
+    _lib.check(L.sq_codebook_balance_books(words.data_ptr(), R, words.shape[1], C, 8, bits, G, bp, want.ctypes.data))
+    wd, bd = words.cuda(), book.cuda()
+    counts = torch.empty(G << bits, dtype=torch.int32, device="cuda")
+    remap = np.zeros(G << bits, np.uint16)
+    args = (wd.data_ptr(), R, words.shape[1], C, 8, bits, G, bd.data_ptr() if G > 1 else None)
+    _lib.check(L.sq_codebook_balance_device(*args, counts.data_ptr(), remap.ctypes.data, _lib.stream_ptr(wd.device)))
+    assert np.array_equal(remap, want)
+    rd = torch.from_numpy(remap.view(np.int16)).cuda()
+    _lib.check(L.sq_codebook_relabel_device(*args, rd.data_ptr(), _lib.stream_ptr(wd.device)))
+    at = tags.numpy() + (book.numpy().astype(np.int64) << bits)[:, None] if G > 1 else tags.numpy()
+    assert torch.equal(wd.cpu(), pack_bits(torch.from_numpy(want[at].astype(np.int64)), bits))
+    m = ctypes.c_void_p()
+    assert L.sq_stream_plan_device(None, R, 1, C, 8, bits, G, None, None, 0, None, ctypes.byref(m), ctypes.byref(ctypes.c_size_t()),
+                                   ctypes.byref(ctypes.c_size_t()), ctypes.byref(ctypes.c_int32()), ctypes.byref(ctypes.c_int32()), None) == _lib.SQ_EINVAL
