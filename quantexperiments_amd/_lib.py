@@ -9,6 +9,7 @@ import torch
 
 _HERE = Path(__file__).resolve().parent
 LIB_PATH = _HERE / "libsqhip.so"
+NATIVE_PATH = _HERE / "_native.so"
 
 SQ_F32, SQ_F16, SQ_BF16 = 0, 1, 2
 SQ_OK, SQ_EINVAL, SQ_EUNSUPPORTED, SQ_EWORKSPACE, SQ_ELAUNCH = 0, -1, -2, -3, -4
@@ -133,6 +134,24 @@ EXPORTS = ("sq_version", "sq_last_error", "sq_dequant", "sq_linear_small", "sq_l
            "sq_workspace_status", "sq_workspace_reset", "sq_noalloc_reset", "sq_stream_spin_limit", "sq_codebook_balance",
            "sq_stream_bytes_books", "sq_stream_build_books", "sq_codebook_balance_books", "sq_stream_counts_bytes", "sq_stream_plan_device",
            "sq_stream_fill_device", "sq_stream_plan_free", "sq_codebook_balance_device", "sq_codebook_relabel_device")
+
+
+_native = None
+
+
+def native():
+    """The native call path (csrc/sq_torch.cpp) on top of lib(): its functions return 0 or a value when they made the call, a
+    negative code for check(), 1 when the caller has to make it.  Raises when it has not been built."""
+    global _native
+    if _native is None:
+        lib()
+        if not NATIVE_PATH.exists():
+            raise RuntimeError(f"{NATIVE_PATH} is missing: build it with `python -m quantexperiments_amd.build`; there is no fallback path")
+        import importlib
+        mod = importlib.import_module(__package__ + "._native")
+        mod.install(importlib.import_module(__package__ + ".kernels")._Workspace.bufs)
+        _native = mod
+    return _native
 
 
 def check(rc: int) -> None:

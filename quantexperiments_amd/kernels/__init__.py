@@ -72,6 +72,28 @@ class _Workspace:
 class PackedLinear(torch.nn.Module):
     """A block linear run from packed tensors."""
 
+    _native = None              # what the native call path keeps of this matrix, made at its first call
+
+    def _make_native(self):
+        s = self.stream is not None
+        o = _lib.native().native(self.words, self.table, self.row_scale, self.row_book, self.row_mask, self.perms, self.row_order, self.stream,
+                                 self.R, self.C, self.d, self.bits, self.G, self.M, self.W, self.stream_runs if s else 0,
+                                 self.stream_groups if s else 0)
+        self.__dict__["_native"] = o
+        return o
+
+    def __setattr__(self, name, value):
+        super().__setattr__(name, value)
+        self.__dict__.pop("_native", None)
+
+    def _apply(self, *args, **kw):                              # .to() and the like replace buffers without setattr
+        r = super()._apply(*args, **kw)
+        self.__dict__.pop("_native", None)
+        return r
+
+    def __getstate__(self):
+        return {k: v for k, v in self.__dict__.items() if k != "_native"}
+
     def __init__(self, words, table, row_scale, row_book, row_mask, perms, K: int, d: int, bias=None,
                  stream: bool | str = True):
         super().__init__()
@@ -380,6 +402,11 @@ def _prep(pieces, x: torch.Tensor, y: torch.Tensor):
 
 def linear_small(pieces, x: torch.Tensor, y: torch.Tensor) -> torch.Tensor:
     """Y[b, off_i + r] for every stacked piece, B = x.shape[0] <= 32 (sq_linear_small)."""
+    rc = _lib.native().linear(pieces, x, y, False)
+    if rc <= 0:
+        if rc:
+            _lib.check(rc)
+        return y
     mats, ldx, ldy = _prep(pieces, x, y)
     dev = x.device
     L = _lib.lib()
@@ -394,6 +421,11 @@ def linear_small(pieces, x: torch.Tensor, y: torch.Tensor) -> torch.Tensor:
 
 def linear_gemm(pieces, x: torch.Tensor, y: torch.Tensor) -> torch.Tensor:
     """Y = X . W^T for T = x.shape[0] activation rows on the MFMA tile kernel (sq_linear_gemm)."""
+    rc = _lib.native().linear(pieces, x, y, True)
+    if rc <= 0:
+        if rc:
+            _lib.check(rc)
+        return y
     mats, ldx, ldy = _prep(pieces, x, y)
     dev = x.device
     L = _lib.lib()
@@ -435,6 +467,11 @@ def _q_check(q: torch.Tensor, sc: torch.Tensor, per_byte: int, qdtype: torch.dty
 def q8_linear(q: torch.Tensor, sc: torch.Tensor, x: torch.Tensor, y: torch.Tensor) -> torch.Tensor:
     """y[:, :V] = x . w^T for the 8-bit block-32 matrix (q int8 [V, C], sc fp16 [V, C/32]); x [B, C]
     fp16 / bf16, y [B, >= V] in x's dtype or fp32 (sq_q8_linear)."""
+    rc = _lib.native().q8_linear(q, sc, x, y)
+    if rc <= 0:
+        if rc:
+            _lib.check(rc)
+        return y
     V, C = _q_check(q, sc, 1, torch.int8, "q8_linear")
     if q.device.type != "cuda" or x.device != q.device or y.device != q.device or sc.device != q.device:
         raise ValueError("q8_linear: q, scale, x and y must be on one GPU (there is no CPU path)")
@@ -470,6 +507,11 @@ def q8_dense(q: torch.Tensor, sc: torch.Tensor, r0: int, r1: int, dtype: torch.d
 def q4_rows(q: torch.Tensor, sc: torch.Tensor, ids: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
     """Rows `ids` (1-D, on the GPU) of the 4-bit block-32 embedding (q uint8 [V, C/2], sc fp16 [V, C/32]) as
     [len(ids), C] in dtype (sq_q4_embed).  q / sc may be pinned host tensors; the output lives where ids do."""
+    out = _lib.native().q4_rows(q, sc, ids, _lib.DTYPES.get(dtype, -1))
+    if type(out) is not int:
+        return out
+    if out < 0:
+        _lib.check(out)
     V, C = _q_check(q, sc, 2, torch.uint8, "q4_rows")
     dev = ids.device
     if dev.type != "cuda":
@@ -500,6 +542,11 @@ def addnorm(h_in: torch.Tensor, add, w: torch.Tensor, eps: float, out: torch.Ten
     w fp16 / bf16 [C]; writes out [B, C] (or [B, M, C] with int32 column orders perms [M, C]) in its dtype and, if
     given, h_out fp32 [B, C] = h_in + add (may be h_in when perms is None).  The reference's addnorm_perm
     (shapequant/kernels/decode_e2e.py:84-108)."""
+    rc = _lib.native().addnorm(h_in, add, w, eps, out, h_out, perms)
+    if rc <= 0:
+        if rc:
+            _lib.check(rc)
+        return out
     dev = h_in.device
     if h_in.dtype != torch.float32 or h_in.dim() != 2 or h_in.stride(1) != 1:
         raise ValueError("addnorm: h_in must be fp32 [B, C] with unit column stride")
@@ -525,6 +572,11 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor, out: torch.Tensor, perms=None
     """out = silu(gate) * up in the tensors' dtype (sq_silu_mul): gate / up fp16 or bf16 [B, C] with the same row
     stride (the two halves of a stacked gate | up output), out [B, C] or [B, M, C] with column orders.  The
     reference's silu_mul_perm (shapequant/kernels/decode_e2e.py:125-136)."""
+    rc = _lib.native().silu_mul(gate, up, out, perms)
+    if rc <= 0:
+        if rc:
+            _lib.check(rc)
+        return out
     dev = gate.device
     if gate.dtype == torch.float32 or gate.dtype not in _lib.DTYPES or gate.dim() != 2 or gate.stride(1) != 1:
         raise ValueError("silu_mul: gate must be fp16 / bf16 [B, C] with unit column stride")
@@ -555,6 +607,11 @@ def linear_small_from(pieces, y: torch.Tensor, x_out: torch.Tensor, *, h_in=None
     x_out [B, C] (contiguous, fp16 / bf16) is always written.  One activation row of pieces on the tag-stream kernel
     runs as ONE launch (the producer fused into the product); everything else as two.  The reference's epi argument
     of proto_runs.gemv (shapequant/kernels/proto_runs.py:505-571)."""
+    rc = _lib.native().linear_from(pieces, y, x_out, h_in, add, w, eps, h_out, gate, up)
+    if rc <= 0:
+        if rc:
+            _lib.check(rc)
+        return y
     norm = h_in is not None
     if norm == (gate is not None):
         raise ValueError("linear_small_from: give either h_in / w or gate / up")
@@ -601,6 +658,11 @@ def linear_small_silu(pieces, x: torch.Tensor, out: torch.Tensor, *, x_out=None,
     partial sums meet), else the two calls through a temporary y.  With h_in / w (and add, eps, h_out, x_out as in
     linear_small_from) the launch also computes its own input, rmsnorm(h_in + add) * w, into x_out; x is then ignored.
     The reference's EPI 2 epilogue of proto_runs.gemv (shapequant/kernels/proto_runs.py:269-287, 505-571)."""
+    rc = _lib.native().linear_silu(pieces, x, out, x_out, h_in, add, w, eps, h_out)
+    if rc <= 0:
+        if rc:
+            _lib.check(rc)
+        return out
     if len(pieces) != 2 or pieces[0].R != pieces[1].R:
         raise ValueError("linear_small_silu: pieces = [gate, up] of one shape")
     R = pieces[0].R

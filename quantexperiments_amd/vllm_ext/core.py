@@ -19,6 +19,7 @@ from __future__ import annotations
 
 import contextlib
 import re
+import sys
 
 import torch
 
@@ -200,6 +201,11 @@ class PackedShards:
     # ------------------------------------------------------------------ forward
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         """x [..., C] -> [..., R] in x's dtype."""
+        y = _lib.native().forward(self, x)
+        if type(y) is not int:
+            return y
+        if y < 0:
+            _lib.check(y)
         shp = x.shape
         if shp[-1] != self.C:
             raise ValueError(f"input size {shp[-1]} != {self.C}")
@@ -395,16 +401,28 @@ class _Trace:
 _trace = _Trace()
 
 
-@torch.library.custom_op("shapequant::linear", mutates_args=())
-def linear_op(x: torch.Tensor, handle: int) -> torch.Tensor:
+# The op's GPU kernel is native (csrc/sq_torch.cpp): it looks the layer up here, makes a PackedShards' call itself and comes
+# back to _linear_in_python for everything else (heads, routes and dtypes it does not cover, the trace).
+torch.library.define("shapequant::linear", "(Tensor x, int handle) -> Tensor", tags=(torch.Tag.pt2_compliant_tag,))
+
+
+def _linear_in_python(x: torch.Tensor, handle: int) -> torch.Tensor:
     y = _REGISTRY[handle].forward(x)
     _trace("linear", handle, x, y)
     return y
 
 
-@linear_op.register_fake
+torch.library.impl("shapequant::linear", "CompositeExplicitAutograd")(_linear_in_python)
+
+
+@torch.library.register_fake("shapequant::linear")
 def _(x: torch.Tensor, handle: int) -> torch.Tensor:
     return x.new_empty(*x.shape[:-1], _REGISTRY[handle].R)
+
+
+linear_op = torch.ops.shapequant.linear
+if _lib.NATIVE_PATH.exists():                       # (not built: the first call that needs a GPU raises)
+    _lib.native().install_op(sys.modules[__name__], _REGISTRY, PackedShards)
 
 
 @torch.library.custom_op("shapequant::embed", mutates_args=())
