@@ -10,6 +10,7 @@ typedef _Float16 half_t;
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef _Float16 half4v __attribute__((ext_vector_type(4)));
 typedef _Float16 half8v __attribute__((ext_vector_type(8)));
+typedef float float2v __attribute__((ext_vector_type(2)));
 typedef float float4v __attribute__((ext_vector_type(4)));
 typedef float float16v __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -21,11 +22,12 @@ constexpr int WAVE = 64;
 __device__ __forceinline__ float h2f(uint16_t b) { return (float)__builtin_bit_cast(half_t, b); }
 __device__ __forceinline__ float bf2f(uint16_t b) { return __builtin_bit_cast(float, (uint32_t)b << 16); }
 
-// fp32 -> bf16 bits, round to nearest even, NaN stays NaN.
-__device__ __forceinline__ uint16_t f2bf(float f) {
-    uint32_t u = __builtin_bit_cast(uint32_t, f);
-    if ((u & 0x7FFFFFFFu) > 0x7F800000u) return (uint16_t)((u >> 16) | 0x40u);
-    return (uint16_t)((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
+// fp32 -> bf16 bits, round to nearest even, NaN stays NaN: one v_cvt_pk_bf16_f32, which takes two values (the rounding
+// written out in integers cost 30 us of a 520 us product with a 2048 x 37888 bf16 output).
+__device__ __forceinline__ uint16_t f2bf(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
+__device__ __forceinline__ uint32_t f2bf_x2(float lo, float hi) {
+    typedef __bf16 bf2v __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((float2v){lo, hi}, bf2v));
 }
 // fp32 -> fp16 bits, round to nearest even.  The empty asm hides where f came from: a multiply feeding this conversion
 // is otherwise folded into v_fma_mixlo_f16, which rounds the exact product to fp16 once, while the same expression
@@ -34,6 +36,11 @@ __device__ __forceinline__ uint16_t f2bf(float f) {
 __device__ __forceinline__ uint16_t f2h(float f) {
     asm("" : "+v"(f));
     return __builtin_bit_cast(uint16_t, (half_t)f);
+}
+
+__device__ __forceinline__ uint32_t f2h_x2(float lo, float hi) {
+    asm("" : "+v"(lo), "+v"(hi));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((float2v){lo, hi}, half2v));
 }
 
 // bf16 bits -> fp16 value (through fp32; exact whenever the value is an fp16 normal,
@@ -135,6 +142,9 @@ size_t small_gemm_route_workspace(const sq_matrix* mats, int n, int B);
 // for these pieces (0: never)
 int small_pass_limit(const sq_matrix* mats, int n);
 size_t gemm_workspace(const sq_matrix* mats, int n, int T);
+// Row scales of a product whose R rows are n stacked pieces: rows end[i - 1] .. end[i] - 1 are scaled by p[i]; n = 0: no scales.
+constexpr int GEMM256_PIECES = 4;
+struct Gemm256Scales { const uint16_t* p[GEMM256_PIECES]; int end[GEMM256_PIECES]; int n; };
 int launch_gemm_dense(const void* w, int w_dtype, int64_t ldw, int R, int C, const void* x, int x_dtype, int64_t ldx,
                       void* y, int y_dtype, int64_t ldy, int T, hipStream_t s, void* ws = nullptr, size_t ws_bytes = 0);
 size_t gemm_dense_workspace(int R, int C, int T);
