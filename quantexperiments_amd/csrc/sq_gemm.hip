@@ -147,7 +147,7 @@ int launch_small_generic(const sq_matrix* mats, int n, const void* x, int x_dtyp
 
 bool gemm256_ok(int C, int64_t ldx, int64_t ldw, const void* x, const void* w);
 size_t gemm256_part_bytes(int T, int R, int C, int cus);
-int launch_gemm256(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ldw, const uint16_t* row_scale, void* y,
+int launch_gemm256(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ldw, const Gemm256Scales& sc, void* y,
                    int y_dtype, int64_t ldy, int y_off, int T, int R, int C, float* part, int cus, hipStream_t s);
 int launch_bf16_to_f16(const uint16_t* x, int64_t ldx, int T, int C, uint16_t* out, hipStream_t s);
 int launch_dequant_with_cvt(const sq_matrix& m, void* out, int64_t ld_out, const uint16_t* x, int64_t ldx, int T, int C,
@@ -194,12 +194,12 @@ size_t small_gemm_route_workspace(const sq_matrix* mats, int n, int B) {
 }
 
 // Pieces that are neighbours in Y are decoded one behind the other and multiplied in ONE tile GEMM over all their
-// rows (their row scales copied into one array): a 512-row k or v projection alone is 2 tiles of 256 rows, a
+// rows: a 512-row k or v projection alone is 2 tiles of 256 rows, a
 // launch that leaves the chip idle (7B q|k|v at 64-255 rows: 139 us as three products, the o projection of q's
 // size: 62 us).
 constexpr size_t STACK_MAX_BYTES = (size_t)1 << 30;
 static bool stacked_route(const sq_matrix* mats, int n) {
-    if (n < 2) return false;
+    if (n < 2 || n > GEMM256_PIECES) return false;
     size_t tot = 0;
     for (int i = 0; i < n; ++i) {
         if (mats[i].R <= 0) return false;
@@ -212,11 +212,6 @@ static int stacked_rows(const sq_matrix* mats, int n) {
     int r = 0;
     for (int i = 0; i < n; ++i) r += mats[i].R;
     return r;
-}
-
-__global__ __launch_bounds__(256) void copy_u16_kernel(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst, int n) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) dst[i] = src[i];
 }
 
 static size_t gemm_workspace_beyond_small(const sq_matrix* mats, int n, int T);
@@ -241,7 +236,7 @@ static size_t gemm_workspace_beyond_small(const sq_matrix* mats, int n, int T) {
     if (big && stacked_route(mats, n)) {
         const int R = stacked_rows(mats, n);
         for (int i = 0; i < n; ++i) need += dense_bytes(mats[i]);
-        return need + align256((size_t)R * 2) + align256((size_t)T * mats[0].C * 2) + gemm256_part_bytes(T, R, mats[0].C, device_cus());
+        return need + align256((size_t)T * mats[0].C * 2) + gemm256_part_bytes(T, R, mats[0].C, device_cus());
     }
     for (int i = 0; i < n; ++i)
         if ((big || !fused_ok(mats[i])) && dense_bytes(mats[i]) > need) need = dense_bytes(mats[i]);
@@ -273,7 +268,7 @@ int launch_gemm_dense(const void* w, int w_dtype, int64_t ldw, int R, int C, con
     if (x_dtype == SQ_F16 && w_dtype == SQ_F16 && T >= GEMM256_MIN_T && gemm256_ok(C, ldx, ldw, x, w)) {
         const size_t part = gemm256_part_bytes(T, R, C, device_cus());
         const bool split = ws && part && ws_bytes >= part;
-        return launch_gemm256((const uint16_t*)x, ldx, (const uint16_t*)w, ldw, nullptr, y, y_dtype, ldy, 0, T, R, C,
+        return launch_gemm256((const uint16_t*)x, ldx, (const uint16_t*)w, ldw, Gemm256Scales{}, y, y_dtype, ldy, 0, T, R, C,
                               split ? (float*)ws : nullptr, split ? device_cus() : 0, s);
     }
     GemmArgs a{};
@@ -343,21 +338,21 @@ int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_
             const int R = stacked_rows(mats, n);
             char* next = wd;
             for (int i = 0; i < n; ++i) next += dense_bytes(mats[i]);
-            uint16_t* scales = (uint16_t*)next;
-            float* part = (float*)(next + align256((size_t)R * 2));
+            float* part = (float*)next;
             char* w = wd;
+            Gemm256Scales sc{};
             int r0 = 0;
             for (int i = 0; i < n; ++i) {
                 const sq_matrix& m = mats[i];
                 int rc = decode(m, w);
                 if (rc) return rc;
-                hipLaunchKernelGGL(copy_u16_kernel, dim3((unsigned)((m.R + 255) / 256)), dim3(256), 0, s, m.row_scale, scales + r0, m.R);
-                rc = check_launch("sq_linear_gemm(row scales)");
-                if (rc) return rc;
                 w += (size_t)m.R * C * 2;                       // rows follow each other without gaps
                 r0 += m.R;
+                sc.p[i] = m.row_scale;
+                sc.end[i] = r0;
             }
-            return launch_gemm256(xh, ldxh, (const uint16_t*)wd, C, scales, y, y_dtype, ldy, mats[0].y_off, T, R, C,
+            sc.n = n;
+            return launch_gemm256(xh, ldxh, (const uint16_t*)wd, C, sc, y, y_dtype, ldy, mats[0].y_off, T, R, C,
                                   gemm256_part_bytes(T, R, C, cus0) ? part : nullptr, cus0, s);
         }
         size_t dense = 0;
@@ -369,7 +364,7 @@ int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_
             if (m.R == 0) continue;
             int rc = decode(m, wd);
             if (rc) return rc;
-            rc = launch_gemm256(xh, ldxh, (const uint16_t*)wd, C, m.row_scale, y, y_dtype, ldy, m.y_off, T, m.R, C,
+            rc = launch_gemm256(xh, ldxh, (const uint16_t*)wd, C, Gemm256Scales{{m.row_scale}, {m.R}, 1}, y, y_dtype, ldy, m.y_off, T, m.R, C,
                                 gemm256_part_bytes(T, m.R, C, cus) ? part : nullptr, cus, s);
             if (rc) return rc;
         }
@@ -455,7 +450,7 @@ int launch_q8_large(const int8_t* q, const uint16_t* sc, int V, int C, const voi
         if (rc) return rc;
         void* yc = (char*)y + (size_t)r0 * ys;
         if (big && gemm256_ok(C, ldxh, C, xh, wd))
-            rc = launch_gemm256(xh, ldxh, (const uint16_t*)wd, C, nullptr, yc, y_dtype, ldy, 0, T, r1 - r0, C,
+            rc = launch_gemm256(xh, ldxh, (const uint16_t*)wd, C, Gemm256Scales{}, yc, y_dtype, ldy, 0, T, r1 - r0, C,
                                 gemm256_part_bytes(T, r1 - r0, C, cus) ? part : nullptr, cus, s);
         else
             rc = launch_gemm_dense(wd, SQ_F16, C, r1 - r0, C, x, x_dtype, ldx, yc, y_dtype, ldy, T, s);

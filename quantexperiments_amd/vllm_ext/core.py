@@ -28,6 +28,7 @@ from ..kernels import (PackedLinear, _Workspace, gemm_dense, linear_gemm, linear
                        q8_linear)
 
 BMAX = _lib.SMALL_BMAX
+STACK_MAX_BYTES = 1 << 30       # most fp16 weights the "dequant" route decodes side by side for one product
 
 # checkpoint suffix of each vLLM (possibly stacked) linear -> the packed pieces, in output order
 STACKED = {
@@ -230,12 +231,18 @@ class PackedShards:
             return linear_gemm(self.rls, x, y)
         # dequant + GEMM: whole pieces ("dequant") or row chunks of ~chunk_bytes ("chunked") decoded to
         # fp16 in the shared scratch, each multiplied into its column slice of Y
+        if x.dtype != torch.float16 and M > BMAX and self.C % 64 == 0:
+            x = x.to(torch.float16)                     # fp16 x fp16 takes the 256 x 256 tile kernel; y keeps its dtype
+        if self.large == "dequant" and self.R * self.C * 2 <= STACK_MAX_BYTES:
+            # one product over the stack: a 1024-row k or v projection alone is a few tiles on an idle chip
+            w = _Workspace.get(self.R * self.C * 2, x.device, kind="dense").view(torch.float16)[:self.R * self.C].view(self.R, self.C)
+            for rl, off in zip(self.rls, self.offs):
+                rl.dense(torch.float16, out=w[off:off + rl.R])
+            return gemm_dense(w, x, y)
         rows = max(self.Rs)
         if self.large == "chunked":
             rows = min(rows, max(128, (self.chunk_bytes // (2 * self.C)) // 128 * 128))
         scratch = _Workspace.get(rows * self.C * 2, x.device, kind="dense").view(torch.float16)
-        if x.dtype != torch.float16 and M > BMAX and self.C % 64 == 0:
-            x = x.to(torch.float16)                     # fp16 x fp16 takes the 256 x 256 tile kernel; y keeps its dtype
         for rl, off in zip(self.rls, self.offs):
             for r0 in range(0, rl.R, rows):
                 r1 = min(rl.R, r0 + rows)

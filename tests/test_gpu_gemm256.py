@@ -1,0 +1,33 @@
+"""The 256 x 256 tile GEMM where its loop and its tile walk have edges: one to four slabs of K, partial tiles both ways, more
+than one super-column of token tiles, unaligned outputs, and stacks with more pieces than one launch scales."""
+
+import numpy as np
+import pytest
+import torch
+
+from quantexperiments_amd.kernels import gemm_dense, linear_gemm
+from tests.helpers import rand_x, rel_max_err, synth, to_device
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T,R,C", [(33, 1, 64), (256, 256, 128), (257, 300, 192), (64, 511, 256), (2305, 260, 64), (4200, 70, 128)])
+@pytest.mark.parametrize("dtype,pad", [(torch.bfloat16, 0), (torch.float16, 8), (torch.float16, 3), (torch.float32, 0)])
+def test_tile_edges(T, R, C, dtype, pad):
+    g = torch.Generator().manual_seed(T + R)
+    x, w = torch.randn(T, C, generator=g).half(), torch.randn(R, C, generator=g).half()
+    ref = (x.float() @ w.float().T).numpy().astype(np.float64)
+    y = torch.full((T, (R + 7) // 8 * 8 + pad), float("nan"), dtype=dtype, device="cuda")
+    gemm_dense(w.cuda(), x.cuda(), y[:, :R])
+    assert rel_max_err(y[:, :R].float().cpu().numpy(), ref) < {torch.float32: 1e-5, torch.float16: 1e-3, torch.bfloat16: 5e-3}[dtype]
+    assert torch.isnan(y[:, R:]).all()
+
+
+@pytest.mark.parametrize("n", [4, 5])
+def test_stack_of_pieces(n):
+    ss = [synth(40 + 3 * i, 128, 8, 13, seed=i) for i in range(n)]
+    x = rand_x(300, 128, torch.bfloat16, seed=n)
+    y = torch.empty(300, sum(s.R for s in ss), dtype=torch.float32, device="cuda")
+    linear_gemm([to_device(s, stream=False) for s in ss], x.cuda(), y)
+    ref = np.concatenate([x.float().numpy().astype(np.float64) @ s.decode().astype(np.float64).T for s in ss], axis=1)
+    assert rel_max_err(y.cpu().numpy(), ref) < 1e-3
