@@ -2,6 +2,7 @@
 //   out[r, perm[mask[r]][j*d + k]] = rn_T( f32(table[book[r]*K + tag[r, j]][k]) * f32(row_scale[r]) )
 // The fp32 product of two fp16 values is exact, so T = fp32 reproduces the CPU decode bit
 // for bit and T = fp16 / bf16 differ from it by exactly one round-to-nearest-even.
+#include <algorithm>
 #include "sq_stream.h"
 
 namespace sq {
@@ -138,6 +139,143 @@ __global__ __launch_bounds__(256) void dequant8x4_cvt_kernel(sq_matrix m, uint16
     *reinterpret_cast<u32x4*>(xout + i) = v;
 }
 
+// d = 4 without column orders, codebooks that fit LDS: persistent workgroups stage their piece's codebook in LDS and decode two
+// neighbouring chunks per lane and step, 16 bytes of 16-bit output (32 of fp32) stored in whole 16-byte pieces, so a wave
+// writes 1 KB of consecutive bytes per instruction.  Four steps are in flight per thread: tags of all four, then the gathers,
+// then the stores.  What bounds it is the write of the dense copy.  One thread per chunk with 2-byte stores and its codeword
+// gathered from L2 took 75 us for 18944 x 3584 (136 MB written), this takes 31.  Up to four stacked pieces share a launch (each
+// gets workgroups by its rows), and a bf16 activation matrix that the product needs as fp16 rides along.
+struct Dequant4Args {
+    sq_matrix m[GEMM256_PIECES];
+    void* out[GEMM256_PIECES];
+    int wg0[GEMM256_PIECES + 1];             // first workgroup of each piece; behind the last piece's: workgroups of the copy
+    int n, r0, raw;                          // r0: first row of the (single) piece that is decoded, its rows end at m.R
+    int64_t ld_out;
+    const uint16_t* x;                       // bf16 [T, C] -> xout fp16 (NULL: no copy)
+    uint16_t* xout;
+    int64_t ldx;
+    int T, C;
+};
+
+template <int DT, int NT>
+__global__ __launch_bounds__(NT) void dequant4_lds_kernel(Dequant4Args a) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char dequant4_lds[];
+    const int wg = (int)blockIdx.x, tid = (int)threadIdx.x;
+    if (wg >= a.wg0[a.n]) {                  // fp16 copy of the activations, 8 elements per thread and step
+        const int64_t total = (int64_t)a.T * a.C / 8, step = (int64_t)(gridDim.x - a.wg0[a.n]) * NT;
+        for (int64_t i = (int64_t)(wg - a.wg0[a.n]) * NT + tid; i < total; i += step) {
+            const int t = (int)(i * 8 / a.C), c = (int)(i * 8 - (int64_t)t * a.C);
+            u32x4 v = *reinterpret_cast<const u32x4*>(a.x + (int64_t)t * a.ldx + c);
+            v.x = bf2h_x2(v.x); v.y = bf2h_x2(v.y); v.z = bf2h_x2(v.z); v.w = bf2h_x2(v.w);
+            *reinterpret_cast<u32x4*>(a.xout + i * 8) = v;
+        }
+        return;
+    }
+    int pi = 0;
+#pragma unroll
+    for (int i = 1; i < GEMM256_PIECES; ++i) pi += i < a.n && wg >= a.wg0[i];
+    const sq_matrix& m = a.m[pi];
+    const int tab16 = (m.G << m.bits) / 2;                      // 16-byte pieces of the codebook
+    for (int i = tid; i < tab16; i += NT)
+        reinterpret_cast<u32x4*>(dequant4_lds)[i] = reinterpret_cast<const u32x4*>(m.table)[i];
+    __syncthreads();
+    const int np = m.C / 8, rows = m.R - a.r0;                  // chunk pairs per row
+    const int nwg = a.wg0[pi + 1] - a.wg0[pi], step = nwg * NT, dr = step / np, dp = step - dr * np;
+    const int first = (wg - a.wg0[pi]) * NT + tid;
+    int r = first / np, p = first - r * np;
+    const uint32_t mask = (1u << m.bits) - 1u;
+    typedef typename store_as<DT>::type OT;
+    OT* out = reinterpret_cast<OT*>(a.out[pi]);
+    while (r < rows) {
+        int rr[4], pp[4];
+        uint64_t w[4];
+        uint32_t book[4];
+        float sc[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            rr[k] = r; pp[k] = p;
+            const int rc = min(r, rows - 1) + a.r0, pos = p * 2 * m.bits, at = pos >> 5;
+            const uint32_t* row = reinterpret_cast<const uint32_t*>(m.tags) + (int64_t)rc * m.W;
+            w[k] = (((uint64_t)row[min(at + 1, m.W - 1)] << 32) | row[at]) >> (pos & 31);
+            book[k] = m.row_book ? (uint32_t)m.row_book[rc] << m.bits : 0u;
+            sc[k] = a.raw ? 1.f : h2f(m.row_scale[rc]);
+            r += dr; p += dp;
+            if (p >= np) { p -= np; ++r; }
+        }
+        u32x2 c[4][2];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            c[k][0] = *reinterpret_cast<const u32x2*>(dequant4_lds + (size_t)(((uint32_t)w[k] & mask) + book[k]) * 8);
+            c[k][1] = *reinterpret_cast<const u32x2*>(dequant4_lds + (size_t)(((uint32_t)(w[k] >> m.bits) & mask) + book[k]) * 8);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (rr[k] >= rows) continue;
+            OT* o = out + (int64_t)rr[k] * a.ld_out + pp[k] * 8;
+            if (DT == SQ_F16 && a.raw) {
+                *reinterpret_cast<u32x4*>(o) = u32x4{c[k][0].x, c[k][0].y, c[k][1].x, c[k][1].y};
+                continue;
+            }
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const uint32_t d = c[k][e >> 1][e & 1];
+                v[2 * e] = h2f((uint16_t)(d & 0xFFFFu)) * sc[k];
+                v[2 * e + 1] = h2f((uint16_t)(d >> 16)) * sc[k];
+            }
+            if constexpr (DT == SQ_F32) {
+                *reinterpret_cast<float4v*>(o) = float4v{v[0], v[1], v[2], v[3]};
+                *reinterpret_cast<float4v*>(o + 4) = float4v{v[4], v[5], v[6], v[7]};
+            } else if constexpr (DT == SQ_F16) {
+                *reinterpret_cast<u32x4*>(o) = u32x4{f2h_x2(v[0], v[1]), f2h_x2(v[2], v[3]), f2h_x2(v[4], v[5]), f2h_x2(v[6], v[7])};
+            } else {
+                *reinterpret_cast<u32x4*>(o) = u32x4{f2bf_x2(v[0], v[1]), f2bf_x2(v[2], v[3]), f2bf_x2(v[4], v[5]), f2bf_x2(v[6], v[7])};
+            }
+        }
+    }
+}
+
+static bool dequant4_ok(const sq_matrix& m, const void* out, int64_t ld_out, int esize) {
+    return m.tags && m.d == 4 && !m.perms && m.C % 8 == 0 && ((int64_t)m.G << m.bits) >= 2 && ((int64_t)m.G << m.bits) * 8 <= 128 * 1024 &&
+           ((uintptr_t)m.table & 15) == 0 && ((uintptr_t)out & 15) == 0 && ld_out * esize % 16 == 0 && (int64_t)m.R * (m.C / 8) < ((int64_t)1 << 30);
+}
+
+// a.m, a.out, a.n, a.r0, a.raw, a.ld_out and the copy are set; the workgroups are dealt here: enough for two codebooks of 64 KB
+// or four of 32 KB per CU, one of 1024 threads where a codebook fills LDS.
+template <int DT>
+static int launch_dequant4(Dequant4Args& a, hipStream_t s) {
+    size_t tab = 0;
+    int64_t pairs = 0;
+    for (int i = 0; i < a.n; ++i) {
+        tab = std::max(tab, (size_t)((int64_t)a.m[i].G << a.m[i].bits) * 8);
+        pairs += (int64_t)(a.m[i].R - a.r0) * (a.m[i].C / 8);
+    }
+    const bool large = tab > 64 * 1024;
+    const int nt = large ? 1024 : 512, per_cu = large ? 1 : (int)std::min<size_t>(4, 160 * 1024 / std::max<size_t>(tab, 1));
+    const int slots = device_cus() * per_cu;
+    int wg = 0;
+    for (int i = 0; i < a.n; ++i) {
+        const int64_t mine = (int64_t)(a.m[i].R - a.r0) * (a.m[i].C / 8);
+        const int64_t most = (mine + 4 * nt - 1) / (4 * nt);     // four pairs per thread at least
+        a.wg0[i] = wg;
+        wg += (int)std::max<int64_t>(1, std::min<int64_t>(most, slots * mine / std::max<int64_t>(pairs, 1)));
+    }
+    for (int i = a.n; i <= GEMM256_PIECES; ++i) a.wg0[i] = wg;
+    if (a.x) wg += (int)std::min<int64_t>(slots, ((int64_t)a.T * a.C / 8 + nt - 1) / nt);
+    if (large) {
+        static bool raised = false;
+        if (!raised) {
+            (void)hipFuncSetAttribute((const void*)dequant4_lds_kernel<DT, 1024>, hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
+            (void)hipGetLastError();
+            raised = true;
+        }
+        hipLaunchKernelGGL((dequant4_lds_kernel<DT, 1024>), dim3((unsigned)wg), dim3(1024), tab, s, a);
+    } else {
+        hipLaunchKernelGGL((dequant4_lds_kernel<DT, 512>), dim3((unsigned)wg), dim3(512), tab, s, a);
+    }
+    return check_launch("sq_dequant");
+}
+
 // Matrices with column orders: scattering 2-byte values straight to HBM costs 4x the plain decode, so a
 // workgroup decodes one row at a time into LDS at its permuted positions (ds_write of one element each, the
 // order read as whole 16/32-byte pieces) and then writes the row out in 16-byte pieces.
@@ -216,6 +354,11 @@ static int launch_dt(const sq_matrix& m, void* out, int64_t ld_out, int r0, int 
         hipLaunchKernelGGL((dequant8x4_kernel<DT>), dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, s, m, (T*)out, ld_out, r0, r1, raw, vec);
         return check_launch("sq_dequant");
     }
+    if (dequant4_ok(m, out, ld_out, (int)sizeof(T))) {
+        Dequant4Args a{};
+        a.m[0] = m; a.m[0].R = r1; a.out[0] = out; a.n = 1; a.r0 = r0; a.raw = raw; a.ld_out = ld_out;
+        return launch_dequant4<DT>(a, s);
+    }
     const unsigned grid = (unsigned)((n + 255) / 256);
     if (m.d == 8) hipLaunchKernelGGL((dequant_kernel<DT, 8>), dim3(grid), dim3(256), 0, s, m, (T*)out, ld_out, r0, r1, raw);
     else if (m.d == 4) hipLaunchKernelGGL((dequant_kernel<DT, 4>), dim3(grid), dim3(256), 0, s, m, (T*)out, ld_out, r0, r1, raw);
@@ -235,6 +378,22 @@ int launch_dequant_with_cvt(const sq_matrix& m, void* out, int64_t ld_out, const
     hipLaunchKernelGGL(dequant8x4_cvt_kernel, dim3((unsigned)(nd + nc)), dim3(256), 0, s, m, (uint16_t*)out, ld_out, x, ldx, T, C, xout,
                        (int)nd, (int)nc);
     return check_launch("sq_linear_gemm(decode + fp16 copy)");
+}
+
+// Raw fp16 decode of up to GEMM256_PIECES pieces, one behind the other at out (rows of C elements), with the fp16 copy of x
+// as above (x NULL: none).  Returns 1 without launching anything when a piece does not take the LDS kernel.
+int launch_dequant_stack(const sq_matrix* mats, int n, void* out, const uint16_t* x, int64_t ldx, int T, int C, uint16_t* xout, hipStream_t s) {
+    if (n < 1 || n > GEMM256_PIECES) return 1;
+    Dequant4Args a{};
+    uint16_t* o = (uint16_t*)out;
+    for (int i = 0; i < n; ++i) {
+        if (mats[i].R <= 0 || !dequant4_ok(mats[i], o, C, 2)) return 1;
+        a.m[i] = mats[i];
+        a.out[i] = o;
+        o += (size_t)mats[i].R * C;
+    }
+    a.n = n; a.raw = 1; a.ld_out = C; a.x = x; a.xout = xout; a.ldx = ldx; a.T = T; a.C = C;
+    return launch_dequant4<SQ_F16>(a, s);
 }
 
 int launch_dequant(const sq_matrix& m, void* out, int out_dtype, int64_t ld_out, int r0, int r1, hipStream_t s, bool raw) {

@@ -150,6 +150,7 @@ size_t gemm256_part_bytes(int T, int R, int C, int cus);
 int launch_gemm256(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ldw, const Gemm256Scales& sc, void* y,
                    int y_dtype, int64_t ldy, int y_off, int T, int R, int C, float* part, int cus, hipStream_t s);
 int launch_bf16_to_f16(const uint16_t* x, int64_t ldx, int T, int C, uint16_t* out, hipStream_t s);
+int launch_dequant_stack(const sq_matrix* mats, int n, void* out, const uint16_t* x, int64_t ldx, int T, int C, uint16_t* xout, hipStream_t s);
 int launch_dequant_with_cvt(const sq_matrix& m, void* out, int64_t ld_out, const uint16_t* x, int64_t ldx, int T, int C,
                             uint16_t* xout, hipStream_t s);
 
@@ -322,7 +323,13 @@ int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_
             xh = (const uint16_t*)ws;
             ldxh = C;
         }
+        auto decode_stack = [&](const sq_matrix* ms, int k, void* w) -> int {
+            const int rc = launch_dequant_stack(ms, k, w, copy_pending ? (const uint16_t*)x : nullptr, ldx, T, C, (uint16_t*)ws, s);
+            if (rc == 0) copy_pending = false;
+            return rc;
+        };
         auto decode = [&](const sq_matrix& m, void* w) -> int {
+            if (const int rc = decode_stack(&m, 1, w); rc <= 0) return rc;
             if (copy_pending) {
                 copy_pending = false;
                 const int rc = launch_dequant_with_cvt(m, w, C, (const uint16_t*)x, ldx, T, C, (uint16_t*)ws, s);
@@ -342,10 +349,12 @@ int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_
             char* w = wd;
             Gemm256Scales sc{};
             int r0 = 0;
+            const int whole = decode_stack(mats, n, w);         // all pieces in one launch, or (1) piece by piece
+            if (whole < 0) return whole;
             for (int i = 0; i < n; ++i) {
                 const sq_matrix& m = mats[i];
-                int rc = decode(m, w);
-                if (rc) return rc;
+                if (whole == 1)
+                    if (int rc = decode(m, w)) return rc;
                 w += (size_t)m.R * C * 2;                       // rows follow each other without gaps
                 r0 += m.R;
                 sc.p[i] = m.row_scale;
