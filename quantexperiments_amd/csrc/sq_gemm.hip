@@ -216,6 +216,7 @@ static int stacked_rows(const sq_matrix* mats, int n) {
 }
 
 static size_t gemm_workspace_beyond_small(const sq_matrix* mats, int n, int T);
+static size_t gemm_workspace_without_mid(const sq_matrix* mats, int n, int T);
 
 size_t gemm_workspace(const sq_matrix* mats, int n, int T) {
     // up to SQ_SMALL_BMAX rows sq_linear_gemm is sq_linear_small, unless the stack goes the other way (see above);
@@ -226,6 +227,12 @@ size_t gemm_workspace(const sq_matrix* mats, int n, int T) {
 }
 
 static size_t gemm_workspace_beyond_small(const sq_matrix* mats, int n, int T) {
+    // (covers the other routes too: the size is asked for without knowing x)
+    const size_t rest = gemm_workspace_without_mid(mats, n, T);
+    return mid_ok(mats, n, T) ? std::max(rest, mid_workspace(mats, n, T)) : rest;
+}
+
+static size_t gemm_workspace_without_mid(const sq_matrix* mats, int n, int T) {
     if (T > SQ_SMALL_BMAX && T <= small_pass_limit(mats, n)) {
         // full passes and the last, shorter one may run different kernels with different needs
         const size_t full = small_workspace(mats, n, SQ_SMALL_BMAX);
@@ -284,9 +291,10 @@ int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_
                 int64_t ldy, int T, void* ws, size_t ws_bytes, void* sums, hipStream_t s) {
     if (T <= SQ_SMALL_BMAX && !small_takes_gemm_route(mats, n, T, x, ldx))
         return launch_small(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, ws_bytes, sums, s);
+    if (mid_ok(mats, n, T) && x_vec_ok(x, ldx, mats[0].C)) return launch_mid(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, ws_bytes, s);
     if (T > SQ_SMALL_BMAX && T <= small_pass_limit(mats, n) && x_vec_ok(x, ldx, mats[0].C)) {
-        // a few passes of the decode-time kernel read the packed tags a few times; decoding to fp16 first
-        // (below) writes and reads 8 to 16 times as many bytes once
+        // stacks that cannot go in one pass (pieces of different formats): a few passes of the decode-time kernel read the packed
+        // tags a few times; decoding to fp16 first (below) writes and reads 8 to 16 times as many bytes once
         const size_t ys = y_dtype == SQ_F32 ? 4 : 2;
         for (int t = 0; t < T; t += SQ_SMALL_BMAX) {
             const int nb = T - t < SQ_SMALL_BMAX ? T - t : SQ_SMALL_BMAX;

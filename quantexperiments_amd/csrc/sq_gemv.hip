@@ -130,7 +130,7 @@ static bool stream_rows(const sq_matrix& m, int B) {
 // ---- matrix-core path (pieces without column orders)
 struct MmaPlan { int RW, NT, KW, ks; };
 
-static bool mma_shape(const sq_matrix& m) { return fast_shape(m) && !m.perms; }
+bool mma_shape(const sq_matrix& m) { return fast_shape(m) && !m.perms; }
 
 // bytes of codebook the matrix-core kernel stages in LDS (0: gathers go through the cache)
 static size_t mma_table_bytes(const sq_matrix& m) {
@@ -168,7 +168,8 @@ static MmaPlan mma_plan(const sq_matrix& m, int B) {
     return best;
 }
 
-// Passes of 32 rows through the matrix-core decode kernel against decode + tile GEMM (7B layer): 77 us per pass
+// For pieces that cannot share one pass (formats or lengths differ), and for the workspace of those that can: passes of 32 rows
+// through the matrix-core decode kernel against decode + tile GEMM (7B layer): 77 us per pass
 // against 600-640 us when the codebook sits in LDS (d = 4), 201 us per pass when its gathers go to L2.  A
 // codebook that fills most of LDS leaves room for fewer waves per workgroup and doubles the cost of a pass
 // (27B layer, 4 books of 4096: 246 us per pass against 800 us).

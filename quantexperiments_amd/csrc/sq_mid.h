@@ -1,0 +1,277 @@
+// Codebook product for more activation rows than a decode step has and fewer than a prefill: T = 33 .. 256 (384 for large d = 4
+// matrices).
+//
+// Decoding the matrix to fp16 first writes and reads eight times its bytes and then multiplies tiles of 256 rows; passes of 32
+// rows through the decode-time kernel gather every codeword once per pass.  Here every codeword is gathered once for all T rows.
+// v_mfma_f32_16x16x32_f16 takes the weights as its A operand (lane l: row l % 16, 8 consecutive k), which are two d = 4
+// codewords (LDS) or one d = 8 codeword (L2), so a lane gathers its operand straight into registers and uses it for all NT
+// tiles of 16 activation rows; the activations are the B operand and come from LDS.
+//
+// Bound: d = 8 by the gathers up to about 128 rows (16 bytes used of the 64 that L2 sends: 18944 x 2 x 3584 take 100 us at 33 rows
+// and 112 at 128), else by LDS: every wave reads all the activations for its 16 or 32 weight rows (12-bit, 18944 x 2 x 3584 at 128
+// rows: 54 us, 640 TFLOP/s).  Before, in passes of 32 rows or decoded first, at 33 / 77 / 128 / 256 rows: d = 8, 18944 x 2 x 3584:
+// 172 / 205 / 205 / 209 us, now 100 / 107 / 112 / 188; 12-bit: 41 / 68 / 102 / 165, now 30 / 40 / 54 / 105.
+//
+//   workgroup   8 waves, two per SIMD so that one gathers while the other multiplies (4 waves: a third slower); each has TW tiles
+//               of 16 weight rows x all NT x 16 activation rows (accumulators TW x NT x 4 registers)
+//   K           in rounds of 4 lane units (UK columns of tags each, as in sq_rows_mfma.h), rounds in stages of S matrix steps;
+//               step j of lane group g is columns (4 round + g) UK + 8 j .. + 7
+//   X           stages of NT x 16 rows x 4 x S x 16 bytes, double buffered in LDS; loaded to registers two stages ahead
+//               (converted bf16 -> fp16 on the way to LDS), one barrier per stage
+//   tags        two rounds ahead; codewords PD steps ahead (one from LDS, three from L2 where the steps are short)
+//   grid        row blocks x ks slices of the rounds; with ks > 1 fp32 partial sums, added by mid_reduce_kernel
+//
+// An X row of a stage is 4 S pieces of 16 bytes; piece c of row t sits at slot c ^ h(t), with h such that the 16 lanes of an
+// LDS clock (rows 0-3, 12-15 of one lane group with rows 4-11 of the next, and so on) fall into 16 different groups of four
+// banks.
+#pragma once
+#include <type_traits>
+#include "sq_rows_mfma.h"
+
+namespace sq {
+
+constexpr int MID_PIECES = 4;
+constexpr int MID_NW = 8;                    // waves per workgroup, two per SIMD
+
+struct MidPiece {
+    sq_matrix m;
+    const uint32_t* tiled;       // tile-major copy of the tags or NULL
+    float* part;                 // ks > 1: fp32 [ks, T, R]
+    int wg0;
+};
+
+struct MidArgs {
+    MidPiece p[MID_PIECES];
+    int n;
+    const uint16_t* x;
+    int64_t ldx;
+    void* y;
+    int64_t ldy;
+    int T, x_dtype, y_dtype;
+    int U, ks, table_bytes;
+};
+
+template <int S> __device__ __forceinline__ int mid_swizzle(int t) {
+    const int b = ((t >> 2) ^ (t >> 3)) & 1;         // rows 4 .. 11
+    if (S == 4) return (t & 1) | (b ^ 1) << 1 | ((t >> 1) & 1) << 2 | ((t >> 3) & 1) << 3;
+    return b | ((t >> 1) & 1) << 1 | ((t >> 3) & 1) << 2;
+}
+
+constexpr int mid_stage_bytes(int NT, int S) { return NT * 16 * S * 64; }
+
+template <int BITS, int D, int NT, int TW, int S, bool BF>
+__global__ __launch_bounds__(64 * MID_NW, 2) void mid_kernel(MidArgs a) {
+    constexpr int UD = unit_of<BITS>::UD, TPU = UD * 32 / BITS, CPS = 8 / D, SPR = TPU / CPS, UK = TPU * D, NST = SPR / S;
+    constexpr int ROWB = S * 64, STAGE = mid_stage_bytes(NT, S), NTH = 64 * MID_NW, PCS = (NT * 64 * S + NTH - 1) / NTH;
+    constexpr int PD = D == 8 && NT * TW < 24 ? 3 : 1, XB = NT <= 8 ? 2 : 1;   // steps that codewords and activations are fetched ahead of
+    static_assert(SPR % S == 0 && SPR % (PD + 1) == 0 && (NST == 1 || NST % 2 == 0), "steps per round");
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (D == 4 && (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)smem != 0u) return;   // (gathers count from LDS address 0)
+    int pi = 0;
+    while (pi + 1 < a.n && (int)blockIdx.x >= a.p[pi + 1].wg0) ++pi;
+    const MidPiece& P = a.p[pi];
+    const sq_matrix& m = P.m;
+    const int w = (int)blockIdx.x - P.wg0, slice = w % a.ks, blk = w / a.ks;
+    const int NR = (a.U + 3) >> 2, NP = (NR + 1) >> 1;                       // rounds, and pairs of them: slices are whole pairs
+    const int r0 = 2 * (int)((int64_t)NP * slice / a.ks), r1 = min(NR, 2 * (int)((int64_t)NP * (slice + 1) / a.ks));
+    unsigned char* xbuf = smem + a.table_bytes;
+
+    // ---- this wave's tiles (tiles past the last row repeat the last one and are not stored)
+    const int ntiles = (m.R + 15) >> 4, tile0 = (blk * MID_NW + wave) * TW;
+    // (byte offsets from a uniform base: one address register per load)
+    const uint32_t us = (P.tiled ? 16 * UD : UD) * 4;                        // bytes between two units of a row
+    const char* tags = reinterpret_cast<const char*>(P.tiled ? P.tiled : reinterpret_cast<const uint32_t*>(m.tags));
+    uint32_t to[TW], bo[TW];
+#pragma unroll
+    for (int i = 0; i < TW; ++i) {
+        const int tile = min(tile0 + i, ntiles - 1), row = min(tile * 16 + li, m.R - 1);
+        to[i] = P.tiled ? ((uint32_t)tile * (uint32_t)a.U * 16u + (uint32_t)li) * (UD * 4) : (uint32_t)row * (uint32_t)m.W * 4u;
+        bo[i] = m.row_book ? (uint32_t)m.row_book[row] << (BITS + (D == 8 ? 4 : 3)) : 0u;
+    }
+    auto load_tags = [&](int round, dwords<UD>* t) {
+        const uint32_t u = (uint32_t)min(4 * round + lg, a.U - 1) * us;
+#pragma unroll
+        for (int i = 0; i < TW; ++i) t[i] = load_unit<UD>(reinterpret_cast<const uint32_t*>(tags + (to[i] + u)));
+    };
+
+    // ---- activations: thread's pieces q = tid + NTH k of a stage, row q / (4 S), piece q % (4 S) = lane group * S + step
+    uint32_t xo[PCS], xl[PCS];
+    int xg[PCS];
+#pragma unroll
+    for (int k = 0; k < PCS; ++k) {
+        const int q = min(tid + NTH * k, NT * 64 * S - 1), t = q / (4 * S), c = q - t * (4 * S), g = c / S, j = c - g * S;
+        xg[k] = g;
+        xo[k] = ((uint32_t)min(t, a.T - 1) * (uint32_t)a.ldx + (uint32_t)(g * UK + j * 8)) * 2u;
+        xl[k] = (uint32_t)(t * ROWB + ((c ^ mid_swizzle<S>(t & 15)) << 4));
+    }
+    // columns past the row's end (the last round's missing units, rounds past the slice) are zeros; what is read in their
+    // place is the row's last unit
+    auto load_x = [&](u32x4* px, int round, int st) {
+        const int left = a.U - 1 - 4 * min(round, NR - 1);                   // the round's last unit
+        const char* base = reinterpret_cast<const char*>(a.x) + (int64_t)min(round, NR - 1) * (8 * UK) + st * (S * 16);
+#pragma unroll
+        for (int k = 0; k < PCS; ++k) px[k] = *reinterpret_cast<const u32x4*>(base + (xo[k] - (uint32_t)(max(xg[k] - left, 0) * (UK * 2))));
+    };
+    auto store_x = [&](const u32x4* px, int buf, int round) {
+        const int units = round < r1 ? a.U - 4 * round : 0;
+#pragma unroll
+        for (int k = 0; k < PCS; ++k) {
+            u32x4 v = px[k];
+            if constexpr (BF) { v.x = bf2h_x2(v.x); v.y = bf2h_x2(v.y); v.z = bf2h_x2(v.z); v.w = bf2h_x2(v.w); }
+            const uint32_t keep = xg[k] < units ? 0xFFFFFFFFu : 0u;
+            v.x &= keep; v.y &= keep; v.z &= keep; v.w &= keep;
+            if ((NT * 64 * S) % NTH == 0 || tid + NTH * k < NT * 64 * S) *reinterpret_cast<u32x4*>(xbuf + buf * STAGE + xl[k]) = v;
+        }
+    };
+    const uint32_t xbase = (uint32_t)(li * ROWB + (((lg * S) ^ mid_swizzle<S>(li)) << 4));
+
+    // ---- codewords of one step
+    auto gather = [&](u32x4* f, const dwords<UD>* t, int step) {
+#pragma unroll
+        for (int i = 0; i < TW; ++i) {
+            if constexpr (D == 8) {
+                f[i] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(m.table) + ((unit_tag<BITS, UD>(t[i], step) << 4) + bo[i]));
+            } else {
+                const u32x2 lo = *(const mma_lds_u32x2*)(uintptr_t)unit_lds_offset<BITS, UD, 3>(t[i], step * 2, bo[i]);
+                const u32x2 hi = *(const mma_lds_u32x2*)(uintptr_t)unit_lds_offset<BITS, UD, 3>(t[i], step * 2 + 1, bo[i]);
+                f[i] = u32x4{lo.x, lo.y, hi.x, hi.y};
+            }
+        }
+    };
+
+    float4v acc[TW][NT];
+#pragma unroll
+    for (int i = 0; i < TW; ++i)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[i][n] = float4v{0.f, 0.f, 0.f, 0.f};
+
+    // Two of everything that is on its way: tags of this round and the next, activations of the next stage and the one after.
+    // A pair's members swap by the parity of the round (the loop is unrolled twice), never by moving registers, which would
+    // wait for the loads.
+    dwords<UD> tag[2][TW];
+    u32x4 px[2][PCS], wf[PD + 1][TW];
+    load_tags(r0, tag[0]);
+    load_x(px[0], r0, 0);
+    load_tags(r0 + 1, tag[1]);
+    load_x(px[1], NST > 1 ? r0 : r0 + 1, NST > 1 ? 1 : 0);
+    if (D == 4) stage_table(m.table, a.table_bytes, smem);
+    store_x(px[0], 0, r0);
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < PD; ++s) gather(wf[s], tag[0], s);
+    auto do_round = [&](auto parity, int round) {
+        constexpr int P = decltype(parity)::value;
+#pragma unroll
+        for (int st = 0; st < NST; ++st) {
+            constexpr int B0 = NST == 1 ? P : 0;                             // LDS buffer and register set of the round's first stage
+            const int q = (B0 + st) & 1;
+            load_x(px[q], round + (st + 2) / NST, (st + 2) % NST);
+            half8v xf[XB][NT];
+            auto read_x = [&](half8v* f, int j) {
+                const unsigned char* xs = xbuf + q * STAGE + (xbase ^ (uint32_t)(j << 4));
+#pragma unroll
+                for (int n = 0; n < NT; ++n) f[n] = *reinterpret_cast<const half8v*>(xs + n * (16 * ROWB));
+            };
+            if (XB == 2) read_x(xf[0], 0);
+#pragma unroll
+            for (int j = 0; j < S; ++j) {
+                const int s = st * S + j;
+                __builtin_amdgcn_sched_barrier(0);
+                if (s + PD < SPR) gather(wf[(s + PD) % (PD + 1)], tag[P], s + PD);
+                else gather(wf[(s + PD) % (PD + 1)], tag[P ^ 1], s + PD - SPR);
+                if (s + PD == SPR - 1) load_tags(round + 2, tag[P]);         // this round's tags have all been used
+                if (XB == 1) read_x(xf[0], j);
+                else if (j + 1 < S) read_x(xf[(j + 1) & (XB - 1)], j + 1);
+                // the next stage's activations, in the middle of this one, where the other wave of the SIMD multiplies
+                if (j == S / 2 - 1) store_x(px[q ^ 1], q ^ 1, round + (st + 1) / NST);
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+#pragma unroll
+                    for (int i = 0; i < TW; ++i)
+                        acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8v, wf[s % (PD + 1)][i]), xf[j & (XB - 1)][n], acc[i][n], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            __syncthreads();
+        }
+    };
+    for (int round = r0; round < r1; round += 2) {                           // (a partner past the slice's end multiplies zeros)
+        do_round(std::integral_constant<int, 0>{}, round);
+        do_round(std::integral_constant<int, 1>{}, round + 1);
+    }
+
+    // ---- lane: activation row 16 n + li, weight rows 16 tile + 4 lg .. + 3
+    const bool vec = m.R % 4 == 0;
+#pragma unroll
+    for (int i = 0; i < TW; ++i) {
+        const int r = (tile0 + i) * 16 + lg * 4;
+        if (r >= m.R) continue;
+        float sc[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sc[e] = h2f(m.row_scale[min(r + e, m.R - 1)]);
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+            const int t = n * 16 + li;
+            if (t >= a.T) continue;
+            if (a.ks > 1) {
+                float* o = P.part + ((int64_t)slice * a.T + t) * m.R + r;
+                if (vec) {
+                    *reinterpret_cast<float4v*>(o) = acc[i][n];
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) if (r + e < m.R) o[e] = acc[i][n][e];
+                }
+                continue;
+            }
+            const int64_t o = (int64_t)t * a.ldy + m.y_off + r;
+            if (a.y_dtype != SQ_F32 && r + 4 <= m.R && ((o | (int64_t)((uintptr_t)a.y >> 1)) & 3) == 0) {
+                const float4v v = acc[i][n];
+                *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(a.y) + o) =
+                    a.y_dtype == SQ_BF16 ? u32x2{f2bf_x2(v[0] * sc[0], v[1] * sc[1]), f2bf_x2(v[2] * sc[2], v[3] * sc[3])}
+                                         : u32x2{f2h_x2(v[0] * sc[0], v[1] * sc[1]), f2h_x2(v[2] * sc[2], v[3] * sc[3])};
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) if (r + e < m.R) store_y(a.y, a.y_dtype, o + e, acc[i][n][e] * sc[e]);
+            }
+        }
+    }
+}
+
+template <int BITS, int D, int NT, int TW, int S, bool BF>
+int launch_mid_dtype(const MidArgs& a, int grid, hipStream_t s) {
+    static bool raised = false;
+    if (!raised) {
+        (void)hipFuncSetAttribute((const void*)mid_kernel<BITS, D, NT, TW, S, BF>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        (void)hipGetLastError();
+        raised = true;
+    }
+    hipLaunchKernelGGL((mid_kernel<BITS, D, NT, TW, S, BF>), dim3((unsigned)grid), dim3(64 * MID_NW), (size_t)a.table_bytes + 2 * mid_stage_bytes(NT, S), s, a);
+    return check_launch("sq_linear_gemm(mid)");
+}
+
+template <int BITS, int D, int NT, int TW, int S>
+int launch_mid_as(const MidArgs& a, int grid, hipStream_t s) {
+    return a.x_dtype == SQ_BF16 ? launch_mid_dtype<BITS, D, NT, TW, S, true>(a, grid, s) : launch_mid_dtype<BITS, D, NT, TW, S, false>(a, grid, s);
+}
+
+// A variant per number of activation tiles; stages half as deep where many tiles or the codebook leave no room in LDS.
+#define SQ_MID_CASE(NT_, TW_, S_) if (nt == NT_ && tw == TW_ && st == S_) return launch_mid_as<BITS, D, NT_, TW_, S_>(a, grid, s);
+template <int BITS, int D>
+int launch_mid_format(const MidArgs& a, int nt, int tw, int st, int grid, hipStream_t s) {
+    SQ_MID_CASE(3, 2, 4) SQ_MID_CASE(3, 1, 4) SQ_MID_CASE(5, 2, 4) SQ_MID_CASE(5, 1, 4) SQ_MID_CASE(8, 2, 4) SQ_MID_CASE(8, 1, 4)
+    SQ_MID_CASE(12, 2, 2) SQ_MID_CASE(12, 1, 2) SQ_MID_CASE(16, 1, 2)
+    if constexpr (D == 8) {
+        SQ_MID_CASE(16, 2, 2)
+    } else {
+        SQ_MID_CASE(3, 2, 2) SQ_MID_CASE(3, 1, 2) SQ_MID_CASE(5, 2, 2) SQ_MID_CASE(5, 1, 2) SQ_MID_CASE(8, 2, 2) SQ_MID_CASE(8, 1, 2)
+    }
+    return SQ_EUNSUPPORTED;
+}
+
+#define SQ_MID_FORMAT(BITS, D)                                                                                             \
+    int launch_mid_b##BITS##d##D(const MidArgs& a, int nt, int tw, int st, int grid, hipStream_t s) {                     \
+        return launch_mid_format<BITS, D>(a, nt, tw, st, grid, s);                                                         \
+    }
+
+}  // namespace sq

@@ -1,0 +1,5 @@
+// Kernels for 33 to a few hundred activation rows for 12-bit tags, chunk width 4.
+#include "sq_mid.h"
+namespace sq {
+SQ_MID_FORMAT(12, 4)
+}

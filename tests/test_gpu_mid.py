@@ -1,0 +1,37 @@
+"""Products of 33 to 384 activation rows in one pass over the tags: edges of the tiles of rows and activation rows, a last round
+with missing units, odd numbers of rounds, K slices, stacks, several codebooks, two tiles of rows per wave, two parts of rows."""
+
+import numpy as np
+import pytest
+import torch
+
+from quantexperiments_amd.kernels import linear_gemm
+from tests.helpers import rand_x, rel_max_err, synth, to_device
+
+pytestmark = pytest.mark.gpu
+
+CASES = [  # rows of the stack's pieces, C, d, bits, G, T
+    ((1,), 64, 8, 16, 1, 33), ((15, 17), 320, 8, 16, 1, 48), ((129,), 3584, 8, 16, 1, 49), ((513, 128), 1600, 8, 16, 2, 81),
+    ((66,), 704, 8, 16, 1, 256), ((33000,), 128, 8, 16, 1, 250),
+    ((1,), 32, 4, 12, 1, 80), ((127, 3, 260), 1056, 4, 12, 1, 128), ((130,), 2080, 4, 12, 4, 129), ((64, 70), 1024, 4, 12, 4, 256),
+    ((33001,), 160, 4, 12, 1, 193), ((32768,), 96, 4, 12, 1, 241), ((4096,), 16384, 4, 12, 1, 257),
+    ((257,), 576, 4, 10, 1, 192), ((40, 8), 1600, 4, 10, 2, 34), ((131,), 1536, 4, 8, 1, 129), ((36,), 64, 4, 8, 1, 255),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c)))
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("stream", [True, False], ids=["tiled", "rows"])
+def test_one_pass_matches_oracle(case, dtype, stream):
+    rows, C, d, bits, G, T = case
+    ss = [synth(R, C, d, bits, G, 1, seed=R + T) for R in rows]
+    lins = [to_device(s, stream=stream and d == 4) for s in ss]
+    x = rand_x(T, C, dtype, seed=T)
+    ref = torch.cat([x.cuda().double() @ torch.from_numpy(s.decode()).cuda().double().T for s in ss], dim=1)
+    y = torch.empty(T, sum(rows), dtype=torch.float32, device="cuda")
+    linear_gemm(lins, x.cuda(), y)
+    assert rel_max_err(y.cpu().numpy(), ref.cpu().numpy()) < 1e-3
+    lowp = torch.empty(T, sum(rows), dtype=dtype, device="cuda")
+    linear_gemm(lins, x.cuda(), lowp)
+    assert torch.equal(lowp, y.to(dtype))
+    assert np.isfinite(lowp.float().cpu().numpy()).all()
