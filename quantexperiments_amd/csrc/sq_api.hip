@@ -130,6 +130,7 @@ int sq_linear_small(const sq_matrix* mats, int32_t n_mats, const void* x, int x_
 static_assert(sq::SQ_WS_HEADER == SQ_WS_HEADER_BYTES, "the header size is part of the ABI");
 static __device__ __align__(256) unsigned char g_static_scratch[SQ_NOALLOC_SCRATCH_BYTES];
 static std::atomic<void*> g_static_scratch_ptr[64];
+constexpr int NOALLOC_ROWS_IN_PLACE = 10;
 
 // This device's copy of the scratch array (its address, looked up on first use with the device current), or nullptr +
 // error.  The array is zero when the code object is loaded, which is what the header must be before the first call:
@@ -153,15 +154,19 @@ int sq_linear_small_noalloc(const sq_matrix* mats, int32_t n_mats, const void* x
     if (rc) return rc;
     if (B > SQ_SMALL_BMAX) return fail(SQ_EINVAL, "sq_linear_small_noalloc: B %d > %d", B, SQ_SMALL_BMAX);
     if (B == 0 || n_mats == 0) return SQ_OK;
-    const size_t need = sq_workspace_bytes(mats, n_mats, B, 0);
+    const size_t inner = (size_t)SQ_NOALLOC_SCRATCH_BYTES - SQ_WS_HEADER;
+    // a stack with column orders whose decoded weights do not fit takes the decode-time kernel, up to the rows where that is
+    // several times slower
+    const bool route = small_takes_gemm_route(mats, n_mats, B, x, ldx);
+    const bool in_place = route && B <= NOALLOC_ROWS_IN_PLACE && small_gemm_route_workspace(mats, n_mats, B) > inner;
+    const size_t need = in_place ? small_workspace(mats, n_mats, B) + SQ_WS_HEADER : sq_workspace_bytes(mats, n_mats, B, 0);
     if (need > (size_t)SQ_NOALLOC_SCRATCH_BYTES)
         return fail(SQ_EWORKSPACE, "sq_linear_small_noalloc: these pieces need %zu bytes of workspace at %d rows, the built-in scratch holds %u "
                                    "(use sq_linear_small with a workspace of the caller's)", need, B, (unsigned)SQ_NOALLOC_SCRATCH_BYTES);
     if ((rc = refuse_if_poisoned("sq_linear_small_noalloc", mats, n_mats))) return rc;
     char* ws = (char*)static_scratch();
     if (!ws) return SQ_ELAUNCH;
-    const size_t inner = (size_t)SQ_NOALLOC_SCRATCH_BYTES - SQ_WS_HEADER;
-    if (small_takes_gemm_route(mats, n_mats, B, x, ldx))
+    if (route && !in_place)
         return launch_gemm(mats, n_mats, x, x_dtype, ldx, y, y_dtype, ldy, B, ws + SQ_WS_HEADER, inner, ws, (hipStream_t)stream);
     return launch_small(mats, n_mats, x, x_dtype, ldx, y, y_dtype, ldy, B, ws + SQ_WS_HEADER, inner, ws, (hipStream_t)stream);
 }

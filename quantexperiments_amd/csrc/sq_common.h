@@ -138,12 +138,18 @@ int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_
 // stacks with column orders and more than a few activation rows: sq_linear_small runs the decode + tile GEMM route
 bool small_takes_gemm_route(const sq_matrix* mats, int n, int B, const void* x, int64_t ldx);
 size_t small_gemm_route_workspace(const sq_matrix* mats, int n, int B);
+constexpr int MID_PIECES = 4;
 // 33 .. a few hundred activation rows in one pass over the tags (sq_mid.h): whether these pieces can take it, and its call
 bool mma_shape(const sq_matrix& m);
 bool mid_ok(const sq_matrix* mats, int n, int T);
 size_t mid_workspace(const sq_matrix* mats, int n, int T);
 int launch_mid(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws,
                size_t ws_bytes, hipStream_t s);
+// the same for weights already decoded to fp16, w[i] = [R, C] of piece i without row scales (1 .. 256 activation rows)
+bool mid_dense_ok(const sq_matrix* mats, int n, int T);
+size_t mid_dense_workspace(const sq_matrix* mats, int n, int T);
+int launch_mid_decoded(const sq_matrix* mats, int n, const void* const* w, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T,
+                       void* ws, hipStream_t s);
 // most activation rows for which passes of SQ_SMALL_BMAX rows through the decode-time kernel beat decode + GEMM
 // for these pieces (0: never), where they cannot share a pass
 int small_pass_limit(const sq_matrix* mats, int n);

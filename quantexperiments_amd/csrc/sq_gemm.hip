@@ -154,6 +154,7 @@ int launch_dequant_stack(const sq_matrix* mats, int n, void* out, const uint16_t
 int launch_dequant_with_cvt(const sq_matrix& m, void* out, int64_t ld_out, const uint16_t* x, int64_t ldx, int T, int C,
                             uint16_t* xout, hipStream_t s);
 
+static bool mid_x_ok(int64_t ldx, int T) { return (int64_t)T * ldx * 2 < (int64_t)1 << 32; }     // 32-bit offsets
 static bool x_vec_ok(const void* x, int64_t ldx, int C) { return C % 8 == 0 && ldx % 8 == 0 && ((uintptr_t)x & 15) == 0; }
 // Activation rows from which the large-tile route (decode each piece once into the workspace as raw fp16
 // codewords, then the 256 x 256 tile GEMM with the row scale in its epilogue) replaces the fused 128 x 128
@@ -174,24 +175,6 @@ static bool big_route(const sq_matrix* mats, int n, int T) {
     for (int i = 0; i < n; ++i)
         if (mats[i].perms) return true;
     return false;
-}
-
-// Activation rows from which sq_linear_small hands a stack with column orders to the route above.
-constexpr int MASKED_GEMM_FROM = 11;
-
-static bool masked_gemm(const sq_matrix* mats, int n, int B) {
-    if (B < MASKED_GEMM_FROM || mats[0].C % 64) return false;
-    for (int i = 0; i < n; ++i)
-        if (mats[i].perms) return true;
-    return false;
-}
-
-bool small_takes_gemm_route(const sq_matrix* mats, int n, int B, const void* x, int64_t ldx) {
-    return masked_gemm(mats, n, B) && x_vec_ok(x, ldx, mats[0].C);
-}
-
-size_t small_gemm_route_workspace(const sq_matrix* mats, int n, int B) {
-    return masked_gemm(mats, n, B) ? gemm_workspace(mats, n, B) : 0;
 }
 
 // Pieces that are neighbours in Y are decoded one behind the other and multiplied in ONE tile GEMM over all their
@@ -215,6 +198,80 @@ static int stacked_rows(const sq_matrix* mats, int n) {
     return r;
 }
 
+// Up to 256 activation rows of what cannot go in one pass over the tags (sq_mid.h): column orders, formats whose rows are not
+// whole lane units, codebooks too large for it.  Pieces are decoded, as many as a launch and STACK_MAX_BYTES take, and multiplied
+// straight from there.
+static int decoded_group(const sq_matrix* mats, int n, int i0, int T) {
+    int k = 0;
+    size_t tot = 0;
+    while (i0 + k < n && k < MID_PIECES && mats[i0 + k].R > 0 && (k == 0 || tot + dense_bytes(mats[i0 + k]) <= STACK_MAX_BYTES)) {
+        if (!mid_dense_ok(mats + i0, k + 1, T)) break;
+        tot += dense_bytes(mats[i0 + k++]);
+    }
+    return k;
+}
+
+// (more rows than half the CUs' worth of 256-row tiles fill the chip in the tile GEMM, whose workgroups read less: 37888 x 3584 at
+// 64 rows, 237 us with it, 248 here; 4608 x 3584 65 and 45, 3584 x 18944 154 and 99, 593 x 1984 60 and 22)
+static bool decoded_route(const sq_matrix* mats, int n, int T) {
+    int64_t rows = 0;
+    for (int i = 0; i < n; ++i) {
+        rows += mats[i].R;
+        if (mats[i].R > 0 && (!mats[i].tags || !decoded_group(mats, n, i, T))) return false;
+    }
+    return rows < (int64_t)128 * device_cus() || mats[0].C % 64;
+}
+
+static size_t decoded_workspace(const sq_matrix* mats, int n, int T) {
+    size_t need = 0;
+    for (int i = 0, k; i < n; i += std::max(k, 1)) {
+        k = decoded_group(mats, n, i, T);
+        size_t tot = k ? mid_dense_workspace(mats + i, k, T) : 0;
+        for (int j = 0; j < k; ++j) tot += dense_bytes(mats[i + j]);
+        need = std::max(need, tot);
+    }
+    return need;
+}
+
+static int launch_decoded(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws,
+                          hipStream_t s) {
+    for (int i = 0, k; i < n; i += std::max(k, 1)) {
+        k = decoded_group(mats, n, i, T);
+        const void* w[MID_PIECES];
+        char* next = (char*)ws;
+        for (int j = 0; j < k; ++j) {
+            w[j] = next;
+            if (const int rc = launch_dequant(mats[i + j], next, SQ_F16, mats[i + j].C, 0, mats[i + j].R, s, /*raw=*/true)) return rc;
+            next += dense_bytes(mats[i + j]);
+        }
+        if (k)
+            if (const int rc = launch_mid_decoded(mats + i, k, w, x, x_dtype, ldx, y, y_dtype, ldy, T, next, s)) return rc;
+    }
+    return SQ_OK;
+}
+
+// Activation rows from which a stack with column orders is decoded and multiplied instead of reading x through its orders:
+// where the rows have tag streams, whose kernel takes up to eight rows at once, 11, or 17 if the decode is long (8 / 10 / 11 rows
+// there and here: 4608 x 3584 46 / 89 us and 43, 37888 x 3584 81 / 118 and 237).  Without, each four rows cost as much again,
+// twice that on long rows (4 / 5 / 8 rows there, and any of them here: 593 x 1984 15 / 23 / 28 us and 18, 16000 x 3584 54 / 91 /
+// 103 and 78, 3584 x 18944 193 / 242 / 384 and 95, at 2 rows 97; 37888 x 3584 at 8 / 9 rows 194 / 272 and 237 in the tile GEMM).
+static bool masked_gemm(const sq_matrix* mats, int n, int B) {
+    bool orders = false;
+    for (int i = 0; i < n; ++i) orders = orders || mats[i].perms;
+    if (!orders) return false;
+    if (small_uses_sums(mats, n)) return decoded_route(mats, n, B) ? B >= 11 : B >= 17 && mats[0].C % 64 == 0;
+    if (decoded_route(mats, n, B)) return B >= (mats[0].C > 8192 ? 3 : 5);
+    return B >= 9 && mats[0].C % 64 == 0;
+}
+
+bool small_takes_gemm_route(const sq_matrix* mats, int n, int B, const void* x, int64_t ldx) {
+    return masked_gemm(mats, n, B) && x_vec_ok(x, ldx, mats[0].C);
+}
+
+size_t small_gemm_route_workspace(const sq_matrix* mats, int n, int B) {
+    return masked_gemm(mats, n, B) ? gemm_workspace(mats, n, B) : 0;
+}
+
 static size_t gemm_workspace_beyond_small(const sq_matrix* mats, int n, int T);
 static size_t gemm_workspace_without_mid(const sq_matrix* mats, int n, int T);
 
@@ -229,7 +286,8 @@ size_t gemm_workspace(const sq_matrix* mats, int n, int T) {
 static size_t gemm_workspace_beyond_small(const sq_matrix* mats, int n, int T) {
     // (covers the other routes too: the size is asked for without knowing x)
     const size_t rest = gemm_workspace_without_mid(mats, n, T);
-    return mid_ok(mats, n, T) ? std::max(rest, mid_workspace(mats, n, T)) : rest;
+    if (mid_ok(mats, n, T)) return std::max(rest, mid_workspace(mats, n, T));
+    return decoded_route(mats, n, T) ? std::max(rest, decoded_workspace(mats, n, T)) : rest;
 }
 
 static size_t gemm_workspace_without_mid(const sq_matrix* mats, int n, int T) {
@@ -291,7 +349,7 @@ int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_
                 int64_t ldy, int T, void* ws, size_t ws_bytes, void* sums, hipStream_t s) {
     if (T <= SQ_SMALL_BMAX && !small_takes_gemm_route(mats, n, T, x, ldx))
         return launch_small(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, ws_bytes, sums, s);
-    if (mid_ok(mats, n, T) && x_vec_ok(x, ldx, mats[0].C)) return launch_mid(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, ws_bytes, s);
+    if (mid_ok(mats, n, T) && x_vec_ok(x, ldx, mats[0].C) && mid_x_ok(ldx, T)) return launch_mid(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, ws_bytes, s);
     if (T > SQ_SMALL_BMAX && T <= small_pass_limit(mats, n) && x_vec_ok(x, ldx, mats[0].C)) {
         // stacks that cannot go in one pass (pieces of different formats): a few passes of the decode-time kernel read the packed
         // tags a few times; decoding to fp16 first (below) writes and reads 8 to 16 times as many bytes once
@@ -319,6 +377,7 @@ int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_
     }
     if (gemm_workspace(mats, n, T) > ws_bytes)
         return fail(SQ_EWORKSPACE, "sq_linear_gemm: workspace %zu < %zu", ws_bytes, gemm_workspace(mats, n, T));
+    if (decoded_route(mats, n, T) && mid_x_ok(ldx, T)) return launch_decoded(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);
     if (big_route(mats, n, T)) {
         const int C = mats[0].C;
         const uint16_t* xh = (const uint16_t*)x;

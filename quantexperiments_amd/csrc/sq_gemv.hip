@@ -414,7 +414,7 @@ int launch_small(const sq_matrix* mats, int n, const void* x, int x_dtype, int64
         for (int k = j - i; k < GEMV_MAX_PIECES; ++k) a.p[k] = a.p[0];
         for (int b0 = 0; b0 < B;) {
             const int left = B - b0;
-            int nbt = left >= 4 ? 4 : left >= 2 ? 2 : 1;
+            int nbt = left >= 3 ? 4 : left;                          // (three rows: 16 us as four, 20 as two and one, 2048 x 2048)
             // fewer activation rows per pass when the registers or the workgroup width do not allow more
             while (nbt > 1 && (cfg_xw(m0.bits, m0.d, pl.S, nbt) > 192 || cfg_lb(m0.bits, m0.d, pl.S, nbt) < wpr * 64)) nbt >>= 1;
             const int lb = cfg_lb(m0.bits, m0.d, pl.S, nbt);

@@ -21,6 +21,10 @@
 //   tags        two rounds ahead; codewords PD steps ahead (one from LDS, three from L2 where the steps are short)
 //   grid        row blocks x ks slices of the rounds; with ks > 1 fp32 partial sums, added by mid_reduce_kernel
 //
+// D = 0: weights already decoded to fp16 (column orders, formats whose rows are not whole lane units).  The A operand is loaded
+// from there, up to seven steps ahead; step j of lane group g is columns 256 round + 32 j + 8 g .. + 7, so that the four lane groups
+// of a row read 64 neighbouring bytes.
+//
 // An X row of a stage is 4 S pieces of 16 bytes; piece c of row t sits at slot c ^ h(t), with h such that the 16 lanes of an
 // LDS clock (rows 0-3, 12-15 of one lane group with rows 4-11 of the next, and so on) fall into 16 different groups of four
 // banks.
@@ -30,12 +34,11 @@
 
 namespace sq {
 
-constexpr int MID_PIECES = 4;
 constexpr int MID_NW = 8;                    // waves per workgroup, two per SIMD
 
 struct MidPiece {
     sq_matrix m;
-    const uint32_t* tiled;       // tile-major copy of the tags or NULL
+    const void* w;               // D = 0: the decoded weights [R, C]; else the tile-major copy of the tags or NULL
     float* part;                 // ks > 1: fp32 [ks, T, R]
     int wg0;
 };
@@ -61,9 +64,12 @@ constexpr int mid_stage_bytes(int NT, int S) { return NT * 16 * S * 64; }
 
 template <int BITS, int D, int NT, int TW, int S, bool BF>
 __global__ __launch_bounds__(64 * MID_NW, 2) void mid_kernel(MidArgs a) {
-    constexpr int UD = unit_of<BITS>::UD, TPU = UD * 32 / BITS, CPS = 8 / D, SPR = TPU / CPS, UK = TPU * D, NST = SPR / S;
+    constexpr bool DENSE = D == 0;
+    constexpr int UD = DENSE ? 1 : unit_of<DENSE ? 16 : BITS>::UD, TPU = DENSE ? 1 : UD * 32 / (DENSE ? 1 : BITS);
+    constexpr int SPR = DENSE ? 8 : TPU / (8 / (DENSE ? 1 : D)), UK = DENSE ? 8 : TPU * D, UPR = DENSE ? 4 * SPR : 4, NST = SPR / S;
+    constexpr int GC = DENSE ? 8 : UK, JC = DENSE ? 32 : 8, UPS = DENSE ? 4 * S : 0;   // columns from lane group to group, from step to step; units per stage
     constexpr int ROWB = S * 64, STAGE = mid_stage_bytes(NT, S), NTH = 64 * MID_NW, PCS = (NT * 64 * S + NTH - 1) / NTH;
-    constexpr int PD = D == 8 && NT * TW < 24 ? 3 : 1, XB = NT <= 8 ? 2 : 1;   // steps that codewords and activations are fetched ahead of
+    constexpr int PD = DENSE ? (NT * TW <= 16 ? 7 : 3) : D == 8 && NT * TW < 24 ? 3 : 1, XB = NT <= 8 ? 2 : 1;   // steps that codewords and activations are fetched ahead of
     static_assert(SPR % S == 0 && SPR % (PD + 1) == 0 && (NST == 1 || NST % 2 == 0), "steps per round");
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lg = lane >> 4;
@@ -74,23 +80,25 @@ __global__ __launch_bounds__(64 * MID_NW, 2) void mid_kernel(MidArgs a) {
     const MidPiece& P = a.p[pi];
     const sq_matrix& m = P.m;
     const int w = (int)blockIdx.x - P.wg0, slice = w % a.ks, blk = w / a.ks;
-    const int NR = (a.U + 3) >> 2, NP = (NR + 1) >> 1;                       // rounds, and pairs of them: slices are whole pairs
+    const int NR = (a.U + UPR - 1) / UPR, NP = (NR + 1) >> 1;                       // rounds, and pairs of them: slices are whole pairs
     const int r0 = 2 * (int)((int64_t)NP * slice / a.ks), r1 = min(NR, 2 * (int)((int64_t)NP * (slice + 1) / a.ks));
     unsigned char* xbuf = smem + a.table_bytes;
 
     // ---- this wave's tiles (tiles past the last row repeat the last one and are not stored)
     const int ntiles = (m.R + 15) >> 4, tile0 = (blk * MID_NW + wave) * TW;
     // (byte offsets from a uniform base: one address register per load)
-    const uint32_t us = (P.tiled ? 16 * UD : UD) * 4;                        // bytes between two units of a row
-    const char* tags = reinterpret_cast<const char*>(P.tiled ? P.tiled : reinterpret_cast<const uint32_t*>(m.tags));
+    const bool tiled = !DENSE && P.w;
+    const uint32_t us = (tiled ? 16 * UD : UD) * 4;                          // bytes between two units of a row
+    const char* tags = reinterpret_cast<const char*>(P.w ? P.w : m.tags);
     uint32_t to[TW], bo[TW];
 #pragma unroll
     for (int i = 0; i < TW; ++i) {
         const int tile = min(tile0 + i, ntiles - 1), row = min(tile * 16 + li, m.R - 1);
-        to[i] = P.tiled ? ((uint32_t)tile * (uint32_t)a.U * 16u + (uint32_t)li) * (UD * 4) : (uint32_t)row * (uint32_t)m.W * 4u;
-        bo[i] = m.row_book ? (uint32_t)m.row_book[row] << (BITS + (D == 8 ? 4 : 3)) : 0u;
+        to[i] = DENSE ? (uint32_t)row * (uint32_t)m.C * 2u : tiled ? ((uint32_t)tile * (uint32_t)a.U * 16u + (uint32_t)li) * (UD * 4) : (uint32_t)row * (uint32_t)m.W * 4u;
+        bo[i] = !DENSE && m.row_book ? (uint32_t)m.row_book[row] << (BITS + (D == 8 ? 4 : 3)) : 0u;
     }
     auto load_tags = [&](int round, dwords<UD>* t) {
+        if (DENSE) return;
         const uint32_t u = (uint32_t)min(4 * round + lg, a.U - 1) * us;
 #pragma unroll
         for (int i = 0; i < TW; ++i) t[i] = load_unit<UD>(reinterpret_cast<const uint32_t*>(tags + (to[i] + u)));
@@ -102,20 +110,21 @@ __global__ __launch_bounds__(64 * MID_NW, 2) void mid_kernel(MidArgs a) {
 #pragma unroll
     for (int k = 0; k < PCS; ++k) {
         const int q = min(tid + NTH * k, NT * 64 * S - 1), t = q / (4 * S), c = q - t * (4 * S), g = c / S, j = c - g * S;
-        xg[k] = g;
-        xo[k] = ((uint32_t)min(t, a.T - 1) * (uint32_t)a.ldx + (uint32_t)(g * UK + j * 8)) * 2u;
+        xg[k] = DENSE ? j * 4 + g : g;
+        xo[k] = ((uint32_t)min(t, a.T - 1) * (uint32_t)a.ldx + (uint32_t)(g * GC + j * JC)) * 2u;
         xl[k] = (uint32_t)(t * ROWB + ((c ^ mid_swizzle<S>(t & 15)) << 4));
     }
     // columns past the row's end (the last round's missing units, rounds past the slice) are zeros; what is read in their
     // place is the row's last unit
     auto load_x = [&](u32x4* px, int round, int st) {
-        const int left = a.U - 1 - 4 * min(round, NR - 1);                   // the round's last unit
-        const char* base = reinterpret_cast<const char*>(a.x) + (int64_t)min(round, NR - 1) * (8 * UK) + st * (S * 16);
+        int left = a.U - 1 - UPR * min(round, NR - 1) - st * UPS;            // the stage's last unit; D = 0: < 0 if it is past the row
+        const char* base = reinterpret_cast<const char*>(a.x) + (int64_t)min(round, NR - 1) * (2 * UPR * UK) + st * (S * JC * 2);
+        if (DENSE && left < 0) base += left * (2 * UK), left = 0;
 #pragma unroll
         for (int k = 0; k < PCS; ++k) px[k] = *reinterpret_cast<const u32x4*>(base + (xo[k] - (uint32_t)(max(xg[k] - left, 0) * (UK * 2))));
     };
-    auto store_x = [&](const u32x4* px, int buf, int round) {
-        const int units = round < r1 ? a.U - 4 * round : 0;
+    auto store_x = [&](const u32x4* px, int buf, int round, int st) {
+        const int units = round < r1 ? a.U - UPR * round - st * UPS : 0;
 #pragma unroll
         for (int k = 0; k < PCS; ++k) {
             u32x4 v = px[k];
@@ -128,10 +137,12 @@ __global__ __launch_bounds__(64 * MID_NW, 2) void mid_kernel(MidArgs a) {
     const uint32_t xbase = (uint32_t)(li * ROWB + (((lg * S) ^ mid_swizzle<S>(li)) << 4));
 
     // ---- codewords of one step
-    auto gather = [&](u32x4* f, const dwords<UD>* t, int step) {
+    auto gather = [&](u32x4* f, const dwords<UD>* t, int round, int step) {
 #pragma unroll
         for (int i = 0; i < TW; ++i) {
-            if constexpr (D == 8) {
+            if constexpr (DENSE) {
+                f[i] = *reinterpret_cast<const u32x4*>(tags + (to[i] + (uint32_t)min(round * (UPR * UK) + step * JC + lg * GC, m.C - 8) * 2u));
+            } else if constexpr (D == 8) {
                 f[i] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(m.table) + ((unit_tag<BITS, UD>(t[i], step) << 4) + bo[i]));
             } else {
                 const u32x2 lo = *(const mma_lds_u32x2*)(uintptr_t)unit_lds_offset<BITS, UD, 3>(t[i], step * 2, bo[i]);
@@ -157,10 +168,10 @@ __global__ __launch_bounds__(64 * MID_NW, 2) void mid_kernel(MidArgs a) {
     load_tags(r0 + 1, tag[1]);
     load_x(px[1], NST > 1 ? r0 : r0 + 1, NST > 1 ? 1 : 0);
     if (D == 4) stage_table(m.table, a.table_bytes, smem);
-    store_x(px[0], 0, r0);
+    store_x(px[0], 0, r0, 0);
     __syncthreads();
 #pragma unroll
-    for (int s = 0; s < PD; ++s) gather(wf[s], tag[0], s);
+    for (int s = 0; s < PD; ++s) gather(wf[s], tag[0], r0, s);
     auto do_round = [&](auto parity, int round) {
         constexpr int P = decltype(parity)::value;
 #pragma unroll
@@ -179,13 +190,13 @@ __global__ __launch_bounds__(64 * MID_NW, 2) void mid_kernel(MidArgs a) {
             for (int j = 0; j < S; ++j) {
                 const int s = st * S + j;
                 __builtin_amdgcn_sched_barrier(0);
-                if (s + PD < SPR) gather(wf[(s + PD) % (PD + 1)], tag[P], s + PD);
-                else gather(wf[(s + PD) % (PD + 1)], tag[P ^ 1], s + PD - SPR);
+                if (s + PD < SPR) gather(wf[(s + PD) % (PD + 1)], tag[P], round, s + PD);
+                else gather(wf[(s + PD) % (PD + 1)], tag[P ^ 1], round + 1, s + PD - SPR);
                 if (s + PD == SPR - 1) load_tags(round + 2, tag[P]);         // this round's tags have all been used
                 if (XB == 1) read_x(xf[0], j);
                 else if (j + 1 < S) read_x(xf[(j + 1) & (XB - 1)], j + 1);
                 // the next stage's activations, in the middle of this one, where the other wave of the SIMD multiplies
-                if (j == S / 2 - 1) store_x(px[q ^ 1], q ^ 1, round + (st + 1) / NST);
+                if (j == S / 2 - 1) store_x(px[q ^ 1], q ^ 1, round + (st + 1) / NST, (st + 1) % NST);
 #pragma unroll
                 for (int n = 0; n < NT; ++n)
 #pragma unroll
@@ -259,9 +270,10 @@ int launch_mid_as(const MidArgs& a, int grid, hipStream_t s) {
 #define SQ_MID_CASE(NT_, TW_, S_) if (nt == NT_ && tw == TW_ && st == S_) return launch_mid_as<BITS, D, NT_, TW_, S_>(a, grid, s);
 template <int BITS, int D>
 int launch_mid_format(const MidArgs& a, int nt, int tw, int st, int grid, hipStream_t s) {
+    if constexpr (D == 0) { SQ_MID_CASE(1, 2, 4) SQ_MID_CASE(1, 1, 4) }
     SQ_MID_CASE(3, 2, 4) SQ_MID_CASE(3, 1, 4) SQ_MID_CASE(5, 2, 4) SQ_MID_CASE(5, 1, 4) SQ_MID_CASE(8, 2, 4) SQ_MID_CASE(8, 1, 4)
     SQ_MID_CASE(12, 2, 2) SQ_MID_CASE(12, 1, 2) SQ_MID_CASE(16, 1, 2)
-    if constexpr (D == 8) {
+    if constexpr (D != 4) {
         SQ_MID_CASE(16, 2, 2)
     } else {
         SQ_MID_CASE(3, 2, 2) SQ_MID_CASE(3, 1, 2) SQ_MID_CASE(5, 2, 2) SQ_MID_CASE(5, 1, 2) SQ_MID_CASE(8, 2, 2) SQ_MID_CASE(8, 1, 2)

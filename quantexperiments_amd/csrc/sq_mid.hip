@@ -9,6 +9,7 @@ int launch_mid_b16d8(const MidArgs&, int, int, int, int, hipStream_t);
 int launch_mid_b12d4(const MidArgs&, int, int, int, int, hipStream_t);
 int launch_mid_b10d4(const MidArgs&, int, int, int, int, hipStream_t);
 int launch_mid_b8d4(const MidArgs&, int, int, int, int, hipStream_t);
+int launch_mid_dense(const MidArgs&, int, int, int, int, hipStream_t);
 
 // y[t, y_off + r] = row_scale[r] * sum over the slices of part[slice][t][r], four rows of one token per thread
 __global__ __launch_bounds__(256) void mid_reduce_kernel(MidArgs a) {
@@ -101,14 +102,14 @@ size_t mid_workspace(const sq_matrix* mats, int n, int T) {
     return need;
 }
 
-static int launch_mid_rows(const sq_matrix* mats, int n, const MidPlan& pl, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype,
+static int launch_mid_rows(const sq_matrix* mats, int n, const MidPlan& pl, const void* const* dense, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype,
                            int64_t ldy, int T, void* ws, hipStream_t s) {
     MidArgs a{};
     const sq_matrix& m0 = mats[0];
     a.n = n;
     a.x = (const uint16_t*)x; a.ldx = ldx; a.y = y; a.ldy = ldy; a.T = T; a.x_dtype = x_dtype; a.y_dtype = y_dtype;
-    a.U = mid_units(m0); a.ks = pl.ks;
-    a.table_bytes = m0.d == 4 ? (m0.G << m0.bits) * 8 : 0;
+    a.U = dense ? m0.C / 8 : mid_units(m0); a.ks = pl.ks;
+    a.table_bytes = !dense && m0.d == 4 ? (m0.G << m0.bits) * 8 : 0;
     int wg = 0;
     int64_t quads = 0;
     char* part = (char*)ws;
@@ -116,7 +117,7 @@ static int launch_mid_rows(const sq_matrix* mats, int n, const MidPlan& pl, cons
         MidPiece& P = a.p[i];
         const sq_matrix& m = mats[i];
         P.m = m;
-        P.tiled = m.stream && tiled_format_ok(m.R, m.W, m.C, m.d, m.bits) && ((uintptr_t)m.stream & 15) == 0 ? (const uint32_t*)m.stream : nullptr;
+        P.w = dense ? dense[i] : m.stream && tiled_format_ok(m.R, m.W, m.C, m.d, m.bits) && ((uintptr_t)m.stream & 15) == 0 ? (const void*)m.stream : nullptr;
         P.part = (float*)part;
         part += mid_part_bytes(m, T, pl.ks);
         P.wg0 = wg;
@@ -124,7 +125,8 @@ static int launch_mid_rows(const sq_matrix* mats, int n, const MidPlan& pl, cons
         quads += (int64_t)T * ((m.R + 3) / 4);
     }
     int rc = SQ_EUNSUPPORTED;
-    if (m0.d == 8) rc = launch_mid_b16d8(a, pl.nt, pl.tw, pl.st, wg, s);
+    if (dense) rc = launch_mid_dense(a, pl.nt, pl.tw, pl.st, wg, s);
+    else if (m0.d == 8) rc = launch_mid_b16d8(a, pl.nt, pl.tw, pl.st, wg, s);
     else if (m0.bits == 12) rc = launch_mid_b12d4(a, pl.nt, pl.tw, pl.st, wg, s);
     else if (m0.bits == 10) rc = launch_mid_b10d4(a, pl.nt, pl.tw, pl.st, wg, s);
     else if (m0.bits == 8) rc = launch_mid_b8d4(a, pl.nt, pl.tw, pl.st, wg, s);
@@ -133,13 +135,46 @@ static int launch_mid_rows(const sq_matrix* mats, int n, const MidPlan& pl, cons
     return check_launch("sq_linear_gemm(mid reduce)");
 }
 
+// For decoded weights: one tile of rows per wave, so that small stacks spread (593 x 1984 at 16 rows: 17 us with the decode, 22
+// with two), K slices of 256 columns at least, up to eight (3584 x 18944 at 64 rows: 99 us with the decode, 119 in four slices,
+// 111 in nine).
+static MidPlan mid_dense_plan(const sq_matrix* mats, int n, int T, int cus) {
+    MidPlan p{0, 1, 4, 1};
+    const int sizes[] = {1, 3, 5, 8, 12, 16};
+    for (int nt : sizes) if (T <= nt * 16) { p.nt = nt; break; }
+    if (p.nt > 8) p.st = 2;
+    int64_t blocks = 0;
+    for (int i = 0; i < n; ++i) blocks += (mats[i].R + 16 * MID_NW - 1) / (16 * MID_NW);
+    p.ks = (int)std::max<int64_t>(1, std::min<int64_t>({cus / std::max<int64_t>(blocks, 1), 8, mats[0].C / 256}));
+    return p;
+}
+
+bool mid_dense_ok(const sq_matrix* mats, int n, int T) {
+    if (n < 1 || n > MID_PIECES || T < 1 || T > 256) return false;
+    for (int i = 0; i < n; ++i)
+        if (mats[i].R <= 0 || mats[i].C != mats[0].C || mats[i].C % 8 || ((int64_t)mats[i].R + 16) * mats[i].C * 2 >= ((int64_t)1 << 32)) return false;
+    return true;
+}
+
+size_t mid_dense_workspace(const sq_matrix* mats, int n, int T) {
+    const MidPlan p = mid_dense_plan(mats, n, T, device_cus());
+    size_t need = 0;
+    for (int i = 0; i < n; ++i) need += mid_part_bytes(mats[i], T, p.ks);
+    return need;
+}
+
+int launch_mid_decoded(const sq_matrix* mats, int n, const void* const* w, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T,
+                       void* ws, hipStream_t s) {
+    return launch_mid_rows(mats, n, mid_dense_plan(mats, n, T, device_cus()), w, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);
+}
+
 int launch_mid(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws,
                size_t ws_bytes, hipStream_t s) {
     if (mid_workspace(mats, n, T) > ws_bytes) return fail(SQ_EWORKSPACE, "sq_linear_gemm: workspace %zu < %zu", ws_bytes, mid_workspace(mats, n, T));
     const int rows = mid_rows(mats, n, T);
     const MidPlan pl = mid_plan(mats, n, rows, device_cus());
     for (int t = 0; t < T; t += rows) {
-        const int rc = launch_mid_rows(mats, n, pl, (const char*)x + (size_t)t * ldx * 2, x_dtype, ldx,
+        const int rc = launch_mid_rows(mats, n, pl, nullptr, (const char*)x + (size_t)t * ldx * 2, x_dtype, ldx,
                                        (char*)y + (size_t)t * ldy * (y_dtype == SQ_F32 ? 4 : 2), y_dtype, ldy, std::min(rows, T - t), ws, s);
         if (rc) return rc;
     }

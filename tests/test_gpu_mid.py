@@ -1,5 +1,6 @@
 """Products of 33 to 384 activation rows in one pass over the tags: edges of the tiles of rows and activation rows, a last round
-with missing units, odd numbers of rounds, K slices, stacks, several codebooks, two tiles of rows per wave, two parts of rows."""
+with missing units, odd numbers of rounds, K slices, stacks, several codebooks, two tiles of rows per wave, two parts of rows; and
+of 3 to 256 rows with weights decoded first."""
 
 import numpy as np
 import pytest
@@ -35,3 +36,25 @@ def test_one_pass_matches_oracle(case, dtype, stream):
     linear_gemm(lins, x.cuda(), lowp)
     assert torch.equal(lowp, y.to(dtype))
     assert np.isfinite(lowp.float().cpu().numpy()).all()
+
+
+DECODED = [  # rows of the stack's pieces, C, d, bits, G, M, T: column orders, rows of broken lane units, stages past the row's end
+    ((1,), 8, 8, 16, 1, 1, 33), ((129, 1, 300), 1984, 8, 16, 1, 16, 15), ((16,), 1984, 8, 16, 1, 16, 256), ((130,), 72, 8, 16, 1, 3, 5),
+    ((70, 50), 1000, 4, 12, 1, 1, 48), ((50, 16), 264, 4, 10, 4, 1, 193), ((257,), 520, 4, 8, 1, 2, 128), ((40, 40, 40, 40, 7), 512, 8, 16, 1, 2, 17),
+    ((33,), 9216, 8, 16, 1, 16, 3), ((12,), 200, 2, 5, 3, 1, 81), ((3584,), 776, 8, 16, 1, 1, 100),
+]
+
+
+@pytest.mark.parametrize("case", DECODED, ids=lambda c: "x".join(map(str, c)))
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+def test_decoded_weights_match_oracle(case, dtype):
+    rows, C, d, bits, G, M, T = case
+    ss = [synth(R, C, d, bits, G, M, seed=R + T) for R in rows]
+    lins = [to_device(s) for s in ss]
+    x = torch.zeros(T, C + 8, dtype=dtype)
+    x[:, :C] = rand_x(T, C, dtype, seed=T)
+    xd = x.cuda()[:, :C]
+    ref = torch.cat([xd.double() @ torch.from_numpy(s.decode()).cuda().double().T for s in ss], dim=1)
+    y = torch.empty(T, sum(rows), dtype=torch.float32, device="cuda")
+    linear_gemm(lins, xd, y)
+    assert rel_max_err(y.cpu().numpy(), ref.cpu().numpy()) < 1e-3
