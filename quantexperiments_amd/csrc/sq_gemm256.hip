@@ -1,17 +1,20 @@
 // Large-tile fp16 GEMM for prefill: Y[T, R] = X[T, C] . W[R, C]^T, fp32 accumulate, optional row scale.
 //
-// Workgroup tile 256 tokens x 256 weight rows, 4 waves in 2 x 2, each a 128 x 128 tile of sixteen v_mfma_f32_32x32x16_f16
-// accumulators (all 256 accumulator registers), one wave per SIMD.  Both operands are K-contiguous fp16 in memory.  The K
-// loop moves in slabs of 64 columns; a slab of ONE operand (256 rows x 128 bytes = 32 KB, whole 128-byte lines: half-line
-// requests get 10.5 TB/s out of L2 over the chip, whole lines 15.2 TB/s) is copied from global memory straight into LDS
-// (global_load_lds_dwordx4: no staging registers) into a ring of five 32 KB slots.  What a lone wave per SIMD needs is that
-// nothing in its instruction stream waits:
+// Workgroup tile 256, 192 or 128 tokens x 256 weight rows (64 MT x 256, chosen by gemm256_plan), 4 waves in 2 x 2, each a
+// 32 MT x 128 tile of v_mfma_f32_32x32x16_f16 accumulators (MT = 4: all 256 accumulator registers), one wave per SIMD.  Both
+// operands are K-contiguous fp16 in memory.  The K loop moves in slabs of 64 columns; a slab of ONE operand (rows of 128 bytes,
+// whole 128-byte lines: half-line requests get 10.5 TB/s out of L2 over the chip, whole lines 15.2 TB/s) is copied from global
+// memory straight into LDS (global_load_lds_dwordx4: no staging registers) into a ring of slots of that operand.  What a lone
+// wave per SIMD needs is that nothing in its instruction stream waits:
 //   * fragments are read one 16-column step ahead of their matrix instructions, one read behind each of the first ones;
 //   * one barrier per slab, two matrix instructions into the slab's last step, when its last fragments have arrived: it
 //     frees the slab's two slots and says that the next slab is complete;
-//   * the slots it frees take W of slab s + 2 at once, behind the reads of the next slab's first fragments, and X of
-//     slab s + 3 during the following steps, so W (the operand with the shorter lead) has a whole slab's time to arrive
-//     (issued over the first two steps of the next slab instead, 8192^3 ran at 1.26 instead of 1.29 PFLOP/s).
+//   * the slots it frees take one operand's slab at once, behind the reads of the next slab's first fragments, and a slab of the
+//     other during the following steps (issued over the first two steps of the next slab instead, 8192^3 ran at 1.26 instead
+//     of 1.29 PFLOP/s).
+// MT = 4 and 3: three W slots, two X slots: W, which comes from memory where X stays in L2, has one to two slabs' time to
+// arrive.  MT = 2, whose slabs take half as long: three W and four X slots, two to three slabs' time (with two and three:
+// 333 x 3584 x 18944 in four 89 us, now 77; 1024 x 7168 x 5120 91 and 81).
 // Eight waves of 128 x 64 (two per SIMD) ran at 1.15 PFLOP/s on 8192^3, in one schedule or as two groups taking turns at
 // matrix and memory phases, with 67 percent of the matrix cores' time used at 1.70 GHz; this one uses 83 percent of it at
 // 1.52 GHz (the chip's power limit: on zeros it reaches 1.71 PFLOP/s) and reads a third less from LDS.  16x16x32
@@ -30,9 +33,13 @@
 
 namespace sq {
 
-constexpr int G_BM = 256, G_BN = 256, G_BK = 64, G_WAVES = 4;
-constexpr int G_SLOTS = 5, G_SLOT_BYTES = 256 * G_BK * 2;        // 5 x 32 KB = all 160 KB of LDS
-constexpr int G_SUPER_T = 8;                 // token tiles that are walked together, see below
+constexpr int G_BN = 256, G_BK = 64, G_WAVES = 4;
+constexpr int G_W_SLOT = G_BN * G_BK * 2;
+constexpr int gemm256_tokens(int mt) { return 64 * mt; }                           // token rows of a tile
+constexpr int gemm256_x_slots(int mt) { return mt == 2 ? 4 : 2; }
+constexpr int gemm256_w_slots(int) { return 3; }
+constexpr int gemm256_lds(int mt) { return gemm256_x_slots(mt) * gemm256_tokens(mt) * G_BK * 2 + gemm256_w_slots(mt) * G_W_SLOT; }     // 160, 144, 160 KB
+constexpr int gemm256_super(int mt) { return 32 / mt; }       // token tiles (about 2048 rows) that are walked together, see below
 
 struct Gemm256Args {
     const uint16_t* x;        // fp16 [T, C], row stride ldx
@@ -45,18 +52,18 @@ struct Gemm256Args {
     // The last round of tiles rarely fills the chip (592 tiles on 256 CUs: 2 full rounds and 80 tiles).  Tiles
     // [0, main_tiles) are multiplied whole; each of the remaining tail tiles is split over kt workgroups, each
     // taking the slabs [kz nk / kt, (kz + 1) nk / kt) and leaving an unscaled fp32 partial tile in
-    // part[(tail tile * kt + kz)][256][256] for gemm256_reduce_kernel.
+    // part[(tail tile * kt + kz)][token rows of a tile][256] for gemm256_reduce_kernel.
     int main_tiles, kt;
     float* part;
 };
 
-// Tile numbers walk super-columns of up to G_SUPER_T token tiles, weight tile after weight tile: consecutive tiles, which
+// Tile numbers walk super-columns of up to `super` token tiles, weight tile after weight tile: consecutive tiles, which
 // run on one XCD at the same time, then share both operands' slabs in its L2 (8192^3, 32 token tiles: 990 us in one column,
 // 900 us in columns of 8).
-__host__ __device__ __forceinline__ void gemm256_tile(int tile, int tiles_t, int tiles_r, int* bt, int* br) {
-    const int full = tiles_r * G_SUPER_T, g = tile / full, l = tile - g * full;
-    const int w = tiles_t - g * G_SUPER_T < G_SUPER_T ? tiles_t - g * G_SUPER_T : G_SUPER_T;
-    *bt = g * G_SUPER_T + l % w;
+__host__ __device__ __forceinline__ void gemm256_tile(int tile, int tiles_t, int tiles_r, int super, int* bt, int* br) {
+    const int full = tiles_r * super, g = tile / full, l = tile - g * full;
+    const int w = tiles_t - g * super < super ? tiles_t - g * super : super;
+    *bt = g * super + l % w;
     *br = l / w;
 }
 
@@ -71,15 +78,15 @@ __device__ __forceinline__ float gemm256_scale(const Gemm256Scales& s, int r) {
     return h2f(p[at]);
 }
 
-constexpr int G_EP_PITCH = 128 * 2 + 16;     // bytes per token row of a wave's 128 x 128 output tile in LDS
-constexpr int G_EP_SCALES = 4 * 128 * G_EP_PITCH;    // behind them: the tile's 256 row scales in fp32
+constexpr int G_EP_PITCH = 128 * 2 + 16;     // bytes per token row of a wave's 32 MT x 128 output tile in LDS
 
 // s_waitcnt immediate that waits until at most n vector-memory operations are outstanding and leaves the
 // other counters alone (gfx9 encoding: vmcnt in bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8)
 constexpr int vmcnt_only(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
 
 // EP: SQ_F16 / SQ_BF16 = results of that type whose rows allow 16-byte stores, SQ_F32 = any type, element by element
-template <int EP>
+// MT: blocks of 32 token rows a wave holds, 64 MT rows a tile
+template <int EP, int MT>
 __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -101,13 +108,14 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a)
         nparts = a.kt;
     }
     int bt, br;
-    gemm256_tile(tile, a.tiles_t, a.tiles_r, &bt, &br);
-    const int t0 = bt * G_BM, r0 = br * G_BN;
-    const int wm = (wave >> 1) * 128, wn = (wave & 1) * 128;
+    gemm256_tile(tile, a.tiles_t, a.tiles_r, gemm256_super(MT), &bt, &br);
+    constexpr int BM = gemm256_tokens(MT), XC = 2 * MT, X_SLOT = BM * G_BK * 2, NM = 4 * MT;     // XC: copies a wave makes of an X slab (of a W slab: 8); NM: products of a step
+    const int t0 = bt * BM, r0 = br * G_BN;
+    const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * 128;
 
-    float16v acc[4][4];                      // [token block][weight-row block]
+    float16v acc[MT][4];                     // [token block][weight-row block]
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -115,20 +123,29 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a)
 
     // Copies.  One global_load_lds_dwordx4 fills 1 KB = 8 LDS rows in lane order, so lane s lands in row
     // s >> 3, slot s & 7 of its block and therefore fetches the piece the swizzle puts there.  Wave w copies
-    // rows 64 w .. 64 w + 63 of an operand slab: 8 instructions.  Global addresses are a uniform base (advanced
-    // per slab) plus per-lane 32-bit byte offsets computed once; rows past the matrix edge re-read the last
-    // row (their outputs are never stored).  Half h = 2 s is X of slab s, h = 2 s + 1 is W of slab s; half h
-    // lives in ring slot h % 5; slabs past the last one re-read the last.
+    // rows 64 w .. 64 w + 63 of a W slab (8 instructions) and a quarter of the X slab's rows.  Global addresses are a
+    // uniform base (advanced per slab) plus per-lane 32-bit byte offsets computed once; rows past the matrix edge re-read
+    // the last row (their outputs are never stored).  One operand is early (E slots, the copies of slab s + E - 1 go out during
+    // the first steps of slab s), the other late (L = E - 1 slots, slab s + L goes out behind the barrier of slab s); slabs
+    // past the last one re-read the last.
+    constexpr bool XE = gemm256_x_slots(MT) > gemm256_w_slots(MT);        // X is the early one
+    constexpr int E = XE ? gemm256_x_slots(MT) : gemm256_w_slots(MT), L = E - 1, EC = XE ? XC : 8, LC = XE ? 8 : XC;
+    static_assert(L == (XE ? gemm256_w_slots(MT) : gemm256_x_slots(MT)), "the waits below count on it");
+    constexpr int W_AT = gemm256_x_slots(MT) * X_SLOT;
+    constexpr int AHEAD = (E - 2) * EC + (L - 2) * LC;                    // copies that may be on their way when slab s + 1 has to be there
     const int lrow = lane >> 3, slot = lane & 7;
-    uint32_t xo[8], wo[8];
+    uint32_t xo[XC], wo[8];
+#pragma unroll
+    for (int j = 0; j < XC; ++j) {
+        const int row = wave * (BM / 4) + j * 8 + lrow;
+        const int t = t0 + row < a.T ? row : a.T - 1 - t0;
+        xo[j] = (uint32_t)(t * (int)a.ldx + (slot ^ ((row >> 1) & 7)) * 8) * 2u;
+    }
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         const int row = wave * 64 + j * 8 + lrow;
-        const int c = slot ^ ((row >> 1) & 7);
-        const int t = t0 + row < a.T ? row : a.T - 1 - t0;
         const int r = r0 + row < a.R ? row : a.R - 1 - r0;
-        xo[j] = (uint32_t)(t * (int)a.ldx + c * 8) * 2u;
-        wo[j] = (uint32_t)(r * (int)a.ldw + c * 8) * 2u;
+        wo[j] = (uint32_t)(r * (int)a.ldw + (slot ^ ((row >> 1) & 7)) * 8) * 2u;
     }
     const int nk_all = a.C / G_BK, k_begin = (int)((int64_t)kz * nk_all / nparts);
     const int nk = (int)((int64_t)(kz + 1) * nk_all / nparts) - k_begin;
@@ -136,85 +153,94 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a)
     const char* wt = reinterpret_cast<const char*>(a.w + (int64_t)r0 * a.ldw + (int64_t)k_begin * G_BK);
     typedef const __attribute__((address_space(1))) void* gptr_t;
     typedef __attribute__((address_space(3))) void* lptr_t;
-    auto copy = [&](const char* from, uint32_t off, int to, int j) {
-        __builtin_amdgcn_global_load_lds((gptr_t)(from + off), (lptr_t)(smem + to * G_SLOT_BYTES + wave * 8192 + j * 1024), 16, 0, 0);
+    auto copy = [&](const char* from, uint32_t off, int to) {
+        __builtin_amdgcn_global_load_lds((gptr_t)(from + off), (lptr_t)(smem + to), 16, 0, 0);
     };
+    auto copy_x = [&](const char* from, int sl, int j) { copy(from, xo[j], sl * X_SLOT + wave * (X_SLOT / 4) + j * 1024); };
+    auto copy_w = [&](const char* from, int sl, int j) { copy(from, wo[j], W_AT + sl * G_W_SLOT + wave * 8192 + j * 1024); };
+    auto slab = [&](int q) { return (q < nk ? q : nk - 1) * (G_BK * 2); };
+    auto copy_early = [&](int q, int sl, int j) { if constexpr (XE) copy_x(xt + slab(q), sl, j); else copy_w(wt + slab(q), sl, j); };
+    auto copy_late = [&](int q, int sl, int j) { if constexpr (XE) copy_w(wt + slab(q), sl, j); else copy_x(xt + slab(q), sl, j); };
 
     // Fragments.  A lane reads row (lane & 31) + 32 i of its wave's rows, piece 2 kk + (lane >> 5); the swizzle
     // term depends on the row modulo 16 only and the column step kk only flips bits 5-6 of the offset, so one
     // offset plus compile-time multiples of 32 rows (4096 bytes) covers all reads of a slab.
-    half8v fx[2][4], fw[2][4];
+    half8v fx[2][MT], fw[2][4];
     const uint32_t foff = (uint32_t)((lane & 31) * 128 + (((lane >> 5) ^ ((lane >> 1) & 7)) << 4));
     auto read_x = [&](int set, int kk, int sl, int i) {
-        fx[set][i] = *reinterpret_cast<const half8v*>(smem + sl * G_SLOT_BYTES + wm * 128 + i * 4096 + (foff ^ (uint32_t)(kk << 5)));
+        fx[set][i] = *reinterpret_cast<const half8v*>(smem + sl * X_SLOT + wm * 128 + i * 4096 + (foff ^ (uint32_t)(kk << 5)));
     };
     auto read_w = [&](int set, int kk, int sl, int j) {
-        fw[set][j] = *reinterpret_cast<const half8v*>(smem + sl * G_SLOT_BYTES + wn * 128 + j * 4096 + (foff ^ (uint32_t)(kk << 5)));
+        fw[set][j] = *reinterpret_cast<const half8v*>(smem + W_AT + sl * G_W_SLOT + wn * 128 + j * 4096 + (foff ^ (uint32_t)(kk << 5)));
     };
     auto mma = [&](int set, int n) {
         acc[n >> 2][n & 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fw[set][n & 3], fx[set][n >> 2], acc[n >> 2][n & 3], 0, 0, 0);
     };
     // the accumulators stay in their registers before and behind the loop (without this the compiler copies all 256 into the
     // other half of the register file at the loop's end, spills, and a launch that needs scratch memory takes 7 us longer)
-#define SQ_PIN() _Pragma("unroll") for (int i = 0; i < 4; ++i) { asm volatile("" : "+a"(acc[i][0]), "+a"(acc[i][1]), "+a"(acc[i][2]), "+a"(acc[i][3])); }
+#define SQ_PIN() _Pragma("unroll") for (int i = 0; i < MT; ++i) { asm volatile("" : "+a"(acc[i][0]), "+a"(acc[i][1]), "+a"(acc[i][2]), "+a"(acc[i][3])); }
 #define SQ_SB() __builtin_amdgcn_sched_barrier(0)
-    // one 16-column step: 16 matrix instructions on `set`, the next step's fragments behind the first of them, up to
-    // three copies behind the others
-    auto step = [&](int set, int kk, int sx, int sw, auto c0, auto c1, auto c2) {
+    // one 16-column step: NM matrix instructions on `set`, the next step's fragments behind the first of them, copies [c0, c1)
+    // of the early operand behind the others
+    auto step = [&](int set, int kk, int sx, int sw, int q, int to, int c0, int c1) {
         mma(set, 0); SQ_SB();
         read_x(set ^ 1, kk, sx, 0); read_w(set ^ 1, kk, sw, 0); SQ_SB();
 #pragma unroll
         for (int i = 1; i < 4; ++i) { mma(set, i); SQ_SB(); read_w(set ^ 1, kk, sw, i); SQ_SB(); }
 #pragma unroll
-        for (int i = 1; i < 4; ++i) { mma(set, 3 + i); SQ_SB(); read_x(set ^ 1, kk, sx, i); SQ_SB(); }
-        mma(set, 7); SQ_SB(); c0(); SQ_SB();
-        mma(set, 8); mma(set, 9); SQ_SB(); c1(); SQ_SB();
-        mma(set, 10); mma(set, 11); SQ_SB(); c2(); SQ_SB();
-        mma(set, 12); mma(set, 13); mma(set, 14); mma(set, 15); SQ_SB();
+        for (int i = 1; i < MT; ++i) { mma(set, 3 + i); SQ_SB(); read_x(set ^ 1, kk, sx, i); SQ_SB(); }
+#pragma unroll
+        for (int n = MT + 3, c = c0; n < NM; ++n) {
+            mma(set, n);
+            if (c < c1 && (MT == 2 || ((n - MT - 3) & 1) == 0)) { SQ_SB(); copy_early(q, to, c); ++c; SQ_SB(); }
+        }
+        SQ_SB();
     };
 
 #pragma unroll
-    for (int j = 0; j < 8; ++j) copy(xt, xo[j], 0, j);
+    for (int q = 0; q < E - 1; ++q) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) copy(wt, wo[j], 1, j);
-    const int slab1 = nk > 1 ? G_BK * 2 : 0;
+        for (int j = 0; j < EC; ++j) copy_early(q, q, j);
+        if (q == L - 1) break;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) copy(xt + slab1, xo[j], 2, j);
-    __builtin_amdgcn_s_waitcnt(vmcnt_only(8));
+        for (int j = 0; j < LC; ++j) copy_late(q, q, j);
+    }
+    __builtin_amdgcn_s_waitcnt(vmcnt_only(AHEAD));
     SQ_SB(); __builtin_amdgcn_s_barrier(); SQ_SB();
 #pragma unroll
-    for (int i = 0; i < 4; ++i) { read_x(0, 0, 0, i); read_w(0, 0, 1, i); }
+    for (int i = 0; i < MT; ++i) read_x(0, 0, 0, i);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) copy(wt + slab1, wo[j], 3, j);
-    int sx = 0, sw = 1;                      // ring slots of the slab being multiplied
+    for (int i = 0; i < 4; ++i) read_w(0, 0, 0, i);
+#pragma unroll
+    for (int j = 0; j < LC; ++j) copy_late(L - 1, L - 1, j);
+    int se = 0, sl = 0;                      // slots of the slab being multiplied
     SQ_PIN();
 #pragma unroll 1
     for (int s = 0; s < nk; ++s) {
-        auto wrap = [](int v) { return v >= G_SLOTS ? v - G_SLOTS : v; };
-        const int lx = wrap(sx + 4), nx = wrap(sx + 2), nw = wrap(sx + 3), lw = sx;      // X of s + 2; X, W of s + 1; W of s + 2
-        const int ahead = (s + 2 < nk ? s + 2 : nk - 1) * (G_BK * 2);
-        const char* xp = xt + ahead;
-        const char* wp = wt + ahead;
-        auto none = [] {};
-        step(0, 1, sx, sw, [&] { copy(xp, xo[0], lx, 0); }, [&] { copy(xp, xo[1], lx, 1); }, [&] { copy(xp, xo[2], lx, 2); });
-        step(1, 2, sx, sw, [&] { copy(xp, xo[3], lx, 3); }, [&] { copy(xp, xo[4], lx, 4); }, [&] { copy(xp, xo[5], lx, 5); });
-        step(0, 3, sx, sw, [&] { copy(xp, xo[6], lx, 6); }, [&] { copy(xp, xo[7], lx, 7); }, none);
-        // last step: this wave's copies of slab s + 1 are waited for (the eight X copies of slab s + 2 stay in flight), then
-        // the barrier: everybody's have landed and everybody has read slab s to the end
+        const int ne = se == E - 1 ? 0 : se + 1, nl = sl == L - 1 ? 0 : sl + 1, to = se == 0 ? E - 1 : se - 1;
+        const int sx = XE ? se : sl, sw = XE ? sl : se, nx = XE ? ne : nl, nw = XE ? nl : ne;
+        constexpr int C1 = (EC + 2) / 3, C2 = 2 * C1 < EC ? 2 * C1 : EC;
+        step(0, 1, sx, sw, s + E - 1, to, 0, C1);
+        step(1, 2, sx, sw, s + E - 1, to, C1, C2);
+        step(0, 3, sx, sw, s + E - 1, to, C2, EC);
+        // last step: this wave's copies of slab s + 1 are waited for (those of later slabs stay in flight), then the
+        // barrier: everybody's have landed and everybody has read slab s to the end
         mma(1, 0); SQ_SB(); mma(1, 1); SQ_SB();
-        __builtin_amdgcn_s_waitcnt(vmcnt_only(8)); SQ_SB();
+        __builtin_amdgcn_s_waitcnt(vmcnt_only(AHEAD)); SQ_SB();
         __builtin_amdgcn_s_barrier(); SQ_SB();
-        read_x(0, 0, nx, 0); read_w(0, 0, nw, 0); SQ_SB(); mma(1, 2); SQ_SB();
-        read_w(0, 0, nw, 1); copy(wp, wo[0], lw, 0); SQ_SB(); mma(1, 3); SQ_SB();
-        read_w(0, 0, nw, 2); copy(wp, wo[1], lw, 1); SQ_SB(); mma(1, 4); SQ_SB();
-        read_w(0, 0, nw, 3); copy(wp, wo[2], lw, 2); SQ_SB(); mma(1, 5); SQ_SB();
-        read_x(0, 0, nx, 1); copy(wp, wo[3], lw, 3); SQ_SB(); mma(1, 6); SQ_SB();
-        read_x(0, 0, nx, 2); copy(wp, wo[4], lw, 4); SQ_SB(); mma(1, 7); SQ_SB();
-        read_x(0, 0, nx, 3); copy(wp, wo[5], lw, 5); SQ_SB(); mma(1, 8); SQ_SB();
-        copy(wp, wo[6], lw, 6); SQ_SB(); mma(1, 9); SQ_SB();
-        copy(wp, wo[7], lw, 7); SQ_SB(); mma(1, 10); SQ_SB();
-        mma(1, 11); mma(1, 12); mma(1, 13); mma(1, 14); mma(1, 15); SQ_SB();
-        sx = nx; sw = nw;
+        read_x(0, 0, nx, 0); read_w(0, 0, nw, 0); SQ_SB();
+#pragma unroll
+        for (int n = 2, c = 0; n < NM; ++n) {
+            mma(1, n); SQ_SB();
+            if (n < 5) read_w(0, 0, nw, n - 1);
+            else if (n < 4 + MT) read_x(0, 0, nx, n - 4);
+            // the copies of the late operand, one behind each product; in the six places of MT = 2 some of the eight go in pairs
+#pragma unroll
+            for (int k = 0; k < (MT == 2 && (n == 5 || n == 6) ? 2 : 1); ++k)
+                if (c < LC) { copy_late(s + L, sl, c); ++c; }
+            SQ_SB();
+        }
+        se = ne; sl = nl;
     }
     SQ_PIN();
 #undef SQ_SB
@@ -223,22 +249,22 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a)
     __syncthreads();                         // every wave is done with the operand ring, and no copy is on its way into it
 
     // Results leave column of registers after column of registers.  A split tile's go to its partial tile as they are.  16-bit
-    // ones go through LDS: every wave lays its 128 x 128 tile out token-major (8 bytes per write) and stores it in 16-byte
+    // ones go through LDS: every wave lays its 32 MT x 128 tile out token-major (8 bytes per write) and stores it in 16-byte
     // pieces, 256 contiguous bytes per token (2-byte stores straight from the accumulators cost 49 us of a 376 us product of
     // a 2048 x 18944 output).
     const int half4 = 4 * (lane >> 5), tok = lane & 31;
-    float* scales = reinterpret_cast<float*>(smem + G_EP_SCALES);
+    float* scales = reinterpret_cast<float*>(smem + 2 * BM * G_EP_PITCH);        // behind the four waves' tiles
     scales[tid] = gemm256_scale(a.sc, r0 + tid < a.R ? r0 + tid : a.R - 1);
     __syncthreads();
-    float* part = a.part + ((int64_t)(tile - a.main_tiles) * a.kt + kz) * (G_BM * G_BN);
-    unsigned char* my = smem + wave * (128 * G_EP_PITCH);
+    float* part = a.part + ((int64_t)(tile - a.main_tiles) * a.kt + kz) * (BM * G_BN);
+    unsigned char* my = smem + wave * (BM / 2 * G_EP_PITCH);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         float4v sc[4];
 #pragma unroll
         for (int g = 0; g < 4; ++g) sc[g] = *reinterpret_cast<const float4v*>(scales + wn + j * 32 + 8 * g + half4);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < MT; ++i) {
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const int tl = i * 32 + tok, rl = j * 32 + 8 * g + half4;
@@ -262,7 +288,7 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a)
     if (EP == SQ_F32 || nparts > 1) return;
     uint16_t* yb = reinterpret_cast<uint16_t*>(a.y);
 #pragma unroll 4
-    for (int k = 0; k < 32; ++k) {
+    for (int k = 0; k < 8 * MT; ++k) {
         const int idx = k * 64 + lane, tl = idx >> 4, piece = idx & 15;
         const int t = t0 + wm + tl, r = r0 + wn + piece * 8;
         if (t >= a.T || r >= a.R) continue;
@@ -290,54 +316,65 @@ __global__ __launch_bounds__(256) void bf16_to_f16_kernel(const uint16_t* __rest
 }
 
 // tail tiles: y[t, y_off + r] = scale of r * sum over kz of part[(tail tile * kt + kz)][t - t0][r - r0]
-__global__ __launch_bounds__(256) void gemm256_reduce_kernel(const float* __restrict__ part, int main_tiles, int kt, int tiles_t,
-                                                             int tiles_r, int T, int R, Gemm256Scales sc, void* y, int64_t ldy,
+__global__ __launch_bounds__(256) void gemm256_reduce_kernel(const float* __restrict__ part, int mt, int main_tiles, int kt,
+                                                             int tiles_t, int tiles_r, int T, int R, Gemm256Scales sc, void* y, int64_t ldy,
                                                              int y_off, int y_dtype) {
-    const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;      // element of a tail tile, 4 per thread
-    const int tail = (int)(i / (G_BM * G_BN)), e = (int)(i - (int64_t)tail * (G_BM * G_BN));
+    const int size = gemm256_tokens(mt) * G_BN, blocks = size / 1024;            // 1024 elements of a tail tile a workgroup
+    const int tail = (int)blockIdx.x / blocks, e = ((int)blockIdx.x - tail * blocks) * 1024 + (int)threadIdx.x * 4;
     int bt, br;
-    gemm256_tile(main_tiles + tail, tiles_t, tiles_r, &bt, &br);
-    const int t = bt * G_BM + e / G_BN, r = br * G_BN + e % G_BN;
+    gemm256_tile(main_tiles + tail, tiles_t, tiles_r, gemm256_super(mt), &bt, &br);
+    const int t = bt * gemm256_tokens(mt) + e / G_BN, r = br * G_BN + e % G_BN;
     if (t >= T) return;
-    const float* p = part + (int64_t)tail * kt * (G_BM * G_BN) + e;
+    const float* p = part + (int64_t)tail * kt * size + e;
     float4v sum = *reinterpret_cast<const float4v*>(p);
-    for (int kz = 1; kz < kt; ++kz) sum += *reinterpret_cast<const float4v*>(p + (int64_t)kz * (G_BM * G_BN));
+    for (int kz = 1; kz < kt; ++kz) sum += *reinterpret_cast<const float4v*>(p + (int64_t)kz * size);
 #pragma unroll
     for (int q = 0; q < 4; ++q)
         if (r + q < R) store_y(y, y_dtype, (int64_t)t * ldy + y_off + r + q, sum[q] * gemm256_scale(sc, r + q));
 }
 
-// How the tiles of a T x R output are dealt to `cus` CUs: whole rounds of whole tiles, and the tiles of the last,
-// partial round split over kt workgroups each (kt = 1: no split) while a part keeps at least 16 slabs.
-struct Gemm256Plan { int main_tiles, tail_tiles, kt; };
-static Gemm256Plan gemm256_plan(int T, int R, int C, int cus) {
-    const int tiles = ((T + G_BM - 1) / G_BM) * ((R + G_BN - 1) / G_BN);
-    Gemm256Plan p{tiles, 0, 1};
-    if (cus < 8) return p;
-    const int main = tiles / cus * cus, tail = tiles - main;          // cus is a multiple of 8 on this hardware
-    if (tail == 0 || main % 8) return p;
-    // kt = the split with the least estimated time of the last round: slabs per part at what a slab takes, 1 us, or 1.65 us
-    // times the share of the CUs that work where the chip's power sets the pace (measured: 112 tiles at once 1.03 us, 256
-    // 1.65), and for a split the reduction's launch and the partial tiles written and read back (0.12 us of the chip's memory
-    // bandwidth per part).  2048 x 18944 x 3584 (80 tiles): not split, 257 us against 266 in three; 2048 x 3584 x 18944 (112
-    // tiles): in two, 253 against 305.
+// How a T x R output is cut: tiles of 64 mt token rows; whole rounds of whole tiles over the `cus` CUs, and the tiles of
+// the last, partial round split over kt workgroups each (kt = 1: no split) while a part keeps at least 16 slabs.
+struct Gemm256Plan { int mt, main_tiles, tail_tiles, kt; };
+
+// Tiles of 256 rows read least per product and are the ones for products of many rounds (8192^3: 826 us, 938 with 192 rows,
+// 1010 with 128); where few tiles leave CUs idle, or most of a tile's rows are past the end, smaller ones win.  The plan with the
+// least estimated time is taken.  A slab takes G_SLAB + G_SLAB_BUSY * (share of the CUs at work) microseconds (the chip's power
+// and its L2 set the pace when it is full; fitted to 32 .. 512 tiles of each height at 3584 columns, where one round takes 42 ..
+// 63 / 55 .. 81 / 70 .. 104 us), a round 5 us at its ends, and a split adds the reduction's launch and the partial tiles written
+// and read back.  Estimated best and measured, tiles of 256 rows unsplit before it (us): 333 x 37888 x 3584 161, now 119;
+// 1024 x 7168 x 5120 95 (in two 85), now 72; 2048 x 3584 x 3584 66, now 52; 2048 x 4608 x 3584 70, now 64; 512 x 3584 x 18944
+// 104 in four, now 88; 2048 x 3584 x 18944 stays with 256 rows in two, 245 (128 rows: 270).
+constexpr double G_SLAB[5] = {0, 0, 0.58, 0.73, 0.98}, G_SLAB_BUSY[5] = {0, 0, 0.42, 0.56, 0.70};
+
+static Gemm256Plan gemm256_plan(int T, int R, int C, int cus, bool split) {
     const int slabs = C / G_BK;
-    int best = 1;
+    const bool rounds = cus >= 8 && cus % 8 == 0;
+    const int n = rounds ? cus : 256;
+    Gemm256Plan best{4, 0, 0, 1};
     double best_t = 1e30;
-    for (int kt = 1; kt <= 4; ++kt) {
-        if (kt > 1 && slabs / kt < 16) break;
-        const int wgs = tail * kt, full = wgs / cus;
-        const double last = wgs % cus ? std::max(1.0, 1.65 * (wgs % cus) / cus) : 0.0;
-        const double t = ((slabs + kt - 1) / kt) * (1.65 * full + last) + (kt > 1 ? 6.0 + wgs * 0.12 : 0.0);
-        if (t < best_t - 1e-9) { best_t = t; best = kt; }
+    for (int mt = 4; mt >= 2; --mt) {
+        const int64_t tiles = (int64_t)((T + gemm256_tokens(mt) - 1) / gemm256_tokens(mt)) * ((R + G_BN - 1) / G_BN);
+        const int main = (int)(tiles / n) * n, tail = (int)(tiles - main);
+        const double slab = G_SLAB[mt] + G_SLAB_BUSY[mt];
+        for (int kt = 1; kt <= (split && rounds && tail ? 4 : 1); ++kt) {
+            if (kt > 1 && slabs / kt < 16) break;
+            const int wgs = tail * kt, of = (slabs + kt - 1) / kt;
+            double t = (double)(main / n) * (slabs * slab + 5.0) + (wgs / n) * (of * slab + 5.0);
+            if (wgs % n) t += of * (G_SLAB[mt] + G_SLAB_BUSY[mt] * (wgs % n) / n) + 5.0;
+            if (kt > 1) t += 4.0 + wgs * mt * 0.015;
+            if (t < best_t - 1e-9) {
+                best_t = t;
+                best = kt > 1 ? Gemm256Plan{mt, main, tail, kt} : Gemm256Plan{mt, (int)tiles, 0, 1};
+            }
+        }
     }
-    if (best < 2) return p;
-    return Gemm256Plan{main, tail, best};
+    return best;
 }
 
 size_t gemm256_part_bytes(int T, int R, int C, int cus) {
-    const Gemm256Plan p = gemm256_plan(T, R, C, cus);
-    return ((size_t)p.tail_tiles * p.kt * G_BM * G_BN * 4 + 255) & ~(size_t)255;
+    const Gemm256Plan p = gemm256_plan(T, R, C, cus, true);
+    return ((size_t)p.tail_tiles * p.kt * gemm256_tokens(p.mt) * G_BN * 4 + 255) & ~(size_t)255;
 }
 
 bool gemm256_ok(int C, int64_t ldx, int64_t ldw, const void* x, const void* w) {
@@ -347,30 +384,34 @@ bool gemm256_ok(int C, int64_t ldx, int64_t ldw, const void* x, const void* w) {
 // x and w fp16.  `part` (gemm256_part_bytes) enables the split of the last round; NULL = no split.
 int launch_gemm256(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ldw, const Gemm256Scales& sc, void* y,
                    int y_dtype, int64_t ldy, int y_off, int T, int R, int C, float* part, int cus, hipStream_t s) {
+    typedef void (*kernel_t)(Gemm256Args);
+    static constexpr kernel_t kernels[3][3] = {
+        {gemm256_kernel<SQ_F16, 2>, gemm256_kernel<SQ_BF16, 2>, gemm256_kernel<SQ_F32, 2>},
+        {gemm256_kernel<SQ_F16, 3>, gemm256_kernel<SQ_BF16, 3>, gemm256_kernel<SQ_F32, 3>},
+        {gemm256_kernel<SQ_F16, 4>, gemm256_kernel<SQ_BF16, 4>, gemm256_kernel<SQ_F32, 4>}};
     static bool raised = false;
     if (!raised) {
-        for (const void* k : {(const void*)gemm256_kernel<SQ_F16>, (const void*)gemm256_kernel<SQ_BF16>, (const void*)gemm256_kernel<SQ_F32>})
-            (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        for (const auto& of : kernels)
+            for (kernel_t k : of) (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         (void)hipGetLastError();
         raised = true;
     }
     Gemm256Args a;
     a.x = x; a.w = w; a.sc = sc; a.y = y; a.ldx = ldx; a.ldw = ldw; a.ldy = ldy;
     a.T = T; a.R = R; a.C = C; a.y_off = y_off; a.y_dtype = y_dtype;
-    a.tiles_t = (T + G_BM - 1) / G_BM;
+    const Gemm256Plan pl = gemm256_plan(T, R, C, cus, part != nullptr);
+    a.tiles_t = (T + gemm256_tokens(pl.mt) - 1) / gemm256_tokens(pl.mt);
     a.tiles_r = (R + G_BN - 1) / G_BN;
-    const Gemm256Plan pl = part ? gemm256_plan(T, R, C, cus) : Gemm256Plan{a.tiles_t * a.tiles_r, 0, 1};
     a.main_tiles = pl.main_tiles;
     a.kt = pl.kt;
     a.part = part;
     const bool vec = y_dtype != SQ_F32 && ((uintptr_t)y & 15) == 0 && ldy % 8 == 0 && y_off % 8 == 0;
     const unsigned grid = (unsigned)(8 * ((pl.main_tiles + 7) / 8 + (pl.tail_tiles * pl.kt + 7) / 8));
-    const auto kernel = !vec ? gemm256_kernel<SQ_F32> : y_dtype == SQ_BF16 ? gemm256_kernel<SQ_BF16> : gemm256_kernel<SQ_F16>;
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(G_WAVES * 64), G_SLOTS * G_SLOT_BYTES, s, a);
+    hipLaunchKernelGGL(kernels[pl.mt - 2][!vec ? 2 : y_dtype == SQ_BF16 ? 1 : 0], dim3(grid), dim3(G_WAVES * 64), gemm256_lds(pl.mt), s, a);
     int rc = check_launch("sq_linear_gemm(gemm256)");
     if (rc || pl.tail_tiles == 0) return rc;
-    const int64_t n4 = (int64_t)pl.tail_tiles * G_BM * G_BN / 4;
-    hipLaunchKernelGGL(gemm256_reduce_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, part, pl.main_tiles, pl.kt,
+    const unsigned blocks = (unsigned)(pl.tail_tiles * (gemm256_tokens(pl.mt) * G_BN / 1024));
+    hipLaunchKernelGGL(gemm256_reduce_kernel, dim3(blocks), dim3(256), 0, s, part, pl.mt, pl.main_tiles, pl.kt,
                        a.tiles_t, a.tiles_r, T, R, sc, y, ldy, y_off, y_dtype);
     return check_launch("sq_linear_gemm(gemm256 reduce)");
 }

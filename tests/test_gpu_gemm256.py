@@ -31,3 +31,22 @@ def test_stack_of_pieces(n):
     linear_gemm([to_device(s, stream=False) for s in ss], x.cuda(), y)
     ref = np.concatenate([x.float().numpy().astype(np.float64) @ s.decode().astype(np.float64).T for s in ss], axis=1)
     assert rel_max_err(y.cpu().numpy(), ref) < 1e-3
+
+
+@pytest.mark.parametrize("T,R,C", [
+    (129, 300, 64), (65, 257, 320), (333, 2000, 2048),              # tiles of 128 token rows, the last also split along K
+    (190, 60000, 64), (185, 60001, 320), (300, 34000, 4096),        # of 192: one slab, five, two rounds with a split last one
+    (250, 65700, 192), (257, 33000, 64), (510, 34000, 4096)])       # of 256
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_tile_heights(T, R, C, dtype):
+    g = torch.Generator(device="cuda").manual_seed(T + R)
+    x, w = (torch.randn(n, C, generator=g, device="cuda").half() for n in (T, R))
+    y = torch.full((T, R + 8), float("nan"), dtype=dtype, device="cuda")
+    gemm_dense(w, x, y[:, :R])
+    ref = x.double() @ w.double().T
+    # C roundings to fp32, in any order, each at most 2^-24 of a partial sum; those of C products of unit normals stay below
+    # 5 sqrt(C), and roundings of random sign add up to less than 6 sqrt(C / 3) of them: 17.4 C 2^-24. A slab
+    # left out is off by 8.
+    bound = 17.4 * C * 2.0 ** -24 + (2.0 ** -8 * ref.abs() if dtype == torch.bfloat16 else 0.0)
+    assert ((y[:, :R].double() - ref).abs() <= bound).all()
+    assert torch.isnan(y[:, R:]).all()
