@@ -334,7 +334,7 @@ __global__ __launch_bounds__(256) void gemm256_reduce_kernel(const float* __rest
 }
 
 // How a T x R output is cut: tiles of 64 mt token rows; whole rounds of whole tiles over the `cus` CUs, and the tiles of
-// the last, partial round split over kt workgroups each (kt = 1: no split) while a part keeps at least 8 slabs.
+// the last, partial round split over kt workgroups each (kt = 1: no split) while a part keeps at least 16 slabs.
 struct Gemm256Plan { int mt, main_tiles, tail_tiles, kt; };
 
 // Tiles of 256 rows read least per product and are the ones for products of many rounds (8192^3: 826 us, 938 with 192 rows,
@@ -345,8 +345,8 @@ struct Gemm256Plan { int mt, main_tiles, tail_tiles, kt; };
 // and read back.  Estimated best and measured, tiles of 256 rows unsplit before it (us): 333 x 37888 x 3584 161, now 119;
 // 1024 x 7168 x 5120 95 (in two 85), now 72; 2048 x 3584 x 3584 66, now 52; 2048 x 4608 x 3584 70, now 64; 512 x 3584 x 18944
 // 104 in four, now 88; 2048 x 3584 x 18944 stays with 256 rows in two, 245 (128 rows: 270).
-// Up to eight parts of at least eight slabs, for few tiles of long rows (the best of up to four parts of at least 16 slabs, now):
-// 333 x 3584 x 18944 83, 71; 700 x 896 x 4864 27, 24; 520 x 1024 x 2048 22.5, 20.6; 257 x 3584 x 3584 27.5, 25.5.
+// Up to eight parts, for few tiles of long rows (with up to four, now): 333 x 3584 x 18944 83, 71.  Parts of 8 slabs would gain 2
+// us on short rows (520 x 1024 x 2048 22.5, 20.6) for twice the workspace.
 constexpr double G_SLAB[5] = {0, 0, 0.58, 0.73, 0.98}, G_SLAB_BUSY[5] = {0, 0, 0.42, 0.56, 0.70};
 
 static Gemm256Plan gemm256_plan(int T, int R, int C, int cus, bool split) {
@@ -360,7 +360,7 @@ static Gemm256Plan gemm256_plan(int T, int R, int C, int cus, bool split) {
         const int main = (int)(tiles / n) * n, tail = (int)(tiles - main);
         const double slab = G_SLAB[mt] + G_SLAB_BUSY[mt];
         for (int kt = 1; kt <= (split && rounds && tail ? 8 : 1); ++kt) {
-            if (kt > 1 && slabs / kt < 8) break;
+            if (kt > 1 && slabs / kt < 16) break;
             const int wgs = tail * kt, of = (slabs + kt - 1) / kt;
             double t = (double)(main / n) * (slabs * slab + 5.0) + (wgs / n) * (of * slab + 5.0);
             if (wgs % n) t += of * (G_SLAB[mt] + G_SLAB_BUSY[mt] * (wgs % n) / n) + 5.0;
