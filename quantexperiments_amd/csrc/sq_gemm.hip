@@ -211,15 +211,19 @@ static int decoded_group(const sq_matrix* mats, int n, int i0, int T) {
     return k;
 }
 
-// (more rows than half the CUs' worth of 256-row tiles fill the chip in the tile GEMM, whose workgroups read less: 37888 x 3584 at
-// 64 rows, 237 us with it, 248 here; 4608 x 3584 65 and 45, 3584 x 18944 154 and 99, 593 x 1984 60 and 22)
+// Where the tile GEMM, whose workgroups read less, is the faster one behind the same decode: with more rows than half the CUs'
+// worth of 256-row tiles, and from 129 activation rows for 24 M weights and more (there and here, us: 37888 x 3584 at 64 rows 216
+// and 248, 30000 x 3584 at 128 / 200 / 256 rows 164 / 154 / 153 and 138 / 169 / 173, 18944 x 3584 96 / 107 / 108 and 103 / 128 /
+// 127, 3584 x 18944 107 / 116 / 120 and 112 / 131 / 134, 4608 x 3584 44 / 46 / 47 and 40 / 46 / 49, 593 x 1984 41 / 41 / 41 and
+// 26 / 32 / 34).
 static bool decoded_route(const sq_matrix* mats, int n, int T) {
     int64_t rows = 0;
     for (int i = 0; i < n; ++i) {
         rows += mats[i].R;
         if (mats[i].R > 0 && (!mats[i].tags || !decoded_group(mats, n, i, T))) return false;
     }
-    return rows < (int64_t)128 * device_cus() || mats[0].C % 64;
+    if (mats[0].C % 64) return true;
+    return rows < (int64_t)128 * device_cus() && (T <= 128 || rows * mats[0].C < (int64_t)24 << 20);
 }
 
 static size_t decoded_workspace(const sq_matrix* mats, int n, int T) {

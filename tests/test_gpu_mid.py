@@ -42,6 +42,7 @@ DECODED = [  # rows of the stack's pieces, C, d, bits, G, M, T: column orders, r
     ((1,), 8, 8, 16, 1, 1, 33), ((129, 1, 300), 1984, 8, 16, 1, 16, 15), ((16,), 1984, 8, 16, 1, 16, 256), ((130,), 72, 8, 16, 1, 3, 5),
     ((70, 50), 1000, 4, 12, 1, 1, 48), ((50, 16), 264, 4, 10, 4, 1, 193), ((257,), 520, 4, 8, 1, 2, 128), ((40, 40, 40, 40, 7), 512, 8, 16, 1, 2, 17),
     ((33,), 9216, 8, 16, 1, 16, 3), ((12,), 200, 2, 5, 3, 1, 81), ((3584,), 776, 8, 16, 1, 1, 100),
+    ((12500, 100), 2048, 8, 16, 1, 16, 129),      # past 128 rows and 24 M weights, in tiles
 ]
 
 
