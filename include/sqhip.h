@@ -37,9 +37,9 @@ typedef struct sq_matrix {
                                  * point then works from the stream (one resident copy, the reference's `compact`) */
     const uint16_t* table;      /* fp16 bits [G*K, d] */
     const uint16_t* row_scale;  /* fp16 bits [R] */
-    const uint8_t*  row_book;   /* [R] or NULL when G == 1 */
-    const uint8_t*  row_mask;   /* [R] or NULL when M == 1 */
-    const int32_t*  perms;      /* [M, C] or NULL when M == 1 */
+    const uint8_t*  row_book;   /* [R], every entry below G, or NULL when G == 1 (the products and the dense decode index */
+    const uint8_t*  row_mask;   /* [R], every entry below M, or NULL when M == 1   with these three and cannot check */
+    const int32_t*  perms;      /* [M, C], each row a permutation of 0 .. C - 1, or NULL when M == 1      them) */
     const int32_t*  row_order;  /* optional [R]: row ids sorted by row_mask (stable); NULL = natural */
     int32_t R, C, d, bits, G, M, W;
     int32_t y_off;              /* first output column of this piece in the stacked Y */
@@ -231,7 +231,9 @@ int sq_codebook_balance_books(const int32_t* tags_host, int32_t R, int32_t W, in
 /* The load-time layouts built on the GPU, from tags that are already there: the same bytes as the host routines above
  * (which stay for tags in host memory), in milliseconds instead of a fraction of a second per matrix.  tags, row_book,
  * counts, out, scratch and remap are DEVICE pointers, row_mask_host and remap_out_host HOST pointers; the plan and balance calls
- * and sq_stream_fill_device synchronise the stream (they are for load time and never run under graph capture).
+ * and sq_stream_fill_device synchronise the stream (they are for load time and never run under graph capture).  Every entry
+ * of row_book is below G: the plan and balance calls refuse a row_book that names another codebook (SQ_EINVAL, nothing is
+ * launched); the other two take what it holds modulo G.
  *   sq_stream_plan_device   makes the plan of the buffer sq_stream_build_books would write (its layout, and for the d = 4
  *                           formats the tile-major copy): *plan_out, the bytes of the buffer and of the scratch the fill
  *                           needs, and runs_out / groups_out as there.  counts: sq_stream_counts_bytes bytes (0 for d = 4).

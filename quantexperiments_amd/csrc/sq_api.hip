@@ -3,6 +3,7 @@
 #include <atomic>
 #include <stdarg.h>
 #include <stdio.h>
+#include <vector>
 #include "sq_stream.h"
 
 namespace sq {
@@ -418,6 +419,16 @@ static int device_build_check(const char* who, const void* tags, int32_t R, int3
     return SQ_OK;
 }
 
+// row_book as the host routines check it, from a copy of it; synchronises
+static int device_books_check(const char* who, int32_t R, int32_t G, const uint8_t* row_book, hipStream_t s) {
+    if (G <= 1) return SQ_OK;
+    std::vector<uint8_t> host((size_t)R);
+    hipError_t e = hipMemcpyAsync(host.data(), row_book, host.size(), hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e != hipSuccess) return fail(SQ_ELAUNCH, "%s: %s", who, hipGetErrorString(e));
+    return books_check(who, R, G, host.data());
+}
+
 size_t sq_stream_counts_bytes(int32_t R, int32_t C, int32_t d, int32_t bits, int32_t G) {
     return d > 0 && stream_format_ok(R, C, d, bits, G) ? stream_counts_bytes(R, C, d, bits, G) : 0;
 }
@@ -431,6 +442,7 @@ int sq_stream_plan_device(const int32_t* tags, int32_t R, int32_t W, int32_t C, 
     if (!(tags && d > 0 && !stream_format_ok(R, C, d, bits, G) && !row_mask_host && tiled_format_ok(R, W, C, d, bits))) {
         if (int rc = device_build_check(who, tags, R, W, C, d, bits, G, row_book)) return rc;
         if (!counts) return fail(SQ_EINVAL, "%s: null counts", who);
+        if (int rc = device_books_check(who, R, G, row_book, (hipStream_t)stream)) return rc;
     }
     return stream_plan_device((const uint32_t*)tags, R, W, C, d, bits, G, G > 1 ? row_book : nullptr, row_mask_host, runs, counts,
                               (StreamDevicePlan**)plan_out, bytes_out, scratch_out, runs_out, groups_out, (hipStream_t)stream);
@@ -448,6 +460,7 @@ int sq_codebook_balance_device(const int32_t* tags, int32_t R, int32_t W, int32_
                                uint32_t* counts, uint16_t* remap_out_host, void* stream) {
     if (int rc = device_build_check("sq_codebook_balance_device", tags, R, W, C, d, bits, G, row_book)) return rc;
     if (!counts || !remap_out_host) return fail(SQ_EINVAL, "sq_codebook_balance_device: null pointer");
+    if (int rc = device_books_check("sq_codebook_balance_device", R, G, row_book, (hipStream_t)stream)) return rc;
     return stream_balance_device((const uint32_t*)tags, R, W, C, d, bits, counts, remap_out_host, G, G > 1 ? row_book : nullptr, (hipStream_t)stream);
 }
 
@@ -455,7 +468,7 @@ int sq_codebook_relabel_device(int32_t* tags, int32_t R, int32_t W, int32_t C, i
                                const uint16_t* remap, void* stream) {
     if (int rc = device_build_check("sq_codebook_relabel_device", tags, R, W, C, d, bits, G, row_book)) return rc;
     if (!remap) return fail(SQ_EINVAL, "sq_codebook_relabel_device: null pointer");
-    return stream_relabel_device((uint32_t*)tags, R, W, C, d, bits, G > 1 ? row_book : nullptr, remap, (hipStream_t)stream);
+    return stream_relabel_device((uint32_t*)tags, R, W, C, d, bits, G, G > 1 ? row_book : nullptr, remap, (hipStream_t)stream);
 }
 
 size_t sq_stream_bytes(const int32_t* tags_host, int32_t R, int32_t W, int32_t C, int32_t d, int32_t bits,

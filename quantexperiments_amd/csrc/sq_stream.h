@@ -95,7 +95,7 @@ int stream_fill_device(const StreamDevicePlan& D, const uint32_t* tags, const ui
 void stream_plan_free(StreamDevicePlan* D);
 int stream_balance_device(const uint32_t* tags, int R, int W, int C, int d, int bits, uint32_t* counts, uint16_t* remap_out, int G,
                           const uint8_t* row_book, hipStream_t s);
-int stream_relabel_device(uint32_t* tags, int R, int W, int C, int d, int bits, const uint8_t* row_book, const uint16_t* remap, hipStream_t s);
+int stream_relabel_device(uint32_t* tags, int R, int W, int C, int d, int bits, int G, const uint8_t* row_book, const uint16_t* remap, hipStream_t s);
 // sq_matrix.stream_runs is sq_stream_build's runs_out: the run count in the low 16 bits, the groups of the longest run
 // in the next 8, the most column orders in one run (less one) in bits 24-26, the steps per unit of the first-steps region
 // (less one) in bits 27-28, bit 30 = the stream carries a relabelled codebook

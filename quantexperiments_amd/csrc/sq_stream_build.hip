@@ -652,13 +652,19 @@ int stream_build_host(const uint32_t* tags, int R, int W, int C, int d, int bits
 // spends its time on (16 cores: 150 ms for 18944 x 3584, 2.5 s for 3584 x 18944 on one).  Whole load of a matrix, tags on
 // the GPU to stream on the GPU, before / now: 3584 x 3584 363 / 2.7 ms, 18944 x 3584 155 / 6.0, 3584 x 18944 2525 / 12.9.
 
+// A row's codebook as these kernels index with it: below G (a power of two) whatever row_book holds, as in the host builder.
+// The callers have refused a row_book that names another one, except where it may have been written since.
+__device__ __forceinline__ uint32_t stream_book(const uint8_t* row_book, int r, int G, int bits) {
+    return row_book ? ((uint32_t)row_book[r] & (uint32_t)(G - 1)) << bits : 0u;
+}
+
 // count[book << bits | label] += 1 for every tag (one wave per row)
-__global__ __launch_bounds__(256) void stream_codeword_count_kernel(const uint32_t* __restrict__ tags, int R, int W, int U, int bits,
+__global__ __launch_bounds__(256) void stream_codeword_count_kernel(const uint32_t* __restrict__ tags, int R, int W, int U, int bits, int G,
                                                                     const uint8_t* __restrict__ row_book, uint32_t* __restrict__ count) {
     const int r = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)), lane = threadIdx.x & 63;
     if (r >= R) return;
     const uint32_t* row = tags + (int64_t)r * W;
-    const uint32_t book = row_book ? (uint32_t)row_book[r] << bits : 0u;
+    const uint32_t book = stream_book(row_book, r, G, bits);
     for (int j = lane; j < U; j += 64) atomicAdd(count + (book | tag_at(row, W, bits, j)), 1u);
 }
 
@@ -668,7 +674,7 @@ __global__ __launch_bounds__(256) void stream_clear_kernel(uint32_t* __restrict_
 }
 
 // rewrites the tags of a matrix through remap[book << bits | label] in place; a thread owns 32 tags, which are whole words
-__global__ __launch_bounds__(256) void stream_relabel_kernel(uint32_t* __restrict__ tags, int R, int W, int U, int bits,
+__global__ __launch_bounds__(256) void stream_relabel_kernel(uint32_t* __restrict__ tags, int R, int W, int U, int bits, int G,
                                                              const uint8_t* __restrict__ row_book, const uint16_t* __restrict__ remap) {
     const int units = (U + 31) / 32;
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -676,7 +682,7 @@ __global__ __launch_bounds__(256) void stream_relabel_kernel(uint32_t* __restric
     const int r = (int)(i / units), u = (int)(i - (int64_t)r * units);
     uint32_t* w = tags + (int64_t)r * W + u * bits;
     const int nw = min(bits, W - u * bits), n = min(32, U - u * 32);
-    const uint16_t* map = remap + ((row_book ? (size_t)row_book[r] : 0) << bits);
+    const uint16_t* map = remap + stream_book(row_book, r, G, bits);
     const uint32_t mask = (1u << bits) - 1u;
     uint64_t in = 0, out = 0;
     int have = 0, held = 0, rd = 0, wr = 0;
@@ -691,14 +697,14 @@ __global__ __launch_bounds__(256) void stream_relabel_kernel(uint32_t* __restric
 }
 
 // cnt[v * R + r]: entries of row r in bucket v (one wave per row; its counters in LDS)
-__global__ __launch_bounds__(64) void stream_count_kernel(const uint32_t* __restrict__ tags, int R, int W, int U, int bits, int PC, int NS, int NV,
+__global__ __launch_bounds__(64) void stream_count_kernel(const uint32_t* __restrict__ tags, int R, int W, int U, int bits, int G, int PC, int NS, int NV,
                                                           const uint8_t* __restrict__ row_book, uint16_t* __restrict__ cnt) {
     extern __shared__ uint32_t stream_count_lds[];
     const int r = (int)blockIdx.x, lane = (int)threadIdx.x;
     for (int v = lane; v < NV; v += 64) stream_count_lds[v] = 0u;
     __syncthreads();
     const uint32_t* row = tags + (int64_t)r * W;
-    const uint32_t book = row_book ? (uint32_t)row_book[r] << bits : 0u;
+    const uint32_t book = stream_book(row_book, r, G, bits);
     for (int j = lane; j < U; j += 64)
         atomicAdd(&stream_count_lds[(j / PC) * NS + (int)((book | tag_at(row, W, bits, j)) >> STREAM_SLICE_BITS)], 1u);
     __syncthreads();
@@ -713,7 +719,7 @@ struct StreamFillArgs {
     const uint32_t* goff;       // [NV * NG + 1]: the groups' steps counted one behind the other
     unsigned char* steps;       // the stream buffer's steps
     unsigned char* work;        // groups that LDS does not hold: STREAM_FILL_BYTES per entry slot of every group
-    int W, U, bits, PC, NS, NV, NG, fs;
+    int W, U, bits, G, PC, NS, NV, NG, fs;
 };
 
 // Bytes one entry slot (64 lanes) of a group takes: 65 words of entries (the odd pitch spreads one lane's entries over the
@@ -777,7 +783,7 @@ __global__ __launch_bounds__(256) void stream_fill_kernel(StreamFillArgs a) {
     int total = 0;
     if (row_id != STREAM_NO_ROW) {
         const uint32_t* row = a.tags + (int64_t)row_id * a.W;
-        const uint32_t book = a.row_book ? (uint32_t)a.row_book[row_id] << a.bits : 0u;
+        const uint32_t book = stream_book(a.row_book, (int)row_id, a.G, a.bits);
         const int kp = v / a.NS, sl = v - kp * a.NS, p0 = kp * a.PC, len = min(a.PC, a.U - p0);
         const int j0 = p0 + len * (t & 3) / 4, j1 = p0 + len * ((t & 3) + 1) / 4;
         int n = 0;
@@ -955,7 +961,7 @@ int stream_balance_device(const uint32_t* tags, int R, int W, int C, int d, int 
                           const uint8_t* row_book, hipStream_t s) {
     const int64_t n = (int64_t)G << bits;
     hipLaunchKernelGGL(stream_clear_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, counts, n);
-    hipLaunchKernelGGL(stream_codeword_count_kernel, dim3((unsigned)((R + 3) / 4)), dim3(256), 0, s, tags, R, W, C / d, bits, row_book, counts);
+    hipLaunchKernelGGL(stream_codeword_count_kernel, dim3((unsigned)((R + 3) / 4)), dim3(256), 0, s, tags, R, W, C / d, bits, G, row_book, counts);
     int rc = check_launch("sq_codebook_balance_device");
     if (rc) return rc;
     std::vector<uint32_t> host((size_t)n);
@@ -968,10 +974,10 @@ int stream_balance_device(const uint32_t* tags, int R, int W, int C, int d, int 
     return SQ_OK;
 }
 
-int stream_relabel_device(uint32_t* tags, int R, int W, int C, int d, int bits, const uint8_t* row_book, const uint16_t* remap, hipStream_t s) {
+int stream_relabel_device(uint32_t* tags, int R, int W, int C, int d, int bits, int G, const uint8_t* row_book, const uint16_t* remap, hipStream_t s) {
     const int64_t n = (int64_t)R * ((C / d + 31) / 32);
     if (n == 0) return SQ_OK;
-    hipLaunchKernelGGL(stream_relabel_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, tags, R, W, C / d, bits, row_book, remap);
+    hipLaunchKernelGGL(stream_relabel_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, tags, R, W, C / d, bits, G, row_book, remap);
     return check_launch("sq_codebook_relabel_device");
 }
 
@@ -1001,7 +1007,7 @@ int stream_plan_device(const uint32_t* tags, int R, int W, int C, int d, int bit
         StreamPlan& P = D->P;
         plan_rows(R, C, d, stream_label_bits(bits, G), row_mask_host, runs, P, false);
         const StreamGeom& g = P.g;
-        hipLaunchKernelGGL(stream_count_kernel, dim3((unsigned)R), dim3(64), (size_t)g.NV * 4, s, tags, R, W, g.U, bits, g.PC, g.NS, g.NV, row_book,
+        hipLaunchKernelGGL(stream_count_kernel, dim3((unsigned)R), dim3(64), (size_t)g.NV * 4, s, tags, R, W, g.U, bits, G, g.PC, g.NS, g.NV, row_book,
                            (uint16_t*)counts);
         int rc = check_launch("sq_stream_plan_device");
         if (rc) return rc;
@@ -1065,7 +1071,7 @@ int stream_fill_device(const StreamDevicePlan& D, const uint32_t* tags, const ui
     a.goff = a.rows + nvg * 64;
     a.steps = out + g.off_steps;
     a.work = scratch + ((lists.size() * 4 + 255) & ~(size_t)255);
-    a.W = D.W; a.U = g.U; a.bits = D.bits; a.PC = g.PC; a.NS = g.NS; a.NV = g.NV; a.NG = g.NG; a.fs = g.fs;
+    a.W = D.W; a.U = g.U; a.bits = D.bits; a.G = D.G; a.PC = g.PC; a.NS = g.NS; a.NV = g.NV; a.NG = g.NG; a.fs = g.fs;
     if (D.in_lds) {
         const size_t lds = (size_t)longest * g.fmt.eps * STREAM_FILL_BYTES;
         (void)hipFuncSetAttribute((const void*)stream_fill_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, STREAM_FILL_LDS);

@@ -69,6 +69,17 @@ class _Workspace:
                 _lib.check(_lib.lib().sq_workspace_reset(b.data_ptr(), b.numel(), _lib.stream_ptr(dev)))
 
 
+def _check_row_ids(ids: torch.Tensor, R: int, n: int, what: str) -> None:
+    """Raise unless the first R entries of `ids` (row_book: a codebook per row; row_mask: a column order per row) exist and lie in
+    0 .. n - 1.  The kernels index memory with them and do not look again."""
+    if ids.numel() < R:
+        raise ValueError(f"{what} has {ids.numel()} entries for {R} rows")
+    if R:
+        lo, hi = torch.stack(ids.reshape(-1)[:R].to(torch.int64).aminmax()).tolist()
+        if lo < 0 or hi >= n:
+            raise ValueError(f"{what} names {lo if lo < 0 else hi} of {n}")
+
+
 class PackedLinear(torch.nn.Module):
     """A block linear run from packed tensors."""
 
@@ -116,6 +127,8 @@ class PackedLinear(torch.nn.Module):
         self.G = table.shape[0] // K
         if (self.G > 1) != (row_book is not None):
             raise ValueError("row_book is needed exactly when the table holds several codebooks")
+        if row_book is not None:
+            _check_row_ids(row_book, R, self.G, "row_book")
         self.register_buffer("words", words.to(torch.int32).contiguous())
         self.register_buffer("table", table.to(torch.float16).contiguous())
         self.register_buffer("row_scale", row_scale.to(torch.float16).contiguous())
@@ -331,12 +344,10 @@ def _build_stream_device(words: torch.Tensor, C: int, d: int, bits: int, row_mas
     book, G = None, 1
     if row_book is not None:
         book, G = row_book if isinstance(row_book, tuple) else (row_book, None)
-        book = book.detach().to(dev, torch.uint8).contiguous()
-        top = int(book.max()) if R else 0
         if G is None:
-            G = 1 << top.bit_length()
-        if top >= G:
-            raise ValueError(f"row_book names codebook {top} of {G}")
+            G = 1 << (int(book.max()).bit_length() if R else 0)
+        _check_row_ids(book, R, G, "row_book")
+        book = book.detach().to(dev, torch.uint8).contiguous()
     new = lambda n: torch.empty(max(n, 1), dtype=torch.uint8, device=dev)
     counts = new(L.sq_stream_counts_bytes(R, C, d, bits, G))
     plan, nbytes, nscratch = ctypes.c_void_p(), ctypes.c_size_t(), ctypes.c_size_t()

@@ -57,3 +57,23 @@ def test_device_relabelling(R, C, bits, G):
     m = ctypes.c_void_p()
     assert L.sq_stream_plan_device(None, R, 1, C, 8, bits, G, None, None, 0, None, ctypes.byref(m), ctypes.byref(ctypes.c_size_t()),
                                    ctypes.byref(ctypes.c_size_t()), ctypes.byref(ctypes.c_int32()), ctypes.byref(ctypes.c_int32()), None) == _lib.SQ_EINVAL
+
+
+@pytest.mark.parametrize("G", [2, 4])
+def test_unknown_codebooks_are_refused_before_a_launch(G):
+    L, R, C, bits = _lib.lib(), 40, 512, 14
+    words = torch.zeros(R, C // 8 * bits // 32, dtype=torch.int32, device="cuda")
+    book = torch.zeros(R, dtype=torch.uint8, device="cuda")
+    book[R - 1] = G
+    counts = torch.full((G << bits,), -1, dtype=torch.int32, device="cuda")
+    remap = np.zeros(G << bits, np.uint16)
+    args = (words.data_ptr(), R, words.shape[1], C, 8, bits, G, book.data_ptr())
+    assert L.sq_codebook_balance_device(*args, counts.data_ptr(), remap.ctypes.data, _lib.stream_ptr(words.device)) == _lib.SQ_EINVAL
+    assert b"row 39 names codebook" in L.sq_last_error()
+    plan, n, k, r, g = ctypes.c_void_p(), ctypes.c_size_t(), ctypes.c_size_t(), ctypes.c_int32(), ctypes.c_int32()
+    assert L.sq_stream_counts_bytes(R, C, 8, bits, G) <= counts.numel() * 4
+    assert L.sq_stream_plan_device(*args, None, 0, counts.data_ptr(), ctypes.byref(plan), ctypes.byref(n), ctypes.byref(k), ctypes.byref(r),
+                                   ctypes.byref(g), _lib.stream_ptr(words.device)) == _lib.SQ_EINVAL and not plan.value
+    assert bool((counts == -1).all())
+    with pytest.raises(ValueError, match="row_book"):
+        build_stream(words, C, 8, bits, row_book=(book, G))

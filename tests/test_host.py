@@ -797,3 +797,24 @@ def test_aux_section_round_trip(tmp_path):
     assert packed.PackedFile(_file(tmp_path)[4]).aux is None          # files without the section still load
     with pytest.raises(ValueError):                                   # the decoders are GPU kernels
         packed.q8_rows(torch.from_numpy(hq), torch.from_numpy(hs))
+
+
+class _OnGpu:
+    """What PackedLinear asks of the tags before it checks the rest; anything that goes on to them fails."""
+    device = torch.device("cuda")
+
+    def __init__(self, *shape):
+        self.shape = shape
+
+
+@pytest.mark.parametrize("d,bits", [(8, 12), (8, 16), (4, 10)])
+@pytest.mark.parametrize("book", [torch.tensor([0, 3, 4]), torch.tensor([0, 255, 1], dtype=torch.uint8), torch.tensor([-1, 0, 2]),
+                                  torch.tensor([256, 0, 1]), torch.tensor([0, 1])], ids=["G", "top", "negative", "wraps", "short"])
+def test_row_book_is_checked_before_anything_runs(d, bits, book):
+    # the kernels index the table, and at load counters in global memory, with these
+    from quantexperiments_amd.kernels import PackedLinear
+    with pytest.raises(ValueError, match="row_book"):
+        PackedLinear(_OnGpu(3, bits), torch.zeros(4 << bits, d), torch.ones(3), book, None, torch.arange(32 * d).view(1, -1), 1 << bits, d)
+    with pytest.raises(AttributeError):                   # ids in range: on to the tags
+        PackedLinear(_OnGpu(3, bits), torch.zeros(4 << bits, d), torch.ones(3), torch.tensor([3, 0, 1]), None,
+                     torch.arange(32 * d).view(1, -1), 1 << bits, d)
