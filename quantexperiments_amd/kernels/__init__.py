@@ -129,12 +129,14 @@ class PackedLinear(torch.nn.Module):
             raise ValueError("row_book is needed exactly when the table holds several codebooks")
         if row_book is not None:
             _check_row_ids(row_book, R, self.G, "row_book")
+        self.has_mask = row_mask is not None and perms.shape[0] > 1
+        self.M = perms.shape[0] if self.has_mask else 1
+        if self.has_mask:
+            _check_row_ids(row_mask, R, self.M, "row_mask")
         self.register_buffer("words", words.to(torch.int32).contiguous())
         self.register_buffer("table", table.to(torch.float16).contiguous())
         self.register_buffer("row_scale", row_scale.to(torch.float16).contiguous())
         self.register_buffer("row_book", None if row_book is None else row_book.to(torch.uint8).contiguous())
-        self.has_mask = row_mask is not None and perms.shape[0] > 1
-        self.M = perms.shape[0] if self.has_mask else 1
         if self.has_mask:
             rm = row_mask.to(torch.uint8).contiguous()
             self.register_buffer("row_mask", rm)

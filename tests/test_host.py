@@ -818,3 +818,15 @@ def test_row_book_is_checked_before_anything_runs(d, bits, book):
     with pytest.raises(AttributeError):                   # ids in range: on to the tags
         PackedLinear(_OnGpu(3, bits), torch.zeros(4 << bits, d), torch.ones(3), torch.tensor([3, 0, 1]), None,
                      torch.arange(32 * d).view(1, -1), 1 << bits, d)
+
+
+@pytest.mark.parametrize("mask", [torch.tensor([0, 2, 3]), torch.tensor([0, 255, 1], dtype=torch.uint8), torch.tensor([-1, 0, 2]), torch.tensor([0, 1])],
+                         ids=["M", "top", "negative", "short"])
+def test_row_mask_is_checked_before_anything_runs(mask):
+    # rows are scattered through the order that this names
+    from quantexperiments_amd.kernels import PackedLinear
+    perms = torch.arange(256).repeat(3, 1)
+    with pytest.raises(ValueError, match="row_mask"):
+        PackedLinear(_OnGpu(3, 16), torch.zeros(1 << 16, 8), torch.ones(3), None, mask, perms, 1 << 16, 8)
+    with pytest.raises(AttributeError):
+        PackedLinear(_OnGpu(3, 16), torch.zeros(1 << 16, 8), torch.ones(3), None, torch.tensor([2, 0, 1]), perms, 1 << 16, 8)
