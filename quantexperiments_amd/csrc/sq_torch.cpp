@@ -61,8 +61,10 @@ PyObject* make_native(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return reinterpret_cast<PyObject*>(o);
 }
 
-// The pieces of a call as the library takes them.  0, NOT_COVERED, or -1 with a Python error set.
-struct Pieces { sq_matrix m[MAX_PIECES]; int n = 0, dev = -1; int64_t rows = 0; };
+// The pieces of a call as the library takes them, and what owns their tensors: the library runs without the GIL, so another
+// thread may set an attribute of a piece (which drops its Native) before the kernels are launched.
+// 0, NOT_COVERED, or -1 with a Python error set.
+struct Pieces { sq_matrix m[MAX_PIECES]; int n = 0, dev = -1; int64_t rows = 0; pybind11::object held[MAX_PIECES]; };
 int unpack_pieces(PyObject* seq, Pieces& p) {
     if (!PyList_CheckExact(seq) && !PyTuple_CheckExact(seq)) return NOT_COVERED;
     const Py_ssize_t n = PySequence_Fast_GET_SIZE(seq);
@@ -76,7 +78,8 @@ int unpack_pieces(PyObject* seq, Pieces& p) {
             o = PyObject_CallMethodObjArgs(piece, s_make_native, nullptr);
             if (!o) return -1;
         }
-        if (Py_TYPE(o) != &NativeType) { Py_DECREF(o); return NOT_COVERED; }
+        p.held[i] = pybind11::reinterpret_steal<pybind11::object>(o);
+        if (Py_TYPE(o) != &NativeType) return NOT_COVERED;
         const Native* nat = reinterpret_cast<Native*>(o);
         sq_matrix& m = p.m[i];
         m = nat->m;
@@ -88,7 +91,6 @@ int unpack_pieces(PyObject* seq, Pieces& p) {
         m.y_off = (int32_t)p.rows;
         p.rows += m.R;
         const int dev = t[1].is_cuda() ? t[1].get_device() : -1;
-        Py_DECREF(o);
         if (dev < 0 || dev >= 64 || (i > 0 && dev != p.dev) || m.C != p.m[0].C) return NOT_COVERED;
         p.dev = dev;
     }
@@ -126,10 +128,12 @@ struct OnDevice {
     ~OnDevice() { if (prev >= 0) c10::hip::set_device((c10::DeviceIndex)prev); }
 };
 
-// The shared workspace of `dev` (kernels._Workspace) if it holds `need` bytes and the stream is not being captured (who was
-// captured with which buffer is recorded in Python).
-bool workspace(int dev, size_t need, hipStream_t s, void** ws, size_t* bytes) {
-    *ws = nullptr; *bytes = 0;
+// The shared workspace of a device (kernels._Workspace), held for as long as the call uses it: the library runs without the
+// GIL, and a call of another thread may meanwhile replace the buffer by a larger one.  (Its kernels are enqueued when the call
+// returns; what is freed after that is given out again behind them on this stream.)
+struct Workspace { at::Tensor held; void* p = nullptr; size_t bytes = 0; };
+// It if it holds `need` bytes and the stream is not being captured (who was captured with which buffer is recorded in Python).
+bool workspace(int dev, size_t need, hipStream_t s, Workspace& ws) {
     if (need == 0) return true;
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) { (void)hipGetLastError(); return false; }
@@ -138,8 +142,9 @@ bool workspace(int dev, size_t need, hipStream_t s, void** ws, size_t* bytes) {
     if (!b || !THPVariable_Check(b)) return false;
     const at::Tensor& t = THPVariable_Unpack(b);
     if ((size_t)t.numel() < need) return false;
-    *ws = t.data_ptr();
-    *bytes = (size_t)t.numel();
+    ws.held = t;
+    ws.p = t.data_ptr();
+    ws.bytes = (size_t)t.numel();
     return true;
 }
 
@@ -150,11 +155,11 @@ int linear_into(const Pieces& p, const at::Tensor& x, const at::Tensor& y, bool 
         return NOT_COVERED;
     const int B = (int)x.size(0);
     OnDevice on(p.dev);
-    void* ws; size_t wsb;
-    if (!workspace(p.dev, sq_workspace_bytes(p.m, p.n, B, gemm), on.stream, &ws, &wsb)) return NOT_COVERED;
+    Workspace ws;
+    if (!workspace(p.dev, sq_workspace_bytes(p.m, p.n, B, gemm), on.stream, ws)) return NOT_COVERED;
     int rc;
     Py_BEGIN_ALLOW_THREADS
-    rc = (gemm ? sq_linear_gemm : sq_linear_small)(p.m, p.n, x.data_ptr(), xd, row_ld(x), y.data_ptr(), yd, row_ld(y), B, ws, wsb, on.stream);
+    rc = (gemm ? sq_linear_gemm : sq_linear_small)(p.m, p.n, x.data_ptr(), xd, row_ld(x), y.data_ptr(), yd, row_ld(y), B, ws.p, ws.bytes, on.stream);
     Py_END_ALLOW_THREADS
     return rc;
 }
@@ -336,11 +341,11 @@ PyObject* linear_from(PyObject*, PyObject* const* a, Py_ssize_t n) {
             pr.mode = SQ_FROM_SILU_MUL; pr.add = g.data_ptr(); pr.up = u.data_ptr(); pr.ld_in = row_ld(g);
         }
         OnDevice on(p.dev);
-        void* ws; size_t wsb;
-        if (!workspace(p.dev, sq_workspace_bytes(p.m, p.n, (int)B, 0), on.stream, &ws, &wsb)) return answer(NOT_COVERED);
+        Workspace ws;
+        if (!workspace(p.dev, sq_workspace_bytes(p.m, p.n, (int)B, 0), on.stream, ws)) return answer(NOT_COVERED);
         int rc;
         Py_BEGIN_ALLOW_THREADS
-        rc = sq_linear_small_from(p.m, p.n, &pr, dt, y.data_ptr(), yd, row_ld(y), (int)B, ws, wsb, on.stream);
+        rc = sq_linear_small_from(p.m, p.n, &pr, dt, y.data_ptr(), yd, row_ld(y), (int)B, ws.p, ws.bytes, on.stream);
         Py_END_ALLOW_THREADS
         return answer(rc);
     )
@@ -370,12 +375,12 @@ PyObject* linear_silu(PyObject*, PyObject* const* a, Py_ssize_t n) {
             pr.h_in = o.h_in; pr.h_out = o.h_out; pr.add = o.add; pr.w = o.w; pr.ld_h = o.ld_h; pr.ld_in = o.ld_add;
         }
         OnDevice on(p.dev);
-        void* ws; size_t wsb;
-        if (!workspace(p.dev, sq_workspace_bytes(p.m, 2, (int)B, 0), on.stream, &ws, &wsb)) return answer(NOT_COVERED);
+        Workspace ws;
+        if (!workspace(p.dev, sq_workspace_bytes(p.m, 2, (int)B, 0), on.stream, ws)) return answer(NOT_COVERED);
         int rc;
         Py_BEGIN_ALLOW_THREADS
         rc = sq_linear_small_silu(p.m, 2, norm ? &pr : nullptr, norm ? nullptr : x.data_ptr(), dt, norm ? 0 : row_ld(x), out.data_ptr(), row_ld(out), (int)B,
-                                  ws, wsb, on.stream);
+                                  ws.p, ws.bytes, on.stream);
         Py_END_ALLOW_THREADS
         if (rc != SQ_EUNSUPPORTED) return answer(rc);
         // no fused kernel for this stack: the product into a temporary, then SiLU * up (which writes whole rows)
@@ -383,8 +388,8 @@ PyObject* linear_silu(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const at::Tensor y = at::empty({B, p.rows}, x.options());
         uint16_t* yp = (uint16_t*)y.data_ptr();
         Py_BEGIN_ALLOW_THREADS
-        rc = norm ? sq_linear_small_from(p.m, 2, &pr, dt, yp, dt, p.rows, (int)B, ws, wsb, on.stream)
-                  : sq_linear_small(p.m, 2, x.data_ptr(), dt, row_ld(x), yp, dt, p.rows, (int)B, ws, wsb, on.stream);
+        rc = norm ? sq_linear_small_from(p.m, 2, &pr, dt, yp, dt, p.rows, (int)B, ws.p, ws.bytes, on.stream)
+                  : sq_linear_small(p.m, 2, x.data_ptr(), dt, row_ld(x), yp, dt, p.rows, (int)B, ws.p, ws.bytes, on.stream);
         if (rc == SQ_OK) rc = sq_silu_mul(yp, yp + p.m[0].R, dt, p.rows, nullptr, 1, (int)B, p.m[0].R, out.data_ptr(), on.stream);
         Py_END_ALLOW_THREADS
         return answer(rc);
@@ -407,12 +412,12 @@ PyObject* q8_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
             y.size(1) < V)
             return answer(NOT_COVERED);
         OnDevice on(dev);
-        void* ws; size_t wsb;
-        if (!workspace(dev, sq_q8_workspace_bytes((int)V, (int)C, (int)x.size(0)), on.stream, &ws, &wsb)) return answer(NOT_COVERED);
+        Workspace ws;
+        if (!workspace(dev, sq_q8_workspace_bytes((int)V, (int)C, (int)x.size(0)), on.stream, ws)) return answer(NOT_COVERED);
         int rc;
         Py_BEGIN_ALLOW_THREADS
         rc = sq_q8_linear((const int8_t*)q.data_ptr(), (const uint16_t*)sc.data_ptr(), (int)V, (int)C, x.data_ptr(), xd, x.stride(0), y.data_ptr(), yd, y.stride(0),
-                          (int)x.size(0), ws, wsb, on.stream);
+                          (int)x.size(0), ws.p, ws.bytes, on.stream);
         Py_END_ALLOW_THREADS
         return answer(rc);
     )

@@ -1,13 +1,15 @@
 """The native call path (csrc/sq_torch.cpp): it follows a matrix whose tensors change, leaves to Python what it does not cover,
-and its op raises in backward."""
+holds what it hands to the library, runs on the current stream, and its op raises in backward."""
 
 import copy
+import sys
+import threading
 
 import pytest
 import torch
 
 from quantexperiments_amd import _lib
-from quantexperiments_amd.kernels import linear_small
+from quantexperiments_amd.kernels import _Workspace, linear_small
 from quantexperiments_amd.vllm_ext import core
 from tests.helpers import rand_x, synth, to_device
 
@@ -45,3 +47,44 @@ def test_op_runs_without_gradients_only():
     assert torch.equal(y.detach(), ps.forward(x.detach()))
     with pytest.raises(NotImplementedError):
         y.sum().backward()
+
+
+def test_second_thread_replaces_workspace_and_matrices():
+    """Calls of one thread while another replaces the shared workspace by larger ones and sets attributes of the matrices: what a
+    call was handed stays its own until it has launched (results stay right, tensors allocated meanwhile are not written to)."""
+    ps = core.PackedShards([to_device(synth(96, 1024, 8, 16, seed=1)), to_device(synth(300, 1024, 8, 16, seed=2))])
+    x = rand_x(2, 1024, torch.bfloat16, seed=3).cuda()
+    want, dev = ps.forward(x), x.device
+    size, others, stop = _Workspace.get(1, dev).numel(), [], threading.Event()
+
+    def replace():
+        for k in range(1, 25):
+            _Workspace.get(size + (k << 20), dev)               # (same stream: torch's default one on both threads)
+            ps.rls[k & 1].row_scale = ps.rls[k & 1].row_scale.clone()
+            others.append(torch.full((size + (k << 20),), 7, dtype=torch.uint8, device=dev))
+        stop.set()
+
+    interval = sys.getswitchinterval()
+    sys.setswitchinterval(1e-5)
+    try:
+        t = threading.Thread(target=replace)
+        t.start()
+        ys = []
+        while not stop.is_set() and len(ys) < 20000:
+            ys.append(ps.forward(x))
+        t.join()
+    finally:
+        sys.setswitchinterval(interval)
+    assert len(ys) > 0 and all(torch.equal(y, want) for y in ys[:: max(1, len(ys) // 200)] + ys[-1:])
+    assert all(bool((o == 7).all()) for o in others)
+
+
+def test_calls_on_a_second_stream():
+    ps = core.PackedShards([to_device(synth(96, 512, 8, 16, seed=1)), to_device(synth(40, 512, 8, 16, seed=2))])
+    x = rand_x(3, 512, torch.bfloat16, seed=3).cuda()
+    want, side = ps.forward(x), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        ys = [_lib.native().forward(ps, x) for _ in range(3)]
+    torch.cuda.synchronize()
+    assert all(torch.is_tensor(y) and torch.equal(y, want) for y in ys)
