@@ -42,8 +42,11 @@ class _Workspace:
         if b is None or b.numel() < nbytes:
             if capturing:
                 raise RuntimeError("sqhip workspace must grow outside graph capture: run this shape once eagerly first")
-            if b is not None and key in cls.captured:
-                cls.retired.append(b)
+            if b is not None:
+                if key in cls.captured:
+                    cls.retired.append(b)
+                # (kernels that still use it may be on another stream than the one it was made on, which gets its memory back)
+                b.record_stream(torch.cuda.current_stream(dev))
             cls.captured.discard(key)
             floor = _lib.WS_HEADER + (1 << 20) if kind == "kernels" else 1 << 20
             b = cls.bufs[key] = torch.zeros(max(nbytes, floor), dtype=torch.uint8, device=dev)   # the header starts at zero

@@ -88,3 +88,16 @@ def test_calls_on_a_second_stream():
         ys = [_lib.native().forward(ps, x) for _ in range(3)]
     torch.cuda.synchronize()
     assert all(torch.is_tensor(y) and torch.equal(y, want) for y in ys)
+
+
+def test_outgrown_workspace_waits_for_the_stream_that_used_it():
+    dev, side = torch.device("cuda", torch.cuda.current_device()), torch.cuda.Stream()
+    size = 24 << 20
+    old = _Workspace.get(size, dev, "other streams").data_ptr()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(200_000_000)                          # stands for a product on the old buffer
+        _Workspace.get(2 * size, dev, "other streams")
+    assert torch.empty(size, dtype=torch.uint8, device=dev).data_ptr() != old
+    torch.cuda.synchronize()
+    del _Workspace.bufs[(str(dev), "other streams")]
