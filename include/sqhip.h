@@ -67,9 +67,9 @@ int sq_dequant(const sq_matrix* m, void* out, int out_dtype, int64_t ld_out, int
  * Replaces proto_runs.gemv (reference shapequant/kernels/proto_runs.py:505-571), cuda_gemv.gemv
  * (cuda_gemv.py:148-172), PackedLinear.gemv (gemv.py:142-156) and RunsBatch.run
  * (batched_runs.py:745-771).  Pieces with M > 1 and pieces with a slice stream need a workspace (see
- * sq_workspace_bytes; the latter keep their partial sums in its header); from 11 activation
- * rows on, a stack that has column orders (and C % 64 == 0, 16-byte aligned x, ldx % 8 == 0) is decoded to
- * fp16 in the workspace and multiplied by the tile GEMM, which is faster than its decode-time kernel there. */
+ * sq_workspace_bytes; the latter keep their partial sums in its header); from 3 to 17 activation rows on, depending
+ * on the stack (csrc/sq_gemm.hip), one that has column orders (with C % 8 == 0, 16-byte aligned x, ldx % 8 == 0) is decoded
+ * to fp16 in the workspace and multiplied from there, which is faster than its decode-time kernel. */
 #define SQ_SMALL_BMAX 32
 int sq_linear_small(const sq_matrix* mats, int32_t n_mats, const void* x, int x_dtype, int64_t ldx,
                     void* y, int y_dtype, int64_t ldy, int32_t B, void* workspace, size_t ws_bytes,
@@ -80,7 +80,9 @@ int sq_linear_small(const sq_matrix* mats, int32_t n_mats, const void* x, int x_
  * arguments, same kernels and bit-identical results, with the workspace (header included) kept in a device array
  * of SQ_NOALLOC_SCRATCH_BYTES that the library itself holds on every GPU it runs on until the process ends.  It has no
  * counterpart in the reference (whose launchers grow torch buffers on demand).  Pieces and row counts whose workspace
- * (sq_workspace_bytes(mats, n_mats, B, 0)) exceeds the array are refused with SQ_EWORKSPACE; nothing is allocated or freed,
+ * (sq_workspace_bytes(mats, n_mats, B, 0)) exceeds the array are refused with SQ_EWORKSPACE, except stacks with column orders
+ * that need so much for their decoded weights only, at up to 10 rows or with C % 64 != 0: those run on the decode-time
+ * kernel, whose results may differ from sq_linear_small's in the order of fp32 additions.  Nothing is allocated or freed,
  * here or in anything it calls.  All calls on one GPU share that GPU's array: calls that overlap in time on one GPU
  * (two streams, two threads) race; calls on one stream are safe. */
 #define SQ_NOALLOC_SCRATCH_BYTES (48u << 20)

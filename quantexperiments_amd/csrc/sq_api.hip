@@ -131,6 +131,10 @@ int sq_linear_small(const sq_matrix* mats, int32_t n_mats, const void* x, int x_
 static_assert(sq::SQ_WS_HEADER == SQ_WS_HEADER_BYTES, "the header size is part of the ABI");
 static __device__ __align__(256) unsigned char g_static_scratch[SQ_NOALLOC_SCRATCH_BYTES];
 static std::atomic<void*> g_static_scratch_ptr[64];
+// Rows up to which a stack with column orders whose decoded weights the scratch cannot hold runs on the decode-time kernel instead
+// of being refused.  Above, where that kernel is several times slower than the decode (see masked_gemm), the caller is told to
+// bring a workspace; rows that are no multiple of 64 columns, whose route through decoded weights is a later addition, run there at
+// every row count.
 constexpr int NOALLOC_ROWS_IN_PLACE = 10;
 
 // This device's copy of the scratch array (its address, looked up on first use with the device current), or nullptr +
@@ -156,18 +160,18 @@ int sq_linear_small_noalloc(const sq_matrix* mats, int32_t n_mats, const void* x
     if (B > SQ_SMALL_BMAX) return fail(SQ_EINVAL, "sq_linear_small_noalloc: B %d > %d", B, SQ_SMALL_BMAX);
     if (B == 0 || n_mats == 0) return SQ_OK;
     const size_t inner = (size_t)SQ_NOALLOC_SCRATCH_BYTES - SQ_WS_HEADER;
-    // a stack with column orders whose decoded weights do not fit takes the decode-time kernel, up to the rows where that is
-    // several times slower
-    const bool route = small_takes_gemm_route(mats, n_mats, B, x, ldx);
-    const bool in_place = route && B <= NOALLOC_ROWS_IN_PLACE && small_gemm_route_workspace(mats, n_mats, B) > inner;
-    const size_t need = in_place ? small_workspace(mats, n_mats, B) + SQ_WS_HEADER : sq_workspace_bytes(mats, n_mats, B, 0);
-    if (need > (size_t)SQ_NOALLOC_SCRATCH_BYTES)
+    // a stack whose decoded weights do not fit takes the decode-time kernel instead (as it does where x is not aligned for the other)
+    const size_t small = small_workspace(mats, n_mats, B), decoded = small_gemm_route_workspace(mats, n_mats, B);
+    const bool in_place = decoded > inner && (B <= NOALLOC_ROWS_IN_PLACE || mats[0].C % 64);
+    const bool route = !in_place && small_takes_gemm_route(mats, n_mats, B, x, ldx);
+    const size_t need = in_place ? small : std::max(small, decoded > inner ? gemm_workspace_without_mid(mats, n_mats, B) : decoded);
+    if (need > inner)
         return fail(SQ_EWORKSPACE, "sq_linear_small_noalloc: these pieces need %zu bytes of workspace at %d rows, the built-in scratch holds %u "
-                                   "(use sq_linear_small with a workspace of the caller's)", need, B, (unsigned)SQ_NOALLOC_SCRATCH_BYTES);
+                                   "(use sq_linear_small with a workspace of the caller's)", need + SQ_WS_HEADER, B, (unsigned)SQ_NOALLOC_SCRATCH_BYTES);
     if ((rc = refuse_if_poisoned("sq_linear_small_noalloc", mats, n_mats))) return rc;
     char* ws = (char*)static_scratch();
     if (!ws) return SQ_ELAUNCH;
-    if (route && !in_place)
+    if (route)
         return launch_gemm(mats, n_mats, x, x_dtype, ldx, y, y_dtype, ldy, B, ws + SQ_WS_HEADER, inner, ws, (hipStream_t)stream);
     return launch_small(mats, n_mats, x, x_dtype, ldx, y, y_dtype, ldy, B, ws + SQ_WS_HEADER, inner, ws, (hipStream_t)stream);
 }

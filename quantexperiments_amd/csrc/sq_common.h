@@ -154,6 +154,8 @@ int launch_mid_decoded(const sq_matrix* mats, int n, const void* const* w, const
 // for these pieces (0: never), where they cannot share a pass
 int small_pass_limit(const sq_matrix* mats, int n);
 size_t gemm_workspace(const sq_matrix* mats, int n, int T);
+// what launch_gemm can do with less: the same product without the kernel of sq_mid.h
+size_t gemm_workspace_without_mid(const sq_matrix* mats, int n, int T);
 // Row scales of a product whose R rows are n stacked pieces: rows end[i - 1] .. end[i] - 1 are scaled by p[i]; n = 0: no scales.
 constexpr int GEMM256_PIECES = 4;
 struct Gemm256Scales { const uint16_t* p[GEMM256_PIECES]; int end[GEMM256_PIECES]; int n; };

@@ -277,7 +277,6 @@ size_t small_gemm_route_workspace(const sq_matrix* mats, int n, int B) {
 }
 
 static size_t gemm_workspace_beyond_small(const sq_matrix* mats, int n, int T);
-static size_t gemm_workspace_without_mid(const sq_matrix* mats, int n, int T);
 
 size_t gemm_workspace(const sq_matrix* mats, int n, int T) {
     // up to SQ_SMALL_BMAX rows sq_linear_gemm is sq_linear_small, unless the stack goes the other way (see above);
@@ -294,7 +293,7 @@ static size_t gemm_workspace_beyond_small(const sq_matrix* mats, int n, int T) {
     return decoded_route(mats, n, T) ? std::max(rest, decoded_workspace(mats, n, T)) : rest;
 }
 
-static size_t gemm_workspace_without_mid(const sq_matrix* mats, int n, int T) {
+size_t gemm_workspace_without_mid(const sq_matrix* mats, int n, int T) {
     if (T > SQ_SMALL_BMAX && T <= small_pass_limit(mats, n)) {
         // full passes and the last, shorter one may run different kernels with different needs
         const size_t full = small_workspace(mats, n, SQ_SMALL_BMAX);
@@ -379,9 +378,10 @@ int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_
         }
         return SQ_OK;
     }
-    if (gemm_workspace(mats, n, T) > ws_bytes)
+    if (decoded_route(mats, n, T) && mid_x_ok(ldx, T) && decoded_workspace(mats, n, T) <= ws_bytes)
+        return launch_decoded(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);
+    if (gemm_workspace_without_mid(mats, n, T) > ws_bytes)
         return fail(SQ_EWORKSPACE, "sq_linear_gemm: workspace %zu < %zu", ws_bytes, gemm_workspace(mats, n, T));
-    if (decoded_route(mats, n, T) && mid_x_ok(ldx, T)) return launch_decoded(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);
     if (big_route(mats, n, T)) {
         const int C = mats[0].C;
         const uint16_t* xh = (const uint16_t*)x;

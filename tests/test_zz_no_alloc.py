@@ -1,14 +1,16 @@
 """sq_linear_small_noalloc (the entry point that allocates nothing: its workspace is a device array inside the
 library) against sq_linear_small with a caller-owned workspace: same kernels, so the outputs must be the same
-bits.  Two calls in a row, the second on a smaller input, through the C ABI."""
+bits.  Two calls in a row, the second on a smaller input, through the C ABI.  Stacks with column orders whose
+product through decoded weights does not fit, against the oracle."""
 
 import ctypes
 
+import numpy as np
 import pytest
 import torch
 
 from quantexperiments_amd import _lib
-from tests.helpers import rand_x, synth, to_device
+from tests.helpers import rand_x, rel_max_err, synth, to_device
 
 pytestmark = pytest.mark.gpu
 
@@ -69,6 +71,30 @@ def test_noalloc_refuses_what_does_not_fit():
     rc = L.sq_linear_small_noalloc(mats, 1, x.data_ptr(), _lib.SQ_BF16, C, y.data_ptr(), _lib.SQ_BF16, R, B, _lib.stream_ptr(x.device))
     assert rc == _lib.SQ_EWORKSPACE and b"built-in scratch" in L.sq_last_error()
     assert L.sq_linear_small_noalloc(mats, 1, x.data_ptr(), _lib.SQ_BF16, C, y.data_ptr(), _lib.SQ_BF16, R, 0, None) == 0
+
+
+# decoded these take more than the 16 MiB behind the header: (R, C, d, bits, M, B, columns that x is off its 16-byte alignment)
+TOO_LARGE = [(2400, 3584, 4, 12, 4, 5, 0), (2400, 3584, 4, 12, 4, 10, 0), (2400, 3584, 4, 12, 4, 7, 1), (1000, 9216, 4, 12, 4, 3, 0),
+            (2400, 3616, 4, 12, 4, 11, 0), (2400, 3616, 4, 12, 4, 32, 0), (2400, 3592, 4, 12, 4, 19, 0), (2400, 3592, 8, 16, 4, 11, 0),
+            (2400, 3592, 8, 16, 16, 32, 0), (2400, 3592, 8, 16, 4, 12, 1),
+            (14473, 512, 4, 10, 2, 17, 0)]      # (only the partial sums do not fit: decoded, in tiles)
+
+
+@pytest.mark.parametrize("case", TOO_LARGE, ids=lambda c: "x".join(map(str, c)))
+def test_noalloc_where_the_decoded_product_does_not_fit(case):
+    R, C, d, bits, M, B, off = case
+    L, s = _lib.lib(), synth(R, C, d, bits, 1, M, seed=B)
+    lin = to_device(s)
+    mats = _lib.matrix_array([lin.descriptor(0)])
+    assert L.sq_workspace_bytes(mats, 1, B, 0) > _lib.NOALLOC_SCRATCH_BYTES
+    x = rand_x(B, C, torch.bfloat16, seed=B)
+    buf = torch.zeros(B, C + 8, dtype=torch.bfloat16, device="cuda")
+    xd = buf[:, off:off + C]
+    xd.copy_(x)
+    y = torch.full((B, R), float("nan"), device="cuda")
+    _lib.check(L.sq_linear_small_noalloc(mats, 1, xd.data_ptr(), _lib.SQ_BF16, C + 8, y.data_ptr(), _lib.SQ_F32, R, B, _lib.stream_ptr(xd.device)))
+    ref = x.double().numpy() @ s.decode().astype(np.float64).T
+    assert rel_max_err(y.cpu().numpy(), ref) < 1e-3
 
 
 def test_noalloc_under_graph_capture_allocates_nothing():
