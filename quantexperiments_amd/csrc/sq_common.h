@@ -138,7 +138,7 @@ int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_
 // stacks with column orders and more than a few activation rows: sq_linear_small runs the decode + tile GEMM route
 bool small_takes_gemm_route(const sq_matrix* mats, int n, int B, const void* x, int64_t ldx);
 size_t small_gemm_route_workspace(const sq_matrix* mats, int n, int B);
-constexpr int MID_PIECES = 4;
+constexpr int MID_PIECES = 8;          // (kernel arguments of 1 KB)
 // 33 .. a few hundred activation rows in one pass over the tags (sq_mid.h): whether these pieces can take it, and its call
 bool mma_shape(const sq_matrix& m);
 bool mid_ok(const sq_matrix* mats, int n, int T);
@@ -157,7 +157,9 @@ size_t gemm_workspace(const sq_matrix* mats, int n, int T);
 // what launch_gemm can do with less: the same product without the kernel of sq_mid.h
 size_t gemm_workspace_without_mid(const sq_matrix* mats, int n, int T);
 // Row scales of a product whose R rows are n stacked pieces: rows end[i - 1] .. end[i] - 1 are scaled by p[i]; n = 0: no scales.
-constexpr int GEMM256_PIECES = 4;
+// (Eight: kernel arguments of 1 KB in the stacked decode; longer stacks take a product per eight pieces.  Four had sent stacks of five
+// pieces through five products.)
+constexpr int GEMM256_PIECES = 8;
 struct Gemm256Scales { const uint16_t* p[GEMM256_PIECES]; int end[GEMM256_PIECES]; int n; };
 int launch_gemm_dense(const void* w, int w_dtype, int64_t ldw, int R, int C, const void* x, int x_dtype, int64_t ldx,
                       void* y, int y_dtype, int64_t ldy, int T, hipStream_t s, void* ws = nullptr, size_t ws_bytes = 0);

@@ -180,10 +180,11 @@ static bool big_route(const sq_matrix* mats, int n, int T) {
 // Pieces that are neighbours in Y are decoded one behind the other and multiplied in ONE tile GEMM over all their
 // rows: a 512-row k or v projection alone is 2 tiles of 256 rows, a
 // launch that leaves the chip idle (7B q|k|v at 64-255 rows: 139 us as three products, the o projection of q's
-// size: 62 us).
+// size: 62 us; 8 pieces of 1024 x 3584 at 333 / 1024 / 2048 rows, 16-bit tags of width 8: 257 / 267 / 304 us one by one,
+// 90 / 106 / 148 in one).
 constexpr size_t STACK_MAX_BYTES = (size_t)1 << 30;
 static bool stacked_route(const sq_matrix* mats, int n) {
-    if (n < 2 || n > GEMM256_PIECES) return false;
+    if (n < 2) return false;
     size_t tot = 0;
     for (int i = 0; i < n; ++i) {
         if (mats[i].R <= 0) return false;
@@ -196,6 +197,11 @@ static int stacked_rows(const sq_matrix* mats, int n) {
     int r = 0;
     for (int i = 0; i < n; ++i) r += mats[i].R;
     return r;
+}
+static size_t stacked_bytes(const sq_matrix* mats, int n) {
+    size_t b = 0;
+    for (int i = 0; i < n; ++i) b += dense_bytes(mats[i]);
+    return b;
 }
 
 // Up to 256 activation rows of what cannot go in one pass over the tags (sq_mid.h): column orders, formats whose rows are not
@@ -303,9 +309,11 @@ size_t gemm_workspace_without_mid(const sq_matrix* mats, int n, int T) {
     size_t need = 0;
     const bool big = big_route(mats, n, T);
     if (big && stacked_route(mats, n)) {
-        const int R = stacked_rows(mats, n);
-        for (int i = 0; i < n; ++i) need += dense_bytes(mats[i]);
-        return need + align256((size_t)T * mats[0].C * 2) + gemm256_part_bytes(T, R, mats[0].C, device_cus());
+        for (int i = 0; i < n; i += GEMM256_PIECES) {
+            const int k = std::min(n - i, GEMM256_PIECES);
+            need = std::max(need, stacked_bytes(mats + i, k) + gemm256_part_bytes(T, stacked_rows(mats + i, k), mats[0].C, device_cus()));
+        }
+        return need + align256((size_t)T * mats[0].C * 2);
     }
     for (int i = 0; i < n; ++i)
         if ((big || !fused_ok(mats[i])) && dense_bytes(mats[i]) > need) need = dense_bytes(mats[i]);
@@ -413,27 +421,30 @@ int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_
         wd += align256((size_t)T * C * 2);
         const int cus0 = device_cus();
         if (stacked_route(mats, n)) {
-            const int R = stacked_rows(mats, n);
-            char* next = wd;
-            for (int i = 0; i < n; ++i) next += dense_bytes(mats[i]);
-            float* part = (float*)next;
-            char* w = wd;
-            Gemm256Scales sc{};
-            int r0 = 0;
-            const int whole = decode_stack(mats, n, w);         // all pieces in one launch, or (1) piece by piece
-            if (whole < 0) return whole;
-            for (int i = 0; i < n; ++i) {
-                const sq_matrix& m = mats[i];
-                if (whole == 1)
-                    if (int rc = decode(m, w)) return rc;
-                w += (size_t)m.R * C * 2;                       // rows follow each other without gaps
-                r0 += m.R;
-                sc.p[i] = m.row_scale;
-                sc.end[i] = r0;
+            for (int i0 = 0; i0 < n; i0 += GEMM256_PIECES) {
+                const sq_matrix* ms = mats + i0;
+                const int k = std::min(n - i0, GEMM256_PIECES), R = stacked_rows(ms, k);
+                float* part = (float*)(wd + stacked_bytes(ms, k));
+                char* w = wd;
+                Gemm256Scales sc{};
+                int r0 = 0;
+                const int whole = decode_stack(ms, k, w);       // all pieces in one launch, or (1) piece by piece
+                if (whole < 0) return whole;
+                for (int i = 0; i < k; ++i) {
+                    const sq_matrix& m = ms[i];
+                    if (whole == 1)
+                        if (int rc = decode(m, w)) return rc;
+                    w += (size_t)m.R * C * 2;                   // rows follow each other without gaps
+                    r0 += m.R;
+                    sc.p[i] = m.row_scale;
+                    sc.end[i] = r0;
+                }
+                sc.n = k;
+                if (int rc = launch_gemm256(xh, ldxh, (const uint16_t*)wd, C, sc, y, y_dtype, ldy, ms[0].y_off, T, R, C,
+                                            gemm256_part_bytes(T, R, C, cus0) ? part : nullptr, cus0, s))
+                    return rc;
             }
-            sc.n = n;
-            return launch_gemm256(xh, ldxh, (const uint16_t*)wd, C, sc, y, y_dtype, ldy, mats[0].y_off, T, R, C,
-                                  gemm256_part_bytes(T, R, C, cus0) ? part : nullptr, cus0, s);
+            return SQ_OK;
         }
         size_t dense = 0;
         for (int i = 0; i < n; ++i) dense = std::max(dense, dense_bytes(mats[i]));

@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 import torch
 
+from quantexperiments_amd import _lib
 from quantexperiments_amd.kernels import gemm_dense, linear_gemm
 from tests.helpers import rand_x, rel_max_err, synth, to_device
 
@@ -31,6 +32,30 @@ def test_stack_of_pieces(n):
     linear_gemm([to_device(s, stream=False) for s in ss], x.cuda(), y)
     ref = np.concatenate([x.float().numpy().astype(np.float64) @ s.decode().astype(np.float64).T for s in ss], axis=1)
     assert rel_max_err(y.cpu().numpy(), ref) < 1e-3
+
+
+@pytest.mark.parametrize("n", [5, 8, 9, 17])
+@pytest.mark.parametrize("d,bits,M", [(8, 16, 1), (8, 16, 3), (4, 12, 1)])
+def test_long_stacks(n, d, bits, M):
+    """Stacks of more pieces than a launch scales: a product per eight, each piece with its own scales and at its own columns; and
+    their workspace, a joint product's per eight pieces."""
+    L, T, C = _lib.lib(), 400, 512
+    ss = [synth(33 + 8 * i, C, d, bits, 1, M, seed=i) for i in range(n)]
+    lins = [to_device(s, stream=False) for s in ss]
+    x = rand_x(T, C, torch.bfloat16, seed=n)
+    rows = sum(s.R for s in ss)
+    y = torch.full((T, rows), float("nan"), dtype=torch.float32, device="cuda")
+    linear_gemm(lins, x.cuda(), y)
+    ref = np.concatenate([x.float().numpy().astype(np.float64) @ s.decode().astype(np.float64).T for s in ss], axis=1)
+    assert rel_max_err(y.cpu().numpy(), ref) < 1e-3
+    dense = lambda of: sum((s.R * C * 2 + 255) // 256 * 256 for s in of)
+    off, mats = 0, []
+    for lin in lins:
+        mats.append(lin.descriptor(off))
+        off += lin.R
+    need = L.sq_workspace_bytes(_lib.matrix_array(mats), n, T, 1) - _lib.WS_HEADER - T * C * 2
+    most = max(dense(ss[i:i + 8]) for i in range(0, n, 8))
+    assert need >= most and need - most < 64 << 20
 
 
 @pytest.mark.parametrize("T,R,C", [

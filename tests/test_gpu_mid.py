@@ -16,6 +16,7 @@ CASES = [  # rows of the stack's pieces, C, d, bits, G, T
     ((66,), 704, 8, 16, 1, 256), ((33000,), 128, 8, 16, 1, 250),
     ((1,), 32, 4, 12, 1, 80), ((127, 3, 260), 1056, 4, 12, 1, 128), ((130,), 2080, 4, 12, 4, 129), ((64, 70), 1024, 4, 12, 4, 256),
     ((33001,), 160, 4, 12, 1, 193), ((32768,), 96, 4, 12, 1, 241), ((4096,), 16384, 4, 12, 1, 257),
+    ((16, 1, 130, 40, 7, 64, 33, 20), 512, 8, 16, 1, 70), ((30, 1, 17, 64, 8, 9, 130), 1024, 4, 12, 1, 40), ((24,) * 9, 512, 8, 16, 1, 90),
     ((257,), 576, 4, 10, 1, 192), ((40, 8), 1600, 4, 10, 2, 34), ((131,), 1536, 4, 8, 1, 129), ((36,), 64, 4, 8, 1, 255),
 ]
 
@@ -42,6 +43,7 @@ DECODED = [  # rows of the stack's pieces, C, d, bits, G, M, T: column orders, r
     ((1,), 8, 8, 16, 1, 1, 33), ((129, 1, 300), 1984, 8, 16, 1, 16, 15), ((16,), 1984, 8, 16, 1, 16, 256), ((130,), 72, 8, 16, 1, 3, 5),
     ((70, 50), 1000, 4, 12, 1, 1, 48), ((50, 16), 264, 4, 10, 4, 1, 193), ((257,), 520, 4, 8, 1, 2, 128), ((40, 40, 40, 40, 7), 512, 8, 16, 1, 2, 17),
     ((33,), 9216, 8, 16, 1, 16, 3), ((12,), 200, 2, 5, 3, 1, 81), ((3584,), 776, 8, 16, 1, 1, 100),
+    ((24, 1, 33, 40, 7, 64, 9, 12, 20), 520, 8, 16, 1, 3, 60),
     ((12500, 100), 2048, 8, 16, 1, 16, 129),      # past 128 rows and 24 M weights, in tiles
 ]
 
