@@ -95,8 +95,9 @@ int sq_linear_small_noalloc(const sq_matrix* mats, int32_t n_mats, const void* x
  * M > 1 are decoded with their column orders into workspace and multiplied from there.  Between
  * SQ_SMALL_BMAX + 1 and 256 rows (384 for large matrices with the codebook in LDS) pieces without column
  * orders gather their codewords once for all rows, in one pass over the packed tags, which is cheaper than
- * decoding the matrix first (pieces whose formats differ: passes of SQ_SMALL_BMAX rows), and up to SQ_SMALL_BMAX rows the call is sq_linear_small; sq_workspace_bytes(which = 1)
- * accounts for whichever route T takes. */
+ * decoding the matrix first (pieces whose formats differ: passes of SQ_SMALL_BMAX rows).  Rows that are no whole lane units and
+ * column orders are decoded up to 256 rows too, into at most 192 MB of workspace at a time.  Up to SQ_SMALL_BMAX rows the call is
+ * sq_linear_small; sq_workspace_bytes(which = 1) accounts for whichever route T takes. */
 int sq_linear_gemm(const sq_matrix* mats, int32_t n_mats, const void* x, int x_dtype, int64_t ldx,
                    void* y, int y_dtype, int64_t ldy, int32_t T, void* workspace, size_t ws_bytes,
                    void* stream);

@@ -205,16 +205,42 @@ static size_t stacked_bytes(const sq_matrix* mats, int n) {
 }
 
 // Up to 256 activation rows of what cannot go in one pass over the tags (sq_mid.h): column orders, formats whose rows are not
-// whole lane units, codebooks too large for it.  Pieces are decoded, as many as a launch and STACK_MAX_BYTES take, and multiplied
-// straight from there.
-static int decoded_group(const sq_matrix* mats, int n, int i0, int T) {
-    int k = 0;
-    size_t tot = 0;
-    while (i0 + k < n && k < MID_PIECES && mats[i0 + k].R > 0 && (k == 0 || tot + dense_bytes(mats[i0 + k]) <= STACK_MAX_BYTES)) {
-        if (!mid_dense_ok(mats + i0, k + 1, T)) break;
-        tot += dense_bytes(mats[i0 + k++]);
+// whole lane units, codebooks too large for it.  Rows are decoded and multiplied straight from there, as many at a time as
+// DECODED_BYTES of workspace hold, evenly cut and across the ends of pieces.  192 MB: what has just been decoded is then still in
+// the 256 MB last-level cache when it is multiplied, and the stacks and matrices below it, whose K is cut less the fewer rows a
+// step has, stay in one (37888 rows of 3592 columns in two steps instead of one at 40 / 128 / 256 rows 156 / 173 / 254 us instead
+// of 215 / 239 / 319, in three 177 / 199 / 275; 34816 x 5128 198 / 230 / 342 instead of 303 / 333 / 435; 5120 x 17416 whole 91 /
+// 102 / 133, in two 117 / 136 / 188).
+constexpr size_t DECODED_BYTES = (size_t)192 << 20;
+struct DecodedRows { sq_matrix m[MID_PIECES]; const sq_matrix* of[MID_PIECES]; int r0[MID_PIECES], n; size_t bytes; };
+
+static int decoded_step_rows(const sq_matrix* mats, int n) {
+    int64_t rows = 0;
+    for (int i = 0; i < n; ++i) rows += mats[i].R;
+    const int64_t bytes = rows * mats[0].C * 2, steps = std::max<int64_t>(1, (bytes + DECODED_BYTES - 1) / DECODED_BYTES);
+    return (int)((rows + steps * 128 - 1) / (steps * 128) * 128);
+}
+
+// The step that begins at row r0 of piece i, each of its parts as a piece of its own to the kernel (which reads the scales and
+// the place in Y of decoded rows, not their tags); i and r0 move behind it.
+static DecodedRows decoded_step(const sq_matrix* mats, int n, int& i, int& r0) {
+    DecodedRows d;
+    d.n = 0; d.bytes = 0;
+    int left = decoded_step_rows(mats, n);
+    while (i < n && d.n < MID_PIECES && left > 0) {
+        const int R = std::min(mats[i].R - r0, left);
+        if (R > 0) {
+            sq_matrix& m = d.m[d.n] = mats[i];
+            m.R = R; m.row_scale += r0; m.y_off += r0;
+            d.of[d.n] = mats + i;
+            d.r0[d.n++] = r0;
+            d.bytes += dense_bytes(m);
+        }
+        left -= R;
+        r0 += R;
+        if (r0 >= mats[i].R) ++i, r0 = 0;
     }
-    return k;
+    return d;
 }
 
 // Where the tile GEMM, whose workgroups read less, is the faster one behind the same decode: with more rows than half the CUs'
@@ -226,7 +252,7 @@ static bool decoded_route(const sq_matrix* mats, int n, int T) {
     int64_t rows = 0;
     for (int i = 0; i < n; ++i) {
         rows += mats[i].R;
-        if (mats[i].R > 0 && (!mats[i].tags || !decoded_group(mats, n, i, T))) return false;
+        if (mats[i].R > 0 && (!mats[i].tags || !mid_dense_ok(mats + i, 1, T))) return false;
     }
     if (mats[0].C % 64) return true;
     return rows < (int64_t)128 * device_cus() && (T <= 128 || rows * mats[0].C < (int64_t)24 << 20);
@@ -234,28 +260,26 @@ static bool decoded_route(const sq_matrix* mats, int n, int T) {
 
 static size_t decoded_workspace(const sq_matrix* mats, int n, int T) {
     size_t need = 0;
-    for (int i = 0, k; i < n; i += std::max(k, 1)) {
-        k = decoded_group(mats, n, i, T);
-        size_t tot = k ? mid_dense_workspace(mats + i, k, T) : 0;
-        for (int j = 0; j < k; ++j) tot += dense_bytes(mats[i + j]);
-        need = std::max(need, tot);
+    for (int i = 0, r0 = 0; i < n;) {
+        const DecodedRows d = decoded_step(mats, n, i, r0);
+        if (d.n) need = std::max(need, d.bytes + mid_dense_workspace(d.m, d.n, T));
     }
     return need;
 }
 
 static int launch_decoded(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws,
                           hipStream_t s) {
-    for (int i = 0, k; i < n; i += std::max(k, 1)) {
-        k = decoded_group(mats, n, i, T);
+    for (int i = 0, r0 = 0; i < n;) {
+        const DecodedRows d = decoded_step(mats, n, i, r0);
         const void* w[MID_PIECES];
         char* next = (char*)ws;
-        for (int j = 0; j < k; ++j) {
+        for (int j = 0; j < d.n; ++j) {
             w[j] = next;
-            if (const int rc = launch_dequant(mats[i + j], next, SQ_F16, mats[i + j].C, 0, mats[i + j].R, s, /*raw=*/true)) return rc;
-            next += dense_bytes(mats[i + j]);
+            if (const int rc = launch_dequant(*d.of[j], next, SQ_F16, mats[0].C, d.r0[j], d.r0[j] + d.m[j].R, s, /*raw=*/true)) return rc;
+            next += dense_bytes(d.m[j]);
         }
-        if (k)
-            if (const int rc = launch_mid_decoded(mats + i, k, w, x, x_dtype, ldx, y, y_dtype, ldy, T, next, s)) return rc;
+        if (d.n)
+            if (const int rc = launch_mid_decoded(d.m, d.n, w, x, x_dtype, ldx, y, y_dtype, ldy, T, next, s)) return rc;
     }
     return SQ_OK;
 }

@@ -153,3 +153,24 @@ def test_neighbour_entry_points_check_arguments_on_the_host():
     assert L.sq_linear_small_from(m, 0, ctypes.byref(pr), bf, p, bf, 64, 1, None, 0, None) == _lib.SQ_EINVAL        # unknown mode
     pr.mode = _lib.SQ_FROM_SILU_MUL
     assert L.sq_linear_small_from(m, 0, ctypes.byref(pr), bf, p, bf, 64, 1, None, 0, None) == _lib.SQ_OK            # no pieces
+
+
+def test_workspace_of_decoded_weights_is_bounded():
+    """Ragged rows and column orders at 33 to 256 activation rows are decoded into the workspace, 192 MB of fp16 at a time."""
+    L, step = _lib.lib(), 192 << 20
+
+    def need(rows, C, d, bits, M, T, which=1):
+        mats, off = [], 0
+        for R in rows:
+            mats.append(_lib.SqMatrix(0x10000, 0x20000, 0x30000, None, 0x50000 if M > 1 else None, 0x60000 if M > 1 else None, None, R, C, d, bits,
+                                      1, M, (C // d * bits + 31) // 32, off))
+            off += R
+        return L.sq_workspace_bytes(_lib.matrix_array(mats), len(rows), T, which) - _lib.WS_HEADER
+
+    for rows in ((18944, 18944), (40000,), (100, 90000, 7), (1000,) * 8, (300000,)):
+        for d, bits in ((8, 16), (4, 12)):
+            for T in (33, 128, 256):
+                for C in (3592, 5128):
+                    dense = sum(rows) * C * 2
+                    assert min(dense, step // 2) <= need(rows, C, d, bits, 1, T) <= min(dense + 4096, step) + 8 * T * 128 * 256 * 4
+    assert need((24, 7), 3592, 8, 16, 16, 20, 0) >= 31 * 3592 * 2                     # decode sizes with column orders go the same way

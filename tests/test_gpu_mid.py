@@ -44,6 +44,7 @@ DECODED = [  # rows of the stack's pieces, C, d, bits, G, M, T: column orders, r
     ((70, 50), 1000, 4, 12, 1, 1, 48), ((50, 16), 264, 4, 10, 4, 1, 193), ((257,), 520, 4, 8, 1, 2, 128), ((40, 40, 40, 40, 7), 512, 8, 16, 1, 2, 17),
     ((33,), 9216, 8, 16, 1, 16, 3), ((12,), 200, 2, 5, 3, 1, 81), ((3584,), 776, 8, 16, 1, 1, 100),
     ((24, 1, 33, 40, 7, 64, 9, 12, 20), 520, 8, 16, 1, 3, 60),
+    ((26000, 300, 29000), 1992, 8, 16, 1, 1, 70), ((57000,), 2056, 4, 8, 1, 2, 40),      # in two steps, cut inside a piece
     ((12500, 100), 2048, 8, 16, 1, 16, 129),      # past 128 rows and 24 M weights, in tiles
 ]
 
