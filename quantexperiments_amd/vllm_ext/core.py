@@ -28,7 +28,13 @@ from ..kernels import (PackedLinear, _Workspace, gemm_dense, linear_gemm, linear
                        q8_linear)
 
 BMAX = _lib.SMALL_BMAX
-STACK_MAX_BYTES = 1 << 30       # most fp16 weights the "dequant" route decodes side by side for one product
+# Most fp16 weights of neighbouring pieces that the "dequant" route decodes side by side for one product (a larger piece goes
+# alone): up to JOINT_ROWS activation rows, and above.  192 MB stay in the 256 MB last-level cache until they are multiplied;
+# with more rows that gain can be less than what two partial rounds of tiles lose against one.  Together / apart, us: 2 x 18944 x
+# 3584, 259 MB, at 40 / 128 rows 204 / 210 and 162 / 172, at 1024 / 2048 400 / 615 and 422 / 639; 18944, 4736, 4736 x 5120, 277 MB
+# (apart: 185 and 92), 227 / 233 and 205 / 215, at 333 / 512 rows 261 / 289 and 284 / 324; 5120, 1024, 1024 x 5120, 70 MB, at 40 /
+# 333 / 1024 81 / 92 / 127 and 117 / 133 / 176.
+JOINT_BYTES, JOINT_ROWS, JOINT_BYTES_MANY_ROWS = 192 << 20, 256, 384 << 20
 
 # checkpoint suffix of each vLLM (possibly stacked) linear -> the packed pieces, in output order
 STACKED = {
@@ -96,6 +102,17 @@ def _graph_ms(fn, calls: int = 10, reps: int = 5) -> float:
         end.record()
     torch.cuda.synchronize()
     return statistics.median(b.elapsed_time(e) for b, e in marks) / calls
+
+
+def joint_pieces(Rs: list, C: int, M: int) -> list:
+    """(first, end) of the runs of pieces that the "dequant" route multiplies together at M activation rows."""
+    limit, groups = JOINT_BYTES if M <= JOINT_ROWS else JOINT_BYTES_MANY_ROWS, []
+    for i in range(len(Rs)):
+        if groups and sum(Rs[groups[-1][0]:i + 1]) * C * 2 <= limit:
+            groups[-1] = (groups[-1][0], i + 1)
+        else:
+            groups.append((i, i + 1))
+    return groups
 
 
 class PackedShards:
@@ -233,12 +250,19 @@ class PackedShards:
         # fp16 in the shared scratch, each multiplied into its column slice of Y
         if x.dtype != torch.float16 and M > BMAX and self.C % 64 == 0:
             x = x.to(torch.float16)                     # fp16 x fp16 takes the 256 x 256 tile kernel; y keeps its dtype
-        if self.large == "dequant" and self.R * self.C * 2 <= STACK_MAX_BYTES:
-            # one product over the stack: a 1024-row k or v projection alone is a few tiles on an idle chip
-            w = _Workspace.get(self.R * self.C * 2, x.device, kind="dense").view(torch.float16)[:self.R * self.C].view(self.R, self.C)
-            for rl, off in zip(self.rls, self.offs):
-                rl.dense(torch.float16, out=w[off:off + rl.R])
-            return gemm_dense(w, x, y)
+        if self.large == "dequant":
+            # one product over pieces that fit together: a 1024-row k or v projection alone is a few tiles on an idle chip
+            groups = joint_pieces(self.Rs, self.C, M)
+            n = max(sum(self.Rs[i:j]) for i, j in groups) * self.C
+            scratch = _Workspace.get(n * 2, x.device, kind="dense").view(torch.float16)
+            for i, j in groups:
+                at = self.offs[i]
+                R = sum(self.Rs[i:j])
+                w = scratch[:R * self.C].view(R, self.C)
+                for rl, off in zip(self.rls[i:j], self.offs[i:j]):
+                    rl.dense(torch.float16, out=w[off - at:off - at + rl.R])
+                gemm_dense(w, x, y[:, at:at + R])
+            return y
         rows = max(self.Rs)
         if self.large == "chunked":
             rows = min(rows, max(128, (self.chunk_bytes // (2 * self.C)) // 128 * 128))

@@ -7,6 +7,7 @@ import torch
 
 from quantexperiments_amd import _lib
 from quantexperiments_amd.kernels import gemm_dense, linear_gemm
+from quantexperiments_amd.vllm_ext import core
 from tests.helpers import rand_x, rel_max_err, synth, to_device
 
 pytestmark = pytest.mark.gpu
@@ -75,3 +76,16 @@ def test_tile_heights(T, R, C, dtype):
     bound = 17.4 * C * 2.0 ** -24 + (2.0 ** -8 * ref.abs() if dtype == torch.bfloat16 else 0.0)
     assert ((y[:, :R].double() - ref).abs() <= bound).all()
     assert torch.isnan(y[:, R:]).all()
+
+
+@pytest.mark.parametrize("limit", [0, 150 * 512 * 2, 1 << 30])
+@pytest.mark.parametrize("T", [40, 800])
+def test_dequant_route_in_groups_of_pieces(limit, T, monkeypatch):
+    monkeypatch.setattr(core, "JOINT_BYTES", limit)
+    monkeypatch.setattr(core, "JOINT_BYTES_MANY_ROWS", limit)
+    ss = [synth(R, 512, 8, 16, 1, 3, seed=R) for R in (100, 40, 10, 141, 9)]
+    ps = core.PackedShards([to_device(s, stream=False) for s in ss], large="dequant")
+    x = rand_x(T, 512, torch.bfloat16, seed=T)
+    y = ps.forward(x.cuda())
+    ref = np.concatenate([x.float().numpy().astype(np.float64) @ s.decode().astype(np.float64).T for s in ss], axis=1)
+    assert rel_max_err(y.float().cpu().numpy(), ref) < 5e-3

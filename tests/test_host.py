@@ -830,3 +830,17 @@ def test_row_mask_is_checked_before_anything_runs(mask):
         PackedLinear(_OnGpu(3, 16), torch.zeros(1 << 16, 8), torch.ones(3), None, mask, perms, 1 << 16, 8)
     with pytest.raises(AttributeError):
         PackedLinear(_OnGpu(3, 16), torch.zeros(1 << 16, 8), torch.ones(3), None, torch.tensor([2, 0, 1]), perms, 1 << 16, 8)
+
+
+def test_pieces_decoded_side_by_side_are_bounded():
+    from quantexperiments_amd.vllm_ext.core import joint_pieces
+    assert joint_pieces([5120, 1024, 1024], 5120, 40) == [(0, 3)]
+    assert joint_pieces([18944, 18944], 3584, 256) == [(0, 1), (1, 2)] and joint_pieces([18944, 18944], 3584, 257) == [(0, 2)]
+    assert joint_pieces([28672, 28672], 8192, 4096) == [(0, 1), (1, 2)]
+    assert joint_pieces([20000, 5000, 5000, 64], 5120, 100) == [(0, 1), (1, 4)]
+    assert joint_pieces([64, 60000, 64, 64], 5120, 100) == [(0, 1), (1, 2), (2, 4)]
+    for M in (40, 4096):
+        for Rs in ([3000] * 9, [19660, 1], [19661, 1], [1] * 3, [40000]):
+            got = joint_pieces(Rs, 5120, M)
+            assert [i for i, _ in got] == [0] + [j for _, j in got[:-1]] and got[-1][1] == len(Rs)
+            assert all(j == i + 1 or sum(Rs[i:j]) * 5120 * 2 <= (192 if M <= 256 else 384) << 20 for i, j in got)
