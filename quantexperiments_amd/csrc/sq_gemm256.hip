@@ -88,9 +88,10 @@ __device__ __forceinline__ float gemm256_scale(const Gemm256Scales& s, int r) {
 
 constexpr int G_EP_PITCH = 128 * 2 + 16;     // bytes per token row of a wave's 32 MT x 128 output tile in LDS
 
-// s_waitcnt immediate that waits until at most n vector-memory operations are outstanding and leaves the
-// other counters alone (gfx9 encoding: vmcnt in bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8)
+// s_waitcnt immediate that waits until at most n vector-memory operations are outstanding (gfx9 encoding: vmcnt in bits 3:0 and
+// 15:14, expcnt 6:4, lgkmcnt 11:8) and leaves the other counters alone, or also until every LDS read of the wave has arrived
 constexpr int vmcnt_only(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
+constexpr int vmcnt_and_lds(int n) { return vmcnt_only(n) & ~(15 << 8); }
 
 // EP: SQ_F16 / SQ_BF16 = results of that type whose rows allow 16-byte stores, SQ_F32 = any type, element by element
 // MT: blocks of 32 token rows a wave holds, 64 MT rows a tile
@@ -231,10 +232,12 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a)
         step(0, 1, sx, sw, s + E - 1, to, 0, C1);
         step(1, 2, sx, sw, s + E - 1, to, C1, C2);
         step(0, 3, sx, sw, s + E - 1, to, C2, EC);
-        // last step: this wave's copies of slab s + 1 are waited for (those of later slabs stay in flight), then the
-        // barrier: everybody's have landed and everybody has read slab s to the end
+        // last step: this wave's copies of slab s + 1 are waited for (those of later slabs stay in flight), and its reads of slab
+        // s, whose slots the copies behind the barrier overwrite; then the barrier: everybody's copies have landed and
+        // everybody has read slab s to the end.  (The reads have arrived for the two products by now, so their wait costs
+        // nothing, but nothing else in the source would ask for all of them.)
         mma(1, 0); SQ_SB(); mma(1, 1); SQ_SB();
-        __builtin_amdgcn_s_waitcnt(vmcnt_only(AHEAD)); SQ_SB();
+        __builtin_amdgcn_s_waitcnt(vmcnt_and_lds(AHEAD)); SQ_SB();
         __builtin_amdgcn_s_barrier(); SQ_SB();
         read_x(0, 0, nx, 0); read_w(0, 0, nw, 0); SQ_SB();
 #pragma unroll
@@ -253,7 +256,7 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a)
     SQ_PIN();
 #undef SQ_SB
 #undef SQ_PIN
-    __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
+    __builtin_amdgcn_s_waitcnt(vmcnt_and_lds(0));
     __syncthreads();                         // every wave is done with the operand ring, and no copy is on its way into it
 
     // Results leave column of registers after column of registers.  A split tile's go to its partial tile as they are.  16-bit

@@ -174,3 +174,31 @@ def test_workspace_of_decoded_weights_is_bounded():
                     dense = sum(rows) * C * 2
                     assert min(dense, step // 2) <= need(rows, C, d, bits, 1, T) <= min(dense + 4096, step) + 8 * T * 128 * 256 * 4
     assert need((24, 7), 3592, 8, 16, 16, 20, 0) >= 31 * 3592 * 2                     # decode sizes with column orders go the same way
+
+
+def test_tile_gemm_waits_for_its_reads_before_the_barrier(tmp_path):
+    """Behind the barrier of a slab the ring's slots are overwritten by copies that no compiler dependence ties to the reads, so
+    the source itself has to wait for them: in the assembly of every variant the wait in front of a barrier behind LDS reads names
+    the LDS counter."""
+    import os
+    import subprocess
+    from quantexperiments_amd import build
+    try:
+        hipcc = build._hipcc()
+    except RuntimeError:
+        pytest.skip("no hipcc")
+    out = tmp_path / "gemm256.s"
+    subprocess.run([hipcc, *build.FLAGS, "-S", "--offload-device-only", str(build.CSRC / "sq_gemm256.hip"), "-o", str(out)], check=True,
+                   capture_output=True, env=dict(os.environ, TMPDIR=str(tmp_path)))
+    variants = 0
+    for body in re.split(r"(?m)^(?=_ZN2sq14gemm256_kernel\w+:)", out.read_text())[1:]:
+        lines = [l.split(";")[0].strip() for l in body[:body.index(".Lfunc_end")].splitlines()]
+        lines = [l for l in lines if l and not l.startswith(".")]
+        reads, waits = False, []
+        for i, l in enumerate(lines):
+            reads = reads or l.startswith("ds_read")
+            if l == "s_barrier" and reads:
+                waits.append(next(w for w in reversed(lines[:i]) if w.startswith("s_waitcnt")))
+        assert waits and all("lgkmcnt(0)" in w for w in waits), waits
+        variants += 1
+    assert variants == 9
