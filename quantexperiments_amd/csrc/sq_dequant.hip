@@ -142,9 +142,10 @@ __global__ __launch_bounds__(256) void dequant8x4_cvt_kernel(sq_matrix m, uint16
 // d = 4 without column orders, codebooks that fit LDS: persistent workgroups stage their piece's codebook in LDS and decode two
 // neighbouring chunks per lane and step, 16 bytes of 16-bit output (32 of fp32) stored in whole 16-byte pieces, so a wave
 // writes 1 KB of consecutive bytes per instruction.  Four steps are in flight per thread: tags of all four, then the gathers,
-// then the stores.  What bounds it is the write of the dense copy.  One thread per chunk with 2-byte stores and its codeword
-// gathered from L2 took 75 us for 18944 x 3584 (136 MB written), this takes 31.  Up to four stacked pieces share a launch (each
-// gets workgroups by its rows), and a bf16 activation matrix that the product needs as fp16 rides along.
+// then the stores.  What bounds it is the write of the dense copy (37888 x 3584 with the copy of 1024 activation rows: 279 MB written
+// and 64 read in 62 us, 5.5 TB/s, what a large copy reaches; LDS is busy 12 % of the time).  One thread per chunk with 2-byte stores
+// and its codeword gathered from L2 took 75 us for 18944 x 3584 (136 MB written), this takes 31.  Up to GEMM256_PIECES stacked pieces share a
+// launch (each gets workgroups by its rows), and a bf16 activation matrix that the product needs as fp16 rides along.
 struct Dequant4Args {
     sq_matrix m[GEMM256_PIECES];
     void* out[GEMM256_PIECES];

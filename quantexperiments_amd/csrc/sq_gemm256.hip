@@ -18,8 +18,10 @@
 // Eight waves of 128 x 64 (two per SIMD) ran at 1.15 PFLOP/s on 8192^3, in one schedule or as two groups taking turns at
 // matrix and memory phases, with 67 percent of the matrix cores' time used at 1.70 GHz; this one uses 83 percent of it at
 // 1.52 GHz (the chip's power limit: on zeros it reaches 1.71 PFLOP/s) and reads a third less from LDS.  16x16x32
-// instructions in the same schedule: 1.26.  Measured, before / now: 8192^3 1.16 / 1.32 PFLOP/s, 4096^3 1.14 / 1.22,
-// 2048 x 37888 x 3584 1.10 / 1.2.
+// instructions in the same schedule: 1.26.  Eight waves / this one, in turn on one machine: 8192^3 966 / 844 us (1.14 / 1.30
+// PFLOP/s), 4096^3 124 / 115, 2048 x 37888 x 3584 525 / 485 (1.06 / 1.15), 2048 x 18944 x 3584 285 / 267, 2048 x 3584 x 18944
+// 275 / 254; 8192^3 takes 820 to 880 us from machine to machine.  (With five slots for either operand's slabs in turn instead of
+// three and two: 820.5 and 821, 111.9 and 111.4, 462.5 and 466.3, 257.5 and 258.4, 243.7 and 244.)
 //
 // LDS rows are 128 bytes; the 16-byte piece c of row r is stored at slot c ^ ((r >> 1) & 7).  A ds_read_b128
 // serves 16 lanes per clock from 64 banks (256 bytes); 16 consecutive rows of one piece then fall on 16
@@ -348,8 +350,8 @@ __global__ __launch_bounds__(256) void gemm256_reduce_kernel(const float* __rest
 // the last, partial round split over kt workgroups each (kt = 1: no split) while a part keeps at least 16 slabs.
 struct Gemm256Plan { int mt, main_tiles, tail_tiles, kt; };
 
-// Tiles of 256 rows read least per product and are the ones for products of many rounds (8192^3: 826 us, 938 with 192 rows,
-// 1010 with 128); where few tiles leave CUs idle, or most of a tile's rows are past the end, smaller ones win.  The plan with the
+// Tiles of 256 rows read least per product and are the ones for products of many rounds (8192^3: 880 us, 963 with 192 rows,
+// 1019 with 128); where few tiles leave CUs idle, or most of a tile's rows are past the end, smaller ones win.  The plan with the
 // least estimated time is taken.  A slab takes G_SLAB + G_SLAB_BUSY * (share of the CUs at work) microseconds (the chip's power
 // and its L2 set the pace when it is full; fitted to 32 .. 512 tiles of each height at 3584 columns, where one round takes 42 ..
 // 63 / 55 .. 81 / 70 .. 104 us), a round 5 us at its ends, and a split adds the reduction's launch and the partial tiles written

@@ -7,10 +7,13 @@
 // codewords (LDS) or one d = 8 codeword (L2), so a lane gathers its operand straight into registers and uses it for all NT
 // tiles of 16 activation rows; the activations are the B operand and come from LDS.
 //
-// Bound: d = 8 by the gathers up to about 128 rows (16 bytes used of the 64 that L2 sends: 18944 x 2 x 3584 take 100 us at 33 rows
-// and 112 at 128), else by LDS: every wave reads all the activations for its 16 or 32 weight rows (12-bit, 18944 x 2 x 3584 at 128
-// rows: 54 us, 640 TFLOP/s).  Before, in passes of 32 rows or decoded first, at 33 / 77 / 128 / 256 rows: d = 8, 18944 x 2 x 3584:
-// 172 / 205 / 205 / 209 us, now 100 / 107 / 112 / 188; 12-bit: 41 / 68 / 102 / 165, now 30 / 40 / 54 / 105.
+// Bound: d = 8 by the gathers up to about 128 rows (one L2 request each, 16 bytes used of the 64 that come: 17 M of 18.5 M requests,
+// 153 G a second, for 18944 x 2 x 3584 at 64 rows, which take 107 us; the matrix cores are busy 15 % of the time).  d = 4 by no pipe
+// alone: with 12-bit tags at 128 rows the matrix cores are busy 47 % of a CU's time and LDS 51 % (every wave reads all the
+// activations for its 32 weight rows; 29 % of it bank conflicts of the codeword reads), taking turns, and the 148 workgroups of
+// 18944 x 2 rows leave 108 CUs without work (58 us, 590 TFLOP/s).  Before, in passes of 32 rows or decoded first, at 33 / 77 / 128 /
+// 256 rows: d = 8, 18944 x 2 x 3584: 172 / 205 / 205 / 209 us, now 100 / 107 / 112 / 188; 12-bit: 41 / 68 / 102 / 165, now 30 / 40 /
+// 54 / 105.
 //
 //   workgroup   8 waves, two per SIMD so that one gathers while the other multiplies (4 waves: a third slower); each has TW tiles
 //               of 16 weight rows x all NT x 16 activation rows (accumulators TW x NT x 4 registers)
