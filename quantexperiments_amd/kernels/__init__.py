@@ -77,10 +77,13 @@ def _check_row_ids(ids: torch.Tensor, R: int, n: int, what: str) -> None:
     0 .. n - 1.  The kernels index memory with them and do not look again."""
     if ids.numel() < R:
         raise ValueError(f"{what} has {ids.numel()} entries for {R} rows")
-    if R:
-        lo, hi = torch.stack(ids.reshape(-1)[:R].to(torch.int64).aminmax()).tolist()
-        if lo < 0 or hi >= n:
-            raise ValueError(f"{what} names {lo if lo < 0 else hi} of {n}")
+    if R == 0 or (ids.dtype == torch.uint8 and n >= 256):
+        return
+    ids = ids.reshape(-1)[:R]
+    # (one reduction and one number back for the file's uint8 tensors: 19 us of a load, 32 the general way)
+    lo, hi = (0, int(ids.max())) if ids.dtype == torch.uint8 else torch.stack(ids.to(torch.int64).aminmax()).tolist()
+    if lo < 0 or hi >= n:
+        raise ValueError(f"{what} names {lo if lo < 0 else hi} of {n}")
 
 
 class PackedLinear(torch.nn.Module):
