@@ -142,6 +142,8 @@ class PackedShards:
         self.Rs = [rl.R for rl in rls]
         self.R = sum(self.Rs)
         self.offs = [sum(self.Rs[:i]) for i in range(len(rls))]
+        # (first piece, end, rows) of the products of the "dequant" route, for few and for many activation rows
+        self.joint = [[(i, j, sum(self.Rs[i:j])) for i, j in joint_pieces(self.Rs, self.C, M)] for M in (1, JOINT_ROWS + 1)]
         self.large, self.chunk_bytes, self.dequant_from = large, chunk_bytes, dequant_from
         self.layout, self.compact = layout, compact
         self.bmax = bmax
@@ -252,16 +254,13 @@ class PackedShards:
             x = x.to(torch.float16)                     # fp16 x fp16 takes the 256 x 256 tile kernel; y keeps its dtype
         if self.large == "dequant":
             # one product over pieces that fit together: a 1024-row k or v projection alone is a few tiles on an idle chip
-            groups = joint_pieces(self.Rs, self.C, M)
-            n = max(sum(self.Rs[i:j]) for i, j in groups) * self.C
-            scratch = _Workspace.get(n * 2, x.device, kind="dense").view(torch.float16)
-            for i, j in groups:
-                at = self.offs[i]
-                R = sum(self.Rs[i:j])
-                w = scratch[:R * self.C].view(R, self.C)
+            groups = self.joint[M > JOINT_ROWS]
+            scratch = _Workspace.get(max(R for _, _, R in groups) * self.C * 2, x.device, kind="dense").view(torch.float16)
+            for i, j, R in groups:
+                at, w = self.offs[i], scratch[:R * self.C].view(R, self.C)
                 for rl, off in zip(self.rls[i:j], self.offs[i:j]):
                     rl.dense(torch.float16, out=w[off - at:off - at + rl.R])
-                gemm_dense(w, x, y[:, at:at + R])
+                gemm_dense(w, x, y if R == self.R else y[:, at:at + R])
             return y
         rows = max(self.Rs)
         if self.large == "chunked":
