@@ -218,7 +218,7 @@ static int decoded_step_rows(const sq_matrix* mats, int n) {
     int64_t rows = 0;
     for (int i = 0; i < n; ++i) rows += mats[i].R;
     const int64_t bytes = rows * mats[0].C * 2, steps = std::max<int64_t>(1, (bytes + DECODED_BYTES - 1) / DECODED_BYTES);
-    return (int)((rows + steps * 128 - 1) / (steps * 128) * 128);
+    return (int)std::max<int64_t>(128, (rows + steps * 128 - 1) / (steps * 128) * 128);     // (also where all pieces are empty)
 }
 
 // The step that begins at row r0 of piece i, each of its parts as a piece of its own to the kernel (which reads the scales and

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 import torch
 
+from quantexperiments_amd import _lib
 from quantexperiments_amd.kernels import linear_gemm
 from tests.helpers import rand_x, rel_max_err, synth, to_device
 
@@ -62,3 +63,20 @@ def test_decoded_weights_match_oracle(case, dtype):
     y = torch.empty(T, sum(rows), dtype=torch.float32, device="cuda")
     linear_gemm(lins, xd, y)
     assert rel_max_err(y.cpu().numpy(), ref.cpu().numpy()) < 1e-3
+
+
+def test_empty_pieces_of_a_decoded_stack():
+    L, C, T = _lib.lib(), 72, 40
+    lin = to_device(synth(30, C, 8, 16, seed=1))
+    x = rand_x(T, C, torch.float16, seed=2).cuda()
+    ref = x.double() @ torch.from_numpy(synth(30, C, 8, 16, seed=1).decode()).cuda().double().T
+    for rows in ((0,), (0, 30, 0), (0, 0)):
+        mats = []
+        for R in rows:
+            mats.append(lin.descriptor(0))
+            mats[-1].R = R
+        y = torch.zeros(T, 30, device="cuda")
+        ws = torch.zeros(max(L.sq_workspace_bytes(_lib.matrix_array(mats), len(mats), T, 1), 256), dtype=torch.uint8, device="cuda")
+        _lib.check(L.sq_linear_gemm(_lib.matrix_array(mats), len(mats), x.data_ptr(), _lib.SQ_F16, C, y.data_ptr(), _lib.SQ_F32, 30, T, ws.data_ptr(),
+                                    ws.numel(), _lib.stream_ptr(x.device)))
+        assert rel_max_err(y.cpu().numpy(), ref.cpu().numpy()) < 1e-3 if 30 in rows else not y.any()
