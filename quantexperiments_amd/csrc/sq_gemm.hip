@@ -269,6 +269,8 @@ static size_t decoded_workspace(const sq_matrix* mats, int n, int T) {
 
 static int launch_decoded(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws,
                           hipStream_t s) {
+    int rows = T;                                                // activation rows at a time: all, unless they span 4 GB
+    while (rows > 1 && !mid_x_ok(ldx, rows)) rows = (rows + 1) / 2;
     for (int i = 0, r0 = 0; i < n;) {
         const DecodedRows d = decoded_step(mats, n, i, r0);
         const void* w[MID_PIECES];
@@ -278,8 +280,10 @@ static int launch_decoded(const sq_matrix* mats, int n, const void* x, int x_dty
             if (const int rc = launch_dequant(*d.of[j], next, SQ_F16, mats[0].C, d.r0[j], d.r0[j] + d.m[j].R, s, /*raw=*/true)) return rc;
             next += dense_bytes(d.m[j]);
         }
-        if (d.n)
-            if (const int rc = launch_mid_decoded(d.m, d.n, w, x, x_dtype, ldx, y, y_dtype, ldy, T, next, s)) return rc;
+        for (int t = 0; d.n && t < T; t += rows)
+            if (const int rc = launch_mid_decoded(d.m, d.n, w, (const char*)x + (size_t)t * ldx * 2, x_dtype, rows > 1 ? ldx : mats[0].C,
+                                                  (char*)y + (size_t)t * ldy * (y_dtype == SQ_F32 ? 4 : 2), y_dtype, ldy, std::min(rows, T - t), next, s))
+                return rc;
     }
     return SQ_OK;
 }
@@ -317,7 +321,9 @@ size_t gemm_workspace(const sq_matrix* mats, int n, int T) {
 }
 
 static size_t gemm_workspace_beyond_small(const sq_matrix* mats, int n, int T) {
-    // (covers the other routes too: the size is asked for without knowing x)
+    // (covers the other routes too: the size is asked for without knowing x; up to SQ_SMALL_BMAX rows the only one is the
+    // decode-time kernel, which the caller adds)
+    if (T <= SQ_SMALL_BMAX && decoded_route(mats, n, T)) return decoded_workspace(mats, n, T);
     const size_t rest = gemm_workspace_without_mid(mats, n, T);
     if (mid_ok(mats, n, T)) return std::max(rest, mid_workspace(mats, n, T));
     return decoded_route(mats, n, T) ? std::max(rest, decoded_workspace(mats, n, T)) : rest;
@@ -410,7 +416,7 @@ int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_
         }
         return SQ_OK;
     }
-    if (decoded_route(mats, n, T) && mid_x_ok(ldx, T) && decoded_workspace(mats, n, T) <= ws_bytes)
+    if (decoded_route(mats, n, T) && decoded_workspace(mats, n, T) <= ws_bytes)
         return launch_decoded(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);
     if (gemm_workspace_without_mid(mats, n, T) > ws_bytes)
         return fail(SQ_EWORKSPACE, "sq_linear_gemm: workspace %zu < %zu", ws_bytes, gemm_workspace(mats, n, T));

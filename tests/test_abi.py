@@ -173,6 +173,10 @@ def test_workspace_of_decoded_weights_is_bounded():
                 for C in (3592, 5128):
                     dense = sum(rows) * C * 2
                     assert min(dense, step // 2) <= need(rows, C, d, bits, 1, T) <= min(dense + 4096, step) + 8 * T * 128 * 256 * 4
+    for rows in ((30000,), (20000, 10000), (1000,) * 8):
+        for C in (5120, 5128):
+            for T in (5, 16, 32):
+                assert need(rows, C, 8, 16, 16, T, 0) <= min(sum(rows) * C * 2 + 4096, step) + 8 * T * 128 * 256 * 4 + 16 * T * C * 2
     for rows in ((0,), (0, 0, 0), (0, 5, 0), (5, 0)):                                 # empty pieces end the walk over the steps like others
         assert need(rows, 72, 8, 16, 1, 40) + _lib.WS_HEADER < _lib.WS_HEADER + (1 << 20)
     assert need((24, 7), 3592, 8, 16, 16, 20, 0) >= 31 * 3592 * 2                     # decode sizes with column orders go the same way

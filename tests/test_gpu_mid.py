@@ -80,3 +80,16 @@ def test_empty_pieces_of_a_decoded_stack():
         _lib.check(L.sq_linear_gemm(_lib.matrix_array(mats), len(mats), x.data_ptr(), _lib.SQ_F16, C, y.data_ptr(), _lib.SQ_F32, 30, T, ws.data_ptr(),
                                     ws.numel(), _lib.stream_ptr(x.device)))
         assert rel_max_err(y.cpu().numpy(), ref.cpu().numpy()) < 1e-3 if 30 in rows else not y.any()
+
+
+@pytest.mark.parametrize("T,ld", [(40, 1 << 26), (5, 1 << 29)])
+def test_decoded_weights_with_activation_rows_that_span_4_gb(T, ld):
+    s = synth(70, 520, 8, 16, 1, 3, seed=T)
+    lin = to_device(s, stream=False)
+    x = rand_x(T, 520, torch.bfloat16, seed=T)
+    big = torch.empty((T - 1) * ld + 520, dtype=torch.bfloat16, device="cuda")
+    xd = big.as_strided((T, 520), (ld, 1))
+    xd.copy_(x)
+    y = torch.empty(T, 70, dtype=torch.float32, device="cuda")
+    linear_gemm([lin], xd, y)
+    assert rel_max_err(y.cpu().numpy(), x.double().numpy() @ s.decode().astype(np.float64).T) < 1e-3
