@@ -243,7 +243,12 @@ int sq_codebook_balance_books(const int32_t* tags_host, int32_t R, int32_t W, in
  *   sq_stream_fill_device   writes the buffer (16-byte aligned, of that size) from the same tags.
  *   sq_stream_plan_free     ends the plan.
  *   sq_codebook_balance_device  sq_codebook_balance_books; counts: (G << bits) * 4 bytes.
- *   sq_codebook_relabel_device  rewrites the tags through remap (G << bits entries) in place. */
+ *   sq_codebook_relabel_device  rewrites the tags through remap (G << bits entries) in place.
+ *   sq_codebook_rebalance_device  both, and the tables' rows moved to their new labels, for n matrices whose shapes and device
+ *                           pointers (tags, table, row_book) mats holds: tags_out[i] and table_out[i] (host arrays of device
+ *                           pointers) are buffers of the size of matrix i's tags and table, scratch one of
+ *                           sq_codebook_rebalance_bytes (0 for arguments the call refuses).  The labels are those of
+ *                           sq_codebook_balance_books.  Launches kernels only; with G > 1 it synchronises first, to check row_book. */
 size_t sq_stream_counts_bytes(int32_t R, int32_t C, int32_t d, int32_t bits, int32_t G);
 int sq_stream_plan_device(const int32_t* tags, int32_t R, int32_t W, int32_t C, int32_t d, int32_t bits, int32_t G, const uint8_t* row_book,
                           const uint8_t* row_mask_host, int32_t runs, void* counts, void** plan_out, size_t* bytes_out, size_t* scratch_out,
@@ -254,6 +259,9 @@ int sq_codebook_balance_device(const int32_t* tags, int32_t R, int32_t W, int32_
                                uint32_t* counts, uint16_t* remap_out_host, void* stream);
 int sq_codebook_relabel_device(int32_t* tags, int32_t R, int32_t W, int32_t C, int32_t d, int32_t bits, int32_t G, const uint8_t* row_book,
                                const uint16_t* remap, void* stream);
+size_t sq_codebook_rebalance_bytes(const sq_matrix* mats, int32_t n);
+int sq_codebook_rebalance_device(const sq_matrix* mats, int32_t n, void* const* tags_out, void* const* table_out, void* scratch, size_t scratch_bytes,
+                                 void* stream);
 
 /* ---- The packed file's block-32 side formats (reference shapequant/packed.py:30-40): the 8-bit output head
  * `aux.lm_head` (q int8 [V, C], scale fp16 [V, C/32], w = q * scale of the row's 32-column block) and the 4-bit

@@ -109,6 +109,10 @@ def lib() -> ctypes.CDLL:
         L.sq_codebook_balance_device.restype = ctypes.c_int
         L.sq_codebook_relabel_device.argtypes = [vp, i32, i32, i32, i32, i32, i32, vp, vp, vp]
         L.sq_codebook_relabel_device.restype = ctypes.c_int
+        L.sq_codebook_rebalance_bytes.argtypes = [mp, i32]
+        L.sq_codebook_rebalance_bytes.restype = sz
+        L.sq_codebook_rebalance_device.argtypes = [mp, i32, pp, pp, vp, sz, vp]
+        L.sq_codebook_rebalance_device.restype = ctypes.c_int
         L.sq_q8_linear.argtypes = [vp, vp, i32, i32, vp, ctypes.c_int, i64, vp, ctypes.c_int, i64, i32, vp, sz, vp]
         L.sq_q8_workspace_bytes.argtypes = [i32, i32, i32]
         L.sq_q8_workspace_bytes.restype = sz
@@ -133,7 +137,8 @@ EXPORTS = ("sq_version", "sq_last_error", "sq_dequant", "sq_linear_small", "sq_l
            "sq_linear_small_from", "sq_linear_small_silu", "sq_gemm_dense_ws", "sq_gemm_dense_workspace_bytes", "sq_linear_small_noalloc",
            "sq_workspace_status", "sq_workspace_reset", "sq_noalloc_reset", "sq_stream_spin_limit", "sq_codebook_balance",
            "sq_stream_bytes_books", "sq_stream_build_books", "sq_codebook_balance_books", "sq_stream_counts_bytes", "sq_stream_plan_device",
-           "sq_stream_fill_device", "sq_stream_plan_free", "sq_codebook_balance_device", "sq_codebook_relabel_device")
+           "sq_stream_fill_device", "sq_stream_plan_free", "sq_codebook_balance_device", "sq_codebook_relabel_device",
+           "sq_codebook_rebalance_bytes", "sq_codebook_rebalance_device")
 
 
 _native = None

@@ -475,6 +475,35 @@ int sq_codebook_relabel_device(int32_t* tags, int32_t R, int32_t W, int32_t C, i
     return stream_relabel_device((uint32_t*)tags, R, W, C, d, bits, G, G > 1 ? row_book : nullptr, remap, (hipStream_t)stream);
 }
 
+static int rebalance_check(const sq_matrix* mats, int32_t n) {
+    const char* who = "sq_codebook_rebalance_device";
+    if (!mats || n < 1) return fail(SQ_EINVAL, "%s: no matrices", who);
+    for (int i = 0; i < n; ++i) {
+        const sq_matrix& m = mats[i];
+        if (int rc = device_build_check(who, m.tags, m.R, m.W, m.C, m.d, m.bits, m.G, m.row_book)) return rc;
+        if (!m.table || ((uintptr_t)m.table & 15)) return fail(SQ_EINVAL, "%s: table must be 16-byte aligned", who);
+    }
+    return SQ_OK;
+}
+
+size_t sq_codebook_rebalance_bytes(const sq_matrix* mats, int32_t n) {
+    return rebalance_check(mats, n) == SQ_OK ? relabel_scratch_bytes(mats, n) : 0;
+}
+
+int sq_codebook_rebalance_device(const sq_matrix* mats, int32_t n, void* const* tags_out, void* const* table_out, void* scratch, size_t scratch_bytes,
+                                 void* stream) {
+    const char* who = "sq_codebook_rebalance_device";
+    if (int rc = rebalance_check(mats, n)) return rc;
+    if (!tags_out || !table_out || !scratch || ((uintptr_t)scratch & 15)) return fail(SQ_EINVAL, "%s: null or unaligned pointer", who);
+    if (scratch_bytes < relabel_scratch_bytes(mats, n)) return fail(SQ_EWORKSPACE, "%s: scratch %zu < %zu", who, scratch_bytes, relabel_scratch_bytes(mats, n));
+    for (int i = 0; i < n; ++i) {
+        if (!tags_out[i] || !table_out[i] || ((uintptr_t)table_out[i] & 15) || tags_out[i] == mats[i].tags || table_out[i] == (const void*)mats[i].table)
+            return fail(SQ_EINVAL, "%s: tags_out and table_out are buffers of their own, table_out 16-byte aligned", who);
+        if (int rc = device_books_check(who, mats[i].R, mats[i].G, mats[i].row_book, (hipStream_t)stream)) return rc;
+    }
+    return launch_relabel(mats, n, tags_out, table_out, scratch, (hipStream_t)stream);
+}
+
 size_t sq_stream_bytes(const int32_t* tags_host, int32_t R, int32_t W, int32_t C, int32_t d, int32_t bits,
                        const uint8_t* row_mask_host, int32_t runs) {
     return sq_stream_bytes_balanced(tags_host, R, W, C, d, bits, row_mask_host, runs, nullptr);

@@ -95,6 +95,10 @@ int stream_fill_device(const StreamDevicePlan& D, const uint32_t* tags, const ui
 void stream_plan_free(StreamDevicePlan* D);
 int stream_balance_device(const uint32_t* tags, int R, int W, int C, int d, int bits, uint32_t* counts, uint16_t* remap_out, int G,
                           const uint8_t* row_book, hipStream_t s);
+// both in one, for up to RELABEL_PIECES matrices per launch, on the device from end to end (sq_relabel.hip)
+constexpr int RELABEL_PIECES = 8;
+size_t relabel_scratch_bytes(const sq_matrix* mats, int n);
+int launch_relabel(const sq_matrix* mats, int n, void* const* tags_out, void* const* table_out, void* scratch, hipStream_t s);
 int stream_relabel_device(uint32_t* tags, int R, int W, int C, int d, int bits, int G, const uint8_t* row_book, const uint16_t* remap, hipStream_t s);
 // sq_matrix.stream_runs is sq_stream_build's runs_out: the run count in the low 16 bits, the groups of the longest run
 // in the next 8, the most column orders in one run (less one) in bits 24-26, the steps per unit of the first-steps region

@@ -182,42 +182,13 @@ class PackedLinear(torch.nn.Module):
         if self.words is None:
             raise RuntimeError("the packed tags of this matrix were dropped (compact): its stream cannot be rebuilt")
         if self.wants_stream and self.balance and not self.relabelled:
-            self._relabel()
+            _relabel([self])
         self.stream, self.stream_runs, self.stream_groups = build_stream(
             self.words, self.C, self.d, self.bits, self.row_mask if self.has_mask else None, runs,
             row_book=None if self.row_book is None else (self.row_book, self.G))
         self.stream_asked = runs
         if self.stream is None:
             self.wants_stream = False
-
-    def _relabel(self) -> None:
-        """Give the codewords new labels so that every slice of 4096 carries the same share of this matrix' tags
-        (sq_codebook_balance: most used codewords first, each to the slice with the fewest tags so far), and keep the
-        relabelled pair: the tags are rewritten through the map and row k of the table moves to row map[k].  Every
-        weight decodes to the same bits as before, the tag-stream kernel's workgroups (one per slice) get equal work
-        whatever the distribution of the tags, and the matrix keeps ONE codebook (a stream that carries its own
-        relabelled copy, sq_stream_build_balanced, costs another 1.1 MiB per matrix).  With several codebooks each is
-        relabelled by itself, over its own slices (sq_codebook_balance_books)."""
-        dev, L = self.words.device, _lib.lib()
-        remap = torch.empty(self.G << self.bits, dtype=torch.int16)
-        counts = torch.empty(self.G << self.bits, dtype=torch.int32, device=dev)
-        args = (self.R, self.W, self.C, self.d, self.bits, self.G, None if self.row_book is None else self.row_book.data_ptr())
-        with torch.cuda.device(dev):
-            rc = L.sq_codebook_balance_device(self.words.data_ptr(), *args, counts.data_ptr(), remap.data_ptr(), _lib.stream_ptr(dev))
-            if rc == _lib.SQ_EUNSUPPORTED:              # a shape the slice stream does not cover: nothing to balance
-                self.relabelled = True
-                return
-            _lib.check(rc)
-            remap = remap.to(dev)
-            self.words = self.words.clone()             # (the caller's tensor keeps the file's labels)
-            _lib.check(L.sq_codebook_relabel_device(self.words.data_ptr(), *args, remap.data_ptr(), _lib.stream_ptr(dev)))
-        # row of the table a codeword moves to: book << bits | new label
-        at = torch.arange(self.G << self.bits, device=dev)
-        at = (at & -(1 << self.bits)) + (remap.to(torch.int64) & 0xFFFF)
-        table = torch.empty_like(self.table)
-        table[at] = self.table
-        self.table = table
-        self.relabelled = True
 
     # ------------------------------------------------------------------ construction
     @classmethod
@@ -296,6 +267,34 @@ class PackedLinear(torch.nn.Module):
             self.stream, self.stream_tiled = None, False
         else:
             self.words = None
+
+
+def _relabel(ms) -> None:
+    """Give the codewords of each of these matrices new labels so that every slice of 4096 carries the same share of its tags
+    (most used codewords first, each to the slice with the fewest tags so far), and keep the relabelled pair: the tags are
+    rewritten and the table's rows moved (sq_codebook_rebalance_device; the caller's tensors keep the file's labels).  Every
+    weight decodes to the same bits as before, the tag-stream kernel's workgroups (one per slice) get equal work whatever the
+    distribution of the tags, and the matrix keeps ONE codebook (a stream that carries its own relabelled copy,
+    sq_stream_build_balanced, costs another 1.1 MiB per matrix).  With several codebooks each is relabelled by itself, over its
+    own slices."""
+    L = _lib.lib()
+    for m in ms:
+        m.relabelled = True
+        if m.table.data_ptr() % 16:
+            m.table = m.table.clone()
+    # (shapes the slice stream does not cover are refused: nothing to balance)
+    todo = [(m, a) for m in ms for a in [_lib.matrix_array([m.descriptor()])] if L.sq_codebook_rebalance_bytes(a, 1)]
+    if not todo:
+        return
+    dev = todo[0][0].device
+    mats = _lib.matrix_array([a[0] for _, a in todo])
+    out = [(torch.empty_like(m.words), torch.empty_like(m.table)) for m, _ in todo]
+    ptrs = [(ctypes.c_void_p * len(out))(*(o[k].data_ptr() for o in out)) for k in (0, 1)]
+    scratch = torch.empty(L.sq_codebook_rebalance_bytes(mats, len(todo)), dtype=torch.uint8, device=dev)
+    with torch.cuda.device(dev):
+        _lib.check(L.sq_codebook_rebalance_device(mats, len(todo), *ptrs, scratch.data_ptr(), scratch.numel(), _lib.stream_ptr(dev)))
+    for (m, _), (words, table) in zip(todo, out):
+        m.words, m.table = words, table
 
 
 def build_stream(words: torch.Tensor, C: int, d: int, bits: int, row_mask=None, runs: int = 0, table=None, row_book=None):
@@ -393,6 +392,7 @@ def prepare_stack(pieces, workgroups: int | None = None) -> None:
     # Smallest piece first: a piece with column orders can need more runs than its share (a run holds the whole
     # groups of a few orders), and what it takes beyond its share comes off the larger pieces' runs, so the launch
     # still fits the device in one round of workgroups.
+    _relabel([p for p in ps if p.stream is None and p.words is not None and p.balance and not p.relabelled])
     rows = sum(p.R for p in ps)
     for p in sorted(ps, key=lambda q: q.R):
         buckets = ((p.G << p.bits) >> 12) * -(-(p.C // p.d) // STREAM_PART_MAX)

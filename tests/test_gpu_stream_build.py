@@ -1,6 +1,7 @@
 """The load-time layouts built on the GPU are the host builder's, byte for byte, and so is the relabelling."""
 
 import ctypes
+import math
 
 import numpy as np
 import pytest
@@ -57,6 +58,53 @@ def test_device_relabelling(R, C, bits, G):
     m = ctypes.c_void_p()
     assert L.sq_stream_plan_device(None, R, 1, C, 8, bits, G, None, None, 0, None, ctypes.byref(m), ctypes.byref(ctypes.c_size_t()),
                                    ctypes.byref(ctypes.c_size_t()), ctypes.byref(ctypes.c_int32()), ctypes.byref(ctypes.c_int32()), None) == _lib.SQ_EINVAL
+
+
+def _counted(R, n, bits, how, g):
+    """Tags [R, n] whose codewords are used: evenly; by a power law (counts of two and three bytes); only the first few (the rest
+    not at all); each a different number of times (more of those than one list of runs holds)."""
+    K = 1 << bits
+    if how == "any":
+        return torch.randint(0, K, (R, n), generator=g)
+    if how == "zipf":
+        return (torch.rand(R, n, generator=g, dtype=torch.float64).mul_(-math.log(K)).exp_() * K).long().clamp_(max=K - 1)
+    if how == "few":
+        return torch.randint(0, 5, (R, n), generator=g) * 3
+    t = torch.repeat_interleave(torch.arange(6300), torch.arange(6300))
+    t = torch.cat([t, torch.full((R * n - t.numel(),), K - 1)])
+    return t[torch.randperm(t.numel(), generator=g)].view(R, n)
+
+
+@pytest.mark.parametrize("R,C,bits,G,W,how", [(1, 8, 13, 1, 1, "any"), (70, 1000, 13, 1, 53, "zipf"), (65, 3584, 16, 1, 224, "any"), (600, 3584, 16, 1, 224, "zipf"),
+                                              (90, 1032, 14, 4, 57, "zipf"), (33, 264, 12, 2, 13, "any"), (300, 512, 15, 2, 30, "few"),
+                                              (4900, 32400, 16, 1, 2025, "each")])
+def test_device_rebalance(R, C, bits, G, W, how):
+    L, g, n = _lib.lib(), torch.Generator().manual_seed(bits + R), C // 8
+    tags = _counted(R, n, bits, how, g)
+    words = torch.full((R, W), -1, dtype=torch.int32)
+    need = (n * bits + 31) // 32
+    words[:, :need] = pack_bits(tags, bits)                     # (W > need: words behind the tags, which stay)
+    book = torch.randint(0, G, (R,), generator=g).to(torch.uint8)
+    table = torch.randn(G << bits, 8, generator=g).half()
+    remap = np.zeros(G << bits, np.uint16)
+    _lib.check(L.sq_codebook_balance_books(words.data_ptr(), R, W, C, 8, bits, G, book.data_ptr() if G > 1 else None, remap.ctypes.data))
+    new = torch.from_numpy(remap.astype(np.int64))
+    at = tags + (book.long() << bits)[:, None] if G > 1 else tags
+    want = words.clone()
+    want[:, :need] = pack_bits(new[at], bits)
+    moved = torch.empty_like(table)
+    moved[(torch.arange(G << bits) >> bits << bits) + new] = table
+    dev = [t.cuda() for t in (words, table, book)]
+    m = _lib.SqMatrix(dev[0].data_ptr(), dev[1].data_ptr(), None, dev[2].data_ptr() if G > 1 else None, None, None, None, R, C, 8, bits, G, 1, W, 0, None, 0, 0)
+    mats = _lib.matrix_array([m] * 9)                           # (more than a launch takes)
+    out = [(torch.empty_like(dev[0]), torch.empty_like(dev[1])) for _ in range(9)]
+    ptrs = [(ctypes.c_void_p * 9)(*(o[k].data_ptr() for o in out)) for k in (0, 1)]
+    scratch = torch.empty(L.sq_codebook_rebalance_bytes(mats, 9), dtype=torch.uint8, device="cuda")
+    args = (mats, 9, *ptrs, scratch.data_ptr())
+    assert L.sq_codebook_rebalance_device(*args, scratch.numel() - 1, None) == _lib.SQ_EWORKSPACE
+    _lib.check(L.sq_codebook_rebalance_device(*args, scratch.numel(), _lib.stream_ptr(dev[0].device)))
+    for w, t in out:
+        assert torch.equal(w.cpu(), want) and torch.equal(t.cpu(), moved)
 
 
 @pytest.mark.parametrize("G", [2, 4])
