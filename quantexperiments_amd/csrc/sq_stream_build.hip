@@ -257,33 +257,14 @@ static void plan_counts(const uint32_t* tags, int R, int W, int bits, const uint
     });
 }
 
-static void plan_places(int R, StreamPlan& P) {
+// From the groups' step counts ([NV * NG]): their offsets, units and places.
+static void plan_layout(const uint32_t* steps, StreamPlan& P) {
     const StreamGeom& g = P.g;
-    P.pos.assign((size_t)g.NV * R, 0);
-    P.goff.assign((size_t)g.NV * g.NG + 1, 0);
-    std::vector<uint32_t> steps((size_t)g.NV * g.NG, 0);
-    parallel_blocks(g.NV, 1, [&](int a, int b) {
-        std::vector<uint32_t> rows;
-        for (int v = a; v < b; ++v) {
-            const uint16_t* c = &P.cnt[(size_t)v * R];
-            for (const StreamRun& run : P.runs) {
-                // rows move between the groups of one column order only: a group reads one copy of x
-                for (int oi = 0; oi < run.norders; ++oi) {
-                    const int ga = run.g0 + run.bound[oi], gb = run.g0 + (oi + 1 < run.norders ? run.bound[oi + 1] : run.ng);
-                    rows.clear();
-                    for (int k = ga * 64; k < gb * 64; ++k)
-                        if (P.base[k] != STREAM_NO_ROW) rows.push_back(P.base[k]);
-                    std::stable_sort(rows.begin(), rows.end(), [c](uint32_t x, uint32_t y) { return c[x] > c[y]; });
-                    for (size_t k = 0; k < rows.size(); ++k) P.pos[(size_t)v * R + rows[k]] = (uint32_t)(ga * 64 + k);
-                    for (size_t k = 0; k < rows.size(); k += 64)
-                        steps[(size_t)v * g.NG + ga + k / 64] = (c[rows[k]] + (uint32_t)g.fmt.eps - 1u) / (uint32_t)g.fmt.eps;
-                }
-            }
-        }
-    });
+    const size_t nvg = (size_t)g.NV * g.NG;
+    P.goff.assign(nvg + 1, 0);
     uint64_t tot = 0;
-    for (size_t k = 0; k < steps.size(); ++k) { P.goff[k] = (uint32_t)tot; tot += steps[k]; }
-    P.goff[steps.size()] = (uint32_t)tot;
+    for (size_t k = 0; k < nvg; ++k) { P.goff[k] = (uint32_t)tot; tot += steps[k]; }
+    P.goff[nvg] = (uint32_t)tot;
     P.logical_steps = tot;
     // Units and places: the first-steps region (NU units x NV buckets x FS steps) comes first, the groups'
     // remaining steps follow bucket after bucket, group after group.
@@ -318,6 +299,32 @@ static void plan_places(int R, StreamPlan& P) {
             if (nst / split >= PF) at += nst - split * PF;
         }
     P.g.total_steps = at;
+}
+
+static void plan_places(int R, StreamPlan& P) {
+    const StreamGeom& g = P.g;
+    P.pos.assign((size_t)g.NV * R, 0);
+    std::vector<uint32_t> steps((size_t)g.NV * g.NG, 0);
+    parallel_blocks(g.NV, 1, [&](int a, int b) {
+        std::vector<uint32_t> rows;
+        for (int v = a; v < b; ++v) {
+            const uint16_t* c = &P.cnt[(size_t)v * R];
+            for (const StreamRun& run : P.runs) {
+                // rows move between the groups of one column order only: a group reads one copy of x
+                for (int oi = 0; oi < run.norders; ++oi) {
+                    const int ga = run.g0 + run.bound[oi], gb = run.g0 + (oi + 1 < run.norders ? run.bound[oi + 1] : run.ng);
+                    rows.clear();
+                    for (int k = ga * 64; k < gb * 64; ++k)
+                        if (P.base[k] != STREAM_NO_ROW) rows.push_back(P.base[k]);
+                    std::stable_sort(rows.begin(), rows.end(), [c](uint32_t x, uint32_t y) { return c[x] > c[y]; });
+                    for (size_t k = 0; k < rows.size(); ++k) P.pos[(size_t)v * R + rows[k]] = (uint32_t)(ga * 64 + k);
+                    for (size_t k = 0; k < rows.size(); k += 64)
+                        steps[(size_t)v * g.NG + ga + k / 64] = (c[rows[k]] + (uint32_t)g.fmt.eps - 1u) / (uint32_t)g.fmt.eps;
+                }
+            }
+        }
+    });
+    plan_layout(steps.data(), P);
 }
 
 static int runs_word(const StreamPlan& P) { return P.g.runs | (P.GR << 16) | ((P.orders_max - 1) << 24) | ((P.g.fs - 1) << 27); }
@@ -649,8 +656,8 @@ int stream_build_host(const uint32_t* tags, int R, int W, int C, int d, int bits
 // ------------------------------------------------------------------------------------------ on the GPU
 //
 // The same buffer, byte for byte, from tags that are already in device memory.  What is serial and small stays on the host
-// (the rows' order and runs, the sort of the rows of a run by entry count, the places); what walks the tags runs here:
-// counting, collecting every lane's entries, ordering them for the LDS banks, encoding.  The ordering is what the host
+// (the rows' order and runs, the groups' places from their step counts); what walks tags or rows runs here: counting, the sort of
+// the rows of a run by entry count, collecting every lane's entries, ordering them for the LDS banks, encoding.  The ordering is what the host
 // spends its time on (16 cores: 150 ms for 18944 x 3584, 2.5 s for 3584 x 18944 on one).  Whole load of a matrix, tags on
 // the GPU to stream on the GPU, before / now: 3584 x 3584 363 / 2.7 ms, 18944 x 3584 155 / 6.0, 3584 x 18944 2525 / 12.9.
 
@@ -977,16 +984,103 @@ int stream_relabel_device(uint32_t* tags, int R, int W, int C, int d, int bits, 
     return check_launch("sq_codebook_relabel_device");
 }
 
+// One column order's rows of one run: groups ga .. ga + ng - 1, places from ga * 64; p0: the run's first place.
+struct StreamSegment { int32_t ga, ng, p0, pad; };
+
+struct StreamSortArgs {
+    const uint16_t* cnt;        // [NV][R]
+    const uint32_t* base;       // [NG * 64]: the row of every place
+    const StreamSegment* seg;
+    uint32_t* steps;            // [NV * NG], or NULL
+    uint32_t* rows;             // [NV * NG * 64]: the row of every lane, or NULL
+    uint16_t* slots;            // the buffer's slots, with rows
+    int R, NG, eps;
+};
+
+// The rows of a segment in one bucket by entry count, most first, equal counts in the order of their places: a bitonic sort of
+// (count, place) in LDS.  Runs of 256 rows (3584 rows in 14, 16 buckets) take 11 us; on the host, with the counts' way there and the
+// places' way back, it was 600 us of every matrix' load, however small.
+__global__ __launch_bounds__(1024) void stream_sort_kernel(StreamSortArgs a) {
+    extern __shared__ uint32_t stream_sort_lds[];
+    const StreamSegment sg = a.seg[blockIdx.x];
+    const int v = (int)blockIdx.y, n = sg.ng * 64, tid = (int)threadIdx.x, nt = (int)blockDim.x;
+    int size = 64;
+    while (size < n) size *= 2;
+    for (int i = tid; i < size; i += nt) {
+        const uint32_t row = i < n ? a.base[sg.ga * 64 + i] : STREAM_NO_ROW;
+        stream_sort_lds[i] = row == STREAM_NO_ROW ? 0xFFFFFFFFu : (8191u - a.cnt[(size_t)v * a.R + row]) << 13 | (uint32_t)i;
+    }
+    for (int k = 2; k <= size; k *= 2)
+        for (int j = k / 2; j > 0; j /= 2) {
+            __syncthreads();
+            for (int t = tid; t < size / 2; t += nt) {
+                const int i = (t & ~(j - 1)) * 2 | (t & (j - 1));
+                const uint32_t x = stream_sort_lds[i], y = stream_sort_lds[i + j];
+                if ((x > y) == ((i & k) == 0)) {
+                    stream_sort_lds[i] = y;
+                    stream_sort_lds[i + j] = x;
+                }
+            }
+        }
+    __syncthreads();
+    for (int i = tid; i < n; i += nt) {
+        const uint32_t key = stream_sort_lds[i], c = key == 0xFFFFFFFFu ? 0u : 8191u - (key >> 13);
+        const size_t at = ((size_t)v * a.NG + sg.ga) * 64 + i;
+        if (a.steps && i % 64 == 0) a.steps[at / 64] = (c + (uint32_t)a.eps - 1u) / (uint32_t)a.eps;
+        if (a.rows) {
+            const uint32_t place = (uint32_t)sg.ga * 64u + (key & 8191u);
+            a.rows[at] = key == 0xFFFFFFFFu ? STREAM_NO_ROW : a.base[place];
+            a.slots[at] = key == 0xFFFFFFFFu ? (uint16_t)STREAM_SLOT_NONE : (uint16_t)((place - (uint32_t)sg.p0) | (c ? STREAM_SLOT_HAS : 0u));
+        }
+    }
+}
+
+// The stream buffer in front of its steps from what the host has planned (heads, runs and rows lie in `plan` one behind the
+// other), and zeros everywhere else.
+__global__ __launch_bounds__(256) void stream_front_kernel(const uint32_t* __restrict__ plan, int64_t heads, int64_t runs0, int64_t runs, int64_t rows0,
+                                                           int64_t rows, uint32_t* __restrict__ out, int64_t words) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= words) return;
+    uint32_t v = 0u;
+    if (i < heads) v = plan[i];
+    else if (i >= runs0 && i < runs0 + runs) v = plan[heads + i - runs0];
+    else if (i >= rows0 && i < rows0 + rows) v = plan[heads + runs + i - rows0];
+    out[i] = v;
+}
+
+static size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
+
+static void launch_count_and_sort(const StreamPlan& P, const uint32_t* tags, int R, int W, int bits, int G, const uint8_t* row_book, uint16_t* cnt,
+                                  const StreamSortArgs& a, int segments, hipStream_t s) {
+    const StreamGeom& g = P.g;
+    int size = 64;
+    while (size < P.GR * 64) size *= 2;
+    hipLaunchKernelGGL(stream_count_kernel, dim3((unsigned)R), dim3(64), (size_t)g.NV * 4, s, tags, R, W, g.U, bits, G, g.PC, g.NS, g.NV, row_book, cnt);
+    hipLaunchKernelGGL(stream_sort_kernel, dim3((unsigned)segments, (unsigned)g.NV), dim3((unsigned)std::min(1024, std::max(64, size / 2))), (size_t)size * 4, s, a);
+}
+
+static std::vector<StreamSegment> plan_segments(const StreamPlan& P) {
+    std::vector<StreamSegment> seg;
+    for (const StreamRun& run : P.runs)
+        for (int i = 0; i < run.norders; ++i)
+            seg.push_back({run.g0 + run.bound[i], (i + 1 < run.norders ? run.bound[i + 1] : run.ng) - run.bound[i], run.g0 * 64, 0});
+    return seg;
+}
+
+// the counts, the groups' step counts, the segments and the places' rows; every column order can leave one group short
 size_t stream_counts_bytes(int R, int C, int d, int bits, int G) {
-    return (size_t)stream_geom(C, d, stream_label_bits(bits, G), 0, 0).NV * R * 2;
+    const size_t NV = (size_t)stream_geom(C, d, stream_label_bits(bits, G), 0, 0).NV, groups = (size_t)R / 64 + 256;
+    return align256(NV * R * 2) + align256(NV * groups * 4) + groups * sizeof(StreamSegment) + groups * 64 * 4;
 }
 
 // A plan on its way from stream_plan_device to stream_fill_device.
 struct StreamDevicePlan {
     StreamPlan P;
+    std::vector<StreamSegment> seg;
+    std::vector<uint32_t> upload;    // heads, runs, rows; then the groups' offsets and the segments
     int R, W, C, d, bits, G;
     bool tiled, in_lds;
-    size_t bytes, scratch;
+    size_t bytes, scratch, at_goff, at_seg, at_rows, at_cnt, at_work;   // places in the scratch
 };
 
 int stream_plan_device(const uint32_t* tags, int R, int W, int C, int d, int bits, int G, const uint8_t* row_book, const uint8_t* row_mask_host,
@@ -1003,24 +1097,48 @@ int stream_plan_device(const uint32_t* tags, int R, int W, int C, int d, int bit
         StreamPlan& P = D->P;
         plan_rows(R, C, d, stream_label_bits(bits, G), row_mask_host, runs, P, false);
         const StreamGeom& g = P.g;
-        hipLaunchKernelGGL(stream_count_kernel, dim3((unsigned)R), dim3(64), (size_t)g.NV * 4, s, tags, R, W, g.U, bits, G, g.PC, g.NS, g.NV, row_book,
-                           (uint16_t*)counts);
-        int rc = check_launch("sq_stream_plan_device");
-        if (rc) return rc;
-        P.cnt.resize((size_t)g.NV * R);
-        hipError_t e = hipMemcpyAsync(P.cnt.data(), counts, P.cnt.size() * 2, hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        const size_t nvg = (size_t)g.NV * g.NG;
+        D->seg = plan_segments(P);
+        char* at = (char*)counts;
+        StreamSortArgs a{};
+        a.cnt = (uint16_t*)at; at += align256((size_t)g.NV * R * 2);
+        a.steps = (uint32_t*)at; at += align256((size_t)g.NV * ((size_t)R / 64 + 256) * 4);
+        a.seg = (StreamSegment*)at;
+        a.base = (uint32_t*)(at + D->seg.size() * sizeof(StreamSegment));
+        a.R = R; a.NG = g.NG; a.eps = g.fmt.eps;
+        std::vector<uint32_t> up(D->seg.size() * (sizeof(StreamSegment) / 4) + P.base.size()), steps(nvg);
+        memcpy(up.data(), D->seg.data(), D->seg.size() * sizeof(StreamSegment));
+        memcpy(up.data() + up.size() - P.base.size(), P.base.data(), P.base.size() * 4);
+        hipError_t e = hipMemcpyAsync(at, up.data(), up.size() * 4, hipMemcpyHostToDevice, s);
         if (e != hipSuccess) return fail(SQ_ELAUNCH, "sq_stream_plan_device: %s", hipGetErrorString(e));
-        plan_places(R, P);
-        plan_slots(R, P);
+        launch_count_and_sort(P, tags, R, W, bits, G, row_book, (uint16_t*)counts, a, (int)D->seg.size(), s);
+        int rc = check_launch("sq_stream_plan_device");
+        e = hipMemcpyAsync(steps.data(), a.steps, nvg * 4, hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);        // (also where the launch failed: the copy out of `up` has ended)
+        if (rc) return rc;
+        if (e != hipSuccess) return fail(SQ_ELAUNCH, "sq_stream_plan_device: %s", hipGetErrorString(e));
+        plan_layout(steps.data(), P);
         if (g.total_steps >= ((uint64_t)1 << 32) || g.runs >= (1 << 16)) return fail(SQ_EUNSUPPORTED, "sq_stream_plan_device: matrix too large");
         D->bytes = g.off_steps + (size_t)g.total_steps * g.fmt.step_bytes;
-        uint32_t longest = 0;
-        for (size_t k = 0; k + 1 < P.goff.size(); ++k) longest = std::max(longest, P.goff[k + 1] - P.goff[k]);
+        const uint32_t longest = nvg ? *std::max_element(steps.begin(), steps.end()) : 0u;
         D->in_lds = (size_t)longest * g.fmt.eps * STREAM_FILL_BYTES <= STREAM_FILL_LDS;
-        // scratch: the rows of the lanes and the groups' offsets, and the groups themselves when one is too long for LDS
-        const size_t lists = (((size_t)g.NV * g.NG * 65 + 1) * 4 + 255) & ~(size_t)255;
-        D->scratch = lists + (D->in_lds ? 0 : (size_t)P.logical_steps * g.fmt.eps * STREAM_FILL_BYTES);
+        // what the host uploads in one piece
+        auto put = [&](const void* p, size_t n) {
+            const uint32_t* w = (const uint32_t*)p;
+            D->upload.insert(D->upload.end(), w, w + n / 4);
+        };
+        put(P.head4.data(), P.head4.size() * 4);
+        put(P.runs.data(), P.runs.size() * sizeof(StreamRun));
+        put(P.base.data(), P.base.size() * 4);
+        D->at_goff = D->upload.size() * 4;
+        put(P.goff.data(), P.goff.size() * 4);
+        D->at_seg = D->upload.size() * 4;
+        put(D->seg.data(), D->seg.size() * sizeof(StreamSegment));
+        // scratch: that, the rows of the lanes, the counts, and the groups themselves when one is too long for LDS
+        D->at_rows = align256(D->upload.size() * 4);
+        D->at_cnt = align256(D->at_rows + nvg * 64 * 4);
+        D->at_work = align256(D->at_cnt + (size_t)g.NV * R * 2);
+        D->scratch = D->at_work + (D->in_lds ? 0 : (size_t)P.logical_steps * g.fmt.eps * STREAM_FILL_BYTES);
         *runs_out = runs_word(P);
         *groups_out = g.NG;
     }
@@ -1041,34 +1159,32 @@ int stream_fill_device(const StreamDevicePlan& D, const uint32_t* tags, const ui
     const StreamPlan& P = D.P;
     const StreamGeom& g = P.g;
     const size_t nvg = (size_t)g.NV * g.NG;
-    // everything before the steps is assembled on the host; the rest starts as zeros
-    std::vector<unsigned char> front(g.off_steps, 0);
-    memcpy(front.data(), P.head4.data(), P.head4.size() * 4);
-    memcpy(front.data() + g.off_runs, P.runs.data(), P.runs.size() * sizeof(StreamRun));
-    memcpy(front.data() + g.off_rows, P.base.data(), P.base.size() * 4);
-    encode_slots(P, (uint16_t*)(front.data() + g.off_slots));
-    std::vector<uint32_t> lists(nvg * 65 + 1);
-    for (size_t k = 0; k < nvg * 64; ++k) {
-        const uint32_t place = P.slot32[k] & STREAM_NO_ROW;
-        lists[k] = place == STREAM_NO_ROW ? STREAM_NO_ROW : P.base[place];
-    }
-    memcpy(lists.data() + nvg * 64, P.goff.data(), (nvg + 1) * 4);
-    hipError_t e = hipMemcpyAsync(out, front.data(), front.size(), hipMemcpyHostToDevice, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(scratch, lists.data(), lists.size() * 4, hipMemcpyHostToDevice, s);
+    hipError_t e = hipMemcpyAsync(scratch, D.upload.data(), D.upload.size() * 4, hipMemcpyHostToDevice, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);            // (the plan may be freed as soon as this call returns)
     if (e != hipSuccess) return fail(SQ_ELAUNCH, "sq_stream_fill_device: %s", hipGetErrorString(e));
-    const int64_t words = (int64_t)((D.bytes - g.off_steps) / 4);
-    hipLaunchKernelGGL(stream_clear_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, s, (uint32_t*)(out + g.off_steps), words);
-    uint32_t longest = 0;
-    for (size_t k = 0; k < nvg; ++k) longest = std::max(longest, P.goff[k + 1] - P.goff[k]);
+    const int64_t words = (int64_t)(D.bytes / 4);
+    hipLaunchKernelGGL(stream_front_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, s, (const uint32_t*)scratch, (int64_t)P.head4.size(),
+                       (int64_t)(g.off_runs / 4), (int64_t)(P.runs.size() * sizeof(StreamRun) / 4), (int64_t)(g.off_rows / 4), (int64_t)P.base.size(),
+                       (uint32_t*)out, words);
+    StreamSortArgs b{};
+    b.cnt = (uint16_t*)(scratch + D.at_cnt);
+    b.base = (const uint32_t*)(out + g.off_rows);
+    b.seg = (const StreamSegment*)(scratch + D.at_seg);
+    b.rows = (uint32_t*)(scratch + D.at_rows);
+    b.slots = (uint16_t*)(out + g.off_slots);
+    b.R = D.R; b.NG = g.NG; b.eps = g.fmt.eps;
+    launch_count_and_sort(P, tags, D.R, D.W, D.bits, D.G, row_book, (uint16_t*)(scratch + D.at_cnt), b, (int)D.seg.size(), s);
     StreamFillArgs a;
     a.tags = tags; a.row_book = row_book;
     a.heads = (const uint32_t*)out;
-    a.rows = (const uint32_t*)scratch;
-    a.goff = a.rows + nvg * 64;
+    a.rows = b.rows;
+    a.goff = (const uint32_t*)(scratch + D.at_goff);
     a.steps = out + g.off_steps;
-    a.work = scratch + ((lists.size() * 4 + 255) & ~(size_t)255);
+    a.work = scratch + D.at_work;
     a.W = D.W; a.U = g.U; a.bits = D.bits; a.G = D.G; a.PC = g.PC; a.NS = g.NS; a.NV = g.NV; a.NG = g.NG; a.fs = g.fs;
     if (D.in_lds) {
+        uint32_t longest = 0;
+        for (size_t k = 0; k < nvg; ++k) longest = std::max(longest, P.goff[k + 1] - P.goff[k]);
         const size_t lds = (size_t)longest * g.fmt.eps * STREAM_FILL_BYTES;
         (void)hipFuncSetAttribute((const void*)stream_fill_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, STREAM_FILL_LDS);
         (void)hipGetLastError();
@@ -1076,10 +1192,7 @@ int stream_fill_device(const StreamDevicePlan& D, const uint32_t* tags, const ui
     } else {
         hipLaunchKernelGGL((stream_fill_kernel<false>), dim3((unsigned)nvg), dim3(256), 0, s, a);
     }
-    int rc = check_launch("sq_stream_fill_device");
-    if (rc) return rc;
-    e = hipStreamSynchronize(s);                                 // the host lists are read until here
-    return e == hipSuccess ? SQ_OK : fail(SQ_ELAUNCH, "sq_stream_fill_device: %s", hipGetErrorString(e));
+    return check_launch("sq_stream_fill_device");
 }
 
 void stream_plan_free(StreamDevicePlan* D) { delete D; }

@@ -17,7 +17,9 @@ pytestmark = pytest.mark.gpu
 CASES = [(1, 64, 8, 16, 1, 1, 0, "any"), (65, 3584, 8, 16, 1, 1, 2, "any"), (200, 3976, 8, 13, 1, 1, 0, "any"), (64, 3968, 8, 14, 1, 1, 1, "any"),
          (300, 5120, 8, 16, 1, 16, 3, "any"), (130, 8 * 4100, 8, 16, 1, 1, 1, "any"), (70, 8 * 4064, 8, 13, 1, 1, 1, "one"), (90, 1024, 8, 12, 4, 1, 2, "any"),
          (40, 512, 8, 15, 2, 3, 0, "low"), (129, 17408, 8, 16, 1, 1, 0, "low"), (17, 640, 4, 10, 1, 1, 0, "any"), (16, 384, 4, 12, 1, 1, 0, "any"),
-         (31, 896, 4, 8, 2, 1, 0, "any")]
+         (31, 896, 4, 8, 2, 1, 0, "any"),
+         # the longest run there is, runs of one and of several column orders with a short last group, two runs of one order
+         (6144, 256, 8, 13, 1, 1, 1, "any"), (6000, 264, 8, 14, 1, 3, 1, "low"), (1030, 64, 8, 16, 1, 16, 2, "one"), (6145, 128, 8, 13, 1, 1, 1, "low")]
 
 
 @pytest.mark.parametrize("R,C,d,bits,G,M,runs,how", CASES)
