@@ -241,6 +241,7 @@ int sq_codebook_balance_books(const int32_t* tags_host, int32_t R, int32_t W, in
  *                           formats the tile-major copy): *plan_out, the bytes of the buffer and of the scratch the fill
  *                           needs, and runs_out / groups_out as there.  counts: sq_stream_counts_bytes bytes (0 for d = 4).
  *   sq_stream_fill_device   writes the buffer (16-byte aligned, of that size) from the same tags.
+ *   sq_stream_fill_stack_device  the same for n matrices side by side (host arrays of their arguments).
  *   sq_stream_plan_free     ends the plan.
  *   sq_codebook_balance_device  sq_codebook_balance_books; counts: (G << bits) * 4 bytes.
  *   sq_codebook_relabel_device  rewrites the tags through remap (G << bits entries) in place.
@@ -254,6 +255,8 @@ int sq_stream_plan_device(const int32_t* tags, int32_t R, int32_t W, int32_t C, 
                           const uint8_t* row_mask_host, int32_t runs, void* counts, void** plan_out, size_t* bytes_out, size_t* scratch_out,
                           int32_t* runs_out, int32_t* groups_out, void* stream);
 int sq_stream_fill_device(const void* plan, const int32_t* tags, const uint8_t* row_book, void* out, void* scratch, void* stream);
+int sq_stream_fill_stack_device(int32_t n, void* const* plans, const int32_t* const* tags, const uint8_t* const* row_books, void* const* outs,
+                                void* const* scratches, void* stream);
 void sq_stream_plan_free(void* plan);
 int sq_codebook_balance_device(const int32_t* tags, int32_t R, int32_t W, int32_t C, int32_t d, int32_t bits, int32_t G, const uint8_t* row_book,
                                uint32_t* counts, uint16_t* remap_out_host, void* stream);

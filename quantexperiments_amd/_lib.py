@@ -103,6 +103,8 @@ def lib() -> ctypes.CDLL:
         L.sq_stream_plan_device.restype = ctypes.c_int
         L.sq_stream_fill_device.argtypes = [vp, vp, vp, vp, vp, vp]
         L.sq_stream_fill_device.restype = ctypes.c_int
+        L.sq_stream_fill_stack_device.argtypes = [i32, pp, pp, pp, pp, pp, vp]
+        L.sq_stream_fill_stack_device.restype = ctypes.c_int
         L.sq_stream_plan_free.argtypes = [vp]
         L.sq_stream_plan_free.restype = None
         L.sq_codebook_balance_device.argtypes = [vp, i32, i32, i32, i32, i32, i32, vp, vp, vp, vp]
@@ -137,7 +139,7 @@ EXPORTS = ("sq_version", "sq_last_error", "sq_dequant", "sq_linear_small", "sq_l
            "sq_linear_small_from", "sq_linear_small_silu", "sq_gemm_dense_ws", "sq_gemm_dense_workspace_bytes", "sq_linear_small_noalloc",
            "sq_workspace_status", "sq_workspace_reset", "sq_noalloc_reset", "sq_stream_spin_limit", "sq_codebook_balance",
            "sq_stream_bytes_books", "sq_stream_build_books", "sq_codebook_balance_books", "sq_stream_counts_bytes", "sq_stream_plan_device",
-           "sq_stream_fill_device", "sq_stream_plan_free", "sq_codebook_balance_device", "sq_codebook_relabel_device",
+           "sq_stream_fill_device", "sq_stream_fill_stack_device", "sq_stream_plan_free", "sq_codebook_balance_device", "sq_codebook_relabel_device",
            "sq_codebook_rebalance_bytes", "sq_codebook_rebalance_device")
 
 

@@ -452,10 +452,22 @@ int sq_stream_plan_device(const int32_t* tags, int32_t R, int32_t W, int32_t C, 
                               (StreamDevicePlan**)plan_out, bytes_out, scratch_out, runs_out, groups_out, (hipStream_t)stream);
 }
 
+int sq_stream_fill_stack_device(int32_t n, void* const* plans, const int32_t* const* tags, const uint8_t* const* row_books, void* const* outs,
+                                void* const* scratches, void* stream) {
+    const char* who = "sq_stream_fill_device";
+    if (n < 1 || !plans || !tags || !row_books || !outs || !scratches) return fail(SQ_EINVAL, "%s: null pointer", who);
+    std::vector<StreamFill> fills;
+    for (int i = 0; i < n; ++i) {
+        if (!plans[i] || !tags[i] || !outs[i]) return fail(SQ_EINVAL, "%s: null pointer", who);
+        if (((uintptr_t)outs[i] & 15) || ((uintptr_t)scratches[i] & 15)) return fail(SQ_EINVAL, "%s: out and scratch must be 16-byte aligned", who);
+        fills.push_back({(const StreamDevicePlan*)plans[i], (const uint32_t*)tags[i], row_books[i], (unsigned char*)outs[i], (unsigned char*)scratches[i]});
+    }
+    return stream_fill_device(fills.data(), n, (hipStream_t)stream);
+}
+
 int sq_stream_fill_device(const void* plan, const int32_t* tags, const uint8_t* row_book, void* out, void* scratch, void* stream) {
-    if (!plan || !tags || !out) return fail(SQ_EINVAL, "sq_stream_fill_device: null pointer");
-    if (((uintptr_t)out & 15) || ((uintptr_t)scratch & 15)) return fail(SQ_EINVAL, "sq_stream_fill_device: out and scratch must be 16-byte aligned");
-    return stream_fill_device(*(const StreamDevicePlan*)plan, (const uint32_t*)tags, row_book, (unsigned char*)out, (unsigned char*)scratch, (hipStream_t)stream);
+    void* p = const_cast<void*>(plan);
+    return sq_stream_fill_stack_device(1, &p, &tags, &row_book, &out, &scratch, stream);
 }
 
 void sq_stream_plan_free(void* plan) { stream_plan_free((StreamDevicePlan*)plan); }

@@ -90,8 +90,8 @@ struct StreamDevicePlan;
 size_t stream_counts_bytes(int R, int C, int d, int bits, int G);
 int stream_plan_device(const uint32_t* tags, int R, int W, int C, int d, int bits, int G, const uint8_t* row_book, const uint8_t* row_mask_host,
                        int runs, void* counts, StreamDevicePlan** out, size_t* bytes, size_t* scratch, int* runs_out, int* groups_out, hipStream_t s);
-int stream_fill_device(const StreamDevicePlan& D, const uint32_t* tags, const uint8_t* row_book, unsigned char* out, unsigned char* scratch,
-                       hipStream_t s);
+struct StreamFill { const StreamDevicePlan* plan; const uint32_t* tags; const uint8_t* row_book; unsigned char *out, *scratch; };
+int stream_fill_device(const StreamFill* fills, int n, hipStream_t s);
 void stream_plan_free(StreamDevicePlan* D);
 int stream_balance_device(const uint32_t* tags, int R, int W, int C, int d, int bits, uint32_t* counts, uint16_t* remap_out, int G,
                           const uint8_t* row_book, hipStream_t s);

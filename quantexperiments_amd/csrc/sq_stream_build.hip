@@ -729,6 +729,12 @@ struct StreamFillArgs {
     unsigned char* steps;       // the stream buffer's steps
     unsigned char* work;        // groups that LDS does not hold: STREAM_FILL_BYTES per entry slot of every group
     int W, U, bits, G, PC, NS, NV, NG, fs;
+    int wg0;                    // the first workgroup of this matrix
+};
+constexpr int STREAM_FILL_PIECES = 8;
+struct StreamFillStack {
+    StreamFillArgs p[STREAM_FILL_PIECES];
+    int n;
 };
 
 // Bytes one entry slot (64 lanes) of a group takes: 65 words of entries (the odd pitch spreads one lane's entries over the
@@ -767,11 +773,15 @@ __device__ __forceinline__ int stream_moved(int hp, int hq, int M, int at, bool 
 // row), orders them (the steps of BankMatch::order_lanes with ties resolved the same way; the 64 threads search a lane's
 // candidates together), and the four waves write the encoded steps to their places.  The search is a serial chain of
 // LDS reads, so what counts is its length: with the four clocks on one wave, 16 threads each, their branches took turns
-// (3584 x 18944: 49 ms against 10; 3584 x 3584: 1.7 against 0.8).
+// (3584 x 18944: 49 ms against 10; 3584 x 3584: 1.7 against 0.8).  Matrices of a stack are filled side by side: each takes the
+// length of that chain however small it is (3584, 512 and 512 rows of 448 chunks: 1.1 ms in one launch, 2.05 in three).
 template <bool LDS>
-__global__ __launch_bounds__(256) void stream_fill_kernel(StreamFillArgs a) {
+__global__ __launch_bounds__(256) void stream_fill_kernel(StreamFillStack stack) {
     extern __shared__ __attribute__((aligned(16))) unsigned char stream_fill_lds[];
-    const int vg = (int)blockIdx.x, v = vg / a.NG, q = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), t = (int)threadIdx.x & 63, sub = t & 15;
+    int pi = 0;
+    while (pi + 1 < stack.n && (int)blockIdx.x >= stack.p[pi + 1].wg0) ++pi;
+    const StreamFillArgs& a = stack.p[pi];
+    const int vg = (int)blockIdx.x - a.wg0, v = vg / a.NG, q = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), t = (int)threadIdx.x & 63, sub = t & 15;
     const StreamFmt f = stream_fmt(a.PC);
     const int nst = (int)a.heads[(size_t)vg * 4 + 1], ns = nst * f.eps;
     if (ns == 0) return;
@@ -1148,50 +1158,74 @@ int stream_plan_device(const uint32_t* tags, int R, int W, int C, int d, int bit
     return SQ_OK;
 }
 
-int stream_fill_device(const StreamDevicePlan& D, const uint32_t* tags, const uint8_t* row_book, unsigned char* out, unsigned char* scratch, hipStream_t s) {
-    if (D.tiled) {
-        const int ud = D.bits == 12 ? 3 : D.bits == 10 ? 5 : 4;
-        const int64_t n = (int64_t)((D.R + 15) / 16) * 16 * (D.W / ud);
-        if (n == 0) return SQ_OK;
-        hipLaunchKernelGGL(tiled_build_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, tags, D.R, D.W, ud, (uint32_t*)out);
-        return check_launch("sq_stream_fill_device");
+int stream_fill_device(const StreamFill* fills, int n, hipStream_t s) {
+    hipError_t e = hipSuccess;
+    bool wait = false;
+    for (int i = 0; i < n && e == hipSuccess; ++i) {
+        const StreamDevicePlan& D = *fills[i].plan;
+        if (D.tiled) continue;
+        e = hipMemcpyAsync(fills[i].scratch, D.upload.data(), D.upload.size() * 4, hipMemcpyHostToDevice, s);
+        wait = true;
     }
-    const StreamPlan& P = D.P;
-    const StreamGeom& g = P.g;
-    const size_t nvg = (size_t)g.NV * g.NG;
-    hipError_t e = hipMemcpyAsync(scratch, D.upload.data(), D.upload.size() * 4, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);            // (the plan may be freed as soon as this call returns)
+    if (wait) {                                                  // (the plans may be freed as soon as this call returns)
+        const hipError_t w = hipStreamSynchronize(s);
+        if (e == hipSuccess) e = w;
+    }
     if (e != hipSuccess) return fail(SQ_ELAUNCH, "sq_stream_fill_device: %s", hipGetErrorString(e));
-    const int64_t words = (int64_t)(D.bytes / 4);
-    hipLaunchKernelGGL(stream_front_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, s, (const uint32_t*)scratch, (int64_t)P.head4.size(),
-                       (int64_t)(g.off_runs / 4), (int64_t)(P.runs.size() * sizeof(StreamRun) / 4), (int64_t)(g.off_rows / 4), (int64_t)P.base.size(),
-                       (uint32_t*)out, words);
-    StreamSortArgs b{};
-    b.cnt = (uint16_t*)(scratch + D.at_cnt);
-    b.base = (const uint32_t*)(out + g.off_rows);
-    b.seg = (const StreamSegment*)(scratch + D.at_seg);
-    b.rows = (uint32_t*)(scratch + D.at_rows);
-    b.slots = (uint16_t*)(out + g.off_slots);
-    b.R = D.R; b.NG = g.NG; b.eps = g.fmt.eps;
-    launch_count_and_sort(P, tags, D.R, D.W, D.bits, D.G, row_book, (uint16_t*)(scratch + D.at_cnt), b, (int)D.seg.size(), s);
-    StreamFillArgs a;
-    a.tags = tags; a.row_book = row_book;
-    a.heads = (const uint32_t*)out;
-    a.rows = b.rows;
-    a.goff = (const uint32_t*)(scratch + D.at_goff);
-    a.steps = out + g.off_steps;
-    a.work = scratch + D.at_work;
-    a.W = D.W; a.U = g.U; a.bits = D.bits; a.G = D.G; a.PC = g.PC; a.NS = g.NS; a.NV = g.NV; a.NG = g.NG; a.fs = g.fs;
-    if (D.in_lds) {
+    StreamFillStack stack{};
+    int wgs = 0;
+    size_t lds = 0;
+    auto fill = [&]() {
+        if (stack.n == 0) return;
+        if (lds) hipLaunchKernelGGL((stream_fill_kernel<true>), dim3((unsigned)wgs), dim3(256), lds, s, stack);
+        else hipLaunchKernelGGL((stream_fill_kernel<false>), dim3((unsigned)wgs), dim3(256), 0, s, stack);
+        stack.n = wgs = 0;
+        lds = 0;
+    };
+    (void)hipFuncSetAttribute((const void*)stream_fill_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, STREAM_FILL_LDS);
+    (void)hipGetLastError();
+    for (int i = 0; i < n; ++i) {
+        const StreamDevicePlan& D = *fills[i].plan;
+        unsigned char *out = fills[i].out, *scratch = fills[i].scratch;
+        if (D.tiled) {
+            const int ud = D.bits == 12 ? 3 : D.bits == 10 ? 5 : 4;
+            const int64_t units = (int64_t)((D.R + 15) / 16) * 16 * (D.W / ud);
+            if (units > 0)
+                hipLaunchKernelGGL(tiled_build_kernel, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, s, fills[i].tags, D.R, D.W, ud, (uint32_t*)out);
+            continue;
+        }
+        const StreamPlan& P = D.P;
+        const StreamGeom& g = P.g;
+        const size_t nvg = (size_t)g.NV * g.NG;
+        const int64_t words = (int64_t)(D.bytes / 4);
+        hipLaunchKernelGGL(stream_front_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, s, (const uint32_t*)scratch, (int64_t)P.head4.size(),
+                           (int64_t)(g.off_runs / 4), (int64_t)(P.runs.size() * sizeof(StreamRun) / 4), (int64_t)(g.off_rows / 4), (int64_t)P.base.size(),
+                           (uint32_t*)out, words);
+        StreamSortArgs b{};
+        b.cnt = (uint16_t*)(scratch + D.at_cnt);
+        b.base = (const uint32_t*)(out + g.off_rows);
+        b.seg = (const StreamSegment*)(scratch + D.at_seg);
+        b.rows = (uint32_t*)(scratch + D.at_rows);
+        b.slots = (uint16_t*)(out + g.off_slots);
+        b.R = D.R; b.NG = g.NG; b.eps = g.fmt.eps;
+        launch_count_and_sort(P, fills[i].tags, D.R, D.W, D.bits, D.G, fills[i].row_book, (uint16_t*)(scratch + D.at_cnt), b, (int)D.seg.size(), s);
         uint32_t longest = 0;
         for (size_t k = 0; k < nvg; ++k) longest = std::max(longest, P.goff[k + 1] - P.goff[k]);
-        const size_t lds = (size_t)longest * g.fmt.eps * STREAM_FILL_BYTES;
-        (void)hipFuncSetAttribute((const void*)stream_fill_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, STREAM_FILL_LDS);
-        (void)hipGetLastError();
-        hipLaunchKernelGGL((stream_fill_kernel<true>), dim3((unsigned)nvg), dim3(256), lds, s, a);
-    } else {
-        hipLaunchKernelGGL((stream_fill_kernel<false>), dim3((unsigned)nvg), dim3(256), 0, s, a);
+        // neighbours whose groups fit LDS, or neighbours whose do not, up to STREAM_FILL_PIECES
+        if (stack.n == STREAM_FILL_PIECES || (stack.n && (lds != 0) != D.in_lds) || (int64_t)wgs + (int64_t)nvg >= ((int64_t)1 << 31)) fill();
+        StreamFillArgs& a = stack.p[stack.n++];
+        a.tags = fills[i].tags; a.row_book = fills[i].row_book;
+        a.heads = (const uint32_t*)out;
+        a.rows = b.rows;
+        a.goff = (const uint32_t*)(scratch + D.at_goff);
+        a.steps = out + g.off_steps;
+        a.work = scratch + D.at_work;
+        a.W = D.W; a.U = g.U; a.bits = D.bits; a.G = D.G; a.PC = g.PC; a.NS = g.NS; a.NV = g.NV; a.NG = g.NG; a.fs = g.fs;
+        a.wg0 = wgs;
+        wgs += (int)nvg;
+        if (D.in_lds) lds = std::max({lds, (size_t)longest * g.fmt.eps * STREAM_FILL_BYTES, (size_t)16});
     }
+    fill();
     return check_launch("sq_stream_fill_device");
 }
 

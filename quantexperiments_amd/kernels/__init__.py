@@ -183,9 +183,14 @@ class PackedLinear(torch.nn.Module):
             raise RuntimeError("the packed tags of this matrix were dropped (compact): its stream cannot be rebuilt")
         if self.wants_stream and self.balance and not self.relabelled:
             _relabel([self])
-        self.stream, self.stream_runs, self.stream_groups = build_stream(
-            self.words, self.C, self.d, self.bits, self.row_mask if self.has_mask else None, runs,
-            row_book=None if self.row_book is None else (self.row_book, self.G))
+        self._set_stream(_fill_streams([self._plan_stream(runs)])[0], runs)
+
+    def _plan_stream(self, runs: int) -> "_StreamPlan":
+        return _StreamPlan(self.words, self.C, self.d, self.bits, self.row_mask if self.has_mask else None, runs,
+                           None if self.row_book is None else (self.row_book, self.G))
+
+    def _set_stream(self, built: tuple, runs: int) -> None:
+        self.stream, self.stream_runs, self.stream_groups = built
         self.stream_asked = runs
         if self.stream is None:
             self.wants_stream = False
@@ -308,7 +313,7 @@ def build_stream(words: torch.Tensor, C: int, d: int, bits: int, row_mask=None, 
     other in its table (sq_stream_build_books; not together with `table`)."""
     L = _lib.lib()
     if words.is_cuda and table is None:
-        return _build_stream_device(words, C, d, bits, row_mask, runs, row_book)
+        return _fill_streams([_StreamPlan(words, C, d, bits, row_mask, runs, row_book)])[0]
     host = words.detach().to("cpu", torch.int32).contiguous()
     mask = None if row_mask is None else row_mask.detach().to("cpu", torch.uint8).contiguous()
     mp = None if mask is None else mask.data_ptr()
@@ -341,38 +346,59 @@ def build_stream(words: torch.Tensor, C: int, d: int, bits: int, row_mask=None, 
     return out.to(words.device), r.value, g.value
 
 
-def _build_stream_device(words: torch.Tensor, C: int, d: int, bits: int, row_mask, runs: int, row_book):
-    """build_stream for tags on the GPU: the library plans on the host from counts taken there and writes the buffer on the
-    GPU (sq_stream_plan_device, sq_stream_fill_device); the tags never leave the device."""
-    L, dev = _lib.lib(), words.device
-    words = words.detach().to(torch.int32).contiguous()
-    mask = None if row_mask is None else row_mask.detach().to("cpu", torch.uint8).contiguous()
-    R, W = words.shape
-    book, G = None, 1
-    if row_book is not None:
-        book, G = row_book if isinstance(row_book, tuple) else (row_book, None)
-        if G is None:
-            G = 1 << (int(book.max()).bit_length() if R else 0)
-        _check_row_ids(book, R, G, "row_book")
-        book = book.detach().to(dev, torch.uint8).contiguous()
-    new = lambda n: torch.empty(max(n, 1), dtype=torch.uint8, device=dev)
-    counts = new(L.sq_stream_counts_bytes(R, C, d, bits, G))
-    plan, nbytes, nscratch = ctypes.c_void_p(), ctypes.c_size_t(), ctypes.c_size_t()
-    r, g = ctypes.c_int32(), ctypes.c_int32()
-    bp = None if book is None else book.data_ptr()
-    with torch.cuda.device(dev):
-        rc = L.sq_stream_plan_device(words.data_ptr(), R, W, C, d, bits, G, bp, None if mask is None else mask.data_ptr(), runs,
-                                     counts.data_ptr(), ctypes.byref(plan), ctypes.byref(nbytes), ctypes.byref(nscratch), ctypes.byref(r),
-                                     ctypes.byref(g), _lib.stream_ptr(dev))
+class _StreamPlan:
+    """A stream that is planned but not written yet (sq_stream_plan_device): runs and groups as build_stream returns them, None
+    runs for a format the load-time layouts do not cover."""
+
+    def __init__(self, words: torch.Tensor, C: int, d: int, bits: int, row_mask, runs: int, row_book):
+        L, dev = _lib.lib(), words.device
+        self.plan = ctypes.c_void_p()
+        self.words = words = words.detach().to(torch.int32).contiguous()
+        mask = None if row_mask is None else row_mask.detach().to("cpu", torch.uint8).contiguous()
+        R, W = words.shape
+        self.book, G = None, 1
+        if row_book is not None:
+            book, G = row_book if isinstance(row_book, tuple) else (row_book, None)
+            if G is None:
+                G = 1 << (int(book.max()).bit_length() if R else 0)
+            _check_row_ids(book, R, G, "row_book")
+            self.book = book.detach().to(dev, torch.uint8).contiguous()
+        counts = torch.empty(max(L.sq_stream_counts_bytes(R, C, d, bits, G), 1), dtype=torch.uint8, device=dev)
+        nbytes, nscratch = ctypes.c_size_t(), ctypes.c_size_t()
+        r, g = ctypes.c_int32(), ctypes.c_int32()
+        with torch.cuda.device(dev):
+            rc = L.sq_stream_plan_device(words.data_ptr(), R, W, C, d, bits, G, None if self.book is None else self.book.data_ptr(),
+                                         None if mask is None else mask.data_ptr(), runs, counts.data_ptr(), ctypes.byref(self.plan),
+                                         ctypes.byref(nbytes), ctypes.byref(nscratch), ctypes.byref(r), ctypes.byref(g), _lib.stream_ptr(dev))
+        self.runs = self.groups = None
         if rc in (_lib.SQ_EUNSUPPORTED, _lib.SQ_EINVAL):          # a format the load-time layouts do not cover
-            return None, 0, 0
+            return
         _lib.check(rc)
-        try:
-            out, scratch = new(nbytes.value), new(nscratch.value)
-            _lib.check(L.sq_stream_fill_device(plan, words.data_ptr(), bp, out.data_ptr(), scratch.data_ptr(), _lib.stream_ptr(dev)))
-        finally:
-            L.sq_stream_plan_free(plan)
-    return out, r.value, g.value
+        self.runs, self.groups, self.nbytes, self.nscratch = r.value, g.value, nbytes.value, nscratch.value
+
+    def __del__(self):
+        if self.plan:
+            _lib.lib().sq_stream_plan_free(self.plan)
+            self.plan = None
+
+
+def _fill_streams(plans) -> list:
+    """(stream, runs, groups) of every plan, their buffers written side by side on the GPU (sq_stream_fill_stack_device)."""
+    todo = [p for p in plans if p.runs is not None]
+    outs, keep = {}, []
+    if todo:
+        dev = todo[0].words.device
+        new = lambda n: torch.empty(max(n, 1), dtype=torch.uint8, device=dev)
+        for p in todo:
+            outs[id(p)] = new(p.nbytes)
+            keep.append(new(p.nscratch))
+        ptrs = lambda ps: (ctypes.c_void_p * len(todo))(*ps)
+        with torch.cuda.device(dev):
+            _lib.check(_lib.lib().sq_stream_fill_stack_device(
+                len(todo), ptrs(p.plan.value for p in todo), ptrs(p.words.data_ptr() for p in todo),
+                ptrs(None if p.book is None else p.book.data_ptr() for p in todo), ptrs(outs[id(p)].data_ptr() for p in todo),
+                ptrs(k.data_ptr() for k in keep), _lib.stream_ptr(dev)))
+    return [(outs[id(p)], p.runs, p.groups) if p.runs is not None else (None, 0, 0) for p in plans]
 
 
 STREAM_PART_MAX = 4064      # chunks per column part of the tag stream (sq_stream.h)
@@ -394,13 +420,21 @@ def prepare_stack(pieces, workgroups: int | None = None) -> None:
     # still fits the device in one round of workgroups.
     _relabel([p for p in ps if p.stream is None and p.words is not None and p.balance and not p.relabelled])
     rows = sum(p.R for p in ps)
+    planned = []
     for p in sorted(ps, key=lambda q: q.R):
         buckets = ((p.G << p.bits) >> 12) * -(-(p.C // p.d) // STREAM_PART_MAX)
         runs = max(1, round(workgroups * p.R / rows / buckets))
         if p.words is not None and (p.stream is None or (runs != p.stream_asked and not (default and len(ps) == 1 and p.stream_asked == 0))):
-            p.build_stream(runs)
-        workgroups = max(workgroups - (p.stream_runs & 0xFFFF) * buckets, buckets)
+            if p.balance and not p.relabelled:
+                _relabel([p])
+            planned.append((p, runs, p._plan_stream(runs)))
+            made = planned[-1][2].runs or 0
+        else:
+            made = p.stream_runs
+        workgroups = max(workgroups - (made & 0xFFFF) * buckets, buckets)
         rows -= p.R
+    for (p, runs, _), built in zip(planned, _fill_streams([plan for _, _, plan in planned])):
+        p._set_stream(built, runs)
 
 
 def _prep(pieces, x: torch.Tensor, y: torch.Tensor):
