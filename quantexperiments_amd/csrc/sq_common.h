@@ -150,6 +150,10 @@ bool mid_dense_ok(const sq_matrix* mats, int n, int T);
 size_t mid_dense_workspace(const sq_matrix* mats, int n, int T);
 int launch_mid_decoded(const sq_matrix* mats, int n, const void* const* w, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T,
                        void* ws, hipStream_t s);
+// more rows in tiles whose weights are gathered on their way into LDS (sq_fused.h)
+bool fused_route(const sq_matrix* mats, int n, int T);
+size_t fused_workspace(const sq_matrix* mats, int n, int T);
+int launch_fused(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, hipStream_t s);
 // most activation rows for which passes of SQ_SMALL_BMAX rows through the decode-time kernel beat decode + GEMM
 // for these pieces (0: never), where they cannot share a pass
 int small_pass_limit(const sq_matrix* mats, int n);

@@ -1,0 +1,178 @@
+// Host side of the product of sq_fused.h: which stacks take it, how the work is cut, the activations in fragment order, and the
+// sum of the K slices.
+#include <algorithm>
+#include "sq_fused.h"
+
+namespace sq {
+
+int launch_fused_b16d8(const FusedArgs&, int, int, int, hipStream_t);
+int launch_fused_b12d4(const FusedArgs&, int, int, int, hipStream_t);
+int launch_fused_b10d4(const FusedArgs&, int, int, int, hipStream_t);
+int launch_fused_b8d4(const FusedArgs&, int, int, int, hipStream_t);
+
+// The activations as the kernel's matrix instructions take them: 1 KB blocks of 16 tokens x 32 columns in fp16, block
+// [token block][step][tile of 16 tokens], in it lane l's 16 bytes: token l % 16, columns (4 round + l / 16) UK + 8 j .. + 7 of step
+// j of a round.  Zeros past the last token and column.  A workgroup turns 16 tokens x one round (4 UK columns, read in whole
+// lines) round in LDS, whose blocks lie 1040 bytes apart so that neighbouring steps' pieces fall on different banks.
+template <int SPR>
+__global__ __launch_bounds__(256) void fused_x_kernel(const uint16_t* __restrict__ x, int64_t ldx, int x_dtype, int T, int C, int NT, int k32,
+                                                      unsigned char* __restrict__ out) {
+    __shared__ __attribute__((aligned(16))) unsigned char turn[SPR * 1040];
+    constexpr int PCS = 4 * SPR;                                          // 16-byte pieces of a token
+    const int round = (int)blockIdx.x, tile = (int)blockIdx.y, tb = tile / NT, n = tile - tb * NT;
+    for (int i = threadIdx.x; i < 16 * PCS; i += 256) {
+        const int tl = i / PCS, c = i - tl * PCS, t = tile * 16 + tl, col = (round * PCS + c) * 8;
+        u32x4 v = u32x4{0u, 0u, 0u, 0u};
+        if (t < T && col < C) {
+            v = *reinterpret_cast<const u32x4*>(x + (int64_t)t * ldx + col);
+            if (x_dtype == SQ_BF16) { v.x = bf2h_x2(v.x); v.y = bf2h_x2(v.y); v.z = bf2h_x2(v.z); v.w = bf2h_x2(v.w); }
+        }
+        *reinterpret_cast<u32x4*>(turn + (c % SPR) * 1040 + ((c / SPR) * 16 + tl) * 16) = v;
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < 16 * PCS; i += 256) {
+        const int j = i >> 6, l = i & 63;
+        *reinterpret_cast<u32x4*>(out + (((int64_t)tb * k32 + round * SPR + j) * NT + n) * 1024 + l * 16) = *reinterpret_cast<const u32x4*>(turn + j * 1040 + l * 16);
+    }
+}
+
+// y[t, y_off + r] = row_scale[r] * sum over the slices of part[slice][t][r], four rows of one token per thread
+__global__ __launch_bounds__(256) void fused_reduce_kernel(FusedArgs a) {
+    int pi = 0;
+    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    while (pi < a.n && i >= (int64_t)a.T * ((a.p[pi].m.R + 3) / 4)) i -= (int64_t)a.T * ((a.p[pi].m.R + 3) / 4), ++pi;
+    if (pi >= a.n) return;
+    const sq_matrix& m = a.p[pi].m;
+    const int q = (m.R + 3) / 4, t = (int)(i / q), r = (int)(i - (int64_t)t * q) * 4;
+    const float* p = a.p[pi].part + (int64_t)t * m.R + r;
+    const int64_t step = (int64_t)a.T * m.R;
+    float4v v = {0.f, 0.f, 0.f, 0.f};
+    if (m.R % 4 == 0) {
+        float4v s[8];                                                     // (all slices on their way at once)
+#pragma unroll
+        for (int k = 0; k < 8; ++k) s[k] = *reinterpret_cast<const float4v*>(p + min(k, a.ks - 1) * step);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) if (k < a.ks) v += s[k];
+    } else {
+        for (int k = 0; k < a.ks; ++k)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] += r + e < m.R ? p[k * step + e] : 0.f;
+    }
+    const int64_t o = (int64_t)t * a.ldy + m.y_off + r;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        if (r + e < m.R) store_y(a.y, a.y_dtype, o + e, v[e] * h2f(m.row_scale[r + e]));
+}
+
+struct FusedPlan { int nw, tw, ks, tbs; };
+
+static int fused_unit_dwords(int bits) { return bits == 12 ? 3 : bits == 10 ? 5 : 4; }
+static int fused_round_steps(const sq_matrix& m) { return fused_unit_dwords(m.bits) * 32 / m.bits / (8 / m.d); }
+static int fused_rounds(const sq_matrix& m) { return (m.W / fused_unit_dwords(m.bits) + 3) / 4; }
+
+// How a product is cut, nw = 0 where the other kernels are the faster ones.  Up to 768 rows, in blocks of up to 384 tokens; rows of
+// the weights in tiles of 32 tw, where a launch should fill the CUs once: what a workgroup takes hardly depends on how many run
+// beside it.  A tile of 64 / 96 / 128 / 160 rows x 333 tokens x 3584 columns takes 66 / 82 / 105 / 125 us with 16-bit tags of
+// width 8 (the weights below), 62 / 72 / 88 / 101 with 10-bit ones of width 4.  Decoded and multiplied in tiles, or in one pass over the tags where
+// that is the faster one (sq_mid.h), against here, us (d = 8, then d = 4):
+//   rows x columns    200 tokens                333                       512                       768
+//   12000 x 3584      75 / 57    58 / 46        79 / 66    71 / 62        79 / 77    69 / 60        92 / 89    84 / 80
+//   18944 x 3584      95 / 72    72 / 55        97 / 83   113 / 72       112 / 111   98 / 83       133 / 127  121 / 109
+//   25000 x 3584     105 / 90    73 / 77 (160)  118 / 109 114 / 97 (160)  143 / 186  124 / 149     210 / 225  180 / 192
+//   37888 x 3584     177 / 106  104 / 79       234 / 130  154 / 102      263 / 216  209 / 164      301 / 246  245 / 206
+//   3584 x 18944      96 / 72    67 / 59       132 / 90   109 / 77       143 / 137  136 / 102      173 / 162  152 / 136
+// so two blocks of tokens need the last round of workgroups nearly full, and rows of 8192 columns and more are cut into K slices of
+// 2048 at least where there are too few tiles (in shorter rows the slices' sums cost what they gain: 4608 x 3584 at 333 tokens 51 us
+// in three, 53 there).  At 1000 tokens 191 / 225 for 18944 rows, 371 / 353 for 37888.
+static FusedPlan fused_plan(const sq_matrix* mats, int n, int T, int cus) {
+    const FusedPlan none{0, 0, 1, 1};
+    if (T < 129 || T > 768) return none;
+    const int tbs = T <= 384 ? 1 : 2, per = (T + tbs - 1) / tbs, nw = per <= 192 ? 3 : per <= 256 ? 4 : 6;
+    const int table = mats[0].d == 4 ? (mats[0].G << mats[0].bits) * 8 : 0, weight[6] = {0, 0, 17, 21, 27, 32};
+    auto fits = [&](int tw) { return fused_lds(mats[0].bits, table, nw, tw, fused_steps(nw), fused_slots(mats[0].d, nw)) <= 160 * 1024; };
+    auto tiles = [&](int tw) {
+        int64_t b = 0;
+        for (int i = 0; i < n; ++i) b += (mats[i].R + 32 * tw - 1) / (32 * tw);
+        return b * tbs;
+    };
+    int64_t rows = 0;
+    for (int i = 0; i < n; ++i) rows += mats[i].R;
+    int tw = 0;
+    int64_t rounds = 0;
+    for (int w = 2; w <= 5; ++w) {
+        const int64_t r = (tiles(w) + cus - 1) / cus;
+        if (fits(w) && (!tw || r * weight[w] < rounds * weight[tw])) tw = w, rounds = r;
+    }
+    if (!tw) return none;
+    const int64_t used = rows * tbs * 100, room = rounds * cus * 32 * tw;     // percent of the weight rows that the rounds have room for
+    if (tbs == 1 ? used >= (rounds == 1 ? 66 : 60) * room : tw >= 3 && used >= 85 * room) return {nw, tw, 1, tbs};
+    if (mats[0].d == 8 && nw == 4 && tbs == 1 && tiles(1) <= cus && used >= 70 * cus * 32) return {nw, 1, 1, tbs};   // (6000 x 3584 at 200 tokens: 43 us, 49 there)
+    const int64_t t3 = tiles(3);
+    const int ks = (int)std::min<int64_t>({8, cus / t3, mats[0].C / 2048});
+    if (fits(3) && mats[0].C >= 8192 && ks > 1 && t3 * ks * 4 >= cus * 3) return {nw, 3, ks, tbs};
+    return none;
+}
+
+static size_t fused_x_bytes(const sq_matrix* mats, const FusedPlan& p) {
+    return (size_t)p.tbs * fused_rounds(mats[0]) * fused_round_steps(mats[0]) * FUSED_TN * p.nw * 1024;
+}
+static size_t fused_part_bytes(const sq_matrix& m, int T, int ks) { return ks > 1 ? (((size_t)ks * T * m.R * 4) + 255) & ~(size_t)255 : 0; }
+
+bool fused_route(const sq_matrix* mats, int n, int T) {
+    if (n < 1 || n > MID_PIECES) return false;
+    for (int i = 0; i < n; ++i) {
+        const sq_matrix &m = mats[i], &m0 = mats[0];
+        if (!mma_shape(m) || m.R <= 0 || m.d != m0.d || m.bits != m0.bits || m.W != m0.W || m.G != m0.G) return false;
+        if (((int64_t)m.R + 16) * m.W * 4 >= ((int64_t)1 << 32)) return false;                 // 32-bit offsets
+        if (m.d == 8 && ((int64_t)m.G << m.bits) * 16 > ((int64_t)1 << 31)) return false;
+        if (m.d == 4 && ((int64_t)m.G << m.bits) * 8 > 128 * 1024) return false;
+    }
+    return fused_plan(mats, n, T, device_cus()).nw != 0;
+}
+
+size_t fused_workspace(const sq_matrix* mats, int n, int T) {
+    const FusedPlan p = fused_plan(mats, n, T, device_cus());
+    size_t need = fused_x_bytes(mats, p);
+    for (int i = 0; i < n; ++i) need += fused_part_bytes(mats[i], T, p.ks);
+    return need;
+}
+
+int launch_fused(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, hipStream_t s) {
+    const FusedPlan p = fused_plan(mats, n, T, device_cus());
+    const sq_matrix& m0 = mats[0];
+    FusedArgs a{};
+    a.n = n; a.y = y; a.ldy = ldy; a.T = T; a.y_dtype = y_dtype; a.ks = p.ks;
+    a.U = m0.W / fused_unit_dwords(m0.bits);
+    a.table_bytes = m0.d == 4 ? (m0.G << m0.bits) * 8 : 0;
+    const int rounds = fused_rounds(m0), spr = fused_round_steps(m0), NT = FUSED_TN * p.nw;
+    a.k32 = rounds * spr;
+    a.x = (const unsigned char*)ws;
+    char* part = (char*)ws + fused_x_bytes(mats, p);
+    int64_t quads = 0;
+    for (int i = 0; i < n; ++i) {
+        FusedPiece& P = a.p[i];
+        const sq_matrix& m = mats[i];
+        P.m = m;
+        P.w = m.stream && tiled_format_ok(m.R, m.W, m.C, m.d, m.bits) && ((uintptr_t)m.stream & 15) == 0 ? (const void*)m.stream : nullptr;
+        P.part = (float*)part;
+        part += fused_part_bytes(m, T, p.ks);
+        P.wg0 = a.per_tb;
+        a.per_tb += (m.R + 32 * p.tw - 1) / (32 * p.tw) * p.ks;
+        quads += (int64_t)T * ((m.R + 3) / 4);
+    }
+    const dim3 xgrid((unsigned)rounds, (unsigned)(p.tbs * NT));
+    if (spr == 8) hipLaunchKernelGGL(fused_x_kernel<8>, xgrid, dim3(256), 0, s, (const uint16_t*)x, ldx, x_dtype, T, m0.C, NT, a.k32, (unsigned char*)ws);
+    else hipLaunchKernelGGL(fused_x_kernel<4>, xgrid, dim3(256), 0, s, (const uint16_t*)x, ldx, x_dtype, T, m0.C, NT, a.k32, (unsigned char*)ws);
+    int rc = check_launch("sq_linear_gemm(fused, activations)");
+    if (rc) return rc;
+    const int grid = a.per_tb * p.tbs;
+    if (m0.d == 8) rc = launch_fused_b16d8(a, p.nw, p.tw, grid, s);
+    else if (m0.bits == 12) rc = launch_fused_b12d4(a, p.nw, p.tw, grid, s);
+    else if (m0.bits == 10) rc = launch_fused_b10d4(a, p.nw, p.tw, grid, s);
+    else rc = launch_fused_b8d4(a, p.nw, p.tw, grid, s);
+    if (rc || p.ks == 1) return rc;
+    hipLaunchKernelGGL(fused_reduce_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s, a);
+    return check_launch("sq_linear_gemm(fused reduce)");
+}
+
+}  // namespace sq

@@ -1,0 +1,5 @@
+// Kernels of sq_fused.h for 8-bit tags, chunk width 4.
+#include "sq_fused.h"
+namespace sq {
+SQ_FUSED_FORMAT(8, 4)
+}

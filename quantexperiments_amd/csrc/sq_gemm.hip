@@ -324,7 +324,7 @@ static size_t gemm_workspace_beyond_small(const sq_matrix* mats, int n, int T) {
     // (covers the other routes too: the size is asked for without knowing x; up to SQ_SMALL_BMAX rows the only one is the
     // decode-time kernel, which the caller adds)
     if (T <= SQ_SMALL_BMAX && decoded_route(mats, n, T)) return decoded_workspace(mats, n, T);
-    const size_t rest = gemm_workspace_without_mid(mats, n, T);
+    const size_t rest = std::max(gemm_workspace_without_mid(mats, n, T), fused_route(mats, n, T) ? fused_workspace(mats, n, T) : (size_t)0);
     if (mid_ok(mats, n, T)) return std::max(rest, mid_workspace(mats, n, T));
     return decoded_route(mats, n, T) ? std::max(rest, decoded_workspace(mats, n, T)) : rest;
 }
@@ -390,6 +390,8 @@ int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_
                 int64_t ldy, int T, void* ws, size_t ws_bytes, void* sums, hipStream_t s) {
     if (T <= SQ_SMALL_BMAX && !small_takes_gemm_route(mats, n, T, x, ldx))
         return launch_small(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, ws_bytes, sums, s);
+    if (x_vec_ok(x, ldx, mats[0].C) && fused_route(mats, n, T) && fused_workspace(mats, n, T) <= ws_bytes)
+        return launch_fused(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);
     if (mid_ok(mats, n, T) && x_vec_ok(x, ldx, mats[0].C) && mid_x_ok(ldx, T)) return launch_mid(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, ws_bytes, s);
     if (T > SQ_SMALL_BMAX && T <= small_pass_limit(mats, n) && x_vec_ok(x, ldx, mats[0].C)) {
         // stacks that cannot go in one pass (pieces of different formats): a few passes of the decode-time kernel read the packed
