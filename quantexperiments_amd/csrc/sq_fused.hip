@@ -1,7 +1,7 @@
-// Host side of the product of sq_fused.h: which stacks take it, how the work is cut, the activations in fragment order, and the
-// sum of the K slices.
+// Host side of the product of sq_fused.h: which stacks take it, how the work is cut, and the activations in fragment order.
 #include <algorithm>
 #include "sq_fused.h"
+#include "sq_slices.h"
 
 namespace sq {
 
@@ -36,34 +36,6 @@ __global__ __launch_bounds__(256) void fused_x_kernel(const uint16_t* __restrict
     }
 }
 
-// y[t, y_off + r] = row_scale[r] * sum over the slices of part[slice][t][r], four rows of one token per thread
-__global__ __launch_bounds__(256) void fused_reduce_kernel(FusedArgs a) {
-    int pi = 0;
-    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    while (pi < a.n && i >= (int64_t)a.T * ((a.p[pi].m.R + 3) / 4)) i -= (int64_t)a.T * ((a.p[pi].m.R + 3) / 4), ++pi;
-    if (pi >= a.n) return;
-    const sq_matrix& m = a.p[pi].m;
-    const int q = (m.R + 3) / 4, t = (int)(i / q), r = (int)(i - (int64_t)t * q) * 4;
-    const float* p = a.p[pi].part + (int64_t)t * m.R + r;
-    const int64_t step = (int64_t)a.T * m.R;
-    float4v v = {0.f, 0.f, 0.f, 0.f};
-    if (m.R % 4 == 0) {
-        float4v s[8];                                                     // (all slices on their way at once)
-#pragma unroll
-        for (int k = 0; k < 8; ++k) s[k] = *reinterpret_cast<const float4v*>(p + min(k, a.ks - 1) * step);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) if (k < a.ks) v += s[k];
-    } else {
-        for (int k = 0; k < a.ks; ++k)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] += r + e < m.R ? p[k * step + e] : 0.f;
-    }
-    const int64_t o = (int64_t)t * a.ldy + m.y_off + r;
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-        if (r + e < m.R) store_y(a.y, a.y_dtype, o + e, v[e] * h2f(m.row_scale[r + e]));
-}
-
 struct FusedPlan { int nw, tw, ks, tbs; };
 
 static int fused_unit_dwords(int bits) { return bits == 12 ? 3 : bits == 10 ? 5 : 4; }
@@ -81,7 +53,8 @@ static int fused_rounds(const sq_matrix& m) { return (m.W / fused_unit_dwords(m.
 //   25000 x 3584     105 / 90    73 / 77 (160)  118 / 109 114 / 97 (160)  143 / 186  124 / 149     210 / 225  180 / 192
 //   37888 x 3584     177 / 106  104 / 79       234 / 130  154 / 102      263 / 216  209 / 164      301 / 246  245 / 206
 //   3584 x 18944      96 / 72    67 / 59       132 / 90   109 / 77       143 / 137  136 / 102      173 / 162  152 / 136
-// so two blocks of tokens need the last round of workgroups nearly full, and rows of 8192 columns and more are cut into K slices of
+// so two blocks of tokens need the last round of workgroups nearly full; a second round is for the widest tiles, where the other way
+// is longer than two of them (d = 8 from 193 tokens, d = 4 from 257); and rows of 8192 columns and more are cut into K slices of
 // 2048 at least where there are too few tiles (in shorter rows the slices' sums cost what they gain: 4608 x 3584 at 333 tokens 51 us
 // in three, 53 there).  At 1000 tokens 191 / 225 for 18944 rows, 371 / 353 for 37888.
 static FusedPlan fused_plan(const sq_matrix* mats, int n, int T, int cus) {
@@ -105,7 +78,8 @@ static FusedPlan fused_plan(const sq_matrix* mats, int n, int T, int cus) {
     }
     if (!tw) return none;
     const int64_t used = rows * tbs * 100, room = rounds * cus * 32 * tw;     // percent of the weight rows that the rounds have room for
-    if (tbs == 1 ? used >= (rounds == 1 ? 66 : 60) * room : tw >= 3 && used >= 85 * room) return {nw, tw, 1, tbs};
+    const bool whole = tbs == 1 ? used >= 66 * room : used >= 85 * room && tw >= 3;
+    if (whole && (rounds == 1 || (tw == 5 && (tbs == 2 || nw == 6 || (nw == 4 && mats[0].d == 8))))) return {nw, tw, 1, tbs};
     if (mats[0].d == 8 && nw == 4 && tbs == 1 && tiles(1) <= cus && used >= 70 * cus * 32) return {nw, 1, 1, tbs};   // (6000 x 3584 at 200 tokens: 43 us, 49 there)
     const int64_t t3 = tiles(3);
     const int ks = (int)std::min<int64_t>({8, cus / t3, mats[0].C / 2048});
@@ -171,7 +145,7 @@ int launch_fused(const sq_matrix* mats, int n, const void* x, int x_dtype, int64
     else if (m0.bits == 10) rc = launch_fused_b10d4(a, p.nw, p.tw, grid, s);
     else rc = launch_fused_b8d4(a, p.nw, p.tw, grid, s);
     if (rc || p.ks == 1) return rc;
-    hipLaunchKernelGGL(fused_reduce_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(slice_sum_kernel<FusedArgs>, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s, a);
     return check_launch("sq_linear_gemm(fused reduce)");
 }
 

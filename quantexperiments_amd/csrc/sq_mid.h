@@ -7,22 +7,21 @@
 // codewords (LDS) or one d = 8 codeword (L2), so a lane gathers its operand straight into registers and uses it for all NT
 // tiles of 16 activation rows; the activations are the B operand and come from LDS.
 //
-// Bound: d = 8 by the gathers up to about 128 rows (one L2 request each, 16 bytes used of the 64 that come: 17 M of 18.5 M requests,
-// 153 G a second, for 18944 x 2 x 3584 at 64 rows, which take 107 us; the matrix cores are busy 15 % of the time).  d = 4 by no pipe
+// Bound: d = 8 by the gathers up to about 128 rows (one L2 request each, 16 bytes used of the 64 that come: 178 G a second for
+// 18944 x 2 x 3584 at 77 rows, which take 96 us; the matrix cores are busy 15 % of the time).  d = 4 by no pipe
 // alone: with 12-bit tags at 128 rows the matrix cores are busy 47 % of a CU's time and LDS 51 % (every wave reads all the
-// activations for its 32 weight rows; 29 % of it bank conflicts of the codeword reads), taking turns, and the 148 workgroups of
-// 18944 x 2 rows leave 108 CUs without work (58 us, 590 TFLOP/s).  Before, in passes of 32 rows or decoded first, at 33 / 77 / 128 /
-// 256 rows: d = 8, 18944 x 2 x 3584: 172 / 205 / 205 / 209 us, now 100 / 107 / 112 / 188; 12-bit: 41 / 68 / 102 / 165, now 30 / 40 /
-// 54 / 105.
+// activations for its 32 weight rows; 29 % of it bank conflicts of the codeword reads), taking turns.  In passes of 32 rows or decoded
+// first, at 33 / 77 / 128 / 256 rows: d = 8, 18944 x 2 x 3584: 172 / 205 / 205 / 209 us, here 90 / 96 / 105 / 188 (sq_fused.h: 108);
+// 12-bit: 41 / 68 / 102 / 165, here 27 / 38 / 53 / 105 (82).
 //
-//   workgroup   8 waves, two per SIMD so that one gathers while the other multiplies (4 waves: a third slower); each has TW tiles
-//               of 16 weight rows x all NT x 16 activation rows (accumulators TW x NT x 4 registers)
+//   workgroup   NW waves, two per SIMD or more so that one gathers while the other multiplies (4 waves: a third slower); each has
+//               TW tiles of 16 weight rows x all NT x 16 activation rows (accumulators TW x NT x 4 registers)
 //   K           in rounds of 4 lane units (UK columns of tags each, as in sq_rows_mfma.h), rounds in stages of S matrix steps;
 //               step j of lane group g is columns (4 round + g) UK + 8 j .. + 7
 //   X           stages of NT x 16 rows x 4 x S x 16 bytes, double buffered in LDS; loaded to registers two stages ahead
 //               (converted bf16 -> fp16 on the way to LDS), one barrier per stage
 //   tags        two rounds ahead; codewords PD steps ahead (one from LDS, three from L2 where the steps are short)
-//   grid        row blocks x ks slices of the rounds; with ks > 1 fp32 partial sums, added by mid_reduce_kernel
+//   grid        row blocks x ks slices of the rounds; with ks > 1 fp32 partial sums, added by slice_sum_kernel
 //
 // D = 0: weights already decoded to fp16 (column orders, formats whose rows are not whole lane units).  The A operand is loaded
 // from there, up to seven steps ahead; step j of lane group g is columns 256 round + 32 j + 8 g .. + 7, so that the four lane groups
@@ -36,8 +35,6 @@
 #include "sq_rows_mfma.h"
 
 namespace sq {
-
-constexpr int MID_NW = 8;                    // waves per workgroup, two per SIMD
 
 struct MidPiece {
     sq_matrix m;
@@ -65,13 +62,13 @@ template <int S> __device__ __forceinline__ int mid_swizzle(int t) {
 
 constexpr int mid_stage_bytes(int NT, int S) { return NT * 16 * S * 64; }
 
-template <int BITS, int D, int NT, int TW, int S, bool BF>
-__global__ __launch_bounds__(64 * MID_NW, 2) void mid_kernel(MidArgs a) {
+template <int BITS, int D, int NT, int TW, int S, int NW, bool BF>
+__global__ __launch_bounds__(64 * NW, 2) void mid_kernel(MidArgs a) {
     constexpr bool DENSE = D == 0;
     constexpr int UD = DENSE ? 1 : unit_of<DENSE ? 16 : BITS>::UD, TPU = DENSE ? 1 : UD * 32 / (DENSE ? 1 : BITS);
     constexpr int SPR = DENSE ? 8 : TPU / (8 / (DENSE ? 1 : D)), UK = DENSE ? 8 : TPU * D, UPR = DENSE ? 4 * SPR : 4, NST = SPR / S;
     constexpr int GC = DENSE ? 8 : UK, JC = DENSE ? 32 : 8, UPS = DENSE ? 4 * S : 0;   // columns from lane group to group, from step to step; units per stage
-    constexpr int ROWB = S * 64, STAGE = mid_stage_bytes(NT, S), NTH = 64 * MID_NW, PCS = (NT * 64 * S + NTH - 1) / NTH;
+    constexpr int ROWB = S * 64, STAGE = mid_stage_bytes(NT, S), NTH = 64 * NW, PCS = (NT * 64 * S + NTH - 1) / NTH;
     constexpr int PD = DENSE ? (NT * TW <= 16 ? 7 : 3) : D == 8 && NT * TW < 24 ? 3 : 1, XB = NT <= 8 ? 2 : 1;   // steps that codewords and activations are fetched ahead of
     static_assert(SPR % S == 0 && SPR % (PD + 1) == 0 && (NST == 1 || NST % 2 == 0), "steps per round");
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -88,7 +85,7 @@ __global__ __launch_bounds__(64 * MID_NW, 2) void mid_kernel(MidArgs a) {
     unsigned char* xbuf = smem + a.table_bytes;
 
     // ---- this wave's tiles (tiles past the last row repeat the last one and are not stored)
-    const int ntiles = (m.R + 15) >> 4, tile0 = (blk * MID_NW + wave) * TW;
+    const int ntiles = (m.R + 15) >> 4, tile0 = (blk * NW + wave) * TW;
     // (byte offsets from a uniform base: one address register per load)
     const bool tiled = !DENSE && P.w;
     const uint32_t us = (tiled ? 16 * UD : UD) * 4;                          // bytes between two units of a row
@@ -252,41 +249,46 @@ __global__ __launch_bounds__(64 * MID_NW, 2) void mid_kernel(MidArgs a) {
     }
 }
 
-template <int BITS, int D, int NT, int TW, int S, bool BF>
+template <int BITS, int D, int NT, int TW, int S, int NW, bool BF>
 int launch_mid_dtype(const MidArgs& a, int grid, hipStream_t s) {
     static bool raised = false;
     if (!raised) {
-        (void)hipFuncSetAttribute((const void*)mid_kernel<BITS, D, NT, TW, S, BF>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        (void)hipFuncSetAttribute((const void*)mid_kernel<BITS, D, NT, TW, S, NW, BF>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         (void)hipGetLastError();
         raised = true;
     }
-    hipLaunchKernelGGL((mid_kernel<BITS, D, NT, TW, S, BF>), dim3((unsigned)grid), dim3(64 * MID_NW), (size_t)a.table_bytes + 2 * mid_stage_bytes(NT, S), s, a);
+    hipLaunchKernelGGL((mid_kernel<BITS, D, NT, TW, S, NW, BF>), dim3((unsigned)grid), dim3(64 * NW), (size_t)a.table_bytes + 2 * mid_stage_bytes(NT, S), s, a);
     return check_launch("sq_linear_gemm(mid)");
 }
 
-template <int BITS, int D, int NT, int TW, int S>
+template <int BITS, int D, int NT, int TW, int S, int NW>
 int launch_mid_as(const MidArgs& a, int grid, hipStream_t s) {
-    return a.x_dtype == SQ_BF16 ? launch_mid_dtype<BITS, D, NT, TW, S, true>(a, grid, s) : launch_mid_dtype<BITS, D, NT, TW, S, false>(a, grid, s);
+    return a.x_dtype == SQ_BF16 ? launch_mid_dtype<BITS, D, NT, TW, S, NW, true>(a, grid, s) : launch_mid_dtype<BITS, D, NT, TW, S, NW, false>(a, grid, s);
 }
 
 // A variant per number of activation tiles; stages half as deep where many tiles or the codebook leave no room in LDS.
-#define SQ_MID_CASE(NT_, TW_, S_) if (nt == NT_ && tw == TW_ && st == S_) return launch_mid_as<BITS, D, NT_, TW_, S_>(a, grid, s);
+#define SQ_MID_CASE(NT_, TW_, S_, NW_) if (nt == NT_ && tw == TW_ && st == S_ && nw == NW_) return launch_mid_as<BITS, D, NT_, TW_, S_, NW_>(a, grid, s);
 template <int BITS, int D>
-int launch_mid_format(const MidArgs& a, int nt, int tw, int st, int grid, hipStream_t s) {
-    if constexpr (D == 0) { SQ_MID_CASE(1, 2, 4) SQ_MID_CASE(1, 1, 4) }
-    SQ_MID_CASE(3, 2, 4) SQ_MID_CASE(3, 1, 4) SQ_MID_CASE(5, 2, 4) SQ_MID_CASE(5, 1, 4) SQ_MID_CASE(8, 2, 4) SQ_MID_CASE(8, 1, 4)
-    SQ_MID_CASE(12, 2, 2) SQ_MID_CASE(12, 1, 2) SQ_MID_CASE(16, 1, 2)
+int launch_mid_format(const MidArgs& a, int nt, int tw, int st, int nw, int grid, hipStream_t s) {
+    if constexpr (D == 0) { SQ_MID_CASE(1, 2, 4, 8) SQ_MID_CASE(1, 1, 4, 8) }
+    SQ_MID_CASE(3, 2, 4, 8) SQ_MID_CASE(3, 1, 4, 8) SQ_MID_CASE(5, 2, 4, 8) SQ_MID_CASE(5, 1, 4, 8) SQ_MID_CASE(8, 2, 4, 8) SQ_MID_CASE(8, 1, 4, 8)
+    SQ_MID_CASE(12, 2, 2, 8) SQ_MID_CASE(12, 1, 2, 8) SQ_MID_CASE(16, 1, 2, 8)
+    if constexpr (D != 0) {
+        SQ_MID_CASE(3, 1, 4, 10) SQ_MID_CASE(3, 1, 4, 12) SQ_MID_CASE(5, 1, 4, 10) SQ_MID_CASE(5, 1, 4, 12) SQ_MID_CASE(12, 1, 2, 12)
+    }
+    if constexpr (D == 8) { SQ_MID_CASE(8, 1, 4, 12) }
     if constexpr (D != 4) {
-        SQ_MID_CASE(16, 2, 2)
+        SQ_MID_CASE(16, 2, 2, 8)
     } else {
-        SQ_MID_CASE(3, 2, 2) SQ_MID_CASE(3, 1, 2) SQ_MID_CASE(5, 2, 2) SQ_MID_CASE(5, 1, 2) SQ_MID_CASE(8, 2, 2) SQ_MID_CASE(8, 1, 2)
+        SQ_MID_CASE(3, 2, 2, 8) SQ_MID_CASE(3, 1, 2, 8) SQ_MID_CASE(5, 2, 2, 8) SQ_MID_CASE(5, 1, 2, 8) SQ_MID_CASE(8, 2, 2, 8) SQ_MID_CASE(8, 1, 2, 8)
+        SQ_MID_CASE(3, 1, 2, 10) SQ_MID_CASE(3, 1, 2, 12) SQ_MID_CASE(5, 1, 2, 10) SQ_MID_CASE(5, 1, 2, 12)
     }
     return SQ_EUNSUPPORTED;
 }
 
 #define SQ_MID_FORMAT(BITS, D)                                                                                             \
-    int launch_mid_b##BITS##d##D(const MidArgs& a, int nt, int tw, int st, int grid, hipStream_t s) {                     \
-        return launch_mid_format<BITS, D>(a, nt, tw, st, grid, s);                                                         \
+    int launch_mid_b##BITS##d##D(const MidArgs& a, int nt, int tw, int st, int nw, int grid, hipStream_t s) {                     \
+        return launch_mid_format<BITS, D>(a, nt, tw, st, nw, grid, s);                                                         \
     }
 
 }  // namespace sq

@@ -1,49 +1,30 @@
-// Host side of the product for 33 to 256 (384) activation rows (kernel: sq_mid.h): which stacks it takes, how the work is
-// cut, and the sum of the K slices.
+// Host side of the product for 33 to 256 (384) activation rows (kernel: sq_mid.h): which stacks it takes, and how the work
+// is cut.
 #include <algorithm>
 #include "sq_mid.h"
+#include "sq_slices.h"
 
 namespace sq {
 
-int launch_mid_b16d8(const MidArgs&, int, int, int, int, hipStream_t);
-int launch_mid_b12d4(const MidArgs&, int, int, int, int, hipStream_t);
-int launch_mid_b10d4(const MidArgs&, int, int, int, int, hipStream_t);
-int launch_mid_b8d4(const MidArgs&, int, int, int, int, hipStream_t);
-int launch_mid_dense(const MidArgs&, int, int, int, int, hipStream_t);
+int launch_mid_b16d8(const MidArgs&, int, int, int, int, int, hipStream_t);
+int launch_mid_b12d4(const MidArgs&, int, int, int, int, int, hipStream_t);
+int launch_mid_b10d4(const MidArgs&, int, int, int, int, int, hipStream_t);
+int launch_mid_b8d4(const MidArgs&, int, int, int, int, int, hipStream_t);
+int launch_mid_dense(const MidArgs&, int, int, int, int, int, hipStream_t);
 
-// y[t, y_off + r] = row_scale[r] * sum over the slices of part[slice][t][r], four rows of one token per thread
-__global__ __launch_bounds__(256) void mid_reduce_kernel(MidArgs a) {
-    int pi = 0;
-    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    while (pi < a.n && i >= (int64_t)a.T * ((a.p[pi].m.R + 3) / 4)) i -= (int64_t)a.T * ((a.p[pi].m.R + 3) / 4), ++pi;
-    if (pi >= a.n) return;
-    const sq_matrix& m = a.p[pi].m;
-    const int q = (m.R + 3) / 4, t = (int)(i / q), r = (int)(i - (int64_t)t * q) * 4;
-    const float* p = a.p[pi].part + (int64_t)t * m.R + r;
-    float4v v = {0.f, 0.f, 0.f, 0.f};
-    for (int s = 0; s < a.ks; ++s, p += (int64_t)a.T * m.R) {
-        if (m.R % 4 == 0) v += *reinterpret_cast<const float4v*>(p);
-        else
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] += r + e < m.R ? p[e] : 0.f;
-    }
-    const int64_t o = (int64_t)t * a.ldy + m.y_off + r;
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-        if (r + e < m.R) store_y(a.y, a.y_dtype, o + e, v[e] * h2f(m.row_scale[r + e]));
-}
-
-struct MidPlan { int nt, tw, st, ks; };
+struct MidPlan { int nt, tw, st, ks, nw; };
 
 static int mid_units(const sq_matrix& m) { return m.W / (m.bits == 12 ? 3 : m.bits == 10 ? 5 : 4); }
 
 // Variants: NT tiles of 16 activation rows (up to 256 rows; a 24-tile variant ran at half the rate), stages of four matrix steps
-// or, where they do not fit beside the codebook, two.  Two tiles of weight rows per wave (256 rows per workgroup) once that
-// makes a workgroup for every other CU: it halves the activations' way through LDS (18944 x 2 rows at 77 activation rows,
-// 12-bit tags, 148 workgroups: 39 us against 47 with one tile and 296).  Fewer rows are cut along K until there is about one
+// or, where they do not fit beside the codebook, two.  A workgroup is 8 waves of a tile of weight rows, which a CU takes two of no
+// faster than one after the other; where that is more workgroups than CUs, ten or twelve waves if one round is then enough, else
+// two tiles per wave, which halves the activations' way through LDS.  18944 x 2 rows in 148 workgroups of 8 x 2 tiles / 237 of ten
+// (198 of twelve at 128 and 192 activation rows), us, at 40 / 77 / 128 / 192: 10-bit tags 31 / 42 / 55 / 78 and 27 / 37 / 57 (not
+// taken) / 71, 16-bit ones of width 8 100 / 109 / 115 / 142 and 90 / 96 / 105 / 135.  Fewer rows are cut along K until there is about one
 // workgroup per CU, in slices of at least 512 columns (3584 x 3584 at 77 rows, 28 blocks: 28 us whole, 18 in seven).
 static MidPlan mid_plan(const sq_matrix* mats, int n, int T, int cus) {
-    MidPlan p{0, 1, 4, 1};
+    MidPlan p{0, 1, 4, 1, 8};
     const int sizes[] = {3, 5, 8, 12, 16};
     for (int nt : sizes) if (T <= nt * 16) { p.nt = nt; break; }
     if (p.nt == 0) return p;
@@ -52,8 +33,17 @@ static MidPlan mid_plan(const sq_matrix* mats, int n, int T, int cus) {
     if (tab + 2 * mid_stage_bytes(p.nt, p.st) > 160 * 1024) { p.nt = 0; return p; }
     int64_t rows = 0;
     for (int i = 0; i < n; ++i) rows += mats[i].R;
-    if (rows >= (int64_t)cus / 2 * 32 * MID_NW) p.tw = 2;
-    const int64_t blocks = (rows + 16 * MID_NW * p.tw - 1) / (16 * MID_NW * p.tw);
+    auto workgroups = [&](int nw) {
+        int64_t w = 0;
+        for (int i = 0; i < n; ++i) w += (mats[i].R + 16 * nw - 1) / (16 * nw);
+        return w;
+    };
+    if (p.nt == 16 ? rows >= (int64_t)cus / 2 * 32 * 8 : workgroups(8) > cus) {
+        if (p.nt <= 5 && workgroups(10) <= cus) p.nw = 10;
+        else if (p.nt <= 12 && !(p.nt == 8 && mats[0].d == 4) && workgroups(12) <= cus) p.nw = 12;
+        else p.tw = 2;
+    }
+    const int64_t blocks = (rows + 16 * p.nw * p.tw - 1) / (16 * p.nw * p.tw);
     p.ks = (int)std::max<int64_t>(1, std::min<int64_t>({cus / std::max<int64_t>(blocks, 1), 8, mats[0].C / 512}));
     return p;
 }
@@ -121,17 +111,17 @@ static int launch_mid_rows(const sq_matrix* mats, int n, const MidPlan& pl, cons
         P.part = (float*)part;
         part += mid_part_bytes(m, T, pl.ks);
         P.wg0 = wg;
-        wg += ((m.R + 16 * MID_NW * pl.tw - 1) / (16 * MID_NW * pl.tw)) * pl.ks;
+        wg += ((m.R + 16 * pl.nw * pl.tw - 1) / (16 * pl.nw * pl.tw)) * pl.ks;
         quads += (int64_t)T * ((m.R + 3) / 4);
     }
     int rc = SQ_EUNSUPPORTED;
-    if (dense) rc = launch_mid_dense(a, pl.nt, pl.tw, pl.st, wg, s);
-    else if (m0.d == 8) rc = launch_mid_b16d8(a, pl.nt, pl.tw, pl.st, wg, s);
-    else if (m0.bits == 12) rc = launch_mid_b12d4(a, pl.nt, pl.tw, pl.st, wg, s);
-    else if (m0.bits == 10) rc = launch_mid_b10d4(a, pl.nt, pl.tw, pl.st, wg, s);
-    else if (m0.bits == 8) rc = launch_mid_b8d4(a, pl.nt, pl.tw, pl.st, wg, s);
+    if (dense) rc = launch_mid_dense(a, pl.nt, pl.tw, pl.st, pl.nw, wg, s);
+    else if (m0.d == 8) rc = launch_mid_b16d8(a, pl.nt, pl.tw, pl.st, pl.nw, wg, s);
+    else if (m0.bits == 12) rc = launch_mid_b12d4(a, pl.nt, pl.tw, pl.st, pl.nw, wg, s);
+    else if (m0.bits == 10) rc = launch_mid_b10d4(a, pl.nt, pl.tw, pl.st, pl.nw, wg, s);
+    else if (m0.bits == 8) rc = launch_mid_b8d4(a, pl.nt, pl.tw, pl.st, pl.nw, wg, s);
     if (rc || pl.ks == 1) return rc;
-    hipLaunchKernelGGL(mid_reduce_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(slice_sum_kernel<MidArgs>, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s, a);
     return check_launch("sq_linear_gemm(mid reduce)");
 }
 
@@ -139,12 +129,12 @@ static int launch_mid_rows(const sq_matrix* mats, int n, const MidPlan& pl, cons
 // with two), K slices of 256 columns at least, up to eight (3584 x 18944 at 64 rows: 99 us with the decode, 119 in four slices,
 // 111 in nine).
 static MidPlan mid_dense_plan(const sq_matrix* mats, int n, int T, int cus) {
-    MidPlan p{0, 1, 4, 1};
+    MidPlan p{0, 1, 4, 1, 8};
     const int sizes[] = {1, 3, 5, 8, 12, 16};
     for (int nt : sizes) if (T <= nt * 16) { p.nt = nt; break; }
     if (p.nt > 8) p.st = 2;
     int64_t blocks = 0;
-    for (int i = 0; i < n; ++i) blocks += (mats[i].R + 16 * MID_NW - 1) / (16 * MID_NW);
+    for (int i = 0; i < n; ++i) blocks += (mats[i].R + 16 * 8 - 1) / (16 * 8);
     p.ks = (int)std::max<int64_t>(1, std::min<int64_t>({cus / std::max<int64_t>(blocks, 1), 8, mats[0].C / 256}));
     return p;
 }

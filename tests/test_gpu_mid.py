@@ -18,6 +18,9 @@ CASES = [  # rows of the stack's pieces, C, d, bits, G, T
     ((1,), 32, 4, 12, 1, 80), ((127, 3, 260), 1056, 4, 12, 1, 128), ((130,), 2080, 4, 12, 4, 129), ((64, 70), 1024, 4, 12, 4, 256),
     ((33001,), 160, 4, 12, 1, 193), ((32768,), 96, 4, 12, 1, 241), ((4096,), 16384, 4, 12, 1, 257),
     ((16, 1, 130, 40, 7, 64, 33, 20), 512, 8, 16, 1, 70), ((30, 1, 17, 64, 8, 9, 130), 1024, 4, 12, 1, 40), ((24,) * 9, 512, 8, 16, 1, 90),
+    # ten and twelve waves per workgroup
+    ((33000,), 64, 8, 16, 1, 34), ((16500, 16501), 192, 8, 16, 1, 80), ((41500,), 64, 8, 16, 1, 65), ((33003,), 64, 8, 16, 1, 128),
+    ((33001,), 96, 4, 12, 1, 50), ((41000, 30), 64, 4, 10, 1, 70), ((33000,), 64, 4, 8, 1, 33), ((33000,), 96, 4, 12, 4, 150), ((33000,), 96, 4, 12, 2, 150),
     ((257,), 576, 4, 10, 1, 192), ((40, 8), 1600, 4, 10, 2, 34), ((131,), 1536, 4, 8, 1, 129), ((36,), 64, 4, 8, 1, 255),
 ]
 
