@@ -61,6 +61,12 @@ const char* sq_last_error(void);
 int sq_dequant(const sq_matrix* m, void* out, int out_dtype, int64_t ld_out, int32_t r0, int32_t r1,
                void* stream);
 
+/* The dense fp16 weights of n_mats stacked pieces that share C, one behind the other: all rows of mats[0], then of mats[1], ...
+ * at out (rows of C elements; as sq_dequant with SQ_F16 and ld_out = C for each), and on the way, if x is not NULL, the fp16 copy
+ * x_out [B, C] of bf16 activations x [B, C] (row stride ldx; C and ldx multiples of 8, x and x_out 16-byte aligned): what
+ * sq_gemm_dense multiplies next.  Pieces of one kind share a launch. */
+int sq_dequant_stack(const sq_matrix* mats, int32_t n_mats, void* out, const void* x, int64_t ldx, int32_t B, void* x_out, void* stream);
+
 /* Decode-time product for B = 1..SQ_SMALL_BMAX activation rows over n_mats stacked pieces that
  * share C: Y[b, y_off + r] for every piece, X [B, C] with row stride ldx, Y row stride ldy
  * (elements).  x_dtype / y_dtype: SQ_F16 or SQ_BF16 (y may also be SQ_F32).

@@ -91,6 +91,33 @@ int sq_dequant(const sq_matrix* m, void* out, int out_dtype, int64_t ld_out, int
     return launch_dequant(*m, out, out_dtype, ld_out, r0, r1, (hipStream_t)stream);
 }
 
+int sq_dequant_stack(const sq_matrix* mats, int32_t n_mats, void* out, const void* x, int64_t ldx, int32_t B, void* x_out, void* stream) {
+    if (n_mats < 0 || (n_mats > 0 && (!mats || !out))) return fail(SQ_EINVAL, "sq_dequant_stack: n_mats %d out %p", n_mats, out);
+    const hipStream_t s = (hipStream_t)stream;
+    for (int i = 0; i < n_mats; ++i) {
+        if (const int rc = check_matrix(mats[i], "sq_dequant_stack")) return rc;
+        if (mats[i].C != mats[0].C) return fail(SQ_EINVAL, "sq_dequant_stack: stacked pieces disagree on the input size (%d vs %d)", mats[i].C, mats[0].C);
+    }
+    const int C = n_mats ? mats[0].C : 0;
+    bool copy = x && B > 0 && n_mats > 0;
+    if (copy && (!x_out || C % 8 || ldx < C || ldx % 8 || ((uintptr_t)x & 15) || ((uintptr_t)x_out & 15)))
+        return fail(SQ_EINVAL, "sq_dequant_stack: the fp16 copy needs 16-byte aligned rows (x %p ldx %lld x_out %p C %d)", x, (long long)ldx, x_out, C);
+    uint16_t* o = (uint16_t*)out;
+    for (int i = 0, k; i < n_mats; i += k) {
+        for (k = 0; i + k < n_mats && k < GEMM256_PIECES && mats[i + k].R > 0;) ++k;
+        int rc = launch_dequant_stack(mats + i, k, o, 0, copy ? (const uint16_t*)x : nullptr, ldx, B, C, (uint16_t*)x_out, s);
+        if (rc < 0) return rc;
+        if (rc == 0) copy = false;
+        k = std::max(k, 1);
+        for (int j = i; j < i + k; ++j) {
+            if (rc > 0 && mats[j].R > 0)
+                if (const int rc2 = launch_dequant(mats[j], o, SQ_F16, C, 0, mats[j].R, s)) return rc2;
+            o += (size_t)mats[j].R * C;
+        }
+    }
+    return copy ? launch_bf16_to_f16((const uint16_t*)x, ldx, B, C, (uint16_t*)x_out, s) : SQ_OK;
+}
+
 // A workspace as the launchers see it: the header (partial sums of the tag-stream kernel) and what lies behind it.  A
 // buffer of at least SQ_WS_HEADER bytes always begins with the header; a smaller one has none and is used from its
 // first byte, which serves pieces that keep no partial sums (a private workspace of a few KB for a d = 4 matrix).

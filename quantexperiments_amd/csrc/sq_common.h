@@ -165,6 +165,8 @@ size_t gemm_workspace_without_mid(const sq_matrix* mats, int n, int T);
 // pieces through five products.)
 constexpr int GEMM256_PIECES = 8;
 struct Gemm256Scales { const uint16_t* p[GEMM256_PIECES]; int end[GEMM256_PIECES]; int n; };
+int launch_bf16_to_f16(const uint16_t* x, int64_t ldx, int T, int C, uint16_t* out, hipStream_t s);
+int launch_dequant_stack(const sq_matrix* mats, int n, void* out, int raw, const uint16_t* x, int64_t ldx, int T, int C, uint16_t* xout, hipStream_t s);
 int launch_gemm_dense(const void* w, int w_dtype, int64_t ldw, int R, int C, const void* x, int x_dtype, int64_t ldx,
                       void* y, int y_dtype, int64_t ldy, int T, hipStream_t s, void* ws = nullptr, size_t ws_bytes = 0);
 size_t gemm_dense_workspace(int R, int C, int T);

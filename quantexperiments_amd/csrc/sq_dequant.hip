@@ -277,56 +277,139 @@ static int launch_dequant4(Dequant4Args& a, hipStream_t s) {
     return check_launch("sq_dequant");
 }
 
-// Matrices with column orders: scattering 2-byte values straight to HBM costs 4x the plain decode, so a
-// workgroup decodes one row at a time into LDS at its permuted positions (ds_write of one element each, the
-// order read as whole 16/32-byte pieces) and then writes the row out in 16-byte pieces.
-template <int DT, int D>   // D = 8 or 4
-__global__ __launch_bounds__(256) void dequant_rows_lds_kernel(sq_matrix m, typename store_as<DT>::type* __restrict__ out,
-                                                               int64_t ld_out, int r0, int r1, int raw, int vec_out) {
+// Matrices with column orders: scattering 2-byte values straight to HBM costs 4x the plain decode, so a workgroup decodes RB rows
+// into LDS at their permuted positions (ds_write of one element each) and then writes them out in 16-byte pieces.
+// What bounds it is L2: a gathered codeword moves 64 bytes, the order 32 per chunk of eight, 13.5 TB/s reach the CUs.  The rows of a
+// workgroup are neighbours in the file's row_order (rows sorted by order), so a thread reads the positions of its chunk once for
+// all of them and again only where the order changes.
+// Stacked pieces share a launch, with the fp16 copy of a bf16 activation matrix behind them: 5120, 1024 and 1024 rows of 5120 with
+// 16-bit tags and the copy of 1024 activation rows take 35 us; in a launch each 25 + 9 + 9 + 13.
+struct OrdersArgs {
+    sq_matrix m[GEMM256_PIECES];
+    void* out[GEMM256_PIECES];
+    int wg0[GEMM256_PIECES + 1];             // first workgroup of each piece; behind the last piece's: workgroups of the copy
+    int n, r0, raw, vec_out;                 // r0: first row of the (single) piece that is decoded, its rows end at m.R
+    int64_t ld_out;
+    const uint16_t* x;                       // bf16 [T, C] -> xout fp16 (NULL: no copy)
+    uint16_t* xout;
+    int64_t ldx;
+    int T, C;
+};
+
+template <int DT, int D, int RB>   // D = 8 or 4; RB = 2 or 1
+__global__ __launch_bounds__(512) void dequant_orders_kernel(OrdersArgs a) {
     typedef typename store_as<DT>::type T;
     extern __shared__ __attribute__((aligned(16))) unsigned char row_smem[];
     T* row_lds = reinterpret_cast<T*>(row_smem);
-    const int C = m.C, nch = C / D, tid = threadIdx.x;
-    constexpr int V = 16 / (int)sizeof(T);              // elements per 16-byte store
-    for (int r = r0 + blockIdx.x; r < r1; r += gridDim.x) {
-        const uint32_t* row = reinterpret_cast<const uint32_t*>(m.tags) + (int64_t)r * m.W;
-        const uint32_t boff = m.row_book ? (uint32_t)m.row_book[r] << m.bits : 0u;
-        const float s = raw ? 1.f : h2f(m.row_scale[r]);
-        const int32_t* pm = m.perms + (int64_t)(m.row_mask ? m.row_mask[r] : 0) * C;
-        for (int j = tid; j < nch; j += 256) {
-            const uint32_t tag = tag_at(row, m.W, m.bits, j) + boff;
-            const uint16_t* cw = m.table + (int64_t)tag * D;
-            uint32_t v[D / 2];
-            int32_t p[D];
-            if (D == 8) {
-                const u32x4 t = *reinterpret_cast<const u32x4*>(cw);
-                v[0] = t[0]; v[1] = t[1]; v[2] = t[2]; v[3] = t[3];
-                const u32x4 p0 = *reinterpret_cast<const u32x4*>(pm + j * 8), p1 = *reinterpret_cast<const u32x4*>(pm + j * 8 + 4);
+    const int wg = (int)blockIdx.x, tid = (int)threadIdx.x, nt = (int)blockDim.x;
+    if (wg >= a.wg0[a.n]) {
+        const int64_t total = (int64_t)a.T * a.C / 8, step = (int64_t)(gridDim.x - a.wg0[a.n]) * nt;
+        for (int64_t i = (int64_t)(wg - a.wg0[a.n]) * nt + tid; i < total; i += step) {
+            const int t = (int)(i * 8 / a.C), c = (int)(i * 8 - (int64_t)t * a.C);
+            u32x4 v = *reinterpret_cast<const u32x4*>(a.x + (int64_t)t * a.ldx + c);
+            v.x = bf2h_x2(v.x); v.y = bf2h_x2(v.y); v.z = bf2h_x2(v.z); v.w = bf2h_x2(v.w);
+            *reinterpret_cast<u32x4*>(a.xout + i * 8) = v;
+        }
+        return;
+    }
+    int pi = 0;
 #pragma unroll
-                for (int k = 0; k < 4; ++k) { p[k] = (int32_t)p0[k]; p[4 + k] = (int32_t)p1[k]; }
+    for (int i = 1; i < GEMM256_PIECES; ++i) pi += i < a.n && wg >= a.wg0[i];
+    const sq_matrix& m = a.m[pi];
+    const int C = m.C, nch = C / D, k0 = a.r0 + (wg - a.wg0[pi]) * RB, cnt = min(RB, m.R - k0);
+    int r[RB], mask[RB];
+    uint32_t boff[RB];
+    float sc[RB];
+#pragma unroll
+    for (int q = 0; q < RB; ++q) {
+        const int k = k0 + min(q, cnt - 1);
+        r[q] = m.row_order ? m.row_order[k] : k;
+        mask[q] = m.row_mask ? m.row_mask[r[q]] : 0;
+        boff[q] = m.row_book ? (uint32_t)m.row_book[r[q]] << m.bits : 0u;
+        sc[q] = a.raw ? 1.f : h2f(m.row_scale[r[q]]);
+    }
+    constexpr int V = 16 / (int)sizeof(T);                      // elements per 16-byte store
+    for (int j = tid; j < nch; j += nt) {
+        uint32_t tag[RB], v[RB][D / 2];
+        int32_t p[D];
+        auto order = [&](int q) {
+            const int32_t* pm = m.perms + (int64_t)mask[q] * C + j * D;
+#pragma unroll
+            for (int h = 0; h < D / 4; ++h) {
+                const u32x4 t = *reinterpret_cast<const u32x4*>(pm + h * 4);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) p[h * 4 + k] = (int32_t)t[k];
+            }
+        };
+#pragma unroll
+        for (int q = 0; q < RB; ++q)
+            tag[q] = tag_at(reinterpret_cast<const uint32_t*>(m.tags) + (int64_t)r[q] * m.W, m.W, m.bits, j) + boff[q];
+        order(0);
+#pragma unroll
+        for (int q = 0; q < RB; ++q) {
+            const uint16_t* cw = m.table + (int64_t)tag[q] * D;
+            if constexpr (D == 8) {
+                const u32x4 t = *reinterpret_cast<const u32x4*>(cw);
+                v[q][0] = t[0]; v[q][1] = t[1]; v[q][2] = t[2]; v[q][3] = t[3];
             } else {
                 const u32x2 t = *reinterpret_cast<const u32x2*>(cw);
-                v[0] = t[0]; v[1] = t[1];
-                const u32x4 p0 = *reinterpret_cast<const u32x4*>(pm + j * 4);
-#pragma unroll
-                for (int k = 0; k < 4; ++k) p[k] = (int32_t)p0[k];
+                v[q][0] = t[0]; v[q][1] = t[1];
             }
+        }
+#pragma unroll
+        for (int q = 0; q < RB; ++q) {
+            if (q && mask[q] != mask[q - 1]) order(q);
+            T* row = row_lds + (size_t)q * C;
 #pragma unroll
             for (int k = 0; k < D / 2; ++k) {
-                row_lds[p[2 * k]] = store_as<DT>::cvt(h2f((uint16_t)(v[k] & 0xFFFFu)) * s);
-                row_lds[p[2 * k + 1]] = store_as<DT>::cvt(h2f((uint16_t)(v[k] >> 16)) * s);
+                row[p[2 * k]] = store_as<DT>::cvt(h2f((uint16_t)(v[q][k] & 0xFFFFu)) * sc[q]);
+                row[p[2 * k + 1]] = store_as<DT>::cvt(h2f((uint16_t)(v[q][k] >> 16)) * sc[q]);
             }
         }
-        __syncthreads();
-        T* o = out + (int64_t)(r - r0) * ld_out;
-        if (vec_out) {
-            for (int c = tid * V; c < C; c += 256 * V)
-                *reinterpret_cast<u32x4*>(o + c) = *reinterpret_cast<const u32x4*>(row_lds + c);
-        } else {
-            for (int c = tid; c < C; c += 256) o[c] = row_lds[c];
-        }
-        __syncthreads();
     }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < RB; ++q) {
+        if (q >= cnt) break;
+        T* o = reinterpret_cast<T*>(a.out[pi]) + (int64_t)(r[q] - a.r0) * a.ld_out;
+        const T* row = row_lds + (size_t)q * C;
+        if (a.vec_out) {
+            for (int c = tid * V; c < C; c += nt * V) *reinterpret_cast<u32x4*>(o + c) = *reinterpret_cast<const u32x4*>(row + c);
+        } else {
+            for (int c = tid; c < C; c += nt) o[c] = row[c];
+        }
+    }
+}
+
+static bool orders_ok(const sq_matrix& m, size_t esize) {
+    return m.tags && m.perms && (m.d == 8 || m.d == 4) && (size_t)m.C * esize <= 65536 && ((uintptr_t)m.perms & 15) == 0 &&
+           ((uintptr_t)m.table & 15) == 0 && m.C % 4 == 0;
+}
+
+// a.m (one d, one C), a.out, a.n, a.r0, a.raw, a.ld_out, a.vec_out and the copy are set.
+// Two rows per workgroup where they are short and many (us with two rows, with one; 16-bit tags and output): 7168 x 5120 31.6, 33.3;
+// 2048 x 5120 12.3, 13.1; 512 x 5120 5.9, 5.3 (two workgroups on a CU hide less); 4096 x 8192 29.4, 29.8; 4096 x 12288 43.5, 42.2;
+// 3584 x 18944 75, 60 (two workgroups' LDS fill a CU); and with rows in no order 35.8, 35.6 at 4096 x 10240.  Four rows: 33.3 at 7168 x 5120.
+template <int DT>
+static int launch_orders(OrdersArgs& a, hipStream_t s) {
+    const int C = a.m[0].C, nch = C / a.m[0].d;
+    const size_t row_bytes = (size_t)C * sizeof(typename store_as<DT>::type);
+    // threads: as few rounds of at most 320 as the chunks need, all rounds nearly full
+    const int rounds = (nch + 319) / 320, nt = std::max(64, ((nch + rounds - 1) / rounds + 63) & ~63);
+    int64_t rows = 0, wg = 0;
+    for (int i = 0; i < a.n; ++i) rows += a.m[i].R - a.r0;
+    const int rb = a.m[0].row_order && row_bytes <= 16384 && rows >= 8 * device_cus() ? 2 : 1;
+    for (int i = 0; i < a.n; ++i) {
+        a.wg0[i] = (int)wg;
+        wg += (a.m[i].R - a.r0 + rb - 1) / rb;
+    }
+    for (int i = a.n; i <= GEMM256_PIECES; ++i) a.wg0[i] = (int)wg;
+    if (a.x) wg += std::min<int64_t>(device_cus() * 4, ((int64_t)a.T * a.C / 8 + nt - 1) / nt);
+    if (wg >= ((int64_t)1 << 31)) return fail(SQ_EINVAL, "sq_dequant: %lld workgroups", (long long)wg);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((unsigned)wg), dim3((unsigned)nt), row_bytes * rb, s, a); };
+    if (a.m[0].d == 8) { if (rb > 1) go(dequant_orders_kernel<DT, 8, 2>); else go(dequant_orders_kernel<DT, 8, 1>); }
+    else { if (rb > 1) go(dequant_orders_kernel<DT, 4, 2>); else go(dequant_orders_kernel<DT, 4, 1>); }
+    return check_launch("sq_dequant");
 }
 
 static bool dequant8x4_ok(const sq_matrix& m, int64_t n) {
@@ -338,17 +421,13 @@ static int launch_dt(const sq_matrix& m, void* out, int64_t ld_out, int r0, int 
     typedef typename store_as<DT>::type T;
     const int64_t n = (int64_t)(r1 - r0) * (m.C / m.d);
     if (n == 0) return SQ_OK;
-    const size_t row_bytes = (size_t)m.C * sizeof(T);
-    if (m.perms && (m.d == 8 || m.d == 4) && row_bytes <= 65536 && ((uintptr_t)m.perms & 15) == 0 && ((uintptr_t)m.table & 15) == 0 &&
-        m.C % 4 == 0) {
+    if (orders_ok(m, sizeof(T))) {
         constexpr int V = 16 / (int)sizeof(T);
-        const int vec_out = ((uintptr_t)out & 15) == 0 && ld_out % V == 0 && m.C % V == 0;
-        const int per_cu = (int)(131072 / row_bytes) < 8 ? (int)(131072 / row_bytes) : 8;       // workgroups that share a CU's LDS
-        const int want = device_cus() * (per_cu < 1 ? 1 : per_cu);
-        const unsigned rgrid = (unsigned)(r1 - r0 < want ? r1 - r0 : want);
-        if (m.d == 8) hipLaunchKernelGGL((dequant_rows_lds_kernel<DT, 8>), dim3(rgrid), dim3(256), row_bytes, s, m, (T*)out, ld_out, r0, r1, raw, vec_out);
-        else hipLaunchKernelGGL((dequant_rows_lds_kernel<DT, 4>), dim3(rgrid), dim3(256), row_bytes, s, m, (T*)out, ld_out, r0, r1, raw, vec_out);
-        return check_launch("sq_dequant");
+        OrdersArgs a{};
+        a.m[0] = m; a.m[0].R = r1; a.out[0] = out; a.n = 1; a.r0 = r0; a.raw = raw; a.ld_out = ld_out;
+        if (r0 > 0 || r1 < m.R) a.m[0].row_order = nullptr;     // part of the rows: taken as they lie
+        a.vec_out = ((uintptr_t)out & 15) == 0 && ld_out % V == 0 && m.C % V == 0;
+        return launch_orders<DT>(a, s);
     }
     if (dequant8x4_ok(m, n)) {
         const int vec = sizeof(T) == 2 && ((uintptr_t)out & 15) == 0 && ld_out % 8 == 0;
@@ -381,19 +460,30 @@ int launch_dequant_with_cvt(const sq_matrix& m, void* out, int64_t ld_out, const
     return check_launch("sq_linear_gemm(decode + fp16 copy)");
 }
 
-// Raw fp16 decode of up to GEMM256_PIECES pieces, one behind the other at out (rows of C elements), with the fp16 copy of x
-// as above (x NULL: none).  Returns 1 without launching anything when a piece does not take the LDS kernel.
-int launch_dequant_stack(const sq_matrix* mats, int n, void* out, const uint16_t* x, int64_t ldx, int T, int C, uint16_t* xout, hipStream_t s) {
-    if (n < 1 || n > GEMM256_PIECES) return 1;
-    Dequant4Args a{};
-    uint16_t* o = (uint16_t*)out;
-    for (int i = 0; i < n; ++i) {
-        if (mats[i].R <= 0 || !dequant4_ok(mats[i], o, C, 2)) return 1;
-        a.m[i] = mats[i];
-        a.out[i] = o;
-        o += (size_t)mats[i].R * C;
+// fp16 decode (raw: without the row scales) of up to GEMM256_PIECES pieces, one behind the other at out (rows of C elements), with
+// the fp16 copy of x as above (x NULL: none).  Returns 1 without launching anything when the pieces do not all take one of the two
+// LDS kernels.
+int launch_dequant_stack(const sq_matrix* mats, int n, void* out, int raw, const uint16_t* x, int64_t ldx, int T, int C, uint16_t* xout, hipStream_t s) {
+    if (n < 1 || n > GEMM256_PIECES || ((uintptr_t)out & 15) || C % 8) return 1;
+    auto fill = [&](auto& a, auto ok) -> bool {
+        uint16_t* o = (uint16_t*)out;
+        for (int i = 0; i < n; ++i) {
+            if (mats[i].R <= 0 || !ok(mats[i], o)) return false;
+            a.m[i] = mats[i];
+            a.out[i] = o;
+            o += (size_t)mats[i].R * C;
+        }
+        a.n = n; a.raw = raw; a.ld_out = C; a.x = x; a.xout = xout; a.ldx = ldx; a.T = T; a.C = C;
+        return true;
+    };
+    if (mats[0].perms) {
+        OrdersArgs a{};
+        if (!fill(a, [&](const sq_matrix& m, uint16_t*) { return orders_ok(m, 2) && m.d == mats[0].d; })) return 1;
+        a.vec_out = 1;
+        return launch_orders<SQ_F16>(a, s);
     }
-    a.n = n; a.raw = 1; a.ld_out = C; a.x = x; a.xout = xout; a.ldx = ldx; a.T = T; a.C = C;
+    Dequant4Args a{};
+    if (!fill(a, [&](const sq_matrix& m, uint16_t* o) { return dequant4_ok(m, o, C, 2); })) return 1;
     return launch_dequant4<SQ_F16>(a, s);
 }
 

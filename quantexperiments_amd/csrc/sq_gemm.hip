@@ -149,8 +149,6 @@ bool gemm256_ok(int C, int64_t ldx, int64_t ldw, const void* x, const void* w);
 size_t gemm256_part_bytes(int T, int R, int C, int cus);
 int launch_gemm256(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ldw, const Gemm256Scales& sc, void* y,
                    int y_dtype, int64_t ldy, int y_off, int T, int R, int C, float* part, int cus, hipStream_t s);
-int launch_bf16_to_f16(const uint16_t* x, int64_t ldx, int T, int C, uint16_t* out, hipStream_t s);
-int launch_dequant_stack(const sq_matrix* mats, int n, void* out, const uint16_t* x, int64_t ldx, int T, int C, uint16_t* xout, hipStream_t s);
 int launch_dequant_with_cvt(const sq_matrix& m, void* out, int64_t ld_out, const uint16_t* x, int64_t ldx, int T, int C,
                             uint16_t* xout, hipStream_t s);
 
@@ -435,7 +433,7 @@ int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_
             ldxh = C;
         }
         auto decode_stack = [&](const sq_matrix* ms, int k, void* w) -> int {
-            const int rc = launch_dequant_stack(ms, k, w, copy_pending ? (const uint16_t*)x : nullptr, ldx, T, C, (uint16_t*)ws, s);
+            const int rc = launch_dequant_stack(ms, k, w, 1, copy_pending ? (const uint16_t*)x : nullptr, ldx, T, C, (uint16_t*)ws, s);
             if (rc == 0) copy_pending = false;
             return rc;
         };

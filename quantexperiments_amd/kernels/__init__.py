@@ -453,6 +453,23 @@ def _prep(pieces, x: torch.Tensor, y: torch.Tensor):
         y.stride(0) if y.shape[0] > 1 else max(y.stride(0), y.shape[1])
 
 
+def dequant_stack(pieces, out: torch.Tensor, x: torch.Tensor | None = None) -> torch.Tensor | None:
+    """fp16 weights of all pieces one below the other into out [sum R, C] (sq_dequant_stack) and, in the same launches, the fp16
+    copy of x (bf16 [B, C], rows of whole 16-byte pieces), which is returned."""
+    dev, C = out.device, pieces[0].C
+    if out.dtype != torch.float16 or not out.is_contiguous() or out.shape != (sum(p.R for p in pieces), C):
+        raise ValueError(f"out must be contiguous fp16 [sum of the pieces' rows, {C}]")
+    if x is not None and (x.dtype != torch.bfloat16 or x.dim() != 2 or x.shape[1] != C or x.stride(1) != 1):
+        raise ValueError(f"x must be bf16 [B, {C}] with unit column stride")
+    xh = None if x is None else torch.empty(x.shape, dtype=torch.float16, device=dev)
+    mats = _lib.matrix_array([p.descriptor() for p in pieces])
+    with torch.cuda.device(dev):
+        _lib.check(_lib.lib().sq_dequant_stack(mats, len(pieces), out.data_ptr(), None if x is None else x.data_ptr(),
+                                               0 if x is None else x.stride(0) if x.shape[0] > 1 else C, 0 if x is None else x.shape[0],
+                                               None if x is None else xh.data_ptr(), _lib.stream_ptr(dev)))
+    return xh
+
+
 def linear_small(pieces, x: torch.Tensor, y: torch.Tensor) -> torch.Tensor:
     """Y[b, off_i + r] for every stacked piece, B = x.shape[0] <= 32 (sq_linear_small)."""
     rc = _lib.native().linear(pieces, x, y, False)

@@ -24,7 +24,7 @@ import sys
 import torch
 
 from .. import _lib
-from ..kernels import (PackedLinear, _Workspace, gemm_dense, linear_gemm, linear_small, prepare_stack, q4_rows, q8_dense,
+from ..kernels import (PackedLinear, _Workspace, dequant_stack, gemm_dense, linear_gemm, linear_small, prepare_stack, q4_rows, q8_dense,
                        q8_linear)
 
 BMAX = _lib.SMALL_BMAX
@@ -250,18 +250,22 @@ class PackedShards:
             return linear_gemm(self.rls, x, y)
         # dequant + GEMM: whole pieces ("dequant") or row chunks of ~chunk_bytes ("chunked") decoded to
         # fp16 in the shared scratch, each multiplied into its column slice of Y
-        if x.dtype != torch.float16 and M > BMAX and self.C % 64 == 0:
-            x = x.to(torch.float16)                     # fp16 x fp16 takes the 256 x 256 tile kernel; y keeps its dtype
+        to_fp16 = x.dtype != torch.float16 and M > BMAX and self.C % 64 == 0    # fp16 x fp16 takes the tile kernel; y keeps its dtype
         if self.large == "dequant":
+            copy = to_fp16 and x.dtype == torch.bfloat16 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
+            if to_fp16 and not copy:
+                x = x.to(torch.float16)
             # one product over pieces that fit together: a 1024-row k or v projection alone is a few tiles on an idle chip
             groups = self.joint[M > JOINT_ROWS]
             scratch = _Workspace.get(max(R for _, _, R in groups) * self.C * 2, x.device, kind="dense").view(torch.float16)
             for i, j, R in groups:
                 at, w = self.offs[i], scratch[:R * self.C].view(R, self.C)
-                for rl, off in zip(self.rls[i:j], self.offs[i:j]):
-                    rl.dense(torch.float16, out=w[off - at:off - at + rl.R])
+                xh = dequant_stack(self.rls[i:j], w, x if copy else None)   # the copy rides along with the first pieces
+                x, copy = x if xh is None else xh, False
                 gemm_dense(w, x, y if R == self.R else y[:, at:at + R])
             return y
+        if to_fp16:
+            x = x.to(torch.float16)
         rows = max(self.Rs)
         if self.large == "chunked":
             rows = min(rows, max(128, (self.chunk_bytes // (2 * self.C)) // 128 * 128))
