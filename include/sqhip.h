@@ -372,8 +372,9 @@ int sq_linear_small_from(const sq_matrix* mats, int32_t n_mats, const sq_produce
  * here every row is finished where its sums meet.  `from` (NULL, or mode SQ_FROM_ADDNORM as in sq_linear_small_from,
  * one activation row; x and ldx are then ignored and from->x_out is the row the launch computes and reads) lets the
  * same launch produce its own input too.  For pieces on the tag-stream kernel without column orders whose streams are
- * cut into the same runs (sq_stream_build with the same `runs`), 1 to 8 activation rows; any other stack returns
- * SQ_EUNSUPPORTED and the caller makes the two calls.  Needs the workspace of sq_linear_small (its header). */
+ * cut into the same runs (sq_stream_build with the same `runs`), 1 to 8 activation rows, and for pieces of one format on
+ * the matrix-core kernel (d = 4) whose two sets of codebooks fit LDS together, 2 rows or more (16-byte aligned x with ldx % 8 == 0, out
+ * not overlapping x, no `from`); any other stack returns SQ_EUNSUPPORTED and the caller makes the two calls.  Needs the workspace of sq_linear_small (tag-stream pieces: its header). */
 int sq_linear_small_silu(const sq_matrix* mats, int32_t n_mats, const sq_producer* from, const void* x, int dtype, int64_t ldx,
                          void* out, int64_t ld_out, int32_t B, void* workspace, size_t ws_bytes, void* stream);
 

@@ -132,6 +132,11 @@ struct MmaPlan { int RW, NT, KW, ks; };
 
 bool mma_shape(const sq_matrix& m) { return fast_shape(m) && !m.perms; }
 
+// the tile-major copy of a piece's tags, NULL if it has none
+static const uint32_t* tiled_piece(const sq_matrix& m) {
+    return m.stream && !m.perms && tiled_format_ok(m.R, m.W, m.C, m.d, m.bits) && ((uintptr_t)m.stream & 15) == 0 ? (const uint32_t*)m.stream : nullptr;
+}
+
 // bytes of codebook the matrix-core kernel stages in LDS (0: gathers go through the cache)
 static size_t mma_table_bytes(const sq_matrix& m) {
     const size_t tab = (size_t)m.G * ((size_t)1 << m.bits) * m.d * 2;
@@ -205,9 +210,28 @@ bool small_uses_sums(const sq_matrix* mats, int n) {
     return false;
 }
 
-// Pieces [0, cnt) share format and row length: one persistent launch (+ one reduction per piece if ks > 1).
+// SiLU(gate) * up written by the matrix-core kernel: the two pieces' codebooks (one format, one shape) fit LDS side by side next to the
+// accumulators of a group of tiles, the rows are not split over workgroups (same plan, so the same sums, as without), and the product
+// by itself would run on this kernel: two activation rows or more.  us, the two launches / this one, 8 rows: 2 x 18944 x 3584 with 12-bit tags
+// 20.4 / 17.6, 8-bit 18.7 / 15.2; 17408 x 5120, 12-bit 28.7 / 25.0, 10-bit in 4 books 26.3 / 24.0; 8960 x 1536, 12-bit 11.8 / 10.1;
+// 1024 x 512, 8-bit 7.6 / 6.6.  But 4864 x 896 (two waves a workgroup) with 64 KB of codebooks 11.7 / 12.0, with 128 KB 13.7 / 17.5: a
+// workgroup's waves fetch the codebooks, at most 24 KB each here.
+static bool mma_fuses_silu(const sq_matrix* mats, int n, int B, const void* x, int64_t ldx) {
+    if (n != 2 || B < 2 || B > SQ_SMALL_BMAX || ldx % 8 || ((uintptr_t)x & 15)) return false;
+    const sq_matrix &g = mats[0], &u = mats[1];
+    if (g.d != 4 || !mma_shape(g) || !mma_shape(u) || g.R <= 0 || g.R != u.R || g.bits != u.bits || g.d != u.d || g.W != u.W || g.G != u.G) return false;
+    if (small_takes_gemm_route(mats, n, B, x, ldx) || tiled_piece(g) == nullptr != (tiled_piece(u) == nullptr)) return false;
+    const size_t tab = mma_table_bytes(g);
+    if (tab == 0 || tab > 64 * 1024) return false;               // (beyond 64 KB two rows take the row-segment kernel)
+    const MmaPlan pl = mma_plan(g, B);
+    const int tpu = unit_dwords(g.bits) * 32 / g.bits;
+    return pl.ks == 1 && 2 * tab <= (size_t)pl.KW * 24 * 1024 && 2 * tab + 16 + std::max((size_t)pl.KW * mma_x_stage_bytes(tpu * g.d), (size_t)mma_group(pl.RW, true) * pl.KW * 64 * pl.NT * 16) <= 160 * 1024;
+}
+
+// Pieces [0, cnt) share format and row length: one persistent launch (+ one reduction per piece if ks > 1).  act: mma_fuses_silu
+// holds for them.
 static int launch_mma_group(const sq_matrix* mats, int cnt, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype,
-                            int64_t ldy, int B, char* ws, size_t& ws_off, int cus, hipStream_t s) {
+                            int64_t ldy, int B, char* ws, size_t& ws_off, int cus, hipStream_t s, bool act = false) {
     const sq_matrix& m0 = mats[0];
     const MmaPlan pl = mma_plan(m0, B);
     MmaArgs a;
@@ -215,12 +239,14 @@ static int launch_mma_group(const sq_matrix* mats, int cnt, const void* x, int x
     a.x = (const uint16_t*)x; a.ldx = ldx; a.y = y; a.ldy = ldy; a.B = B; a.x_dtype = x_dtype; a.y_dtype = y_dtype;
     a.U = m0.W / unit_dwords(m0.bits);
     a.ks = pl.ks;
-    a.table_bytes = (int)mma_table_bytes(m0);
+    a.act = act;
+    const int per = act ? 2 : 1;                                 // pieces whose tiles a workgroup walks in turn
+    a.table_bytes = (int)mma_table_bytes(m0) * per;
     const int threads = pl.KW * 64;
     // LDS behind the codebook: the waves' accumulators of the tiles between two barriers (MMA_TT tiles when the codebook
     // is read through the cache; with the codebook in LDS as many as the workgroup walks, if they fit: sized below)
     const size_t red_tile = (size_t)pl.KW * 64 * pl.NT * 16;
-    const int pft = mma_pft(pl.RW);
+    const int pft = mma_group(pl.RW, act);
     a.tg = a.table_bytes ? pft : 0;
     const int tpu = unit_dwords(m0.bits) * 32 / m0.bits;
     const size_t xstage = (size_t)pl.KW * mma_x_stage_bytes(tpu * m0.d);      // the waves' activation staging areas (same LDS)
@@ -241,27 +267,27 @@ static int launch_mma_group(const sq_matrix* mats, int cnt, const void* x, int x
         MmaPiece& P = a.p[k];
         P.m = mats[k];
         const sq_matrix& mk = mats[k];
-        P.tiled = mk.stream && !mk.perms && tiled_format_ok(mk.R, mk.W, mk.C, mk.d, mk.bits) && ((uintptr_t)mk.stream & 15) == 0
-                      ? (const uint32_t*)mk.stream : nullptr;
+        P.tiled = tiled_piece(mk);
         P.part = nullptr;
         if (pl.ks > 1) {
             P.part = (float*)(ws + ws_off);
             ws_off += mma_part_bytes(mats[k], B);
         }
         const int ntiles = (mats[k].R + 15) / 16;
-        int nshare = (int)((mats[k].R * (int64_t)slots / rows_total) / pl.ks);
+        int nshare = (int)((mats[k].R * per * (int64_t)slots / rows_total) / pl.ks);
         if (nshare > ntiles) nshare = ntiles;
         if (nshare < 1) nshare = 1;
         P.wg_begin = wg;
         P.wg_count = nshare * pl.ks;
-        wg += P.wg_count;
+        if (!act || k) wg += P.wg_count;
     }
+    if (act) a.n = 1;                                            // (every workgroup begins with piece 0)
     for (int k = cnt; k < GEMV_MAX_PIECES; ++k) a.p[k] = a.p[0];
     if (a.table_bytes) {
         int most = 1;                                            // most tiles one workgroup walks
         for (int k = 0; k < cnt; ++k) {
             const int ntiles = (mats[k].R + 15) / 16, nshare = a.p[k].wg_count / pl.ks;
-            most = std::max(most, (ntiles + nshare - 1) / nshare);
+            most = std::max(most, (ntiles + nshare - 1) / nshare * per);
         }
         const size_t room = (size_t)(160 * 1024) / rc - a.table_bytes - 16;
         int fit = (int)(room / red_tile) / pft * pft;
@@ -314,6 +340,11 @@ bool small_fuses_silu(const sq_matrix* mats, int n, int B) {
 int launch_small_silu(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* act, int64_t ld_act, int B,
                       void* sums, hipStream_t s, const sq_producer* from) {
     const bool x_ok = (B == 1 || ldx % 8 == 0) && (((uintptr_t)x & 15) == 0);
+    const char *xb = (const char*)x, *xe = xb + ((int64_t)(B - 1) * ldx + mats[0].C) * 2, *ob = (const char*)act, *oe = ob + ((int64_t)(B - 1) * ld_act + mats[0].R) * 2;
+    if (!from && mma_fuses_silu(mats, n, B, x, ldx) && (oe <= xb || xe <= ob)) {     // (act written over x: the two launches)
+        size_t off = 0;
+        return launch_mma_group(mats, 2, x, x_dtype, ldx, act, x_dtype, ld_act, B, nullptr, off, device_cus(), s, true);
+    }
     if (!small_fuses_silu(mats, n, B) || !(x_ok || from) || (from && !small_fuses_producer(mats, n, B)))
         return fail(SQ_EUNSUPPORTED, "sq_linear_small_silu: no fused kernel for this stack (run sq_linear_small, then sq_silu_mul)");
     if (!sums) return fail(SQ_EWORKSPACE, "sq_linear_small_silu: these pieces need a workspace (its header holds their partial sums)");

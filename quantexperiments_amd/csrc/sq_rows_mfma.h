@@ -48,13 +48,15 @@ struct MmaArgs {
     int U;                // lane units per row
     int ks;               // workgroup-level column slices
     int table_bytes;      // bytes of codebook staged in LDS (0 = read through cache)
-    int tg;               // codebook in LDS: 16-row tiles whose accumulators LDS holds between two barriers (a multiple of mma_pft(RW))
+    int tg;               // codebook in LDS: 16-row tiles whose accumulators LDS holds between two barriers (a multiple of mma_group())
+    int act;              // 1: the two pieces are a gate and an up projection, y receives SiLU(gate) * up (16-bit)
 };
 
 constexpr int MMA_TT = 4;     // 16-row tiles multiplied between two workgroup barriers (codebook read through the cache)
 // codebook in LDS: tiles of tags in flight per lane (fewer when a lane's part of a tile is long: registers)
 // (2 to 5 tiles in flight measure alike on the 7B shapes)
 constexpr int mma_pft(int RW) { return RW >= 8 ? 2 : 3; }
+constexpr int mma_group(int RW, bool act) { return act && mma_pft(RW) % 2 ? 2 * mma_pft(RW) : mma_pft(RW); }     // ACT: whole pairs
 // LDS per wave in which a round's activations (16 tokens x 4 lane units of UK columns, fp16) pass from whole-line loads
 // to the lanes that use them; it lies where the accumulators are added afterwards
 constexpr int mma_x_stage_bytes(int UK) { return 16 * (4 * UK * 2 + 16); }
@@ -88,7 +90,11 @@ __device__ __forceinline__ uint32_t bf2h_pk(uint32_t v) { return bf2h_x2(v); }
 // codebook in LDS, which fit four waves per SIMD; 8 otherwise.
 constexpr int mma_waves_max(int x_operands, bool lds_tab) { return lds_tab && x_operands <= 8 ? 16 : 8; }
 
-template <int BITS, int D, int RW, int NT, bool LDS_TAB>
+// ACT (codebooks in LDS): p[0] is a gate and p[1] an up projection of one shape, both codebooks are staged, a workgroup walks the
+// two pieces' tiles in turn (virtual tile i: tile i / 2 of piece i % 2), and the wave that adds up a pair of tiles writes SiLU(gate) * up,
+// with the same roundings as the product followed by silu_mul_kernel.  It saves that launch and the trip of gate and up through memory
+// (2 x 18944 x 3584, 12-bit tags, 8 rows: 20.4 us, now 17.6).
+template <int BITS, int D, int RW, int NT, bool LDS_TAB, bool ACT = false>
 __global__ __launch_bounds__(64 * mma_waves_max(RW * ((unit_of<BITS>::UD * 32 / BITS) / (8 / D)) * NT, LDS_TAB))
 void rows_mfma_kernel(MmaArgs a) {
     constexpr int UD = unit_of<BITS>::UD;
@@ -187,6 +193,8 @@ void rows_mfma_kernel(MmaArgs a) {
     constexpr int XROW = XRB + 16;                           // a token's row in the staging area (the 16 tokens' reads spread over the banks)
     constexpr int XTPI = 1024 / XRB;                         // tokens per load instruction
     static_assert(16 / XTPI == SPU, "a round's activations are SPU loads per token tile");
+    constexpr int F = ACT ? 2 : 1;                           // pieces whose tiles a workgroup walks
+    const MmaPiece& P1 = a.p[F - 1];
     unsigned char* xst = smem + a.table_bytes + 16 + wave * mma_x_stage_bytes(UK);
     const int xtl = lane / (XRB / 16), xob = (lane % (XRB / 16)) * 16;    // this lane's token (within an instruction) and byte in the round
     u32x4 xraw[RW][NT][SPU];
@@ -201,28 +209,32 @@ void rows_mfma_kernel(MmaArgs a) {
                 col = col < m.C ? col : m.C - 8;             // (columns past the row's end: any valid address, the operand is zeroed)
                 xraw[n][nt][j] = *reinterpret_cast<const u32x4*>(a.x + (int64_t)(tok < a.B ? tok : a.B - 1) * a.ldx + col);
             }
-    fetch(t0 < t1 ? t0 : ntiles - 1, tA, sc[0]);             // (no branch around the loads; a workgroup without tiles reads the last one)
+    if constexpr (!ACT) fetch(t0 < t1 ? t0 : ntiles - 1, tA, sc[0]);     // (no branch around the loads; a workgroup without tiles reads the last one)
     // (codebook in LDS: the tags of the first tiles in flight, without a branch around the loads so that the waits count
     // them exactly: the two layouts differ in a base and a stride, chosen once)
     constexpr int PFT = LDS_TAB ? mma_pft(RW) : 1;
     const bool til = P.tiled != nullptr;
     const uint32_t* fbase = til ? P.tiled + li * UD : tags;
+    const uint32_t* fbase1 = ACT ? (til ? P1.tiled + li * UD : reinterpret_cast<const uint32_t*>(P1.m.tags)) : fbase;
+    const uint8_t* bkp1 = !ACT ? bkp : P1.m.row_book ? P1.m.row_book : reinterpret_cast<const uint8_t*>(P1.m.row_scale);
     uint32_t fo[RW];
 #pragma unroll
     for (int n = 0; n < RW; ++n) fo[n] = til ? uoff[n] * 16u : uoff[n];
-    auto fetch_tags = [&](int t, Tile& T) {
-        const int row0 = t << 4;
+    auto fetch_tags = [&](int i, Tile& T) {
+        const int t = i / F, row0 = t << 4;
         const int r = row0 + li < m.R ? row0 + li : m.R - 1;
-        const uint32_t* bp = fbase + (til ? (size_t)t * a.U * 16 * UD : (size_t)r * m.W);
-        T.book = bkp[r];                                  // (first: loads return in order, the tags' waits then cover it)
+        const bool second = ACT && (i & 1);
+        const uint32_t* bp = (second ? fbase1 : fbase) + (til ? (size_t)t * a.U * 16 * UD : (size_t)r * m.W);
+        T.book = (second ? bkp1 : bkp)[r];                                  // (first: loads return in order, the tags' waits then cover it)
 #pragma unroll
         for (int n = 0; n < RW; ++n) T.t[n] = load_unit<UD>(bp + fo[n]);
     };
     Tile ring[PFT];
+    const int i0 = t0 * F, i1 = t1 * F;                      // this workgroup's (virtual) tiles
     if constexpr (LDS_TAB) {
-        ring[0] = tA;
+        if constexpr (!ACT) ring[0] = tA;
 #pragma unroll
-        for (int q = 1; q < PFT; ++q) fetch_tags(min(t0 + q, max(t1 - 1, t0)), ring[q]);
+        for (int q = ACT ? 0 : 1; q < PFT; ++q) fetch_tags(min(i0 + q, max(i1 - 1, i0)), ring[q]);
     }
     // the B operands: this wave's activations as fp16, in registers for the whole kernel
     half8v xb[RW][SPU][NT];
@@ -255,8 +267,12 @@ void rows_mfma_kernel(MmaArgs a) {
     if (table_dma) {
         typedef const __attribute__((address_space(1))) void* gptr_t;
         typedef __attribute__((address_space(3))) void* lptr_t;
-        for (int c = wave; c < (a.table_bytes >> 10); c += KW)
-            __builtin_amdgcn_global_load_lds((gptr_t)(table + (size_t)c * 1024 + lane * 16), (lptr_t)(smem + c * 1024), 16, 0, 0);
+        const int half = a.table_bytes >> 11;
+        for (int c = wave; c < (a.table_bytes >> 10); c += KW) {
+            const unsigned char* from = table + (size_t)c * 1024;
+            if (ACT && c >= half) from = reinterpret_cast<const unsigned char*>(P1.m.table) + (size_t)(c - half) * 1024;
+            __builtin_amdgcn_global_load_lds((gptr_t)(from + lane * 16), (lptr_t)(smem + c * 1024), 16, 0, 0);
+        }
     } else if (LDS_TAB) {
         stage_table(m.table, a.table_bytes, smem);
     }
@@ -270,14 +286,15 @@ void rows_mfma_kernel(MmaArgs a) {
     // One tile: NS = RW * SPU matrix instructions.  The codeword gathers run PD instructions ahead of the
     // matrix instruction that consumes them, so LDS latency overlaps the multiplies of earlier steps.
     constexpr int NS = RW * SPU, PD = NS < 6 ? NS : 6;
-    auto multiply = [&](const Tile& cur, float4v (&acc)[NT]) {
+    // (tab: byte offset of the piece's codebooks in LDS)
+    auto multiply = [&](const Tile& cur, float4v (&acc)[NT], uint32_t tab = 0) {
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) acc[nt] = float4v{0.f, 0.f, 0.f, 0.f};
         u32x4 av[NS];
         auto gather = [&](int k) {
             const int n = k / SPU, s = k - n * SPU;
             const bool dead = !all_live && !live[n];
-            const uint32_t bo = ((cur.book & bkmask) << BITS) * ESZ;    // byte offset of the row's codebook
+            const uint32_t bo = ((cur.book & bkmask) << BITS) * ESZ + tab;      // byte offset of the row's codebook
             if (D == 8) {
                 if (LDS_TAB) {
                     av[k] = *reinterpret_cast<const mma_lds_u32x4*>((uintptr_t)unit_lds_offset<BITS, UD, 4>(cur.t[n], s, bo));
@@ -321,21 +338,22 @@ void rows_mfma_kernel(MmaArgs a) {
         // LDS, and the waves meet once per a.tg tiles (once per launch when the workgroup's tiles all fit), after which
         // each tile is added up by one wave (round robin), scaled and stored.
         if (t0 >= t1) return;                                 // (uniform in the workgroup; the launcher gives every one a tile)
+        auto tab_of = [&](int i) { return ACT && (i & 1) ? (uint32_t)a.table_bytes / 2 : 0u; };
         auto tile_done = [&](int tl, const float4v (&acc)[NT]) {
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) red[((tl * KW + wave) * 64 + lane) * NT + nt] = acc[nt];
         };
-        for (int tg = t0; tg < t1; tg += a.tg) {
-            const int te = min(tg + a.tg, t1);
-            if (tg > t0) __syncthreads();                     // the previous group's sums have been read
+        for (int tg = i0; tg < i1; tg += a.tg) {
+            const int te = min(tg + a.tg, i1);
+            if (tg > i0) __syncthreads();                     // the previous group's sums have been read
             int t = tg;
             for (; t + PFT <= te; t += PFT) {
 #pragma unroll
                 for (int q = 0; q < PFT; ++q) {
                     float4v acc[NT];
-                    multiply(ring[q], acc);
+                    multiply(ring[q], acc, tab_of(t + q));
                     __builtin_amdgcn_sched_barrier(0);
-                    fetch_tags(min(t + q + PFT, t1 - 1), ring[q]);
+                    fetch_tags(min(t + q + PFT, i1 - 1), ring[q]);
                     __builtin_amdgcn_sched_barrier(0);
                     tile_done(t + q - tg, acc);
                 }
@@ -344,10 +362,37 @@ void rows_mfma_kernel(MmaArgs a) {
             for (int q = 0; q < PFT; ++q)
                 if (t + q < te) {                             // (the last group's last tiles: nothing left to fetch)
                     float4v acc[NT];
-                    multiply(ring[q], acc);
+                    multiply(ring[q], acc, tab_of(t + q));
                     tile_done(t + q - tg, acc);
                 }
             __syncthreads();
+            auto sum_of = [&](int tl, int nt) {
+                float4v s4 = red[((tl * KW) * 64 + lane) * NT + nt];
+                for (int k = 1; k < KW; ++k) {
+                    const float4v o = red[((tl * KW + k) * 64 + lane) * NT + nt];
+                    s4.x += o.x; s4.y += o.y; s4.z += o.z; s4.w += o.w;
+                }
+                return s4;
+            };
+            if constexpr (ACT) {
+                for (int tl = 2 * wave; tl < te - tg; tl += 2 * KW) {
+                    const int row0 = ((tg + tl) >> 1) << 4;
+#pragma unroll
+                    for (int nt = 0; nt < NT; ++nt) {
+                        const float4v g4 = sum_of(tl, nt), u4 = sum_of(tl + 1, nt);
+                        const int tok = nt * 16 + li;
+                        if (tok >= a.B) continue;
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) {
+                            const int r = row0 + 4 * lg + v;
+                            if (r >= m.R) continue;
+                            reinterpret_cast<uint16_t*>(a.y)[(int64_t)tok * a.ldy + r] =
+                                silu_mul_one(round16(g4[v] * h2f(m.row_scale[r]), a.y_dtype), round16(u4[v] * h2f(P1.m.row_scale[r]), a.y_dtype), a.y_dtype);
+                        }
+                    }
+                }
+                continue;
+            }
             for (int tl = wave; tl < te - tg; tl += KW) {
                 const int row0 = (tg + tl) << 4;
                 float scl[4];
@@ -358,11 +403,7 @@ void rows_mfma_kernel(MmaArgs a) {
                 }
 #pragma unroll
                 for (int nt = 0; nt < NT; ++nt) {
-                    float4v s4 = red[((tl * KW) * 64 + lane) * NT + nt];
-                    for (int k = 1; k < KW; ++k) {
-                        const float4v o = red[((tl * KW + k) * 64 + lane) * NT + nt];
-                        s4.x += o.x; s4.y += o.y; s4.z += o.z; s4.w += o.w;
-                    }
+                    const float4v s4 = sum_of(tl, nt);
                     const int tok = nt * 16 + li;
                     if (tok >= a.B) continue;
 #pragma unroll
@@ -451,10 +492,12 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
 template <int BITS, int D, int RW, int NT>
 static inline int mma_inst(int op, const MmaArgs& a, int grid, int threads, size_t smem, hipStream_t s) {
     void (*k)(MmaArgs) = a.table_bytes ? rows_mfma_kernel<BITS, D, RW, NT, true> : rows_mfma_kernel<BITS, D, RW, NT, false>;
+    if constexpr (D == 4)
+        if (a.act) k = rows_mfma_kernel<BITS, D, RW, NT, true, true>;
     if (op == 1) {
         static std::mutex mu;
         static std::unordered_map<uint64_t, int> cache;
-        const uint64_t key = ((uint64_t)threads << 40) | ((uint64_t)(a.table_bytes != 0) << 39) | (uint64_t)smem;
+        const uint64_t key = ((uint64_t)threads << 40) | ((uint64_t)(a.table_bytes != 0) << 39) | ((uint64_t)a.act << 38) | (uint64_t)smem;
         std::lock_guard<std::mutex> lock(mu);
         auto it = cache.find(key);
         if (it != cache.end()) return it->second;

@@ -194,10 +194,10 @@ def test_decode_layer_chain_under_graph():
 
 
 # ------------------------------------------------------------------ products that compute their own activations
-def _stack(shapes, bits, M, seed, d=8):
+def _stack(shapes, bits, M, seed, d=8, G=1):
     from quantexperiments_amd.kernels import prepare_stack
     from tests.helpers import synth, to_device
-    ss = [synth(R, C, d, bits, 1, M, seed=seed + i) for i, (R, C) in enumerate(shapes)]
+    ss = [synth(R, C, d, bits, G, M, seed=seed + i) for i, (R, C) in enumerate(shapes)]
     lins = [to_device(s) for s in ss]
     prepare_stack(lins)
     return ss, lins
@@ -300,6 +300,26 @@ def test_linear_small_silu_equals_two_calls(case, dtype):
                                          _lib.stream_ptr(x.device))
     torch.cuda.synchronize()
     assert rc == (0 if fused else _lib.SQ_EUNSUPPORTED)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("R,C,bits,G", [(1, 128, 12, 1), (260, 3584, 12, 1), (5000, 896, 8, 1), (16700, 640, 10, 2), (77, 5120, 8, 8), (40, 18944, 12, 1),
+                                        (33, 512, 12, 2), (50, 2048, 12, 4)])
+def test_silu_on_the_way_out_of_the_matrix_core_kernel(R, C, bits, G, dtype):
+    """Codebooks in LDS: one pair of tiles, many and a ragged last one, several groups of them, one and two activation tiles; rows that
+    are split over workgroups and codebooks that do not fit twice take the two calls.  Bit for bit what the two calls give."""
+    from quantexperiments_amd.kernels import linear_small, linear_small_silu, silu_mul
+    ss, lins = _stack([(R, C), (R, C)], bits, 1, seed=R + C, d=4, G=G)
+    for B in (2, 3, 8, 17, 32):
+        x = rand_x(B, C + 8, dtype, seed=B).cuda()[:, :C]
+        y = torch.empty(B, 2 * R, dtype=dtype, device="cuda")
+        linear_small(lins, x, y)
+        want = torch.empty(B, R, dtype=dtype, device="cuda")
+        silu_mul(y[:, :R], y[:, R:], want)
+        got = torch.full((B, R + 3), 5.0, dtype=dtype, device="cuda")
+        linear_small_silu(lins, x, got[:, :R])
+        assert torch.equal(got[:, :R], want), B
+        assert bool((got[:, R:] == 5.0).all())
 
 
 def test_full_size_gate_up_with_silu_on_the_way_out():
