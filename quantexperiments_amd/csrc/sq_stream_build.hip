@@ -659,7 +659,7 @@ int stream_build_host(const uint32_t* tags, int R, int W, int C, int d, int bits
 // (the rows' order and runs, the groups' places from their step counts); what walks tags or rows runs here: counting, the sort of
 // the rows of a run by entry count, collecting every lane's entries, ordering them for the LDS banks, encoding.  The ordering is what the host
 // spends its time on (16 cores: 150 ms for 18944 x 3584, 2.5 s for 3584 x 18944 on one).  Whole load of a matrix, tags on
-// the GPU to stream on the GPU, before / now: 3584 x 3584 363 / 2.7 ms, 18944 x 3584 155 / 6.0, 3584 x 18944 2525 / 12.9.
+// the GPU to stream on the GPU, the host builder / this one: 3584 x 3584 363 / 0.83 ms, 18944 x 3584 155 / 1.8, 3584 x 18944 2525 / 4.4.
 
 // A row's codebook as these kernels index with it: below G (a power of two) whatever row_book holds, as in the host builder.
 // The callers have refused a row_book that names another one, except where it may have been written since.
@@ -763,18 +763,51 @@ __device__ __forceinline__ int min64(int v) {
 }
 __device__ __forceinline__ int stream_ga(uint32_t e) { return (int)(e & 15u); }
 __device__ __forceinline__ int stream_gb(uint32_t e) { return (int)((e >> STREAM_SLICE_BITS) & 15u); }
-// fullest group of a histogram (maximum M, held by `at` groups) once a lane leaves a group of hp and joins another of hq
-__device__ __forceinline__ int stream_moved(int hp, int hq, int M, int at, bool same) {
-    if (same) return M;
-    return hq + 1 > M ? hq + 1 : (hp == M && at == 1 && hq + 1 < M) ? M - 1 : M;
+// thread K of each four
+template <int K> __device__ __forceinline__ int quad_lane(int v) { return __builtin_amdgcn_update_dpp(v, v, K * 0x55, 0xF, 0xF, false); }
+// The dwords that hold tags j .. j + 7 of a row (j a multiple of 8 behind the start of a part; past the row's end: its last dword),
+// and the tags in them.
+typedef uint32_t u32x4_by4 __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void stream_fetch8(const uint32_t* row, int W, int bits, int j, uint32_t (&d)[5]) {
+    const int w = (int)((int64_t)j * bits >> 5);
+    d[4] = 0u;
+    if (w + 5 <= W) {
+        const u32x4_by4 x = *reinterpret_cast<const u32x4_by4*>(row + w);
+        d[0] = x[0]; d[1] = x[1]; d[2] = x[2]; d[3] = x[3];
+        if (bits != 16 || (j & 1)) d[4] = row[w + 4];
+    } else {
+#pragma unroll
+        for (int i = 0; i < 5; ++i) d[i] = row[min(w + i, W - 1)];
+    }
+}
+__device__ __forceinline__ void stream_split8(const uint32_t (&d)[5], int bits, int j, uint32_t (&g)[8]) {
+    if (bits == 16 && (j & 1) == 0) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) g[k] = d[k / 2] >> (k % 2 * 16) & 0xFFFFu;
+        return;
+    }
+    const uint32_t s = (uint32_t)((int64_t)j * bits & 31), mask = (1u << bits) - 1u;
+    uint32_t x[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] = __builtin_amdgcn_alignbit(d[i + 1], d[i], s);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        g[k] = x[0] & mask;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) x[i] = __builtin_amdgcn_alignbit(x[i + 1], x[i], bits);
+        x[3] >>= bits;
+    }
 }
 
 // One workgroup per (bucket, group), one wave per clock of the group: it collects its 16 rows' entries (four threads per
 // row), orders them (the steps of BankMatch::order_lanes with ties resolved the same way; the 64 threads search a lane's
-// candidates together), and the four waves write the encoded steps to their places.  The search is a serial chain of
-// LDS reads, so what counts is its length: with the four clocks on one wave, 16 threads each, their branches took turns
-// (3584 x 18944: 49 ms against 10; 3584 x 3584: 1.7 against 0.8).  Matrices of a stack are filled side by side: each takes the
-// length of that chain however small it is (3584, 512 and 512 rows of 448 chunks: 1.1 ms in one launch, 2.05 in three).
+// candidates together), and the four waves write the encoded steps to their places.  Each wave is one serial chain, four or five of
+// them share a SIMD, and the older go first, so what counts is the instructions and the LDS round trips of a link (one clock per
+// wave: with four on one wave their branches took turns, 3584 x 18944 49 ms against 10).  3584, 512 and 512 rows of 448 chunks in one
+// launch take 0.44 ms, 1.02 with tags collected one by one (470 us of it; now 16 us a group: eight tags a thread and load), the
+// greedy fill through LDS counters (200 us; registers and ballots about half) and a search for every lane of every slot (350 us; now
+// only for the lanes that a ballot finds in a fullest group, with half the arithmetic).  Matrices of a stack are filled side by
+// side: each takes the length of its chains however small it is (one launch each: 1.9 times as long).
 template <bool LDS>
 __global__ __launch_bounds__(256) void stream_fill_kernel(StreamFillStack stack) {
     extern __shared__ __attribute__((aligned(16))) unsigned char stream_fill_lds[];
@@ -790,7 +823,7 @@ __global__ __launch_bounds__(256) void stream_fill_kernel(StreamFillStack stack)
     uint8_t* h = mem + (size_t)ns * (260 + 32 * q);                          // this clock's [slot][32]: codeword groups, x groups
     uint8_t* mx = mem + (size_t)ns * (260 + 128 + 4 * q);                    // and [slot][4]: their maxima
 
-    // entries of the clock's rows in this bucket, in chunk order: thread t counts, then writes a quarter of row t / 4
+    // entries of the clock's rows in this bucket, in chunk order: the four threads of a row take 32 of its tags at a time, eight each
     const int crow = STREAM_CLOCK_LANES_DEV[q][t >> 2];
     const uint32_t row_id = a.rows[(size_t)vg * 64 + crow];
     int total = 0;
@@ -798,22 +831,30 @@ __global__ __launch_bounds__(256) void stream_fill_kernel(StreamFillStack stack)
         const uint32_t* row = a.tags + (int64_t)row_id * a.W;
         const uint32_t book = stream_book(a.row_book, (int)row_id, a.G, a.bits);
         const int kp = v / a.NS, sl = v - kp * a.NS, p0 = kp * a.PC, len = min(a.PC, a.U - p0);
-        const int j0 = p0 + len * (t & 3) / 4, j1 = p0 + len * ((t & 3) + 1) / 4;
-        int n = 0;
-        for (int j = j0; j < j1; ++j) n += (int)((book | tag_at(row, a.W, a.bits, j)) >> STREAM_SLICE_BITS) == sl;
-        int before = 0;
+        uint32_t d[5], ahead[5];
+        stream_fetch8(row, a.W, a.bits, p0 + (t & 3) * 8, d);
+        for (int i0 = 0; i0 < len; i0 += 32) {
+            const int i = i0 + (t & 3) * 8;
+            stream_fetch8(row, a.W, a.bits, p0 + i + 32, ahead);
+            uint32_t g[8];
+            stream_split8(d, a.bits, p0 + i, g);
+            int n = 0;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int c = __shfl(n, (t & ~3) + k, 64);
-            before += k < (t & 3) ? c : 0;
-            total += c;
-        }
-        for (int j = j0; j < j1; ++j) {
-            const uint32_t g = book | tag_at(row, a.W, a.bits, j);
-            if ((int)(g >> STREAM_SLICE_BITS) == sl && before < ns) {
-                ent[before * 65 + crow] = (g & ((1u << STREAM_SLICE_BITS) - 1u)) | ((uint32_t)(j - p0) << STREAM_SLICE_BITS);
-                ++before;
+            for (int k = 0; k < 8; ++k) {
+                g[k] |= book;
+                n += (int)(g[k] >> STREAM_SLICE_BITS) == sl && i + k < len;
             }
+            const int n0 = quad_lane<0>(n), n1 = quad_lane<1>(n), n2 = quad_lane<2>(n), n3 = quad_lane<3>(n);
+            int slot = total + ((t & 3) > 0 ? n0 : 0) + ((t & 3) > 1 ? n1 : 0) + ((t & 3) > 2 ? n2 : 0);
+            total += n0 + n1 + n2 + n3;
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                if ((int)(g[k] >> STREAM_SLICE_BITS) == sl && i + k < len) {
+                    if (slot < ns) ent[slot * 65 + crow] = (g[k] & ((1u << STREAM_SLICE_BITS) - 1u)) | ((uint32_t)(i + k) << STREAM_SLICE_BITS);
+                    ++slot;
+                }
+#pragma unroll
+            for (int k = 0; k < 5; ++k) d[k] = ahead[k];
         }
     }
     for (int i = t; i < ns * 8; i += 64) reinterpret_cast<uint32_t*>(h)[i] = 0u;
@@ -834,66 +875,117 @@ __global__ __launch_bounds__(256) void stream_fill_kernel(StreamFillStack stack)
     for (int l = 0; l < 16; ++l)
         if (__builtin_amdgcn_readlane(rank, l) == sub) at_rank = l;
     const int ranked = __shfl(packed, at_rank, 64);
-    for (int n = 0; n < most; ++n)
+    if (most <= 64) {
+        // thread t holds entry t of every lane; the slot's counts are nibbles of two scalars (the newest, which may be the 16th of its
+        // group, is held back), and the first cheapest entry is the first set bit of a ballot: no LDS in the chain, a dozen vector
+        // instructions a link, which is what counts with four waves and more on a SIMD
+        uint32_t E[16];
+#pragma unroll
         for (int d = 0; d < 16; ++d) {
-            const int pk = __builtin_amdgcn_readlane(ranked, d), cl = pk >> 6, ln = pk & 63;
-            if (cl <= n) continue;
-            int key = 0x7FFFFFFF;                                            // cost << 16 | slot: the first cheapest
-            for (int i = n + t; i < cl; i += 64) {
-                const uint32_t e = ent[i * 65 + ln];
-                key = min(key, ((int)h[n * 32 + stream_ga(e)] + (int)h[n * 32 + 16 + stream_gb(e)]) << 16 | i);
-            }
-            const int bi = min64(key) & 0xFFFF;
-            const uint32_t en = ent[n * 65 + ln], eb = ent[bi * 65 + ln];
-            if (t == 0) {
-                ent[n * 65 + ln] = eb;
-                ent[bi * 65 + ln] = en;
-                ++h[n * 32 + stream_ga(eb)];
-                ++h[n * 32 + 16 + stream_gb(eb)];
-            }
-            __threadfence_block();
+            const int pk = __builtin_amdgcn_readlane(ranked, d);
+            E[d] = t < pk >> 6 ? ent[t * 65 + (pk & 63)] : 0u;
         }
+        for (int n = 0; n < most; ++n) {
+            uint64_t A = 0, B = 0, newA = 0, newB = 0;
+#pragma unroll
+            for (int d = 0; d < 16; ++d) {
+                const int cl = __builtin_amdgcn_readlane(ranked, d) >> 6;
+                if (cl <= n) continue;
+                A += newA;
+                B += newB;
+                const uint64_t open = (~0ull >> (64 - cl)) & (~0ull << n);   // entries n .. cl - 1
+                const int cost = ((int)(A >> 4 * stream_ga(E[d])) & 15) + ((int)(B >> 4 * stream_gb(E[d])) & 15);
+                uint64_t best = 0;
+                for (int c = 0; best == 0; ++c) best = __ballot(cost == c) & open;      // (entry n is open: its cost ends the loop)
+                const int bi = __builtin_ctzll(best);
+                const int en = __builtin_amdgcn_readlane((int)E[d], n), eb = __builtin_amdgcn_readlane((int)E[d], bi);
+                E[d] = (uint32_t)(t == n ? eb : t == bi ? en : (int)E[d]);
+                newA = 1ull << 4 * stream_ga((uint32_t)eb);
+                newB = 1ull << 4 * stream_gb((uint32_t)eb);
+            }
+            const uint64_t C = t < 16 ? A : B, newC = t < 16 ? newA : newB;
+            if (t < 32) h[n * 32 + t] = (uint8_t)(((C >> 4 * sub) & 15) + ((newC >> 4 * sub) & 15));
+        }
+#pragma unroll
+        for (int d = 0; d < 16; ++d) {
+            const int pk = __builtin_amdgcn_readlane(ranked, d);
+            if (t < pk >> 6) ent[t * 65 + (pk & 63)] = E[d];
+        }
+        __threadfence_block();
+    } else {
+        for (int n = 0; n < most; ++n)
+            for (int d = 0; d < 16; ++d) {
+                const int pk = __builtin_amdgcn_readlane(ranked, d), cl = pk >> 6, ln = pk & 63;
+                if (cl <= n) continue;
+                int key = 0x7FFFFFFF;                                        // cost << 16 | slot: the first cheapest
+                for (int i = n + t; i < cl; i += 64) {
+                    const uint32_t e = ent[i * 65 + ln];
+                    key = min(key, ((int)h[n * 32 + stream_ga(e)] + (int)h[n * 32 + 16 + stream_gb(e)]) << 16 | i);
+                }
+                const int bi = min64(key) & 0xFFFF;
+                const uint32_t en = ent[n * 65 + ln], eb = ent[bi * 65 + ln];
+                if (t == 0) {
+                    ent[n * 65 + ln] = eb;
+                    ent[bi * 65 + ln] = en;
+                    ++h[n * 32 + stream_ga(eb)];
+                    ++h[n * 32 + 16 + stream_gb(eb)];
+                }
+                __threadfence_block();
+            }
+    }
+    // the maxima of four slots at a time, 16 threads each
     auto rescan = [&](int n) {
         const int ca = h[n * 32 + sub], cb = h[n * 32 + 16 + sub];
         const int ma = max16(ca), mb = max16(cb);
         const int na = add16(ma > 0 && ca == ma), nb = add16(mb > 0 && cb == mb);
-        if (t == 0) *reinterpret_cast<uint32_t*>(mx + n * 4) = (uint32_t)ma | (uint32_t)na << 8 | (uint32_t)mb << 16 | (uint32_t)nb << 24;
+        if (sub == 0) *reinterpret_cast<uint32_t*>(mx + n * 4) = (uint32_t)ma | (uint32_t)na << 8 | (uint32_t)mb << 16 | (uint32_t)nb << 24;
     };
-    for (int n = 0; n < most; ++n) rescan(n);
+    for (int n = 0; n < most; n += 4) rescan(min(n + (t >> 4), most - 1));
     __threadfence_block();
     for (int pass = 0; pass < STREAM_CLIMB; ++pass)
         for (int n = 0; n < most; ++n) {
             const uint8_t* an = h + n * 32;
             const uint8_t* bn = an + 16;
-            uint32_t xw = *reinterpret_cast<const uint32_t*>(mx + n * 4);    // maximum and how many groups hold it, twice
-            xw = (uint32_t)__builtin_amdgcn_readfirstlane((int)xw);
-            if ((int)(xw & 0xFF) + (int)(xw >> 16 & 0xFF) <= 2) continue;
-            for (int l = 0; l < 16; ++l) {
-                const int pk = packed_of(l), cl = pk >> 6, ln = pk & 63;
-                if (cl <= n) continue;
-                const int x0 = (int)(xw & 0xFF), x1 = (int)(xw >> 8 & 0xFF), x2 = (int)(xw >> 16 & 0xFF), x3 = (int)(xw >> 24);
-                const uint32_t e = ent[n * 65 + ln];
-                const int ae = stream_ga(e), be = stream_gb(e), ane = an[ae], bne = bn[be];
-                if (!((ane == x0 && x0 > 1) || (bne == x2 && x2 > 1))) continue;
-                constexpr int NO_MOVE = 1 << 30;                             // (delta + 2^17) << 13 | slot, delta < 0
-                int key = NO_MOVE;
+            int x0, x1, x2, x3, ane16 = 0, bne16 = 0;                        // maximum and how many groups hold it, twice; thread `sub`:
+            uint32_t e16 = 0;                                                // its lane's entry and the counts of its groups
+            auto look = [&]() {                                              // the lanes that are in a fullest group, one bit each
+                const int xw = __builtin_amdgcn_readfirstlane((int)*reinterpret_cast<const uint32_t*>(mx + n * 4));
+                x0 = xw & 0xFF; x1 = xw >> 8 & 0xFF; x2 = xw >> 16 & 0xFF; x3 = xw >> 24 & 0xFF;
+                if (x0 + x2 <= 2) return 0u;
+                if (cnt > n) {
+                    e16 = ent[n * 65 + my_lane];
+                    ane16 = an[stream_ga(e16)];
+                    bne16 = bn[stream_gb(e16)];
+                }
+                return (uint32_t)__ballot(cnt > n && ((ane16 == x0 && x0 > 1) || (bne16 == x2 && x2 > 1))) & 0xFFFFu;
+            };
+            uint32_t todo = look();
+            while (todo) {
+                const int l = __builtin_ctz(todo), pk = packed_of(l), cl = pk >> 6, ln = pk & 63;
+                todo &= todo - 1;
+                const uint32_t e = (uint32_t)__builtin_amdgcn_readlane((int)e16, l);
+                const int ae = stream_ga(e), be = stream_gb(e), ane = __builtin_amdgcn_readlane(ane16, l), bne = __builtin_amdgcn_readlane(bne16, l);
+                // What a swap with slot m changes: the fullest group's count of slot n once e left for f's group, of slot m the other way
+                // round (a group that alone is fullest lets the maximum sink by one, the joined one may raise it), and for ties the
+                // squares, which weigh less than one clock.  Nothing where f's group is e's (the slot itself).
+                const int an0 = x0 - (ane == x0 && x1 == 1), bn0 = x2 - (bne == x2 && x3 == 1);
+                int key = 0;                                                 // delta << 13 | slot; only gains are below 0
                 for (int m = t; m < cl; m += 64) {
                     const uint32_t fm = ent[m * 65 + ln];
                     const int af = stream_ga(fm), bf = stream_gb(fm);
                     const uint8_t* am = h + m * 32;
                     const uint8_t* bq = am + 16;
-                    const uint32_t xm = *reinterpret_cast<const uint32_t*>(mx + m * 4);
-                    const int y0 = (int)(xm & 0xFF), y1 = (int)(xm >> 8 & 0xFF), y2 = (int)(xm >> 16 & 0xFF), y3 = (int)(xm >> 24);
+                    const int xm = *reinterpret_cast<const int*>(mx + m * 4), y0 = xm & 0xFF, y2 = xm >> 16 & 0xFF;
                     const int anf = an[af], bnf = bn[bf], ame = am[ae], amf = am[af], bqe = bq[be], bqf = bq[bf];
-                    const int clocks = stream_moved(ane, anf, x0, x1, ae == af) + stream_moved(bne, bnf, x2, x3, be == bf) +
-                                       stream_moved(amf, ame, y0, y1, ae == af) + stream_moved(bqf, bqe, y2, y3, be == bf) - (x0 + x2 + y0 + y2);
-                    const int sq = (af != ae ? 4 + 2 * (anf - ane + ame - amf) : 0) + (bf != be ? 4 + 2 * (bnf - bne + bqe - bqf) : 0);
-                    const int delta = clocks * 1024 + sq;
-                    if (m != n && clocks <= 0 && delta < 0) key = min(key, (delta + (1 << 17)) << 13 | m);
+                    const int am0 = (xm & 0xFFFF) == (amf | 1 << 8) ? y0 - 1 : y0, bm0 = xm >> 16 == (bqf | 1 << 8) ? y2 - 1 : y2;
+                    const int da = (max(anf + 1, an0) + max(ame + 1, am0) - x0 - y0) * 1024 + 4 + 2 * (anf - ane + ame - amf);
+                    const int db = (max(bnf + 1, bn0) + max(bqe + 1, bm0) - x2 - y2) * 1024 + 4 + 2 * (bnf - bne + bqe - bqf);
+                    const int delta = (af != ae ? da : 0) + (bf != be ? db : 0);
+                    if (delta < 0) key = min(key, delta * 8192 + m);
                 }
+                if (!__any(key < 0)) continue;                               // (nothing changed: the other bits stand)
                 key = min64(key);
-                if (key == NO_MOVE) continue;
-                const int bm = key & 0x1FFF;
+                const int bm = key & 0x1FFF;                                 // (the least key: the largest gain, its first slot)
                 const uint32_t fm = ent[bm * 65 + ln];
                 if (t == 0) {
                     const int af = stream_ga(fm), bf = stream_gb(fm);
@@ -903,33 +995,34 @@ __global__ __launch_bounds__(256) void stream_fill_kernel(StreamFillStack stack)
                     ent[bm * 65 + ln] = e;
                 }
                 __threadfence_block();
-                rescan(n);
-                rescan(bm);
+                rescan(t & 16 ? bm : n);
                 __threadfence_block();
-                xw = (uint32_t)__builtin_amdgcn_readfirstlane((int)*reinterpret_cast<const uint32_t*>(mx + n * 4));
-                if ((int)(xw & 0xFF) + (int)(xw >> 16 & 0xFF) <= 2) break;
+                todo = look() & (0xFFFEu << l);
             }
         }
     // padding: a lane that has run out repeats one of its codewords (least used bank group) against a zero chunk of x; a
     // lane without entries reads what a neighbour reads (in a clock without any entry: codeword 0 against a zero chunk)
     for (int n = 0; n < ns; ++n) {
-        int donor = __builtin_amdgcn_readfirstlane(min16(cnt > n ? sub : 16));
-        for (int l = 0; l < 16; ++l) {
-            const int pk = packed_of(l), cl = pk >> 6, ln = pk & 63;
-            if (cl > n || cl == 0) continue;
+        const uint32_t full = (uint32_t)__ballot(cnt > n) & 0xFFFFu;
+        uint32_t todo = (uint32_t)__ballot(cnt <= n && cnt > 0) & 0xFFFFu;
+        const int donor = full ? __builtin_ctz(full) : todo ? __builtin_ctz(todo) : 16;
+        int ca = h[n * 32 + sub], cb = h[n * 32 + 16 + sub];                 // thread `sub`: the counts of group sub
+        while (todo) {
+            const int l = __builtin_ctz(todo), pk = packed_of(l), cl = pk >> 6, ln = pk & 63;
+            todo &= todo - 1;
             int key = 0x7FFFFFFF;
-            for (int i = t; i < cl; i += 64) key = min(key, (int)h[n * 32 + stream_ga(ent[i * 65 + ln])] << 16 | i);
-            const int bi = min64(key) & 0xFFFF;
-            const int kb = min16((int)h[n * 32 + 16 + sub] << 4 | sub) & 15;
-            const uint32_t c = (ent[bi * 65 + ln] & ((1u << STREAM_SLICE_BITS) - 1u)) | ((uint32_t)(a.PC + kb) << STREAM_SLICE_BITS);
-            if (t == 0) {
-                ent[n * 65 + ln] = c;
-                ++h[n * 32 + stream_ga(c)];
-                ++h[n * 32 + 16 + stream_gb(c)];
+            for (int i0 = 0; i0 < cl; i0 += 64) {                            // (all threads: a count comes from the thread that has it)
+                const int i = min(i0 + t, cl - 1);
+                key = min(key, __shfl(ca, stream_ga(ent[i * 65 + ln]), 64) << 16 | i);
             }
-            __threadfence_block();
-            if (donor == 16) donor = l;
+            const int bi = min64(key) & 0xFFFF;
+            const int kb = min16(cb << 4 | sub) & 15;
+            const uint32_t c = (ent[bi * 65 + ln] & ((1u << STREAM_SLICE_BITS) - 1u)) | ((uint32_t)(a.PC + kb) << STREAM_SLICE_BITS);
+            if (t == 0) ent[n * 65 + ln] = c;
+            ca += sub == stream_ga(c);
+            cb += sub == stream_gb(c);
         }
+        __threadfence_block();
         const int dl = packed_of(donor & 15) & 63;
         if (cnt == 0 && t < 16) ent[n * 65 + my_lane] = donor < 16 ? ent[n * 65 + dl] : has_row ? (uint32_t)a.PC << STREAM_SLICE_BITS : 0u;
     }

@@ -19,7 +19,10 @@ CASES = [(1, 64, 8, 16, 1, 1, 0, "any"), (65, 3584, 8, 16, 1, 1, 2, "any"), (200
          (40, 512, 8, 15, 2, 3, 0, "low"), (129, 17408, 8, 16, 1, 1, 0, "low"), (17, 640, 4, 10, 1, 1, 0, "any"), (16, 384, 4, 12, 1, 1, 0, "any"),
          (31, 896, 4, 8, 2, 1, 0, "any"),
          # the longest run there is, runs of one and of several column orders with a short last group, two runs of one order
-         (6144, 256, 8, 13, 1, 1, 1, "any"), (6000, 264, 8, 14, 1, 3, 1, "low"), (1030, 64, 8, 16, 1, 16, 2, "one"), (6145, 128, 8, 13, 1, 1, 1, "low")]
+         (6144, 256, 8, 13, 1, 1, 1, "any"), (6000, 264, 8, 14, 1, 3, 1, "low"), (1030, 64, 8, 16, 1, 16, 2, "one"), (6145, 128, 8, 13, 1, 1, 1, "low"),
+         # entries of a lane below, at and beyond what a wave's registers hold; a second part that begins at an odd chunk
+         (40, 8 * 63, 8, 16, 1, 1, 1, "one"), (33, 8 * 64, 8, 14, 1, 1, 1, "one"), (70, 8 * 65, 8, 15, 1, 1, 1, "one"),
+         (66, 8 * 4069, 8, 16, 1, 1, 1, "any"), (21, 8 * 4069, 8, 14, 1, 1, 1, "low")]
 
 
 @pytest.mark.parametrize("R,C,d,bits,G,M,runs,how", CASES)
