@@ -143,31 +143,41 @@ static size_t mma_table_bytes(const sq_matrix& m) {
     return tab <= 128 * 1024 ? tab : 0;
 }
 
-// Rounds per wave, waves per workgroup and workgroup-level column slices that cover ceil(U / 4) rounds
-// with the fewest idle rounds (ties: more rounds per wave, i.e. fewer waves to add up).
+// Rounds per wave, waves per workgroup and workgroup-level column slices that cover ceil(U / 4) rounds.
+// Gathers from L2 (d = 8 and codebooks beyond LDS): the fewest idle rounds (ties: more rounds per wave, fewer waves to add up).
+// Codebooks in LDS: a tile is a chain of LDS round trips in every wave, so few waves leave the LDS idle, and a wave with all the
+// rounds its registers hold spends 5 us on fetching its activations; from 7 waves on the gathers' bank conflicts are the bound.
+// Extra column slices cost a launch that adds them up.  us at 4 rows, fewest idle rounds / this rule: 2 x 17408 x 5120, 12-bit tags
+// 25.1 (5 waves of 8 rounds) / 18.4 (10 of 4), with 4 books 27.4 / 24.8; 5120 x 17408 19.6 / 15.8; 2 x 14336 x 4096, 10-bit 18.0 / 13.5;
+// 4864 x 896, 8-bit 7.5 (1 wave) / 4.8 (4); 2 x 2048 x 2048, 4 books 9.4 / 6.3; 7 waves of 4 against 14 of 2 are alike (28 rounds).  With two
+// token tiles the sums to add are twice as long and 3 waves are enough (6 waves of 1 round: 15.8, 3 of 2: 11.9, 2 x 8960 x 1536).
 static MmaPlan mma_plan(const sq_matrix& m, int B) {
     const int ud = unit_dwords(m.bits), tpu = ud * 32 / m.bits, spu = tpu / (8 / m.d);
     const int rounds = (m.W / ud + 3) / 4, r1 = 32 / spu;
     MmaPlan best{0, 0, 0, 0};
     double best_cost = 1e30;
     const int NT = B > 16 ? 2 : 1;
-    // waves per workgroup: 8 (16 for the variants with few activation operands per lane, which fit four waves per SIMD),
-    // or as many as leave room in the CU's 160 KB of LDS, next to a codebook that is staged there (4 books of 4096 d = 4
-    // entries fill 128 KB), for their accumulators of the tiles in flight and their activation staging areas.  Long rows
-    // then take more, shorter column slices: 7B down, 148 rounds, at 4 rows: 15.1 us with 15 waves x 2 rounds x 5 slices
+    // waves per workgroup: mma_waves_max, or as many as leave room in the CU's 160 KB of LDS, next to a codebook that is staged there
+    // (4 books of 4096 d = 4 entries fill 128 KB), for their accumulators of the tiles in flight and their activation staging areas.
+    // Long rows then take more, shorter column slices: 7B down, 148 rounds, at 4 rows: 15.1 us with 15 waves x 2 rounds x 5 slices
     // against 18.4 with 7 x 8 x 3, reduction launch included.
     const size_t tab = mma_table_bytes(m);
-    for (int rw = NT == 1 ? r1 : r1 / 2; rw >= 1 && rw >= r1 / 4; rw /= 2) {
+    for (int rw = NT == 1 && !tab ? r1 : r1 / 2; rw >= 1 && rw >= r1 / 4; rw /= 2) {
         const int need = (rounds + rw - 1) / rw;
         int mk = 8;
         if (tab) {
             const size_t room = 160 * 1024 - tab - 16;
-            const size_t per_wave = std::max((size_t)64 * NT * 16 * mma_pft(rw), (size_t)mma_x_stage_bytes(tpu * m.d));
+            const size_t per_wave = std::max((size_t)64 * NT * 16 * mma_pft(rw, NT), (size_t)mma_x_stage_bytes(tpu * m.d, mma_x_tokens_min(NT)));
             mk = (int)std::min<size_t>(mma_waves_max(rw * spu * NT, true), room / per_wave);
             if (mk < 1) continue;
         }
         const int ks = (need + mk - 1) / mk, kw = (need + ks - 1) / ks;
-        const double cost = (double)rw * kw * ks / rounds + 0.03 * (ks - 1) + 0.002 * kw;
+        const double idle = (double)rw * kw * ks / rounds;
+        double cost = idle + 0.03 * (ks - 1) + 0.002 * kw;
+        if (tab) {
+            const double few = std::min(kw, NT == 1 ? 7 : 3);
+            cost = idle + 5.5 / (few * few) + 0.004 * kw + (ks > 1 ? 0.2 + 0.018 * (ks - 1) : 0.0);
+        }
         if (cost < best_cost - 1e-9) { best_cost = cost; best = MmaPlan{rw, NT, kw, ks}; }
     }
     return best;
@@ -225,7 +235,7 @@ static bool mma_fuses_silu(const sq_matrix* mats, int n, int B, const void* x, i
     if (tab == 0 || tab > 64 * 1024) return false;               // (beyond 64 KB two rows take the row-segment kernel)
     const MmaPlan pl = mma_plan(g, B);
     const int tpu = unit_dwords(g.bits) * 32 / g.bits;
-    return pl.ks == 1 && 2 * tab <= (size_t)pl.KW * 24 * 1024 && 2 * tab + 16 + std::max((size_t)pl.KW * mma_x_stage_bytes(tpu * g.d), (size_t)mma_group(pl.RW, true) * pl.KW * 64 * pl.NT * 16) <= 160 * 1024;
+    return pl.ks == 1 && 2 * tab <= (size_t)pl.KW * 24 * 1024 && 2 * tab + 16 + std::max((size_t)pl.KW * mma_x_stage_bytes(tpu * g.d, mma_x_tokens_min(pl.NT)), (size_t)mma_group(pl.RW, pl.NT, true) * pl.KW * 64 * pl.NT * 16) <= 160 * 1024;
 }
 
 // Pieces [0, cnt) share format and row length: one persistent launch (+ one reduction per piece if ks > 1).  act: mma_fuses_silu
@@ -246,10 +256,12 @@ static int launch_mma_group(const sq_matrix* mats, int cnt, const void* x, int x
     // LDS behind the codebook: the waves' accumulators of the tiles between two barriers (MMA_TT tiles when the codebook
     // is read through the cache; with the codebook in LDS as many as the workgroup walks, if they fit: sized below)
     const size_t red_tile = (size_t)pl.KW * 64 * pl.NT * 16;
-    const int pft = mma_group(pl.RW, act);
+    const int pft = mma_group(pl.RW, pl.NT, act);
     a.tg = a.table_bytes ? pft : 0;
     const int tpu = unit_dwords(m0.bits) * 32 / m0.bits;
-    const size_t xstage = (size_t)pl.KW * mma_x_stage_bytes(tpu * m0.d);      // the waves' activation staging areas (same LDS)
+    // 9 to 16 rows go through the staging areas at once where 16 tokens fit (7 waves of 12-bit tags: 7.6 us, in two parts 8.4)
+    a.xt = !a.table_bytes || (B > 8 && (size_t)a.table_bytes + 16 + (size_t)pl.KW * mma_x_stage_bytes(tpu * m0.d, 16) <= 160 * 1024) ? 16 : mma_x_tokens_min(pl.NT);
+    const size_t xstage = (size_t)pl.KW * mma_x_stage_bytes(tpu * m0.d, a.xt);      // the waves' activation staging areas (same LDS)
     size_t smem = (size_t)a.table_bytes + 16 + std::max(xstage, a.table_bytes ? (size_t)a.tg * red_tile : pl.KW > 1 ? (size_t)MMA_TT * red_tile : 0);
     int rc = SQ_EUNSUPPORTED;
 #define SQ_CASE(BI, DD) if (m0.bits == BI && m0.d == DD) rc = launch_mma_b##BI##d##DD(OP, a, pl.RW, pl.NT, GRID, threads, smem, s)

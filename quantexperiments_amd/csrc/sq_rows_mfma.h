@@ -49,17 +49,20 @@ struct MmaArgs {
     int ks;               // workgroup-level column slices
     int table_bytes;      // bytes of codebook staged in LDS (0 = read through cache)
     int tg;               // codebook in LDS: 16-row tiles whose accumulators LDS holds between two barriers (a multiple of mma_group())
+    int xt;               // tokens of a staging area: 16, or 8 (one token tile)
     int act;              // 1: the two pieces are a gate and an up projection, y receives SiLU(gate) * up (16-bit)
 };
 
 constexpr int MMA_TT = 4;     // 16-row tiles multiplied between two workgroup barriers (codebook read through the cache)
-// codebook in LDS: tiles of tags in flight per lane (fewer when a lane's part of a tile is long: registers)
-// (2 to 5 tiles in flight measure alike on the 7B shapes)
-constexpr int mma_pft(int RW) { return RW >= 8 ? 2 : 3; }
-constexpr int mma_group(int RW, bool act) { return act && mma_pft(RW) % 2 ? 2 * mma_pft(RW) : mma_pft(RW); }     // ACT: whole pairs
-// LDS per wave in which a round's activations (16 tokens x 4 lane units of UK columns, fp16) pass from whole-line loads
-// to the lanes that use them; it lies where the accumulators are added afterwards
-constexpr int mma_x_stage_bytes(int UK) { return 16 * (4 * UK * 2 + 16); }
+// codebook in LDS: tiles of tags in flight per lane (two where a third one's registers would cost a wave per SIMD; 2 to 5 tiles
+// in flight measure alike on the 7B shapes)
+constexpr int mma_pft(int RW, int NT) { return RW >= 8 || (RW >= 4 && NT == 1) ? 2 : 3; }
+constexpr int mma_group(int RW, int NT, bool act) { return act && mma_pft(RW, NT) % 2 ? 2 * mma_pft(RW, NT) : mma_pft(RW, NT); }     // ACT: whole pairs
+// LDS per wave in which a round's activations (`tokens` x 4 lane units of UK columns, fp16) pass from whole-line loads to the lanes
+// that use them; it lies where the accumulators are added afterwards.  16 tokens at a time, or 8 (MmaArgs.xt): enough for up to
+// 8 rows, and what lets twice the waves start next to 128 KB of codebooks.
+constexpr int mma_x_stage_bytes(int UK, int tokens) { return tokens * (4 * UK * 2 + 16); }
+constexpr int mma_x_tokens_min(int NT) { return NT == 1 ? 8 : 16; }
 
 // Optional timeline of the first wave of every workgroup (debug builds define SQ_TRACE_POINT).
 #ifndef SQ_TRACE_POINT
@@ -86,15 +89,15 @@ typedef __attribute__((address_space(3))) u32x4 mma_lds_u32x4;
 // kernel differ from the batch-1 one on the same input)
 __device__ __forceinline__ uint32_t bf2h_pk(uint32_t v) { return bf2h_x2(v); }
 
-// Waves per workgroup: up to 16 for the variants whose lanes hold at most 8 activation operands (32 registers) beside a
-// codebook in LDS, which fit four waves per SIMD; 8 otherwise.
-constexpr int mma_waves_max(int x_operands, bool lds_tab) { return lds_tab && x_operands <= 8 ? 16 : 8; }
+// Waves per workgroup beside a codebook in LDS: 16 (four per SIMD) for the variants whose lanes hold at most 8 activation operands (32
+// registers), 12 for those with 16; 8 otherwise.
+constexpr int mma_waves_max(int x_operands, bool lds_tab) { return !lds_tab ? 8 : x_operands <= 8 ? 16 : x_operands <= 16 ? 12 : 8; }
 
 // ACT (codebooks in LDS): p[0] is a gate and p[1] an up projection of one shape, both codebooks are staged, a workgroup walks the
 // two pieces' tiles in turn (virtual tile i: tile i / 2 of piece i % 2), and the wave that adds up a pair of tiles writes SiLU(gate) * up,
 // with the same roundings as the product followed by silu_mul_kernel.  It saves that launch and the trip of gate and up through memory
 // (2 x 18944 x 3584, 12-bit tags, 8 rows: 20.4 us, now 17.6).
-template <int BITS, int D, int RW, int NT, bool LDS_TAB, bool ACT = false>
+template <int BITS, int D, int RW, int NT, bool LDS_TAB, bool ACT = false, int XT = 16>
 __global__ __launch_bounds__(64 * mma_waves_max(RW * ((unit_of<BITS>::UD * 32 / BITS) / (8 / D)) * NT, LDS_TAB))
 void rows_mfma_kernel(MmaArgs a) {
     constexpr int UD = unit_of<BITS>::UD;
@@ -195,7 +198,7 @@ void rows_mfma_kernel(MmaArgs a) {
     static_assert(16 / XTPI == SPU, "a round's activations are SPU loads per token tile");
     constexpr int F = ACT ? 2 : 1;                           // pieces whose tiles a workgroup walks
     const MmaPiece& P1 = a.p[F - 1];
-    unsigned char* xst = smem + a.table_bytes + 16 + wave * mma_x_stage_bytes(UK);
+    unsigned char* xst = smem + a.table_bytes + 16 + wave * mma_x_stage_bytes(UK, XT);
     const int xtl = lane / (XRB / 16), xob = (lane % (XRB / 16)) * 16;    // this lane's token (within an instruction) and byte in the round
     u32x4 xraw[RW][NT][SPU];
 #pragma unroll
@@ -212,7 +215,7 @@ void rows_mfma_kernel(MmaArgs a) {
     if constexpr (!ACT) fetch(t0 < t1 ? t0 : ntiles - 1, tA, sc[0]);     // (no branch around the loads; a workgroup without tiles reads the last one)
     // (codebook in LDS: the tags of the first tiles in flight, without a branch around the loads so that the waits count
     // them exactly: the two layouts differ in a base and a stride, chosen once)
-    constexpr int PFT = LDS_TAB ? mma_pft(RW) : 1;
+    constexpr int PFT = LDS_TAB ? mma_pft(RW, NT) : 1;
     const bool til = P.tiled != nullptr;
     const uint32_t* fbase = til ? P.tiled + li * UD : tags;
     const uint32_t* fbase1 = ACT ? (til ? P1.tiled + li * UD : reinterpret_cast<const uint32_t*>(P1.m.tags)) : fbase;
@@ -237,31 +240,51 @@ void rows_mfma_kernel(MmaArgs a) {
         for (int q = ACT ? 0 : 1; q < PFT; ++q) fetch_tags(min(i0 + q, max(i1 - 1, i0)), ring[q]);
     }
     // the B operands: this wave's activations as fp16, in registers for the whole kernel
+    constexpr bool WHOLE = XT == 16;                             // else tokens 0 .. 7 first, then 8 .. 15 in the same place
+    static_assert(WHOLE || (XT == 8 && NT == 1), "one token tile in parts of 8");
     half8v xb[RW][SPU][NT];
+    auto stage = [&](u32x4 v, int row) {
+        if (a.x_dtype == SQ_BF16) { v.x = bf2h_pk(v.x); v.y = bf2h_pk(v.y); v.z = bf2h_pk(v.z); v.w = bf2h_pk(v.w); }
+        *reinterpret_cast<u32x4*>(xst + row * XROW + xob) = v;
+    };
+    // (the lanes of a wave exchange data here: its LDS instructions run in order, the fences keep the compiler from
+    // moving a lane's reads before its writes)
+    auto exchange = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    const unsigned char* xmine = xst + (WHOLE ? li : li & 7) * XROW + lg * (UK * 2);
 #pragma unroll
     for (int n = 0; n < RW; ++n)
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
+            constexpr int HALF = 8 / XTPI;
 #pragma unroll
-            for (int j = 0; j < SPU; ++j) {
-                u32x4 v = xraw[n][nt][j];
-                if (a.x_dtype == SQ_BF16) { v.x = bf2h_pk(v.x); v.y = bf2h_pk(v.y); v.z = bf2h_pk(v.z); v.w = bf2h_pk(v.w); }
-                *reinterpret_cast<u32x4*>(xst + (j * XTPI + xtl) * XROW + xob) = v;
-            }
-            // (the lanes of a wave exchange data here: its LDS instructions run in order, the fences keep the compiler from
-            // moving a lane's reads before its writes)
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            for (int j = 0; j < HALF; ++j) stage(xraw[n][nt][j], j * XTPI + xtl);
+            if (WHOLE)
+#pragma unroll
+                for (int j = HALF; j < SPU; ++j) stage(xraw[n][nt][j], j * XTPI + xtl);
+            exchange();
+            const bool mine = live[n] && nt * 16 + li < a.B;
 #pragma unroll
             for (int s = 0; s < SPU; ++s) {
-                u32x4 v = *reinterpret_cast<const u32x4*>(xst + li * XROW + lg * (UK * 2) + s * 16);
-                if (!(live[n] && nt * 16 + li < a.B)) v = u32x4{0u, 0u, 0u, 0u};
+                u32x4 v = *reinterpret_cast<const u32x4*>(xmine + s * 16);
+                if (!(mine && (WHOLE || li < 8))) v = u32x4{0u, 0u, 0u, 0u};
                 xb[n][s][nt] = __builtin_bit_cast(half8v, v);
             }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            exchange();
+            if (!WHOLE && a.B > 8) {
+#pragma unroll
+                for (int j = HALF; j < SPU; ++j) stage(xraw[n][nt][j], j * XTPI + xtl - 8);
+                exchange();
+#pragma unroll
+                for (int s = 0; s < SPU; ++s) {
+                    const u32x4 v = *reinterpret_cast<const u32x4*>(xmine + s * 16);
+                    if (mine && li >= 8) xb[n][s][nt] = __builtin_bit_cast(half8v, v);
+                }
+                exchange();
+            }
         }
     // (a codebook of whole KB goes memory -> LDS without passing through registers, a wave instruction per KB)
     if (table_dma) {
@@ -491,13 +514,19 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
 // op 0: launch; op 1: workgroups of `threads` threads and `smem` bytes of LDS that fit on one CU
 template <int BITS, int D, int RW, int NT>
 static inline int mma_inst(int op, const MmaArgs& a, int grid, int threads, size_t smem, hipStream_t s) {
-    void (*k)(MmaArgs) = a.table_bytes ? rows_mfma_kernel<BITS, D, RW, NT, true> : rows_mfma_kernel<BITS, D, RW, NT, false>;
-    if constexpr (D == 4)
-        if (a.act) k = rows_mfma_kernel<BITS, D, RW, NT, true, true>;
+    // (with its codebooks in LDS, d = 4, a wave never takes the most rounds it could: see mma_plan)
+    constexpr bool LDS = D == 4 && !(NT == 1 && RW * ((unit_of<BITS>::UD * 32 / BITS) / (8 / D)) > 16);
+    void (*k)(MmaArgs) = rows_mfma_kernel<BITS, D, RW, NT, false>;
+    if constexpr (LDS) {
+        if (a.table_bytes) k = a.act ? rows_mfma_kernel<BITS, D, RW, NT, true, true> : rows_mfma_kernel<BITS, D, RW, NT, true>;
+        if constexpr (NT == 1)
+            if (a.xt == 8 && a.table_bytes) k = a.act ? rows_mfma_kernel<BITS, D, RW, NT, true, true, 8> : rows_mfma_kernel<BITS, D, RW, NT, true, false, 8>;
+    }
+    if (a.table_bytes && !LDS) return fail(SQ_EUNSUPPORTED, "sq_linear_small: no matrix-core kernel for %d rounds and codebooks in LDS", RW);
     if (op == 1) {
         static std::mutex mu;
         static std::unordered_map<uint64_t, int> cache;
-        const uint64_t key = ((uint64_t)threads << 40) | ((uint64_t)(a.table_bytes != 0) << 39) | ((uint64_t)a.act << 38) | (uint64_t)smem;
+        const uint64_t key = ((uint64_t)threads << 40) | ((uint64_t)(a.table_bytes != 0) << 39) | ((uint64_t)a.act << 38) | ((uint64_t)(a.xt == 8) << 37) | (uint64_t)smem;
         std::lock_guard<std::mutex> lock(mu);
         auto it = cache.find(key);
         if (it != cache.end()) return it->second;
