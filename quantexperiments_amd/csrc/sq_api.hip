@@ -573,7 +573,11 @@ int sq_q8_linear(const int8_t* q, const uint16_t* scale, int32_t V, int32_t C, c
     if (!x || !y) return fail(SQ_EINVAL, "sq_q8_linear: null x / y");
     if (B > 1 && (ldx < C || ldy < V)) return fail(SQ_EINVAL, "sq_q8_linear: ldx %lld / ldy %lld too small", (long long)ldx, (long long)ldy);
     const bool has_ws = workspace && ws_bytes >= SQ_WS_HEADER;
-    if (q8_mid(C, B))
+    // (rows that are not whole 256-column chunks: the calls that the other routes take, without a workspace up to SQ_SMALL_BMAX rows and
+    // only aligned ones beyond, stay theirs)
+    const bool mid = C % 256 == 0 || ((has_ws && ws_bytes - SQ_WS_HEADER >= q8_mid_workspace(V, C, B)) &&
+                                      (B <= SQ_SMALL_BMAX || (ldx % 8 == 0 && ((uintptr_t)x & 15) == 0)));
+    if (q8_mid(V, C, B) && mid)
         return launch_q8_mid(q, scale, V, C, x, x_dtype, ldx, y, y_dtype, ldy, B, has_ws ? (char*)workspace + SQ_WS_HEADER : nullptr,
                              has_ws ? ws_bytes - SQ_WS_HEADER : 0, (hipStream_t)stream);
     if (B <= SQ_SMALL_BMAX) return launch_q8_small(q, scale, V, C, x, x_dtype, ldx, y, y_dtype, ldy, B, (hipStream_t)stream);
@@ -583,7 +587,7 @@ int sq_q8_linear(const int8_t* q, const uint16_t* scale, int32_t V, int32_t C, c
 
 size_t sq_q8_workspace_bytes(int32_t V, int32_t C, int32_t B) {
     if (C <= 0 || C % 32) return 0;
-    const size_t inner = q8_mid(C, B) ? q8_mid_workspace(C, B) : q8_workspace(V, C, B);
+    const size_t inner = q8_mid(V, C, B) ? std::max(q8_mid_workspace(V, C, B), C % 256 ? q8_workspace(V, C, B) : (size_t)0) : q8_workspace(V, C, B);
     return inner ? inner + SQ_WS_HEADER : 0;
 }
 

@@ -181,7 +181,7 @@ __global__ __launch_bounds__(256, 2) void q8_gemv_kernel(Q8Args a) {
     }
 }
 
-// ---- 3 .. Q8_MFMA_MAX_ROWS activation rows (C % 256 == 0): fp16 MFMA, 16, 32 or 64 activation rows per pass.
+// ---- 3 .. Q8_MFMA_MAX_ROWS activation rows (C % 64 == 0): fp16 MFMA, 16, 32 or 64 activation rows per pass.
 // v_mfma_f32_16x16x32_f16 operand layout: A: lane l supplies weight row l % 16, k = 8 * (l / 16) .. + 7; B: token
 // l % 16, the same k; D: lane l holds token l % 16, weight rows 4 * (l / 16) .. + 3.  Weights are the A operand and a
 // wave owns 16 rows.  The rows reach the wave through LDS: global_load_lds (no registers in between) fetches them in
@@ -233,7 +233,10 @@ constexpr int q8l_lds_bytes(int nblk, int waves, int d, int xs) { return 2 * nbl
 
 // NBLK 16-token blocks, WAVES waves per workgroup, ring of D steps per wave (one being multiplied, D - 1 in flight),
 // x chunks of XS steps (128 XS columns; the first 16 NBLK XS / 4 waves copy 4 / XS tokens of every chunk each)
-template <int NBLK, int WAVES, int D, int XS>
+// ANY_C: rows of any whole pairs of blocks (C % 64 == 0).  The steps behind the row's end copy its last pieces again and multiply
+// nothing.  Such rows ran on the exact-product kernel, so their block scales stay out of the fp16 weights: a matrix instruction takes
+// the 32 columns of one block (lane group g: columns 8 g .. 8 g + 7) and its sums, fp32, are multiplied by the block's scales.
+template <int NBLK, int WAVES, int D, int XS, bool ANY_C>
 __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel(Q8MfmaArgs a) {
     static_assert((D == 3 || D == 4) && (XS == 2 || (XS == 1 && D == 3)), "wait counts below are written out for these");
     constexpr int Q8L_D = D, Q8L_WAVE_BYTES = q8l_wave_bytes(D);
@@ -247,7 +250,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel
     const bool active = task_raw < a.tasks;
     const int task = active ? task_raw : a.tasks - 1;
     const int r = lane & 15, g = lane >> 4;
-    const int C = a.C, nblk = C >> 5, nsteps = C >> 7, nchunks = nsteps / XS;
+    const int C = a.C, nblk = C >> 5, nsteps = ANY_C ? ((C + 255) >> 8) * 2 : C >> 7, nchunks = nsteps / XS;
 
     typedef const __attribute__((address_space(1))) void* gptr_t;
     typedef __attribute__((address_space(3))) void* lptr_t;
@@ -255,33 +258,38 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel
     // at slot p ^ (t % 16), so the 16 lanes of a read clock (16 tokens, one piece) spread over 16 bank groups
     constexpr int TPI = 4 / XS, LPT = 64 / TPI;                 // tokens per instruction, lanes (= pieces) per token
     uint32_t xsrc;
+    int xcol;                                                   // this lane's column in a chunk
     {
         const int rowx = wave * TPI + lane / LPT;
         const int piece = (lane % LPT) ^ (rowx & 15);
-        xsrc = (uint32_t)(min(rowx, a.B - 1) * a.ldxh + piece * 8);
+        xcol = piece * 8;
+        xsrc = (uint32_t)(min(rowx, a.B - 1) * a.ldxh + (ANY_C ? 0 : xcol));
     }
     const bool xo = wave * TPI < 16 * NBLK;                     // this wave takes part in the x copies
     auto copy_x = [&](int c) {
-        if (xo) __builtin_amdgcn_global_load_lds((gptr_t)(a.xh + c * (XS * 128) + xsrc), (lptr_t)(xs + (c & 1) * XBUF + wave * TPI * XPITCH), 16, 0, 0);
+        const uint32_t at = ANY_C ? (uint32_t)min(c * (XS * 128) + xcol, C - 8) : (uint32_t)(c * (XS * 128));
+        if (xo) __builtin_amdgcn_global_load_lds((gptr_t)(a.xh + at + xsrc), (lptr_t)(xs + (c & 1) * XBUF + wave * TPI * XPITCH), 16, 0, 0);
     };
     // weights: instruction n of a step fills rows 8 n .. 8 n + 7; lane i lands in row 8 n + i / 8, slot i % 8 and
     // fetches the piece the swizzle keeps there
     const int8_t* wsrc[2];
+    int wcol[2];                                                // this lane's column in a step
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
         const int rw = 8 * n + (lane >> 3);
         const int piece = (lane & 7) ^ ((rw >> 1) & 7);
-        wsrc[n] = a.q + (int64_t)min(task * 16 + rw, a.V - 1) * C + piece * 16;
+        wcol[n] = piece * 16;
+        wsrc[n] = a.q + (int64_t)min(task * 16 + rw, a.V - 1) * C + (ANY_C ? 0 : wcol[n]);
     }
     auto copy_w = [&](int s) {
 #pragma unroll
         for (int n = 0; n < 2; ++n)
-            __builtin_amdgcn_global_load_lds((gptr_t)(wsrc[n] + s * 128), (lptr_t)(wl + (s % Q8L_D) * 2048 + n * 1024), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((gptr_t)(wsrc[n] + (ANY_C ? min(s * 128 + wcol[n], C - 16) : s * 128)), (lptr_t)(wl + (s % Q8L_D) * 2048 + n * 1024), 16, 0, 0);
     };
     // scales of chunk c: lane i fetches dword i % 4 of row i / 4
-    const char* ssrc = (const char*)(a.sc + (int64_t)min(task * 16 + (lane >> 2), a.V - 1) * nblk) + (lane & 3) * 4;
+    const char* ssrc = (const char*)(a.sc + (int64_t)min(task * 16 + (lane >> 2), a.V - 1) * nblk) + (ANY_C ? 0 : (lane & 3) * 4);
     auto copy_s = [&](int c) {
-        __builtin_amdgcn_global_load_lds((gptr_t)(ssrc + c * 16), (lptr_t)(sl_ + (c % (D - 1)) * 256), 4, 0, 0);
+        __builtin_amdgcn_global_load_lds((gptr_t)(ssrc + (ANY_C ? min(c * 16 + (lane & 3) * 4, nblk * 2 - 4) : c * 16)), (lptr_t)(sl_ + (c % (D - 1)) * 256), 4, 0, 0);
     };
     const uint32_t xrow = (uint32_t)r * XPITCH, xsw = (uint32_t)r;
     const uint32_t wsw = (uint32_t)((r >> 1) & 7);
@@ -334,6 +342,37 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel
         }
         __builtin_amdgcn_sched_barrier(0);
         const unsigned char* st = wl + (s % Q8L_D) * 2048;
+        if constexpr (ANY_C) {
+            u32x2 sb[4];                                        // the four blocks' scales of this lane's four output rows
+#pragma unroll
+            for (int v = 0; v < 4; ++v) sb[v] = *reinterpret_cast<const u32x2*>(sl_ + (c % (D - 1)) * 256 + (4 * g + v) * 16 + odd * 8);
+            const unsigned char* xc = xs + (cx & 1) * XBUF + xrow;
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                if (s * 4 + b >= nblk) break;                   // (uniform: behind the row's end)
+                const u32x2 wq = *reinterpret_cast<const u32x2*>(st + r * 128 + (((uint32_t)(2 * b + (g >> 1)) ^ wsw) << 4) + (g & 1) * 8);
+                half2v p[4];
+                i8x4_to_h2(wq[0], p[0], p[1]);
+                i8x4_to_h2(wq[1], p[2], p[3]);
+                half8v w;
+                float sf[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    w[2 * k] = p[k][0]; w[2 * k + 1] = p[k][1];
+                    sf[k] = h2f((uint16_t)(sb[k][b >> 1] >> ((b & 1) * 16)));
+                }
+                const uint32_t px = (uint32_t)((s % XS) * 16 + b * 4 + g);
+#pragma unroll
+                for (int nb = 0; nb < NBLK; ++nb) {
+                    const half8v xv = *reinterpret_cast<const half8v*>(xc + nb * (16 * XPITCH) + ((px ^ xsw) << 4));
+                    const float4v d = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, xv, float4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) acc[nb][v] += sf[v] * d[v];
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            continue;
+        }
         const u32x4 wq[2] = {*reinterpret_cast<const u32x4*>(st + w0), *reinterpret_cast<const u32x4*>(st + w1)};
         const half_t sh = __builtin_bit_cast(half_t, *reinterpret_cast<const uint16_t*>(sl_ + (c % (D - 1)) * 256 + r * 16 + odd * 8 + g * 2));
         const half2v s2 = {sh, sh};
@@ -467,18 +506,27 @@ static int q8_pass_rows(int B, int C) {
     return nb;
 }
 
-// The MFMA passes need C % 256 == 0 (whole 256-column chunks of x) and 64 activation rows of C halves within
-// 32-bit offsets.
-static bool q8_mfma_ok(int C) { return C % 256 == 0 && (int64_t)C * 64 < ((int64_t)1 << 31); }
+// The MFMA passes need whole 4-byte pairs of block scales and 64 activation rows of C halves within 32-bit offsets.
+static bool q8_mfma_ok(int C) { return C % 64 == 0 && (int64_t)C * 64 < ((int64_t)1 << 31); }
 
 // from 3 rows the MFMA passes win over the 4-row kernel (152,064 x 3,584: 106 against 148 us; 248,320 x 5,120: 246
 // against 255 us); 2 rows stay on the exact-product kernel (106-115 / 228 us)
-bool q8_mid(int C, int B) { return B > 2 && B <= Q8_MFMA_MAX_ROWS && q8_mfma_ok(C); }
-size_t q8_mid_workspace(int C, int B) { return q8_mid(C, B) ? (((size_t)B * C * 2) + 255) & ~(size_t)255 : 0; }
+// Rows that are not whole 256-column chunks, us, exact-product kernel or (above 32 rows) decode + tile GEMM / these passes: 25 rows of
+// 141,347 x 1,408 348 / 47, of 9,823 x 3,456 102 / 29, 8 of 70,061 x 1,216 63 / 24.5.  A small grid is bound by the length of a wave's
+// chain, 0.8 us per 128 columns: 3 rows of 9,823 x 3,456 15.9 / 24, of 16,000 x 1,216 8.3 / 10.7, of 32,000 x 640 8.9 / 7.9, of 30,000 x 1,216
+// 15.1 / 12.1; 5 of 9,823 x 3,456 25.0 / 23.5; 64 of it 45.5 / 55, of 16,000 x 3,456 62 / 52, of 8,211 x 576 33 / 18.  A second pass: 100 rows of
+// 30,000 x 1,216 41.3 / 41.9, of 32,000 x 640 33.6 / 27.6, of 50,000 x 3,520 203 / 106, 200 of 70,061 x 1,216 164 / 170.
+bool q8_mid(int V, int C, int B) {
+    if (B <= 2 || !q8_mfma_ok(C)) return false;
+    if (C % 256 == 0) return B <= Q8_MFMA_MAX_ROWS;
+    if (B <= 4 || B > 64) return V >= 30000 && B <= 128;
+    return B <= 32 || V >= 16000 || C <= 2048;
+}
+size_t q8_mid_workspace(int V, int C, int B) { return q8_mid(V, C, B) ? (((size_t)B * C * 2) + 255) & ~(size_t)255 : 0; }
 
 int launch_q8_mid(const int8_t* q, const uint16_t* sc, int V, int C, const void* x, int x_dtype, int64_t ldx, void* y,
                   int y_dtype, int64_t ldy, int B, void* ws, size_t ws_bytes, hipStream_t s) {
-    if (ws_bytes < q8_mid_workspace(C, B)) return fail(SQ_EWORKSPACE, "sq_q8_linear: workspace %zu < %zu", ws_bytes, q8_mid_workspace(C, B));
+    if (ws_bytes < q8_mid_workspace(V, C, B)) return fail(SQ_EWORKSPACE, "sq_q8_linear: workspace %zu < %zu", ws_bytes, q8_mid_workspace(V, C, B));
     const size_t ys = y_dtype == SQ_F32 ? 4 : 2;
     // fp16 activations with 16-byte aligned rows are copied to LDS from where they are; anything else goes through
     // an fp16 copy in the workspace first
@@ -505,29 +553,33 @@ int launch_q8_mid(const int8_t* q, const uint16_t* sc, int V, int C, const void*
         a.y = (char*)y + (size_t)b0 * ldy * ys;
         a.ldy = ldy; a.V = V; a.C = C; a.B = B - b0 < pass ? B - b0 : pass; a.y_dtype = y_dtype; a.tasks = tasks;
         a.vec_y = ((uintptr_t)a.y & 7) == 0 && ldy % 4 == 0;
-        static bool raised = false;
-        if (!raised) {
-            (void)hipFuncSetAttribute((const void*)q8_mfma_kernel<1, 8, 3, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-            (void)hipFuncSetAttribute((const void*)q8_mfma_kernel<2, 16, 3, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-            (void)hipFuncSetAttribute((const void*)q8_mfma_kernel<2, 8, 3, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-            (void)hipFuncSetAttribute((const void*)q8_mfma_kernel<4, 16, 3, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-            (void)hipGetLastError();
-            raised = true;
-        }
         // 17-32 rows: one workgroup of 16 waves per CU sharing 256-column x chunks, unless its workgroups fill the last
         // round of the chip badly; then 8 waves with 128-column chunks (a barrier per step, two workgroups per CU).
         // Measured: 152,064 x 3,584 (594 workgroups of 16 waves, 2.3 rounds) 126 against 116 us; 248,320 x 5,120
         // (970, 3.8 rounds) 265 against 278 us.
         const int cus = device_cus(), n16 = (tasks + 15) / 16;
         const bool x128 = (double)n16 / ((double)((n16 + cus - 1) / cus) * cus) < 0.85;
+        auto go = [&](void (*kernel)(Q8MfmaArgs), int waves, size_t lds) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)((tasks + waves - 1) / waves)), dim3((unsigned)waves * 64), lds, s, a);
+        };
+        static bool raised = false;
+        if (!raised) {
+            for (void (*k)(Q8MfmaArgs) : {q8_mfma_kernel<1, 8, 3, 2, false>, q8_mfma_kernel<2, 16, 3, 2, false>, q8_mfma_kernel<2, 8, 3, 1, false>,
+                                          q8_mfma_kernel<4, 16, 3, 1, false>, q8_mfma_kernel<1, 8, 3, 2, true>, q8_mfma_kernel<2, 16, 3, 2, true>,
+                                          q8_mfma_kernel<2, 8, 3, 1, true>, q8_mfma_kernel<4, 16, 3, 1, true>})
+                (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+            (void)hipGetLastError();
+            raised = true;
+        }
+        const bool any = C % 256 != 0;
         if (a.B > 32)                                           // 33-64 rows: 16 waves share 128-column chunks of 64 tokens
-            hipLaunchKernelGGL((q8_mfma_kernel<4, 16, 3, 1>), dim3((unsigned)((tasks + 15) / 16)), dim3(1024), q8l_lds_bytes(4, 16, 3, 1), s, a);
+            go(any ? q8_mfma_kernel<4, 16, 3, 1, true> : q8_mfma_kernel<4, 16, 3, 1, false>, 16, q8l_lds_bytes(4, 16, 3, 1));
         else if (a.B > 16 && x128)
-            hipLaunchKernelGGL((q8_mfma_kernel<2, 8, 3, 1>), dim3((unsigned)((tasks + 7) / 8)), dim3(512), q8l_lds_bytes(2, 8, 3, 1), s, a);
+            go(any ? q8_mfma_kernel<2, 8, 3, 1, true> : q8_mfma_kernel<2, 8, 3, 1, false>, 8, q8l_lds_bytes(2, 8, 3, 1));
         else if (a.B > 16)
-            hipLaunchKernelGGL((q8_mfma_kernel<2, 16, 3, 2>), dim3((unsigned)((tasks + 15) / 16)), dim3(1024), q8l_lds_bytes(2, 16, 3, 2), s, a);
+            go(any ? q8_mfma_kernel<2, 16, 3, 2, true> : q8_mfma_kernel<2, 16, 3, 2, false>, 16, q8l_lds_bytes(2, 16, 3, 2));
         else
-            hipLaunchKernelGGL((q8_mfma_kernel<1, 8, 3, 2>), dim3((unsigned)((tasks + 7) / 8)), dim3(512), q8l_lds_bytes(1, 8, 3, 2), s, a);
+            go(any ? q8_mfma_kernel<1, 8, 3, 2, true> : q8_mfma_kernel<1, 8, 3, 2, false>, 8, q8l_lds_bytes(1, 8, 3, 2));
         rc = check_launch("q8_mfma_kernel");
         if (rc) return rc;
         b0 += a.B;

@@ -551,7 +551,12 @@ def q8_linear(q: torch.Tensor, sc: torch.Tensor, x: torch.Tensor, y: torch.Tenso
     L = _lib.lib()
     with torch.cuda.device(dev):
         need = L.sq_q8_workspace_bytes(V, C, x.shape[0])
-        ws = _Workspace.get(need, dev) if need else None
+        try:
+            ws = _Workspace.get(need, dev) if need else None
+        except RuntimeError:                                    # being captured, and none is there yet
+            if C % 256 == 0 or x.shape[0] > _lib.SMALL_BMAX:
+                raise
+            ws = None                                           # (these run without one too)
         _lib.check(L.sq_q8_linear(q.data_ptr(), sc.data_ptr(), V, C, x.data_ptr(), _lib.DTYPES[x.dtype], x.stride(0),
                                   y.data_ptr(), _lib.DTYPES[y.dtype], y.stride(0), x.shape[0],
                                   None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(),
