@@ -514,13 +514,14 @@ static bool q8_mfma_ok(int C) { return C % 64 == 0 && (int64_t)C * 64 < ((int64_
 // Rows that are not whole 256-column chunks, us, exact-product kernel or (above 32 rows) decode + tile GEMM / these passes: 25 rows of
 // 141,347 x 1,408 348 / 47, of 9,823 x 3,456 102 / 29, 8 of 70,061 x 1,216 63 / 24.5.  A small grid is bound by the length of a wave's
 // chain, 0.8 us per 128 columns: 3 rows of 9,823 x 3,456 15.9 / 24, of 16,000 x 1,216 8.3 / 10.7, of 32,000 x 640 8.9 / 7.9, of 30,000 x 1,216
-// 15.1 / 12.1; 5 of 9,823 x 3,456 25.0 / 23.5; 64 of it 45.5 / 55, of 16,000 x 3,456 62 / 52, of 8,211 x 576 33 / 18.  A second pass: 100 rows of
+// 15.1 / 12.1; 5 of 9,823 x 3,456 25.0 / 24.2, of 4,096 x 1,408 10.2 / 12.3; 16 of 1,024 x 1,408 23.3 / 12.4; 64 of 9,823 x 3,456 45.5 / 55, of 16,000 x 3,456 62 / 52, of 8,211 x 576 33 / 18.  A second pass: 100 rows of
 // 30,000 x 1,216 41.3 / 41.9, of 32,000 x 640 33.6 / 27.6, of 50,000 x 3,520 203 / 106, 200 of 70,061 x 1,216 164 / 170.
 bool q8_mid(int V, int C, int B) {
     if (B <= 2 || !q8_mfma_ok(C)) return false;
     if (C % 256 == 0) return B <= Q8_MFMA_MAX_ROWS;
     if (B <= 4 || B > 64) return V >= 30000 && B <= 128;
-    return B <= 32 || V >= 16000 || C <= 2048;
+    if (B <= 8) return V >= 8000;
+    return V >= 1024 && (B <= 32 || V >= 16000 || C <= 2048);
 }
 size_t q8_mid_workspace(int V, int C, int B) { return q8_mid(V, C, B) ? (((size_t)B * C * 2) + 255) & ~(size_t)255 : 0; }
 
