@@ -44,13 +44,13 @@ static int fused_rounds(const sq_matrix& m) { return (m.W / fused_unit_dwords(m.
 
 // How a product is cut, nw = 0 where the other kernels are the faster ones.  Up to 768 rows, in blocks of up to 384 tokens; rows of
 // the weights in tiles of 32 tw, where a launch should fill the CUs once: what a workgroup takes hardly depends on how many run
-// beside it.  A tile of 64 / 96 / 128 / 160 rows x 333 tokens x 3584 columns takes 66 / 82 / 105 / 125 us with 16-bit tags of
-// width 8 (the weights below), 62 / 72 / 88 / 101 with 10-bit ones of width 4.  Decoded and multiplied in tiles, or in one pass over the tags where
+// beside it.  A tile of 64 / 96 / 128 / 160 rows x 333 tokens x 3584 columns takes 66 / 83 / 104 / 123 us with 16-bit tags of
+// width 8 (the weights below), 62 / 73 / 85 / 103 with 10-bit ones of width 4.  Decoded and multiplied in tiles, or in one pass over the tags where
 // that is the faster one (sq_mid.h), against here, us (d = 8, then d = 4):
 //   rows x columns    200 tokens                333                       512                       768
 //   12000 x 3584      75 / 57    58 / 46        79 / 66    71 / 62        79 / 77    69 / 60        92 / 89    84 / 80
 //   18944 x 3584      95 / 72    72 / 55        97 / 83   113 / 72       112 / 111   98 / 83       133 / 127  121 / 109
-//   25000 x 3584     105 / 90    73 / 77 (160)  118 / 109 114 / 97 (160)  143 / 186  124 / 149     210 / 225  180 / 192
+//   25000 x 3584     105 / 83    75 / 63       126 / 96  115 / 81       143 / 186  124 / 149     210 / 225  180 / 192
 //   37888 x 3584     177 / 106  104 / 79       234 / 130  154 / 102      263 / 216  209 / 164      301 / 246  245 / 206
 //   3584 x 18944      96 / 72    67 / 59       132 / 90   109 / 77       143 / 137  136 / 102      173 / 162  152 / 136
 // so two blocks of tokens need the last round of workgroups nearly full; a second round is for the widest tiles, where the other way
