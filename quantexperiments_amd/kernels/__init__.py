@@ -9,6 +9,7 @@ here computes on the CPU and nothing falls back to PyTorch ops.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import math
 
@@ -346,9 +347,16 @@ def build_stream(words: torch.Tensor, C: int, d: int, bits: int, row_mask=None, 
     return out.to(words.device), r.value, g.value
 
 
+def _on(dev):
+    """torch.cuda.device(dev), which takes 3 us to enter and leave, where dev is not the current device anyway."""
+    return contextlib.nullcontext() if torch.cuda.current_device() == dev.index else torch.cuda.device(dev)
+
+
 class _StreamPlan:
     """A stream that is planned but not written yet (sq_stream_plan_device): runs and groups as build_stream returns them, None
     runs for a format the load-time layouts do not cover."""
+
+    __slots__ = ("plan", "words", "book", "runs", "groups", "nbytes", "nscratch")
 
     def __init__(self, words: torch.Tensor, C: int, d: int, bits: int, row_mask, runs: int, row_book):
         L, dev = _lib.lib(), words.device
@@ -366,7 +374,7 @@ class _StreamPlan:
         counts = torch.empty(max(L.sq_stream_counts_bytes(R, C, d, bits, G), 1), dtype=torch.uint8, device=dev)
         nbytes, nscratch = ctypes.c_size_t(), ctypes.c_size_t()
         r, g = ctypes.c_int32(), ctypes.c_int32()
-        with torch.cuda.device(dev):
+        with _on(dev):
             rc = L.sq_stream_plan_device(words.data_ptr(), R, W, C, d, bits, G, None if self.book is None else self.book.data_ptr(),
                                          None if mask is None else mask.data_ptr(), runs, counts.data_ptr(), ctypes.byref(self.plan),
                                          ctypes.byref(nbytes), ctypes.byref(nscratch), ctypes.byref(r), ctypes.byref(g), _lib.stream_ptr(dev))
@@ -384,20 +392,27 @@ class _StreamPlan:
 
 def _fill_streams(plans) -> list:
     """(stream, runs, groups) of every plan, their buffers written side by side on the GPU (sq_stream_fill_stack_device)."""
+    if len(plans) == 1:                                         # (5 us less than a list of one: a tile-major copy takes 30)
+        p = plans[0]
+        if p.runs is None:
+            return [(None, 0, 0)]
+        dev = p.words.device
+        out, scratch = (torch.empty(max(k, 1), dtype=torch.uint8, device=dev) for k in (p.nbytes, p.nscratch))
+        with _on(dev):
+            _lib.check(_lib.lib().sq_stream_fill_device(p.plan, p.words.data_ptr(), None if p.book is None else p.book.data_ptr(), out.data_ptr(),
+                                                        scratch.data_ptr(), _lib.stream_ptr(dev)))
+        return [(out, p.runs, p.groups)]
     todo = [p for p in plans if p.runs is not None]
     outs, keep = {}, []
+    for p in todo:
+        outs[id(p)] = torch.empty(max(p.nbytes, 1), dtype=torch.uint8, device=p.words.device)
+        keep.append(torch.empty(max(p.nscratch, 1), dtype=torch.uint8, device=p.words.device))
     if todo:
-        dev = todo[0].words.device
-        new = lambda n: torch.empty(max(n, 1), dtype=torch.uint8, device=dev)
-        for p in todo:
-            outs[id(p)] = new(p.nbytes)
-            keep.append(new(p.nscratch))
-        ptrs = lambda ps: (ctypes.c_void_p * len(todo))(*ps)
-        with torch.cuda.device(dev):
-            _lib.check(_lib.lib().sq_stream_fill_stack_device(
-                len(todo), ptrs(p.plan.value for p in todo), ptrs(p.words.data_ptr() for p in todo),
-                ptrs(None if p.book is None else p.book.data_ptr() for p in todo), ptrs(outs[id(p)].data_ptr() for p in todo),
-                ptrs(k.data_ptr() for k in keep), _lib.stream_ptr(dev)))
+        dev, n = todo[0].words.device, len(todo)
+        rows = zip(*((p.plan.value, p.words.data_ptr(), None if p.book is None else p.book.data_ptr(), outs[id(p)].data_ptr(), k.data_ptr())
+                     for p, k in zip(todo, keep)))
+        with _on(dev):
+            _lib.check(_lib.lib().sq_stream_fill_stack_device(n, *((ctypes.c_void_p * n)(*r) for r in rows), _lib.stream_ptr(dev)))
     return [(outs[id(p)], p.runs, p.groups) if p.runs is not None else (None, 0, 0) for p in plans]
 
 
@@ -463,7 +478,7 @@ def dequant_stack(pieces, out: torch.Tensor, x: torch.Tensor | None = None) -> t
         raise ValueError(f"x must be bf16 [B, {C}] with unit column stride")
     xh = None if x is None else torch.empty(x.shape, dtype=torch.float16, device=dev)
     mats = _lib.matrix_array([p.descriptor() for p in pieces])
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.check(_lib.lib().sq_dequant_stack(mats, len(pieces), out.data_ptr(), None if x is None else x.data_ptr(),
                                                0 if x is None else x.stride(0) if x.shape[0] > 1 else C, 0 if x is None else x.shape[0],
                                                None if x is None else xh.data_ptr(), _lib.stream_ptr(dev)))
