@@ -232,7 +232,8 @@ constexpr int q8l_wave_bytes(int d) { return d * 2048 + (d - 1) * 256; }
 constexpr int q8l_lds_bytes(int nblk, int waves, int d, int xs) { return 2 * nblk * 16 * xs * 256 + waves * q8l_wave_bytes(d); }
 
 // NBLK 16-token blocks, WAVES waves per workgroup, ring of D steps per wave (one being multiplied, D - 1 in flight),
-// x chunks of XS steps (128 XS columns; the first 16 NBLK XS / 4 waves copy 4 / XS tokens of every chunk each)
+// x chunks of XS steps (128 XS columns; a copy moves 4 / XS tokens, so the first 4 NBLK XS waves make one of every chunk, or all
+// waves XI of them)
 // ANY_C: rows of any whole pairs of blocks (C % 64 == 0).  The steps behind the row's end copy its last pieces again and multiply
 // nothing.  Such rows ran on the exact-product kernel, so their block scales stay out of the fp16 weights: a matrix instruction takes
 // the 32 columns of one block (lane group g: columns 8 g .. 8 g + 7) and its sums, fp32, are multiplied by the block's scales.
@@ -257,18 +258,24 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel
     // activations: one copy instruction moves 1 KB = 4 / XS tokens of a chunk; the 16-byte piece p of token t is kept
     // at slot p ^ (t % 16), so the 16 lanes of a read clock (16 tokens, one piece) spread over 16 bank groups
     constexpr int TPI = 4 / XS, LPT = 64 / TPI;                 // tokens per instruction, lanes (= pieces) per token
-    uint32_t xsrc;
-    int xcol;                                                   // this lane's column in a chunk
-    {
-        const int rowx = wave * TPI + lane / LPT;
+    constexpr int XI = 16 * NBLK / TPI > WAVES ? 16 * NBLK / TPI / WAVES : 1;     // copies a wave makes of a chunk
+    uint32_t xsrc[XI];
+    int xcol[XI];                                               // this lane's column in a chunk
+#pragma unroll
+    for (int i = 0; i < XI; ++i) {
+        const int rowx = (wave * XI + i) * TPI + lane / LPT;
         const int piece = (lane % LPT) ^ (rowx & 15);
-        xcol = piece * 8;
-        xsrc = (uint32_t)(min(rowx, a.B - 1) * a.ldxh + (ANY_C ? 0 : xcol));
+        xcol[i] = piece * 8;
+        xsrc[i] = (uint32_t)(min(rowx, a.B - 1) * a.ldxh + (ANY_C ? 0 : xcol[i]));
     }
-    const bool xo = wave * TPI < 16 * NBLK;                     // this wave takes part in the x copies
+    const bool xo = wave * XI * TPI < 16 * NBLK;                // this wave takes part in the x copies
     auto copy_x = [&](int c) {
-        const uint32_t at = ANY_C ? (uint32_t)min(c * (XS * 128) + xcol, C - 8) : (uint32_t)(c * (XS * 128));
-        if (xo) __builtin_amdgcn_global_load_lds((gptr_t)(a.xh + at + xsrc), (lptr_t)(xs + (c & 1) * XBUF + wave * TPI * XPITCH), 16, 0, 0);
+        if (xo)
+#pragma unroll
+            for (int i = 0; i < XI; ++i) {
+                const uint32_t at = ANY_C ? (uint32_t)min(c * (XS * 128) + xcol[i], C - 8) : (uint32_t)(c * (XS * 128));
+                __builtin_amdgcn_global_load_lds((gptr_t)(a.xh + at + xsrc[i]), (lptr_t)(xs + (c & 1) * XBUF + (wave * XI + i) * TPI * XPITCH), 16, 0, 0);
+            }
     };
     // weights: instruction n of a step fills rows 8 n .. 8 n + 7; lane i lands in row 8 n + i / 8, slot i % 8 and
     // fetches the piece the swizzle keeps there
@@ -303,7 +310,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel
     // S(c) goes right before W(2c); step s starts (even s: after the wait and the barrier, then X(s/2 + 1)) with the
     // refill of step s + D - 1.  Waits count the operations that may stay in flight:
     //   even s (needs X, S, W of its chunk):  D = 3: W(s+1) -> 2;           D = 4: W(s+1) S W(s+2) -> 5
-    //   odd s (needs W(s)):  D = 3: X S W(s+1) W(s+2) -> 5 + x;  D = 4: S W(s+1) X W(s+2) S W(s+3) -> 8 + x
+    //   odd s (needs W(s)):  D = 3: X S W(s+1) W(s+2) -> 5 + x;  D = 4: S W(s+1) X W(s+2) S W(s+3) -> 8 + x   (x: this wave's XI copies)
     // and fall back to "everything" near the end of the row, where refills stop.
     auto refill = [&](int f) {
         if (f < nsteps) {
@@ -334,7 +341,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel
         } else {
             refill(s + D - 1);
             if (s + D - 1 < nsteps) {
-                if (xo) __builtin_amdgcn_s_waitcnt(q8_vmcnt(D == 3 ? 6 : 9));
+                if (xo) __builtin_amdgcn_s_waitcnt(q8_vmcnt((D == 3 ? 5 : 8) + XI));
                 else __builtin_amdgcn_s_waitcnt(q8_vmcnt(D == 3 ? 5 : 8));
             } else {
                 __builtin_amdgcn_s_waitcnt(q8_vmcnt(0));
@@ -514,14 +521,15 @@ static bool q8_mfma_ok(int C) { return C % 64 == 0 && (int64_t)C * 64 < ((int64_
 // Rows that are not whole 256-column chunks, us, exact-product kernel or (above 32 rows) decode + tile GEMM / these passes: 25 rows of
 // 141,347 x 1,408 348 / 47, of 9,823 x 3,456 102 / 29, 8 of 70,061 x 1,216 63 / 24.5.  A small grid is bound by the length of a wave's
 // chain, 0.8 us per 128 columns: 3 rows of 9,823 x 3,456 15.9 / 24, of 16,000 x 1,216 8.3 / 10.7, of 32,000 x 640 8.9 / 7.9, of 30,000 x 1,216
-// 15.1 / 12.1; 5 of 9,823 x 3,456 25.0 / 24.2, of 4,096 x 1,408 10.2 / 12.3; 16 of 1,024 x 1,408 23.3 / 12.4; 64 of 9,823 x 3,456 45.5 / 55, of 16,000 x 3,456 62 / 52, of 8,211 x 576 33 / 18.  A second pass: 100 rows of
+// 15.1 / 12.1; 5 of 9,823 x 3,456 25.2 / 22.6, of 8,192 x 1,408 10.4 / 11.7; 16 of 1,024 x 1,408 23.3 / 12.4; 64 of 9,823 x 3,456 45.5 / 39,
+// of 16,000 x 3,456 59.5 / 38, of 8,211 x 576 33 / 18.  A second pass: 100 rows of
 // 30,000 x 1,216 41.3 / 41.9, of 32,000 x 640 33.6 / 27.6, of 50,000 x 3,520 203 / 106, 200 of 70,061 x 1,216 164 / 170.
 bool q8_mid(int V, int C, int B) {
     if (B <= 2 || !q8_mfma_ok(C)) return false;
     if (C % 256 == 0) return B <= Q8_MFMA_MAX_ROWS;
     if (B <= 4 || B > 64) return V >= 30000 && B <= 128;
-    if (B <= 8) return V >= 8000;
-    return V >= 1024 && (B <= 32 || V >= 16000 || C <= 2048);
+    if (B <= 8) return V >= 9000;
+    return V >= 1024 && (B <= 32 || V >= 8000 || C <= 2048);
 }
 size_t q8_mid_workspace(int V, int C, int B) { return q8_mid(V, C, B) ? (((size_t)B * C * 2) + 255) & ~(size_t)255 : 0; }
 
@@ -567,13 +575,26 @@ int launch_q8_mid(const int8_t* q, const uint16_t* sc, int V, int C, const void*
         if (!raised) {
             for (void (*k)(Q8MfmaArgs) : {q8_mfma_kernel<1, 8, 3, 2, false>, q8_mfma_kernel<2, 16, 3, 2, false>, q8_mfma_kernel<2, 8, 3, 1, false>,
                                           q8_mfma_kernel<4, 16, 3, 1, false>, q8_mfma_kernel<1, 8, 3, 2, true>, q8_mfma_kernel<2, 16, 3, 2, true>,
-                                          q8_mfma_kernel<2, 8, 3, 1, true>, q8_mfma_kernel<4, 16, 3, 1, true>})
+                                          q8_mfma_kernel<2, 8, 3, 1, true>, q8_mfma_kernel<4, 16, 3, 1, true>, q8_mfma_kernel<4, 8, 3, 1, false>,
+                                          q8_mfma_kernel<4, 8, 3, 1, true>})
                 (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
             (void)hipGetLastError();
             raised = true;
         }
         const bool any = C % 256 != 0;
-        if (a.B > 32)                                           // 33-64 rows: 16 waves share 128-column chunks of 64 tokens
+        // Small heads: half the waves per workgroup, each making twice the copies of x, spread the same waves over twice the CUs (a wave's
+        // chain of LDS reads, conversions and matrix instructions is what they take).  us, before / so: 16 rows of 9,728 x 3,584 19.7 /
+        // 17.8, of 10,000 x 2,048 12.7 / 12.1, of 30,000 x 2,048 14.3 / 14.8; 64 rows of 9,728 x 3,584 44.7 / 30.5, of 32,000 x 3,584 45.9 / 31.9,
+        // of 60,000 x 2,048 31.0 / 37.4.
+        const int n8 = (tasks + 7) / 8;
+        const bool small = a.B > 32 ? n8 <= cus : n8 <= cus / 2;
+        if (small && a.B > 32)
+            go(any ? q8_mfma_kernel<4, 8, 3, 1, true> : q8_mfma_kernel<4, 8, 3, 1, false>, 8, q8l_lds_bytes(4, 8, 3, 1));
+        else if (small && a.B > 16)
+            go(any ? q8_mfma_kernel<2, 4, 3, 1, true> : q8_mfma_kernel<2, 4, 3, 1, false>, 4, q8l_lds_bytes(2, 4, 3, 1));
+        else if (small)
+            go(any ? q8_mfma_kernel<1, 4, 3, 2, true> : q8_mfma_kernel<1, 4, 3, 2, false>, 4, q8l_lds_bytes(1, 4, 3, 2));
+        else if (a.B > 32)                                           // 33-64 rows: 16 waves share 128-column chunks of 64 tokens
             go(any ? q8_mfma_kernel<4, 16, 3, 1, true> : q8_mfma_kernel<4, 16, 3, 1, false>, 16, q8l_lds_bytes(4, 16, 3, 1));
         else if (a.B > 16 && x128)
             go(any ? q8_mfma_kernel<2, 8, 3, 1, true> : q8_mfma_kernel<2, 8, 3, 1, false>, 8, q8l_lds_bytes(2, 8, 3, 1));
