@@ -524,10 +524,12 @@ static bool q8_mfma_ok(int C) { return C % 64 == 0 && (int64_t)C * 64 < ((int64_
 // 15.1 / 12.1; 5 of 9,823 x 3,456 25.2 / 22.6, of 8,192 x 1,408 10.4 / 11.7; 16 of 1,024 x 1,408 23.3 / 12.4; 64 of 9,823 x 3,456 45.5 / 39,
 // of 16,000 x 3,456 59.5 / 38, of 8,211 x 576 33 / 18.  A second pass: 100 rows of
 // 30,000 x 1,216 41.3 / 41.9, of 32,000 x 640 33.6 / 27.6, of 50,000 x 3,520 203 / 106, 200 of 70,061 x 1,216 164 / 170.
+// 3 rows of 105,038 x 3,392, which the 256 MB last-level cache does not hold from call to call: 86.5 / 90.5; 5 take two passes there.
 bool q8_mid(int V, int C, int B) {
     if (B <= 2 || !q8_mfma_ok(C)) return false;
     if (C % 256 == 0) return B <= Q8_MFMA_MAX_ROWS;
-    if (B <= 4 || B > 64) return V >= 30000 && B <= 128;
+    if (B <= 4) return V >= 30000 && (int64_t)V * C <= (int64_t)240 << 20;
+    if (B > 64) return V >= 30000 && B <= 128;
     if (B <= 8) return V >= 9000;
     return V >= 1024 && (B <= 32 || V >= 8000 || C <= 2048);
 }
