@@ -1251,20 +1251,14 @@ int stream_plan_device(const uint32_t* tags, int R, int W, int C, int d, int bit
     return SQ_OK;
 }
 
-int stream_fill_device(const StreamFill* fills, int n, hipStream_t s) {
-    hipError_t e = hipSuccess;
-    bool wait = false;
-    for (int i = 0; i < n && e == hipSuccess; ++i) {
+// Enqueues what writes the buffers.
+static int launch_stream_fill(const StreamFill* fills, int n, hipStream_t s) {
+    for (int i = 0; i < n; ++i) {
         const StreamDevicePlan& D = *fills[i].plan;
         if (D.tiled) continue;
-        e = hipMemcpyAsync(fills[i].scratch, D.upload.data(), D.upload.size() * 4, hipMemcpyHostToDevice, s);
-        wait = true;
+        const hipError_t e = hipMemcpyAsync(fills[i].scratch, D.upload.data(), D.upload.size() * 4, hipMemcpyHostToDevice, s);
+        if (e != hipSuccess) return fail(SQ_ELAUNCH, "sq_stream_fill_device: %s", hipGetErrorString(e));
     }
-    if (wait) {                                                  // (the plans may be freed as soon as this call returns)
-        const hipError_t w = hipStreamSynchronize(s);
-        if (e == hipSuccess) e = w;
-    }
-    if (e != hipSuccess) return fail(SQ_ELAUNCH, "sq_stream_fill_device: %s", hipGetErrorString(e));
     StreamFillStack stack{};
     int wgs = 0;
     size_t lds = 0;
@@ -1320,6 +1314,15 @@ int stream_fill_device(const StreamFill* fills, int n, hipStream_t s) {
     }
     fill();
     return check_launch("sq_stream_fill_device");
+}
+
+// The buffers are whole when this returns: the caller may free the plans, the scratch and the tags and may multiply on any stream.
+// (Also where a launch failed: what was enqueued before it still reads the plans and writes the buffers.)
+int stream_fill_device(const StreamFill* fills, int n, hipStream_t s) {
+    const int rc = launch_stream_fill(fills, n, s);
+    const hipError_t e = hipStreamSynchronize(s);
+    if (rc || e == hipSuccess) return rc;
+    return fail(SQ_ELAUNCH, "sq_stream_fill_device: %s", hipGetErrorString(e));
 }
 
 void stream_plan_free(StreamDevicePlan* D) { delete D; }

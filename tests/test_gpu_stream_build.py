@@ -8,8 +8,9 @@ import pytest
 import torch
 
 from quantexperiments_amd import _lib
-from quantexperiments_amd.kernels import build_stream
+from quantexperiments_amd.kernels import build_stream, linear_small, prepare_stack
 from quantexperiments_amd.packed import pack_bits
+from tests.helpers import rand_x, rel_max_err, synth, to_device
 
 pytestmark = pytest.mark.gpu
 
@@ -130,3 +131,32 @@ def test_unknown_codebooks_are_refused_before_a_launch(G):
     assert bool((counts == -1).all())
     with pytest.raises(ValueError, match="row_book"):
         build_stream(words, C, 8, bits, row_book=(book, G))
+
+
+@pytest.mark.parametrize("rows,C,d,bits,G,M", [((300,), 1024, 8, 16, 1, 1), ((600, 65, 66), 3584, 8, 16, 1, 1), ((130, 40), 512, 8, 14, 2, 3),
+                                               ((40,), 8 * 4069, 8, 13, 1, 1), ((300,), 3584, 4, 12, 1, 1), ((300,), 896, 4, 8, 2, 1)])
+def test_layouts_are_whole_when_they_are_handed_back(rows, C, d, bits, G, M):
+    """Built under one stream, multiplied on another that waits for nothing."""
+    ss = [synth(R, C, d, bits, G, M, seed=R) for R in rows]
+    lins = [to_device(s, stream=False) for s in ss]             # (the tensors themselves, in place before the side stream begins)
+    x = rand_x(1, C, torch.float16, seed=1).cuda()
+    y = torch.zeros(1, sum(rows), device="cuda")
+    torch.cuda.synchronize()
+    built = []
+    with torch.cuda.stream(side := torch.cuda.Stream()):
+        if len(lins) == 1:
+            lins[0].wants_stream = d == 8
+            lins[0].build_stream()
+            built.append(side.query())
+            lins[0].stream_tiled = d == 4
+        else:
+            for lin in lins:
+                lin.wants_stream = True
+            prepare_stack(lins)
+            built.append(side.query())
+    assert built == [True] and all(lin.stream is not None for lin in lins)
+    with torch.cuda.stream(torch.cuda.Stream()):
+        linear_small(lins, x, y)
+    torch.cuda.synchronize()
+    want = np.concatenate([x.cpu().double().numpy() @ s.decode().astype(np.float64).T for s in ss], axis=1)
+    assert rel_max_err(y.cpu().numpy(), want) < 1e-5            # (exact products, fp32 sums)
