@@ -15,15 +15,3 @@ def pytest_configure(config):
 @pytest.fixture(scope="session")
 def golden_dir():
     return ROOT / "tests" / "golden"
-
-
-@pytest.fixture(scope="module", autouse=True)
-def _device_memory_given_back():
-    """torch keeps what a file's tests freed; the next file begins with an empty cache, as when it runs alone (how long an allocation
-    takes decides what two threads of a test get to do beside each other)."""
-    yield
-    import sys
-    torch = sys.modules.get("torch")
-    if torch is not None and torch.cuda.is_initialized():
-        torch.cuda.synchronize()
-        torch.cuda.empty_cache()

@@ -55,27 +55,31 @@ def test_second_thread_replaces_workspace_and_matrices():
     ps = core.PackedShards([to_device(synth(96, 1024, 8, 16, seed=1)), to_device(synth(300, 1024, 8, 16, seed=2))])
     x = rand_x(2, 1024, torch.bfloat16, seed=3).cuda()
     want, dev = ps.forward(x), x.device
-    size, others, stop = _Workspace.get(1, dev).numel(), [], threading.Event()
+    size, others = _Workspace.get(1, dev).numel(), []
+    called, replaced, ys = threading.Semaphore(0), [], []
 
     def replace():
         for k in range(1, 25):
+            if not called.acquire(timeout=60):                  # (one replacement per call at least, beside the calls that follow)
+                return
             _Workspace.get(size + (k << 20), dev)               # (same stream: torch's default one on both threads)
             ps.rls[k & 1].row_scale = ps.rls[k & 1].row_scale.clone()
             others.append(torch.full((size + (k << 20),), 7, dtype=torch.uint8, device=dev))
-        stop.set()
+            replaced.append(len(ys))
 
     interval = sys.getswitchinterval()
     sys.setswitchinterval(1e-5)
     try:
         t = threading.Thread(target=replace)
         t.start()
-        ys = []
-        while not stop.is_set() and len(ys) < 20000:
+        while t.is_alive() and len(ys) < 20000:
             ys.append(ps.forward(x))
+            called.release()
         t.join()
     finally:
         sys.setswitchinterval(interval)
-    assert len(ys) > 0 and all(torch.equal(y, want) for y in ys[:: max(1, len(ys) // 200)] + ys[-1:])
+    assert len(replaced) == 24 and replaced[0] >= 1 and len(ys) >= 24
+    assert all(torch.equal(y, want) for y in ys[:: max(1, len(ys) // 200)] + ys[-1:])
     assert all(bool((o == 7).all()) for o in others)
 
 
