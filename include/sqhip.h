@@ -88,7 +88,8 @@ int sq_linear_small(const sq_matrix* mats, int32_t n_mats, const void* x, int x_
  * counterpart in the reference (whose launchers grow torch buffers on demand).  Pieces and row counts whose workspace
  * (sq_workspace_bytes(mats, n_mats, B, 0)) exceeds the array are refused with SQ_EWORKSPACE, except stacks with column orders
  * that need so much for their decoded weights only, at up to 10 rows or with C % 64 != 0: those run on the decode-time
- * kernel, whose results may differ from sq_linear_small's in the order of fp32 additions.  Nothing is allocated or freed,
+ * kernel, whose results may differ from sq_linear_small's in the order of fp32 additions, and d = 4 pieces whose rows one launch
+ * takes whole as well, which then differ in the same way (sq_linear_small with too small a workspace too).  Nothing is allocated or freed,
  * here or in anything it calls.  All calls on one GPU share that GPU's array: calls that overlap in time on one GPU
  * (two streams, two threads) race; calls on one stream are safe. */
 #define SQ_NOALLOC_SCRATCH_BYTES (48u << 20)

@@ -188,7 +188,9 @@ int sq_linear_small_noalloc(const sq_matrix* mats, int32_t n_mats, const void* x
     if (B == 0 || n_mats == 0) return SQ_OK;
     const size_t inner = (size_t)SQ_NOALLOC_SCRATCH_BYTES - SQ_WS_HEADER;
     // a stack whose decoded weights do not fit takes the decode-time kernel instead (as it does where x is not aligned for the other)
-    const size_t small = small_workspace(mats, n_mats, B), decoded = small_gemm_route_workspace(mats, n_mats, B);
+    size_t small = small_workspace(mats, n_mats, B);
+    if (small > inner) small = small_workspace_least(mats, n_mats, B);
+    const size_t decoded = small_gemm_route_workspace(mats, n_mats, B);
     const bool in_place = decoded > inner && (B <= NOALLOC_ROWS_IN_PLACE || mats[0].C % 64);
     const bool route = !in_place && small_takes_gemm_route(mats, n_mats, B, x, ldx);
     const size_t need = in_place ? small : std::max(small, decoded > inner ? gemm_workspace_without_mid(mats, n_mats, B) : decoded);

@@ -131,6 +131,7 @@ bool small_fuses_silu(const sq_matrix* mats, int n, int B);
 int launch_small_silu(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* act, int64_t ld_act, int B,
                       void* sums, hipStream_t s, const sq_producer* from = nullptr);
 size_t small_workspace(const sq_matrix* mats, int n, int B);
+size_t small_workspace_least(const sq_matrix* mats, int n, int B);     // what launch_small can do with
 // some piece runs the tag-stream kernel, whose partial sums live in the workspace header (`sums` above)
 bool small_uses_sums(const sq_matrix* mats, int n);
 int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype,

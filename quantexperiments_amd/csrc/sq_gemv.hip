@@ -183,6 +183,26 @@ static MmaPlan mma_plan(const sq_matrix& m, int B) {
     return best;
 }
 
+// The widest variant, whose waves hold all the rounds their registers can, where it takes a row in one launch and mma_plan's does not
+// (KW = 0: it does not): up to 8192 columns, from 6145 or, beside 128 KB of codebooks, 5633.
+static MmaPlan mma_whole_row(const sq_matrix& m, int B) {
+    const MmaPlan none{0, 0, 0, 0};
+    const size_t tab = mma_table_bytes(m);
+    if (!tab || B > 16 || m.d != 4 || mma_plan(m, B).ks == 1) return none;
+    const int ud = unit_dwords(m.bits), tpu = ud * 32 / m.bits, spu = tpu / (8 / m.d), rw = 32 / spu;
+    const int need = ((m.W / ud + 3) / 4 + rw - 1) / rw;
+    const size_t per_wave = std::max((size_t)64 * 16 * mma_pft(rw, 1), (size_t)mma_x_stage_bytes(tpu * m.d, mma_x_tokens_min(1)));
+    if (need > (int)std::min<size_t>(mma_waves_max(rw * spu, true), (160 * 1024 - tab - 16) / per_wave)) return none;
+    return MmaPlan{rw, 1, need, 1};
+}
+
+// Such a launch is slow to begin (its waves fetch all their activations first), column slices cost a reduction launch for every piece
+// and the sums' way through memory, three of them share few rows' tiles badly.  us, slices / one launch, 8 rows: one piece of 8192 x 8192 with 8-, 10- and 12-bit
+// tags 11.8 / 11.9, 12.0 / 13.5, 12.1 / 13.5, of 14336 rows 14.6 / 15.2, 15.9 / 17.5, 15.3 / 17.6, of 20480 17.9 / 16.7, 19.4 / 19.4, 19.0 / 19.5,
+// of 28672 21.6 / 19.9, 23.5 / 23.1, 23.2 / 23.0; two of 4096 rows 13.9 / 12.1, 14.7 / 13.5, 14.3 / 13.5, two of 18944 29.8 / 25.6, 32.0 / 29.5,
+// 31.3 / 29.8; four books of 12-bit tags in three slices, 8192 x 6272 14.4 / 13.0, two of 8192 rows 23.5 / 16.7.
+static bool mma_whole_row_pays(const sq_matrix& m0, int cnt, const MmaPlan& slices) { return cnt > 1 || m0.R >= 20000 || slices.ks > 2; }
+
 // For pieces that cannot share one pass (formats or lengths differ), and for the workspace of those that can: passes of 32 rows
 // through the matrix-core decode kernel against decode + tile GEMM (7B layer): 77 us per pass
 // against 600-640 us when the codebook sits in LDS (d = 4), 201 us per pass when its gathers go to L2.  A
@@ -204,15 +224,19 @@ static size_t mma_part_bytes(const sq_matrix& m, int B) {
     return pl.ks > 1 ? ((((size_t)pl.ks * B * m.R * 4) + 255) & ~(size_t)255) : 0;
 }
 
-size_t small_workspace(const sq_matrix* mats, int n, int B) {
+// tight: the pieces that can run without partial sums do
+static size_t small_need(const sq_matrix* mats, int n, int B, bool tight) {
     size_t tot = 0;
     for (int i = 0; i < n; ++i) {
         if (stream_rows(mats[i], B)) continue;                   // its partial sums live in the workspace header
-        if (mma_shape(mats[i])) tot += mma_part_bytes(mats[i], B);
+        if (mma_shape(mats[i])) tot += tight && mma_whole_row(mats[i], B).KW ? 0 : mma_part_bytes(mats[i], B);
         else if (mats[i].perms && fast_shape(mats[i])) tot += xp_bytes(mats[i], B);
     }
     return tot;
 }
+
+size_t small_workspace(const sq_matrix* mats, int n, int B) { return small_need(mats, n, B, false); }
+size_t small_workspace_least(const sq_matrix* mats, int n, int B) { return small_need(mats, n, B, true); }
 
 bool small_uses_sums(const sq_matrix* mats, int n) {
     for (int i = 0; i < n; ++i)
@@ -239,11 +263,15 @@ static bool mma_fuses_silu(const sq_matrix* mats, int n, int B, const void* x, i
 }
 
 // Pieces [0, cnt) share format and row length: one persistent launch (+ one reduction per piece if ks > 1).  act: mma_fuses_silu
-// holds for them.
+// holds for them.  whole: the workspace has no room for partial sums that mma_whole_row can do without.
 static int launch_mma_group(const sq_matrix* mats, int cnt, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype,
-                            int64_t ldy, int B, char* ws, size_t& ws_off, int cus, hipStream_t s, bool act = false) {
+                            int64_t ldy, int B, char* ws, size_t& ws_off, int cus, hipStream_t s, bool act = false, bool whole = false) {
     const sq_matrix& m0 = mats[0];
-    const MmaPlan pl = mma_plan(m0, B);
+    MmaPlan pl = mma_plan(m0, B);
+    if (pl.ks > 1 && !act && (whole || mma_whole_row_pays(m0, cnt, pl))) {
+        const MmaPlan one = mma_whole_row(m0, B);
+        if (one.KW) pl = one;
+    }
     MmaArgs a;
     a.n = cnt;
     a.x = (const uint16_t*)x; a.ldx = ldx; a.y = y; a.ldy = ldy; a.B = B; a.x_dtype = x_dtype; a.y_dtype = y_dtype;
@@ -366,7 +394,8 @@ int launch_small_silu(const sq_matrix* mats, int n, const void* x, int x_dtype, 
 int launch_small(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype,
                  int64_t ldy, int B, void* ws, size_t ws_bytes, void* sums, hipStream_t s, const sq_producer* from) {
     if (from && !small_fuses_producer(mats, n, B)) return fail(SQ_EUNSUPPORTED, "sq_linear_small_from: no fused kernel for this stack");
-    if (small_workspace(mats, n, B) > ws_bytes)
+    const bool tight = small_workspace(mats, n, B) > ws_bytes;
+    if (tight && small_workspace_least(mats, n, B) > ws_bytes)
         return fail(SQ_EWORKSPACE, "sq_linear_small: workspace %zu < %zu", ws_bytes, small_workspace(mats, n, B));
     const int cus = device_cus();
     const bool x_ok = (B == 1 || ldx % 8 == 0) && (((uintptr_t)x & 15) == 0);   // 16-byte activation loads
@@ -395,7 +424,7 @@ int launch_small(const sq_matrix* mats, int n, const void* x, int x_dtype, int64
             if (segs_fits(mats + i, j - i, B, cus)) {
                 int rc = launch_segs_group(mats + i, j - i, x, x_dtype, ldx, y, y_dtype, ldy, B, cus, s);
                 if (rc) return rc;
-                for (int k = i; k < j; ++k) ws_off += mma_part_bytes(mats[k], B);   // (what small_workspace counted for them)
+                ws_off += small_need(mats + i, j - i, B, tight);     // (what was counted for them)
                 i = j;
                 continue;
             }
@@ -405,7 +434,7 @@ int launch_small(const sq_matrix* mats, int n, const void* x, int x_dtype, int64
             while (j < n && j - i < GEMV_MAX_PIECES && mma_shape(mats[j]) && mats[j].bits == m0.bits && mats[j].d == m0.d &&
                    mats[j].W == m0.W && mats[j].G == m0.G && mats[j].R > 0)
                 ++j;
-            int rc = launch_mma_group(mats + i, j - i, x, x_dtype, ldx, y, y_dtype, ldy, B, (char*)ws, ws_off, cus, s);
+            int rc = launch_mma_group(mats + i, j - i, x, x_dtype, ldx, y, y_dtype, ldy, B, (char*)ws, ws_off, cus, s, false, tight);
             if (rc) return rc;
             i = j;
             continue;
@@ -416,9 +445,7 @@ int launch_small(const sq_matrix* mats, int n, const void* x, int x_dtype, int64
         if (pl.TS == 0) {
             int rc = launch_small_generic(mats + i, 1, x, x_dtype, ldx, y, y_dtype, ldy, B, s);
             if (rc) return rc;
-            if (stream_rows(m0, B)) {}
-            else if (mma_shape(m0)) ws_off += mma_part_bytes(m0, B);
-            else if (m0.perms && fast_shape(m0)) ws_off += xp_bytes(m0, B);
+            ws_off += small_need(mats + i, 1, B, tight);
             ++i;
             continue;
         }

@@ -514,15 +514,21 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
 // op 0: launch; op 1: workgroups of `threads` threads and `smem` bytes of LDS that fit on one CU
 template <int BITS, int D, int RW, int NT>
 static inline int mma_inst(int op, const MmaArgs& a, int grid, int threads, size_t smem, hipStream_t s) {
-    // (with its codebooks in LDS, d = 4, a wave never takes the most rounds it could: see mma_plan)
-    constexpr bool LDS = D == 4 && !(NT == 1 && RW * ((unit_of<BITS>::UD * 32 / BITS) / (8 / D)) > 16);
+    // (the widest variant with codebooks in LDS is for rows that only it takes in one launch, which have no fused SiLU: see mma_whole_row)
+    constexpr bool LDS = D == 4, WIDEST = NT == 1 && RW * ((unit_of<BITS>::UD * 32 / BITS) / (8 / D)) > 16;
     void (*k)(MmaArgs) = rows_mfma_kernel<BITS, D, RW, NT, false>;
     if constexpr (LDS) {
-        if (a.table_bytes) k = a.act ? rows_mfma_kernel<BITS, D, RW, NT, true, true> : rows_mfma_kernel<BITS, D, RW, NT, true>;
+        if (a.table_bytes) k = rows_mfma_kernel<BITS, D, RW, NT, true>;
         if constexpr (NT == 1)
-            if (a.xt == 8 && a.table_bytes) k = a.act ? rows_mfma_kernel<BITS, D, RW, NT, true, true, 8> : rows_mfma_kernel<BITS, D, RW, NT, true, false, 8>;
+            if (a.xt == 8 && a.table_bytes) k = rows_mfma_kernel<BITS, D, RW, NT, true, false, 8>;
+        if constexpr (!WIDEST) {
+            if (a.table_bytes && a.act) k = rows_mfma_kernel<BITS, D, RW, NT, true, true>;
+            if constexpr (NT == 1)
+                if (a.xt == 8 && a.table_bytes && a.act) k = rows_mfma_kernel<BITS, D, RW, NT, true, true, 8>;
+        }
     }
-    if (a.table_bytes && !LDS) return fail(SQ_EUNSUPPORTED, "sq_linear_small: no matrix-core kernel for %d rounds and codebooks in LDS", RW);
+    if (a.table_bytes && (!LDS || (WIDEST && a.act)))
+        return fail(SQ_EUNSUPPORTED, "sq_linear_small: no matrix-core kernel for %d rounds and codebooks in LDS", RW);
     if (op == 1) {
         static std::mutex mu;
         static std::unordered_map<uint64_t, int> cache;

@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 import torch
 
+from quantexperiments_amd import _lib
 from quantexperiments_amd.kernels import linear_small
 from tests.helpers import rand_x, rel_max_err, synth, to_device
 
@@ -24,3 +25,27 @@ def test_against_the_oracle(R, C, bits, G):
         # products of fp16 values are exact in fp32; C sums of them round at 2^-24 of a partial sum, in any order: below
         # sqrt(C) 2^-24 of the largest result by a wide margin
         assert rel_max_err(y.cpu().numpy(), x.half().float().numpy().astype(np.float64) @ w.T) < 1e-5, B
+
+
+@pytest.mark.parametrize("C,bits,G", [(5760, 12, 4), (6208, 12, 1), (6912, 12, 4), (7168, 8, 1), (7680, 10, 4), (8192, 12, 2), (8192, 10, 1), (8192, 8, 1)])
+@pytest.mark.parametrize("rows", [(20001,), (50, 17, 300)])
+def test_rows_that_one_launch_takes_whole(rows, C, bits, G):
+    """Stacks and tall matrices, and any of these where the workspace has no room for partial sums (none at all here)."""
+    L, dev = _lib.lib(), torch.device("cuda", torch.cuda.current_device())
+    ss = [synth(R, C, 4, bits, G, 1, seed=R + C) for R in rows]
+    lins = [to_device(s) for s in ss]
+    w = torch.cat([torch.from_numpy(s.decode()).cuda().double() for s in ss])
+    offs = [sum(rows[:i]) for i in range(len(rows))]
+    for B, dtype in ((2, torch.bfloat16), (5, torch.float16), (8, torch.bfloat16), (9, torch.float16), (16, torch.bfloat16)):
+        x = rand_x(B, C, dtype, seed=B).cuda()
+        want = (x.half().double() @ w.T).cpu().numpy()
+        y = torch.full((B, sum(rows)), float("nan"), device="cuda")
+        linear_small(lins, x, y)
+        assert rel_max_err(y.cpu().numpy(), want) < 1e-5, B         # (see above)
+        for off, lin in ((offs, lins), ([0], lins[:1])):
+            mats = _lib.matrix_array([m.descriptor(o) for m, o in zip(lin, off)])
+            n = sum(m.R for m in lin)
+            y.fill_(float("nan"))
+            _lib.check(L.sq_linear_small(mats, len(lin), x.data_ptr(), _lib.DTYPES[dtype], C, y.data_ptr(), _lib.SQ_F32, sum(rows), B, None, 0,
+                                         _lib.stream_ptr(dev)))
+            assert rel_max_err(y[:, :n].cpu().numpy(), want[:, :n]) < 1e-5 and bool(y[:, n:].isnan().all()), B
