@@ -240,9 +240,10 @@ int sq_codebook_balance_books(const int32_t* tags_host, int32_t R, int32_t W, in
 
 /* The load-time layouts built on the GPU, from tags that are already there: the same bytes as the host routines above
  * (which stay for tags in host memory), in milliseconds instead of a fraction of a second per matrix.  tags, row_book,
- * counts, out, scratch and remap are DEVICE pointers, row_mask_host and remap_out_host HOST pointers; the balance calls, the plan
- * calls (for a slice stream) and the fill calls synchronise the stream (they are for load time and never run under graph capture):
- * when a fill call returns its buffers are whole for every stream, and its tags, scratch and plans are free.  Every entry
+ * counts, out, scratch and remap are DEVICE pointers, row_mask_host and remap_out_host HOST pointers; the balance calls, and the plan
+ * and fill calls of a slice stream, synchronise the stream (they are for load time and never run under graph capture): when such a
+ * fill call returns its buffers are whole for every stream, and its tags, scratch and plans are free.  The fill of tile-major copies
+ * alone is enqueued like a product: tags and buffers stay, and other streams wait for this one.  Every entry
  * of row_book is below G: the plan and balance calls refuse a row_book that names another codebook (SQ_EINVAL, nothing is
  * launched); the other two take what it holds modulo G.
  *   sq_stream_plan_device   makes the plan of the buffer sq_stream_build_books would write (its layout, and for the d = 4

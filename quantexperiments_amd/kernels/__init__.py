@@ -88,9 +88,9 @@ def _check_row_ids(ids: torch.Tensor, R: int, n: int, what: str) -> None:
 
 
 class PackedLinear(torch.nn.Module):
-    """A block linear run from packed tensors.  Its load-time layout (build_stream, or prepare_stack for stream="later") is waited for:
-    a matrix built under one stream may be used on any other as soon as the call that builds its layout has returned.  A matrix
-    without one (stream=False, formats no layout covers) is ordered like any tensor, by the stream it was made on."""
+    """A block linear run from packed tensors.  A slice stream (codebooks beyond LDS) is waited for: the matrix may be used on any
+    stream as soon as the call that builds it (the constructor, or prepare_stack for stream="later") has returned.  Without one,
+    the matrix is ordered like any tensor, by the stream it was made on."""
 
     _native = None              # what the native call path keeps of this matrix, made at its first call
 
