@@ -57,8 +57,11 @@ constexpr int fused_stage_bytes(int NW, int TW, int S) { return S * (FUSED_RN * 
 // LDS that a tile's tags of one round take: a unit per lane, 16 bytes apart (a 12-byte load to LDS leaves its lanes 16 bytes apart
 // too), the fifth dwords of 20-byte units behind them
 constexpr int fused_tag_bytes(int bits) { return bits == 10 ? 1280 : 1024; }
+// d = 4: eight zero bytes behind the stages for the units past a row's end.  With two books of 12-bit tags this variant fills LDS to the last
+// byte without them: there the codewords read are replaced by zeros (which costs other variants up to 4 percent).
+constexpr bool fused_zero_word(int bits, int NW, int TW) { return !(bits == 12 && NW == 3 && TW == 4); }
 constexpr int fused_lds(int bits, int table_bytes, int NW, int TW, int S, int NB) {
-    return table_bytes + 2 * FUSED_RN * TW * fused_tag_bytes(bits) + NB * fused_stage_bytes(NW, TW, S);
+    return table_bytes + 2 * FUSED_RN * TW * fused_tag_bytes(bits) + NB * fused_stage_bytes(NW, TW, S) + (table_bytes && fused_zero_word(bits, NW, TW) ? 8 : 0);
 }
 
 template <int BITS, int D, int NW, int TW, int S, int NB>
@@ -129,7 +132,14 @@ __global__ __launch_bounds__(512, 2) void fused_kernel(FusedArgs a) {
     // the held tags' codewords into the stage buffer at `buf`, 1 KB a tile and step in the lanes' order.  d = 8: from L2, straight
     // into LDS.  d = 4: out of the codebook in LDS to registers (gather_w), from there into the buffer (put_w).
     u32x4 word[S][PT];
-    auto gather_w = [&](int step0, unsigned char* buf) {
+    // A round's units past the row's end are zeros (products of the row's last unit with the zeros of X would be NaN where one of its
+    // codewords is not finite): d = 8, this lane's zeros of X; d = 4, zeros in LDS.
+    constexpr bool ZW = fused_zero_word(BITS, NW, TW);
+    const unsigned char* xzero = a.x + ((int64_t)tb * a.k32 + a.k32 - 1) * (NT * 1024) + lane * 16;
+    const uint32_t wzero = (uint32_t)(a.table_bytes + 2 * RT * TB + NB * STAGE);
+    auto gather_w = [&](int round, int step0, unsigned char* buf) {
+        const bool past = 4 * round + lg >= a.U;
+        const uint32_t mask = ZW && past ? 0u : ((1u << BITS) - 1u) << 3;
 #pragma unroll
         for (int i = 0; i < PT; ++i) {
             if (D == 8 && !(i ? both : mine)) continue;
@@ -137,12 +147,12 @@ __global__ __launch_bounds__(512, 2) void fused_kernel(FusedArgs a) {
             for (int jj = 0; jj < S; ++jj) {
                 const int step = step0 + jj;
                 if constexpr (D == 8) {
-                    __builtin_amdgcn_global_load_lds((gptr_t)(table + ((unit_tag<BITS, UD>(held[jj][i], step) << 4) + bo[i])),
-                                                     (lptr_t)(buf + (jj * RT + wave + 8 * i) * 1024), 16, 0, 0);
+                    const char* from = table + ((unit_tag<BITS, UD>(held[jj][i], step) << 4) + bo[i]);
+                    __builtin_amdgcn_global_load_lds((gptr_t)(past ? (const char*)xzero : from), (lptr_t)(buf + (jj * RT + wave + 8 * i) * 1024), 16, 0, 0);
                 } else {
-                    const u32x2 lo = *(const mma_lds_u32x2*)(uintptr_t)unit_lds_offset<BITS, UD, 3>(held[jj][i], step * 2, bo[i]);
-                    const u32x2 hi = *(const mma_lds_u32x2*)(uintptr_t)unit_lds_offset<BITS, UD, 3>(held[jj][i], step * 2 + 1, bo[i]);
-                    word[jj][i] = u32x4{lo.x, lo.y, hi.x, hi.y};
+                    const u32x2 lo = *(const mma_lds_u32x2*)(uintptr_t)unit_lds_offset<BITS, UD, 3>(held[jj][i], step * 2, ZW && past ? wzero : bo[i], mask);
+                    const u32x2 hi = *(const mma_lds_u32x2*)(uintptr_t)unit_lds_offset<BITS, UD, 3>(held[jj][i], step * 2 + 1, ZW && past ? wzero : bo[i], mask);
+                    word[jj][i] = !ZW && past ? u32x4{0u, 0u, 0u, 0u} : u32x4{lo.x, lo.y, hi.x, hi.y};
                 }
             }
         }
@@ -173,13 +183,17 @@ __global__ __launch_bounds__(512, 2) void fused_kernel(FusedArgs a) {
 
     load_tags(r0, r0 & 1);
     load_tags(r0 + 1, (r0 + 1) & 1);
-    if (D == 4) { stage_table(m.table, a.table_bytes, smem); __syncthreads(); }
+    if (D == 4) {
+        stage_table(m.table, a.table_bytes, smem);
+        if (ZW && tid == 0) *reinterpret_cast<u32x2*>(smem + wzero) = u32x2{0u, 0u};
+        __syncthreads();
+    }
     __builtin_amdgcn_s_waitcnt(fused_wait(0));
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int q = 0; q < NB; ++q) {
         hold(r0 & 1, q * S);
-        gather_w(q * S, ring + q * STAGE);
+        gather_w(r0, q * S, ring + q * STAGE);
         put_w(ring + q * STAGE);
         copy_x(r0 * SPR + q * S, ring + q * STAGE);
     }
@@ -234,7 +248,7 @@ __global__ __launch_bounds__(512, 2) void fused_kernel(FusedArgs a) {
                 }
                 if (q == Q - 2) {
                     // this stage's buffer is free: the stage NB further on goes there
-                    gather_w(ps * S, buf);
+                    gather_w(round + pr, ps * S, buf);
                     copy_x((round + pr) * SPR + ps * S, buf);
                     if (ps + 1 < NST) hold((round + pr) & 1, (ps + 1) * S);
                     else { hold((round + pr + 1) & 1, 0); load_tags(round + pr + 2, (round + pr) & 1); }

@@ -72,14 +72,14 @@ constexpr int mma_x_tokens_min(int NT) { return NT == 1 ? 8 : 16; }
 // LDS byte offset of the codeword of tag t of a unit, counted from the start of the dynamic LDS: the tag times 2^SH (the
 // codeword size) plus `bo`, the byte offset of the row's codebook, whose bits lie above the tag's: one shift (or
 // v_alignbit_b32 for a tag that straddles two dwords, which starts past bit SH) and one v_and_or_b32
+// (mask: the tag's bits where they end up, or 0: the offset is then `bo` itself)
 template <int BITS, int UD, int SH>
-__device__ __forceinline__ uint32_t unit_lds_offset(const dwords<UD>& u, int t, uint32_t bo) {
+__device__ __forceinline__ uint32_t unit_lds_offset(const dwords<UD>& u, int t, uint32_t bo, uint32_t mask = ((1u << BITS) - 1u) << SH) {
     const int p = t * BITS, w = p >> 5, s = p & 31;
-    constexpr uint32_t MASK = ((1u << BITS) - 1u) << SH;
     uint32_t v;
     if (s + BITS <= 32) v = s >= SH ? u.v[w] >> (s - SH) : u.v[w] << (SH - s);
     else v = __builtin_amdgcn_alignbit(u.v[w + 1 < UD ? w + 1 : w], u.v[w], s - SH);
-    return (v & MASK) | bo;
+    return (v & mask) | bo;
 }
 typedef __attribute__((address_space(3))) u32x2 mma_lds_u32x2;
 typedef __attribute__((address_space(3))) u32x4 mma_lds_u32x4;

@@ -4,7 +4,7 @@ perms = seeded_perms(C, M, seed + 1); reference tests/test_kernels.py:15-26)."""
 
 from __future__ import annotations
 
-from dataclasses import dataclass
+from dataclasses import dataclass, replace
 
 import numpy as np
 import torch
@@ -65,3 +65,14 @@ def rand_x(B, C, dtype, seed=0, scale=1.0):
 
 def rel_max_err(got: np.ndarray, ref: np.ndarray) -> float:
     return float(np.abs(got.astype(np.float64) - ref).max() / max(np.abs(ref).max(), 1e-30))
+
+
+def with_infinity(s: Synth, row: int) -> Synth:
+    """s with a last codeword that holds one +inf and that only the last chunk of `row` names."""
+    top = s.K - 1
+    tags = np.minimum(s.tags, top - 1)
+    tags[row, -1] = top
+    table = s.table.copy()
+    book = 0 if s.row_book is None else int(s.row_book[row])
+    table[book * s.K + top, s.d - 1] = np.inf
+    return replace(s, tags=tags, words=O.pack_bits(tags, s.bits), table=table)

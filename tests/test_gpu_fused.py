@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from quantexperiments_amd.kernels import linear_gemm
-from tests.helpers import rand_x, rel_max_err, synth, to_device
+from tests.helpers import rand_x, rel_max_err, synth, to_device, with_infinity
 
 pytestmark = pytest.mark.gpu
 
@@ -39,3 +39,18 @@ def test_matches_oracle(case, dtype, stream):
     linear_gemm(lins, xd, lowp[:, :sum(rows)])
     assert torch.equal(lowp[:, :sum(rows)], y.to(dtype)) and not lowp[:, sum(rows):].any()
     assert np.isfinite(lowp.float().cpu().numpy()).all()
+
+
+@pytest.mark.parametrize("R,C,d,bits,G,T", [(11003, 64, 8, 16, 1, 129), (24577, 320, 8, 16, 1, 333), (12100, 704, 8, 16, 1, 700), (10900, 96, 4, 12, 1, 140),
+                                            (30000, 160, 4, 12, 2, 150), (12001, 192, 4, 10, 4, 384), (18500, 1088, 4, 8, 1, 640)])
+def test_missing_units_meet_no_codeword(R, C, d, bits, G, T):
+    """A last round with missing units, behind a row that ends in a codeword with an infinity: the row's results are infinite, not NaN."""
+    s = with_infinity(synth(R, C, d, bits, G, 1, seed=R), 5)
+    x = rand_x(T, C, torch.float16, seed=T).abs() + 0.125
+    y = torch.empty(T, R, dtype=torch.float32, device="cuda")
+    linear_gemm([to_device(s)], x.cuda(), y)
+    ref = torch.from_numpy(s.decode()).cuda().double()
+    assert bool(torch.isposinf(y[:, 5]).all()) and bool(torch.isinf(ref[5]).any())
+    ref[5] = 0
+    y[:, 5] = 0
+    assert rel_max_err(y.cpu().numpy(), (x.cuda().double() @ ref.T).cpu().numpy()) < 1e-5       # (exact products, fp32 sums)
