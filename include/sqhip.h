@@ -15,7 +15,9 @@
  * the host, reference shapequant/masks.py:334-342).  Row r decodes as
  *     u[r, j*d + k] = f32(table[row_book[r]*K + tag[r, j]][k]) * f32(row_scale[r])
  *     w[r, perms[row_mask[r]][c]] = u[r, c]
- * and the layer computes Y[t, y_off + r] = sum_c X[t, c] * w[r, c] with fp32 accumulation.
+ * and the layer computes Y[t, y_off + r] = sum_c X[t, c] * w[r, c] with fp32 accumulation.  A row that names a codeword which is not
+ * finite has results that are not finite; an infinity may come out as NaN (idle lanes of the kernels for up to 256 rows, 384 of
+ * large d = 4 matrices, multiply codewords of the row with zeros).  Other rows are not touched.
  */
 #ifndef SQHIP_H
 #define SQHIP_H

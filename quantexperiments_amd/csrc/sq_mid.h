@@ -136,14 +136,19 @@ __global__ __launch_bounds__(64 * NW, 2) void mid_kernel(MidArgs a) {
     };
     const uint32_t xbase = (uint32_t)(li * ROWB + (((lg * S) ^ mid_swizzle<S>(li)) << 4));
 
-    // ---- codewords of one step
+    // ---- codewords of one step.  In units past the row's end, whose X is zeros, a codeword that is not finite would make NaN of them: from
+    // memory these read zeros (an offset past the end of the buffer); from LDS the row's last unit again, as in sq_rows_mfma.h (a choice
+    // per codeword costs 4 to 9 % at 33 to 128 rows, 18944 x 2 x 3584 with 12-bit tags).
+    const __amdgpu_buffer_rsrc_t words = __builtin_amdgcn_make_buffer_rsrc((void*)(DENSE ? (const void*)tags : (const void*)m.table), 0,
+                                                                           DENSE ? (uint32_t)m.R * (uint32_t)m.C * 2u : D == 8 ? (uint32_t)m.G << (BITS + 4) : 0u, 0x00027000);
     auto gather = [&](u32x4* f, const dwords<UD>* t, int round, int step) {
+        const int col = round * (UPR * UK) + step * JC + lg * GC;
+        const bool past = DENSE ? col >= m.C : 4 * round + lg >= a.U;
 #pragma unroll
         for (int i = 0; i < TW; ++i) {
-            if constexpr (DENSE) {
-                f[i] = *reinterpret_cast<const u32x4*>(tags + (to[i] + (uint32_t)min(round * (UPR * UK) + step * JC + lg * GC, m.C - 8) * 2u));
-            } else if constexpr (D == 8) {
-                f[i] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(m.table) + ((unit_tag<BITS, UD>(t[i], step) << 4) + bo[i]));
+            if constexpr (D != 4) {
+                const uint32_t at = DENSE ? to[i] + (uint32_t)col * 2u : (unit_tag<DENSE ? 16 : BITS, UD>(t[i], step) << 4) + bo[i];
+                f[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(words, past ? 0xFFFFFFF0u : at, 0, 0));
             } else {
                 const u32x2 lo = *(const mma_lds_u32x2*)(uintptr_t)unit_lds_offset<BITS, UD, 3>(t[i], step * 2, bo[i]);
                 const u32x2 hi = *(const mma_lds_u32x2*)(uintptr_t)unit_lds_offset<BITS, UD, 3>(t[i], step * 2 + 1, bo[i]);

@@ -8,7 +8,7 @@ import torch
 
 from quantexperiments_amd import _lib
 from quantexperiments_amd.kernels import linear_gemm
-from tests.helpers import rand_x, rel_max_err, synth, to_device
+from tests.helpers import rand_x, rel_max_err, synth, to_device, with_infinity
 
 pytestmark = pytest.mark.gpu
 
@@ -96,3 +96,20 @@ def test_decoded_weights_with_activation_rows_that_span_4_gb(T, ld):
     y = torch.empty(T, 70, dtype=torch.float32, device="cuda")
     linear_gemm([lin], xd, y)
     assert rel_max_err(y.cpu().numpy(), x.double().numpy() @ s.decode().astype(np.float64).T) < 1e-3
+
+
+@pytest.mark.parametrize("R,C,d,bits,G,M,T", [(129, 64, 8, 16, 1, 1, 33), (300, 320, 8, 16, 2, 1, 120), (40, 2112, 8, 16, 1, 1, 250), (60, 72, 8, 16, 1, 1, 5),
+                                              (70, 1000, 4, 12, 1, 1, 48), (50, 1984, 8, 16, 1, 3, 100)])
+def test_missing_units_meet_no_codeword(R, C, d, bits, G, M, T):
+    """A last round with missing units (or, of decoded weights, missing columns) behind a row that ends in a codeword with an infinity:
+    the row's results are infinite, not NaN."""
+    s = with_infinity(synth(R, C, d, bits, G, M, seed=R), 5)
+    x = rand_x(T, C, torch.float16, seed=T).abs() + 0.125
+    y = torch.empty(T, R, dtype=torch.float32, device="cuda")
+    linear_gemm([to_device(s, stream=d == 4)], x.cuda(), y)     # (the slice stream is a layout for fewer rows)
+    ref = torch.from_numpy(s.decode()).cuda().double()
+    assert bool(torch.isposinf(y[:, 5]).all()) and bool(torch.isinf(ref[5]).any())
+    ref[5] = 0
+    y[:, 5] = 0
+    # exact products and fp32 sums; weights that were decoded first are rounded to fp16 with their scale, 2^-11 of each
+    assert rel_max_err(y.cpu().numpy(), (x.cuda().double() @ ref.T).cpu().numpy()) < (1e-5 if C % 64 == 0 and M == 1 else 5e-4)

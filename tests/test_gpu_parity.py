@@ -9,7 +9,8 @@ import torch
 
 from oracle import c_oracle
 from oracle import sq_oracle as O
-from tests.helpers import rand_x, rel_max_err, synth, to_device
+from quantexperiments_amd.kernels import linear_gemm, linear_small
+from tests.helpers import rand_x, rel_max_err, synth, to_device, with_infinity
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-3
@@ -1239,3 +1240,20 @@ def test_random_lds_codebook_shapes_match_oracle():
         ref = np.concatenate(refs, axis=1)
         assert rel_max_err(y[:, :Rt].cpu().numpy(), ref) < TOL, (it, C, bits, G, B, [p.R for p in pieces])
         assert bool((y[:, Rt:] == 3.0).all()), it
+
+
+@pytest.mark.parametrize("R,C,d,bits,G,M", [(300, 1024, 8, 16, 1, 1), (130, 520, 8, 14, 2, 3), (300, 1056, 4, 12, 1, 1), (70, 1000, 4, 12, 1, 1), (90, 896, 4, 8, 4, 1)])
+def test_codeword_with_an_infinity_stays_in_its_row(R, C, d, bits, G, M):
+    s = with_infinity(synth(R, C, d, bits, G, M, seed=R), 5)
+    lin = to_device(s)
+    w = torch.from_numpy(s.decode()).cuda().double()
+    assert bool(torch.isinf(w[5]).any())
+    w[5] = 0
+    for B in (1, 2, 4, 8, 9, 20, 32, 40):
+        x = rand_x(B, C, torch.float16, seed=B).abs() + 0.125
+        y = torch.empty(B, R, dtype=torch.float32, device="cuda")
+        (linear_small if B <= 32 else linear_gemm)([lin], x.cuda(), y)
+        assert not bool(torch.isfinite(y[:, 5]).any()), B
+        y[:, 5] = 0
+        # (weights decoded first are rounded to fp16 with their scale, 2^-11 of each)
+        assert rel_max_err(y.cpu().numpy(), (x.cuda().double() @ w.T).cpu().numpy()) < 5e-4, B
