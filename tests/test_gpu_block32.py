@@ -294,3 +294,27 @@ def test_q8_full_vocabulary_shape_properties():
     y2 = torch.empty(1, V, dtype=torch.float32, device="cuda")
     q8_linear(q, sc, x[6:7] * 2, y2)
     assert torch.equal(y2, y1 * 2)
+
+
+def test_q8_product_without_memory_for_its_workspace_raises():
+    """The shared workspace is gone and the device's memory taken: an error, not a slower kernel."""
+    from quantexperiments_amd.kernels import _Workspace, q8_linear
+    V, C, B = 9000, 1408, 9
+    q = torch.zeros(V, C, dtype=torch.int8, device="cuda")
+    sc = torch.zeros(V, C // 32, dtype=torch.float16, device="cuda")
+    x, y = torch.zeros(B, C, dtype=torch.bfloat16, device="cuda"), torch.empty(B, V, device="cuda")
+    kept, hog = _Workspace.bufs.pop(("cuda:0", "kernels"), None), []
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (1 << 20)) / total)
+    try:
+        with pytest.raises(torch.OutOfMemoryError):
+            for _ in range(10_000):                             # (free blocks that are still held beside others)
+                hog.append(torch.empty(20 << 20, dtype=torch.uint8, device="cuda"))
+        with pytest.raises(torch.OutOfMemoryError):
+            q8_linear(q, sc, x, y)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+        if kept is not None:
+            _Workspace.bufs["cuda:0", "kernels"] = kept
