@@ -14,6 +14,7 @@
 #include <ATen/core/dispatch/Dispatcher.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pybind.h>
@@ -170,7 +171,8 @@ bool tensors(PyObject* const* a, int n) {
     return true;
 }
 
-#define SQ_GUARD(...) try { __VA_ARGS__ } catch (const std::exception& e) { if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what()); return nullptr; }
+// (torch's own translation: an allocation that fails is a torch.OutOfMemoryError here too)
+#define SQ_GUARD(...) try { __VA_ARGS__ } catch (...) { if (!PyErr_Occurred()) torch::translate_exception_to_python(std::current_exception()); return nullptr; }
 
 // linear(pieces, x, y, gemm)
 PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -413,7 +415,14 @@ PyObject* q8_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
             return answer(NOT_COVERED);
         OnDevice on(dev);
         Workspace ws;
-        if (!workspace(dev, sq_q8_workspace_bytes((int)V, (int)C, (int)x.size(0)), on.stream, ws)) return answer(NOT_COVERED);
+        const size_t need = sq_q8_workspace_bytes((int)V, (int)C, (int)x.size(0));
+        if (need && C % 256 && x.size(0) <= SQ_SMALL_BMAX) {     // (a buffer of its own: see kernels.q8_linear)
+            ws.held = at::empty({(int64_t)need}, q.options().dtype(at::kByte));
+            ws.p = ws.held.data_ptr();
+            ws.bytes = need;
+        } else if (!workspace(dev, need, on.stream, ws)) {
+            return answer(NOT_COVERED);
+        }
         int rc;
         Py_BEGIN_ALLOW_THREADS
         rc = sq_q8_linear((const int8_t*)q.data_ptr(), (const uint16_t*)sc.data_ptr(), (int)V, (int)C, x.data_ptr(), xd, x.stride(0), y.data_ptr(), yd, y.stride(0),

@@ -56,11 +56,6 @@ class _Workspace:
         return b
 
     @classmethod
-    def holds(cls, nbytes: int, dev, kind: str = "kernels") -> bool:
-        b = cls.bufs.get((str(dev), kind))
-        return b is not None and b.numel() >= nbytes
-
-    @classmethod
     def status(cls, dev) -> None:
         """Synchronise and raise if a launch on this device's workspace gave up waiting for a partial sum
         (sq_workspace_status); every launch since then has written NaN."""
@@ -573,12 +568,9 @@ def q8_linear(q: torch.Tensor, sc: torch.Tensor, x: torch.Tensor, y: torch.Tenso
     L = _lib.lib()
     with torch.cuda.device(dev):
         need = L.sq_q8_workspace_bytes(V, C, x.shape[0])
-        # (up to SMALL_BMAX rows that are not whole 256-column chunks run without one too: being captured, with none there yet)
-        optional = C % 256 != 0 and x.shape[0] <= _lib.SMALL_BMAX
-        if need and not (optional and torch.cuda.is_current_stream_capturing() and not _Workspace.holds(need, dev)):
-            ws = _Workspace.get(need, dev)
-        else:
-            ws = None
+        # (rows that are not whole 256-column chunks: up to SMALL_BMAX of them share nothing, so that streams may run them side by side)
+        own = C % 256 != 0 and x.shape[0] <= _lib.SMALL_BMAX
+        ws = None if not need else torch.empty(need, dtype=torch.uint8, device=dev) if own else _Workspace.get(need, dev)
         _lib.check(L.sq_q8_linear(q.data_ptr(), sc.data_ptr(), V, C, x.data_ptr(), _lib.DTYPES[x.dtype], x.stride(0),
                                   y.data_ptr(), _lib.DTYPES[y.dtype], y.stride(0), x.shape[0],
                                   None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(),

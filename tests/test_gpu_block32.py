@@ -318,3 +318,34 @@ def test_q8_product_without_memory_for_its_workspace_raises():
         torch.cuda.set_per_process_memory_fraction(1.0)
         if kept is not None:
             _Workspace.bufs["cuda:0", "kernels"] = kept
+
+
+@pytest.mark.parametrize("V,C,B", [(30016, 640, 3), (9008, 576, 8), (1040, 1408, 9), (8000, 64, 32)])
+@pytest.mark.parametrize("native", [True, False], ids=["native", "python"])
+def test_q8_products_of_broken_chunks_share_nothing(V, C, B, native, monkeypatch):
+    """bf16 rows that are not whole 256-column chunks leave the shared workspace alone (two streams may run them at once), eagerly and
+    in a graph, each replay the same."""
+    from quantexperiments_amd import _lib
+    from quantexperiments_amd.kernels import _Workspace, q8_linear
+    if not native:
+        monkeypatch.setattr(_lib.native(), "q8_linear", lambda *a: 1)
+    q, sc, deq = _q8_parts(V, C, seed=V + B)
+    tq, ts = _dev(q, sc)
+    x = rand_x(B, C, torch.bfloat16, seed=B).cuda()
+    dev = x.device
+    L = _lib.lib()
+    shared = _Workspace.get(L.sq_q8_workspace_bytes(V, C, B), dev)[_lib.WS_HEADER:]
+    shared.fill_(0x5A)
+    y = torch.empty(B, V, device=dev)
+    q8_linear(tq, ts, x, y)
+    assert bool((shared == 0x5A).all())
+    assert rel_max_err(y.cpu().numpy(), x.cpu().double().numpy() @ np.asarray(deq, np.float64).T) < 1e-5   # (exact products, fp32 sums)
+    want = y.clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        q8_linear(tq, ts, x, y)
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want) and bool((shared == 0x5A).all())
