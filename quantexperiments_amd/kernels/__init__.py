@@ -287,22 +287,22 @@ def _relabel(ms) -> None:
     own slices."""
     L = _lib.lib()
     for m in ms:
-        m.relabelled = True
         if m.table.data_ptr() % 16:
             m.table = m.table.clone()
     # (shapes the slice stream does not cover are refused: nothing to balance)
     todo = [(m, a) for m in ms for a in [_lib.matrix_array([m.descriptor()])] if L.sq_codebook_rebalance_bytes(a, 1)]
-    if not todo:
-        return
-    dev = todo[0][0].device
-    mats = _lib.matrix_array([a[0] for _, a in todo])
-    out = [(torch.empty_like(m.words), torch.empty_like(m.table)) for m, _ in todo]
-    ptrs = [(ctypes.c_void_p * len(out))(*(o[k].data_ptr() for o in out)) for k in (0, 1)]
-    scratch = torch.empty(L.sq_codebook_rebalance_bytes(mats, len(todo)), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
-        _lib.check(L.sq_codebook_rebalance_device(mats, len(todo), *ptrs, scratch.data_ptr(), scratch.numel(), _lib.stream_ptr(dev)))
-    for (m, _), (words, table) in zip(todo, out):
-        m.words, m.table = words, table
+    if todo:
+        dev = todo[0][0].device
+        mats = _lib.matrix_array([a[0] for _, a in todo])
+        out = [(torch.empty_like(m.words), torch.empty_like(m.table)) for m, _ in todo]
+        ptrs = [(ctypes.c_void_p * len(out))(*(o[k].data_ptr() for o in out)) for k in (0, 1)]
+        scratch = torch.empty(L.sq_codebook_rebalance_bytes(mats, len(todo)), dtype=torch.uint8, device=dev)
+        with torch.cuda.device(dev):
+            _lib.check(L.sq_codebook_rebalance_device(mats, len(todo), *ptrs, scratch.data_ptr(), scratch.numel(), _lib.stream_ptr(dev)))
+        for (m, _), (words, table) in zip(todo, out):
+            m.words, m.table = words, table
+    for m in ms:                                                # (only now: what failed is done again by the next build)
+        m.relabelled = True
 
 
 def build_stream(words: torch.Tensor, C: int, d: int, bits: int, row_mask=None, runs: int = 0, table=None, row_book=None):

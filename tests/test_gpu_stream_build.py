@@ -160,3 +160,20 @@ def test_layouts_are_whole_when_they_are_handed_back(rows, C, d, bits, G, M):
     torch.cuda.synchronize()
     want = np.concatenate([x.cpu().double().numpy() @ s.decode().astype(np.float64).T for s in ss], axis=1)
     assert rel_max_err(y.cpu().numpy(), want) < 1e-5            # (exact products, fp32 sums)
+
+
+def test_a_relabelling_that_failed_is_done_again(monkeypatch):
+    """The launch fails once: nothing of the matrices has changed, and the next build relabels them."""
+    L, ss = _lib.lib(), [synth(R, 1024, 8, 16, seed=R) for R in (200, 70)]
+    want, lins = [[to_device(s, stream="later") for s in ss] for _ in range(2)]
+    prepare_stack(want)
+    before = [(m.words, m.table) for m in lins]
+    with monkeypatch.context() as mp:
+        mp.setattr(L, "sq_codebook_rebalance_device", lambda *a: _lib.SQ_ELAUNCH)
+        with pytest.raises(RuntimeError):
+            prepare_stack(lins)
+    assert all(m.stream is None and not m.relabelled and m.words is w and m.table is t for m, (w, t) in zip(lins, before))
+    prepare_stack(lins)
+    for m, w, (words, _) in zip(lins, want, before):
+        assert not torch.equal(m.words, words) and m.relabelled and torch.equal(m.words, w.words)
+        assert torch.equal(m.table, w.table) and torch.equal(m.stream, w.stream) and m.stream_runs == w.stream_runs
