@@ -104,6 +104,13 @@ bool fused_route(const sq_matrix* mats, int n, int T) {
     return fused_plan(mats, n, T, device_cus()).nw != 0;
 }
 
+// For tests: the variant that a stack takes at T rows, as token tiles | weight tiles << 8 | K slices << 16 | token blocks << 24; 0: another kernel.
+extern "C" __attribute__((visibility("default"))) int32_t sq_fused_variant_for_tests(const sq_matrix* mats, int32_t n, int32_t T) {
+    if (!fused_route(mats, n, T)) return 0;
+    const FusedPlan p = fused_plan(mats, n, T, device_cus());
+    return p.nw | p.tw << 8 | p.ks << 16 | p.tbs << 24;
+}
+
 size_t fused_workspace(const sq_matrix* mats, int n, int T) {
     const FusedPlan p = fused_plan(mats, n, T, device_cus());
     size_t need = fused_x_bytes(mats, p);
