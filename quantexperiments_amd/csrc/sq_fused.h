@@ -29,6 +29,11 @@ namespace sq {
 
 constexpr int FUSED_TN = 4, FUSED_RN = 2;    // waves of a workgroup: token quarters x row halves, two per SIMD
 
+// 16 bytes per lane from offset `at` of a buffer to LDS, 16 bytes apart; zeros where the offset lies past its end
+__device__ __forceinline__ void buffer_to_lds16(__amdgpu_buffer_rsrc_t buffer, uint32_t at, __attribute__((address_space(3))) void* to) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(buffer, to, 16, at, 0, 0, 0);
+}
+
 struct FusedPiece {
     sq_matrix m;
     const void* w;               // tile-major copy of the tags, or NULL
@@ -89,7 +94,6 @@ __global__ __launch_bounds__(512, 2) void fused_kernel(FusedArgs a) {
     const bool tiled = P.w != nullptr;
     const uint32_t us = (tiled ? 16 * UD : UD) * 4;
     const char* tags = reinterpret_cast<const char*>(P.w ? P.w : m.tags);
-    const char* table = reinterpret_cast<const char*>(m.table);
     uint32_t to[PT], bo[PT];
     const bool mine = wave < RT, both = wave + 8 < RT;
 #pragma unroll
@@ -133,9 +137,9 @@ __global__ __launch_bounds__(512, 2) void fused_kernel(FusedArgs a) {
     // into LDS.  d = 4: out of the codebook in LDS to registers (gather_w), from there into the buffer (put_w).
     u32x4 word[S][PT];
     // A round's units past the row's end are zeros (products of the row's last unit with the zeros of X would be NaN where one of its
-    // codewords is not finite): d = 8, this lane's zeros of X; d = 4, zeros in LDS.
+    // codewords is not finite): d = 8, an offset past the end of the codebooks, which reads as zeros; d = 4, zeros in LDS.
     constexpr bool ZW = fused_zero_word(BITS, NW, TW);
-    const unsigned char* xzero = a.x + ((int64_t)tb * a.k32 + a.k32 - 1) * (NT * 1024) + lane * 16;
+    const __amdgpu_buffer_rsrc_t words = __builtin_amdgcn_make_buffer_rsrc((void*)m.table, 0, D == 8 ? (uint32_t)m.G << (BITS + 4) : 0u, 0x00027000);
     const uint32_t wzero = (uint32_t)(a.table_bytes + 2 * RT * TB + NB * STAGE);
     auto gather_w = [&](int round, int step0, unsigned char* buf) {
         const bool past = 4 * round + lg >= a.U;
@@ -147,8 +151,7 @@ __global__ __launch_bounds__(512, 2) void fused_kernel(FusedArgs a) {
             for (int jj = 0; jj < S; ++jj) {
                 const int step = step0 + jj;
                 if constexpr (D == 8) {
-                    const char* from = table + ((unit_tag<BITS, UD>(held[jj][i], step) << 4) + bo[i]);
-                    __builtin_amdgcn_global_load_lds((gptr_t)(past ? (const char*)xzero : from), (lptr_t)(buf + (jj * RT + wave + 8 * i) * 1024), 16, 0, 0);
+                    buffer_to_lds16(words, (unit_tag<BITS, UD>(held[jj][i], step) << 4) | (past ? 0xFFFFFFF0u : bo[i]), (lptr_t)(buf + (jj * RT + wave + 8 * i) * 1024));
                 } else {
                     const u32x2 lo = *(const mma_lds_u32x2*)(uintptr_t)unit_lds_offset<BITS, UD, 3>(held[jj][i], step * 2, ZW && past ? wzero : bo[i], mask);
                     const u32x2 hi = *(const mma_lds_u32x2*)(uintptr_t)unit_lds_offset<BITS, UD, 3>(held[jj][i], step * 2 + 1, ZW && past ? wzero : bo[i], mask);
