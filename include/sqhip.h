@@ -3,8 +3,8 @@
  * One shared library, libsqhip.so, replaces every GPU launch site of the reference's
  * codebook linear layer.  All pointers inside sq_matrix and all x / y / out / workspace
  * pointers are DEVICE pointers owned by the caller; nothing here allocates or frees
- * device memory and nothing synchronises the host: every call only enqueues kernels on
- * `stream` (a hipStream_t passed as void*; NULL = the default stream), so calls can be
+ * device memory and nothing synchronises the host (but for the load-time and status calls that
+ * say so): every call only enqueues kernels on `stream` (a hipStream_t passed as void*; NULL = the default stream), so calls can be
  * recorded into a HIP graph.  Functions return SQ_OK or a negative SQ_E* code and keep a
  * message for sq_last_error() (thread local).
  *
@@ -16,8 +16,8 @@
  *     u[r, j*d + k] = f32(table[row_book[r]*K + tag[r, j]][k]) * f32(row_scale[r])
  *     w[r, perms[row_mask[r]][c]] = u[r, c]
  * and the layer computes Y[t, y_off + r] = sum_c X[t, c] * w[r, c] with fp32 accumulation.  A row that names a codeword which is not
- * finite has results that are not finite; an infinity may come out as NaN (idle lanes of the kernels for up to 256 rows, 384 of
- * large d = 4 matrices, multiply codewords of the row with zeros).  Other rows are not touched.
+ * finite has results that are not finite; an infinity may come out as NaN (idle lanes of the decode-time kernels, and of the d = 4
+ * kernel for 33 to 384 rows, multiply codewords of the row with zeros).  Other rows are not touched.
  */
 #ifndef SQHIP_H
 #define SQHIP_H
