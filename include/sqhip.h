@@ -130,7 +130,7 @@ size_t sq_gemm_dense_workspace_bytes(int32_t R, int32_t C, int32_t T);
 
 /* Bytes of workspace sq_linear_small (which = 0) or sq_linear_gemm (which = 1) needs for these
  * pieces at `rows` activation rows (which = 2 / 3: the same for a workspace that serves these pieces only, see
- * below); the caller grows its buffer before any graph capture
+ * below; which = 4 / 5: the least that up to SQ_SMALL_BMAX rows can run with, slower where it is less); the caller grows its buffer before any graph capture
  * (the reference grows its buffers the same way: batched_runs.py:628-640, runs_gemm.py:396-404).
  * A workspace must be 256-byte aligned.  One of at least SQ_WS_HEADER_BYTES begins with a header of that size,
  * which must be ZERO when the workspace is first handed to the library and which nobody else may write

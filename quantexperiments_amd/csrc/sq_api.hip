@@ -319,8 +319,10 @@ size_t sq_gemm_dense_workspace_bytes(int32_t R, int32_t C, int32_t T) {
 size_t sq_workspace_bytes(const sq_matrix* mats, int32_t n_mats, int32_t rows, int which) {
     if (!mats || n_mats <= 0 || rows <= 0) return 0;
     // which & 1 = 0 covers both kernels a stack with column orders may take (the caller's x decides, see sq_linear_small)
-    const size_t inner = (which & 1) == 0 ? std::max(small_workspace(mats, n_mats, rows), small_gemm_route_workspace(mats, n_mats, rows))
-                                          : gemm_workspace(mats, n_mats, rows);
+    const size_t inner = (which & 4) && rows <= SQ_SMALL_BMAX
+                             ? std::max(small_workspace_least(mats, n_mats, rows), small_gemm_route_workspace(mats, n_mats, rows))
+                         : (which & 1) == 0 ? std::max(small_workspace(mats, n_mats, rows), small_gemm_route_workspace(mats, n_mats, rows))
+                                            : gemm_workspace(mats, n_mats, rows);
     const bool sums = small_uses_sums(mats, n_mats);
     // which & 2: a workspace of the caller's own for these pieces alone: no header unless they keep partial sums in
     // it (or need so much that the buffer would be taken for one that begins with a header)

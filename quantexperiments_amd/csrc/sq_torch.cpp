@@ -149,6 +149,17 @@ bool workspace(int dev, size_t need, hipStream_t s, Workspace& ws) {
     return true;
 }
 
+// The workspace of a product: the shared one; a buffer of the call's own where the pieces could run without any (their partial sums
+// only make them faster), so that streams may run them side by side.
+bool product_workspace(const Pieces& p, int rows, int which, const at::Tensor& like, hipStream_t s, Workspace& ws) {
+    const size_t need = sq_workspace_bytes(p.m, p.n, rows, which);
+    if (need == 0 || rows > SQ_SMALL_BMAX || sq_workspace_bytes(p.m, p.n, rows, which | 4) != 0) return workspace(p.dev, need, s, ws);
+    ws.bytes = sq_workspace_bytes(p.m, p.n, rows, which | 2);
+    ws.held = at::empty({(int64_t)ws.bytes}, like.options().dtype(at::kByte));
+    ws.p = ws.held.data_ptr();
+    return true;
+}
+
 int linear_into(const Pieces& p, const at::Tensor& x, const at::Tensor& y, bool gemm) {
     const int xd = dtype_of(x), yd = dtype_of(y);
     if (!is16(xd) || yd < 0 || !matrix_on(x, p.dev) || !matrix_on(y, p.dev) || x.size(0) != y.size(0) || y.size(1) != p.rows || x.size(1) != p.m[0].C ||
@@ -157,7 +168,7 @@ int linear_into(const Pieces& p, const at::Tensor& x, const at::Tensor& y, bool 
     const int B = (int)x.size(0);
     OnDevice on(p.dev);
     Workspace ws;
-    if (!workspace(p.dev, sq_workspace_bytes(p.m, p.n, B, gemm), on.stream, ws)) return NOT_COVERED;
+    if (!product_workspace(p, B, gemm, x, on.stream, ws)) return NOT_COVERED;
     int rc;
     Py_BEGIN_ALLOW_THREADS
     rc = (gemm ? sq_linear_gemm : sq_linear_small)(p.m, p.n, x.data_ptr(), xd, row_ld(x), y.data_ptr(), yd, row_ld(y), B, ws.p, ws.bytes, on.stream);
@@ -344,7 +355,7 @@ PyObject* linear_from(PyObject*, PyObject* const* a, Py_ssize_t n) {
         }
         OnDevice on(p.dev);
         Workspace ws;
-        if (!workspace(p.dev, sq_workspace_bytes(p.m, p.n, (int)B, 0), on.stream, ws)) return answer(NOT_COVERED);
+        if (!product_workspace(p, (int)B, 0, y, on.stream, ws)) return answer(NOT_COVERED);
         int rc;
         Py_BEGIN_ALLOW_THREADS
         rc = sq_linear_small_from(p.m, p.n, &pr, dt, y.data_ptr(), yd, row_ld(y), (int)B, ws.p, ws.bytes, on.stream);
@@ -378,7 +389,7 @@ PyObject* linear_silu(PyObject*, PyObject* const* a, Py_ssize_t n) {
         }
         OnDevice on(p.dev);
         Workspace ws;
-        if (!workspace(p.dev, sq_workspace_bytes(p.m, 2, (int)B, 0), on.stream, ws)) return answer(NOT_COVERED);
+        if (!product_workspace(p, (int)B, 0, out, on.stream, ws)) return answer(NOT_COVERED);
         int rc;
         Py_BEGIN_ALLOW_THREADS
         rc = sq_linear_small_silu(p.m, 2, norm ? &pr : nullptr, norm ? nullptr : x.data_ptr(), dt, norm ? 0 : row_ld(x), out.data_ptr(), row_ld(out), (int)B,

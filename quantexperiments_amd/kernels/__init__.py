@@ -470,6 +470,16 @@ def _prep(pieces, x: torch.Tensor, y: torch.Tensor):
         y.stride(0) if y.shape[0] > 1 else max(y.stride(0), y.shape[1])
 
 
+def _product_workspace(mats, n: int, rows: int, which: int, dev):
+    """The workspace of a product (None: it needs none): the shared one, or a buffer of the call's own where the pieces could run
+    without any (their partial sums only make them faster), so that streams may run them side by side."""
+    L = _lib.lib()
+    need = L.sq_workspace_bytes(mats, n, rows, which)
+    if need and rows <= _lib.SMALL_BMAX and not L.sq_workspace_bytes(mats, n, rows, which | 4):
+        return torch.empty(L.sq_workspace_bytes(mats, n, rows, which | 2), dtype=torch.uint8, device=dev)
+    return _Workspace.get(need, dev) if need else None
+
+
 def dequant_stack(pieces, out: torch.Tensor, x: torch.Tensor | None = None) -> torch.Tensor | None:
     """fp16 weights of all pieces one below the other into out [sum R, C] (sq_dequant_stack) and, in the same launches, the fp16
     copy of x (bf16 [B, C], rows of whole 16-byte pieces), which is returned."""
@@ -498,8 +508,7 @@ def linear_small(pieces, x: torch.Tensor, y: torch.Tensor) -> torch.Tensor:
     dev = x.device
     L = _lib.lib()
     with torch.cuda.device(dev):
-        need = L.sq_workspace_bytes(mats, len(pieces), x.shape[0], 0)
-        ws = _Workspace.get(need, dev) if need else None
+        ws = _product_workspace(mats, len(pieces), x.shape[0], 0, dev)
         _lib.check(L.sq_linear_small(mats, len(pieces), x.data_ptr(), _lib.DTYPES[x.dtype], ldx, y.data_ptr(),
                                      _lib.DTYPES[y.dtype], ldy, x.shape[0], None if ws is None else ws.data_ptr(),
                                      0 if ws is None else ws.numel(), _lib.stream_ptr(dev)))
@@ -517,8 +526,7 @@ def linear_gemm(pieces, x: torch.Tensor, y: torch.Tensor) -> torch.Tensor:
     dev = x.device
     L = _lib.lib()
     with torch.cuda.device(dev):
-        need = L.sq_workspace_bytes(mats, len(pieces), x.shape[0], 1)
-        ws = _Workspace.get(need, dev) if need else None
+        ws = _product_workspace(mats, len(pieces), x.shape[0], 1, dev)
         _lib.check(L.sq_linear_gemm(mats, len(pieces), x.data_ptr(), _lib.DTYPES[x.dtype], ldx, y.data_ptr(),
                                     _lib.DTYPES[y.dtype], ldy, x.shape[0], None if ws is None else ws.data_ptr(),
                                     0 if ws is None else ws.numel(), _lib.stream_ptr(dev)))
@@ -731,8 +739,7 @@ def linear_small_from(pieces, y: torch.Tensor, x_out: torch.Tensor, *, h_in=None
         pr.mode, pr.add, pr.up, pr.ld_in = _lib.SQ_FROM_SILU_MUL, gate.data_ptr(), up.data_ptr(), _row_ld(gate)
     L = _lib.lib()
     with torch.cuda.device(dev):
-        need = L.sq_workspace_bytes(mats, len(pieces), x_out.shape[0], 0)
-        ws = _Workspace.get(need, dev) if need else None
+        ws = _product_workspace(mats, len(pieces), x_out.shape[0], 0, dev)
         _lib.check(L.sq_linear_small_from(mats, len(pieces), ctypes.byref(pr), _lib.DTYPES[dt], y.data_ptr(), _lib.DTYPES[y.dtype],
                                           ldy, x_out.shape[0], None if ws is None else ws.data_ptr(),
                                           0 if ws is None else ws.numel(), _lib.stream_ptr(dev)))
@@ -775,8 +782,7 @@ def linear_small_silu(pieces, x: torch.Tensor, out: torch.Tensor, *, x_out=None,
         if add is not None:
             pr.add, pr.ld_in = add.data_ptr(), _row_ld(add)
     with torch.cuda.device(dev):
-        need = L.sq_workspace_bytes(mats, 2, B, 0)
-        ws = _Workspace.get(need, dev) if need else None
+        ws = _product_workspace(mats, 2, B, 0, dev)
         rc = L.sq_linear_small_silu(mats, 2, None if pr is None else ctypes.byref(pr), None if norm else xin.data_ptr(), _lib.DTYPES[dt],
                                     0 if norm else _row_ld(xin), out.data_ptr(), _row_ld(out), B,
                                     None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), _lib.stream_ptr(dev))

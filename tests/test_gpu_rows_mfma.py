@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from quantexperiments_amd import _lib
-from quantexperiments_amd.kernels import linear_small
+from quantexperiments_amd.kernels import _Workspace, linear_small
 from tests.helpers import rand_x, rel_max_err, synth, to_device
 
 pytestmark = pytest.mark.gpu
@@ -49,3 +49,31 @@ def test_rows_that_one_launch_takes_whole(rows, C, bits, G):
             _lib.check(L.sq_linear_small(mats, len(lin), x.data_ptr(), _lib.DTYPES[dtype], C, y.data_ptr(), _lib.SQ_F32, sum(rows), B, None, 0,
                                          _lib.stream_ptr(dev)))
             assert rel_max_err(y[:, :n].cpu().numpy(), want[:, :n]) < 1e-5 and bool(y[:, n:].isnan().all()), B
+
+
+@pytest.mark.parametrize("rows,C,bits,G,B", [((300,), 8192, 12, 1, 8), ((300,), 6912, 12, 4, 16), ((40, 300), 7168, 8, 1, 2)])
+@pytest.mark.parametrize("native", [True, False], ids=["native", "python"])
+def test_products_that_need_no_sums_share_nothing(rows, C, bits, G, B, native, monkeypatch):
+    """The partial sums of rows that one launch could take whole leave the shared workspace alone (two streams may run them at once),
+    eagerly and in a graph, each replay the same."""
+    if not native:
+        monkeypatch.setattr(_lib.native(), "linear", lambda *a: 1)
+    ss = [synth(R, C, 4, bits, G, 1, seed=R + C) for R in rows]
+    lins = [to_device(s) for s in ss]
+    x = rand_x(B, C, torch.bfloat16, seed=B).cuda()
+    mats = _lib.matrix_array([m.descriptor() for m in lins])
+    shared = _Workspace.get(_lib.lib().sq_workspace_bytes(mats, len(lins), B, 0), x.device)[_lib.WS_HEADER:]
+    shared.fill_(0x5A)
+    y = torch.empty(B, sum(rows), device="cuda")
+    linear_small(lins, x, y)
+    want = np.concatenate([x.cpu().half().double().numpy() @ s.decode().astype(np.float64).T for s in ss], axis=1)
+    assert rel_max_err(y.cpu().numpy(), want) < 1e-5 and bool((shared == 0x5A).all())
+    first = y.clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        linear_small(lins, x, y)
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, first) and bool((shared == 0x5A).all())
