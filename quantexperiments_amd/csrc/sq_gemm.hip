@@ -166,9 +166,11 @@ static size_t dense_bytes(const sq_matrix& m) { return (((size_t)m.R * m.C * 2) 
 
 // The decode + 256 x 256 tile route: from GEMM256_MIN_T rows, and for stacks with column orders at any row count
 // (their decode-time kernel is the slow one: 27B-shaped layer with 16 orders, 880 us at 16 rows and 1746 us at 32
-// against 625 us here).
+// against 625 us here).  Rows that end within a slab of 64 columns take it from BROKEN_DECODED_T on, up to where they are decoded in steps
+// of bounded workspace (5120 x 2080: 34-38 us there at 200 rows, 38-44 here at 400; in the 128 x 128 kernel 80-120).
+constexpr int BROKEN_DECODED_T = 256;
 static bool big_route(const sq_matrix* mats, int n, int T) {
-    if (mats[0].C % 64) return false;
+    if (mats[0].C % 64) return mats[0].C % 8 == 0 && T > BROKEN_DECODED_T;
     if (T >= GEMM256_MIN_T) return true;
     for (int i = 0; i < n; ++i)
         if (mats[i].perms) return true;
@@ -243,7 +245,7 @@ static DecodedRows decoded_step(const sq_matrix* mats, int n, int& i, int& r0) {
 
 // Where the tile GEMM, whose workgroups read less, is the faster one behind the same decode: with more rows than half the CUs'
 // worth of 256-row tiles, and from 129 activation rows for 24 M weights and more (there and here, us: 37888 x 3584 at 64 rows 216
-// and 248, 30000 x 3584 at 128 / 200 / 256 rows 164 / 154 / 153 and 138 / 169 / 173, 18944 x 3584 96 / 107 / 108 and 103 / 128 /
+// and 248; 30000 x 3584 at 128 / 200 / 256 rows 164 / 154 / 153 and 138 / 169 / 173, 18944 x 3584 96 / 107 / 108 and 103 / 128 /
 // 127, 3584 x 18944 107 / 116 / 120 and 112 / 131 / 134, 4608 x 3584 44 / 46 / 47 and 40 / 46 / 49, 593 x 1984 41 / 41 / 41 and
 // 26 / 32 / 34).
 static bool decoded_route(const sq_matrix* mats, int n, int T) {
@@ -354,6 +356,13 @@ size_t gemm_workspace_without_mid(const sq_matrix* mats, int n, int T) {
     return need;
 }
 
+static size_t gathered_workspace(const sq_matrix* mats, int n) {
+    size_t need = 0;
+    for (int i = 0; i < n; ++i)
+        if (!fused_ok(mats[i])) need = std::max(need, dense_bytes(mats[i]));
+    return need;
+}
+
 static int run(const GemmArgs& a, int d, bool dense, hipStream_t s) {
     const dim3 grid((a.m.R + BN - 1) / BN, (a.T + BM - 1) / BM);
     if (dense) hipLaunchKernelGGL((gemm_kernel<8, true>), grid, dim3(256), 0, s, a);
@@ -371,7 +380,7 @@ int launch_gemm_dense(const void* w, int w_dtype, int64_t ldw, int R, int C, con
     if (!x_vec_ok(x, ldx, C) || !x_vec_ok(w, ldw, C))
         return fail(SQ_EUNSUPPORTED, "sq_gemm_dense: C, ldx, ldw must be multiples of 8 and pointers 16-byte aligned");
     if (x_dtype == SQ_F16 && w_dtype == SQ_F16 && T >= GEMM256_MIN_T && gemm256_ok(C, ldx, ldw, x, w)) {
-        const size_t part = gemm256_part_bytes(T, R, C, device_cus());
+        const size_t part = gemm_dense_workspace(R, C, T);      // (none is asked for where the last slab is broken)
         const bool split = ws && part && ws_bytes >= part;
         return launch_gemm256((const uint16_t*)x, ldx, (const uint16_t*)w, ldw, Gemm256Scales{}, y, y_dtype, ldy, 0, T, R, C,
                               split ? (float*)ws : nullptr, split ? device_cus() : 0, s);
@@ -418,9 +427,11 @@ int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_
     }
     if (decoded_route(mats, n, T) && decoded_workspace(mats, n, T) <= ws_bytes)
         return launch_decoded(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);
-    if (gemm_workspace_without_mid(mats, n, T) > ws_bytes)
+    const bool room = gemm_workspace_without_mid(mats, n, T) <= ws_bytes;
+    // (rows of a broken slab run in 128 x 128 tiles where the workspace holds less: what that kernel cannot gather itself)
+    if (!room && (mats[0].C % 64 == 0 || gathered_workspace(mats, n) > ws_bytes))
         return fail(SQ_EWORKSPACE, "sq_linear_gemm: workspace %zu < %zu", ws_bytes, gemm_workspace(mats, n, T));
-    if (big_route(mats, n, T)) {
+    if (room && big_route(mats, n, T)) {
         const int C = mats[0].C;
         const uint16_t* xh = (const uint16_t*)x;
         int64_t ldxh = ldx;
@@ -526,7 +537,7 @@ static int q8_chunk_rows(int V, int C) {
     return rows < V ? (int)rows : V;
 }
 
-static bool q8_big(int T, int C) { return T >= GEMM256_MIN_T && C % 64 == 0; }
+static bool q8_big(int T, int C) { return T >= GEMM256_MIN_T && C % 8 == 0; }
 
 size_t q8_workspace(int V, int C, int T) {
     if (T <= SQ_SMALL_BMAX || V <= 0) return 0;

@@ -4,7 +4,7 @@
 // 32 MT x 128 tile of v_mfma_f32_32x32x16_f16 accumulators (MT = 4: all 256 accumulator registers), one wave per SIMD.  Both
 // operands are K-contiguous fp16 in memory.  The K loop moves in slabs of 64 columns; a slab of ONE operand (rows of 128 bytes,
 // whole 128-byte lines: half-line requests get 10.5 TB/s out of L2 over the chip, whole lines 15.2 TB/s) is copied from global
-// memory straight into LDS (global_load_lds_dwordx4: no staging registers) into a ring of slots of that operand.  What a lone
+// memory straight into LDS (buffer_load_dwordx4 ... lds: no staging registers) into a ring of slots of that operand.  What a lone
 // wave per SIMD needs is that nothing in its instruction stream waits:
 //   * fragments are read one 16-column step ahead of their matrix instructions, one read behind each of the first ones;
 //   * one barrier per slab, two matrix instructions into the slab's last step, when its last fragments have arrived: it
@@ -132,13 +132,15 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a)
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
 
-    // Copies.  One global_load_lds_dwordx4 fills 1 KB = 8 LDS rows in lane order, so lane s lands in row
+    // Copies.  One buffer_load_dwordx4 to LDS fills 1 KB = 8 LDS rows in lane order, so lane s lands in row
     // s >> 3, slot s & 7 of its block and therefore fetches the piece the swizzle puts there.  Wave w copies
     // rows 64 w .. 64 w + 63 of a W slab (8 instructions) and a quarter of the X slab's rows.  Global addresses are a
     // uniform base (advanced per slab) plus per-lane 32-bit byte offsets computed once; rows past the matrix edge re-read
     // the last row (their outputs are never stored).  One operand is early (E slots, the copies of slab s + E - 1 go out during
     // the first steps of slab s), the other late (L = E - 1 slots, slab s + L goes out behind the barrier of slab s); slabs
-    // past the last one re-read the last.
+    // past the last one re-read the last.  The pieces of the row's last slab that lie past its end (C % 64 != 0) are asked for past the
+    // end of the buffer, which puts zeros into LDS, for both operands (global_load_lds instead of the buffers, for whole slabs: level;
+    // rows of broken slabs ran in the 128 x 128 kernel: 5120 x 2080 at 400 / 1500 rows 80-120 / 126-194 us, now 38-43 / 47-53).
     constexpr bool XE = gemm256_x_slots(MT) > gemm256_w_slots(MT);        // X is the early one
     constexpr int E = XE ? gemm256_x_slots(MT) : gemm256_w_slots(MT), L = E - 1, EC = XE ? XC : 8, LC = XE ? 8 : XC;
     static_assert(L == (XE ? gemm256_w_slots(MT) : gemm256_x_slots(MT)), "the waits below count on it");
@@ -158,20 +160,24 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a)
         const int r = r0 + row < a.R ? row : a.R - 1 - r0;
         wo[j] = (uint32_t)(r * (int)a.ldw + (slot ^ ((row >> 1) & 7)) * 8) * 2u;
     }
-    const int nk_all = a.C / G_BK, k_begin = (int)((int64_t)kz * nk_all / nparts);
+    const int nk_all = (a.C + G_BK - 1) / G_BK, k_begin = (int)((int64_t)kz * nk_all / nparts);
     const int nk = (int)((int64_t)(kz + 1) * nk_all / nparts) - k_begin;
     const char* xt = reinterpret_cast<const char*>(a.x + (int64_t)t0 * a.ldx + (int64_t)k_begin * G_BK);
     const char* wt = reinterpret_cast<const char*>(a.w + (int64_t)r0 * a.ldw + (int64_t)k_begin * G_BK);
-    typedef const __attribute__((address_space(1))) void* gptr_t;
     typedef __attribute__((address_space(3))) void* lptr_t;
-    auto copy = [&](const char* from, uint32_t off, int to) {
-        __builtin_amdgcn_global_load_lds((gptr_t)(from + off), (lptr_t)(smem + to), 16, 0, 0);
+    const int lastk = nk_all - 1 - k_begin;  // the row's last slab, counted from this part's first
+    bool past[2];                            // this lane's piece of it lies past the row's end, in even and odd copies (whose rows' swizzles differ by 4)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) past[h] = (slot ^ (h * 4 + (lrow >> 1))) * 8 >= a.C - (nk_all - 1) * G_BK;
+    auto copy = [&](const char* base, int q, uint32_t off, int j, int to) {
+        const int sb = q < nk ? q : nk - 1;
+        const __amdgpu_buffer_rsrc_t buf = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, 0xFFFFFF00u, 0x00027000);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, (lptr_t)(smem + to), 16, sb == lastk && past[j & 1] ? 0xFFFFFFF0u : off, sb * (G_BK * 2), 0, 0);
     };
-    auto copy_x = [&](const char* from, int sl, int j) { copy(from, xo[j], sl * X_SLOT + wave * (X_SLOT / 4) + j * 1024); };
-    auto copy_w = [&](const char* from, int sl, int j) { copy(from, wo[j], W_AT + sl * G_W_SLOT + wave * 8192 + j * 1024); };
-    auto slab = [&](int q) { return (q < nk ? q : nk - 1) * (G_BK * 2); };
-    auto copy_early = [&](int q, int sl, int j) { if constexpr (XE) copy_x(xt + slab(q), sl, j); else copy_w(wt + slab(q), sl, j); };
-    auto copy_late = [&](int q, int sl, int j) { if constexpr (XE) copy_w(wt + slab(q), sl, j); else copy_x(xt + slab(q), sl, j); };
+    auto copy_x = [&](int q, int sl, int j) { copy(xt, q, xo[j], j, sl * X_SLOT + wave * (X_SLOT / 4) + j * 1024); };
+    auto copy_w = [&](int q, int sl, int j) { copy(wt, q, wo[j], j, W_AT + sl * G_W_SLOT + wave * 8192 + j * 1024); };
+    auto copy_early = [&](int q, int sl, int j) { if constexpr (XE) copy_x(q, sl, j); else copy_w(q, sl, j); };
+    auto copy_late = [&](int q, int sl, int j) { if constexpr (XE) copy_w(q, sl, j); else copy_x(q, sl, j); };
 
     // Fragments.  A lane reads row (lane & 31) + 32 i of its wave's rows, piece 2 kk + (lane >> 5); the swizzle
     // term depends on the row modulo 16 only and the column step kk only flips bits 5-6 of the offset, so one
@@ -363,7 +369,7 @@ struct Gemm256Plan { int mt, main_tiles, tail_tiles, kt; };
 constexpr double G_SLAB[5] = {0, 0, 0.58, 0.73, 0.98}, G_SLAB_BUSY[5] = {0, 0, 0.42, 0.56, 0.70};
 
 static Gemm256Plan gemm256_plan(int T, int R, int C, int cus, bool split) {
-    const int slabs = C / G_BK;
+    const int slabs = (C + G_BK - 1) / G_BK;
     const bool rounds = cus >= 8 && cus % 8 == 0;
     const int n = rounds ? cus : 256;
     Gemm256Plan best{4, 0, 0, 1};
@@ -393,7 +399,7 @@ size_t gemm256_part_bytes(int T, int R, int C, int cus) {
 }
 
 bool gemm256_ok(int C, int64_t ldx, int64_t ldw, const void* x, const void* w) {
-    return C % 64 == 0 && ldx % 8 == 0 && ldw % 8 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0;
+    return C % 8 == 0 && ldx % 8 == 0 && ldw % 8 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0;
 }
 
 // x and w fp16.  `part` (gemm256_part_bytes) enables the split of the last round; NULL = no split.

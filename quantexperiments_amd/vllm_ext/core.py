@@ -250,7 +250,7 @@ class PackedShards:
             return linear_gemm(self.rls, x, y)
         # dequant + GEMM: whole pieces ("dequant") or row chunks of ~chunk_bytes ("chunked") decoded to
         # fp16 in the shared scratch, each multiplied into its column slice of Y
-        to_fp16 = x.dtype != torch.float16 and M > BMAX and self.C % 64 == 0    # fp16 x fp16 takes the tile kernel; y keeps its dtype
+        to_fp16 = x.dtype != torch.float16 and M > BMAX and self.C % 8 == 0     # fp16 x fp16 takes the tile kernel; y keeps its dtype
         if self.large == "dequant":
             copy = to_fp16 and x.dtype == torch.bfloat16 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
             if to_fp16 and not copy:

@@ -89,3 +89,32 @@ def test_dequant_route_in_groups_of_pieces(limit, T, monkeypatch):
     y = ps.forward(x.cuda())
     ref = np.concatenate([x.float().numpy().astype(np.float64) @ s.decode().astype(np.float64).T for s in ss], axis=1)
     assert rel_max_err(y.float().cpu().numpy(), ref) < 5e-3
+
+
+@pytest.mark.parametrize("T,R,C", [
+    (33, 70, 8), (64, 300, 56), (129, 257, 72), (200, 890, 8968), (333, 2000, 2040),      # tiles of 128 token rows, also split along K
+    (190, 60000, 88), (300, 34000, 4120), (250, 65700, 200), (510, 34000, 4104)])       # of 192 and 256
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_broken_slabs(T, R, C, dtype):
+    """Rows whose last slab of 64 columns is not whole, between columns that hold NaN."""
+    g = torch.Generator(device="cuda").manual_seed(T + R)
+    x, w = (torch.full((n, C + 72), float("nan"), dtype=torch.float16, device="cuda") for n in (T, R))
+    for t in (x, w):
+        t[:, :C] = torch.randn(t.shape[0], C, generator=g, device="cuda").half()
+    y = torch.full((T, R + 8), float("nan"), dtype=dtype, device="cuda")
+    gemm_dense(w[:, :C], x[:, :C], y[:, :R])
+    ref = x[:, :C].double() @ w[:, :C].double().T
+    bound = 17.4 * C * 2.0 ** -24 + (2.0 ** -8 * ref.abs() if dtype == torch.bfloat16 else 0.0)     # as in test_tile_heights
+    assert ((y[:, :R].double() - ref).abs() <= bound).all()
+    assert torch.isnan(y[:, R:]).all()
+
+
+@pytest.mark.parametrize("large", ["fused", "dequant"])
+@pytest.mark.parametrize("d,bits,G,M,C,T", [(4, 10, 4, 1, 1360, 300), (4, 12, 1, 1, 2056, 700), (8, 16, 1, 1, 1032, 260), (8, 16, 1, 3, 1096, 600), (4, 8, 1, 1, 1992, 257)])
+def test_broken_rows_in_tiles(d, bits, G, M, C, T, large):
+    ss = [synth(R, C, d, bits, G, M, seed=R) for R in (100, 41, 300)]
+    ps = core.PackedShards([to_device(s, stream=False) for s in ss], large=large)
+    x = rand_x(T, C, torch.bfloat16, seed=T)
+    y = ps.forward(x.cuda())
+    ref = np.concatenate([x.float().numpy().astype(np.float64) @ s.decode().astype(np.float64).T for s in ss], axis=1)
+    assert rel_max_err(y.float().cpu().numpy(), ref) < 5e-3
