@@ -184,9 +184,10 @@ void sq_stream_spin_limit(int32_t polls);
  * with a layout chosen for LDS gathers.
  *
  * The same two calls serve the formats whose codebook lives in LDS (d = 4 with 8-, 10- or 12-bit tags, one column
- * order, rows of whole 128/160/96-bit units): for them the buffer is a tile-major copy of the tags (the units of
- * each 16-row tile stored unit by unit, as large as the tags rounded up to 16 rows) that lets the decode-time
- * kernel read with fully coalesced loads; `runs` is ignored, *runs_out = *groups_out = 0, and the caller passes
+ * order, C % 8 == 0, W as short as the tags allow): for them the buffer is a tile-major copy of the tags (their 128/160/96-bit units of
+ * each 16-row tile stored unit by unit, as large as the tags rounded up to whole units and 16 rows) that lets the decode-time
+ * kernel read with fully coalesced loads, and rows that end within a unit, here filled up with zeros, take that kernel at all
+ * (up to SQ_SMALL_BMAX rows; without the copy they run on the vector kernels); `runs` is ignored, *runs_out = *groups_out = 0, and the caller passes
  * the device copy in sq_matrix.stream with stream_runs = stream_groups = 0.  It is optional like the slice
  * stream (the reference keeps such a copy too: shapequant/kernels/batched_runs.py tile_words); these formats
  * always need their tags. */

@@ -369,7 +369,7 @@ int sq_noalloc_reset(void* stream) {
 size_t sq_stream_bytes_balanced(const int32_t* tags_host, int32_t R, int32_t W, int32_t C, int32_t d, int32_t bits,
                                 const uint8_t* row_mask_host, int32_t runs, const void* table_host) {
     if (!tags_host || d <= 0 || (int64_t)W * 32 < (int64_t)(C / d) * bits) return 0;
-    if (!stream_format_ok(R, C, d, bits)) return !row_mask_host && tiled_format_ok(R, W, C, d, bits) ? tiled_bytes(R, W) : 0;
+    if (!stream_format_ok(R, C, d, bits)) return !row_mask_host && tiled_format_ok(R, W, C, d, bits) ? tiled_bytes(R, C, bits) : 0;
     return stream_bytes_host((const uint32_t*)tags_host, R, W, C, d, bits, row_mask_host, runs, (const uint16_t*)table_host);
 }
 
@@ -378,8 +378,8 @@ int sq_stream_build_balanced(const int32_t* tags_host, int32_t R, int32_t W, int
                              int32_t* runs_out, int32_t* groups_out) {
     if (!tags_host || !out_host || !runs_out || !groups_out) return fail(SQ_EINVAL, "sq_stream_build: null pointer");
     if (d > 0 && !stream_format_ok(R, C, d, bits) && !row_mask_host && tiled_format_ok(R, W, C, d, bits)) {
-        if (out_bytes < tiled_bytes(R, W)) return fail(SQ_EINVAL, "sq_stream_build: out_bytes %zu < %zu", out_bytes, tiled_bytes(R, W));
-        tiled_build((const uint32_t*)tags_host, R, W, bits, (uint32_t*)out_host);
+        if (out_bytes < tiled_bytes(R, C, bits)) return fail(SQ_EINVAL, "sq_stream_build: out_bytes %zu < %zu", out_bytes, tiled_bytes(R, C, bits));
+        tiled_build((const uint32_t*)tags_host, R, W, C, bits, (uint32_t*)out_host);
         *runs_out = 0;
         *groups_out = 0;
         return SQ_OK;

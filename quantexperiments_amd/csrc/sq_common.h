@@ -180,8 +180,11 @@ int launch_segs_group(const sq_matrix* mats, int cnt, const void* x, int x_dtype
 
 // tile-major copy of the tags for the matrix-core decode kernel (host routines, sq_gemv.hip)
 bool tiled_format_ok(int R, int W, int C, int d, int bits);
-size_t tiled_bytes(int R, int W);
-void tiled_build(const uint32_t* tags, int R, int W, int bits, uint32_t* out);
+int unit_dwords(int bits);
+int row_units(int C, int d, int bits);             // lane units of a row, the last one perhaps not whole
+bool whole_units(const sq_matrix& m);              // its rows are whole lane units, without pad bits
+size_t tiled_bytes(int R, int C, int bits);
+void tiled_build(const uint32_t* tags, int R, int W, int C, int bits, uint32_t* out);
 
 // the block-32 side formats (8-bit output head, 4-bit embedding)
 int launch_q8_small(const int8_t* q, const uint16_t* sc, int V, int C, const void* x, int x_dtype, int64_t ldx, void* y,

@@ -43,39 +43,42 @@ __global__ __launch_bounds__(256) void permute_x_kernel(const uint16_t* __restri
 int launch_small_generic(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y,
                          int y_dtype, int64_t ldy, int B, hipStream_t s);
 
-static int unit_dwords(int bits) { return bits == 12 ? 3 : bits == 10 ? 5 : 4; }
+int unit_dwords(int bits) { return bits == 12 ? 3 : bits == 10 ? 5 : 4; }
+int row_units(int C, int d, int bits) { const int tags = unit_dwords(bits) * 32 / bits; return (C / d + tags - 1) / tags; }
+
+bool whole_units(const sq_matrix& m) { return m.W % unit_dwords(m.bits) == 0 && (int64_t)(m.C / m.d) * m.bits == (int64_t)m.W * 32; }
 
 static bool fast_shape(const sq_matrix& m) {
     if (!m.tags) return false;                                   // held as its tag stream only
     const bool fmt = (m.d == 8 && m.bits == 16) || (m.d == 4 && (m.bits == 12 || m.bits == 10 || m.bits == 8));
     if (!fmt) return false;
-    if (m.W % unit_dwords(m.bits)) return false;                 // rows must be whole units
     if (((uintptr_t)m.tags & 15) || ((uintptr_t)m.table & 15)) return false;
-    if ((int64_t)(m.C / m.d) * m.bits != (int64_t)m.W * 32) return false;   // no pad bits inside the last unit
-    return true;
+    return whole_units(m);
 }
 
 // ---- tile-major copy of the tags for the matrix-core decode kernel (d = 4 formats, whose codebooks live in
 // LDS and which have no slice stream).  In the file's row-major layout the 16 lanes of a quarter wave read 16
 // different rows, 48 bytes each; in the copy the units of a 16-row tile are stored unit by unit,
 //     tiled[((t * U + u) * 16 + i) * UD + w] = tags[(16 t + i) * W + u * UD + w]      (rows past R: zeros)
-// so the same 16 lanes read 16 * UD consecutive dwords and a wave load covers one contiguous piece.
+// so the same 16 lanes read 16 * UD consecutive dwords and a wave load covers one contiguous piece.  Rows that end within a
+// unit (of whole pieces of 8 columns) have it filled up with zeros: in the copy every unit is whole, so these rows take the matrix-core
+// kernel too (5120 x 2064, 12-bit tags, at 2 / 16 / 32 rows on the vector kernel 27 / 134 / 264 us; now 6.5 / 7 / 10.5).
 bool tiled_format_ok(int R, int W, int C, int d, int bits) {
     if (!(d == 4 && (bits == 12 || bits == 10 || bits == 8))) return false;
-    if (R <= 0 || C % d || W % unit_dwords(bits)) return false;
-    return (int64_t)(C / d) * bits == (int64_t)W * 32;
+    if (R <= 0 || C <= 0 || C % 8) return false;
+    return ((int64_t)(C / d) * bits + 31) / 32 == W;
 }
 
-size_t tiled_bytes(int R, int W) { return (size_t)((R + 15) / 16) * 16 * W * 4; }
+size_t tiled_bytes(int R, int C, int bits) { return (size_t)((R + 15) / 16) * 16 * row_units(C, 4, bits) * unit_dwords(bits) * 4; }
 
-void tiled_build(const uint32_t* tags, int R, int W, int bits, uint32_t* out) {
-    const int ud = unit_dwords(bits), U = W / ud, ntiles = (R + 15) / 16;
+void tiled_build(const uint32_t* tags, int R, int W, int C, int bits, uint32_t* out) {
+    const int ud = unit_dwords(bits), U = row_units(C, 4, bits), ntiles = (R + 15) / 16;
     for (int t = 0; t < ntiles; ++t)
         for (int u = 0; u < U; ++u)
             for (int i = 0; i < 16; ++i) {
                 uint32_t* dst = out + (((size_t)t * U + u) * 16 + i) * ud;
                 const int r = t * 16 + i;
-                for (int w = 0; w < ud; ++w) dst[w] = r < R ? tags[(size_t)r * W + u * ud + w] : 0u;
+                for (int w = 0; w < ud; ++w) dst[w] = r < R && u * ud + w < W ? tags[(size_t)r * W + u * ud + w] : 0u;
             }
 }
 
@@ -137,6 +140,11 @@ static const uint32_t* tiled_piece(const sq_matrix& m) {
     return m.stream && !m.perms && tiled_format_ok(m.R, m.W, m.C, m.d, m.bits) && ((uintptr_t)m.stream & 15) == 0 ? (const uint32_t*)m.stream : nullptr;
 }
 
+// what the decode-time kernel takes: those shapes, and rows that end within a unit where they have a tile-major copy
+static bool mma_rows(const sq_matrix& m) {
+    return mma_shape(m) || (m.tags && !m.perms && ((uintptr_t)m.table & 15) == 0 && tiled_piece(m) && !whole_units(m) && ((int64_t)m.G << m.bits) * m.d * 2 <= 128 * 1024);
+}
+
 // bytes of codebook the matrix-core kernel stages in LDS (0: gathers go through the cache)
 static size_t mma_table_bytes(const sq_matrix& m) {
     const size_t tab = (size_t)m.G * ((size_t)1 << m.bits) * m.d * 2;
@@ -153,7 +161,7 @@ static size_t mma_table_bytes(const sq_matrix& m) {
 // token tiles the sums to add are twice as long and 3 waves are enough (6 waves of 1 round: 15.8, 3 of 2: 11.9, 2 x 8960 x 1536).
 static MmaPlan mma_plan(const sq_matrix& m, int B) {
     const int ud = unit_dwords(m.bits), tpu = ud * 32 / m.bits, spu = tpu / (8 / m.d);
-    const int rounds = (m.W / ud + 3) / 4, r1 = 32 / spu;
+    const int rounds = (row_units(m.C, m.d, m.bits) + 3) / 4, r1 = 32 / spu;
     MmaPlan best{0, 0, 0, 0};
     double best_cost = 1e30;
     const int NT = B > 16 ? 2 : 1;
@@ -190,7 +198,7 @@ static MmaPlan mma_whole_row(const sq_matrix& m, int B) {
     const size_t tab = mma_table_bytes(m);
     if (!tab || B > 16 || m.d != 4 || mma_plan(m, B).ks == 1) return none;
     const int ud = unit_dwords(m.bits), tpu = ud * 32 / m.bits, spu = tpu / (8 / m.d), rw = 32 / spu;
-    const int need = ((m.W / ud + 3) / 4 + rw - 1) / rw;
+    const int need = ((row_units(m.C, m.d, m.bits) + 3) / 4 + rw - 1) / rw;
     const size_t per_wave = std::max((size_t)64 * 16 * mma_pft(rw, 1), (size_t)mma_x_stage_bytes(tpu * m.d, mma_x_tokens_min(1)));
     if (need > (int)std::min<size_t>(mma_waves_max(rw * spu, true), (160 * 1024 - tab - 16) / per_wave)) return none;
     return MmaPlan{rw, 1, need, 1};
@@ -224,12 +232,16 @@ static size_t mma_part_bytes(const sq_matrix& m, int B) {
     return pl.ks > 1 ? ((((size_t)pl.ks * B * m.R * 4) + 255) & ~(size_t)255) : 0;
 }
 
+// Rows that end within a unit ran without a workspace before they had a copy: where it has no room for partial sums that only slices
+// of such a row need, they still do, on the vector kernels.
+static bool mma_without_room(const sq_matrix& m, int B) { return !whole_units(m) && mma_plan(m, B).ks > 1 && !mma_whole_row(m, B).KW; }
+
 // tight: the pieces that can run without partial sums do
 static size_t small_need(const sq_matrix* mats, int n, int B, bool tight) {
     size_t tot = 0;
     for (int i = 0; i < n; ++i) {
         if (stream_rows(mats[i], B)) continue;                   // its partial sums live in the workspace header
-        if (mma_shape(mats[i])) tot += tight && mma_whole_row(mats[i], B).KW ? 0 : mma_part_bytes(mats[i], B);
+        if (mma_rows(mats[i])) tot += tight && (mma_whole_row(mats[i], B).KW || mma_without_room(mats[i], B)) ? 0 : mma_part_bytes(mats[i], B);
         else if (mats[i].perms && fast_shape(mats[i])) tot += xp_bytes(mats[i], B);
     }
     return tot;
@@ -275,9 +287,10 @@ static int launch_mma_group(const sq_matrix* mats, int cnt, const void* x, int x
     MmaArgs a;
     a.n = cnt;
     a.x = (const uint16_t*)x; a.ldx = ldx; a.y = y; a.ldy = ldy; a.B = B; a.x_dtype = x_dtype; a.y_dtype = y_dtype;
-    a.U = m0.W / unit_dwords(m0.bits);
+    a.U = row_units(m0.C, m0.d, m0.bits);
     a.ks = pl.ks;
     a.act = act;
+    a.broken = !whole_units(m0);
     const int per = act ? 2 : 1;                                 // pieces whose tiles a workgroup walks in turn
     a.table_bytes = (int)mma_table_bytes(m0) * per;
     const int threads = pl.KW * 64;
@@ -429,9 +442,9 @@ int launch_small(const sq_matrix* mats, int n, const void* x, int x_dtype, int64
                 continue;
             }
         }
-        if (mma_shape(m0) && x_ok) {
+        if (mma_rows(m0) && x_ok && !(tight && mma_without_room(m0, B))) {
             int j = i + 1;
-            while (j < n && j - i < GEMV_MAX_PIECES && mma_shape(mats[j]) && mats[j].bits == m0.bits && mats[j].d == m0.d &&
+            while (j < n && j - i < GEMV_MAX_PIECES && mma_rows(mats[j]) && mats[j].bits == m0.bits && mats[j].d == m0.d &&
                    mats[j].W == m0.W && mats[j].G == m0.G && mats[j].R > 0)
                 ++j;
             int rc = launch_mma_group(mats + i, j - i, x, x_dtype, ldx, y, y_dtype, ldy, B, (char*)ws, ws_off, cus, s, false, tight);

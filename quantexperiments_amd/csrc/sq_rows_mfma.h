@@ -30,7 +30,7 @@ namespace sq {
 
 struct MmaPiece {
     sq_matrix m;
-    const uint32_t* tiled; // tile-major copy of the tags (sq_matrix.stream of a d = 4 format) or NULL
+    const uint32_t* tiled; // tile-major copy of the tags (sq_matrix.stream of a d = 4 format) or NULL (rows of whole units only)
     float* part;          // ks > 1: fp32 [ks, B, R] unscaled partial sums of this piece
     int wg_begin;         // first workgroup of this piece
     int wg_count;         // nshare * ks workgroups
@@ -50,6 +50,7 @@ struct MmaArgs {
     int table_bytes;      // bytes of codebook staged in LDS (0 = read through cache)
     int tg;               // codebook in LDS: 16-row tiles whose accumulators LDS holds between two barriers (a multiple of mma_group())
     int xt;               // tokens of a staging area: 16, or 8 (one token tile)
+    int broken;           // 1: the rows end within a unit (codebook in LDS, tile-major copies, no act)
     int act;              // 1: the two pieces are a gate and an up projection, y receives SiLU(gate) * up (16-bit)
 };
 
@@ -97,7 +98,9 @@ constexpr int mma_waves_max(int x_operands, bool lds_tab) { return !lds_tab ? 8 
 // two pieces' tiles in turn (virtual tile i: tile i / 2 of piece i % 2), and the wave that adds up a pair of tiles writes SiLU(gate) * up,
 // with the same roundings as the product followed by silu_mul_kernel.  It saves that launch and the trip of gate and up through memory
 // (2 x 18944 x 3584, 12-bit tags, 8 rows: 20.4 us, now 17.6).
-template <int BITS, int D, int RW, int NT, bool LDS_TAB, bool ACT = false, int XT = 16>
+// BROKEN (codebooks in LDS, tile-major copies): the row's last unit has columns past the row's end.  Their codewords, and those of the units
+// behind it, are read from 16 zero bytes behind the codebook (a choice per codeword, which whole rows do without).
+template <int BITS, int D, int RW, int NT, bool LDS_TAB, bool ACT = false, int XT = 16, bool BROKEN = false>
 __global__ __launch_bounds__(64 * mma_waves_max(RW * ((unit_of<BITS>::UD * 32 / BITS) / (8 / D)) * NT, LDS_TAB))
 void rows_mfma_kernel(MmaArgs a) {
     constexpr int UD = unit_of<BITS>::UD;
@@ -120,7 +123,7 @@ void rows_mfma_kernel(MmaArgs a) {
     const int t0 = (int)((int64_t)ntiles * share / nshare), t1 = (int)((int64_t)ntiles * (share + 1) / nshare);
     SQ_TRACE_POINT(0);
 
-    // LDS: [codebook][16 bytes, unused][reduction buffer: TT tiles x KW waves x 64 lanes x NT x 16 bytes]
+    // LDS: [codebook][16 bytes: zeros if BROKEN][reduction buffer: TT tiles x KW waves x 64 lanes x NT x 16 bytes]
     // (the codeword gathers form LDS addresses as numbers counted from the start of the dynamic LDS, which is address 0 in a
     // kernel without static LDS; a build in which it is not leaves y unwritten, which no test survives)
     if (LDS_TAB && (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)smem != 0u) return;
@@ -131,15 +134,15 @@ void rows_mfma_kernel(MmaArgs a) {
     bool live[RW];
     bool lane_live = true;
     uint32_t uoff[RW];
-    int ucol[RW];
+    int cols[RW];                            // columns of the row from this lane's unit on
 #pragma unroll
     for (int n = 0; n < RW; ++n) {
         const int u = 4 * (rbase + n) + lg;
         live[n] = u < a.U;
+        cols[n] = m.C - u * UK;
         lane_live = lane_live && live[n];
         const int uc = live[n] ? u : a.U - 1;
         uoff[n] = (uint32_t)uc * UD;
-        ucol[n] = uc * UK;
     }
     // Units past the row's end (only in waves that cover the tail of the columns) contribute exact zeros: their
     // activation operands are zero, and what they multiply with is the row's own last unit again (with the codebook in
@@ -267,10 +270,11 @@ void rows_mfma_kernel(MmaArgs a) {
                 for (int j = HALF; j < SPU; ++j) stage(xraw[n][nt][j], j * XTPI + xtl);
             exchange();
             const bool mine = live[n] && nt * 16 + li < a.B;
+            auto real = [&](int s) { return mine && (!BROKEN || s * 8 < cols[n]); };
 #pragma unroll
             for (int s = 0; s < SPU; ++s) {
                 u32x4 v = *reinterpret_cast<const u32x4*>(xmine + s * 16);
-                if (!(mine && (WHOLE || li < 8))) v = u32x4{0u, 0u, 0u, 0u};
+                if (!(real(s) && (WHOLE || li < 8))) v = u32x4{0u, 0u, 0u, 0u};
                 xb[n][s][nt] = __builtin_bit_cast(half8v, v);
             }
             exchange();
@@ -281,7 +285,7 @@ void rows_mfma_kernel(MmaArgs a) {
 #pragma unroll
                 for (int s = 0; s < SPU; ++s) {
                     const u32x4 v = *reinterpret_cast<const u32x4*>(xmine + s * 16);
-                    if (mine && li >= 8) xb[n][s][nt] = __builtin_bit_cast(half8v, v);
+                    if (real(s) && li >= 8) xb[n][s][nt] = __builtin_bit_cast(half8v, v);
                 }
                 exchange();
             }
@@ -299,6 +303,7 @@ void rows_mfma_kernel(MmaArgs a) {
     } else if (LDS_TAB) {
         stage_table(m.table, a.table_bytes, smem);
     }
+    if (BROKEN && tid < 4) reinterpret_cast<uint32_t*>(smem + a.table_bytes)[tid] = 0u;
     SQ_TRACE_POINT(1);
     // every wave has taken its operands out of the staging area (and, with the codebook in LDS, the codebook has landed
     // and the first tile's tags with it)
@@ -328,8 +333,10 @@ void rows_mfma_kernel(MmaArgs a) {
             } else {
                 u32x2 c0, c1;
                 if (LDS_TAB) {
-                    c0 = *reinterpret_cast<const mma_lds_u32x2*>((uintptr_t)unit_lds_offset<BITS, UD, 3>(cur.t[n], 2 * s, bo));
-                    c1 = *reinterpret_cast<const mma_lds_u32x2*>((uintptr_t)unit_lds_offset<BITS, UD, 3>(cur.t[n], 2 * s + 1, bo));
+                    uint32_t o0 = unit_lds_offset<BITS, UD, 3>(cur.t[n], 2 * s, bo), o1 = unit_lds_offset<BITS, UD, 3>(cur.t[n], 2 * s + 1, bo);
+                    if (BROKEN && s * 8 >= cols[n]) o0 = o1 = (uint32_t)a.table_bytes;
+                    c0 = *reinterpret_cast<const mma_lds_u32x2*>((uintptr_t)o0);
+                    c1 = *reinterpret_cast<const mma_lds_u32x2*>((uintptr_t)o1);
                 } else {
                     const uint32_t g0 = unit_tag<BITS, UD>(cur.t[n], 2 * s);
                     const uint32_t g1 = unit_tag<BITS, UD>(cur.t[n], 2 * s + 1);
@@ -521,18 +528,22 @@ static inline int mma_inst(int op, const MmaArgs& a, int grid, int threads, size
         if (a.table_bytes) k = rows_mfma_kernel<BITS, D, RW, NT, true>;
         if constexpr (NT == 1)
             if (a.xt == 8 && a.table_bytes) k = rows_mfma_kernel<BITS, D, RW, NT, true, false, 8>;
+        if (a.table_bytes && a.broken) k = rows_mfma_kernel<BITS, D, RW, NT, true, false, 16, true>;
+        if constexpr (NT == 1)
+            if (a.xt == 8 && a.table_bytes && a.broken) k = rows_mfma_kernel<BITS, D, RW, NT, true, false, 8, true>;
         if constexpr (!WIDEST) {
             if (a.table_bytes && a.act) k = rows_mfma_kernel<BITS, D, RW, NT, true, true>;
             if constexpr (NT == 1)
                 if (a.xt == 8 && a.table_bytes && a.act) k = rows_mfma_kernel<BITS, D, RW, NT, true, true, 8>;
         }
     }
+    if (a.broken && !(LDS && a.table_bytes)) return fail(SQ_EUNSUPPORTED, "sq_linear_small: rows that end within a lane unit need their codebook in LDS");
     if (a.table_bytes && (!LDS || (WIDEST && a.act)))
         return fail(SQ_EUNSUPPORTED, "sq_linear_small: no matrix-core kernel for %d rounds and codebooks in LDS", RW);
     if (op == 1) {
         static std::mutex mu;
         static std::unordered_map<uint64_t, int> cache;
-        const uint64_t key = ((uint64_t)threads << 40) | ((uint64_t)(a.table_bytes != 0) << 39) | ((uint64_t)a.act << 38) | ((uint64_t)(a.xt == 8) << 37) | (uint64_t)smem;
+        const uint64_t key = ((uint64_t)threads << 40) | ((uint64_t)(a.table_bytes != 0) << 39) | ((uint64_t)a.act << 38) | ((uint64_t)(a.xt == 8) << 37) | ((uint64_t)a.broken << 36) | (uint64_t)smem;
         std::lock_guard<std::mutex> lock(mu);
         auto it = cache.find(key);
         if (it != cache.end()) return it->second;

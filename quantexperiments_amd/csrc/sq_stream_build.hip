@@ -1051,8 +1051,7 @@ __global__ __launch_bounds__(256) void stream_fill_kernel(StreamFillStack stack)
 }
 
 // the tile-major copy of the tags (tiled_build) from tags in device memory: a thread moves one unit of a row
-__global__ __launch_bounds__(256) void tiled_build_kernel(const uint32_t* __restrict__ tags, int R, int W, int ud, uint32_t* __restrict__ out) {
-    const int U = W / ud;
+__global__ __launch_bounds__(256) void tiled_build_kernel(const uint32_t* __restrict__ tags, int R, int W, int U, int ud, uint32_t* __restrict__ out) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;          // (tile, unit, row of the tile)
     if (i >= (int64_t)((R + 15) / 16) * 16 * U) return;
     const int k = (int)(i & 15);
@@ -1060,7 +1059,7 @@ __global__ __launch_bounds__(256) void tiled_build_kernel(const uint32_t* __rest
     const int u = (int)(tu % U), r = (int)(tu / U) * 16 + k;
     uint32_t* dst = out + i * ud;
     const uint32_t* src = tags + (int64_t)r * W + u * ud;
-    for (int w = 0; w < ud; ++w) dst[w] = r < R ? src[w] : 0u;
+    for (int w = 0; w < ud; ++w) dst[w] = r < R && u * ud + w < W ? src[w] : 0u;
 }
 
 int stream_balance_device(const uint32_t* tags, int R, int W, int C, int d, int bits, uint32_t* counts, uint16_t* remap_out, int G,
@@ -1193,7 +1192,7 @@ int stream_plan_device(const uint32_t* tags, int R, int W, int C, int d, int bit
     D->tiled = !stream_format_ok(R, C, d, bits, G);
     D->in_lds = false;
     if (D->tiled) {
-        D->bytes = tiled_bytes(R, W);
+        D->bytes = tiled_bytes(R, C, bits);
         D->scratch = 0;
         *runs_out = *groups_out = 0;
     } else {
@@ -1275,10 +1274,10 @@ static int launch_stream_fill(const StreamFill* fills, int n, hipStream_t s) {
         const StreamDevicePlan& D = *fills[i].plan;
         unsigned char *out = fills[i].out, *scratch = fills[i].scratch;
         if (D.tiled) {
-            const int ud = D.bits == 12 ? 3 : D.bits == 10 ? 5 : 4;
-            const int64_t units = (int64_t)((D.R + 15) / 16) * 16 * (D.W / ud);
+            const int ud = unit_dwords(D.bits), U = row_units(D.C, D.d, D.bits);
+            const int64_t units = (int64_t)((D.R + 15) / 16) * 16 * U;
             if (units > 0)
-                hipLaunchKernelGGL(tiled_build_kernel, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, s, fills[i].tags, D.R, D.W, ud, (uint32_t*)out);
+                hipLaunchKernelGGL(tiled_build_kernel, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, s, fills[i].tags, D.R, D.W, U, ud, (uint32_t*)out);
             continue;
         }
         const StreamPlan& P = D.P;

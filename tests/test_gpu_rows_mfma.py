@@ -6,8 +6,9 @@ import pytest
 import torch
 
 from quantexperiments_amd import _lib
-from quantexperiments_amd.kernels import _Workspace, linear_small
-from tests.helpers import rand_x, rel_max_err, synth, to_device
+from quantexperiments_amd.kernels import _Workspace, linear_gemm, linear_small
+from oracle import sq_oracle as O
+from tests.helpers import rand_x, rel_max_err, synth, to_device, with_infinity
 
 pytestmark = pytest.mark.gpu
 
@@ -77,3 +78,49 @@ def test_products_that_need_no_sums_share_nothing(rows, C, bits, G, B, native, m
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, first) and bool((shared == 0x5A).all())
+
+
+@pytest.mark.parametrize("C,bits,G", [(8, 12, 1), (40, 10, 1), (72, 8, 1), (1360, 10, 4), (2056, 12, 1), (2080, 8, 4), (2928, 10, 1), (5624, 12, 4), (6168, 8, 1),
+                                      (8968, 12, 1), (17416, 10, 1)])
+@pytest.mark.parametrize("rows", [(1,), (300, 17)])
+def test_rows_that_end_within_a_unit(rows, C, bits, G):
+    """Their tile-major copy is filled up to whole units, and what lies behind a row stays out of its results: the columns of x (NaN here)
+    and the codewords of the filling (an infinity that no other tag names)."""
+    ss = [synth(R, C, 4, bits, G, 1, seed=R + C) for R in rows]
+    for s in ss:
+        s.tags[:] = np.maximum(s.tags, 1)
+        s.words[:] = O.pack_bits(s.tags, bits)
+        s.table[:: s.K] = np.inf
+    lins = [to_device(s) for s in ss]
+    assert all(m.stream_tiled for m in lins)
+    w = torch.cat([torch.from_numpy(s.decode()).cuda().double() for s in ss])
+    for B, dtype in ((1, torch.bfloat16), (2, torch.float16), (8, torch.bfloat16), (16, torch.float16), (17, torch.bfloat16), (32, torch.float16),
+                     (33, torch.bfloat16), (77, torch.float16), (200, torch.bfloat16), (260, torch.float16)):
+        x = torch.full((B, C + 64), float("nan"), dtype=dtype, device="cuda")
+        x[:, :C] = rand_x(B, C, dtype, seed=B).cuda()
+        x = x[:, :C]
+        y = torch.full((B, sum(rows)), float("nan"), device="cuda")
+        (linear_small if B <= 32 else linear_gemm)(lins, x, y)
+        assert rel_max_err(y.cpu().numpy(), (x.half().double() @ w.T).cpu().numpy()) < 1e-5, B      # (see above)
+
+
+def test_infinity_at_the_end_of_a_broken_row():
+    s = with_infinity(synth(70, 2056, 4, 12, seed=1), 5)
+    for B in (1, 8, 32):
+        x = rand_x(B, 2056, torch.float16, seed=B).abs() + 0.125
+        y = torch.empty(B, 70, device="cuda")
+        linear_small([to_device(s)], x.cuda(), y)
+        assert bool(torch.isposinf(y[:, 5]).all()) and bool(y[:, :5].isfinite().all()) and bool(y[:, 6:].isfinite().all())
+
+
+@pytest.mark.parametrize("C,B", [(2056, 16), (17416, 8), (17416, 40)])
+def test_rows_that_end_within_a_unit_without_a_workspace(C, B):
+    """What ran without one before such rows had a copy still does."""
+    L, dev = _lib.lib(), torch.device("cuda", torch.cuda.current_device())
+    s = synth(70, C, 4, 12, seed=C)
+    lin = to_device(s)
+    x = rand_x(B, C, torch.float16, seed=B).cuda()
+    y = torch.full((B, 70), float("nan"), device="cuda")
+    call = L.sq_linear_small if B <= 32 else L.sq_linear_gemm
+    _lib.check(call(_lib.matrix_array([lin.descriptor()]), 1, x.data_ptr(), _lib.SQ_F16, C, y.data_ptr(), _lib.SQ_F32, 70, B, None, 0, _lib.stream_ptr(dev)))
+    assert rel_max_err(y.cpu().numpy(), x.cpu().double().numpy() @ s.decode().astype(np.float64).T) < 1e-5

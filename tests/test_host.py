@@ -746,6 +746,32 @@ def test_tile_major_copy_of_d4_tags(R, C, bits):
             assert L.sq_stream_bytes(w2.ctypes.data_as(ctypes.c_void_p), R, w2.shape[1], C - 32, 4, bits, None, 0) == 0
 
 
+@pytest.mark.parametrize("R,C,bits", [(70, 392, 12), (16, 72, 8), (33, 648, 10), (1, 8, 12), (17, 88, 10)])
+def test_tile_major_copy_of_broken_rows(R, C, bits):
+    """Rows that end within a unit: as the copy of rows that go on to its end with zeros."""
+    import ctypes
+    from quantexperiments_amd import _lib
+    L = _lib.lib()
+    rng = np.random.default_rng(R + bits)
+    tags = rng.integers(0, 1 << bits, (R, C // 4))
+    words = np.ascontiguousarray(O.pack_bits(tags, bits))
+    ud, W = {12: 3, 10: 5, 8: 4}[bits], words.shape[1]
+    per, nt = ud * 32 // bits, -(-R // 16)
+    U = -(-(C // 4) // per)
+    full = O.pack_bits(np.pad(tags, ((0, 0), (0, U * per - C // 4))), bits)
+    padded = np.zeros((nt * 16, U * ud), np.int32)
+    padded[:R] = full
+    ptr = words.ctypes.data_as(ctypes.c_void_p)
+    n = L.sq_stream_bytes(ptr, R, W, C, 4, bits, None, 0)
+    assert n == padded.nbytes
+    out = np.full(n // 4, -1, np.int32)
+    r, g = ctypes.c_int32(7), ctypes.c_int32(7)
+    assert L.sq_stream_build(ptr, R, W, C, 4, bits, None, 0, out.ctypes.data_as(ctypes.c_void_p), n, ctypes.byref(r), ctypes.byref(g)) == 0
+    assert r.value == 0 and g.value == 0
+    assert np.array_equal(out, padded.reshape(nt, 16, U, ud).transpose(0, 2, 1, 3).reshape(-1))
+    assert L.sq_stream_bytes(ptr, R, W, C - 4, 4, bits, None, 0) == 0             # (rows of half pieces of 8 columns have none)
+
+
 class _TinyLM(torch.nn.Module):
     """The attributes aux_from_model reads off an HF causal LM."""
 
