@@ -248,13 +248,19 @@ static DecodedRows decoded_step(const sq_matrix* mats, int n, int& i, int& r0) {
 // and 248; 30000 x 3584 at 128 / 200 / 256 rows 164 / 154 / 153 and 138 / 169 / 173, 18944 x 3584 96 / 107 / 108 and 103 / 128 /
 // 127, 3584 x 18944 107 / 116 / 120 and 112 / 131 / 134, 4608 x 3584 44 / 46 / 47 and 40 / 46 / 49, 593 x 1984 41 / 41 / 41 and
 // 26 / 32 / 34).
+bool has_orders(const sq_matrix* mats, int n) {
+    for (int i = 0; i < n; ++i)
+        if (mats[i].perms) return true;
+    return false;
+}
+
 static bool decoded_route(const sq_matrix* mats, int n, int T) {
     int64_t rows = 0;
     for (int i = 0; i < n; ++i) {
         rows += mats[i].R;
         if (mats[i].R > 0 && (!mats[i].tags || !mid_dense_ok(mats + i, 1, T))) return false;
     }
-    if (mats[0].C % 64) return true;
+    if (mats[0].C % 64 || (T <= SQ_SMALL_BMAX && !has_orders(mats, n))) return true;
     return rows < (int64_t)128 * device_cus() && (T <= 128 || rows * mats[0].C < (int64_t)24 << 20);
 }
 
@@ -293,17 +299,24 @@ static int launch_decoded(const sq_matrix* mats, int n, const void* x, int x_dty
 // there and here: 4608 x 3584 46 / 89 us and 43, 37888 x 3584 81 / 118 and 237).  Without, each four rows cost as much again,
 // twice that on long rows (4 / 5 / 8 rows there, and any of them here: 593 x 1984 15 / 23 / 28 us and 18, 16000 x 3584 54 / 91 /
 // 103 and 78, 3584 x 18944 193 / 242 / 384 and 95, at 2 rows 97; 37888 x 3584 at 8 / 9 rows 194 / 272 and 237 in the tile GEMM).
+// Without orders, from VECTOR_DECODED_B rows, stacks of which the decode-time product would run a piece on the vector kernels: 16-bit tags of
+// rows that end within a lane unit, tags of other widths, codebooks beyond the cache (5120 x 2080, 16-bit tags, at 16 / 32 rows 212 /
+// 415 us there).
+constexpr int VECTOR_DECODED_B = 3;
 static bool masked_gemm(const sq_matrix* mats, int n, int B) {
-    bool orders = false;
-    for (int i = 0; i < n; ++i) orders = orders || mats[i].perms;
-    if (!orders) return false;
+    if (!has_orders(mats, n)) {
+        bool vector = false;
+        for (int i = 0; i < n; ++i) vector = vector || small_vector(mats[i], B);
+        return vector && B >= VECTOR_DECODED_B && decoded_route(mats, n, B);
+    }
     if (small_uses_sums(mats, n)) return decoded_route(mats, n, B) ? B >= 11 : B >= 17 && mats[0].C % 64 == 0;
     if (decoded_route(mats, n, B)) return B >= (mats[0].C > 8192 ? 3 : 5);
     return B >= 9 && mats[0].C % 64 == 0;
 }
 
-bool small_takes_gemm_route(const sq_matrix* mats, int n, int B, const void* x, int64_t ldx) {
-    return masked_gemm(mats, n, B) && x_vec_ok(x, ldx, mats[0].C);
+// (stacks without orders can do without: where the workspace has no room they run on the decode-time kernel)
+bool small_takes_gemm_route(const sq_matrix* mats, int n, int B, const void* x, int64_t ldx, size_t ws_bytes) {
+    return masked_gemm(mats, n, B) && x_vec_ok(x, ldx, mats[0].C) && (has_orders(mats, n) || decoded_workspace(mats, n, B) <= ws_bytes);
 }
 
 size_t small_gemm_route_workspace(const sq_matrix* mats, int n, int B) {
@@ -395,11 +408,12 @@ int launch_gemm_dense(const void* w, int w_dtype, int64_t ldw, int R, int C, con
 
 int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype,
                 int64_t ldy, int T, void* ws, size_t ws_bytes, void* sums, hipStream_t s) {
-    if (T <= SQ_SMALL_BMAX && !small_takes_gemm_route(mats, n, T, x, ldx))
+    if (T <= SQ_SMALL_BMAX && !small_takes_gemm_route(mats, n, T, x, ldx, ws_bytes))
         return launch_small(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, ws_bytes, sums, s);
     if (x_vec_ok(x, ldx, mats[0].C) && fused_route(mats, n, T) && fused_workspace(mats, n, T) <= ws_bytes)
         return launch_fused(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);
-    if (mid_ok(mats, n, T) && x_vec_ok(x, ldx, mats[0].C) && mid_x_ok(ldx, T)) return launch_mid(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, ws_bytes, s);
+    if (mid_ok(mats, n, T) && x_vec_ok(x, ldx, mats[0].C) && mid_x_ok(ldx, T))
+        return launch_mid(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, ws_bytes, s);
     if (T > SQ_SMALL_BMAX && T <= small_pass_limit(mats, n) && x_vec_ok(x, ldx, mats[0].C)) {
         // stacks that cannot go in one pass (pieces of different formats): a few passes of the decode-time kernel read the packed
         // tags a few times; decoding to fp16 first (below) writes and reads 8 to 16 times as many bytes once

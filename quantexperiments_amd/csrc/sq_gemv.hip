@@ -145,6 +145,8 @@ static bool mma_rows(const sq_matrix& m) {
     return mma_shape(m) || (m.tags && !m.perms && ((uintptr_t)m.table & 15) == 0 && tiled_piece(m) && !whole_units(m) && ((int64_t)m.G << m.bits) * m.d * 2 <= 128 * 1024);
 }
 
+bool small_vector(const sq_matrix& m, int B) { return m.R > 0 && m.tags && !m.perms && !stream_rows(m, B) && !mma_rows(m); }
+
 // bytes of codebook the matrix-core kernel stages in LDS (0: gathers go through the cache)
 static size_t mma_table_bytes(const sq_matrix& m) {
     const size_t tab = (size_t)m.G * ((size_t)1 << m.bits) * m.d * 2;

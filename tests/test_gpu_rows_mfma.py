@@ -124,3 +124,22 @@ def test_rows_that_end_within_a_unit_without_a_workspace(C, B):
     call = L.sq_linear_small if B <= 32 else L.sq_linear_gemm
     _lib.check(call(_lib.matrix_array([lin.descriptor()]), 1, x.data_ptr(), _lib.SQ_F16, C, y.data_ptr(), _lib.SQ_F32, 70, B, None, 0, _lib.stream_ptr(dev)))
     assert rel_max_err(y.cpu().numpy(), x.cpu().double().numpy() @ s.decode().astype(np.float64).T) < 1e-5
+
+
+@pytest.mark.parametrize("d,bits,C,G", [(8, 16, 2080, 1), (8, 16, 5000, 1), (8, 14, 1024, 1), (4, 14, 512, 1), (4, 12, 2056, 8), (8, 5, 264, 1)])
+@pytest.mark.parametrize("room", [True, False])
+def test_formats_of_the_vector_kernels(d, bits, C, G, room):
+    """From three rows their weights are decoded first, where the workspace has room."""
+    L, dev = _lib.lib(), torch.device("cuda", torch.cuda.current_device())
+    ss = [synth(R, C, d, bits, G, 1, seed=R) for R in (130, 9)]
+    lins = [to_device(s, stream=False) for s in ss]
+    w = np.concatenate([s.decode() for s in ss]).astype(np.float64)
+    for B in (2, 3, 9, 32):
+        x = rand_x(B, C, torch.bfloat16, seed=B).cuda()
+        y = torch.full((B, 139), float("nan"), device="cuda")
+        if room:
+            linear_small(lins, x, y)
+        else:
+            mats = _lib.matrix_array([lins[0].descriptor(0), lins[1].descriptor(130)])
+            _lib.check(L.sq_linear_small(mats, 2, x.data_ptr(), _lib.SQ_BF16, C, y.data_ptr(), _lib.SQ_F32, 139, B, None, 0, _lib.stream_ptr(dev)))
+        assert rel_max_err(y.cpu().numpy(), x.half().double().cpu().numpy() @ w.T) < 1e-5, B
