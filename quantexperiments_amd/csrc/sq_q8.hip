@@ -6,6 +6,7 @@
 // weight streaming for a handful of activation rows: every byte of q is read once from HBM and nothing is
 // reused, so the kernel is built around full-line loads (one wave load = 1 KB of one weight row), many loads in
 // flight per wave, and as few VALU operations per weight byte as the fp16 dot-product instruction allows.
+#include <type_traits>
 #include "sq_common.h"
 
 namespace sq {
@@ -181,7 +182,7 @@ __global__ __launch_bounds__(256, 2) void q8_gemv_kernel(Q8Args a) {
     }
 }
 
-// ---- 3 .. Q8_MFMA_MAX_ROWS activation rows (C % 64 == 0): fp16 MFMA, 16, 32 or 64 activation rows per pass.
+// ---- 3 .. Q8_MFMA_MAX_ROWS activation rows: fp16 MFMA, 16, 32 or 64 activation rows per pass.
 // v_mfma_f32_16x16x32_f16 operand layout: A: lane l supplies weight row l % 16, k = 8 * (l / 16) .. + 7; B: token
 // l % 16, the same k; D: lane l holds token l % 16, weight rows 4 * (l / 16) .. + 3.  Weights are the A operand and a
 // wave owns 16 rows.  The rows reach the wave through LDS: global_load_lds (no registers in between) fetches them in
@@ -228,25 +229,30 @@ constexpr int q8_vmcnt(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | 
 
 // weights ring + scales of d - 1 chunks (with a ring of 4 steps the scales of chunk c + 2 are requested while chunk c
 // is still being multiplied)
-constexpr int q8l_wave_bytes(int d) { return d * 2048 + (d - 1) * 256; }
-constexpr int q8l_lds_bytes(int nblk, int waves, int d, int xs) { return 2 * nblk * 16 * xs * 256 + waves * q8l_wave_bytes(d); }
+enum { Q8_CHUNKS, Q8_PAIRS, Q8_ODD };       // rows of whole 256-column chunks, of whole pairs of blocks, of an odd number of blocks
+constexpr int q8l_scale_bytes(int rows) { return rows == Q8_ODD ? 512 : 256; }
+constexpr int q8l_wave_bytes(int d, int rows) { return d * 2048 + (d - 1) * q8l_scale_bytes(rows); }
+constexpr int q8l_lds_bytes(int nblk, int waves, int d, int xs, int rows) { return 2 * nblk * 16 * xs * 256 + waves * q8l_wave_bytes(d, rows); }
 
 // NBLK 16-token blocks, WAVES waves per workgroup, ring of D steps per wave (one being multiplied, D - 1 in flight),
 // x chunks of XS steps (128 XS columns; a copy moves 4 / XS tokens, so the first 4 NBLK XS waves make one of every chunk, or all
 // waves XI of them)
-// ANY_C: rows of any whole pairs of blocks (C % 64 == 0).  The steps behind the row's end copy its last pieces again and multiply
-// nothing.  Such rows ran on the exact-product kernel, so their block scales stay out of the fp16 weights: a matrix instruction takes
+// ROWS: Q8_PAIRS (C % 64 == 0) and Q8_ODD are rows that end within a chunk.  The steps behind the row's end copy its last pieces again and
+// multiply nothing.  Such rows ran on the exact-product kernel, so their block scales stay out of the fp16 weights: a matrix instruction takes
 // the 32 columns of one block (lane group g: columns 8 g .. 8 g + 7) and its sums, fp32, are multiplied by the block's scales.
-template <int NBLK, int WAVES, int D, int XS, bool ANY_C>
+// Scales come in 4-byte pairs; every other row of an odd number of blocks begins within one, so there each comes by itself (a 2-byte copy per
+// lane, which leaves them 4 bytes apart; twice the copies).
+template <int NBLK, int WAVES, int D, int XS, int ROWS>
 __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel(Q8MfmaArgs a) {
     static_assert((D == 3 || D == 4) && (XS == 2 || (XS == 1 && D == 3)), "wait counts below are written out for these");
-    constexpr int Q8L_D = D, Q8L_WAVE_BYTES = q8l_wave_bytes(D);
+    constexpr bool ANY_C = ROWS != Q8_CHUNKS;
+    constexpr int Q8L_D = D, Q8L_WAVE_BYTES = q8l_wave_bytes(D, ROWS), SB = q8l_scale_bytes(ROWS), SC = SB / 256;      // SC: copies of a chunk's scales
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     unsigned char* xs = smem;                                   // [2][16 NBLK tokens][256 XS bytes]
     constexpr int XPITCH = XS * 256, XBUF = NBLK * 16 * XPITCH;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     unsigned char* wl = smem + 2 * XBUF + wave * Q8L_WAVE_BYTES;  // this wave's ring
-    unsigned char* sl_ = wl + Q8L_D * 2048;                        // this wave's scales: [D - 1][16 rows][16 bytes]
+    unsigned char* sl_ = wl + Q8L_D * 2048;                        // this wave's scales: [D - 1][16 rows][SB / 16 bytes]
     const int task_raw = blockIdx.x * WAVES + wave;
     const bool active = task_raw < a.tasks;
     const int task = active ? task_raw : a.tasks - 1;
@@ -293,10 +299,19 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel
         for (int n = 0; n < 2; ++n)
             __builtin_amdgcn_global_load_lds((gptr_t)(wsrc[n] + (ANY_C ? min(s * 128 + wcol[n], C - 16) : s * 128)), (lptr_t)(wl + (s % Q8L_D) * 2048 + n * 1024), 16, 0, 0);
     };
-    // scales of chunk c: lane i fetches dword i % 4 of row i / 4
+    // scales of chunk c: lane i fetches dword i % 4 of row i / 4 (Q8_ODD: scale i % 8 of rows i / 8 and 8 + i / 8)
+    const uint16_t* sodd[2];
+#pragma unroll
+    for (int n = 0; n < 2; ++n) sodd[n] = a.sc + (int64_t)min(task * 16 + 8 * n + (lane >> 3), a.V - 1) * nblk;
     const char* ssrc = (const char*)(a.sc + (int64_t)min(task * 16 + (lane >> 2), a.V - 1) * nblk) + (ANY_C ? 0 : (lane & 3) * 4);
     auto copy_s = [&](int c) {
-        __builtin_amdgcn_global_load_lds((gptr_t)(ssrc + (ANY_C ? min(c * 16 + (lane & 3) * 4, nblk * 2 - 4) : c * 16)), (lptr_t)(sl_ + (c % (D - 1)) * 256), 4, 0, 0);
+        if constexpr (ROWS == Q8_ODD) {
+#pragma unroll
+            for (int n = 0; n < 2; ++n)
+                __builtin_amdgcn_global_load_lds((gptr_t)(sodd[n] + min(c * 8 + (lane & 7), nblk - 1)), (lptr_t)(sl_ + (c % (D - 1)) * SB + n * 256), 2, 0, 0);
+            return;
+        }
+        __builtin_amdgcn_global_load_lds((gptr_t)(ssrc + (ANY_C ? min(c * 16 + (lane & 3) * 4, nblk * 2 - 4) : c * 16)), (lptr_t)(sl_ + (c % (D - 1)) * SB), 4, 0, 0);
     };
     const uint32_t xrow = (uint32_t)r * XPITCH, xsw = (uint32_t)r;
     const uint32_t wsw = (uint32_t)((r >> 1) & 7);
@@ -309,8 +324,8 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel
     // Issue order per wave (X = this wave's x copy of a chunk, S = scales of a chunk, W = the 2 copies of a step):
     // S(c) goes right before W(2c); step s starts (even s: after the wait and the barrier, then X(s/2 + 1)) with the
     // refill of step s + D - 1.  Waits count the operations that may stay in flight:
-    //   even s (needs X, S, W of its chunk):  D = 3: W(s+1) -> 2;           D = 4: W(s+1) S W(s+2) -> 5
-    //   odd s (needs W(s)):  D = 3: X S W(s+1) W(s+2) -> 5 + x;  D = 4: S W(s+1) X W(s+2) S W(s+3) -> 8 + x   (x: this wave's XI copies)
+    //   even s (needs X, S, W of its chunk):  D = 3: W(s+1) -> 2;           D = 4: W(s+1) S W(s+2) -> 4 + SC
+    //   odd s (needs W(s)):  D = 3: X S W(s+1) W(s+2) -> 4 + SC + x;  D = 4: S W(s+1) X W(s+2) S W(s+3) -> 6 + 2 SC + x   (x: this wave's XI copies)
     // and fall back to "everything" near the end of the row, where refills stop.
     auto refill = [&](int f) {
         if (f < nsteps) {
@@ -325,14 +340,14 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel
         const int c = s >> 1, odd = s & 1, cx = s / XS;         // chunk of scales, step in it, chunk of x
         if (XS == 1) {
             // every step opens an x chunk: X(s) was issued one step ago, before [S] W(s + 1)
-            if (s + 1 < nsteps) { if (odd) __builtin_amdgcn_s_waitcnt(q8_vmcnt(3)); else __builtin_amdgcn_s_waitcnt(q8_vmcnt(2)); }
+            if (s + 1 < nsteps) { if (odd) __builtin_amdgcn_s_waitcnt(q8_vmcnt(2 + SC)); else __builtin_amdgcn_s_waitcnt(q8_vmcnt(2)); }
             else __builtin_amdgcn_s_waitcnt(q8_vmcnt(0));
             __builtin_amdgcn_s_barrier();
             __builtin_amdgcn_sched_barrier(0);
             if (cx + 1 < nchunks) copy_x(cx + 1);
             refill(s + D - 1);
         } else if (!odd) {
-            if (s + D - 2 < nsteps) __builtin_amdgcn_s_waitcnt(q8_vmcnt(D == 3 ? 2 : 5));
+            if (s + D - 2 < nsteps) __builtin_amdgcn_s_waitcnt(q8_vmcnt(D == 3 ? 2 : 4 + SC));
             else __builtin_amdgcn_s_waitcnt(q8_vmcnt(0));
             __builtin_amdgcn_s_barrier();
             __builtin_amdgcn_sched_barrier(0);
@@ -341,8 +356,8 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel
         } else {
             refill(s + D - 1);
             if (s + D - 1 < nsteps) {
-                if (xo) __builtin_amdgcn_s_waitcnt(q8_vmcnt((D == 3 ? 5 : 8) + XI));
-                else __builtin_amdgcn_s_waitcnt(q8_vmcnt(D == 3 ? 5 : 8));
+                if (xo) __builtin_amdgcn_s_waitcnt(q8_vmcnt((D == 3 ? 4 + SC : 6 + 2 * SC) + XI));
+                else __builtin_amdgcn_s_waitcnt(q8_vmcnt(D == 3 ? 4 + SC : 6 + 2 * SC));
             } else {
                 __builtin_amdgcn_s_waitcnt(q8_vmcnt(0));
             }
@@ -350,9 +365,10 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel
         __builtin_amdgcn_sched_barrier(0);
         const unsigned char* st = wl + (s % Q8L_D) * 2048;
         if constexpr (ANY_C) {
-            u32x2 sb[4];                                        // the four blocks' scales of this lane's four output rows
+            typedef std::conditional_t<ROWS == Q8_ODD, u32x4, u32x2> scales_t;
+            scales_t sb[4];                                     // the four blocks' scales of this lane's four output rows
 #pragma unroll
-            for (int v = 0; v < 4; ++v) sb[v] = *reinterpret_cast<const u32x2*>(sl_ + (c % (D - 1)) * 256 + (4 * g + v) * 16 + odd * 8);
+            for (int v = 0; v < 4; ++v) sb[v] = *reinterpret_cast<const scales_t*>(sl_ + (c % (D - 1)) * SB + ((4 * g + v) * 2 + odd) * (SB / 32));
             const unsigned char* xc = xs + (cx & 1) * XBUF + xrow;
 #pragma unroll
             for (int b = 0; b < 4; ++b) {
@@ -366,7 +382,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
                     w[2 * k] = p[k][0]; w[2 * k + 1] = p[k][1];
-                    sf[k] = h2f((uint16_t)(sb[k][b >> 1] >> ((b & 1) * 16)));
+                    sf[k] = h2f((uint16_t)(ROWS == Q8_ODD ? sb[k][b] : sb[k][b >> 1] >> ((b & 1) * 16)));
                 }
                 const uint32_t px = (uint32_t)((s % XS) * 16 + b * 4 + g);
 #pragma unroll
@@ -381,7 +397,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel
             continue;
         }
         const u32x4 wq[2] = {*reinterpret_cast<const u32x4*>(st + w0), *reinterpret_cast<const u32x4*>(st + w1)};
-        const half_t sh = __builtin_bit_cast(half_t, *reinterpret_cast<const uint16_t*>(sl_ + (c % (D - 1)) * 256 + r * 16 + odd * 8 + g * 2));
+        const half_t sh = __builtin_bit_cast(half_t, *reinterpret_cast<const uint16_t*>(sl_ + (c % (D - 1)) * SB + r * 16 + odd * 8 + g * 2));
         const half2v s2 = {sh, sh};
         const unsigned char* xc = xs + (cx & 1) * XBUF + xrow;
 #pragma unroll
@@ -513,8 +529,8 @@ static int q8_pass_rows(int B, int C) {
     return nb;
 }
 
-// The MFMA passes need whole 4-byte pairs of block scales and 64 activation rows of C halves within 32-bit offsets.
-static bool q8_mfma_ok(int C) { return C % 64 == 0 && (int64_t)C * 64 < ((int64_t)1 << 31); }
+// The MFMA passes need 64 activation rows of C halves within 32-bit offsets.
+static bool q8_mfma_ok(int C) { return C % 32 == 0 && (int64_t)C * 64 < ((int64_t)1 << 31); }
 
 // from 3 rows the MFMA passes win over the 4-row kernel (152,064 x 3,584: 106 against 148 us; 248,320 x 5,120: 246
 // against 255 us); 2 rows stay on the exact-product kernel (106-115 / 228 us)
@@ -524,10 +540,14 @@ static bool q8_mfma_ok(int C) { return C % 64 == 0 && (int64_t)C * 64 < ((int64_
 // 15.1 / 12.1; 5 of 9,823 x 3,456 25.2 / 22.6, of 8,192 x 1,408 10.4 / 11.7; 16 of 1,024 x 1,408 23.3 / 12.4; 64 of 9,823 x 3,456 45.5 / 39,
 // of 16,000 x 3,456 59.5 / 38, of 8,211 x 576 33 / 18.  A second pass: 100 rows of
 // 30,000 x 1,216 41.3 / 41.9, of 32,000 x 640 33.6 / 27.6, of 50,000 x 3,520 203 / 106, 200 of 70,061 x 1,216 164 / 170.
+// Rows of an odd number of blocks: 8 / 16 / 32 / 64 rows of 150,000 x 3,488 246 / 490 / 974 / 877 (127 / 131 / 144 / 189 here), of 8,400 x 2,528 24 / 45 / 88 /
+// 95 (24 / 19 / 24 / 32), 4 of 60,000 x 2,080 39 / 30; of 30,000 x 608 both are done before an eager call is issued, 4 / 5 / 8 rows 14 / 17 / 20 there and 17.5
+// here, whose calls take a buffer and launch a copy of x.
 // 3 rows of 105,038 x 3,392, which the 256 MB last-level cache does not hold from call to call: 86.5 / 90.5; 5 take two passes there.
 bool q8_mid(int V, int C, int B) {
     if (B <= 2 || !q8_mfma_ok(C)) return false;
     if (C % 256 == 0) return B <= Q8_MFMA_MAX_ROWS;
+    if (C % 64 && B <= 5 && (int64_t)V * C < (int64_t)48 << 20) return false;
     if (B <= 4) return V >= 30000 && (int64_t)V * C <= (int64_t)240 << 20;
     if (B > 64) return V >= 30000 && B <= 128;
     if (B <= 8) return V >= 9000;
@@ -570,20 +590,19 @@ int launch_q8_mid(const int8_t* q, const uint16_t* sc, int V, int C, const void*
         // (970, 3.8 rounds) 265 against 278 us.
         const int cus = device_cus(), n16 = (tasks + 15) / 16;
         const bool x128 = (double)n16 / ((double)((n16 + cus - 1) / cus) * cus) < 0.85;
-        auto go = [&](void (*kernel)(Q8MfmaArgs), int waves, size_t lds) {
-            hipLaunchKernelGGL(kernel, dim3((unsigned)((tasks + waves - 1) / waves)), dim3((unsigned)waves * 64), lds, s, a);
+        const int rows = C % 256 == 0 ? Q8_CHUNKS : C % 64 == 0 ? Q8_PAIRS : Q8_ODD;
+        auto go = [&](auto chunks, auto pairs, auto odd, int nblk, int waves, int xs) {
+            hipLaunchKernelGGL(rows == Q8_CHUNKS ? chunks : rows == Q8_PAIRS ? pairs : odd, dim3((unsigned)((tasks + waves - 1) / waves)), dim3((unsigned)waves * 64),
+                               q8l_lds_bytes(nblk, waves, 3, xs, rows), s, a);
         };
         static bool raised = false;
         if (!raised) {
-            for (void (*k)(Q8MfmaArgs) : {q8_mfma_kernel<1, 8, 3, 2, false>, q8_mfma_kernel<2, 16, 3, 2, false>, q8_mfma_kernel<2, 8, 3, 1, false>,
-                                          q8_mfma_kernel<4, 16, 3, 1, false>, q8_mfma_kernel<1, 8, 3, 2, true>, q8_mfma_kernel<2, 16, 3, 2, true>,
-                                          q8_mfma_kernel<2, 8, 3, 1, true>, q8_mfma_kernel<4, 16, 3, 1, true>, q8_mfma_kernel<4, 8, 3, 1, false>,
-                                          q8_mfma_kernel<4, 8, 3, 1, true>})
-                (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+            auto raise = [](auto... k) { ((void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024), ...); };
+#define SQ_Q8(N, W, D, X) q8_mfma_kernel<N, W, D, X, Q8_CHUNKS>, q8_mfma_kernel<N, W, D, X, Q8_PAIRS>, q8_mfma_kernel<N, W, D, X, Q8_ODD>
+            raise(SQ_Q8(1, 8, 3, 2), SQ_Q8(2, 16, 3, 2), SQ_Q8(2, 8, 3, 1), SQ_Q8(4, 16, 3, 1), SQ_Q8(4, 8, 3, 1));
             (void)hipGetLastError();
             raised = true;
         }
-        const bool any = C % 256 != 0;
         // Small heads: half the waves per workgroup, each making twice the copies of x, spread the same waves over twice the CUs (a wave's
         // chain of LDS reads, conversions and matrix instructions is what they take).  us, before / so: 16 rows of 9,728 x 3,584 19.7 /
         // 17.8, of 10,000 x 2,048 12.7 / 12.1, of 30,000 x 2,048 14.3 / 14.8; 64 rows of 9,728 x 3,584 44.7 / 30.5, of 32,000 x 3,584 45.9 / 31.9,
@@ -591,19 +610,20 @@ int launch_q8_mid(const int8_t* q, const uint16_t* sc, int V, int C, const void*
         const int n8 = (tasks + 7) / 8;
         const bool small = a.B > 32 ? n8 <= cus : n8 <= cus / 2;
         if (small && a.B > 32)
-            go(any ? q8_mfma_kernel<4, 8, 3, 1, true> : q8_mfma_kernel<4, 8, 3, 1, false>, 8, q8l_lds_bytes(4, 8, 3, 1));
+            go(SQ_Q8(4, 8, 3, 1), 4, 8, 1);
         else if (small && a.B > 16)
-            go(any ? q8_mfma_kernel<2, 4, 3, 1, true> : q8_mfma_kernel<2, 4, 3, 1, false>, 4, q8l_lds_bytes(2, 4, 3, 1));
+            go(SQ_Q8(2, 4, 3, 1), 2, 4, 1);
         else if (small)
-            go(any ? q8_mfma_kernel<1, 4, 3, 2, true> : q8_mfma_kernel<1, 4, 3, 2, false>, 4, q8l_lds_bytes(1, 4, 3, 2));
+            go(SQ_Q8(1, 4, 3, 2), 1, 4, 2);
         else if (a.B > 32)                                           // 33-64 rows: 16 waves share 128-column chunks of 64 tokens
-            go(any ? q8_mfma_kernel<4, 16, 3, 1, true> : q8_mfma_kernel<4, 16, 3, 1, false>, 16, q8l_lds_bytes(4, 16, 3, 1));
+            go(SQ_Q8(4, 16, 3, 1), 4, 16, 1);
         else if (a.B > 16 && x128)
-            go(any ? q8_mfma_kernel<2, 8, 3, 1, true> : q8_mfma_kernel<2, 8, 3, 1, false>, 8, q8l_lds_bytes(2, 8, 3, 1));
+            go(SQ_Q8(2, 8, 3, 1), 2, 8, 1);
         else if (a.B > 16)
-            go(any ? q8_mfma_kernel<2, 16, 3, 2, true> : q8_mfma_kernel<2, 16, 3, 2, false>, 16, q8l_lds_bytes(2, 16, 3, 2));
+            go(SQ_Q8(2, 16, 3, 2), 2, 16, 2);
         else
-            go(any ? q8_mfma_kernel<1, 8, 3, 2, true> : q8_mfma_kernel<1, 8, 3, 2, false>, 8, q8l_lds_bytes(1, 8, 3, 2));
+            go(SQ_Q8(1, 8, 3, 2), 1, 8, 2);
+#undef SQ_Q8
         rc = check_launch("q8_mfma_kernel");
         if (rc) return rc;
         b0 += a.B;

@@ -349,3 +349,19 @@ def test_q8_products_of_broken_chunks_share_nothing(V, C, B, native, monkeypatch
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, want) and bool((shared == 0x5A).all())
+
+
+@pytest.mark.parametrize("V,C", [(1031, 32), (1040, 96), (1050, 224), (1900, 1376), (8100, 2144), (16001, 2528), (30003, 608)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_q8_rows_of_an_odd_number_of_blocks(V, C, dtype):
+    """As above; every other row's scales begin within a pair, and the last rows end where the buffers do."""
+    from quantexperiments_amd.kernels import q8_linear
+    q, sc, _ = _q8_parts(V, C, seed=V + C)
+    tq, ts = torch.from_numpy(q).cuda(), torch.from_numpy(sc).cuda()
+    for B in (3, 8, 16, 17, 32, 33, 64, 100):
+        x = rand_x(B, C + 8, dtype, seed=B).cuda()[:, :C]
+        y = torch.full((B, V + 2), 5.0, device="cuda")
+        q8_linear(tq, ts, x, y[:, :V])
+        exact = B <= 32 or V >= 30000 or (1024 <= V and B <= 64 and (V >= 8000 or C <= 2048))
+        assert rel_max_err(y[:, :V].cpu().numpy(), O.q8_linear(x.half().float().cpu().numpy(), q, sc)) < (1e-5 if exact else 2.0 ** -11), B
+        assert bool((y[:, V:] == 5.0).all())
