@@ -88,8 +88,8 @@ int sq_linear_small(const sq_matrix* mats, int32_t n_mats, const void* x, int x_
  * arguments, same kernels and bit-identical results, with the workspace (header included) kept in a device array
  * of SQ_NOALLOC_SCRATCH_BYTES that the library itself holds on every GPU it runs on until the process ends.  It has no
  * counterpart in the reference (whose launchers grow torch buffers on demand).  Pieces and row counts whose workspace
- * (sq_workspace_bytes(mats, n_mats, B, 0)) exceeds the array are refused with SQ_EWORKSPACE, except stacks with column orders
- * that need so much for their decoded weights only, without column orders, at up to 10 rows or with C % 64 != 0: those run on the decode-time
+ * (sq_workspace_bytes(mats, n_mats, B, 0)) exceeds the array are refused with SQ_EWORKSPACE, except stacks
+ * that need so much for their decoded weights only, where they have no column orders, up to 10 rows or C % 64 != 0: those run on the decode-time
  * kernel, whose results may differ from sq_linear_small's in the order of fp32 additions, and d = 4 pieces whose rows one launch
  * takes whole as well, which then differ in the same way (sq_linear_small with too small a workspace too).  Nothing is allocated or freed,
  * here or in anything it calls.  All calls on one GPU share that GPU's array: calls that overlap in time on one GPU
@@ -288,7 +288,7 @@ int sq_codebook_rebalance_device(const sq_matrix* mats, int32_t n, void* const* 
  * sq_q8_linear: Y[b, v] = sum_c X[b, c] * w[v, c] for B activation rows, fp32 accumulation with the block scale
  * applied to each block's fp32 sum (the reference kernel's arithmetic, shapequant/kernels/batched_runs.py:376-440).
  * One or two rows stream q through an exact-product kernel that needs no workspace; 3 .. 320 rows run fp16 MFMA passes of up to 64
- * rows with the block scale folded into the fp16 weight (one rounding) when C % 256 == 0, and, for other multiples of 64 and as far as
+ * rows with the block scale folded into the fp16 weight (one rounding) when C % 256 == 0, and, for other widths and as far as
  * they pay, with exact products and the scale on each block's fp32 sum (without a workspace up to SQ_SMALL_BMAX rows run on
  * the exact-product kernel, 4 per pass).  The passes need the workspace sq_q8_workspace_bytes names (an fp16 copy of
  * the activations).  It replaces gemv_q8_batched /
