@@ -107,15 +107,26 @@ template <int N, typename T> __device__ __forceinline__ int deal_below(T v) {
     else return (int)(ror16<N>(v) < v) + deal_below<N + 1>(v);
 }
 
+// A step of the dealing: of sorted codewords k .. k + n - 1, number j goes to the slice of rank j % nf, whose next free label is base[j % nf]
+// before the step, as its j / nf-th.
+struct DealStep {
+    uint32_t k, n, nf, inverse;              // inverse: j / nf for j <= 65536 is the high half of j * inverse (nf > 1)
+    uint16_t base[16];
+};
+constexpr int DEAL_STEPS = 256, DEAL_LONG = 4096;
+static_assert(DEAL_STEPS * sizeof(DealStep) <= DEAL_WAVES * 256 * 4, "the steps lie where the digits were counted");
+
 // One workgroup per codebook.  Codewords go, most used first (equal counts by id), to the slice with the fewest tags so far that
 // has room (ties: the lowest).  What bounds it is that this is a chain of 65,536 choices, 4 ms at 150 clocks each.  But of
 // codewords of equal count c the slices whose loads lie less than c above the least take one each, in order of load, before any
 // gets a second one or a slice that is further behind gets one; so a step deals a round to those slices, or as many rounds as
-// leave that so.  The codewords are sorted by count with a stable radix sort, 8 bits a pass (counts below 256 tags a codeword
-// are one), ids in LDS and between two passes in registers (a wave owns a 16th of them).
-// 65,536 codewords: 3584 x 448 evenly spread tags 155 us (sorting 65, the runs' starts 34, 73 steps 55), 18944 x 448 215, 5120 x
-// 640 of a power law 1.04 ms (1162 steps).  On the host, with the copies and the synchronisation around it, 480 us of a load for
-// every matrix of a stack, now 155 for all of them.
+// leave that so.  One wave works the steps out, up to DEAL_STEPS ahead (its chain is instructions: with all sixteen doing the same beside
+// it a step took twice as long), then all write the codewords' labels.  The codewords are sorted by count with a stable radix sort, 8 bits
+// a pass, ids in LDS and between two passes in registers (a wave owns a 16th of them); counts below 256, the usual ones, are one pass of
+// as many bits as they have, read from the counts in order, and its digits' places are where the runs of equal counts start.
+// 65,536 codewords: 3584 x 448 evenly spread tags 95 us (sorting 40, 73 steps 42, labels 19), 190 with the sort in general passes, the runs' starts
+// searched in the sorted counts and every wave at the steps; 1057 x 64 58, 130; 5120 x 640 of a power law 0.89 ms (a load of that matrix 2.62 ms, 3.23).
+// On the host, with the copies and the synchronisation around it, 480 us of a load for every matrix of a stack.
 template <int PER, typename T>               // ids per lane: K / DEAL_NT (0: codebooks of one slice); a slice's tags (less than 2^(bits - 4))
 __global__ __launch_bounds__(DEAL_NT) void deal_kernel(RelabelArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char deal_lds[];
@@ -130,151 +141,265 @@ __global__ __launch_bounds__(DEAL_NT) void deal_kernel(RelabelArgs a) {
         for (int k = tid; k < K; k += DEAL_NT) remap[k] = (uint16_t)k;
     } else {
     uint16_t* ids = reinterpret_cast<uint16_t*>(deal_lds);                  // [65536]
-    uint32_t* ctr = reinterpret_cast<uint32_t*>(deal_lds + 65536 * 2);      // [digit][wave]
+    uint32_t* ctr = reinterpret_cast<uint32_t*>(deal_lds + 65536 * 2);      // [wave][digit]
     uint16_t* starts = reinterpret_cast<uint16_t*>(ctr + DEAL_WAVES * 256);
     __shared__ uint32_t shared_most, wave_sum4[4], wave_starts[DEAL_WAVES];
+    __shared__ int shared_steps, shared_long;
 
     const int w0 = wave * (K / DEAL_WAVES);                                 // the wave's first id
     uint32_t most = 0;
 #pragma unroll 8
-    for (int i = 0; i < PER; ++i) {
-        const int k = i * DEAL_NT + tid;
-        most = max(most, count[k]);
-        ids[k] = (uint16_t)k;
-    }
+    for (int i = 0; i < PER; ++i) most = max(most, count[w0 + i * 64 + lane]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) most = max(most, (uint32_t)__shfl_xor((int)most, o, 64));
     if (tid == 0) shared_most = 0u;
     __syncthreads();
-    atomicMax(&shared_most, most);
+    if (lane == 0) atomicMax(&shared_most, most);
     __syncthreads();
-    most = shared_most;
-    for (int shift = 0; shift < 32 && (most >> shift) != 0; shift += 8) {
+    most = (uint32_t)__builtin_amdgcn_readfirstlane((int)shared_most);
+    const bool single = most < 256;
+    const int nb = single ? max(1, 32 - __builtin_clz(most | 1u)) : 8;       // bits of a digit; the largest comes first
+    const uint32_t top = (1u << nb) - 1u;
+    int runs = 0;
+    auto clear = [&]() {
         for (int k = tid; k < DEAL_WAVES * 256; k += DEAL_NT) ctr[k] = 0u;
         __syncthreads();
-        uint32_t held[PER / 2], digits[PER / 4];                            // ids in pairs, digits in fours
-#pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            if (i % 8 == 0) __builtin_amdgcn_sched_barrier(0);              // (as many loads at a time as there are registers for)
-            const uint32_t id = ids[w0 + i * 64 + lane], dg = 255u - ((count[id] >> shift) & 255u);
-            held[i / 2] = i % 2 ? held[i / 2] | id << 16 : id;
-            digits[i / 4] = i % 4 ? digits[i / 4] | dg << (8 * (i % 4)) : dg;
-            // (a wave all of whose digits are the same, as the high ones mostly are, would queue at one counter)
-            if (__all((int)dg == __builtin_amdgcn_readfirstlane((int)dg))) { if (lane == 0) atomicAdd(&ctr[dg * DEAL_WAVES + wave], 64u); }
-            else atomicAdd(&ctr[dg * DEAL_WAVES + wave], 1u);
-        }
+    };
+    auto tally = [&](uint32_t dg) {          // (a wave all of whose digits are the same, as the high ones mostly are, would queue at one counter)
+        if (__all((int)dg == __builtin_amdgcn_readfirstlane((int)dg))) { if (lane == 0) atomicAdd(&ctr[wave * 256 + dg], 64u); }
+        else atomicAdd(&ctr[wave * 256 + dg], 1u);
+    };
+    // exclusive sums over (digit, wave): thread d < 256 takes the 16 waves of digit d.  The digits in use are the runs of a single pass.
+    auto sums = [&]() {
         __syncthreads();
-#pragma unroll
-        for (int i = 0; i < PER / 2; ++i) asm volatile("" : "+v"(held[i]));  // (kept packed: unpacked ahead of their use they spill)
-#pragma unroll
-        for (int i = 0; i < PER / 4; ++i) asm volatile("" : "+v"(digits[i]));
-        // exclusive sums over (digit, wave): thread d < 256 takes the 16 waves of digit d
         uint32_t mine = 0, before = 0;
+        uint64_t used = 0;
         if (tid < 256) {
-            for (int w = 0; w < DEAL_WAVES; ++w) mine += ctr[tid * DEAL_WAVES + w];
+            for (int w = 0; w < DEAL_WAVES; ++w) mine += ctr[w * 256 + tid];
             before = mine;
 #pragma unroll
             for (int o = 1; o < 64; o <<= 1) {
                 const uint32_t v = __shfl_up(before, o, 64);
                 if (lane >= o) before += v;
             }
-            if (lane == 63) wave_sum4[wave] = before;
+            used = __ballot(mine > 0);
+            if (lane == 63) {
+                wave_sum4[wave] = before;
+                wave_starts[wave] = (uint32_t)__popcll(used);
+            }
         }
         __syncthreads();
+        runs = (int)(wave_starts[0] + wave_starts[1] + wave_starts[2] + wave_starts[3]);
         if (tid < 256) {
-            uint32_t at = before - mine;
-            for (int w = 0; w < wave; ++w) at += wave_sum4[w];
+            uint32_t at = before - mine, run = (uint32_t)__popcll(used & (((uint64_t)1 << lane) - 1));
+            for (int w = 0; w < wave; ++w) {
+                at += wave_sum4[w];
+                run += wave_starts[w];
+            }
+            if (mine > 0) starts[run] = (uint16_t)at;
             for (int w = 0; w < DEAL_WAVES; ++w) {
-                const uint32_t n = ctr[tid * DEAL_WAVES + w];
-                ctr[tid * DEAL_WAVES + w] = at;
+                const uint32_t n = ctr[w * 256 + tid];
+                ctr[w * 256 + tid] = at;
                 at += n;
             }
         }
         __syncthreads();
+    };
+    auto place = [&](uint32_t dg, uint32_t id, int bits) {
+        uint32_t lo = ~0u, hi = ~0u;                                        // the lanes whose digit is the same
+#pragma unroll
+        for (int b = 0; b < bits; ++b) {
+            const uint32_t mask = (uint32_t)-(int)((dg >> b) & 1);
+            const uint64_t set = __ballot(mask != 0);
+            lo &= ~((uint32_t)set ^ mask);
+            hi &= ~((uint32_t)(set >> 32) ^ mask);
+        }
+        const uint64_t same = (uint64_t)hi << 32 | lo;
+        const int rank = __popcll(same & (((uint64_t)1 << lane) - 1));
+        volatile uint32_t* c = &ctr[wave * 256 + dg];                // (this wave's counter: its LDS accesses stay in order)
+        const uint32_t at = *c;
+        ids[at + rank] = (uint16_t)id;
+        if (rank == 0) *c = at + (uint32_t)__popcll(same);
+        __threadfence_block();
+    };
+    if (single) {
+        clear();
+        // (few digits: 2^copies counters of each, its lanes dealt among them, or they would queue: 4 bits 24 us, now 7)
+        const int copies = nb <= 6 ? 8 - nb : 0;
+        uint32_t* mine = ctr + wave * 256;
+#pragma unroll 8
+        for (int i = 0; i < PER; ++i) atomicAdd(&mine[(top - count[w0 + i * 64 + lane]) << copies | (uint32_t)(lane & ((1 << copies) - 1))], 1u);
+        if (copies) {
+            const u32x4 four = *reinterpret_cast<const u32x4*>(mine + lane * 4);
+            uint32_t of = four.x + four.y + four.z + four.w;
+            for (int o = 1; o < 1 << (copies - 2); o <<= 1) of += (uint32_t)__shfl_xor((int)of, o, 64);
+            __threadfence_block();           // (a wave's own counters: its LDS accesses stay in order)
+            *reinterpret_cast<u32x4*>(mine + lane * 4) = u32x4{0u, 0u, 0u, 0u};
+            __threadfence_block();
+            if ((lane & ((1 << (copies - 2)) - 1)) == 0) mine[lane >> (copies - 2)] = of;
+        }
+        sums();
+        for (int i0 = 0; i0 < PER; i0 += 8) {
+            uint32_t c8[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) c8[i] = count[w0 + (i0 + i) * 64 + lane];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) place(top - c8[i], (uint32_t)(w0 + (i0 + i) * 64 + lane), nb);
+        }
+        __syncthreads();
+    } else {
+#pragma unroll 8
+        for (int i = 0; i < PER; ++i) ids[w0 + i * 64 + lane] = (uint16_t)(w0 + i * 64 + lane);
+    }
+    for (int shift = 0; !single && shift < 32 && (most >> shift) != 0; shift += 8) {
+        clear();
+        uint32_t held[PER / 2];                                             // ids in pairs
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
-            __builtin_amdgcn_sched_barrier(0);
-            const uint32_t dg = (digits[i / 4] >> (8 * (i % 4))) & 255u;
-            uint64_t same = ~(uint64_t)0;
+            if (i % 8 == 0) __builtin_amdgcn_sched_barrier(0);              // (as many loads at a time as there are registers for)
+            const uint32_t id = ids[w0 + i * 64 + lane];
+            held[i / 2] = i % 2 ? held[i / 2] | id << 16 : id;
+            tally(top - ((count[id] >> shift) & 255u));
+        }
 #pragma unroll
-            for (int b = 0; b < 8; ++b) {
-                const uint64_t set = __ballot((dg >> b) & 1);
-                same &= (dg >> b) & 1 ? set : ~set;
+        for (int i = 0; i < PER / 2; ++i) asm volatile("" : "+v"(held[i]));  // (kept packed: unpacked ahead of their use they spill)
+        sums();
+#pragma unroll
+        for (int i = 0; i < PER; i += 8) {
+            __builtin_amdgcn_sched_barrier(0);
+            uint32_t c8[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) c8[j] = count[(held[(i + j) / 2] >> (16 * (j % 2))) & 0xFFFFu];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                __builtin_amdgcn_sched_barrier(0);
+                place(top - ((c8[j] >> shift) & 255u), held[(i + j) / 2] >> (16 * (j % 2)), 8);
             }
-            const int rank = __popcll(same & (((uint64_t)1 << lane) - 1));
-            volatile uint32_t* c = &ctr[dg * DEAL_WAVES + wave];            // (this wave's counter: its LDS accesses stay in order)
-            const uint32_t at = *c;
-            ids[at + rank] = (uint16_t)(held[i / 2] >> (16 * (i % 2)));
-            if (rank == 0) *c = at + (uint32_t)__popcll(same);
-            __threadfence_block();
         }
         __syncthreads();
     }
 
-    // where runs of equal counts start, in order
-    int found = 0;
-    uint64_t firsts = 0;                                                    // bit i: this lane's id i starts one
+    if (!single) {                           // where runs of equal counts start, in order
+        int found = 0;
+        uint64_t firsts = 0;                                                // bit i: this lane's id i starts one
 #pragma unroll 8
-    for (int i = 0; i < PER; ++i) {
-        const int k = w0 + i * 64 + lane;
-        const bool first = k == 0 || count[ids[k]] != count[ids[k - 1]];
-        firsts |= (uint64_t)first << i;
-        found += __popcll(__ballot(first));
-    }
-    if (lane == 0) wave_starts[wave] = (uint32_t)found;
-    __syncthreads();
-    int at = 0, runs = 0;
-    for (int w = 0; w < DEAL_WAVES; ++w) {
-        if (w < wave) at += (int)wave_starts[w];
-        runs += (int)wave_starts[w];
-    }
-#pragma unroll 8
-    for (int i = 0; i < PER; ++i) {
-        const bool first = firsts >> i & 1;
-        const uint64_t all = __ballot(first);
-        const int o = at + __popcll(all & (((uint64_t)1 << lane) - 1));
-        if (first && o < DEAL_RUNS) starts[o] = (uint16_t)(w0 + i * 64 + lane);
-        at += __popcll(all);
-    }
-    __syncthreads();
-
-    // every wave deals, each the same; of the codewords of one step a wave writes every 16th group of 64
-    T load = 0;                                                             // tags and codewords of slice sl
-    int fill = 0;
-    auto deal = [&](int k, int m, T c) {
-        while (m > 0) {
-            const bool open = sl < NS && fill < DEAL_SLICE;
-            const T none = ~(T)0, key = open ? load << 4 | (T)sl : none, least = deal_min16(key), lo = least >> 4;
-            // the slices that are next (c = 0: the least loaded one until it is full) and their order
-            const bool next = open && (c ? load - lo < c : key == least);
-            const int nf = __popcll(__ballot(next) & 0xFFFF), below = deal_below<1>(key), rank = next ? below : 16;
-            const int by_rank = __builtin_amdgcn_ds_permute(((lane & 48) | (next ? rank : 15)) * 4, sl);
-            const int room = (int)deal_min16((uint32_t)(next ? DEAL_SLICE - fill : DEAL_SLICE));
-            // whole rounds: until the codewords or the room end, or the least loaded of them passes one that was behind
-            int q = min(m / nf, room), last = room;
-            const T above = deal_min16(open && !next ? load : none);
-            if (c && above != none && above - lo < (uint64_t)c * (uint64_t)(q + 1)) last = min(room, (int)((above - lo) / c));
-            q = min(q, last);
-            const int rem = q == m / nf && q < last ? m - q * nf : 0, n = q * nf + rem;
-            const uint32_t inverse = 0xFFFFFFFFu / (uint32_t)nf + 1u;       // j / nf for j < 65536 from the high half of a product
-            for (int j0 = wave * 64; j0 < n; j0 += DEAL_NT) {
-                const int j = j0 + lane, round = nf == 1 ? j : (int)__umulhi((uint32_t)j, inverse), s = __shfl(by_rank, j - round * nf, 64), place = __shfl(fill, s, 64) + round;
-                if (j < n) remap[ids[k + j]] = (uint16_t)(s * DEAL_SLICE + place);
-            }
-            const int got = next ? q + (rank < rem) : 0;
-            load += c * (T)got;
-            fill += got;
-            k += n;
-            m -= n;
+        for (int i = 0; i < PER; ++i) {
+            const int k = w0 + i * 64 + lane;
+            const bool first = k == 0 || count[ids[k]] != count[ids[k - 1]];
+            firsts |= (uint64_t)first << i;
+            found += __popcll(__ballot(first));
         }
-    };
-    const int listed = min(runs, DEAL_RUNS);
-    for (int r0 = 0; r0 < listed; r0 += 64) {
-        const int r = min(r0 + lane, listed - 1), k = starts[r], end = r + 1 < listed ? starts[r + 1] : listed == runs ? K : k + 1;
-        const uint32_t c = count[ids[k]];
-        for (int i = 0; i < min(64, listed - r0); ++i)
-            deal(__builtin_amdgcn_readlane(k, i), __builtin_amdgcn_readlane(end - k, i), (uint32_t)__builtin_amdgcn_readlane((int)c, i));
+        if (lane == 0) wave_starts[wave] = (uint32_t)found;
+        __syncthreads();
+        int at = 0;
+        runs = 0;
+        for (int w = 0; w < DEAL_WAVES; ++w) {
+            if (w < wave) at += (int)wave_starts[w];
+            runs += (int)wave_starts[w];
+        }
+#pragma unroll 8
+        for (int i = 0; i < PER; ++i) {
+            const bool first = firsts >> i & 1;
+            const uint64_t all = __ballot(first);
+            const int o = at + __popcll(all & (((uint64_t)1 << lane) - 1));
+            if (first && o < DEAL_RUNS) starts[o] = (uint16_t)(w0 + i * 64 + lane);
+            at += __popcll(all);
+        }
+        __syncthreads();
     }
-    if (listed < runs)
-        for (int k = starts[listed - 1] + 1; k < K; ++k) deal(k, 1, (uint32_t)__builtin_amdgcn_readfirstlane((int)count[ids[k]]));
+
+    DealStep* steps = reinterpret_cast<DealStep*>(ctr);
+    // wave 0: tags and codewords of slice sl; 64 runs at a time, one a lane (behind DEAL_RUNS of them 64 codewords), and what is left of the run it deals
+    const int listed = min(runs, DEAL_RUNS);
+    T load = 0, c = 0;
+    int fill = 0, next_run = 0, next_lone = listed < runs ? starts[listed - 1] + 1 : K, have = 0, at = 0, lane_k = 0, lane_m = 0, k = 0, m = 0;
+    uint32_t lane_c = 0, lane_r = 0, recip = 0;
+    const uint32_t lane_inverse = lane > 1 ? 0xFFFFFFFFu / (uint32_t)lane + 1u : 0u;       // (of nf = 2 .. 16, divisions out of the chain)
+    bool more = true;
+    while (more) {
+        if (wave == 0) {
+            int ns = 0, first_long = DEAL_STEPS;
+            while (ns < DEAL_STEPS) {
+                if (m == 0) {
+                    if (at == have) {
+                        if (next_run < listed) {
+                            const int r = min(next_run + lane, listed - 1);
+                            lane_k = starts[r];
+                            lane_m = (r + 1 < listed ? starts[r + 1] : listed == runs ? K : lane_k + 1) - lane_k;
+                            have = min(64, listed - next_run);
+                            next_run += have;
+                        } else if (next_lone < K) {
+                            lane_k = min(next_lone + lane, K - 1);
+                            lane_m = 1;
+                            have = min(64, K - next_lone);
+                            next_lone += have;
+                        } else {
+                            break;
+                        }
+                        lane_c = count[ids[lane_k]];
+                        lane_r = lane_c ? 0xFFFFFFFFu / lane_c : 0u;
+                        at = 0;
+                    }
+                    k = __builtin_amdgcn_readlane(lane_k, at);
+                    m = __builtin_amdgcn_readlane(lane_m, at);
+                    c = (T)(uint32_t)__builtin_amdgcn_readlane((int)lane_c, at);
+                    recip = (uint32_t)__builtin_amdgcn_readlane((int)lane_r, at);
+                    ++at;
+                }
+                const bool open = sl < NS && fill < DEAL_SLICE;
+                const T none = ~(T)0, key = open ? load << 4 | (T)sl : none, least = deal_min16(key), lo = least >> 4;
+                // the slices that are next (c = 0: the least loaded one until it is full) and their order
+                const bool next = open && (c ? load - lo < c : key == least);
+                const int nf = __popcll(__ballot(next) & 0xFFFF), rank = deal_below<1>(key);
+                const int room = (int)deal_min16((uint32_t)(next ? DEAL_SLICE - fill : DEAL_SLICE));
+                const uint32_t inverse = (uint32_t)__builtin_amdgcn_readlane((int)lane_inverse, nf);
+                const int rounds = nf == 1 ? m : (int)__umulhi((uint32_t)m, inverse);
+                // whole rounds: until the codewords or the room end, or the least loaded of them passes one that was behind
+                int q = min(rounds, room), last = room;
+                const T above = deal_min16(open && !next ? load : none);
+                if (c && above != none && above - lo < (uint64_t)c * (uint64_t)(q + 1)) {
+                    uint32_t of;                                             // (above - lo) / c
+                    if constexpr (sizeof(T) == 4) {                          // (the product is one too small at most, or none)
+                        of = __umulhi((uint32_t)(above - lo), recip);
+                        of += (above - lo) - of * (uint32_t)c >= (uint32_t)c;
+                    } else {
+                        of = (uint32_t)((above - lo) / c);
+                    }
+                    last = min(room, (int)of);
+                }
+                q = min(q, last);
+                const int rem = q == rounds && q < last ? m - q * nf : 0, n = q * nf + rem;
+                if (n > DEAL_LONG) first_long = min(first_long, ns);
+                DealStep& st = steps[ns++];
+                if (lane == 0) { st.k = (uint32_t)k; st.n = (uint32_t)n; st.nf = (uint32_t)nf; st.inverse = inverse; }
+                if (lane < 16 && next) st.base[rank] = (uint16_t)(sl * DEAL_SLICE + fill);
+                const int got = next ? q + (rank < rem) : 0;
+                load += c * (T)got;
+                fill += got;
+                k += n;
+                m -= n;
+            }
+            if (lane == 0) { shared_steps = ns; shared_long = first_long; }
+        }
+        __syncthreads();
+        const int ns = shared_steps;
+        more = ns == DEAL_STEPS;
+        auto write = [&](int i, int j0, int stride) {
+            const int n = (int)steps[i].n, nf = (int)steps[i].nf, first = (int)steps[i].k;
+            const uint32_t inverse = steps[i].inverse;
+            const int base = steps[i].base[sl];
+#pragma unroll 4
+            for (; j0 < n; j0 += stride) {
+                const int j = min(j0 + lane, n - 1), round = nf == 1 ? j : (int)__umulhi((uint32_t)j, inverse), label = __shfl(base, j - round * nf, 64) + round;
+                remap[ids[first + j]] = (uint16_t)label;
+            }
+        };
+        for (int i = wave; i < ns; i += DEAL_WAVES)                          // a wave a step, but of long ones every wave each 16th group of 64 codewords
+            if (steps[i].n <= DEAL_LONG) write(i, 0, 64);
+        for (int i = shared_long; i < ns; ++i)
+            if (steps[i].n > DEAL_LONG) write(i, wave * 64, DEAL_NT);
+        __syncthreads();
+    }
     }
 }
 

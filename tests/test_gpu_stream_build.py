@@ -177,3 +177,25 @@ def test_a_relabelling_that_failed_is_done_again(monkeypatch):
     for m, w, (words, _) in zip(lins, want, before):
         assert not torch.equal(m.words, words) and m.relabelled and torch.equal(m.words, w.words)
         assert torch.equal(m.table, w.table) and torch.equal(m.stream, w.stream) and m.stream_runs == w.stream_runs
+
+
+@pytest.mark.parametrize("bits", [13, 16])
+@pytest.mark.parametrize("most", [1, 2, 3, 7, 8, 15, 16, 31, 32, 63, 64, 127, 128, 255, 256, 300])
+def test_dealing_by_largest_count(most, bits):
+    """Every width of the digit that the codewords are sorted by, and two digits; codewords without tags are one long step."""
+    L, g, R, C = _lib.lib(), torch.Generator().manual_seed(most), 40, 8 * 200
+    pool = torch.randperm(1 << bits, generator=g)[:R * 200 // most + 1].repeat_interleave(torch.randint(1, most + 1, (R * 200 // most + 1,), generator=g))
+    tags = torch.cat([torch.full((most,), int(pool[0])), pool[pool != pool[0]], torch.arange(R * 200) % (1 << bits)])[:R * 200]
+    assert most == 1 or int(torch.bincount(tags).max()) >= most
+    tags = tags[torch.randperm(R * 200, generator=g)].view(R, 200)
+    words = pack_bits(tags, bits)
+    remap = np.zeros(1 << bits, np.uint16)
+    _lib.check(L.sq_codebook_balance_books(words.data_ptr(), R, words.shape[1], C, 8, bits, 1, None, remap.ctypes.data))
+    wd, td = words.cuda(), torch.randn(1 << bits, 8, generator=g).half().cuda()
+    mats = _lib.matrix_array([_lib.SqMatrix(wd.data_ptr(), td.data_ptr(), None, None, None, None, None, R, C, 8, bits, 1, 1, words.shape[1], 0, None, 0, 0)])
+    wo, to = torch.empty_like(wd), torch.empty_like(td)
+    scratch = torch.empty(L.sq_codebook_rebalance_bytes(mats, 1), dtype=torch.uint8, device="cuda")
+    _lib.check(L.sq_codebook_rebalance_device(mats, 1, *((ctypes.c_void_p * 1)(t.data_ptr()) for t in (wo, to)), scratch.data_ptr(), scratch.numel(), None))
+    new = torch.from_numpy(remap.astype(np.int64))
+    assert torch.equal(wo.cpu(), pack_bits(new[tags], bits))
+    assert torch.equal(to.cpu()[new], td.cpu())
