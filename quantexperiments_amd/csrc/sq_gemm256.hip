@@ -1,34 +1,41 @@
 // Large-tile fp16 GEMM for prefill: Y[T, R] = X[T, C] . W[R, C]^T, fp32 accumulate, optional row scale.
 //
 // Workgroup tile 256, 192 or 128 tokens x 256 weight rows (64 MT x 256, chosen by gemm256_plan), 4 waves in 2 x 2, each a
-// 32 MT x 128 tile of v_mfma_f32_32x32x16_f16 accumulators (MT = 4: all 256 accumulator registers), one wave per SIMD.  Both
+// 32 MT x 128 tile of v_mfma_f32_16x16x32_f16 accumulators (MT = 4: all 256 accumulator registers), one wave per SIMD.  Both
 // operands are K-contiguous fp16 in memory.  The K loop moves in slabs of 64 columns; a slab of ONE operand (rows of 128 bytes,
 // whole 128-byte lines: half-line requests get 10.5 TB/s out of L2 over the chip, whole lines 15.2 TB/s) is copied from global
-// memory straight into LDS (buffer_load_dwordx4 ... lds: no staging registers) into a ring of slots of that operand.  What a lone
-// wave per SIMD needs is that nothing in its instruction stream waits:
-//   * fragments are read one 16-column step ahead of their matrix instructions, one read behind each of the first ones;
-//   * one barrier per slab, two matrix instructions into the slab's last step, when its last fragments have arrived: it
+// memory straight into LDS (buffer_load_dwordx4 ... lds: no staging registers) into a ring of slots of that operand.
+//
+// Bound: the chip's power.  Matrix instructions alone, on normally distributed operands held in registers, reach 1.69 PFLOP/s as
+// 32x32x16 and 1.95 as 16x16x32 (2.42 both on zeros, where the clock stays at its limit): the accumulators a product reads
+// and writes cost power, and 16x16x32 has half of them per operation.  What else takes power or clocks in the loop counts the same way:
+//   * the products are written out as instructions: of the builtin's 128 accumulators the compiler moves some away and back in every
+//     step (0.9 vector instructions a product; in that form 16x16x32 was slower than 32x32x16, 1.26 and 1.29 PFLOP/s on 8192^3);
+//   * a slab's 128 products of a wave share the loop with 32 LDS reads, 16 copies and about 30 other instructions: four copies
+//     share an LDS base, pieces past a row's end change the copies' offsets once, in front of the last slab, and the ring's offsets
+//     are worked out between products.  With an offset chosen per copy and bases per copy: 74 instead of 80 % of the matrix
+//     cores' time;
+//   * a product's neighbours share an operand (rows of blocks walked to and fro: 0.4 %).
+// 8192^3 / 2048 x 37888 x 3584, in turn on one machine: 835 / 472 us as 32x32x16, 758 / 437 as 16x16x32, 727 / 415 with the lean loop
+// (1.51 PFLOP/s).
+//
+// What a lone wave per SIMD needs is that nothing in its instruction stream waits:
+//   * X blocks are read in place, a row of products behind their last use, the weights' blocks one 32-column step ahead;
+//   * one barrier per slab, eight products into the slab's last step, when its last fragments have arrived: it
 //     frees the slab's two slots and says that the next slab is complete;
-//   * the slots it frees take one operand's slab at once, behind the reads of the next slab's first fragments, and a slab of the
-//     other during the following steps (issued over the first two steps of the next slab instead, 8192^3 ran at 1.26 instead
-//     of 1.29 PFLOP/s).
+//   * the slots it frees take one operand's slab behind the barrier, among the reads of the next slab's first fragments, and a slab
+//     of the other during the next slab's first step.
 // MT = 4 and 3: three W slots, two X slots: W, which comes from memory where X stays in L2, has one to two slabs' time to
 // arrive.  MT = 2, whose slabs take half as long: three W and four X slots, two to three slabs' time (with two and three:
-// 333 x 3584 x 18944 in four 89 us, now 77; 1024 x 7168 x 5120 91 and 81).
-// Eight waves of 128 x 64 (two per SIMD) ran at 1.15 PFLOP/s on 8192^3, in one schedule or as two groups taking turns at
-// matrix and memory phases, with 67 percent of the matrix cores' time used at 1.70 GHz; this one uses 83 percent of it at
-// 1.52 GHz (the chip's power limit: on zeros it reaches 1.71 PFLOP/s) and reads a third less from LDS.  16x16x32
-// instructions in the same schedule: 1.26.  Eight waves / this one, in turn on one machine: 8192^3 966 / 844 us (1.14 / 1.30
-// PFLOP/s), 4096^3 124 / 115, 2048 x 37888 x 3584 525 / 485 (1.06 / 1.15), 2048 x 18944 x 3584 285 / 267, 2048 x 3584 x 18944
-// 275 / 254; 8192^3 takes 820 to 880 us from machine to machine.  (With five slots for either operand's slabs in turn instead of
-// three and two: 820.5 and 821, 111.9 and 111.4, 462.5 and 466.3, 257.5 and 258.4, 243.7 and 244.)
+// 333 x 3584 x 18944 in four 89 us, now 77; 1024 x 7168 x 5120 91 and 81).  Eight waves of 128 x 64 (two per SIMD) ran at 1.15
+// PFLOP/s on 8192^3, in one schedule or as two groups taking turns at matrix and memory phases.
 //
 // LDS rows are 128 bytes; the 16-byte piece c of row r is stored at slot c ^ ((r >> 1) & 7).  A ds_read_b128
-// serves 16 lanes per clock from 64 banks (256 bytes); 16 consecutive rows of one piece then fall on 16
-// different 16-byte bank groups ((r & 1) * 8 + slot), so the operand reads are conflict free.
+// serves 16 lanes per clock from 64 banks (256 bytes), rows 0-3 and 12-15 of one piece with rows 4-11 of the next; they fall on
+// 16 different 16-byte bank groups ((r & 1) * 8 + slot), so the operand reads are conflict free.
 //
-// Operand layout of v_mfma_f32_32x32x16_f16, lane l: A row / B column l % 32, k = 8 * (l / 32) .. + 7;
-// D[v], v = 0..15: row 8 * (v / 4) + 4 * (l / 32) + v % 4, column l % 32.  Rows of D are weight rows, columns are tokens,
+// Operand layout of v_mfma_f32_16x16x32_f16, lane l: A row / B column l % 16, k = 8 * (l / 16) .. + 7;
+// D[v], v = 0..3: row 4 * (l / 16) + v, column l % 16.  Rows of D are weight rows, columns are tokens,
 // so a lane holds 4 consecutive outputs of one token in a row of registers.
 #include <algorithm>
 #include "sq_common.h"
@@ -120,17 +127,15 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a)
     }
     int bt, br;
     gemm256_tile(tile, a.tiles_t, a.tiles_r, gemm256_super(MT), &bt, &br);
-    constexpr int BM = gemm256_tokens(MT), XC = 2 * MT, X_SLOT = BM * G_BK * 2, NM = 4 * MT;     // XC: copies a wave makes of an X slab (of a W slab: 8); NM: products of a step
+    constexpr int BM = gemm256_tokens(MT), XC = 2 * MT, X_SLOT = BM * G_BK * 2, TB = 2 * MT, NM = 8 * TB;     // XC: copies a wave makes of an X slab (of a W slab: 8); TB: its blocks of 16 tokens; NM: products of a step
     const int t0 = bt * BM, r0 = br * G_BN;
     const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * 128;
 
-    float16v acc[MT][4];                     // [token block][weight-row block]
+    float4v acc[TB][8];                      // [token block][weight-row block]
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+    for (int i = 0; i < TB; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+        for (int j = 0; j < 8; ++j) acc[i][j] = float4v{0.f, 0.f, 0.f, 0.f};
 
     // Copies.  One buffer_load_dwordx4 to LDS fills 1 KB = 8 LDS rows in lane order, so lane s lands in row
     // s >> 3, slot s & 7 of its block and therefore fetches the piece the swizzle puts there.  Wave w copies
@@ -152,115 +157,139 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a)
     for (int j = 0; j < XC; ++j) {
         const int row = wave * (BM / 4) + j * 8 + lrow;
         const int t = t0 + row < a.T ? row : a.T - 1 - t0;
-        xo[j] = (uint32_t)(t * (int)a.ldx + (slot ^ ((row >> 1) & 7)) * 8) * 2u;
+        xo[j] = (uint32_t)(t * (int)a.ldx + (slot ^ ((row >> 1) & 7)) * 8) * 2u + (uint32_t)(3 - (j & 3)) * 1024u;
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         const int row = wave * 64 + j * 8 + lrow;
         const int r = r0 + row < a.R ? row : a.R - 1 - r0;
-        wo[j] = (uint32_t)(r * (int)a.ldw + (slot ^ ((row >> 1) & 7)) * 8) * 2u;
+        wo[j] = (uint32_t)(r * (int)a.ldw + (slot ^ ((row >> 1) & 7)) * 8) * 2u + (uint32_t)(3 - (j & 3)) * 1024u;
     }
     const int nk_all = (a.C + G_BK - 1) / G_BK, k_begin = (int)((int64_t)kz * nk_all / nparts);
     const int nk = (int)((int64_t)(kz + 1) * nk_all / nparts) - k_begin;
-    const char* xt = reinterpret_cast<const char*>(a.x + (int64_t)t0 * a.ldx + (int64_t)k_begin * G_BK);
-    const char* wt = reinterpret_cast<const char*>(a.w + (int64_t)r0 * a.ldw + (int64_t)k_begin * G_BK);
+    const char* xt = reinterpret_cast<const char*>(a.x + (int64_t)t0 * a.ldx + (int64_t)k_begin * G_BK) - 3072;
+    const char* wt = reinterpret_cast<const char*>(a.w + (int64_t)r0 * a.ldw + (int64_t)k_begin * G_BK) - 3072;
     typedef __attribute__((address_space(3))) void* lptr_t;
     const int lastk = nk_all - 1 - k_begin;  // the row's last slab, counted from this part's first
     bool past[2];                            // this lane's piece of it lies past the row's end, in even and odd copies (whose rows' swizzles differ by 4)
 #pragma unroll
     for (int h = 0; h < 2; ++h) past[h] = (slot ^ (h * 4 + (lrow >> 1))) * 8 >= a.C - (nk_all - 1) * G_BK;
-    auto copy = [&](const char* base, int q, uint32_t off, int j, int to) {
-        const int sb = q < nk ? q : nk - 1;
-        const __amdgpu_buffer_rsrc_t buf = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, 0xFFFFFF00u, 0x00027000);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, (lptr_t)(smem + to), 16, sb == lastk && past[j & 1] ? 0xFFFFFFF0u : off, sb * (G_BK * 2), 0, 0);
+    // (four copies share an LDS base: the instruction's own offset, 1024 j, counts for LDS and memory, so the lanes' offsets hold that
+    // much less, and bases that start 3072 bytes early keep them positive)
+    constexpr uint32_t PAST = 0xFFFF0000u;
+    auto copy = [&](const char* base, int at, uint32_t off, int to, int j) {
+        const __amdgpu_buffer_rsrc_t buf = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, PAST, 0x00027000);
+        const lptr_t lds = (lptr_t)(smem + to);
+        if ((j & 3) == 0) __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, lds, 16, off, at, 0, 0);
+        if ((j & 3) == 1) __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, lds, 16, off, at, 1024, 0);
+        if ((j & 3) == 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, lds, 16, off, at, 2048, 0);
+        if ((j & 3) == 3) __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, lds, 16, off, at, 3072, 0);
     };
-    auto copy_x = [&](int q, int sl, int j) { copy(xt, q, xo[j], j, sl * X_SLOT + wave * (X_SLOT / 4) + j * 1024); };
-    auto copy_w = [&](int q, int sl, int j) { copy(wt, q, wo[j], j, W_AT + sl * G_W_SLOT + wave * 8192 + j * 1024); };
-    auto copy_early = [&](int q, int sl, int j) { if constexpr (XE) copy_x(q, sl, j); else copy_w(q, sl, j); };
-    auto copy_late = [&](int q, int sl, int j) { if constexpr (XE) copy_w(q, sl, j); else copy_x(q, sl, j); };
+    // `at`: the slab's first column in bytes, `to`: its slot's offset
+    auto copy_x = [&](int at, int to, int j) { copy(xt, at, xo[j], to + wave * (X_SLOT / 4) + (j & ~3) * 1024, j); };
+    auto copy_w = [&](int at, int to, int j) { copy(wt, at, wo[j], to + W_AT + wave * 8192 + (j & ~3) * 1024, j); };
+    auto copy_early = [&](int at, int to, int j) { if constexpr (XE) copy_x(at, to, j); else copy_w(at, to, j); };
+    auto copy_late = [&](int at, int to, int j) { if constexpr (XE) copy_w(at, to, j); else copy_x(at, to, j); };
+    constexpr int ES = XE ? X_SLOT : G_W_SLOT, LS = XE ? G_W_SLOT : X_SLOT;      // their slots' sizes
+    // from the row's last slab on the pieces past its end are asked for past the buffer's end
+    const int plast = lastk < nk && a.C % G_BK != 0 ? lastk : INT_MAX;
+    auto end_early = [&](int q) {
+        if (q < plast) return;
+#pragma unroll
+        for (int j = 0; j < EC; ++j) { uint32_t& o = XE ? xo[j] : wo[j]; o = past[j & 1] ? PAST : o; }
+    };
+    auto end_late = [&](int q) {
+        if (q < plast) return;
+#pragma unroll
+        for (int j = 0; j < LC; ++j) { uint32_t& o = XE ? wo[j] : xo[j]; o = past[j & 1] ? PAST : o; }
+    };
+    auto column = [&](int q) { return (q < nk ? q : nk - 1) * (G_BK * 2); };
 
-    // Fragments.  A lane reads row (lane & 31) + 32 i of its wave's rows, piece 2 kk + (lane >> 5); the swizzle
-    // term depends on the row modulo 16 only and the column step kk only flips bits 5-6 of the offset, so one
-    // offset plus compile-time multiples of 32 rows (4096 bytes) covers all reads of a slab.
-    half8v fx[2][MT], fw[2][4];
-    const uint32_t foff = (uint32_t)((lane & 31) * 128 + (((lane >> 5) ^ ((lane >> 1) & 7)) << 4));
-    auto read_x = [&](int set, int kk, int sl, int i) {
-        fx[set][i] = *reinterpret_cast<const half8v*>(smem + sl * X_SLOT + wm * 128 + i * 4096 + (foff ^ (uint32_t)(kk << 5)));
+    // Fragments.  A lane reads row (lane & 15) + 16 i of its wave's rows, piece 4 kk + (lane >> 4); the swizzle term depends on the
+    // row modulo 16 only and the column step kk only flips bit 6 of the offset, so one offset plus compile-time multiples of
+    // 16 rows (2048 bytes) covers all reads of a slab.
+    half8v fx[TB], fw[2][8];
+    const uint32_t foff = (uint32_t)((lane & 15) * 128 + (((lane >> 4) ^ ((lane >> 1) & 7)) << 4));
+    auto read_x = [&](int kk, int at, int i) {
+        fx[i] = *reinterpret_cast<const half8v*>(smem + at + wm * 128 + i * 2048 + (foff ^ (uint32_t)(kk << 6)));
     };
-    auto read_w = [&](int set, int kk, int sl, int j) {
-        fw[set][j] = *reinterpret_cast<const half8v*>(smem + W_AT + sl * G_W_SLOT + wn * 128 + j * 4096 + (foff ^ (uint32_t)(kk << 5)));
+    auto read_w = [&](int set, int kk, int at, int j) {
+        fw[set][j] = *reinterpret_cast<const half8v*>(smem + W_AT + at + wn * 128 + j * 2048 + (foff ^ (uint32_t)(kk << 6)));
     };
+    // product n of a step: token block n / 8, weight-row block n % 8, to and fro
     auto mma = [&](int set, int n) {
-        acc[n >> 2][n & 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fw[set][n & 3], fx[set][n >> 2], acc[n >> 2][n & 3], 0, 0, 0);
+        const int i = n >> 3, j = i & 1 ? 7 - (n & 7) : n & 7;
+        asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(fw[set][j]), "v"(fx[i]));
     };
     // the accumulators stay in their registers before and behind the loop (without this the compiler copies all 256 into the
     // other half of the register file at the loop's end, spills, and a launch that needs scratch memory takes 7 us longer)
-#define SQ_PIN() _Pragma("unroll") for (int i = 0; i < MT; ++i) { asm volatile("" : "+a"(acc[i][0]), "+a"(acc[i][1]), "+a"(acc[i][2]), "+a"(acc[i][3])); }
+#define SQ_PIN() _Pragma("unroll") for (int i = 0; i < TB; ++i) { asm volatile("" : "+a"(acc[i][0]), "+a"(acc[i][1]), "+a"(acc[i][2]), "+a"(acc[i][3]), "+a"(acc[i][4]), "+a"(acc[i][5]), "+a"(acc[i][6]), "+a"(acc[i][7])); }
 #define SQ_SB() __builtin_amdgcn_sched_barrier(0)
-    // one 16-column step: NM matrix instructions on `set`, the next step's fragments behind the first of them, copies [c0, c1)
-    // of the early operand behind the others
-    auto step = [&](int set, int kk, int sx, int sw, int q, int to, int c0, int c1) {
-        mma(set, 0); SQ_SB();
-        read_x(set ^ 1, kk, sx, 0); read_w(set ^ 1, kk, sw, 0); SQ_SB();
-#pragma unroll
-        for (int i = 1; i < 4; ++i) { mma(set, i); SQ_SB(); read_w(set ^ 1, kk, sw, i); SQ_SB(); }
-#pragma unroll
-        for (int i = 1; i < MT; ++i) { mma(set, 3 + i); SQ_SB(); read_x(set ^ 1, kk, sx, i); SQ_SB(); }
-#pragma unroll
-        for (int n = MT + 3, c = c0; n < NM; ++n) {
-            mma(set, n);
-            if (c < c1 && (MT == 2 || ((n - MT - 3) & 1) == 0)) { SQ_SB(); copy_early(q, to, c); ++c; SQ_SB(); }
-        }
-        SQ_SB();
-    };
 
 #pragma unroll
     for (int q = 0; q < E - 1; ++q) {
+        end_early(q);
 #pragma unroll
-        for (int j = 0; j < EC; ++j) copy_early(q, q, j);
+        for (int j = 0; j < EC; ++j) copy_early(column(q), q * ES, j);
         if (q == L - 1) break;
+        end_late(q);
 #pragma unroll
-        for (int j = 0; j < LC; ++j) copy_late(q, q, j);
+        for (int j = 0; j < LC; ++j) copy_late(column(q), q * LS, j);
     }
     __builtin_amdgcn_s_waitcnt(vmcnt_only(AHEAD));
     SQ_SB(); __builtin_amdgcn_s_barrier(); SQ_SB();
 #pragma unroll
-    for (int i = 0; i < MT; ++i) read_x(0, 0, 0, i);
+    for (int i = 0; i < TB - 2; ++i) read_x(0, 0, i);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) read_w(0, 0, 0, i);
+    for (int j = 0; j < 8; ++j) read_w(0, 0, 0, j);
+    end_late(L - 1);
 #pragma unroll
-    for (int j = 0; j < LC; ++j) copy_late(L - 1, L - 1, j);
-    int se = 0, sl = 0;                      // slots of the slab being multiplied
+    for (int j = 0; j < LC; ++j) copy_late(column(L - 1), (L - 1) * LS, j);
+    // the slots (byte offsets) of the slab being multiplied, of the next one, and the one the early copies go to; the column of the
+    // slab that is copied.  Worked out between the products, a little at a time: a scalar instruction in front of them takes four
+    // clocks of the matrix core's time.
+    int ce = 0, cl = 0, ne = 0, nl = 0, to = (E - 1) * ES, at = column(L);
     SQ_PIN();
+    asm volatile("s_nop 7");                 // (no wait of the compiler's between the zeroed accumulators and a written-out product)
 #pragma unroll 1
     for (int s = 0; s < nk; ++s) {
-        const int ne = se == E - 1 ? 0 : se + 1, nl = sl == L - 1 ? 0 : sl + 1, to = se == 0 ? E - 1 : se - 1;
-        const int sx = XE ? se : sl, sw = XE ? sl : se, nx = XE ? ne : nl, nw = XE ? nl : ne;
-        constexpr int C1 = (EC + 2) / 3, C2 = 2 * C1 < EC ? 2 * C1 : EC;
-        step(0, 1, sx, sw, s + E - 1, to, 0, C1);
-        step(1, 2, sx, sw, s + E - 1, to, C1, C2);
-        step(0, 3, sx, sw, s + E - 1, to, C2, EC);
-        // last step: this wave's copies of slab s + 1 are waited for (those of later slabs stay in flight), and its reads of slab
-        // s, whose slots the copies behind the barrier overwrite; then the barrier: everybody's copies have landed and
-        // everybody has read slab s to the end.  (The reads have arrived for the two products by now, so their wait costs
-        // nothing, but nothing else in the source would ask for all of them.)
-        mma(1, 0); SQ_SB(); mma(1, 1); SQ_SB();
-        __builtin_amdgcn_s_waitcnt(vmcnt_and_lds(AHEAD)); SQ_SB();
-        __builtin_amdgcn_s_barrier(); SQ_SB();
-        read_x(0, 0, nx, 0); read_w(0, 0, nw, 0); SQ_SB();
+        if (s + L >= plast) { end_early(s + L); end_late(s + L); }
+        // first step: its last X blocks, the second step's fragments, the early copies of slab s + L
 #pragma unroll
-        for (int n = 2, c = 0; n < NM; ++n) {
-            mma(1, n); SQ_SB();
-            if (n < 5) read_w(0, 0, nw, n - 1);
-            else if (n < 4 + MT) read_x(0, 0, nx, n - 4);
-            // the copies of the late operand, one behind each product; in the six places of MT = 2 some of the eight go in pairs
-#pragma unroll
-            for (int k = 0; k < (MT == 2 && (n == 5 || n == 6) ? 2 : 1); ++k)
-                if (c < LC) { copy_late(s + L, sl, c); ++c; }
+        for (int n = 0; n < NM; ++n) {
+            mma(0, n); SQ_SB();
+            if (n < 2) read_x(0, XE ? ce : cl, TB - 1 - n);
+            if (n >= 2 && n <= 16 && n % 2 == 0) read_w(1, 1, XE ? cl : ce, n / 2 - 1);
+            if (n % 8 == 1 && n > 8 && n < NM - 8) read_x(1, XE ? ce : cl, n / 8 - 1);
+            if (n % 4 == 3 && n / 4 < EC) copy_early(at, to, n / 4);
+            if (n == NM - 6) { ne = ce + ES; SQ_SB(); }
+            if (n == NM - 5) { ne = ne == E * ES ? 0 : ne; SQ_SB(); }
+            if (n == NM - 4) { nl = cl + LS; SQ_SB(); }
+            if (n == NM - 3) { nl = nl == L * LS ? 0 : nl; SQ_SB(); }
+            if (n == NM - 2) { to = ce; SQ_SB(); }
             SQ_SB();
         }
-        se = ne; sl = nl;
+        // second step: this wave's copies of slab s + 1 are waited for (those of later slabs stay in flight), and its reads of slab
+        // s, whose slots the copies behind the barrier overwrite; then the barrier: everybody's copies have landed and
+        // everybody has read slab s to the end.  (Six products behind the last of those reads their wait costs little.)
+#pragma unroll
+        for (int n = 0; n < NM; ++n) {
+            mma(1, n); SQ_SB();
+            if (n < 2) read_x(1, XE ? ce : cl, TB - 1 - n);
+            if (n == 7) {
+                __builtin_amdgcn_s_waitcnt(vmcnt_and_lds(AHEAD)); SQ_SB();
+                __builtin_amdgcn_s_barrier(); SQ_SB();
+            }
+            if (n >= 8 && n <= 22 && n % 2 == 0) read_w(0, 0, XE ? nl : ne, n / 2 - 4);
+            if (n % 8 == 1 && n > 8 && n < NM - 8) read_x(0, XE ? ne : nl, n / 8 - 1);
+            constexpr int GAP = MT == 2 ? 2 : 4;
+            if (n >= 11 && (n - 11) % GAP == 0 && (n - 11) / GAP < LC) copy_late(at, cl, (n - 11) / GAP);
+            if (n == NM - 4) { at = column(s + 1 + L); SQ_SB(); }
+            if (n == NM - 3) { ce = ne; cl = nl; SQ_SB(); }
+            SQ_SB();
+        }
     }
+    asm volatile("s_nop 15\n\ts_nop 15");    // the last products' results are behind the loop before they are read
     SQ_PIN();
 #undef SQ_SB
 #undef SQ_PIN
@@ -271,37 +300,33 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a)
     // ones go through LDS: every wave lays its 32 MT x 128 tile out token-major (8 bytes per write) and stores it in 16-byte
     // pieces, 256 contiguous bytes per token (2-byte stores straight from the accumulators cost 49 us of a 376 us product of
     // a 2048 x 18944 output).
-    const int half4 = 4 * (lane >> 5), tok = lane & 31;
+    const int quad4 = 4 * (lane >> 4), tok = lane & 15;
     float* scales = reinterpret_cast<float*>(smem + 2 * BM * G_EP_PITCH);        // behind the four waves' tiles
     scales[tid] = gemm256_scale<true>(a.sc, r0 + tid < a.R ? r0 + tid : a.R - 1);
     __syncthreads();
     float* part = a.part + ((int64_t)(tile - a.main_tiles) * a.kt + kz) * (BM * G_BN);
     unsigned char* my = smem + wave * (BM / 2 * G_EP_PITCH);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        float4v sc[4];
+    for (int j = 0; j < 8; ++j) {
+        const int rl = j * 16 + quad4;
+        const float4v sc = *reinterpret_cast<const float4v*>(scales + wn + rl);
 #pragma unroll
-        for (int g = 0; g < 4; ++g) sc[g] = *reinterpret_cast<const float4v*>(scales + wn + j * 32 + 8 * g + half4);
+        for (int i = 0; i < TB; ++i) {
+            const int tl = i * 16 + tok;
+            const float4v val = acc[i][j];
+            if (nparts > 1) {
+                *reinterpret_cast<float4v*>(part + (wm + tl) * G_BN + wn + rl) = val;
+            } else if constexpr (EP != SQ_F32) {
+                const float4v o = val * sc;
+                *reinterpret_cast<u32x2*>(my + tl * G_EP_PITCH + rl * 2) =
+                    EP == SQ_BF16 ? u32x2{f2bf_x2(o[0], o[1]), f2bf_x2(o[2], o[3])} : u32x2{f2h_x2(o[0], o[1]), f2h_x2(o[2], o[3])};
+            } else {
+                const int t = t0 + wm + tl, r = r0 + wn + rl;
 #pragma unroll
-        for (int i = 0; i < MT; ++i) {
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int tl = i * 32 + tok, rl = j * 32 + 8 * g + half4;
-                const float4v val = {acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
-                if (nparts > 1) {
-                    *reinterpret_cast<float4v*>(part + (wm + tl) * G_BN + wn + rl) = val;
-                } else if constexpr (EP != SQ_F32) {
-                    const float4v o = val * sc[g];
-                    *reinterpret_cast<u32x2*>(my + tl * G_EP_PITCH + rl * 2) =
-                        EP == SQ_BF16 ? u32x2{f2bf_x2(o[0], o[1]), f2bf_x2(o[2], o[3])} : u32x2{f2h_x2(o[0], o[1]), f2h_x2(o[2], o[3])};
-                } else {
-                    const int t = t0 + wm + tl, r = r0 + wn + rl;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (t < a.T && r + e < a.R) store_y(a.y, a.y_dtype, (int64_t)t * a.ldy + a.y_off + r + e, val[e] * sc[g][e]);
-                }
+                for (int e = 0; e < 4; ++e)
+                    if (t < a.T && r + e < a.R) store_y(a.y, a.y_dtype, (int64_t)t * a.ldy + a.y_off + r + e, val[e] * sc[e]);
             }
-            __builtin_amdgcn_sched_barrier(0);
+            if (i & 1) __builtin_amdgcn_sched_barrier(0);
         }
     }
     if (EP == SQ_F32 || nparts > 1) return;
