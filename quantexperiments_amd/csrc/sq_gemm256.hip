@@ -38,6 +38,9 @@
 // D[v], v = 0..3: row 4 * (l / 16) + v, column l % 16.  Rows of D are weight rows, columns are tokens,
 // so a lane holds 4 consecutive outputs of one token in a row of registers.
 #include <algorithm>
+#include <climits>
+#include <type_traits>
+#include <utility>
 #include "sq_common.h"
 
 namespace sq {
@@ -76,12 +79,12 @@ __host__ __device__ __forceinline__ void gemm256_tile(int tile, int tiles_t, int
     *br = l / w;
 }
 
-// scale of weight row r (1 without scales).  FLAT: tested against all eight pieces, without a loop, which the tile kernel with all its
+// scale of weight row r as fp16 bits (1 without scales).  FLAT: tested against all eight pieces, without a loop, which the tile kernel with all its
 // accumulators alive has no registers for (136 bytes of scratch per lane); else against as many as there are (the reduction, four
 // look-ups a thread, takes 2 us less of 333 x 37888 x 3584 that way).
 template <bool FLAT>
-__device__ __forceinline__ float gemm256_scale(const Gemm256Scales& s, int r) {
-    if (s.n == 0) return 1.f;
+__device__ __forceinline__ uint16_t gemm256_scale(const Gemm256Scales& s, int r) {
+    if (s.n == 0) return 0x3C00;
     const uint16_t* p = s.p[0];
     int at = r;
     auto test = [&](int i) { if (r >= s.end[i - 1]) { p = s.p[i]; at = r - s.end[i - 1]; } };
@@ -92,92 +95,157 @@ __device__ __forceinline__ float gemm256_scale(const Gemm256Scales& s, int r) {
 #pragma unroll 1
         for (int i = 1; i < s.n; ++i) test(i);
     }
-    return h2f(p[at]);
+    return p[at];
 }
-
-constexpr int G_EP_PITCH = 128 * 2 + 16;     // bytes per token row of a wave's 32 MT x 128 output tile in LDS
 
 // s_waitcnt immediate that waits until at most n vector-memory operations are outstanding (gfx9 encoding: vmcnt in bits 3:0 and
 // 15:14, expcnt 6:4, lgkmcnt 11:8) and leaves the other counters alone, or also until every LDS read of the wave has arrived
 constexpr int vmcnt_only(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
 constexpr int vmcnt_and_lds(int n) { return vmcnt_only(n) & ~(15 << 8); }
 
+// The accumulators are named registers, a[4 (8 i + j)] .. + 3 for token block i and weight-row block j, which no value of the compiler's
+// lives in (tests/test_abi.py): written as variables, 256 of 256 registers live over a loop with branches, they spill.
+template <int R> __device__ __forceinline__ void acc_product(half8v w, half8v x) {
+    asm volatile("v_mfma_f32_16x16x32_f16 a[%0:%1], %2, %3, a[%0:%1]" :: "n"(R), "n"(R + 3), "v"(w), "v"(x));
+}
+template <int R> __device__ __forceinline__ void acc_clear16(half8v z) {       // sixteen of them, as a product of zeros
+    asm volatile("v_mfma_f32_32x32x16_f16 a[%0:%1], %2, %2, 0" :: "n"(R), "n"(R + 15), "v"(z));
+}
+template <int R> __device__ __forceinline__ float4v acc_read() {
+    float4v v;
+    asm volatile("v_accvgpr_read_b32 %0, a[%4]\n\tv_accvgpr_read_b32 %1, a[%5]\n\tv_accvgpr_read_b32 %2, a[%6]\n\tv_accvgpr_read_b32 %3, a[%7]"
+                 : "=v"(v[0]), "=v"(v[1]), "=v"(v[2]), "=v"(v[3]) : "n"(R), "n"(R + 1), "n"(R + 2), "n"(R + 3));
+    return v;
+}
+template <int N> __device__ __forceinline__ void acc_claim() {                 // the kernel needs the first N of them
+    if constexpr (N == 128) asm volatile("" ::: "a127");
+    if constexpr (N == 192) asm volatile("" ::: "a191");
+    if constexpr (N == 256) asm volatile("" ::: "a255");
+}
+
+// calls f with the numbers 0 .. N - 1 as types
+template <class F, int... I> __device__ __forceinline__ void each(F f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
+template <int N, class F> __device__ __forceinline__ void each(F f) { each(f, std::make_integer_sequence<int, N>{}); }
+
+// What a workgroup multiplies: a whole tile, or one of the parts of a tail tile.
+struct Gemm256Item { int tile, kz, nparts, t0, r0, k_begin, nk; };
+
 // EP: SQ_F16 / SQ_BF16 = results of that type whose rows allow 16-byte stores, SQ_F32 = any type, element by element
 // MT: blocks of 32 token rows a wave holds, 64 MT rows a tile
+//
+// A workgroup per CU takes tile after tile: the copies run L slabs ahead of the products over the end of a tile, so the next
+// tile's first slabs arrive while the last products run and the results leave, and the stores of the results have two slabs of
+// the next tile to get through.  A workgroup per tile spent 9 us a round of tiles beyond its slabs, 4 to 5 of them on the stores;
+// the power limit takes part of that back: gate|up of 2048 rows with its decode (2 x 18944 x 3584, five rounds) 536 -> 523 us, a
+// layer of 2048 rows 980 -> 968, 8192^3 with its decode 809 -> 802, products of one round level.
+#define SQ_INLINE __attribute__((always_inline))
+
 template <int EP, int MT>
 __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // Workgroups are dealt round-robin to the 8 XCDs (each with its own L2), so XCD x = blockIdx % 8 takes one
     // contiguous run of whole tiles (a weight tile is then fetched by one L2 only) and, after those, one
-    // contiguous run of tail parts.  The grid is padded; surplus workgroups leave.
-    const int ntiles = a.tiles_t * a.tiles_r;
-    const int xcd = (int)(blockIdx.x & 7), jx = (int)(blockIdx.x >> 3);
+    // contiguous run of tail parts; its workgroups take them in turn.
+    const int ntiles = a.tiles_t * a.tiles_r, xcd = (int)(blockIdx.x & 7), stride = (int)(gridDim.x >> 3);
     const int main_per = (a.main_tiles + 7) >> 3, parts = (ntiles - a.main_tiles) * a.kt, parts_per = (parts + 7) >> 3;
-    int tile, kz = 0, nparts = 1;
-    if (jx < main_per) {
-        tile = xcd * main_per + jx;
-        if (tile >= a.main_tiles) return;
-    } else {
-        const int pidx = xcd * parts_per + (jx - main_per);
-        if (jx - main_per >= parts_per || pidx >= parts) return;
-        tile = a.main_tiles + pidx / a.kt;
-        kz = pidx - (pidx / a.kt) * a.kt;
-        nparts = a.kt;
-    }
-    int bt, br;
-    gemm256_tile(tile, a.tiles_t, a.tiles_r, gemm256_super(MT), &bt, &br);
+    const int main_mine = min(main_per, a.main_tiles - xcd * main_per), items = main_per + max(0, min(parts_per, parts - xcd * parts_per));
     constexpr int BM = gemm256_tokens(MT), XC = 2 * MT, X_SLOT = BM * G_BK * 2, TB = 2 * MT, NM = 8 * TB;     // XC: copies a wave makes of an X slab (of a W slab: 8); TB: its blocks of 16 tokens; NM: products of a step
-    const int t0 = bt * BM, r0 = br * G_BN;
+    const int nk_all = (a.C + G_BK - 1) / G_BK;
+    auto valid = [&](int j) SQ_INLINE {                // this item, or the workgroup's next one where the XCD's run of tiles is shorter than others'
+        while (j >= main_mine && j < main_per) j += stride;
+        return j;
+    };
+    auto item = [&](int j) SQ_INLINE {
+        Gemm256Item it;
+        it.tile = xcd * main_per + j; it.kz = 0; it.nparts = 1;
+        if (j >= main_per) {
+            const unsigned p = (unsigned)(xcd * parts_per + (j - main_per)), kt = (unsigned)a.kt;
+            it.tile = a.main_tiles + (int)(p / kt);
+            it.kz = (int)(p % kt);
+            it.nparts = a.kt;
+        }
+        int bt, br;
+        gemm256_tile(it.tile, a.tiles_t, a.tiles_r, gemm256_super(MT), &bt, &br);
+        it.t0 = bt * BM; it.r0 = br * G_BN;
+        it.k_begin = (int)((unsigned)it.kz * (unsigned)nk_all / (unsigned)it.nparts);
+        it.nk = (int)((unsigned)(it.kz + 1) * (unsigned)nk_all / (unsigned)it.nparts) - it.k_begin;
+        // (the same for all lanes, but the divisions are vector code)
+        it.tile = __builtin_amdgcn_readfirstlane(it.tile); it.kz = __builtin_amdgcn_readfirstlane(it.kz);
+        it.t0 = __builtin_amdgcn_readfirstlane(it.t0); it.r0 = __builtin_amdgcn_readfirstlane(it.r0);
+        it.nparts = __builtin_amdgcn_readfirstlane(it.nparts); it.k_begin = __builtin_amdgcn_readfirstlane(it.k_begin); it.nk = __builtin_amdgcn_readfirstlane(it.nk);
+        return it;
+    };
+    int jm = valid((int)(blockIdx.x >> 3));  // the item being multiplied, and the one being copied
+    if (jm >= items) return;
+    int jc = jm;
     const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * 128;
 
-    float4v acc[TB][8];                      // [token block][weight-row block]
-#pragma unroll
-    for (int i = 0; i < TB; ++i)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) acc[i][j] = float4v{0.f, 0.f, 0.f, 0.f};
+    acc_claim<32 * TB>();
 
     // Copies.  One buffer_load_dwordx4 to LDS fills 1 KB = 8 LDS rows in lane order, so lane s lands in row
     // s >> 3, slot s & 7 of its block and therefore fetches the piece the swizzle puts there.  Wave w copies
     // rows 64 w .. 64 w + 63 of a W slab (8 instructions) and a quarter of the X slab's rows.  Global addresses are a
-    // uniform base (advanced per slab) plus per-lane 32-bit byte offsets computed once; rows past the matrix edge re-read
-    // the last row (their outputs are never stored).  One operand is early (E slots, the copies of slab s + E - 1 go out during
-    // the first steps of slab s), the other late (L = E - 1 slots, slab s + L goes out behind the barrier of slab s); slabs
-    // past the last one re-read the last.  The pieces of the row's last slab that lie past its end (C % 64 != 0) are asked for past the
-    // end of the buffer, which puts zeros into LDS, for both operands (global_load_lds instead of the buffers, for whole slabs: level;
-    // rows of broken slabs ran in the 128 x 128 kernel: 5120 x 2080 at 400 / 1500 rows 80-120 / 126-194 us, now 38-43 / 47-53).
+    // uniform base, a uniform column (advanced per slab) and per-lane 32-bit byte offsets computed once a tile; rows past the matrix
+    // edge re-read the last row (their outputs are never stored).  One operand is early (E slots, the copies of slab s + L go out
+    // during the first step of slab s), the other late (L = E - 1 slots, the copies go out behind the barrier of slab s); behind the
+    // last item's last slab that one is read again.  The pieces of a row's last slab that lie past its end (C % 64 != 0) are asked
+    // for past the end of the buffer, which puts zeros into LDS, for both operands (global_load_lds instead of the buffers, for whole
+    // slabs: level; rows of broken slabs ran in the 128 x 128 kernel: 5120 x 2080 at 400 / 1500 rows 80-120 / 126-194 us, now 38-43 / 47-53).
     constexpr bool XE = gemm256_x_slots(MT) > gemm256_w_slots(MT);        // X is the early one
     constexpr int E = XE ? gemm256_x_slots(MT) : gemm256_w_slots(MT), L = E - 1, EC = XE ? XC : 8, LC = XE ? 8 : XC;
     static_assert(L == (XE ? gemm256_w_slots(MT) : gemm256_x_slots(MT)), "the waits below count on it");
     constexpr int W_AT = gemm256_x_slots(MT) * X_SLOT;
+    constexpr int ES = XE ? X_SLOT : G_W_SLOT, LS = XE ? G_W_SLOT : X_SLOT;      // the slots' sizes
     constexpr int AHEAD = (E - 2) * EC + (L - 2) * LC;                    // copies that may be on their way when slab s + 1 has to be there
-    const int lrow = lane >> 3, slot = lane & 7;
-    uint32_t xo[XC], wo[8];
-#pragma unroll
-    for (int j = 0; j < XC; ++j) {
-        const int row = wave * (BM / 4) + j * 8 + lrow;
-        const int t = t0 + row < a.T ? row : a.T - 1 - t0;
-        xo[j] = (uint32_t)(t * (int)a.ldx + (slot ^ ((row >> 1) & 7)) * 8) * 2u + (uint32_t)(3 - (j & 3)) * 1024u;
-    }
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const int row = wave * 64 + j * 8 + lrow;
-        const int r = r0 + row < a.R ? row : a.R - 1 - r0;
-        wo[j] = (uint32_t)(r * (int)a.ldw + (slot ^ ((row >> 1) & 7)) * 8) * 2u + (uint32_t)(3 - (j & 3)) * 1024u;
-    }
-    const int nk_all = (a.C + G_BK - 1) / G_BK, k_begin = (int)((int64_t)kz * nk_all / nparts);
-    const int nk = (int)((int64_t)(kz + 1) * nk_all / nparts) - k_begin;
-    const char* xt = reinterpret_cast<const char*>(a.x + (int64_t)t0 * a.ldx + (int64_t)k_begin * G_BK) - 3072;
-    const char* wt = reinterpret_cast<const char*>(a.w + (int64_t)r0 * a.ldw + (int64_t)k_begin * G_BK) - 3072;
     typedef __attribute__((address_space(3))) void* lptr_t;
-    const int lastk = nk_all - 1 - k_begin;  // the row's last slab, counted from this part's first
-    bool past[2];                            // this lane's piece of it lies past the row's end, in even and odd copies (whose rows' swizzles differ by 4)
+    const int lrow = lane >> 3, slot = lane & 7;
+    bool past[2];                            // this lane's piece of a row's last slab lies past its end, in even and odd copies (whose rows' swizzles differ by 4)
 #pragma unroll
     for (int h = 0; h < 2; ++h) past[h] = (slot ^ (h * 4 + (lrow >> 1))) * 8 >= a.C - (nk_all - 1) * G_BK;
     // (four copies share an LDS base: the instruction's own offset, 1024 j, counts for LDS and memory, so the lanes' offsets hold that
     // much less, and bases that start 3072 bytes early keep them positive)
     constexpr uint32_t PAST = 0xFFFF0000u;
-    auto copy = [&](const char* base, int at, uint32_t off, int to, int j) {
+    uint32_t xo[XC], wo[8];
+    const char *xt, *wt;
+    int at, left, step;                      // the copied slab's first column in bytes, the item's slabs from it on, bytes to the next slab
+    int last;                                // 1 in an item that ends with a slab that the row does not fill, until that is the next
+    auto row_end = [&]() SQ_INLINE {
+#pragma unroll
+        for (int j = 0; j < XC; ++j) xo[j] = past[j & 1] ? PAST : xo[j];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) wo[j] = past[j & 1] ? PAST : wo[j];
+    };
+    auto copy_from = [&](int j) SQ_INLINE {
+        const Gemm256Item it = item(j);
+        int lc = lane;
+        asm volatile("" : "+v"(lc));         // (or what depends on the lane alone is worked out in front of the loop and kept in registers that it lacks)
+        const int row0 = lc >> 3, piece0 = ((lc & 7) ^ (row0 >> 1)) * 16;
+#pragma unroll
+        for (int j = 0; j < XC; ++j) {       // (rows 8 j on: their swizzle is that of rows 0 or 8)
+            const int t = min(wave * (BM / 4) + j * 8 + row0, a.T - 1 - it.t0);
+            xo[j] = (uint32_t)(t * (int)a.ldx * 2 + (piece0 ^ ((j & 1) << 6))) + (uint32_t)(3 - (j & 3)) * 1024u;
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int r = min(wave * 64 + j * 8 + row0, a.R - 1 - it.r0);
+            wo[j] = (uint32_t)(r * (int)a.ldw * 2 + (piece0 ^ ((j & 1) << 6))) + (uint32_t)(3 - (j & 3)) * 1024u;
+        }
+        xt = reinterpret_cast<const char*>(a.x + (int64_t)it.t0 * a.ldx + (int64_t)it.k_begin * G_BK) - 3072;
+        wt = reinterpret_cast<const char*>(a.w + (int64_t)it.r0 * a.ldw + (int64_t)it.k_begin * G_BK) - 3072;
+        at = 0; left = it.nk; step = G_BK * 2;
+        last = a.C % G_BK != 0 && it.kz == it.nparts - 1 ? 1 : 0;
+        if (left == last) { row_end(); last = 0; }
+    };
+    auto next_slab = [&]() SQ_INLINE {
+        at += step;
+        if (__builtin_expect(--left > last, 1)) return;
+        if (left == 1) { row_end(); last = 0; return; }
+        jc = valid(jc + stride);
+        if (jc < items) copy_from(jc);
+        else { at -= step; step = 0; left = INT_MAX; }
+    };
+    auto copy = [&](const char* base, uint32_t off, int to, int j) SQ_INLINE {
         const __amdgpu_buffer_rsrc_t buf = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, PAST, 0x00027000);
         const lptr_t lds = (lptr_t)(smem + to);
         if ((j & 3) == 0) __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, lds, 16, off, at, 0, 0);
@@ -185,168 +253,202 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a)
         if ((j & 3) == 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, lds, 16, off, at, 2048, 0);
         if ((j & 3) == 3) __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, lds, 16, off, at, 3072, 0);
     };
-    // `at`: the slab's first column in bytes, `to`: its slot's offset
-    auto copy_x = [&](int at, int to, int j) { copy(xt, at, xo[j], to + wave * (X_SLOT / 4) + (j & ~3) * 1024, j); };
-    auto copy_w = [&](int at, int to, int j) { copy(wt, at, wo[j], to + W_AT + wave * 8192 + (j & ~3) * 1024, j); };
-    auto copy_early = [&](int at, int to, int j) { if constexpr (XE) copy_x(at, to, j); else copy_w(at, to, j); };
-    auto copy_late = [&](int at, int to, int j) { if constexpr (XE) copy_w(at, to, j); else copy_x(at, to, j); };
-    constexpr int ES = XE ? X_SLOT : G_W_SLOT, LS = XE ? G_W_SLOT : X_SLOT;      // their slots' sizes
-    // from the row's last slab on the pieces past its end are asked for past the buffer's end
-    const int plast = lastk < nk && a.C % G_BK != 0 ? lastk : INT_MAX;
-    auto end_early = [&](int q) {
-        if (q < plast) return;
-#pragma unroll
-        for (int j = 0; j < EC; ++j) { uint32_t& o = XE ? xo[j] : wo[j]; o = past[j & 1] ? PAST : o; }
-    };
-    auto end_late = [&](int q) {
-        if (q < plast) return;
-#pragma unroll
-        for (int j = 0; j < LC; ++j) { uint32_t& o = XE ? wo[j] : xo[j]; o = past[j & 1] ? PAST : o; }
-    };
-    auto column = [&](int q) { return (q < nk ? q : nk - 1) * (G_BK * 2); };
+    // `to`: the slot's offset
+    auto copy_x = [&](int to, int j) SQ_INLINE { copy(xt, xo[j], to + wave * (X_SLOT / 4) + (j & ~3) * 1024, j); };
+    auto copy_w = [&](int to, int j) SQ_INLINE { copy(wt, wo[j], to + W_AT + wave * 8192 + (j & ~3) * 1024, j); };
+    auto copy_early = [&](int to, int j) SQ_INLINE { if constexpr (XE) copy_x(to, j); else copy_w(to, j); };
+    auto copy_late = [&](int to, int j) SQ_INLINE { if constexpr (XE) copy_w(to, j); else copy_x(to, j); };
 
     // Fragments.  A lane reads row (lane & 15) + 16 i of its wave's rows, piece 4 kk + (lane >> 4); the swizzle term depends on the
     // row modulo 16 only and the column step kk only flips bit 6 of the offset, so one offset plus compile-time multiples of
     // 16 rows (2048 bytes) covers all reads of a slab.
     half8v fx[TB], fw[2][8];
     const uint32_t foff = (uint32_t)((lane & 15) * 128 + (((lane >> 4) ^ ((lane >> 1) & 7)) << 4));
-    auto read_x = [&](int kk, int at, int i) {
+    auto read_x = [&](int kk, int at, int i) SQ_INLINE {
         fx[i] = *reinterpret_cast<const half8v*>(smem + at + wm * 128 + i * 2048 + (foff ^ (uint32_t)(kk << 6)));
     };
-    auto read_w = [&](int set, int kk, int at, int j) {
+    auto read_w = [&](int set, int kk, int at, int j) SQ_INLINE {
         fw[set][j] = *reinterpret_cast<const half8v*>(smem + W_AT + at + wn * 128 + j * 2048 + (foff ^ (uint32_t)(kk << 6)));
     };
     // product n of a step: token block n / 8, weight-row block n % 8, to and fro
-    auto mma = [&](int set, int n) {
-        const int i = n >> 3, j = i & 1 ? 7 - (n & 7) : n & 7;
-        asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(fw[set][j]), "v"(fx[i]));
+    auto mma = [&](auto set, auto n) SQ_INLINE {
+        constexpr int S = decltype(set)::value, N = decltype(n)::value, i = N >> 3, j = i & 1 ? 7 - (N & 7) : N & 7;
+        acc_product<4 * (8 * i + j)>(fw[S][j], fx[i]);
     };
-    // the accumulators stay in their registers before and behind the loop (without this the compiler copies all 256 into the
-    // other half of the register file at the loop's end, spills, and a launch that needs scratch memory takes 7 us longer)
-#define SQ_PIN() _Pragma("unroll") for (int i = 0; i < TB; ++i) { asm volatile("" : "+a"(acc[i][0]), "+a"(acc[i][1]), "+a"(acc[i][2]), "+a"(acc[i][3]), "+a"(acc[i][4]), "+a"(acc[i][5]), "+a"(acc[i][6]), "+a"(acc[i][7])); }
+    // (the waits of both directions are written out: the compiler does not know what is in the accumulators)
+    auto clear = [&]() SQ_INLINE {
+        asm volatile("s_nop 15\n\ts_nop 15");
+        each<2 * TB>([&](auto q) SQ_INLINE { acc_clear16<16 * decltype(q)::value>(half8v{}); });
+        asm volatile("s_nop 15\n\ts_nop 15");
+    };
 #define SQ_SB() __builtin_amdgcn_sched_barrier(0)
 
+    copy_from(jc);
+#pragma unroll 1
+    for (int q = 0; q < L; ++q) {
 #pragma unroll
-    for (int q = 0; q < E - 1; ++q) {
-        end_early(q);
+        for (int j = 0; j < EC; ++j) copy_early(q * ES, j);
 #pragma unroll
-        for (int j = 0; j < EC; ++j) copy_early(column(q), q * ES, j);
-        if (q == L - 1) break;
-        end_late(q);
-#pragma unroll
-        for (int j = 0; j < LC; ++j) copy_late(column(q), q * LS, j);
+        for (int j = 0; j < LC; ++j) copy_late(q * LS, j);
+        next_slab();
     }
-    __builtin_amdgcn_s_waitcnt(vmcnt_only(AHEAD));
+    __builtin_amdgcn_s_waitcnt(vmcnt_only((L - 1) * (EC + LC)));
     SQ_SB(); __builtin_amdgcn_s_barrier(); SQ_SB();
 #pragma unroll
     for (int i = 0; i < TB - 2; ++i) read_x(0, 0, i);
 #pragma unroll
     for (int j = 0; j < 8; ++j) read_w(0, 0, 0, j);
-    end_late(L - 1);
-#pragma unroll
-    for (int j = 0; j < LC; ++j) copy_late(column(L - 1), (L - 1) * LS, j);
-    // the slots (byte offsets) of the slab being multiplied, of the next one, and the one the early copies go to; the column of the
-    // slab that is copied.  Worked out between the products, a little at a time: a scalar instruction in front of them takes four
-    // clocks of the matrix core's time.
-    int ce = 0, cl = 0, ne = 0, nl = 0, to = (E - 1) * ES, at = column(L);
-    SQ_PIN();
-    asm volatile("s_nop 7");                 // (no wait of the compiler's between the zeroed accumulators and a written-out product)
-#pragma unroll 1
-    for (int s = 0; s < nk; ++s) {
-        if (s + L >= plast) { end_early(s + L); end_late(s + L); }
+    // the slots (byte offsets) of the slab being multiplied, of the next one, and the one the early copies go to.  Worked out between
+    // the products, a little at a time: a scalar instruction in front of them takes four clocks of the matrix core's time.
+    int ce = 0, cl = 0, ne = 0, nl = 0, to = (E - 1) * ES;
+    // the 16-byte stores a wave makes of a whole tile's results, which the next tile's first slab need not wait for
+    constexpr int STORES = 8 * MT;
+    static_assert(AHEAD + STORES < 64, "what the counter holds");
+    Gemm256Item it = item(jm);
+    int togo = it.nk;                        // slabs to the item's end
+    int stores = 0;                          // 1: the item before this one left in STORES stores and this is the first slab behind them
+    // EVENT: a slab that may be an item's first or last one or the last one before the copies go on to another item (or come to a
+    // row's broken end); the others have no branches
+    auto slab = [&](auto event) SQ_INLINE {
+        constexpr bool EVENT = decltype(event)::value;
         // first step: its last X blocks, the second step's fragments, the early copies of slab s + L
-#pragma unroll
-        for (int n = 0; n < NM; ++n) {
-            mma(0, n); SQ_SB();
+        each<NM>([&](auto nn) SQ_INLINE {
+            constexpr int n = decltype(nn)::value;
+            mma(std::integral_constant<int, 0>{}, nn); SQ_SB();
             if (n < 2) read_x(0, XE ? ce : cl, TB - 1 - n);
             if (n >= 2 && n <= 16 && n % 2 == 0) read_w(1, 1, XE ? cl : ce, n / 2 - 1);
             if (n % 8 == 1 && n > 8 && n < NM - 8) read_x(1, XE ? ce : cl, n / 8 - 1);
-            if (n % 4 == 3 && n / 4 < EC) copy_early(at, to, n / 4);
+            if (n % 4 == 3 && n / 4 < EC) copy_early(to, n / 4);
             if (n == NM - 6) { ne = ce + ES; SQ_SB(); }
             if (n == NM - 5) { ne = ne == E * ES ? 0 : ne; SQ_SB(); }
             if (n == NM - 4) { nl = cl + LS; SQ_SB(); }
             if (n == NM - 3) { nl = nl == L * LS ? 0 : nl; SQ_SB(); }
             if (n == NM - 2) { to = ce; SQ_SB(); }
             SQ_SB();
-        }
-        // second step: this wave's copies of slab s + 1 are waited for (those of later slabs stay in flight), and its reads of slab
+        });
+        // second step: this wave's copies of slab s + 1 are waited for (those of later slabs stay in flight, and the stores of the
+        // item before, which went out behind slab s + 1's copies where s is an item's first slab), and its reads of slab
         // s, whose slots the copies behind the barrier overwrite; then the barrier: everybody's copies have landed and
         // everybody has read slab s to the end.  (Six products behind the last of those reads their wait costs little.)
-#pragma unroll
-        for (int n = 0; n < NM; ++n) {
-            mma(1, n); SQ_SB();
+        each<NM>([&](auto nn) SQ_INLINE {
+            constexpr int n = decltype(nn)::value, GAP = MT == 2 ? 2 : 4;
+            mma(std::integral_constant<int, 1>{}, nn); SQ_SB();
             if (n < 2) read_x(1, XE ? ce : cl, TB - 1 - n);
             if (n == 7) {
-                __builtin_amdgcn_s_waitcnt(vmcnt_and_lds(AHEAD)); SQ_SB();
-                __builtin_amdgcn_s_barrier(); SQ_SB();
+                if (!EVENT || !stores) __builtin_amdgcn_s_waitcnt(vmcnt_and_lds(AHEAD));
+                else __builtin_amdgcn_s_waitcnt(vmcnt_and_lds(AHEAD + STORES));
+                SQ_SB(); __builtin_amdgcn_s_barrier(); SQ_SB();
             }
             if (n >= 8 && n <= 22 && n % 2 == 0) read_w(0, 0, XE ? nl : ne, n / 2 - 4);
             if (n % 8 == 1 && n > 8 && n < NM - 8) read_x(0, XE ? ne : nl, n / 8 - 1);
-            constexpr int GAP = MT == 2 ? 2 : 4;
-            if (n >= 11 && (n - 11) % GAP == 0 && (n - 11) / GAP < LC) copy_late(at, cl, (n - 11) / GAP);
-            if (n == NM - 4) { at = column(s + 1 + L); SQ_SB(); }
+            if (n >= 11 && (n - 11) % GAP == 0 && (n - 11) / GAP < LC) copy_late(cl, (n - 11) / GAP);
+            if (n == NM - 4) { if constexpr (EVENT) next_slab(); else at += step; SQ_SB(); }
             if (n == NM - 3) { ce = ne; cl = nl; SQ_SB(); }
             SQ_SB();
+        });
+    };
+    uint32_t scale[2] = {};                  // of weight rows lane and 64 + lane of this wave's 128, fp16
+    clear();
+    while (true) {
+        const int plain = stores ? 0 : min(togo, left - last) - 1;
+#pragma unroll 1
+        for (int s = 0; s < plain; ++s) slab(std::false_type{});
+        if (plain > 0) { togo -= plain; left -= plain; }
+        // (asked for a slab ahead: behind the loop their latency would be the tile's)
+        if (togo == 1) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) scale[h] = gemm256_scale<true>(a.sc, min(it.r0 + wn + h * 64 + lane, a.R - 1));
         }
-    }
-    asm volatile("s_nop 15\n\ts_nop 15");    // the last products' results are behind the loop before they are read
-    SQ_PIN();
-#undef SQ_SB
-#undef SQ_PIN
-    __builtin_amdgcn_s_waitcnt(vmcnt_and_lds(0));
-    __syncthreads();                         // every wave is done with the operand ring, and no copy is on its way into it
+        slab(std::true_type{});
+        stores = 0;
+        if (--togo > 0) continue;
+        asm volatile("s_nop 15\n\ts_nop 15");    // the last products' results are there before they are read
 
-    // Results leave column of registers after column of registers.  A split tile's go to its partial tile as they are.  16-bit
-    // ones go through LDS: every wave lays its 32 MT x 128 tile out token-major (8 bytes per write) and stores it in 16-byte
-    // pieces, 256 contiguous bytes per token (2-byte stores straight from the accumulators cost 49 us of a 376 us product of
-    // a 2048 x 18944 output).
-    const int quad4 = 4 * (lane >> 4), tok = lane & 15;
-    float* scales = reinterpret_cast<float*>(smem + 2 * BM * G_EP_PITCH);        // behind the four waves' tiles
-    scales[tid] = gemm256_scale<true>(a.sc, r0 + tid < a.R ? r0 + tid : a.R - 1);
-    __syncthreads();
-    float* part = a.part + ((int64_t)(tile - a.main_tiles) * a.kt + kz) * (BM * G_BN);
-    unsigned char* my = smem + wave * (BM / 2 * G_EP_PITCH);
+        // Results leave block of 16 tokens after block.  A split tile's go to its partial tile as they are.  16-bit ones go
+        // through LDS, two blocks (MT = 2: one) at a time: every wave lays them out token-major, 256 bytes a token, in its quarter of
+        // the early operand's slot of the slab that everybody has read to the end (the quarter that it copies into next itself),
+        // 16-byte piece c of token t at slot c ^ (t % 16), and stores them in 16-byte pieces, 256 contiguous bytes per token
+        // (2-byte stores straight from the accumulators cost 49 us of a 376 us product of a 2048 x 18944 output).
+        int le = lane;
+        const int64_t ldy = a.ldy;
+        asm volatile("" : "+v"(le));             // (nothing of what follows is worked out in front of the loop and kept in registers that it lacks)
+        const int quad = le >> 4, tok = le & 15;
+        const int split = it.nparts - 1;
+        stores = __builtin_amdgcn_readfirstlane(EP != SQ_F32 && split == 0 && it.t0 + BM <= a.T && it.r0 + G_BN <= a.R ? 1 : 0);
+        float* part = a.part + ((int64_t)(it.tile - a.main_tiles) * a.kt + it.kz) * (BM * G_BN);
+        float4v sc[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const int rl = j * 16 + quad4;
-        const float4v sc = *reinterpret_cast<const float4v*>(scales + wn + rl);
+        for (int j = 0; j < 8; ++j)
 #pragma unroll
-        for (int i = 0; i < TB; ++i) {
-            const int tl = i * 16 + tok;
-            const float4v val = acc[i][j];
-            if (nparts > 1) {
-                *reinterpret_cast<float4v*>(part + (wm + tl) * G_BN + wn + rl) = val;
-            } else if constexpr (EP != SQ_F32) {
-                const float4v o = val * sc;
-                *reinterpret_cast<u32x2*>(my + tl * G_EP_PITCH + rl * 2) =
-                    EP == SQ_BF16 ? u32x2{f2bf_x2(o[0], o[1]), f2bf_x2(o[2], o[3])} : u32x2{f2h_x2(o[0], o[1]), f2h_x2(o[2], o[3])};
-            } else {
-                const int t = t0 + wm + tl, r = r0 + wn + rl;
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (t < a.T && r + e < a.R) store_y(a.y, a.y_dtype, (int64_t)t * a.ldy + a.y_off + r + e, val[e] * sc[e]);
+            for (int e = 0; e < 4; ++e) sc[j][e] = h2f((uint16_t)__builtin_amdgcn_ds_bpermute(((j & 3) * 16 + 4 * quad + e) * 4, (int)scale[j >> 2]));
+        constexpr int TBP = ES / 4 / 4096;
+        static_assert(TB % TBP == 0, "whole passes");
+        unsigned char* my = smem + (XE ? 0 : W_AT) + to + wave * (ES / 4);
+        uint16_t* dst = reinterpret_cast<uint16_t*>(a.y) + (int64_t)(it.t0 + wm) * ldy + a.y_off + it.r0 + wn + (quad * ldy + tok * 8);
+        each<TB / TBP>([&](auto pp) SQ_INLINE {
+            constexpr int p = decltype(pp)::value;
+            auto block = [&](auto q, auto use) SQ_INLINE {
+                constexpr int b = decltype(q)::value / 8, j = decltype(q)::value % 8;
+                use(b, j, acc_read<4 * (8 * (p * TBP + b) + j)>());
+            };
+            if (split) {
+                each<8 * TBP>([&](auto q) SQ_INLINE {
+                    block(q, [&](int b, int j, float4v val) {
+                        *reinterpret_cast<float4v*>(part + (wm + (p * TBP + b) * 16 + tok) * G_BN + wn + j * 16 + 4 * quad) = val;
+                    });
+                });
+                return;
             }
-            if (i & 1) __builtin_amdgcn_sched_barrier(0);
-        }
-    }
-    if (EP == SQ_F32 || nparts > 1) return;
-    uint16_t* yb = reinterpret_cast<uint16_t*>(a.y);
-#pragma unroll 4
-    for (int k = 0; k < 8 * MT; ++k) {
-        const int idx = k * 64 + lane, tl = idx >> 4, piece = idx & 15;
-        const int t = t0 + wm + tl, r = r0 + wn + piece * 8;
-        if (t >= a.T || r >= a.R) continue;
-        const u32x4 v = *reinterpret_cast<const u32x4*>(my + tl * G_EP_PITCH + piece * 16);
-        uint16_t* dst = yb + (int64_t)t * a.ldy + a.y_off + r;
-        if (r + 8 <= a.R) {
-            *reinterpret_cast<u32x4*>(dst) = v;
-        } else {
+            if constexpr (EP == SQ_F32) {
+                each<8 * TBP>([&](auto q) SQ_INLINE {
+                    block(q, [&](int b, int j, float4v val) {
+                        const int t = it.t0 + wm + (p * TBP + b) * 16 + tok, r = it.r0 + wn + j * 16 + 4 * quad;
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
-                if (r + e < a.R) dst[e] = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
-        }
+                        for (int e = 0; e < 4; ++e)
+                            if (t < a.T && r + e < a.R) store_y(a.y, a.y_dtype, (int64_t)t * ldy + a.y_off + r + e, val[e] * sc[j][e]);
+                    });
+                });
+                return;
+            }
+            each<8 * TBP>([&](auto q) SQ_INLINE {
+                block(q, [&](int b, int j, float4v val) {
+                    const float4v o = val * sc[j];
+                    *reinterpret_cast<u32x2*>(my + (b * 16 + tok) * 256 + (((2 * j + (quad >> 1)) ^ tok) * 16) + (quad & 1) * 8) =
+                        EP == SQ_BF16 ? u32x2{f2bf_x2(o[0], o[1]), f2bf_x2(o[2], o[3])} : u32x2{f2h_x2(o[0], o[1]), f2h_x2(o[2], o[3])};
+                });
+            });
+            u32x4 v[4 * TBP];
+#pragma unroll
+            for (int k = 0; k < 4 * TBP; ++k) v[k] = *reinterpret_cast<const u32x4*>(my + (k * 4 + quad) * 256 + ((tok ^ ((k * 4 + quad) & 15)) * 16));
+            if (stores) {
+#pragma unroll
+                for (int k = 0; k < 4 * TBP; ++k) { *reinterpret_cast<u32x4*>(dst) = v[k]; dst += 4 * ldy; }
+                return;
+            }
+#pragma unroll
+            for (int k = 0; k < 4 * TBP; ++k) {
+                const int t = it.t0 + wm + p * TBP * 16 + k * 4 + quad, over = it.r0 + wn + tok * 8 - a.R;     // (-8 and less: all eight are rows of W)
+                if (t < a.T && over <= -8) {
+                    *reinterpret_cast<u32x4*>(dst) = v[k];
+                } else if (t < a.T) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        if (e + over < 0) dst[e] = (uint16_t)(v[k][e >> 1] >> (16 * (e & 1)));
+                }
+                dst += 4 * ldy;
+            }
+        });
+        jm = valid(jm + stride);
+        if (jm >= items) break;
+        it = item(jm);
+        togo = it.nk;
+        clear();
     }
+#undef SQ_SB
+    __builtin_amdgcn_s_waitcnt(vmcnt_only(0));       // no copy is on its way into LDS that is another workgroup's by then
 }
+
+#undef SQ_INLINE
 
 // fp16 copy of a bf16 activation matrix (round to nearest even; exact for every fp16-normal value)
 __global__ __launch_bounds__(256) void bf16_to_f16_kernel(const uint16_t* __restrict__ x, int64_t ldx, int T, int C,
@@ -374,7 +476,7 @@ __global__ __launch_bounds__(256) void gemm256_reduce_kernel(const float* __rest
     for (int kz = 1; kz < kt; ++kz) sum += *reinterpret_cast<const float4v*>(p + (int64_t)kz * size);
 #pragma unroll
     for (int q = 0; q < 4; ++q)
-        if (r + q < R) store_y(y, y_dtype, (int64_t)t * ldy + y_off + r + q, sum[q] * gemm256_scale<false>(sc, r + q));
+        if (r + q < R) store_y(y, y_dtype, (int64_t)t * ldy + y_off + r + q, sum[q] * h2f(gemm256_scale<false>(sc, r + q)));
 }
 
 // How a T x R output is cut: tiles of 64 mt token rows; whole rounds of whole tiles over the `cus` CUs, and the tiles of
@@ -452,7 +554,8 @@ int launch_gemm256(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ld
     a.kt = pl.kt;
     a.part = part;
     const bool vec = y_dtype != SQ_F32 && ((uintptr_t)y & 15) == 0 && ldy % 8 == 0 && y_off % 8 == 0;
-    const unsigned grid = (unsigned)(8 * ((pl.main_tiles + 7) / 8 + (pl.tail_tiles * pl.kt + 7) / 8));
+    const int per = (pl.main_tiles + 7) / 8 + (pl.tail_tiles * pl.kt + 7) / 8;       // an XCD's tiles and parts
+    const unsigned grid = (unsigned)(8 * std::min(per, std::max(1, device_cus() / 8)));
     hipLaunchKernelGGL(kernels[pl.mt - 2][!vec ? 2 : y_dtype == SQ_BF16 ? 1 : 0], dim3(grid), dim3(G_WAVES * 64), gemm256_lds(pl.mt), s, a);
     int rc = check_launch("sq_linear_gemm(gemm256)");
     if (rc || pl.tail_tiles == 0) return rc;

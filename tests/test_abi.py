@@ -208,3 +208,28 @@ def test_tile_gemm_waits_for_its_reads_before_the_barrier(tmp_path):
         assert waits and all("lgkmcnt(0)" in w for w in waits), waits
         variants += 1
     assert variants == 9
+
+
+def test_tile_gemm_accumulators_and_stores(tmp_path):
+    """The accumulators are registers that the source names, so nothing else may live in them; and a tile's first slab does not wait
+    for the 8 MT stores of the whole tile before it, so there have to be that many (as many again at a matrix' edges, 16 MT of a part's)."""
+    import os
+    import subprocess
+    from quantexperiments_amd import build
+    try:
+        hipcc = build._hipcc()
+    except RuntimeError:
+        pytest.skip("no hipcc")
+    out = tmp_path / "gemm256.s"
+    subprocess.run([hipcc, *build.FLAGS, "-S", "--offload-device-only", str(build.CSRC / "sq_gemm256.hip"), "-o", str(out)], check=True,
+                   capture_output=True, env=dict(os.environ, TMPDIR=str(tmp_path)))
+    variants = 0
+    for body in re.split(r"(?m)^(?=_ZN2sq14gemm256_kernel\w+:)", out.read_text())[1:]:
+        lines = [l.split(";")[0].strip() for l in body[:body.index(".Lfunc_end")].splitlines()]
+        lines = [l for l in lines if l and not l.startswith(".")]
+        assert all(l.startswith(("v_mfma_", "v_accvgpr_read")) for l in lines if re.search(r"\ba(\[\d|\d)", l))
+        ep, mt = map(int, re.match(r"_ZN2sq14gemm256_kernelILi(\d)ELi(\d)E", body).groups())
+        if ep:
+            assert sum(l.startswith("global_store_dwordx4") for l in lines) == 32 * mt
+        variants += 1
+    assert variants == 9

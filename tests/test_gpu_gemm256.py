@@ -78,6 +78,24 @@ def test_tile_heights(T, R, C, dtype):
     assert torch.isnan(y[:, R:]).all()
 
 
+@pytest.mark.parametrize("T,R,C", [
+    (512, 70400, 64), (520, 70000, 72), (512, 40960, 192), (700, 33000, 328),        # tiles of 256 token rows: one to six slabs, whole and broken
+    (192, 140000, 64), (380, 70000, 136), (128, 140032, 64), (121, 140000, 200)])    # of 192 and 128
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_tiles_one_after_another(T, R, C, dtype):
+    """Several tiles to a workgroup, whole ones and ones at the matrix' edges in turn, whose 16-bit results leave in 16-byte pieces
+    while the next tile's slabs arrive."""
+    g = torch.Generator(device="cuda").manual_seed(T + R)
+    x, w = (torch.randn(n, C, generator=g, device="cuda").half() for n in (T, R))
+    y = torch.full((T, R + 8), float("nan"), dtype=dtype, device="cuda")
+    for _ in range(3):
+        gemm_dense(w, x, y[:, :R])
+    ref = x.double() @ w.double().T
+    bound = 17.4 * C * 2.0 ** -24 + 2.0 ** (-8 if dtype == torch.bfloat16 else -11) * ref.abs()     # as in test_tile_heights
+    assert ((y[:, :R].double() - ref).abs() <= bound).all()
+    assert torch.isnan(y[:, R:]).all()
+
+
 @pytest.mark.parametrize("limit", [0, 150 * 512 * 2, 1 << 30])
 @pytest.mark.parametrize("T", [40, 800])
 def test_dequant_route_in_groups_of_pieces(limit, T, monkeypatch):
