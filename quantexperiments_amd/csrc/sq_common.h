@@ -95,10 +95,22 @@ __device__ __forceinline__ uint32_t tag_at(const uint32_t* __restrict__ row, int
     return (uint32_t)(v >> s) & ((1u << bits) - 1u);
 }
 
+// Sum over the wave, the same in every lane: v += v of lane ^ 32, then ^ 16, 8, 4, 2, 1.  In registers: swaps of half waves and of
+// rows of 16 lanes, and rotations of a row, whose values repeat every 8, 4, 2 lanes by the time they are rotated by 4, 2, 1 (through
+// __shfl_xor, six LDS round trips one behind the other, an add + norm of 8 x 3584 took 0.3 us more).
+template <int N> __device__ __forceinline__ float row_rotated(float v) {
+    const int i = __builtin_bit_cast(int, v);
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, 0x120 + N, 0xF, 0xF, false));
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+    const uint32_t a = __builtin_bit_cast(uint32_t, v);
+    const auto h = __builtin_amdgcn_permlane32_swap(a, a, false, false);
+    v = __builtin_bit_cast(float, (uint32_t)h[0]) + __builtin_bit_cast(float, (uint32_t)h[1]);
+    const uint32_t b = __builtin_bit_cast(uint32_t, v);
+    const auto r = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+    v = __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
+    v += row_rotated<8>(v); v += row_rotated<4>(v); v += row_rotated<2>(v);
+    return v + row_rotated<1>(v);
 }
 
 // A caller's workspace starts with SQ_WS_HEADER bytes that only the tag-stream kernel touches: the partial sums its

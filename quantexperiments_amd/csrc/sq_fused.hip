@@ -129,7 +129,6 @@ int launch_fused(const sq_matrix* mats, int n, const void* x, int x_dtype, int64
     a.k32 = rounds * spr;
     a.x = (const unsigned char*)ws;
     char* part = (char*)ws + fused_x_bytes(mats, p);
-    int64_t quads = 0;
     for (int i = 0; i < n; ++i) {
         FusedPiece& P = a.p[i];
         const sq_matrix& m = mats[i];
@@ -139,7 +138,6 @@ int launch_fused(const sq_matrix* mats, int n, const void* x, int x_dtype, int64
         part += fused_part_bytes(m, T, p.ks);
         P.wg0 = a.per_tb;
         a.per_tb += (m.R + 32 * p.tw - 1) / (32 * p.tw) * p.ks;
-        quads += (int64_t)T * ((m.R + 3) / 4);
     }
     const dim3 xgrid((unsigned)rounds, (unsigned)(p.tbs * NT));
     if (spr == 8) hipLaunchKernelGGL(fused_x_kernel<8>, xgrid, dim3(256), 0, s, (const uint16_t*)x, ldx, x_dtype, T, m0.C, NT, a.k32, (unsigned char*)ws);
@@ -152,8 +150,7 @@ int launch_fused(const sq_matrix* mats, int n, const void* x, int x_dtype, int64
     else if (m0.bits == 10) rc = launch_fused_b10d4(a, p.nw, p.tw, grid, s);
     else rc = launch_fused_b8d4(a, p.nw, p.tw, grid, s);
     if (rc || p.ks == 1) return rc;
-    hipLaunchKernelGGL(slice_sum_kernel<FusedArgs>, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s, a);
-    return check_launch("sq_linear_gemm(fused reduce)");
+    return launch_slice_sum(a.p, n, a.ks, T, y, y_dtype, ldy, s);
 }
 
 }  // namespace sq

@@ -1,6 +1,7 @@
 // Host side of the decode-time product: picks the team geometry per shape, fuses stacked pieces
 // into one persistent launch, prepares permuted activations for pieces with column orders.
 #include "sq_rows_mfma.h"
+#include "sq_slices.h"
 #include "sq_stream.h"
 
 namespace sq {
@@ -13,17 +14,6 @@ int launch_mma_b16d8(int, const MmaArgs&, int, int, int, int, size_t, hipStream_
 int launch_mma_b12d4(int, const MmaArgs&, int, int, int, int, size_t, hipStream_t);
 int launch_mma_b10d4(int, const MmaArgs&, int, int, int, int, size_t, hipStream_t);
 int launch_mma_b8d4(int, const MmaArgs&, int, int, int, int, size_t, hipStream_t);
-
-__global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ part, int ks, int B, int R,
-                                                            const uint16_t* __restrict__ row_scale, void* y, int64_t ldy,
-                                                            int y_off, int y_dtype) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= B * R) return;
-    const int b = i / R, r = i - b * R;
-    float v = 0.f;
-    for (int s = 0; s < ks; ++s) v += part[((int64_t)s * B + b) * R + r];
-    store_y(y, y_dtype, (int64_t)b * ldy + y_off + r, v * h2f(row_scale[r]));
-}
 
 // xp[m, b, c] = fp16(x[b, perms[m, c]])
 __global__ __launch_bounds__(256) void permute_x_kernel(const uint16_t* __restrict__ x, int64_t ldx, int x_dtype,
@@ -357,15 +347,7 @@ static int launch_mma_group(const sq_matrix* mats, int cnt, const void* x, int x
 #undef GRID
 #undef SQ_CASE
     if (rc) return rc;
-    if (pl.ks > 1)
-        for (int k = 0; k < cnt; ++k) {
-            const sq_matrix& mk = mats[k];
-            hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((B * mk.R + 255) / 256)), dim3(256), 0, s,
-                               a.p[k].part, pl.ks, B, mk.R, mk.row_scale, y, ldy, mk.y_off, y_dtype);
-            rc = check_launch("sq_linear_small(splitk_reduce)");
-            if (rc) return rc;
-        }
-    return SQ_OK;
+    return pl.ks > 1 ? launch_slice_sum(a.p, cnt, pl.ks, B, y, y_dtype, ldy, s) : SQ_OK;
 }
 
 // (Pieces with column orders would gather the producer's three operands through every order of a run from memory:

@@ -101,7 +101,6 @@ static int launch_mid_rows(const sq_matrix* mats, int n, const MidPlan& pl, cons
     a.U = dense ? m0.C / 8 : mid_units(m0); a.ks = pl.ks;
     a.table_bytes = !dense && m0.d == 4 ? (m0.G << m0.bits) * 8 : 0;
     int wg = 0;
-    int64_t quads = 0;
     char* part = (char*)ws;
     for (int i = 0; i < n; ++i) {
         MidPiece& P = a.p[i];
@@ -112,7 +111,6 @@ static int launch_mid_rows(const sq_matrix* mats, int n, const MidPlan& pl, cons
         part += mid_part_bytes(m, T, pl.ks);
         P.wg0 = wg;
         wg += ((m.R + 16 * pl.nw * pl.tw - 1) / (16 * pl.nw * pl.tw)) * pl.ks;
-        quads += (int64_t)T * ((m.R + 3) / 4);
     }
     int rc = SQ_EUNSUPPORTED;
     if (dense) rc = launch_mid_dense(a, pl.nt, pl.tw, pl.st, pl.nw, wg, s);
@@ -121,8 +119,7 @@ static int launch_mid_rows(const sq_matrix* mats, int n, const MidPlan& pl, cons
     else if (m0.bits == 10) rc = launch_mid_b10d4(a, pl.nt, pl.tw, pl.st, pl.nw, wg, s);
     else if (m0.bits == 8) rc = launch_mid_b8d4(a, pl.nt, pl.tw, pl.st, pl.nw, wg, s);
     if (rc || pl.ks == 1) return rc;
-    hipLaunchKernelGGL(slice_sum_kernel<MidArgs>, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s, a);
-    return check_launch("sq_linear_gemm(mid reduce)");
+    return launch_slice_sum(a.p, n, a.ks, T, y, y_dtype, ldy, s);
 }
 
 // For decoded weights: one tile of rows per wave, so that small stacks spread (593 x 1984 at 16 rows: 17 us with the decode, 22

@@ -11,15 +11,20 @@ namespace sq {
 constexpr int NB_THREADS = 1024;
 constexpr int NB_MAX_LDS_C = 32256;          // a row staged as 16-bit values for the column-order copies: 63 KB of LDS
 
-// sum over the workgroup, the same value in every thread
+// sum over the workgroup, the same value in every thread: its waves' sums in turn (those of missing waves are zeros, all 16 are
+// read at once: one by one, in a loop over as many as there are, 8 x 3584 took 0.4 us more).  Called once.
 __device__ __forceinline__ float block_sum(float v, float* red) {
     v = wave_sum(v);
-    const int wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    if ((threadIdx.x & 63) == 0) red[wave] = v;
+    const int tid = threadIdx.x, nw = blockDim.x >> 6;
+    if ((tid & 63) == 0) red[tid >> 6] = v;
+    if (tid >= nw && tid < NB_THREADS / 64) red[tid] = 0.f;
     __syncthreads();
+    float4v s[NB_THREADS / 256];
+#pragma unroll
+    for (int i = 0; i < NB_THREADS / 256; ++i) s[i] = reinterpret_cast<const float4v*>(red)[i];
     float t = 0.f;
-    for (int i = 0; i < nw; ++i) t += red[i];                   // same order in every thread
-    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NB_THREADS / 64; ++i) t += s[i >> 2][i & 3];
     return t;
 }
 
@@ -40,8 +45,9 @@ struct AddnormArgs {
 // element i of h_out after its last read of element i of h_in, so h_out may be h_in then.
 __global__ __launch_bounds__(NB_THREADS) void addnorm_kernel(AddnormArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint16_t row16[];
-    __shared__ float red[NB_THREADS / 64];
-    const int b = blockIdx.x / a.blocks_per_row, part = blockIdx.x % a.blocks_per_row;
+    __shared__ __attribute__((aligned(16))) float red[NB_THREADS / 64];
+    int b = blockIdx.x, part = 0;
+    if (a.blocks_per_row > 1) b = blockIdx.x / a.blocks_per_row, part = blockIdx.x % a.blocks_per_row;
     const float* h = a.h_in + (int64_t)b * a.ld_h;
     const int64_t ab = (int64_t)b * a.ld_add;
     uint16_t* out = reinterpret_cast<uint16_t*>(a.out);
@@ -169,7 +175,9 @@ int launch_addnorm(const float* h_in, float* h_out, int64_t ld_h, const void* ad
     // 16-byte accesses: whole chunks, every row of every tensor 16-byte aligned
     a.vec = C % 8 == 0 && (B == 1 || (ld_h % 4 == 0 && (!add || ld_add % 8 == 0))) &&
             ((((uintptr_t)h_in | (uintptr_t)h_out | (uintptr_t)add | (uintptr_t)w | (uintptr_t)out) & 15) == 0);
-    hipLaunchKernelGGL(addnorm_kernel, dim3((unsigned)(B * a.blocks_per_row)), dim3(NB_THREADS), perms ? (size_t)C * 2 : 0, s, a);
+    // (a chunk per thread: waves without one would only be started and waited for)
+    const int chunks = C / 8, threads = a.vec && !perms && chunks < NB_THREADS ? (chunks + 63) / 64 * 64 : NB_THREADS;
+    hipLaunchKernelGGL(addnorm_kernel, dim3((unsigned)(B * a.blocks_per_row)), dim3((unsigned)threads), perms ? (size_t)C * 2 : 0, s, a);
     return check_launch("sq_addnorm");
 }
 

@@ -20,7 +20,7 @@
 // every MMA_TT tiles when the codebook is read through the cache, after all the tiles of the workgroup (as
 // many as LDS holds accumulators for: MmaArgs.tg) when it sits in LDS, so that the waves of a launch of the
 // 7B shapes meet once.  Rows longer than KW * RW rounds are split over `ks` workgroups whose
-// partial sums go to a workspace and are added, in slice order, by splitk_reduce_kernel.
+// partial sums go to a workspace and are added, in slice order, by slice_sum_kernel.
 #pragma once
 #include <mutex>
 #include <unordered_map>
@@ -512,11 +512,6 @@ void rows_mfma_kernel(MmaArgs a) {
     }
     SQ_TRACE_POINT(19);
 }
-
-// y[b, y_off + r] = row_scale[r] * sum over column slices (in slice order) of part[s, b, r]
-__global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ part, int ks, int B, int R,
-                                                            const uint16_t* __restrict__ row_scale, void* y, int64_t ldy,
-                                                            int y_off, int y_dtype);
 
 // op 0: launch; op 1: workgroups of `threads` threads and `smem` bytes of LDS that fit on one CU
 template <int BITS, int D, int RW, int NT>

@@ -52,6 +52,20 @@ def test_rows_that_one_launch_takes_whole(rows, C, bits, G):
             assert rel_max_err(y[:, :n].cpu().numpy(), want[:, :n]) < 1e-5 and bool(y[:, n:].isnan().all()), B
 
 
+@pytest.mark.parametrize("rows", [(40,), (37, 64, 21), (33, 40)])
+@pytest.mark.parametrize("C,bits", [(18944, 12), (66560, 12), (98304, 8)])       # 5 slices, and more than eight
+def test_sums_of_slices(rows, C, bits):
+    """Rows in quads and not, pieces behind pieces of odd rows (whose results then begin anywhere), every result type."""
+    ss = [synth(R, C, 4, bits, 1, 1, seed=R + bits) for R in rows]
+    lins, w = [to_device(s) for s in ss], np.concatenate([s.decode().astype(np.float64) for s in ss])
+    x = rand_x(3, C, torch.bfloat16, seed=C)
+    want = x.half().float().numpy().astype(np.float64) @ w.T
+    for dtype, tol in ((torch.float32, 1e-5), (torch.float16, 2.0 ** -11 + 1e-5), (torch.bfloat16, 2.0 ** -8 + 1e-5)):      # (the first as above)
+        y = torch.full((3, sum(rows)), float("nan"), dtype=dtype, device="cuda")
+        linear_small(lins, x.cuda(), y)
+        assert rel_max_err(y.float().cpu().numpy(), want) < tol, dtype
+
+
 @pytest.mark.parametrize("rows,C,bits,G,B", [((300,), 8192, 12, 1, 8), ((300,), 6912, 12, 4, 16), ((40, 300), 7168, 8, 1, 2)])
 @pytest.mark.parametrize("native", [True, False], ids=["native", "python"])
 def test_products_that_need_no_sums_share_nothing(rows, C, bits, G, B, native, monkeypatch):
