@@ -58,9 +58,9 @@ def test_sums_of_slices(rows, C, bits):
     """Rows in quads and not, pieces behind pieces of odd rows (whose results then begin anywhere), every result type."""
     ss = [synth(R, C, 4, bits, 1, 1, seed=R + bits) for R in rows]
     lins, w = [to_device(s) for s in ss], np.concatenate([s.decode().astype(np.float64) for s in ss])
-    x = rand_x(3, C, torch.bfloat16, seed=C)
-    want = x.half().float().numpy().astype(np.float64) @ w.T
     for dtype, tol in ((torch.float32, 1e-5), (torch.float16, 2.0 ** -11 + 1e-5), (torch.bfloat16, 2.0 ** -8 + 1e-5)):      # (the first as above)
+        x = rand_x(3, C, torch.float16 if dtype == torch.float32 else dtype, seed=C)
+        want = x.half().float().numpy().astype(np.float64) @ w.T
         y = torch.full((3, sum(rows)), float("nan"), dtype=dtype, device="cuda")
         linear_small(lins, x.cuda(), y)
         assert rel_max_err(y.float().cpu().numpy(), want) < tol, dtype
