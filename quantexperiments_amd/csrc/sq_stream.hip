@@ -104,8 +104,8 @@ template <int PRO>
 __device__ __forceinline__ ProRaw pro_fetch(const StreamArgs& a, int ci) {
     ProRaw r;
     const u32x4 hi = reinterpret_cast<const u32x4*>(a.w)[ci];
-    u32x4 lo = u32x4{0u, 0u, 0u, 0u};
-    if (a.add) lo = reinterpret_cast<const u32x4*>(a.add)[ci];
+    // (without a branch, behind which the loads would be waited for; nothing to add: not looked at)
+    const u32x4 lo = reinterpret_cast<const u32x4*>(a.add ? a.add : a.w)[ci];
 #pragma unroll
     for (int k = 0; k < 4; ++k) { r.lo[k] = lo[k]; r.hi[k] = hi[k]; }
     if (PRO == 1) {
@@ -121,7 +121,8 @@ __device__ __forceinline__ float pro_f(uint32_t pair, int k, int dtype) {
 }
 // v = h + add of element k of a fetched chunk (PRO 1)
 __device__ __forceinline__ float pro_v(const StreamArgs& a, const ProRaw& r, int k) {
-    return a.add ? r.h[k] + pro_f(r.lo[k >> 1], k, a.x_dtype) : r.h[k];
+    const float sum = r.h[k] + pro_f(r.lo[k >> 1], k, a.x_dtype);
+    return a.add ? sum : r.h[k];
 }
 template <int PRO>
 __device__ __forceinline__ u32x4 pro_finish(const StreamArgs& a, const ProRaw& r, float rstd) {
@@ -327,7 +328,11 @@ __global__ __launch_bounds__(STREAM_NW * 64) void stream_kernel(StreamArgs a) {
     // The error word of the exchange, requested now and looked at when y is written: once a launch on this workspace
     // has given up waiting, partial sums may have arrived late and the header may be dirty; every launch then writes
     // NaN until the host has reset the workspace.
-    const uint32_t err0 = __hip_atomic_load(a.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // (Through a vector index, as `head`: else some variants make it a scalar on the spot, behind a wait for a memory round trip;
+    // two rows of a 7B layer 73.6 us, now 72.2.)
+    int err_at = 0;
+    asm volatile("" : "+v"(err_at));
+    const uint32_t err0 = __hip_atomic_load(a.err + err_at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     int kcur = wave, knext = 2 * NW - 1 - wave;
     if (split > 1) {                                            // one share of one group per wave, or nothing
         kcur = wave < ng * split ? wave / split : ng;
@@ -346,22 +351,17 @@ __global__ __launch_bounds__(STREAM_NW * 64) void stream_kernel(StreamArgs a) {
     const u32x2 head_w = *reinterpret_cast<const u32x2*>(gw + kc0);
     const uint32_t head_s = slots[(size_t)kc0 * 64 + lane];
     __builtin_amdgcn_sched_barrier(0);
-    // The codebook slice is copied global -> LDS without passing through registers (a wave instruction moves 1 KB, lane l
-    // to the wave's base + 16 l).
-    {
-        const unsigned char* src = reinterpret_cast<const unsigned char*>(P.table) + (size_t)s * STREAM_TAB;
-#pragma unroll
-        for (int k = 0; k < STREAM_TAB / (NTH * 16); ++k)
-            if (k >= kd)
-                __builtin_amdgcn_global_load_lds((stream_gptr_t)(src + ((size_t)k * NTH + tid) * 16),
-                                                 (stream_lptr_t)(lds + (k * NTH + wave * 64) * 16), 16, 0, 0);
-    }
-    __builtin_amdgcn_sched_barrier(0);
     StreamHeadRaw hn;
     evec nx[STREAM_PF];
 #pragma unroll
     for (int q = 0; q < STREAM_PF; ++q) nx[q] = F::zero();
 
+    // a barrier behind this wave's LDS reads and writes (__syncthreads would wait for the slice's copies too)
+    auto lds_barrier = [&]() {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
     // Stage this part of the NB activation rows (as fp16); the first group's steps are requested before anything waits
     // for the staging loads.
     {
@@ -376,12 +376,86 @@ __global__ __launch_bounds__(STREAM_NW * 64) void stream_kernel(StreamArgs a) {
             it_o[k] = no > 1 ? it / nc : 0;
             it_c[k] = it - it_o[k] * nc;
         }
-        if (PRO != 0) {
-            // every operand of the produced row is requested before anything waits: this thread's chunks, then
-            // (PRO 1) its share of the whole row for the mean square
-            ProRaw raw[NX];
+        // Every operand of a produced row is requested before anything waits: this thread's chunks, then (PRO 1, a row in several
+        // parts) its chunk of the whole row for the mean square; in one part these are the same, and all lanes ask for one chunk.
+        ProRaw raw[NX], rown;
+        if constexpr (PRO != 0) {
 #pragma unroll
             for (int k = 0; k < NX; ++k) raw[k] = pro_fetch<PRO>(a, c0 + it_c[k]);
+            if constexpr (NX == 1) rown = pro_fetch<1>(a, nc == P.U ? 0 : min(tid, P.U - 1));
+        }
+        // LATE: rows behind the codebook slice (see there), also in the variants that lack the registers; gathers from memory, which
+        // wait for their positions, always
+        constexpr bool LATE = PRO == 0 && (NB < 4 || (ORD && NB * NX > 4));
+        auto rows = [&](bool natural, bool gathered) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                const uint16_t* xr = a.x + (int64_t)min(b, a.nb - 1) * a.ldx;
+                if (perms == nullptr) {
+                    if (!natural) continue;
+                    const u32x4* xsrc = reinterpret_cast<const u32x4*>(xr) + c0;
+#pragma unroll
+                    for (int k = 0; k < NX; ++k) xq[b][k] = xsrc[min(tid + k * NTH, nc - 1)];
+                } else if (a.xtmp > 0) {
+                    if (!natural) continue;
+                    // column orders, the row in natural order first: its chunks go to LDS below and the copies are
+                    // gathered from there (one part per row here, so the row has at most NX * NTH chunks)
+                    const u32x4* xsrc = reinterpret_cast<const u32x4*>(xr);
+#pragma unroll
+                    for (int k = 0; k < NX; ++k) xq[b][k] = xsrc[min(tid + k * NTH, P.U - 1)];
+                } else if (gathered) {
+                    // chunk j of a row with column order m multiplies x[perm_m[8 j .. 8 j + 7]]
+#pragma unroll
+                    for (int k = 0; k < NX; ++k) {
+                        if (k > 0 && tid + k * NTH >= total) { xq[b][k] = xq[b][0]; continue; }
+                        const int32_t* pk = perms + (size_t)byte_of(ord_lo, ord_hi, it_o[k]) * P.C + (size_t)(c0 + it_c[k]) * 8;
+                        const u32x4 i0 = *reinterpret_cast<const u32x4*>(pk), i1 = *reinterpret_cast<const u32x4*>(pk + 4);
+                        const uint32_t e0 = xr[i0.x], e1 = xr[i0.y], e2 = xr[i0.z], e3 = xr[i0.w];
+                        const uint32_t e4 = xr[i1.x], e5 = xr[i1.y], e6 = xr[i1.z], e7 = xr[i1.w];
+                        xq[b][k] = u32x4{e0 | (e1 << 16), e2 | (e3 << 16), e4 | (e5 << 16), e6 | (e7 << 16)};
+                    }
+                }
+            }
+        };
+        if (PRO == 0 && !LATE) rows(true, false);
+        // Column orders through LDS: a scattered 2-byte read from memory occupies the address unit for a clock per lane
+        // (8 reads per chunk and copy: microseconds once a run has several orders), the same read from LDS costs a few
+        // clocks per wave.  The positions come from memory meanwhile.
+        u32x4 ix[NX][2];
+        auto positions = [&]() {
+            if (!via_lds) return;
+#pragma unroll
+            for (int k = 0; k < NX; ++k) {
+                const int32_t* pk = perms + (size_t)byte_of(ord_lo, ord_hi, it_o[k]) * P.C + (size_t)(c0 + it_c[k]) * 8;
+                ix[k][0] = *reinterpret_cast<const u32x4*>(pk);
+                ix[k][1] = *reinterpret_cast<const u32x4*>(pk + 4);
+            }
+        };
+        if (!LATE) positions();
+        // The codebook slice is copied global -> LDS without passing through registers (a wave instruction moves 1 KB, lane l to the
+        // wave's base + 16 l), behind the loads of four and eight rows and of a produced row: vector loads come back in order, and in
+        // front of them it held up what is worked out of the rows until all of it had arrived (a 7B layer of 4 rows
+        // 102.0 us, now 100.3, a layer of 1024 columns and 6 rows 63.1, 60.1; for fewer rows, whose loads are soon through, the slice goes first: 5120, 1024 and 1024 x 5120 with
+        // column orders 13.1 us, 13.5 the other way round).  Through a buffer: behind global_load_lds the compiler waits for every load instead of counting them
+        // (two rows: a layer is level or 1 % faster that way).
+        __builtin_amdgcn_sched_barrier(0);
+        const unsigned char* slice = reinterpret_cast<const unsigned char*>(P.table) + (size_t)s * STREAM_TAB;
+        const __amdgpu_buffer_rsrc_t table = __builtin_amdgcn_make_buffer_rsrc((void*)slice, 0, STREAM_TAB, 0x00027000);
+#pragma unroll
+        for (int k = 0; k < STREAM_TAB / (NTH * 16); ++k) {
+            if (k < kd) continue;
+            const stream_lptr_t to = (stream_lptr_t)(lds + (k * NTH + wave * 64) * 16);
+            if constexpr (NB == 2) __builtin_amdgcn_global_load_lds((stream_gptr_t)(slice + ((size_t)k * NTH + tid) * 16), to, 16, 0, 0);
+            else __builtin_amdgcn_raw_ptr_buffer_load_lds(table, to, 16, tid * 16, k * NTH * 16, 0, 0);
+        }
+        if (PRO == 0 && (LATE || (ORD && perms != nullptr))) rows(LATE, true);
+        if (LATE) positions();
+        __builtin_amdgcn_sched_barrier(0);
+        SQ_TRACE_DEP(8, "v", head_s);
+        hn = StreamHeadRaw{head_w.x, head_w.y, head_s, kcur};
+        first_steps(kcur, nx);
+        __builtin_amdgcn_sched_barrier(0);
+        if (PRO != 0) {
             float rstd = 0.f;
             if (PRO == 1) {
                 // Mean square of the whole row in the stand-alone kernel's order, so both give the same bits: slot j
@@ -400,7 +474,7 @@ __global__ __launch_bounds__(STREAM_NW * 64) void stream_kernel(StreamArgs a) {
                             for (int e = 0; e < 8; ++e) { const float vv = pro_v(a, raw[k], e); ps = __builtin_fmaf(vv, vv, ps); }
                         }
                 } else if (P.U <= NTH) {                        // one chunk per slot
-                    const ProRaw r1 = pro_fetch<1>(a, min(tid, P.U - 1));
+                    const ProRaw r1 = NX == 1 ? rown : pro_fetch<1>(a, min(tid, P.U - 1));
                     if (tid < P.U) {
 #pragma unroll
                         for (int e = 0; e < 8; ++e) { const float vv = pro_v(a, r1, e); ps = __builtin_fmaf(vv, vv, ps); }
@@ -414,7 +488,7 @@ __global__ __launch_bounds__(STREAM_NW * 64) void stream_kernel(StreamArgs a) {
                 }
                 ps = wave_sum(ps);
                 if (lane == 0) red[wave] = ps;
-                __syncthreads();
+                lds_barrier();
                 float tot = 0.f;
 #pragma unroll
                 for (int q = 0; q < NW; ++q) tot += red[q];
@@ -439,51 +513,6 @@ __global__ __launch_bounds__(STREAM_NW * 64) void stream_kernel(StreamArgs a) {
                 }
             }
         }
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            const uint16_t* xr = a.x + (int64_t)min(b, a.nb - 1) * a.ldx;
-            if (PRO != 0) {
-                // filled above
-            } else if (perms == nullptr) {
-                const u32x4* xsrc = reinterpret_cast<const u32x4*>(xr) + c0;
-#pragma unroll
-                for (int k = 0; k < NX; ++k) xq[b][k] = xsrc[min(tid + k * NTH, nc - 1)];
-            } else if (a.xtmp > 0) {
-                // column orders, the row in natural order first: its chunks go to LDS below and the copies are
-                // gathered from there (one part per row here, so the row has at most NX * NTH chunks)
-                const u32x4* xsrc = reinterpret_cast<const u32x4*>(xr);
-#pragma unroll
-                for (int k = 0; k < NX; ++k) xq[b][k] = xsrc[min(tid + k * NTH, P.U - 1)];
-            } else {
-                // chunk j of a row with column order m multiplies x[perm_m[8 j .. 8 j + 7]]
-#pragma unroll
-                for (int k = 0; k < NX; ++k) {
-                    if (k > 0 && tid + k * NTH >= total) { xq[b][k] = xq[b][0]; continue; }
-                    const int32_t* pk = perms + (size_t)byte_of(ord_lo, ord_hi, it_o[k]) * P.C + (size_t)(c0 + it_c[k]) * 8;
-                    const u32x4 i0 = *reinterpret_cast<const u32x4*>(pk), i1 = *reinterpret_cast<const u32x4*>(pk + 4);
-                    const uint32_t e0 = xr[i0.x], e1 = xr[i0.y], e2 = xr[i0.z], e3 = xr[i0.w];
-                    const uint32_t e4 = xr[i1.x], e5 = xr[i1.y], e6 = xr[i1.z], e7 = xr[i1.w];
-                    xq[b][k] = u32x4{e0 | (e1 << 16), e2 | (e3 << 16), e4 | (e5 << 16), e6 | (e7 << 16)};
-                }
-            }
-        }
-        // Column orders through LDS: a scattered 2-byte read from memory occupies the address unit for a clock per lane
-        // (8 reads per chunk and copy: microseconds once a run has several orders), the same read from LDS costs a few
-        // clocks per wave.  The positions come from memory meanwhile.
-        u32x4 ix[NX][2];
-        if (via_lds) {
-#pragma unroll
-            for (int k = 0; k < NX; ++k) {
-                const int32_t* pk = perms + (size_t)byte_of(ord_lo, ord_hi, it_o[k]) * P.C + (size_t)(c0 + it_c[k]) * 8;
-                ix[k][0] = *reinterpret_cast<const u32x4*>(pk);
-                ix[k][1] = *reinterpret_cast<const u32x4*>(pk + 4);
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        SQ_TRACE_DEP(8, "v", head_s);
-        hn = StreamHeadRaw{head_w.x, head_w.y, head_s, kcur};
-        first_steps(kcur, nx);
-        __builtin_amdgcn_sched_barrier(0);
         SQ_TRACE_DEP(9, "v", xq[0][0].x);
         if (via_lds) {
             unsigned char* tmp = a.xtmp_own ? reinterpret_cast<unsigned char*>(flag + 20) : lds;   // [NB][a.xtmp]
@@ -493,7 +522,7 @@ __global__ __launch_bounds__(STREAM_NW * 64) void stream_kernel(StreamArgs a) {
                 for (int k = 0; k < NX; ++k)
                     if (tid + k * NTH < P.U) reinterpret_cast<u32x4*>(tmp + b * a.xtmp)[tid + k * NTH] = xq[b][k];
             }
-            __syncthreads();
+            lds_barrier();
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
                 const uint16_t* xt = reinterpret_cast<const uint16_t*>(tmp + b * a.xtmp);
@@ -506,7 +535,7 @@ __global__ __launch_bounds__(STREAM_NW * 64) void stream_kernel(StreamArgs a) {
                     xq[b][k] = u32x4{e0 | (e1 << 16), e2 | (e3 << 16), e4 | (e5 << 16), e6 | (e7 << 16)};
                 }
             }
-            if (kd > 0) __syncthreads();                        // every wave has what it reads of the rows: the slice may land
+            if (kd > 0) lds_barrier();                          // every wave has what it reads of the rows: the slice may land
             const unsigned char* src = reinterpret_cast<const unsigned char*>(P.table) + (size_t)s * STREAM_TAB;
 #pragma unroll
             for (int k = 0; k < STREAM_TAB / (NTH * 16); ++k)
