@@ -228,11 +228,24 @@ static size_t mma_part_bytes(const sq_matrix& m, int B) {
 // of such a row need, they still do, on the vector kernels.
 static bool mma_without_room(const sq_matrix& m, int B) { return !whole_units(m) && mma_plan(m, B).ks > 1 && !mma_whole_row(m, B).KW; }
 
+// How many pieces, the first one on, run on the kernel of sq_sieve.hip: none that has tag streams for these rows
+static int sieve_len(const sq_matrix* mats, int n, int B) {
+    int k = 0;
+    while (k < n && mma_rows(mats[k]) && !stream_rows(mats[k], B)) ++k;
+    return sieve_group(mats, k, B);
+}
+
 // tight: the pieces that can run without partial sums do
-static size_t small_need(const sq_matrix* mats, int n, int B, bool tight) {
+// (a group that sq_sieve.hip takes runs there unless the workspace is tight or x not aligned: then piece by piece as below)
+static size_t small_need(const sq_matrix* mats, int n, int B, bool tight, bool sieve = true) {
     size_t tot = 0;
     for (int i = 0; i < n; ++i) {
         if (stream_rows(mats[i], B)) continue;                   // its partial sums live in the workspace header
+        if (const int k = tight || !sieve ? 0 : sieve_len(mats + i, n - i, B); k > 0) {
+            tot += std::max(sieve_workspace(mats + i, k, B), small_need(mats + i, k, B, false, false));
+            i += k - 1;
+            continue;
+        }
         if (mma_rows(mats[i])) tot += tight && (mma_whole_row(mats[i], B).KW || mma_without_room(mats[i], B)) ? 0 : mma_part_bytes(mats[i], B);
         else if (mats[i].perms && fast_shape(mats[i])) tot += xp_bytes(mats[i], B);
     }
@@ -410,6 +423,12 @@ int launch_small(const sq_matrix* mats, int n, const void* x, int x_dtype, int64
             int rc = launch_stream_group(mats + i, j - i, x, x_dtype, ldx, y, y_dtype, ldy, B, (char*)sums, s, from);
             if (rc) return rc;
             i = j;
+            continue;
+        }
+        if (const int k = tight || !x_ok ? 0 : sieve_len(mats + i, n - i, B); k > 0) {
+            if (const int rc = launch_sieve(mats + i, k, x, x_dtype, ldx, y, y_dtype, ldy, B, (char*)ws + ws_off, s)) return rc;
+            ws_off += std::max(sieve_workspace(mats + i, k, B), small_need(mats + i, k, B, false, false));       // (what was counted for them)
+            i += k;
             continue;
         }
         if (B <= 2 && x_ok && segs_shape(m0) && (B == 1 || mma_table_bytes(m0) > 64 * 1024)) {
