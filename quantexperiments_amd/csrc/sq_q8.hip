@@ -197,7 +197,10 @@ __global__ __launch_bounds__(256, 2) void q8_gemv_kernel(Q8Args a) {
 // LDS, where the workgroup keeps the current 256-column chunk of the fp16 activations (global_load_lds, double
 // buffered, one barrier per chunk).  The block scale is folded into the fp16 weight (one rounding, as the
 // reference's tile kernel does, shapequant/kernels/batched_runs.py:442-447): all 16 weights of a piece sit in one
-// block.  A first form loaded the operand layout straight from memory (lane = row, 16 bytes per lane): every
+// block.  What bounds a pass: HBM up to 32 rows of a large head; beyond that, and in small heads, LDS reads (18 KB of fragments per tile and
+// step at 64 rows, an eighth of them weights), conversions and matrix instructions of the waves of a CU, which barely overlap (64 rows of 8,000 x
+// 3,584: 29 us, without the products 27, without what is in LDS read at all 18; two tiles of weights per fragment of x 44, each fragment read
+// a step's start ahead 32).  A first form loaded the operand layout straight from memory (lane = row, 16 bytes per lane): every
 // quarter wave then touches 16 different cache lines, and it stayed at 4.1-4.4 TB/s where this one reaches
 // 5.2-5.5 TB/s (the one-row kernel: 5.7); 32 rows per wave on the 32x32x16 instruction was slower still.
 constexpr int Q8_MFMA_MAX_ROWS = 320;           // up to here passes of 64 beat decode + tile GEMM (152,064 x 3,584: 151 us per pass,
@@ -217,11 +220,12 @@ __global__ __launch_bounds__(256) void q8_x_kernel(const uint16_t* __restrict__ 
 struct Q8MfmaArgs {
     const int8_t* q;
     const uint16_t* sc;
-    const uint16_t* xh;     // fp16 [B, ldxh], rows 16-byte aligned
+    const uint16_t* xh;     // fp16, or bf16 where the kernel converts it, [B, ldxh], rows 16-byte aligned
     void* y;
     int64_t ldy;
     int ldxh;
     int V, C, B, y_dtype, tasks;
+    int groups;             // groups of 16 NBLK tokens, each in workgroups of its own
     int vec_y;              // y rows allow 8-byte stores of 16-bit results (y 8-byte aligned, ldy % 4 == 0)
 };
 
@@ -242,9 +246,29 @@ constexpr int q8l_lds_bytes(int nblk, int waves, int d, int xs, int rows) { retu
 // the 32 columns of one block (lane group g: columns 8 g .. 8 g + 7) and its sums, fp32, are multiplied by the block's scales.
 // Scales come in 4-byte pairs; every other row of an odd number of blocks begins within one, so there each comes by itself (a 2-byte copy per
 // lane, which leaves them 4 bytes apart; twice the copies).
-template <int NBLK, int WAVES, int D, int XS, int ROWS>
+// CVT: x is bf16 and becomes fp16 on its way into LDS: its pieces are loaded into registers where they would be copied, converted and written
+// behind the last product of the chunk (a launch that converted x first took 3 us of an eager call, 5 of the product's time on the device).
+// The load is written out, and waited for by count like the copies beside it: the compiler would wait for all of those.  Its registers are
+// named, above all that a kernel needs (106), since a compiler moves values that it believes to be there already.
+template <int I> using int_c = std::integral_constant<int, I>;
+constexpr int Q8_XR = 112;                      // 4 of them a piece
+template <int I>
+__device__ __forceinline__ void q8_x_load(const uint16_t* src) {
+    asm volatile("global_load_dwordx4 v[%1:%2], %0, off" ::"v"(src), "n"(Q8_XR + 4 * I), "n"(Q8_XR + 4 * I + 3)
+                 : "memory", "v112", "v113", "v114", "v115", "v116", "v117", "v118", "v119", "v120", "v121", "v122", "v123", "v124", "v125", "v126", "v127");
+}
+template <int I, int NEWER>                     // piece I, once all but the wave's NEWER last operations are done
+__device__ __forceinline__ u32x4 q8_x_take() {
+    uint32_t v[4];
+    asm volatile("s_waitcnt vmcnt(%4)\n\tv_mov_b32 %0, v[%5]\n\tv_mov_b32 %1, v[%6]\n\tv_mov_b32 %2, v[%7]\n\tv_mov_b32 %3, v[%8]"
+                 : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3])
+                 : "n"(NEWER), "n"(Q8_XR + 4 * I), "n"(Q8_XR + 4 * I + 1), "n"(Q8_XR + 4 * I + 2), "n"(Q8_XR + 4 * I + 3) : "memory");
+    return u32x4{v[0], v[1], v[2], v[3]};
+}
+constexpr int q8l_x_copies(int nblk, int waves, int xs) { return 4 * nblk * xs > waves ? 4 * nblk * xs / waves : 1; }
+template <int NBLK, int WAVES, int D, int XS, int ROWS, bool CVT, int XI = q8l_x_copies(NBLK, WAVES, XS)>
 __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel(Q8MfmaArgs a) {
-    static_assert((D == 3 || D == 4) && (XS == 2 || (XS == 1 && D == 3)), "wait counts below are written out for these");
+    static_assert((D == 3 || (D == 4 && !CVT)) && (XS == 2 || (XS == 1 && D == 3)) && XI <= 4, "wait counts below are written out for these");
     constexpr bool ANY_C = ROWS != Q8_CHUNKS;
     constexpr int Q8L_D = D, Q8L_WAVE_BYTES = q8l_wave_bytes(D, ROWS), SB = q8l_scale_bytes(ROWS), SC = SB / 256;      // SC: copies of a chunk's scales
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -253,7 +277,12 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     unsigned char* wl = smem + 2 * XBUF + wave * Q8L_WAVE_BYTES;  // this wave's ring
     unsigned char* sl_ = wl + Q8L_D * 2048;                        // this wave's scales: [D - 1][16 rows][SB / 16 bytes]
-    const int task_raw = blockIdx.x * WAVES + wave;
+    // the workgroups of the same weights are 8 apart: on one die, whose L2 the second finds them in
+    const int tgroup = (blockIdx.x >> 3) % a.groups;
+    const int task_raw = (int)((blockIdx.x >> 3) / a.groups * 8 + (blockIdx.x & 7)) * (int)(blockDim.x >> 6) + wave;
+    if (task_raw - wave >= a.tasks) return;                     // (all waves of the workgroup)
+    const uint16_t* xh = a.xh + (int64_t)tgroup * (NBLK * 16) * a.ldxh;
+    const int nrows = min(a.B - tgroup * (NBLK * 16), NBLK * 16);
     const bool active = task_raw < a.tasks;
     const int task = active ? task_raw : a.tasks - 1;
     const int r = lane & 15, g = lane >> 4;
@@ -264,7 +293,6 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel
     // activations: one copy instruction moves 1 KB = 4 / XS tokens of a chunk; the 16-byte piece p of token t is kept
     // at slot p ^ (t % 16), so the 16 lanes of a read clock (16 tokens, one piece) spread over 16 bank groups
     constexpr int TPI = 4 / XS, LPT = 64 / TPI;                 // tokens per instruction, lanes (= pieces) per token
-    constexpr int XI = 16 * NBLK / TPI > WAVES ? 16 * NBLK / TPI / WAVES : 1;     // copies a wave makes of a chunk
     uint32_t xsrc[XI];
     int xcol[XI];                                               // this lane's column in a chunk
 #pragma unroll
@@ -272,16 +300,33 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel
         const int rowx = (wave * XI + i) * TPI + lane / LPT;
         const int piece = (lane % LPT) ^ (rowx & 15);
         xcol[i] = piece * 8;
-        xsrc[i] = (uint32_t)(min(rowx, a.B - 1) * a.ldxh + (ANY_C ? 0 : xcol[i]));
+        xsrc[i] = (uint32_t)(min(rowx, nrows - 1) * a.ldxh + (ANY_C ? 0 : xcol[i]));
     }
     const bool xo = wave * XI * TPI < 16 * NBLK;                // this wave takes part in the x copies
-    auto copy_x = [&](int c) {
-        if (xo)
-#pragma unroll
-            for (int i = 0; i < XI; ++i) {
+    auto copy_x = [&](int c) __attribute__((always_inline)) {
+        if (!xo) return;
+        auto piece = [&](auto i_) __attribute__((always_inline)) {
+            constexpr int i = decltype(i_)::value;
+            if constexpr (i < XI) {
                 const uint32_t at = ANY_C ? (uint32_t)min(c * (XS * 128) + xcol[i], C - 8) : (uint32_t)(c * (XS * 128));
-                __builtin_amdgcn_global_load_lds((gptr_t)(a.xh + at + xsrc[i]), (lptr_t)(xs + (c & 1) * XBUF + (wave * XI + i) * TPI * XPITCH), 16, 0, 0);
+                const uint16_t* src = xh + at + xsrc[i];
+                if constexpr (CVT) q8_x_load<i>(src);
+                else __builtin_amdgcn_global_load_lds((gptr_t)src, (lptr_t)(xs + (c & 1) * XBUF + (wave * XI + i) * TPI * XPITCH), 16, 0, 0);
             }
+        };
+        piece(int_c<0>()); piece(int_c<1>()); piece(int_c<2>()); piece(int_c<3>());
+    };
+    // CVT: chunk c, once all but the wave's `newer` last operations are done
+    auto put_x = [&](int c, auto newer) __attribute__((always_inline)) {
+        if (!xo) return;
+        auto piece = [&](auto i_) __attribute__((always_inline)) {
+            constexpr int i = decltype(i_)::value;
+            if constexpr (i < XI) {
+                const u32x4 v = q8_x_take<i, decltype(newer)::value>();
+                *reinterpret_cast<u32x4*>(xs + (c & 1) * XBUF + (wave * XI + i) * TPI * XPITCH + lane * 16) = u32x4{bf2h_x2(v.x), bf2h_x2(v.y), bf2h_x2(v.z), bf2h_x2(v.w)};
+            }
+        };
+        piece(int_c<0>()); piece(int_c<1>()); piece(int_c<2>()); piece(int_c<3>());
     };
     // weights: instruction n of a step fills rows 8 n .. 8 n + 7; lane i lands in row 8 n + i / 8, slot i % 8 and
     // fetches the piece the swizzle keeps there
@@ -336,19 +381,36 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel
     copy_x(0);
 #pragma unroll
     for (int t = 0; t < D - 1; ++t) refill(t);
-    for (int s = 0; s < nsteps; ++s) {
-        const int c = s >> 1, odd = s & 1, cx = s / XS;         // chunk of scales, step in it, chunk of x
+    if constexpr (CVT) put_x(0, int_c<4 + SC>());
+    // CVT: x of the next chunk, before the barrier that opens it.  Behind its load: the refills of the chunk's steps
+    auto next_x = [&](int s) __attribute__((always_inline)) {
+        if constexpr (CVT) {
+            const int cx = s / XS, f = s + D - 1;               // (f: the step that this one's refill was for)
+            if ((XS == 2 && !(s & 1)) || cx + 1 >= nchunks) return;
+            if (f >= nsteps) put_x(cx + 1, int_c<0>());
+            else if (XS == 2) put_x(cx + 1, int_c<4 + SC>());
+            else if (f & 1) put_x(cx + 1, int_c<2>());
+            else put_x(cx + 1, int_c<2 + SC>());
+        }
+    };
+    // (the wait before a barrier, also for this wave's writes to LDS where there are any)
+    auto ready = [&](auto newer) __attribute__((always_inline)) {
+        if constexpr (CVT) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(q8_vmcnt(decltype(newer)::value));
+    };
+    auto step = [&](int s, auto odd) __attribute__((always_inline)) {
+        const int c = s >> 1, cx = s / XS;         // chunk of scales, step in it, chunk of x
         if (XS == 1) {
             // every step opens an x chunk: X(s) was issued one step ago, before [S] W(s + 1)
-            if (s + 1 < nsteps) { if (odd) __builtin_amdgcn_s_waitcnt(q8_vmcnt(2 + SC)); else __builtin_amdgcn_s_waitcnt(q8_vmcnt(2)); }
-            else __builtin_amdgcn_s_waitcnt(q8_vmcnt(0));
+            if (s + 1 < nsteps) { if (odd) ready(int_c<2 + SC>()); else ready(int_c<2>()); }
+            else ready(int_c<0>());
             __builtin_amdgcn_s_barrier();
             __builtin_amdgcn_sched_barrier(0);
             if (cx + 1 < nchunks) copy_x(cx + 1);
             refill(s + D - 1);
         } else if (!odd) {
-            if (s + D - 2 < nsteps) __builtin_amdgcn_s_waitcnt(q8_vmcnt(D == 3 ? 2 : 4 + SC));
-            else __builtin_amdgcn_s_waitcnt(q8_vmcnt(0));
+            if (s + D - 2 < nsteps) ready(int_c<D == 3 ? 2 : 4 + SC>());
+            else ready(int_c<0>());
             __builtin_amdgcn_s_barrier();
             __builtin_amdgcn_sched_barrier(0);
             if (cx + 1 < nchunks) copy_x(cx + 1);
@@ -394,7 +456,8 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
-            continue;
+            next_x(s);
+            return;
         }
         const u32x4 wq[2] = {*reinterpret_cast<const u32x4*>(st + w0), *reinterpret_cast<const u32x4*>(st + w1)};
         const half_t sh = __builtin_bit_cast(half_t, *reinterpret_cast<const uint16_t*>(sl_ + (c % (D - 1)) * SB + r * 16 + odd * 8 + g * 2));
@@ -424,13 +487,24 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel
             }
         }
         __builtin_amdgcn_sched_barrier(0);
+        next_x(s);
+    };
+    // Pairs of steps, each compiled for its place: us, step by step / so, 24 rows of 20,000 x 3,584 27.0 / 24.5, 64 of 8,000 x 3,584 23.3 / 21.4, 16 of
+    // 152,064 x 3,584 112.5 / 111.2; but 24 and 32 rows of fp16 of the last 117.5 and 120.4 / 119.2 and 122.7
+    if constexpr (!CVT && NBLK == 2 && WAVES == 8 && !ANY_C) {
+        for (int s = 0; s < nsteps; ++s) step(s, s & 1);
+    } else {
+        for (int s = 0; s < nsteps; s += 2) {
+            step(s, int_c<0>());
+            step(s + 1, int_c<1>());
+        }
     }
     if (!active) return;
     const int orow = task * 16 + g * 4;
 #pragma unroll
     for (int nb = 0; nb < NBLK; ++nb) {
-        const int tok = nb * 16 + r;
-        if (tok >= a.B) continue;
+        if (nb * 16 + r >= nrows) continue;
+        const int tok = tgroup * (NBLK * 16) + nb * 16 + r;
         if (a.vec_y && a.y_dtype != SQ_F32 && orow + 4 <= a.V) {
             uint16_t o[4];
 #pragma unroll
@@ -559,12 +633,16 @@ int launch_q8_mid(const int8_t* q, const uint16_t* sc, int V, int C, const void*
                   int y_dtype, int64_t ldy, int B, void* ws, size_t ws_bytes, hipStream_t s) {
     if (ws_bytes < q8_mid_workspace(V, C, B)) return fail(SQ_EWORKSPACE, "sq_q8_linear: workspace %zu < %zu", ws_bytes, q8_mid_workspace(V, C, B));
     const size_t ys = y_dtype == SQ_F32 ? 4 : 2;
-    // fp16 activations with 16-byte aligned rows are copied to LDS from where they are; anything else goes through
-    // an fp16 copy in the workspace first
+    // Activations with 16-byte aligned rows go to LDS from where they are, anything else goes through an fp16 copy in the workspace first; bf16 too
+    // where many rows (> 32) make the conversion in the kernel, 0.17 us per step of 128 columns and round of workgroups, longer than the launch.
+    // us per eager call, copy / converted in the kernel: 4 rows of 8,000 x 1,024 16.7 / 14.5, of 32,000 x 3,584 24.2 / 22.1, 16 of 64,000 x 2,048 27.1 /
+    // 25.0, of 152,064 x 3,584 111.9 / 109.7; 64 of 32,000 x 1,024 16.8 / 14.6, of 8,000 x 3,584 20.4 / 23.3, of 152,064 x 3,584 151 / 160.
     const uint16_t* xh = (const uint16_t*)x;
     int64_t ldxh = ldx;
+    const int cus = device_cus(), tasks = (V + 15) / 16, n4 = (tasks + 3) / 4, n8 = (tasks + 7) / 8, n16 = (tasks + 15) / 16;
+    bool cvt = x_dtype == SQ_BF16 && (B <= 32 || (n8 <= cus && C <= 1920));
     int rc;
-    if (x_dtype != SQ_F16 || ((uintptr_t)x & 15) || ldx % 8 || ldx * 64 >= ((int64_t)1 << 31)) {
+    if ((x_dtype != SQ_F16 && !cvt) || ((uintptr_t)x & 15) || ldx % 8 || ldx * 64 >= ((int64_t)1 << 31)) {
         const int64_t n = (int64_t)B * C;
         const int64_t want = (n + 255) / 256;
         hipLaunchKernelGGL(q8_x_kernel, dim3((unsigned)(want < 4096 ? want : 4096)), dim3(256), 0, s, (const uint16_t*)x, ldx, B,
@@ -573,8 +651,8 @@ int launch_q8_mid(const int8_t* q, const uint16_t* sc, int V, int C, const void*
         if (rc) return rc;
         xh = (const uint16_t*)ws;
         ldxh = C;
+        cvt = false;
     }
-    const int tasks = (V + 15) / 16;
     for (int b0 = 0; b0 < B;) {
         const int pass = B - b0 > 32 ? 64 : 32;                  // activation rows of this pass at most
         Q8MfmaArgs a{};
@@ -588,42 +666,59 @@ int launch_q8_mid(const int8_t* q, const uint16_t* sc, int V, int C, const void*
         // round of the chip badly; then 8 waves with 128-column chunks (a barrier per step, two workgroups per CU).
         // Measured: 152,064 x 3,584 (594 workgroups of 16 waves, 2.3 rounds) 126 against 116 us; 248,320 x 5,120
         // (970, 3.8 rounds) 265 against 278 us.
-        const int cus = device_cus(), n16 = (tasks + 15) / 16;
         const bool x128 = (double)n16 / ((double)((n16 + cus - 1) / cus) * cus) < 0.85;
         const int rows = C % 256 == 0 ? Q8_CHUNKS : C % 64 == 0 ? Q8_PAIRS : Q8_ODD;
+        a.groups = 1;
         auto go = [&](auto chunks, auto pairs, auto odd, int nblk, int waves, int xs) {
-            hipLaunchKernelGGL(rows == Q8_CHUNKS ? chunks : rows == Q8_PAIRS ? pairs : odd, dim3((unsigned)((tasks + waves - 1) / waves)), dim3((unsigned)waves * 64),
-                               q8l_lds_bytes(nblk, waves, 3, xs, rows), s, a);
+            const int wgs = (tasks + waves - 1) / waves;
+            hipLaunchKernelGGL(rows == Q8_CHUNKS ? chunks : rows == Q8_PAIRS ? pairs : odd, dim3((unsigned)(a.groups > 1 ? (wgs + 7) / 8 * 8 * a.groups : wgs)),
+                               dim3((unsigned)waves * 64), q8l_lds_bytes(nblk, waves, 3, xs, rows), s, a);
         };
         static bool raised = false;
         if (!raised) {
             auto raise = [](auto... k) { ((void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024), ...); };
-#define SQ_Q8(N, W, D, X) q8_mfma_kernel<N, W, D, X, Q8_CHUNKS>, q8_mfma_kernel<N, W, D, X, Q8_PAIRS>, q8_mfma_kernel<N, W, D, X, Q8_ODD>
-            raise(SQ_Q8(1, 8, 3, 2), SQ_Q8(2, 16, 3, 2), SQ_Q8(2, 8, 3, 1), SQ_Q8(4, 16, 3, 1), SQ_Q8(4, 8, 3, 1));
+#define SQ_Q8C(CV, N, W, D, X, ...) q8_mfma_kernel<N, W, D, X, Q8_CHUNKS, CV, ##__VA_ARGS__>, q8_mfma_kernel<N, W, D, X, Q8_PAIRS, CV, ##__VA_ARGS__>, q8_mfma_kernel<N, W, D, X, Q8_ODD, CV, ##__VA_ARGS__>
+#define SQ_Q8(...) SQ_Q8C(false, __VA_ARGS__), SQ_Q8C(true, __VA_ARGS__)
+            raise(SQ_Q8(1, 8, 3, 2), SQ_Q8(2, 16, 3, 2), SQ_Q8(2, 8, 3, 1), SQ_Q8(4, 16, 3, 1), SQ_Q8(4, 8, 3, 1), SQ_Q8(4, 8, 3, 1, 4));
+#undef SQ_Q8
             (void)hipGetLastError();
             raised = true;
         }
-        // Small heads: half the waves per workgroup, each making twice the copies of x, spread the same waves over twice the CUs (a wave's
-        // chain of LDS reads, conversions and matrix instructions is what they take).  us, before / so: 16 rows of 9,728 x 3,584 19.7 /
+#define SQ_GO(N, W, X, WAVES, ...) do { if (cvt) go(SQ_Q8C(true, N, W, 3, X, ##__VA_ARGS__), N, WAVES, X); else go(SQ_Q8C(false, N, W, 3, X, ##__VA_ARGS__), N, WAVES, X); } while (0)
+        // Small heads: half the waves per workgroup, each making twice the copies of x, spread the same waves over twice the CUs (LDS reads,
+        // conversions and matrix instructions are what they take).  us, before / so: 16 rows of 9,728 x 3,584 19.7 /
         // 17.8, of 10,000 x 2,048 12.7 / 12.1, of 30,000 x 2,048 14.3 / 14.8; 64 rows of 9,728 x 3,584 44.7 / 30.5, of 32,000 x 3,584 45.9 / 31.9,
-        // of 60,000 x 2,048 31.0 / 37.4.
-        const int n8 = (tasks + 7) / 8;
+        // of 60,000 x 2,048 31.0 / 37.4.  Where the weights' tiles still leave half of the CUs idle, groups of tokens take workgroups of their
+        // own: 64 rows of 8,000 x 3,584 29.4 / 18.5, of 16,000 x 3,456 37.5 / 25.8 (of 20,000 x 3,584, more than half, 29.3 / 31.4), 24 of 8,000 x 3,584
+        // 20.0 / 17.9, of 16,000 x 3,456 27.9 / 23.5.
+        // 33-64 rows of larger heads: two workgroups of 7 waves to a CU where those of 16 fill the last round badly (64 rows of 152,064 x 896 52.7 / 44.7,
+        // of 152,064 x 3,584 151.8 / 150.4, of 100,000 x 2,048 55.7 / 50.8, of 40,000 x 3,584 45.7 / 39.9; of 64,000 x 2,048, one round, 33.9 / 41.6); with
+        // the scales of an odd number of blocks two do not fit (152,064 x 1,056 69 / 79).
         const bool small = a.B > 32 ? n8 <= cus : n8 <= cus / 2;
-        if (small && a.B > 32)
-            go(SQ_Q8(4, 8, 3, 1), 4, 8, 1);
-        else if (small && a.B > 16)
-            go(SQ_Q8(2, 4, 3, 1), 2, 4, 1);
-        else if (small)
-            go(SQ_Q8(1, 4, 3, 2), 1, 4, 2);
-        else if (a.B > 32)                                           // 33-64 rows: 16 waves share 128-column chunks of 64 tokens
-            go(SQ_Q8(4, 16, 3, 1), 4, 16, 1);
-        else if (a.B > 16 && x128)
-            go(SQ_Q8(2, 8, 3, 1), 2, 8, 1);
-        else if (a.B > 16)
-            go(SQ_Q8(2, 16, 3, 2), 2, 16, 2);
-        else
-            go(SQ_Q8(1, 8, 3, 2), 1, 8, 2);
-#undef SQ_Q8
+        if (small && a.B > 32 && 2 * n4 <= cus) {
+            a.groups = 2;
+            SQ_GO(2, 4, 1, 4);
+        } else if (small && a.B > 32 && 2 * n8 <= cus) {
+            a.groups = 2;
+            SQ_GO(2, 8, 1, 8);
+        } else if (small && a.B > 32) {
+            SQ_GO(4, 8, 1, 8);
+        } else if (small) {
+            a.groups = a.B > 16 ? 2 : 1;
+            SQ_GO(1, 4, 2, 4);
+        } else if (a.B > 32 && x128 && rows != Q8_ODD) {
+            SQ_GO(4, 8, 1, 7, 4);
+        } else if (a.B > 32) {                                       // 33-64 rows: 16 waves share 128-column chunks of 64 tokens
+            SQ_GO(4, 16, 1, 16);
+        } else if (a.B > 16 && x128) {
+            SQ_GO(2, 8, 1, 8);
+        } else if (a.B > 16) {
+            SQ_GO(2, 16, 2, 16);
+        } else {
+            SQ_GO(1, 8, 2, 8);
+        }
+#undef SQ_GO
+#undef SQ_Q8C
         rc = check_launch("q8_mfma_kernel");
         if (rc) return rc;
         b0 += a.B;

@@ -233,3 +233,37 @@ def test_tile_gemm_accumulators_and_stores(tmp_path):
             assert sum(l.startswith("global_store_dwordx4") for l in lines) == 32 * mt
         variants += 1
     assert variants == 9
+
+
+def test_head_conversion_leaves_loads_alone(tmp_path):
+    """The head kernels that convert their activations load them in an asm statement and wait for them, by count, in another: nothing
+    the compiler puts anywhere may read or write the registers that these name."""
+    import os
+    import subprocess
+    from quantexperiments_amd import build
+    try:
+        hipcc = build._hipcc()
+    except RuntimeError:
+        pytest.skip("no hipcc")
+    out = tmp_path / "q8.s"
+    subprocess.run([hipcc, *build.FLAGS, "-S", "--offload-device-only", str(build.CSRC / "sq_q8.hip"), "-o", str(out)], check=True,
+                   capture_output=True, env=dict(os.environ, TMPDIR=str(tmp_path)))
+    variants = 0
+    for body in re.split(r"(?m)^(?=_ZN2sq14q8_mfma_kernel\w+:)", out.read_text())[1:]:
+        if "Lb1E" not in body.split(":", 1)[0]:
+            continue
+        asm, loads, takes = False, 0, 0
+        for l in body[:body.index(".Lfunc_end")].splitlines():
+            asm = True if "#ASMSTART" in l else False if "#ASMEND" in l else asm
+            l = l.split(";")[0].strip()
+            if not l or l.startswith(".") or l.endswith(":"):
+                continue
+            used = {r for m in re.finditer(r"\bv(?:\[(\w+)(?::(\w+))?\]|(\d+)\b)", l) for r in range(int(m[1] or m[3], 0), int(m[2] or m[1] or m[3], 0) + 1)}
+            if asm and used & set(range(112, 128)):
+                assert l.startswith(("global_load_dwordx4 v[", "v_mov_b32")), l
+                loads, takes = loads + l.startswith("global"), takes + l.startswith("v_mov")
+            else:
+                assert not used & set(range(112, 128)) and not l.startswith("scratch_"), l
+        assert loads and takes >= 4 * loads
+        variants += 1
+    assert variants == 24

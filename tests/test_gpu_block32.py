@@ -365,3 +365,24 @@ def test_q8_rows_of_an_odd_number_of_blocks(V, C, dtype):
         exact = B <= 32 or V >= 30000 or (1024 <= V and B <= 64 and (V >= 8000 or C <= 2048))
         assert rel_max_err(y[:, :V].cpu().numpy(), O.q8_linear(x.half().float().cpu().numpy(), q, sc)) < (1e-5 if exact else 2.0 ** -11), B
         assert bool((y[:, V:] == 5.0).all())
+
+
+@pytest.mark.parametrize("V,C", [(2100, 256), (8180, 512), (8200, 320), (16380, 96), (16400, 256), (33000, 768), (40007, 64), (40007, 160), (65540, 256)])
+def test_q8_workgroups_and_conversions(V, C):
+    """Every way the matrix-core passes are cut: groups of tokens in workgroups of their own (heads of up to 128 and 256 workgroups of
+    four and eight waves), seven waves where sixteen fill the last round badly, and around their lines.  bf16 rows that the kernel
+    converts, rows it takes from a copy (2 bytes off, which more than 32 rows of broken chunks may not be) and fp16 rows hold the same fp16 values and meet the same products in the same order:
+    the same bits.  Bounds as above: one rounding of a weight at 2^-11 where the scale is folded into it."""
+    from quantexperiments_amd.kernels import q8_linear
+    q, sc, deq = _q8_parts(V, C, seed=V + C)
+    tq, ts, w = torch.from_numpy(q).cuda(), torch.from_numpy(sc).cuda(), torch.from_numpy(np.ascontiguousarray(deq)).cuda().double()
+    for B in (3, 16, 17, 31, 33, 47, 49, 64):
+        x = rand_x(B, C + 8, torch.bfloat16, seed=B).cuda()
+        off = x if B > 32 and C % 256 else torch.zeros(B * (C + 8) + 1, dtype=torch.bfloat16, device="cuda")[1:].view(B, C + 8).copy_(x)
+        ys = [torch.full((B, V + 2), 5.0, device="cuda") for _ in range(3)]
+        for y, xi in zip(ys, (x, off, x.half())):
+            assert (xi.data_ptr() % 16 == 0) == (xi is not off or off is x)
+            q8_linear(tq, ts, xi[:, :C], y[:, :V])
+        assert torch.equal(ys[0], ys[1]) and torch.equal(ys[0], ys[2]) and bool((ys[0][:, V:] == 5.0).all()), B
+        ref = x[:, :C].double() @ w.T
+        assert float((ys[0][:, :V].double() - ref).abs().max() / ref.abs().max()) < 2.0 ** -11, B
