@@ -566,34 +566,26 @@ __global__ __launch_bounds__(256) void q8_dequant_kernel(const int8_t* __restric
     }
 }
 
-// Embedding rows: one 16-byte load (32 weights, one block) per thread.  Ids outside [0, V) give a row of zeros.
-template <int DT>
+// Embedding rows: 8 weights and one 16-byte store per thread, so a wave stores whole lines one after another (a block of 32 weights per thread left 64
+// bytes between the lanes' stores and a quarter of the waves: 2,048 rows of 3,584 columns, 14.7 MB of results, 9.0 us, 6.9 so; with a head of
+// 16 rows of 152,064 x 3,584 120.3 / 118.2 us).  Numbers of pieces are 32-bit where they fit: a division for each.  Ids outside [0, V) give a row of zeros.
+template <int DT, class I>
 __global__ __launch_bounds__(256) void q4_embed_kernel(const uint8_t* __restrict__ q, const uint16_t* __restrict__ sc,
-                                                       int V, int C, const int64_t* __restrict__ ids, int64_t n_ids,
+                                                       int V, int C, const int64_t* __restrict__ ids, I total,
                                                        typename store_as<DT>::type* __restrict__ out, int64_t ld_out, int vec) {
-    typedef typename store_as<DT>::type T;
-    const int nblk = C >> 5;
-    const int64_t total = n_ids * nblk;
-    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < total; t += (int64_t)gridDim.x * 256) {
-        const int64_t i = t / nblk;
-        const int b = (int)(t - i * nblk);
+    const int nblk = C >> 5, pieces = C >> 3;
+    for (I t = (I)blockIdx.x * 256 + threadIdx.x; t < total; t += (I)gridDim.x * 256) {
+        const I i = t / pieces;
+        const int p = (int)(t - i * pieces);
         const int64_t id = ids[i];
-        T* dst = out + i * ld_out + b * 32;
-        float o[32];
-        if (id < 0 || id >= V) {
+        float o[8] = {};
+        if (id >= 0 && id < V) {
+            const uint32_t w = *reinterpret_cast<const uint32_t*>(q + id * (C >> 1) + p * 4);
+            const float s = h2f(sc[id * nblk + (p >> 2)]);
 #pragma unroll
-            for (int k = 0; k < 32; ++k) o[k] = 0.f;
-        } else {
-            const u32x4 v = *reinterpret_cast<const u32x4*>(q + id * (C >> 1) + b * 16);
-            const float s = h2f(sc[id * nblk + b]);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const uint32_t w = v[k];
-#pragma unroll
-                for (int e = 0; e < 8; ++e) o[8 * k + e] = (float)((int)((w >> (4 * e)) & 15u) - 8) * s;
-            }
+            for (int e = 0; e < 8; ++e) o[e] = (float)((int)((w >> (4 * e)) & 15u) - 8) * s;
         }
-        store_run<DT, 32>(dst, o, vec != 0);
+        store_run<DT, 8>(out + (int64_t)i * ld_out + p * 8, o, vec != 0);
     }
 }
 
@@ -774,18 +766,20 @@ int launch_q8_dequant(const int8_t* q, const uint16_t* sc, int C, void* out, int
 
 int launch_q4_embed(const uint8_t* q, const uint16_t* sc, int V, int C, const int64_t* ids, int64_t n_ids, void* out,
                     int out_dtype, int64_t ld_out, hipStream_t s) {
-    const int64_t total = n_ids * (C >> 5);
+    const int64_t total = n_ids * (C >> 3);
     if (total == 0) return SQ_OK;
     const int64_t want = (total + 255) / 256;
     const unsigned grid = (unsigned)(want < 65536 ? want : 65536);
     const int64_t per16 = out_dtype == SQ_F32 ? 4 : 8;
     const int vec = ((uintptr_t)out & 15) == 0 && ld_out % per16 == 0;
-    if (out_dtype == SQ_F32)
-        hipLaunchKernelGGL(q4_embed_kernel<SQ_F32>, dim3(grid), dim3(256), 0, s, q, sc, V, C, ids, n_ids, (float*)out, ld_out, vec);
-    else if (out_dtype == SQ_F16)
-        hipLaunchKernelGGL(q4_embed_kernel<SQ_F16>, dim3(grid), dim3(256), 0, s, q, sc, V, C, ids, n_ids, (uint16_t*)out, ld_out, vec);
-    else
-        hipLaunchKernelGGL(q4_embed_kernel<SQ_BF16>, dim3(grid), dim3(256), 0, s, q, sc, V, C, ids, n_ids, (uint16_t*)out, ld_out, vec);
+#define SQ_GO(DT) do { \
+        if (total < ((int64_t)1 << 31)) hipLaunchKernelGGL((q4_embed_kernel<DT, uint32_t>), dim3(grid), dim3(256), 0, s, q, sc, V, C, ids, (uint32_t)total, (store_as<DT>::type*)out, ld_out, vec); \
+        else hipLaunchKernelGGL((q4_embed_kernel<DT, int64_t>), dim3(grid), dim3(256), 0, s, q, sc, V, C, ids, total, (store_as<DT>::type*)out, ld_out, vec); \
+    } while (0)
+    if (out_dtype == SQ_F32) SQ_GO(SQ_F32);
+    else if (out_dtype == SQ_F16) SQ_GO(SQ_F16);
+    else SQ_GO(SQ_BF16);
+#undef SQ_GO
     return check_launch("q4_embed_kernel");
 }
 
