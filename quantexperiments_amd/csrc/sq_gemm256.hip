@@ -450,6 +450,242 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a)
 
 #undef SQ_INLINE
 
+constexpr int G_EP_PITCH = 128 * 2 + 16;     // bytes per token row of a wave's 32 MT x 128 output tile in LDS
+
+// The product of at most a tile (or a part of one) per workgroup: what a workgroup needs to go from tile to tile, products that know about events,
+// accumulators it names, addresses in front of every tile, is longer than the slabs of a small product.  us, the kernel above / this one:
+// 264 x 576 x 576 16.0 / 12.4, x 2176 20.0 / 18.9, 264 x 4352 x 576 14.5 / 13.5, 1024 x 7168 x 5120 level; of two rounds and more the one above is
+// the faster (see there).
+template <int EP, int MT>
+__global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_one_kernel(Gemm256Args a) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // Workgroups are dealt round-robin to the 8 XCDs (each with its own L2), so XCD x = blockIdx % 8 takes one
+    // contiguous run of whole tiles (a weight tile is then fetched by one L2 only) and, after those, one
+    // contiguous run of tail parts.  The grid is padded; surplus workgroups leave.
+    const int ntiles = a.tiles_t * a.tiles_r;
+    const int xcd = (int)(blockIdx.x & 7), jx = (int)(blockIdx.x >> 3);
+    const int main_per = (a.main_tiles + 7) >> 3, parts = (ntiles - a.main_tiles) * a.kt, parts_per = (parts + 7) >> 3;
+    int tile, kz = 0, nparts = 1;
+    if (jx < main_per) {
+        tile = xcd * main_per + jx;
+        if (tile >= a.main_tiles) return;
+    } else {
+        const int pidx = xcd * parts_per + (jx - main_per);
+        if (jx - main_per >= parts_per || pidx >= parts) return;
+        tile = a.main_tiles + pidx / a.kt;
+        kz = pidx - (pidx / a.kt) * a.kt;
+        nparts = a.kt;
+    }
+    int bt, br;
+    gemm256_tile(tile, a.tiles_t, a.tiles_r, gemm256_super(MT), &bt, &br);
+    constexpr int BM = gemm256_tokens(MT), XC = 2 * MT, X_SLOT = BM * G_BK * 2, TB = 2 * MT, NM = 8 * TB;     // XC: copies a wave makes of an X slab (of a W slab: 8); TB: its blocks of 16 tokens; NM: products of a step
+    const int t0 = bt * BM, r0 = br * G_BN;
+    const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * 128;
+
+    float4v acc[TB][8];                      // [token block][weight-row block]
+#pragma unroll
+    for (int i = 0; i < TB; ++i)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[i][j] = float4v{0.f, 0.f, 0.f, 0.f};
+
+    // Copies, as above; slabs past the last one re-read the last.
+    constexpr bool XE = gemm256_x_slots(MT) > gemm256_w_slots(MT);        // X is the early one
+    constexpr int E = XE ? gemm256_x_slots(MT) : gemm256_w_slots(MT), L = E - 1, EC = XE ? XC : 8, LC = XE ? 8 : XC;
+    static_assert(L == (XE ? gemm256_w_slots(MT) : gemm256_x_slots(MT)), "the waits below count on it");
+    constexpr int W_AT = gemm256_x_slots(MT) * X_SLOT;
+    constexpr int AHEAD = (E - 2) * EC + (L - 2) * LC;                    // copies that may be on their way when slab s + 1 has to be there
+    const int lrow = lane >> 3, slot = lane & 7;
+    uint32_t xo[XC], wo[8];
+#pragma unroll
+    for (int j = 0; j < XC; ++j) {
+        const int row = wave * (BM / 4) + j * 8 + lrow;
+        const int t = t0 + row < a.T ? row : a.T - 1 - t0;
+        xo[j] = (uint32_t)(t * (int)a.ldx + (slot ^ ((row >> 1) & 7)) * 8) * 2u + (uint32_t)(3 - (j & 3)) * 1024u;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const int row = wave * 64 + j * 8 + lrow;
+        const int r = r0 + row < a.R ? row : a.R - 1 - r0;
+        wo[j] = (uint32_t)(r * (int)a.ldw + (slot ^ ((row >> 1) & 7)) * 8) * 2u + (uint32_t)(3 - (j & 3)) * 1024u;
+    }
+    const int nk_all = (a.C + G_BK - 1) / G_BK, k_begin = (int)((int64_t)kz * nk_all / nparts);
+    const int nk = (int)((int64_t)(kz + 1) * nk_all / nparts) - k_begin;
+    const char* xt = reinterpret_cast<const char*>(a.x + (int64_t)t0 * a.ldx + (int64_t)k_begin * G_BK) - 3072;
+    const char* wt = reinterpret_cast<const char*>(a.w + (int64_t)r0 * a.ldw + (int64_t)k_begin * G_BK) - 3072;
+    typedef __attribute__((address_space(3))) void* lptr_t;
+    const int lastk = nk_all - 1 - k_begin;  // the row's last slab, counted from this part's first
+    bool past[2];                            // this lane's piece of it lies past the row's end, in even and odd copies (whose rows' swizzles differ by 4)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) past[h] = (slot ^ (h * 4 + (lrow >> 1))) * 8 >= a.C - (nk_all - 1) * G_BK;
+    constexpr uint32_t PAST = 0xFFFF0000u;
+    auto copy = [&](const char* base, int at, uint32_t off, int to, int j) {
+        const __amdgpu_buffer_rsrc_t buf = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, PAST, 0x00027000);
+        const lptr_t lds = (lptr_t)(smem + to);
+        if ((j & 3) == 0) __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, lds, 16, off, at, 0, 0);
+        if ((j & 3) == 1) __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, lds, 16, off, at, 1024, 0);
+        if ((j & 3) == 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, lds, 16, off, at, 2048, 0);
+        if ((j & 3) == 3) __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, lds, 16, off, at, 3072, 0);
+    };
+    // `at`: the slab's first column in bytes, `to`: its slot's offset
+    auto copy_x = [&](int at, int to, int j) { copy(xt, at, xo[j], to + wave * (X_SLOT / 4) + (j & ~3) * 1024, j); };
+    auto copy_w = [&](int at, int to, int j) { copy(wt, at, wo[j], to + W_AT + wave * 8192 + (j & ~3) * 1024, j); };
+    auto copy_early = [&](int at, int to, int j) { if constexpr (XE) copy_x(at, to, j); else copy_w(at, to, j); };
+    auto copy_late = [&](int at, int to, int j) { if constexpr (XE) copy_w(at, to, j); else copy_x(at, to, j); };
+    constexpr int ES = XE ? X_SLOT : G_W_SLOT, LS = XE ? G_W_SLOT : X_SLOT;      // their slots' sizes
+    // from the row's last slab on the pieces past its end are asked for past the buffer's end
+    const int plast = lastk < nk && a.C % G_BK != 0 ? lastk : INT_MAX;
+    auto end_early = [&](int q) {
+        if (q < plast) return;
+#pragma unroll
+        for (int j = 0; j < EC; ++j) { uint32_t& o = XE ? xo[j] : wo[j]; o = past[j & 1] ? PAST : o; }
+    };
+    auto end_late = [&](int q) {
+        if (q < plast) return;
+#pragma unroll
+        for (int j = 0; j < LC; ++j) { uint32_t& o = XE ? wo[j] : xo[j]; o = past[j & 1] ? PAST : o; }
+    };
+    auto column = [&](int q) { return (q < nk ? q : nk - 1) * (G_BK * 2); };
+
+    // Fragments, as above
+    half8v fx[TB], fw[2][8];
+    const uint32_t foff = (uint32_t)((lane & 15) * 128 + (((lane >> 4) ^ ((lane >> 1) & 7)) << 4));
+    auto read_x = [&](int kk, int at, int i) {
+        fx[i] = *reinterpret_cast<const half8v*>(smem + at + wm * 128 + i * 2048 + (foff ^ (uint32_t)(kk << 6)));
+    };
+    auto read_w = [&](int set, int kk, int at, int j) {
+        fw[set][j] = *reinterpret_cast<const half8v*>(smem + W_AT + at + wn * 128 + j * 2048 + (foff ^ (uint32_t)(kk << 6)));
+    };
+    // product n of a step: token block n / 8, weight-row block n % 8, to and fro
+    auto mma = [&](int set, int n) {
+        const int i = n >> 3, j = i & 1 ? 7 - (n & 7) : n & 7;
+        asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(fw[set][j]), "v"(fx[i]));
+    };
+    // the accumulators stay in their registers before and behind the loop (without this the compiler copies all 256 into the
+    // other half of the register file at the loop's end, spills, and a launch that needs scratch memory takes 7 us longer)
+#define SQ_PIN() _Pragma("unroll") for (int i = 0; i < TB; ++i) { asm volatile("" : "+a"(acc[i][0]), "+a"(acc[i][1]), "+a"(acc[i][2]), "+a"(acc[i][3]), "+a"(acc[i][4]), "+a"(acc[i][5]), "+a"(acc[i][6]), "+a"(acc[i][7])); }
+#define SQ_SB() __builtin_amdgcn_sched_barrier(0)
+
+#pragma unroll
+    for (int q = 0; q < E - 1; ++q) {
+        end_early(q);
+#pragma unroll
+        for (int j = 0; j < EC; ++j) copy_early(column(q), q * ES, j);
+        if (q == L - 1) break;
+        end_late(q);
+#pragma unroll
+        for (int j = 0; j < LC; ++j) copy_late(column(q), q * LS, j);
+    }
+    __builtin_amdgcn_s_waitcnt(vmcnt_only(AHEAD));
+    SQ_SB(); __builtin_amdgcn_s_barrier(); SQ_SB();
+#pragma unroll
+    for (int i = 0; i < TB - 2; ++i) read_x(0, 0, i);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) read_w(0, 0, 0, j);
+    end_late(L - 1);
+#pragma unroll
+    for (int j = 0; j < LC; ++j) copy_late(column(L - 1), (L - 1) * LS, j);
+    // the slots (byte offsets) of the slab being multiplied, of the next one, and the one the early copies go to; the column of the
+    // slab that is copied.  Worked out between the products, a little at a time: a scalar instruction in front of them takes four
+    // clocks of the matrix core's time.
+    int ce = 0, cl = 0, ne = 0, nl = 0, to = (E - 1) * ES, at = column(L);
+    SQ_PIN();
+    asm volatile("s_nop 7");                 // (no wait of the compiler's between the zeroed accumulators and a written-out product)
+#pragma unroll 1
+    for (int s = 0; s < nk; ++s) {
+        if (s + L >= plast) { end_early(s + L); end_late(s + L); }
+        // first step: its last X blocks, the second step's fragments, the early copies of slab s + L
+#pragma unroll
+        for (int n = 0; n < NM; ++n) {
+            mma(0, n); SQ_SB();
+            if (n < 2) read_x(0, XE ? ce : cl, TB - 1 - n);
+            if (n >= 2 && n <= 16 && n % 2 == 0) read_w(1, 1, XE ? cl : ce, n / 2 - 1);
+            if (n % 8 == 1 && n > 8 && n < NM - 8) read_x(1, XE ? ce : cl, n / 8 - 1);
+            if (n % 4 == 3 && n / 4 < EC) copy_early(at, to, n / 4);
+            if (n == NM - 6) { ne = ce + ES; SQ_SB(); }
+            if (n == NM - 5) { ne = ne == E * ES ? 0 : ne; SQ_SB(); }
+            if (n == NM - 4) { nl = cl + LS; SQ_SB(); }
+            if (n == NM - 3) { nl = nl == L * LS ? 0 : nl; SQ_SB(); }
+            if (n == NM - 2) { to = ce; SQ_SB(); }
+            SQ_SB();
+        }
+        // second step, with the wait and the barrier as above
+#pragma unroll
+        for (int n = 0; n < NM; ++n) {
+            mma(1, n); SQ_SB();
+            if (n < 2) read_x(1, XE ? ce : cl, TB - 1 - n);
+            if (n == 7) {
+                __builtin_amdgcn_s_waitcnt(vmcnt_and_lds(AHEAD)); SQ_SB();
+                __builtin_amdgcn_s_barrier(); SQ_SB();
+            }
+            if (n >= 8 && n <= 22 && n % 2 == 0) read_w(0, 0, XE ? nl : ne, n / 2 - 4);
+            if (n % 8 == 1 && n > 8 && n < NM - 8) read_x(0, XE ? ne : nl, n / 8 - 1);
+            constexpr int GAP = MT == 2 ? 2 : 4;
+            if (n >= 11 && (n - 11) % GAP == 0 && (n - 11) / GAP < LC) copy_late(at, cl, (n - 11) / GAP);
+            if (n == NM - 4) { at = column(s + 1 + L); SQ_SB(); }
+            if (n == NM - 3) { ce = ne; cl = nl; SQ_SB(); }
+            SQ_SB();
+        }
+    }
+    asm volatile("s_nop 15\n\ts_nop 15");    // the last products' results are behind the loop before they are read
+    SQ_PIN();
+#undef SQ_SB
+#undef SQ_PIN
+    __builtin_amdgcn_s_waitcnt(vmcnt_and_lds(0));
+    __syncthreads();                         // every wave is done with the operand ring, and no copy is on its way into it
+
+    // Results leave column of registers after column of registers.  A split tile's go to its partial tile as they are.  16-bit
+    // ones go through LDS: every wave lays its 32 MT x 128 tile out token-major (8 bytes per write) and stores it in 16-byte
+    // pieces, 256 contiguous bytes per token (2-byte stores straight from the accumulators cost 49 us of a 376 us product of
+    // a 2048 x 18944 output).
+    const int quad4 = 4 * (lane >> 4), tok = lane & 15;
+    float* scales = reinterpret_cast<float*>(smem + 2 * BM * G_EP_PITCH);        // behind the four waves' tiles
+    scales[tid] = h2f(gemm256_scale<true>(a.sc, r0 + tid < a.R ? r0 + tid : a.R - 1));
+    __syncthreads();
+    float* part = a.part + ((int64_t)(tile - a.main_tiles) * a.kt + kz) * (BM * G_BN);
+    unsigned char* my = smem + wave * (BM / 2 * G_EP_PITCH);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const int rl = j * 16 + quad4;
+        const float4v sc = *reinterpret_cast<const float4v*>(scales + wn + rl);
+#pragma unroll
+        for (int i = 0; i < TB; ++i) {
+            const int tl = i * 16 + tok;
+            const float4v val = acc[i][j];
+            if (nparts > 1) {
+                *reinterpret_cast<float4v*>(part + (wm + tl) * G_BN + wn + rl) = val;
+            } else if constexpr (EP != SQ_F32) {
+                const float4v o = val * sc;
+                *reinterpret_cast<u32x2*>(my + tl * G_EP_PITCH + rl * 2) =
+                    EP == SQ_BF16 ? u32x2{f2bf_x2(o[0], o[1]), f2bf_x2(o[2], o[3])} : u32x2{f2h_x2(o[0], o[1]), f2h_x2(o[2], o[3])};
+            } else {
+                const int t = t0 + wm + tl, r = r0 + wn + rl;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (t < a.T && r + e < a.R) store_y(a.y, a.y_dtype, (int64_t)t * a.ldy + a.y_off + r + e, val[e] * sc[e]);
+            }
+            if (i & 1) __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    if (EP == SQ_F32 || nparts > 1) return;
+    uint16_t* yb = reinterpret_cast<uint16_t*>(a.y);
+#pragma unroll 4
+    for (int k = 0; k < 8 * MT; ++k) {
+        const int idx = k * 64 + lane, tl = idx >> 4, piece = idx & 15;
+        const int t = t0 + wm + tl, r = r0 + wn + piece * 8;
+        if (t >= a.T || r >= a.R) continue;
+        const u32x4 v = *reinterpret_cast<const u32x4*>(my + tl * G_EP_PITCH + piece * 16);
+        uint16_t* dst = yb + (int64_t)t * a.ldy + a.y_off + r;
+        if (r + 8 <= a.R) {
+            *reinterpret_cast<u32x4*>(dst) = v;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                if (r + e < a.R) dst[e] = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
+        }
+    }
+}
+
 // fp16 copy of a bf16 activation matrix (round to nearest even; exact for every fp16-normal value)
 __global__ __launch_bounds__(256) void bf16_to_f16_kernel(const uint16_t* __restrict__ x, int64_t ldx, int T, int C,
                                                           uint16_t* __restrict__ out) {
@@ -533,14 +769,15 @@ bool gemm256_ok(int C, int64_t ldx, int64_t ldw, const void* x, const void* w) {
 int launch_gemm256(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ldw, const Gemm256Scales& sc, void* y,
                    int y_dtype, int64_t ldy, int y_off, int T, int R, int C, float* part, int cus, hipStream_t s) {
     typedef void (*kernel_t)(Gemm256Args);
-    static constexpr kernel_t kernels[3][3] = {
-        {gemm256_kernel<SQ_F16, 2>, gemm256_kernel<SQ_BF16, 2>, gemm256_kernel<SQ_F32, 2>},
-        {gemm256_kernel<SQ_F16, 3>, gemm256_kernel<SQ_BF16, 3>, gemm256_kernel<SQ_F32, 3>},
-        {gemm256_kernel<SQ_F16, 4>, gemm256_kernel<SQ_BF16, 4>, gemm256_kernel<SQ_F32, 4>}};
+#define SQ_MT(MT) {{gemm256_kernel<SQ_F16, MT>, gemm256_kernel<SQ_BF16, MT>, gemm256_kernel<SQ_F32, MT>}, \
+                   {gemm256_one_kernel<SQ_F16, MT>, gemm256_one_kernel<SQ_BF16, MT>, gemm256_one_kernel<SQ_F32, MT>}}
+    static constexpr kernel_t kernels[3][2][3] = {SQ_MT(2), SQ_MT(3), SQ_MT(4)};
+#undef SQ_MT
     static bool raised = false;
     if (!raised) {
-        for (const auto& of : kernels)
-            for (kernel_t k : of) (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        for (const auto& mt : kernels)
+            for (const auto& one : mt)
+                for (kernel_t k : one) (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         (void)hipGetLastError();
         raised = true;
     }
@@ -555,8 +792,9 @@ int launch_gemm256(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ld
     a.part = part;
     const bool vec = y_dtype != SQ_F32 && ((uintptr_t)y & 15) == 0 && ldy % 8 == 0 && y_off % 8 == 0;
     const int per = (pl.main_tiles + 7) / 8 + (pl.tail_tiles * pl.kt + 7) / 8;       // an XCD's tiles and parts
-    const unsigned grid = (unsigned)(8 * std::min(per, std::max(1, device_cus() / 8)));
-    hipLaunchKernelGGL(kernels[pl.mt - 2][!vec ? 2 : y_dtype == SQ_BF16 ? 1 : 0], dim3(grid), dim3(G_WAVES * 64), gemm256_lds(pl.mt), s, a);
+    const int most = std::max(1, device_cus() / 8);
+    const unsigned grid = (unsigned)(8 * std::min(per, most));
+    hipLaunchKernelGGL(kernels[pl.mt - 2][per <= most][!vec ? 2 : y_dtype == SQ_BF16 ? 1 : 0], dim3(grid), dim3(G_WAVES * 64), gemm256_lds(pl.mt), s, a);
     int rc = check_launch("sq_linear_gemm(gemm256)");
     if (rc || pl.tail_tiles == 0) return rc;
     const unsigned blocks = (unsigned)(pl.tail_tiles * (gemm256_tokens(pl.mt) * G_BN / 1024));

@@ -267,3 +267,33 @@ def test_head_conversion_leaves_loads_alone(tmp_path):
         assert loads and takes >= 4 * loads
         variants += 1
     assert variants == 24
+
+
+def test_one_tile_gemm_waits_for_its_reads_before_the_barrier(tmp_path):
+    """As for the tile kernel: the copies behind a slab's barrier overwrite slots that LDS reads may still be on their way from; and its
+    accumulators, tied to written-out products, are not copied or spilled within the loop over the slabs."""
+    import os
+    import subprocess
+    from quantexperiments_amd import build
+    try:
+        hipcc = build._hipcc()
+    except RuntimeError:
+        pytest.skip("no hipcc")
+    out = tmp_path / "gemm256.s"
+    subprocess.run([hipcc, *build.FLAGS, "-S", "--offload-device-only", str(build.CSRC / "sq_gemm256.hip"), "-o", str(out)], check=True,
+                   capture_output=True, env=dict(os.environ, TMPDIR=str(tmp_path)))
+    variants = 0
+    for body in re.split(r"(?m)^(?=_ZN2sq18gemm256_one_kernel\w+:)", out.read_text())[1:]:
+        lines = [l.split(";")[0].strip() for l in body[:body.index(".Lfunc_end")].splitlines()]
+        lines = [l for l in lines if l and not (l.startswith(".") and not l.startswith(".LBB"))]
+        reads, waits = False, []
+        for i, l in enumerate(lines):
+            reads = reads or l.startswith("ds_read")
+            if l == "s_barrier" and reads:
+                waits.append(next(w for w in reversed(lines[:i]) if w.startswith("s_waitcnt")))
+        assert waits and all("lgkmcnt(0)" in w for w in waits), waits
+        first = next(i for i, l in enumerate(lines) if l.startswith("v_mfma"))
+        last = max(i for i, l in enumerate(lines) if l.startswith("v_mfma"))
+        assert not any(l.startswith(("v_accvgpr", "scratch_")) for l in lines[first:last])
+        variants += 1
+    assert variants == 9
