@@ -60,6 +60,7 @@ struct Gemm256Args {
     void* y;
     int64_t ldx, ldw, ldy;
     int T, R, C, y_off, y_dtype;
+    int y_align;              // alignment of the rows of 16-bit results: 16 bytes, 4 or 2
     int tiles_t, tiles_r;     // token / weight-row tiles (for the workgroup -> tile mapping)
     // The last round of tiles rarely fills the chip (592 tiles on 256 CUs: 2 full rounds and 80 tiles).  Tiles
     // [0, main_tiles) are multiplied whole; each of the remaining tail tiles is split over kt workgroups, each
@@ -130,7 +131,10 @@ template <int N, class F> __device__ __forceinline__ void each(F f) { each(f, st
 // What a workgroup multiplies: a whole tile, or one of the parts of a tail tile.
 struct Gemm256Item { int tile, kz, nparts, t0, r0, k_begin, nk; };
 
-// EP: SQ_F16 / SQ_BF16 = results of that type whose rows allow 16-byte stores, SQ_F32 = any type, element by element
+// EP: SQ_F16 / SQ_BF16 = results of that type, SQ_F32 = fp32 ones, element by element.  Rows of 16-bit results that allow no 16-byte stores leave in
+// pieces of 4 bytes, or 2, a token's 128 by one wave (element by element,
+// straight from the accumulators: 496 rows of 666 x 512 with their decode 26.4 us, 19.0 so, 2048 of 18945 x 3584 345 / 303, 2000 of 2 x 18946 x 1024
+// 361 / 204, 1024 of 2 x 4098 x 2048 76.6 / 55.9).
 // MT: blocks of 32 token rows a wave holds, 64 MT rows a tile
 //
 // A workgroup per CU takes tile after tile: the copies run L slabs ahead of the products over the end of a tile, so the next
@@ -138,6 +142,13 @@ struct Gemm256Item { int tile, kz, nparts, t0, r0, k_begin, nk; };
 // the next tile to get through.  A workgroup per tile spent 9 us a round of tiles beyond its slabs, 4 to 5 of them on the stores;
 // the power limit takes part of that back: gate|up of 2048 rows with its decode (2 x 18944 x 3584, five rounds) 536 -> 523 us, a
 // layer of 2048 rows 980 -> 968, 8192^3 with its decode 809 -> 802, products of one round level.
+// two results of one token: rows of W up to the last one (over: beyond it, -2 and less for both)
+__device__ __forceinline__ void store_pair(uint16_t* at, uint32_t v, int over, int align) {
+    if (align == 4 && over <= -2) { *reinterpret_cast<uint32_t*>(at) = v; return; }
+    if (over < 0) at[0] = (uint16_t)v;
+    if (over < -1) at[1] = (uint16_t)(v >> 16);
+}
+
 #define SQ_INLINE __attribute__((always_inline))
 
 template <int EP, int MT>
@@ -374,7 +385,7 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a)
         asm volatile("" : "+v"(le));             // (nothing of what follows is worked out in front of the loop and kept in registers that it lacks)
         const int quad = le >> 4, tok = le & 15;
         const int split = it.nparts - 1;
-        stores = __builtin_amdgcn_readfirstlane(EP != SQ_F32 && split == 0 && it.t0 + BM <= a.T && it.r0 + G_BN <= a.R ? 1 : 0);
+        stores = __builtin_amdgcn_readfirstlane(EP != SQ_F32 && a.y_align == 16 && split == 0 && it.t0 + BM <= a.T && it.r0 + G_BN <= a.R ? 1 : 0);
         float* part = a.part + ((int64_t)(it.tile - a.main_tiles) * a.kt + it.kz) * (BM * G_BN);
         float4v sc[8];
 #pragma unroll
@@ -417,6 +428,16 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a)
                         EP == SQ_BF16 ? u32x2{f2bf_x2(o[0], o[1]), f2bf_x2(o[2], o[3])} : u32x2{f2h_x2(o[0], o[1]), f2h_x2(o[2], o[3])};
                 });
             });
+            if (a.y_align != 16) {
+                const int over = it.r0 + wn + 2 * le - a.R;      // (-2 and less: both are rows of W)
+                uint16_t* pair = reinterpret_cast<uint16_t*>(a.y) + (int64_t)(it.t0 + wm + p * TBP * 16) * ldy + a.y_off + it.r0 + wn + 2 * le;
+#pragma unroll 4
+                for (int k = 0; k < 16 * TBP; ++k, pair += ldy) {
+                    const uint32_t v2 = *reinterpret_cast<const uint32_t*>(my + k * 256 + (((le >> 2) ^ (k & 15)) * 16) + (le & 3) * 4);
+                    if (it.t0 + wm + p * TBP * 16 + k < a.T) store_pair(pair, v2, over, a.y_align);
+                }
+                return;
+            }
             u32x4 v[4 * TBP];
 #pragma unroll
             for (int k = 0; k < 4 * TBP; ++k) v[k] = *reinterpret_cast<const u32x4*>(my + (k * 4 + quad) * 256 + ((tok ^ ((k * 4 + quad) & 15)) * 16));
@@ -669,6 +690,13 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_one_kernel(Gemm256Arg
     }
     if (EP == SQ_F32 || nparts > 1) return;
     uint16_t* yb = reinterpret_cast<uint16_t*>(a.y);
+    if (a.y_align != 16) {
+        uint16_t* pair = yb + (int64_t)(t0 + wm) * a.ldy + a.y_off + r0 + wn + 2 * lane;
+#pragma unroll 4
+        for (int k = 0; k < BM / 2; ++k, pair += a.ldy)
+            if (t0 + wm + k < a.T) store_pair(pair, *reinterpret_cast<const uint32_t*>(my + k * G_EP_PITCH + lane * 4), r0 + wn + 2 * lane - a.R, a.y_align);
+        return;
+    }
 #pragma unroll 4
     for (int k = 0; k < 8 * MT; ++k) {
         const int idx = k * 64 + lane, tl = idx >> 4, piece = idx & 15;
@@ -790,11 +818,11 @@ int launch_gemm256(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ld
     a.main_tiles = pl.main_tiles;
     a.kt = pl.kt;
     a.part = part;
-    const bool vec = y_dtype != SQ_F32 && ((uintptr_t)y & 15) == 0 && ldy % 8 == 0 && y_off % 8 == 0;
+    a.y_align = ((uintptr_t)y & 15) == 0 && ldy % 8 == 0 && y_off % 8 == 0 ? 16 : ((uintptr_t)y & 3) == 0 && ldy % 2 == 0 && y_off % 2 == 0 ? 4 : 2;
     const int per = (pl.main_tiles + 7) / 8 + (pl.tail_tiles * pl.kt + 7) / 8;       // an XCD's tiles and parts
     const int most = std::max(1, device_cus() / 8);
     const unsigned grid = (unsigned)(8 * std::min(per, most));
-    hipLaunchKernelGGL(kernels[pl.mt - 2][per <= most][!vec ? 2 : y_dtype == SQ_BF16 ? 1 : 0], dim3(grid), dim3(G_WAVES * 64), gemm256_lds(pl.mt), s, a);
+    hipLaunchKernelGGL(kernels[pl.mt - 2][per <= most][y_dtype == SQ_F32 ? 2 : y_dtype == SQ_BF16 ? 1 : 0], dim3(grid), dim3(G_WAVES * 64), gemm256_lds(pl.mt), s, a);
     int rc = check_launch("sq_linear_gemm(gemm256)");
     if (rc || pl.tail_tiles == 0) return rc;
     const unsigned blocks = (unsigned)(pl.tail_tiles * (gemm256_tokens(pl.mt) * G_BN / 1024));

@@ -136,3 +136,21 @@ def test_broken_rows_in_tiles(d, bits, G, M, C, T, large):
     y = ps.forward(x.cuda())
     ref = np.concatenate([x.float().numpy().astype(np.float64) @ s.decode().astype(np.float64).T for s in ss], axis=1)
     assert rel_max_err(y.float().cpu().numpy(), ref) < 5e-3
+
+
+@pytest.mark.parametrize("T,R,C", [(130, 2, 64), (257, 299, 192), (700, 1026, 128), (300, 700, 4160), (2049, 9001, 64), (1500, 16514, 128)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_rows_of_results_without_16_byte_stores(T, R, C, dtype):
+    """16-bit results whose rows allow stores of 4 bytes or 2: the same products and the same rounding as rows that allow 16, so the same
+    bits; one tile per workgroup, several, parts of tiles; nothing is written beside the rows."""
+    g = torch.Generator(device="cuda").manual_seed(T + R)
+    x = torch.randn(T, C, device="cuda", generator=g).half()
+    w = torch.randn(R, C, device="cuda", generator=g).half()
+    want = torch.zeros(T, (R + 15) // 8 * 8, dtype=dtype, device="cuda")
+    gemm_dense(w, x, want[:, :R])
+    for ld, off in ((R + 3 + (R + 3) % 2, 2), (R + 4 + (R + 5) % 2, 0), (R + 4, 1)):
+        y = torch.full((T * ld + 16,), 5.0, dtype=dtype, device="cuda")
+        rows = y[off:off + T * ld].view(T, ld)
+        gemm_dense(w, x, rows[:, :R])
+        assert torch.equal(rows[:, :R], want[:, :R]), (ld, off)
+        assert bool((rows[:, R:] == 5.0).all()) and bool((y[:off] == 5.0).all()) and bool((y[off + T * ld:] == 5.0).all())
