@@ -80,6 +80,13 @@ template <> struct store_as<SQ_F32> { typedef float type; static __device__ __fo
 template <> struct store_as<SQ_F16> { typedef uint16_t type; static __device__ __forceinline__ uint16_t cvt(float f) { return f2h(f); } };
 template <> struct store_as<SQ_BF16> { typedef uint16_t type; static __device__ __forceinline__ uint16_t cvt(float f) { return f2bf(f); } };
 
+// Two 16-bit results of one token, of neighbouring weight rows; over: the first one's row less the number of rows (-2 and less: both are there)
+__device__ __forceinline__ void store_pair(uint16_t* at, uint32_t v, int over, bool whole) {
+    if (whole && over <= -2) { *reinterpret_cast<uint32_t*>(at) = v; return; }
+    if (over < 0) at[0] = (uint16_t)v;
+    if (over < -1) at[1] = (uint16_t)(v >> 16);
+}
+
 __device__ __forceinline__ void store_y(void* y, int y_dtype, int64_t o, float v) {
     if (y_dtype == SQ_BF16) reinterpret_cast<uint16_t*>(y)[o] = f2bf(v);
     else if (y_dtype == SQ_F16) reinterpret_cast<uint16_t*>(y)[o] = f2h(v);

@@ -142,13 +142,6 @@ struct Gemm256Item { int tile, kz, nparts, t0, r0, k_begin, nk; };
 // the next tile to get through.  A workgroup per tile spent 9 us a round of tiles beyond its slabs, 4 to 5 of them on the stores;
 // the power limit takes part of that back: gate|up of 2048 rows with its decode (2 x 18944 x 3584, five rounds) 536 -> 523 us, a
 // layer of 2048 rows 980 -> 968, 8192^3 with its decode 809 -> 802, products of one round level.
-// two results of one token: rows of W up to the last one (over: beyond it, -2 and less for both)
-__device__ __forceinline__ void store_pair(uint16_t* at, uint32_t v, int over, int align) {
-    if (align == 4 && over <= -2) { *reinterpret_cast<uint32_t*>(at) = v; return; }
-    if (over < 0) at[0] = (uint16_t)v;
-    if (over < -1) at[1] = (uint16_t)(v >> 16);
-}
-
 #define SQ_INLINE __attribute__((always_inline))
 
 template <int EP, int MT>
@@ -434,7 +427,7 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a)
 #pragma unroll 4
                 for (int k = 0; k < 16 * TBP; ++k, pair += ldy) {
                     const uint32_t v2 = *reinterpret_cast<const uint32_t*>(my + k * 256 + (((le >> 2) ^ (k & 15)) * 16) + (le & 3) * 4);
-                    if (it.t0 + wm + p * TBP * 16 + k < a.T) store_pair(pair, v2, over, a.y_align);
+                    if (it.t0 + wm + p * TBP * 16 + k < a.T) store_pair(pair, v2, over, a.y_align == 4);
                 }
                 return;
             }
@@ -694,7 +687,7 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_one_kernel(Gemm256Arg
         uint16_t* pair = yb + (int64_t)(t0 + wm) * a.ldy + a.y_off + r0 + wn + 2 * lane;
 #pragma unroll 4
         for (int k = 0; k < BM / 2; ++k, pair += a.ldy)
-            if (t0 + wm + k < a.T) store_pair(pair, *reinterpret_cast<const uint32_t*>(my + k * G_EP_PITCH + lane * 4), r0 + wn + 2 * lane - a.R, a.y_align);
+            if (t0 + wm + k < a.T) store_pair(pair, *reinterpret_cast<const uint32_t*>(my + k * G_EP_PITCH + lane * 4), r0 + wn + 2 * lane - a.R, a.y_align == 4);
         return;
     }
 #pragma unroll 4
