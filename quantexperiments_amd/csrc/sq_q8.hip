@@ -608,7 +608,7 @@ static bool q8_mfma_ok(int C) { return C % 32 == 0 && (int64_t)C * 64 < ((int64_
 // 30,000 x 1,216 41.3 / 41.9, of 32,000 x 640 33.6 / 27.6, of 50,000 x 3,520 203 / 106, 200 of 70,061 x 1,216 164 / 170.
 // Rows of an odd number of blocks: 8 / 16 / 32 / 64 rows of 150,000 x 3,488 246 / 490 / 974 / 877 (127 / 131 / 144 / 189 here), of 8,400 x 2,528 24 / 45 / 88 /
 // 95 (24 / 19 / 24 / 32), 4 of 60,000 x 2,080 39 / 30; of 30,000 x 608 both are done before an eager call is issued, 4 / 5 / 8 rows 14 / 17 / 20 there and 17.5
-// here, whose calls take a buffer and launch a copy of x.
+// here, when its calls still launched a copy of x.
 // 3 rows of 105,038 x 3,392, which the 256 MB last-level cache does not hold from call to call: 86.5 / 90.5; 5 take two passes there.
 bool q8_mid(int V, int C, int B) {
     if (B <= 2 || !q8_mfma_ok(C)) return false;
