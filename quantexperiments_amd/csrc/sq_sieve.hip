@@ -53,6 +53,9 @@ struct SieveArgs {
 __device__ __forceinline__ int sieve_swizzle(int t) { return (t & 3) | ((t >> 3) & 1) << 2; }
 constexpr int SIEVE_STAGE = 16 * 512;
 
+// s_waitcnt immediate that waits until at most n vector-memory operations are outstanding (gfx9 encoding: vmcnt in bits 3:0 and 15:14)
+constexpr int sieve_vmcnt_only(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
+
 template <int TW>
 __global__ __launch_bounds__(64 * SIEVE_WAVES) void sieve_kernel(SieveArgs a) {
     constexpr int NTH = 64 * SIEVE_WAVES;
@@ -78,6 +81,7 @@ __global__ __launch_bounds__(64 * SIEVE_WAVES) void sieve_kernel(SieveArgs a) {
     for (int k = 0; k < SIEVE_TAB / (NTH * 16); ++k)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(table, (sieve_lptr_t)(smem + (k * NTH + wave * 64) * 16), 16, tid * 16, k * NTH * 16, 0, 0);
     if (tid < 8) reinterpret_cast<uint32_t*>(smem + SIEVE_TAB)[tid] = 0u;       // (and the flag behind it)
+    __builtin_amdgcn_sched_barrier(0);       // (the wait for the slice counts the loads behind it)
 
     // ---- this wave's tiles (tiles past the last row repeat the last one and are not stored; waves without a tile only stage)
     const int ntiles = (m.R + 15) >> 4, tile0 = (blk * SIEVE_WAVES + wave) * TW;
@@ -143,7 +147,11 @@ __global__ __launch_bounds__(64 * SIEVE_WAVES) void sieve_kernel(SieveArgs a) {
     px[1] = load_x(r0 + 1);
     store_x(px[0], 0, r0);
     place_tags(r0, tag[0]);
-    __syncthreads();                         // (and the slice has landed)
+    // every wave gathers what others have copied, and no barrier waits for copies: this wave's part of the slice has landed once no more
+    // operations are on their way than it has issued behind it for the second round, TW of tags and one of activations
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(sieve_vmcnt_only(TW + 1));
+    __syncthreads();
     if (work) {
 #pragma unroll
         for (int q = 0; q < PF; ++q) wf[q] = gather(tag[0][q % TW][q / TW >> 1], q / TW & 1);

@@ -297,3 +297,33 @@ def test_one_tile_gemm_waits_for_its_reads_before_the_barrier(tmp_path):
         assert not any(l.startswith(("v_accvgpr", "scratch_")) for l in lines[first:last])
         variants += 1
     assert variants == 9
+
+
+def test_sieve_waits_for_its_codebook_slice(tmp_path):
+    """Every wave gathers from the whole slice, which the waves have copied to LDS between them: in front of the first barrier the source
+    has to wait for this wave's copies itself, for no barrier does.  In the assembly of every variant the wait right there leaves at most
+    as many operations on their way as have been issued, on every path, behind the last copy."""
+    import os
+    import subprocess
+    from quantexperiments_amd import build
+    try:
+        hipcc = build._hipcc()
+    except RuntimeError:
+        pytest.skip("no hipcc")
+    out = tmp_path / "sieve.s"
+    subprocess.run([hipcc, *build.FLAGS, "-S", "--offload-device-only", str(build.CSRC / "sq_sieve.hip"), "-o", str(out)], check=True,
+                   capture_output=True, env=dict(os.environ, TMPDIR=str(tmp_path)))
+    variants = 0
+    for body in re.split(r"(?m)^(?=_ZN2sq12sieve_kernel\w+:)", out.read_text())[1:]:
+        tiles = int(re.match(r"_ZN2sq12sieve_kernelILi(\d)E", body)[1])
+        lines = [l.split(";")[0].strip() for l in body[:body.index(".Lfunc_end")].splitlines()]
+        lines = [l for l in lines if l and (not l.startswith(".") or l.startswith(".LBB"))]
+        barrier = lines.index("s_barrier")
+        copies = [i for i, l in enumerate(lines) if l.startswith("buffer_load") and l.endswith(" lds")]
+        assert len(copies) == 8 and copies[-1] < barrier
+        branch = next(i for i, l in enumerate(lines) if i > copies[-1] and l.startswith(("s_cbranch", ".LBB")))
+        behind = sum(l.startswith(("global_load", "buffer_load", "flat_load")) for l in lines[copies[-1] + 1:branch])
+        wait = re.fullmatch(r"s_waitcnt .*vmcnt\((\d+)\).*", lines[barrier - 1])
+        assert wait and int(wait[1]) <= min(tiles + 1, behind), lines[barrier - 4:barrier + 1]
+        variants += 1
+    assert variants == 4
