@@ -147,7 +147,7 @@ int sq_linear_small(const sq_matrix* mats, int32_t n_mats, const void* x, int x_
     if ((rc = refuse_if_poisoned("sq_linear_small", mats, n_mats))) return rc;
     const WsParts w = split_workspace(workspace, ws_bytes);
     if (w.sums) (void)stream_host_flag((hipStream_t)stream, true);      // (one pinned host word per device, first call only)
-    if (small_takes_gemm_route(mats, n_mats, B, x, ldx, w.inner_bytes))
+    if (small_takes_gemm_route(mats, n_mats, B, x, ldx))
         return launch_gemm(mats, n_mats, x, x_dtype, ldx, y, y_dtype, ldy, B, w.inner, w.inner_bytes, w.sums, (hipStream_t)stream);
     return launch_small(mats, n_mats, x, x_dtype, ldx, y, y_dtype, ldy, B, w.inner, w.inner_bytes, w.sums, (hipStream_t)stream);
 }
@@ -191,7 +191,7 @@ int sq_linear_small_noalloc(const sq_matrix* mats, int32_t n_mats, const void* x
     size_t small = small_workspace(mats, n_mats, B);
     if (small > inner) small = small_workspace_least(mats, n_mats, B);
     const size_t decoded = small_gemm_route_workspace(mats, n_mats, B);
-    const bool in_place = decoded > inner && (B <= NOALLOC_ROWS_IN_PLACE || mats[0].C % 64 || !has_orders(mats, n_mats));
+    const bool in_place = decoded > inner && (B <= NOALLOC_ROWS_IN_PLACE || mats[0].C % 64);
     const bool route = !in_place && small_takes_gemm_route(mats, n_mats, B, x, ldx);
     const size_t need = in_place ? small : std::max(small, decoded > inner ? gemm_workspace_without_mid(mats, n_mats, B) : decoded);
     if (need > inner)
@@ -248,7 +248,7 @@ int sq_linear_small_from(const sq_matrix* mats, int32_t n_mats, const sq_produce
                                   C, from->eps, from->x_out, x_dtype, s)
                  : launch_silu_mul(from->add, from->up, x_dtype, from->ld_in, nullptr, 1, B, C, from->x_out, s);
     if (rc) return rc;
-    if (small_takes_gemm_route(mats, n_mats, B, from->x_out, C, wsb))
+    if (small_takes_gemm_route(mats, n_mats, B, from->x_out, C))
         return launch_gemm(mats, n_mats, from->x_out, x_dtype, C, y, y_dtype, ldy, B, ws, wsb, has_ws ? workspace : nullptr, s);
     return launch_small(mats, n_mats, from->x_out, x_dtype, C, y, y_dtype, ldy, B, ws, wsb, has_ws ? workspace : nullptr, s);
 }
@@ -320,7 +320,7 @@ size_t sq_workspace_bytes(const sq_matrix* mats, int32_t n_mats, int32_t rows, i
     if (!mats || n_mats <= 0 || rows <= 0) return 0;
     // which & 1 = 0 covers both kernels a stack with column orders may take (the caller's x decides, see sq_linear_small)
     const size_t inner = (which & 4) && rows <= SQ_SMALL_BMAX
-                             ? std::max(small_workspace_least(mats, n_mats, rows), has_orders(mats, n_mats) ? small_gemm_route_workspace(mats, n_mats, rows) : (size_t)0)
+                             ? std::max(small_workspace_least(mats, n_mats, rows), small_gemm_route_workspace(mats, n_mats, rows))
                          : (which & 1) == 0 ? std::max(small_workspace(mats, n_mats, rows), small_gemm_route_workspace(mats, n_mats, rows))
                                             : gemm_workspace(mats, n_mats, rows);
     const bool sums = small_uses_sums(mats, n_mats);

@@ -159,12 +159,15 @@ bool small_uses_sums(const sq_matrix* mats, int n);
 int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype,
                 int64_t ldy, int T, void* ws, size_t ws_bytes, void* sums, hipStream_t s);
 // stacks with column orders and more than a few activation rows: sq_linear_small runs the decode + tile GEMM route
-bool small_takes_gemm_route(const sq_matrix* mats, int n, int B, const void* x, int64_t ldx, size_t ws_bytes = ~(size_t)0);
+bool small_takes_gemm_route(const sq_matrix* mats, int n, int B, const void* x, int64_t ldx);
 size_t small_gemm_route_workspace(const sq_matrix* mats, int n, int B);
 bool has_orders(const sq_matrix* mats, int n);
 constexpr int MID_PIECES = 8;          // (kernel arguments of 1 KB)
-// the piece would run on the vector kernels at B rows, which take every few rows as long again
+// the piece would run on the vector kernels at B rows; how many such pieces sq_linear_small decodes and multiplies from there; their call
 bool small_vector(const sq_matrix& m, int B);
+int vector_decoded(const sq_matrix* mats, int n, int B);
+size_t decoded_workspace(const sq_matrix* mats, int n, int T);
+int launch_decoded(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, hipStream_t s);
 // 33 .. a few hundred activation rows in one pass over the tags (sq_mid.h): whether these pieces can take it, and its call
 bool mma_shape(const sq_matrix& m);
 bool mid_ok(const sq_matrix* mats, int n, int T);

@@ -169,12 +169,15 @@ static size_t dense_bytes(const sq_matrix& m) { return (((size_t)m.R * m.C * 2) 
 // against 625 us here).  Rows that end within a slab of 64 columns take it from BROKEN_DECODED_T on, up to where they are decoded in steps
 // of bounded workspace (5120 x 2080: 34-38 us there at 200 rows, 38-44 here at 400; in the 128 x 128 kernel 80-120).
 constexpr int BROKEN_DECODED_T = 256;
-static bool big_route(const sq_matrix* mats, int n, int T) {
-    if (mats[0].C % 64) return mats[0].C % 8 == 0 && T > BROKEN_DECODED_T;
-    if (T >= GEMM256_MIN_T) return true;
+bool has_orders(const sq_matrix* mats, int n) {
     for (int i = 0; i < n; ++i)
         if (mats[i].perms) return true;
     return false;
+}
+
+static bool big_route(const sq_matrix* mats, int n, int T) {
+    if (mats[0].C % 64) return mats[0].C % 8 == 0 && T > BROKEN_DECODED_T;
+    return T >= GEMM256_MIN_T || has_orders(mats, n);
 }
 
 // Pieces that are neighbours in Y are decoded one behind the other and multiplied in ONE tile GEMM over all their
@@ -248,23 +251,17 @@ static DecodedRows decoded_step(const sq_matrix* mats, int n, int& i, int& r0) {
 // and 248; 30000 x 3584 at 128 / 200 / 256 rows 164 / 154 / 153 and 138 / 169 / 173, 18944 x 3584 96 / 107 / 108 and 103 / 128 /
 // 127, 3584 x 18944 107 / 116 / 120 and 112 / 131 / 134, 4608 x 3584 44 / 46 / 47 and 40 / 46 / 49, 593 x 1984 41 / 41 / 41 and
 // 26 / 32 / 34).
-bool has_orders(const sq_matrix* mats, int n) {
-    for (int i = 0; i < n; ++i)
-        if (mats[i].perms) return true;
-    return false;
-}
-
 static bool decoded_route(const sq_matrix* mats, int n, int T) {
     int64_t rows = 0;
     for (int i = 0; i < n; ++i) {
         rows += mats[i].R;
         if (mats[i].R > 0 && (!mats[i].tags || !mid_dense_ok(mats + i, 1, T))) return false;
     }
-    if (mats[0].C % 64 || (T <= SQ_SMALL_BMAX && !has_orders(mats, n))) return true;
+    if (mats[0].C % 64) return true;
     return rows < (int64_t)128 * device_cus() && (T <= 128 || rows * mats[0].C < (int64_t)24 << 20);
 }
 
-static size_t decoded_workspace(const sq_matrix* mats, int n, int T) {
+size_t decoded_workspace(const sq_matrix* mats, int n, int T) {
     size_t need = 0;
     for (int i = 0, r0 = 0; i < n;) {
         const DecodedRows d = decoded_step(mats, n, i, r0);
@@ -273,8 +270,7 @@ static size_t decoded_workspace(const sq_matrix* mats, int n, int T) {
     return need;
 }
 
-static int launch_decoded(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws,
-                          hipStream_t s) {
+int launch_decoded(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, hipStream_t s) {
     int rows = T;                                                // activation rows at a time: all, unless they span 4 GB
     while (rows > 1 && !mid_x_ok(ldx, rows)) rows = (rows + 1) / 2;
     for (int i = 0, r0 = 0; i < n;) {
@@ -299,28 +295,31 @@ static int launch_decoded(const sq_matrix* mats, int n, const void* x, int x_dty
 // there and here: 4608 x 3584 46 / 89 us and 43, 37888 x 3584 81 / 118 and 237).  Without, each four rows cost as much again,
 // twice that on long rows (4 / 5 / 8 rows there, and any of them here: 593 x 1984 15 / 23 / 28 us and 18, 16000 x 3584 54 / 91 /
 // 103 and 78, 3584 x 18944 193 / 242 / 384 and 95, at 2 rows 97; 37888 x 3584 at 8 / 9 rows 194 / 272 and 237 in the tile GEMM).
-// Without orders, from VECTOR_DECODED_B rows, stacks of which the decode-time product would run a piece on the vector kernels: 16-bit tags of
-// rows that end within a lane unit, tags of other widths, codebooks beyond the cache (5120 x 2080, 16-bit tags, at 16 / 32 rows 212 /
-// 415 us there).
-constexpr int VECTOR_DECODED_B = 3;
 static bool masked_gemm(const sq_matrix* mats, int n, int B) {
-    if (!has_orders(mats, n)) {
-        bool vector = false;
-        for (int i = 0; i < n; ++i) vector = vector || small_vector(mats[i], B);
-        return vector && B >= VECTOR_DECODED_B && decoded_route(mats, n, B);
-    }
+    if (!has_orders(mats, n)) return false;
     if (small_uses_sums(mats, n)) return decoded_route(mats, n, B) ? B >= 11 : B >= 17 && mats[0].C % 64 == 0;
     if (decoded_route(mats, n, B)) return B >= (mats[0].C > 8192 ? 3 : 5);
     return B >= 9 && mats[0].C % 64 == 0;
 }
 
-// (stacks without orders can do without: where the workspace has no room they run on the decode-time kernel)
-bool small_takes_gemm_route(const sq_matrix* mats, int n, int B, const void* x, int64_t ldx, size_t ws_bytes) {
-    return masked_gemm(mats, n, B) && x_vec_ok(x, ldx, mats[0].C) && (has_orders(mats, n) || decoded_workspace(mats, n, B) <= ws_bytes);
+bool small_takes_gemm_route(const sq_matrix* mats, int n, int B, const void* x, int64_t ldx) {
+    return masked_gemm(mats, n, B) && x_vec_ok(x, ldx, mats[0].C);
 }
 
 size_t small_gemm_route_workspace(const sq_matrix* mats, int n, int B) {
     return masked_gemm(mats, n, B) ? gemm_workspace(mats, n, B) : 0;
+}
+
+// Without orders: how many pieces, the first one on, are decoded and multiplied from there at B rows because the decode-time product would
+// run them on the vector kernels (16-bit tags of rows that end within a lane unit, tags of other widths, codebooks beyond LDS), which
+// take every few rows as long again: from VECTOR_DECODED_B rows (5120 x 2080, 16-bit tags, at 16 / 32 rows 212 / 415 us there, 24 / 25
+// here).  Their neighbours in the stack keep their kernels, which read tags.
+constexpr int VECTOR_DECODED_B = 3;
+int vector_decoded(const sq_matrix* mats, int n, int B) {
+    if (B < VECTOR_DECODED_B) return 0;
+    int k = 0, found = 0;
+    for (; k < n && (mats[k].R == 0 || (small_vector(mats[k], B) && mid_dense_ok(mats + k, 1, B))); ++k) found += mats[k].R > 0;
+    return found ? k : 0;
 }
 
 static size_t gemm_workspace_beyond_small(const sq_matrix* mats, int n, int T);
@@ -408,7 +407,7 @@ int launch_gemm_dense(const void* w, int w_dtype, int64_t ldw, int R, int C, con
 
 int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype,
                 int64_t ldy, int T, void* ws, size_t ws_bytes, void* sums, hipStream_t s) {
-    if (T <= SQ_SMALL_BMAX && !small_takes_gemm_route(mats, n, T, x, ldx, ws_bytes))
+    if (T <= SQ_SMALL_BMAX && !small_takes_gemm_route(mats, n, T, x, ldx))
         return launch_small(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, ws_bytes, sums, s);
     if (x_vec_ok(x, ldx, mats[0].C) && fused_route(mats, n, T) && fused_workspace(mats, n, T) <= ws_bytes)
         return launch_fused(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);

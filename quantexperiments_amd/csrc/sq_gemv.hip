@@ -235,7 +235,7 @@ static int sieve_len(const sq_matrix* mats, int n, int B) {
     return sieve_group(mats, k, B);
 }
 
-// tight: the pieces that can run without partial sums do
+// tight: the pieces that can run without partial sums or decoded weights do
 // (a group that sq_sieve.hip takes runs there unless the workspace is tight or x not aligned: then piece by piece as below)
 static size_t small_need(const sq_matrix* mats, int n, int B, bool tight, bool sieve = true) {
     size_t tot = 0;
@@ -252,7 +252,16 @@ static size_t small_need(const sq_matrix* mats, int n, int B, bool tight, bool s
     return tot;
 }
 
-size_t small_workspace(const sq_matrix* mats, int n, int B) { return small_need(mats, n, B, false); }
+size_t small_workspace(const sq_matrix* mats, int n, int B) {
+    size_t need = small_need(mats, n, B, false);
+    if (has_orders(mats, n)) return need;
+    for (int i = 0; i < n; ++i)                                  // (decoded weights: a launch's own, from the workspace's first byte on)
+        if (const int k = vector_decoded(mats + i, n - i, B); k > 0) {
+            need = std::max(need, decoded_workspace(mats + i, k, B));
+            i += k - 1;
+        }
+    return need;
+}
 size_t small_workspace_least(const sq_matrix* mats, int n, int B) { return small_need(mats, n, B, true); }
 
 bool small_uses_sums(const sq_matrix* mats, int n) {
@@ -404,7 +413,7 @@ int launch_small_silu(const sq_matrix* mats, int n, const void* x, int x_dtype, 
 int launch_small(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype,
                  int64_t ldy, int B, void* ws, size_t ws_bytes, void* sums, hipStream_t s, const sq_producer* from) {
     if (from && !small_fuses_producer(mats, n, B)) return fail(SQ_EUNSUPPORTED, "sq_linear_small_from: no fused kernel for this stack");
-    const bool tight = small_workspace(mats, n, B) > ws_bytes;
+    const bool tight = small_need(mats, n, B, false) > ws_bytes, orders = has_orders(mats, n);
     if (tight && small_workspace_least(mats, n, B) > ws_bytes)
         return fail(SQ_EWORKSPACE, "sq_linear_small: workspace %zu < %zu", ws_bytes, small_workspace(mats, n, B));
     const int cus = device_cus();
@@ -423,6 +432,11 @@ int launch_small(const sq_matrix* mats, int n, const void* x, int x_dtype, int64
             int rc = launch_stream_group(mats + i, j - i, x, x_dtype, ldx, y, y_dtype, ldy, B, (char*)sums, s, from);
             if (rc) return rc;
             i = j;
+            continue;
+        }
+        if (const int k = orders || !x_ok ? 0 : vector_decoded(mats + i, n - i, B); k > 0 && decoded_workspace(mats + i, k, B) <= ws_bytes) {
+            if (const int rc = launch_decoded(mats + i, k, x, x_dtype, ldx, y, y_dtype, ldy, B, ws, s)) return rc;
+            i += k;
             continue;
         }
         if (const int k = tight || !x_ok ? 0 : sieve_len(mats + i, n - i, B); k > 0) {

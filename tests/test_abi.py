@@ -182,6 +182,22 @@ def test_workspace_of_decoded_weights_is_bounded():
     assert need((24, 7), 3592, 8, 16, 16, 20, 0) >= 31 * 3592 * 2                     # decode sizes with column orders go the same way
 
 
+def test_mixed_stacks_decode_only_what_needs_it():
+    """From 3 rows a piece of a format without a matrix-core kernel is decoded into the workspace; its neighbours' tags are read."""
+    L = _lib.lib()
+    mat = lambda R, C, d, bits, off: _lib.SqMatrix(0x10000, 0x20000, 0x30000, None, None, None, None, R, C, d, bits, 1, 1, (C // d * bits + 31) // 32, off)
+    need = lambda mats, B, which: L.sq_workspace_bytes(_lib.matrix_array(mats), len(mats), B, which)
+    for d, bits in ((8, 16), (4, 12)):
+        for B in (3, 16, 32):
+            large, small = mat(18944, 3584, d, bits, 0), mat(64, 3584, 8, 14, 18944)
+            alone = max(need([large], B, 0), _lib.WS_HEADER), need([small], B, 0)
+            assert 64 * 3584 * 2 <= alone[1] - _lib.WS_HEADER < 4 << 20
+            for which in (0, 1):
+                assert max(alone) <= need([large, small], B, which) < _lib.WS_HEADER + 32 * 18944 * B * 4 + (4 << 20)
+                assert need([large, small], B, which) == need([small, large], B, which) == need([large, small, mat(0, 3584, d, bits, 19008)], B, which)
+    assert need([mat(64, 3584, 8, 14, 0)], 2, 0) == 0
+
+
 def test_tile_gemm_waits_for_its_reads_before_the_barrier(tmp_path):
     """Behind the barrier of a slab the ring's slots are overwritten by copies that no compiler dependence ties to the reads, so
     the source itself has to wait for them: in the assembly of every variant the wait in front of a barrier behind LDS reads names

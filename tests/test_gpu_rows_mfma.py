@@ -157,3 +157,31 @@ def test_formats_of_the_vector_kernels(d, bits, C, G, room):
             mats = _lib.matrix_array([lins[0].descriptor(0), lins[1].descriptor(130)])
             _lib.check(L.sq_linear_small(mats, 2, x.data_ptr(), _lib.SQ_BF16, C, y.data_ptr(), _lib.SQ_F32, 139, B, None, 0, _lib.stream_ptr(dev)))
         assert rel_max_err(y.cpu().numpy(), x.half().double().cpu().numpy() @ w.T) < 1e-5, B
+
+
+@pytest.mark.parametrize("d,bits", [(8, 16), (4, 12)])
+@pytest.mark.parametrize("stream", [True, False])
+@pytest.mark.parametrize("noalloc", [True, False])
+def test_mixed_stacks(d, bits, stream, noalloc):
+    """Pieces that are decoded first beside pieces whose tags are read: each runs as it does alone."""
+    L, C = _lib.lib(), 1024
+    formats = [(700, d, bits), (40, 8, 14), (33, 4, 14), (300, d, bits), (17, 8, 5)]
+    ss = [synth(R, C, dd, b, 1, 1, seed=R) for R, dd, b in formats]
+    lins = [to_device(s, stream=stream) for s in ss]
+    R = sum(f[0] for f in formats)
+    w = np.concatenate([s.decode() for s in ss]).astype(np.float64)
+    for B in (2, 3, 9, 32):
+        x = rand_x(B, C, torch.bfloat16, seed=B).cuda()
+        y = torch.full((B, R), float("nan"), device="cuda")
+        if noalloc:
+            offs = np.cumsum([0] + [f[0] for f in formats])
+            mats = _lib.matrix_array([lin.descriptor(int(o)) for lin, o in zip(lins, offs)])
+            _lib.check(L.sq_linear_small_noalloc(mats, len(lins), x.data_ptr(), _lib.SQ_BF16, C, y.data_ptr(), _lib.SQ_F32, R, B, _lib.stream_ptr(x.device)))
+        else:
+            linear_small(lins, x, y)
+        assert rel_max_err(y.cpu().numpy(), x.half().double().cpu().numpy() @ w.T) < 1e-5, B
+        for i in (0, 3):
+            o = sum(f[0] for f in formats[:i])
+            alone = torch.empty(B, formats[i][0], device="cuda")
+            linear_small([lins[i]], x, alone)
+            assert torch.equal(y[:, o:o + formats[i][0]], alone), (B, i)
