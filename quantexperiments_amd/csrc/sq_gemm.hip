@@ -12,6 +12,7 @@
 //   B: col l % 32, k = 8 * (l / 32) .. + 7        (weight rows)
 //   D[v], v = 0..15: row 8 * (v / 4) + 4 * (l / 32) + v % 4, col l % 32
 #include <algorithm>
+#include <cmath>
 #include "sq_common.h"
 
 namespace sq {
@@ -310,16 +311,35 @@ size_t small_gemm_route_workspace(const sq_matrix* mats, int n, int B) {
     return masked_gemm(mats, n, B) ? gemm_workspace(mats, n, B) : 0;
 }
 
+// What a piece takes on the vector kernel, in microseconds: columns one behind the other in a lane, and weights over the chip, both per pass of
+// four rows and slower the less the caches near a CU hold of the codebook.  Fitted to 27 eager calls of 256, 2048 and 16384 rows of 512 to
+// 1544 columns, 6-, 14- and 16-bit tags, at 3 to 6 activation rows (most within 15 %).
+static double vector_us(const sq_matrix& m, int B) {
+    const double columns = m.C * 1e-3, weights = m.R * columns * 1e-3, table = ((double)m.G * m.d * 2) * ((int64_t)1 << m.bits);
+    const int passes = (B + 3) / 4;
+    if (table <= 32 * 1024) return 4.5 + std::hypot((1.25 * B + 3.1 * (passes - 1)) * columns, 2.2 * passes * weights);
+    return (table > 512 * 1024 ? 7.5 : 5.5) + std::hypot((2.2 * B + 2.4 * (passes - 1)) * columns, 4.2 * passes * weights);
+}
+
 // Without orders: how many pieces, the first one on, are decoded and multiplied from there at B rows because the decode-time product would
-// run them on the vector kernels (16-bit tags of rows that end within a lane unit, tags of other widths, codebooks beyond LDS), which
-// take every few rows as long again: from VECTOR_DECODED_B rows (5120 x 2080, 16-bit tags, at 16 / 32 rows 212 / 415 us there, 24 / 25
-// here).  Their neighbours in the stack keep their kernels, which read tags.
+// run them on the vector kernel (16-bit tags of rows that end within a lane unit, tags of other widths, codebooks beyond LDS), which
+// takes every few rows as long again: from VECTOR_DECODED_B rows, where the decode, a product and a sum of slices take less (vector
+// kernel / decoded, us at 3 / 4 / 5 rows: 5120 x 2080, 16-bit tags, 58 / 66 / 107 and 24 at any; 300 x 2080 21 / 25 / 36, 14; 512 x 1024,
+// 14-bit tags of width 4, 10.8 / 12.5 / 18.2, 17.7; 4864 x 896, 6-bit, 13.8 / 15.8 / 21.5, 20; 2048 x 512, 6-bit, 7.9 / 8.0 / 9.7, 17; 16384 x
+// 512 23 / 27 / 36, 20).  Their neighbours in the stack keep their kernels, which read tags.
 constexpr int VECTOR_DECODED_B = 3;
 int vector_decoded(const sq_matrix* mats, int n, int B) {
     if (B < VECTOR_DECODED_B) return 0;
-    int k = 0, found = 0;
-    for (; k < n && (mats[k].R == 0 || (small_vector(mats[k], B) && mid_dense_ok(mats + k, 1, B))); ++k) found += mats[k].R > 0;
-    return found ? k : 0;
+    int k = 0;
+    double vector = 0.0, decoded = 0.0;
+    for (; k < n; ++k) {
+        const sq_matrix& m = mats[k];
+        if (m.R == 0) continue;
+        if (!small_vector(m, B) || !mid_dense_ok(&m, 1, B)) break;
+        vector += vector_us(m, B);
+        decoded += (decoded > 0.0 ? 3.0 : m.d == 8 ? 13.5 : 16.5) + 0.7e-6 * m.R * m.C;
+    }
+    return vector > decoded ? k : 0;
 }
 
 static size_t gemm_workspace_beyond_small(const sq_matrix* mats, int n, int T);

@@ -196,6 +196,11 @@ def test_mixed_stacks_decode_only_what_needs_it():
                 assert max(alone) <= need([large, small], B, which) < _lib.WS_HEADER + 32 * 18944 * B * 4 + (4 << 20)
                 assert need([large, small], B, which) == need([small, large], B, which) == need([large, small, mat(0, 3584, d, bits, 19008)], B, which)
     assert need([mat(64, 3584, 8, 14, 0)], 2, 0) == 0
+    # few short rows are through the vector kernel before a decode is: none of it is asked for
+    for R, C, d, bits, rows in ((512, 1024, 4, 14, 3), (512, 1024, 4, 14, 4), (2048, 512, 4, 6, 5), (4864, 896, 4, 6, 4), (256, 520, 8, 16, 4)):
+        assert need([mat(R, C, d, bits, 0)], rows, 0) == 0
+    for R, C, d, bits, rows in ((512, 1024, 4, 14, 6), (16384, 512, 4, 6, 4), (4864, 896, 4, 6, 8), (256, 2080, 8, 16, 3), (5120, 2080, 8, 16, 3)):
+        assert need([mat(R, C, d, bits, 0)], rows, 0) >= _lib.WS_HEADER + R * C * 2
 
 
 def test_tile_gemm_waits_for_its_reads_before_the_barrier(tmp_path):
