@@ -146,7 +146,10 @@ int launch_small(const sq_matrix* mats, int n, const void* x, int x_dtype, int64
 // one activation row of these pieces is a single launch of the tag-stream kernel, which can produce its own x
 int sieve_group(const sq_matrix* mats, int n, int T);
 size_t sieve_workspace(const sq_matrix* mats, int n, int T);
-int launch_sieve(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, hipStream_t s);
+// what launch_sieve can do with, in more launches: SIEVE_ROOM, which sq_linear_small_noalloc has, or less where there is less to keep
+constexpr size_t SIEVE_ROOM = (size_t)16 << 20;
+size_t sieve_workspace_least(const sq_matrix* mats, int n, int T);
+int launch_sieve(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, size_t ws_bytes, hipStream_t s);
 bool small_fuses_producer(const sq_matrix* mats, int n, int B);
 // the two pieces are a gate and an up projection whose launch can write SiLU(gate) * up itself
 bool small_fuses_silu(const sq_matrix* mats, int n, int B);

@@ -235,17 +235,12 @@ static int sieve_len(const sq_matrix* mats, int n, int B) {
     return sieve_group(mats, k, B);
 }
 
-// tight: the pieces that can run without partial sums or decoded weights do
-// (a group that sq_sieve.hip takes runs there unless the workspace is tight or x not aligned: then piece by piece as below)
-static size_t small_need(const sq_matrix* mats, int n, int B, bool tight, bool sieve = true) {
+// What the pieces' kernels keep side by side; not what a launch has from the workspace's first byte on for itself (small_workspace).
+// tight: the pieces that can run without partial sums do
+static size_t small_need(const sq_matrix* mats, int n, int B, bool tight) {
     size_t tot = 0;
     for (int i = 0; i < n; ++i) {
         if (stream_rows(mats[i], B)) continue;                   // its partial sums live in the workspace header
-        if (const int k = tight || !sieve ? 0 : sieve_len(mats + i, n - i, B); k > 0) {
-            tot += std::max(sieve_workspace(mats + i, k, B), small_need(mats + i, k, B, false, false));
-            i += k - 1;
-            continue;
-        }
         if (mma_rows(mats[i])) tot += tight && (mma_whole_row(mats[i], B).KW || mma_without_room(mats[i], B)) ? 0 : mma_part_bytes(mats[i], B);
         else if (mats[i].perms && fast_shape(mats[i])) tot += xp_bytes(mats[i], B);
     }
@@ -254,12 +249,16 @@ static size_t small_need(const sq_matrix* mats, int n, int B, bool tight, bool s
 
 size_t small_workspace(const sq_matrix* mats, int n, int B) {
     size_t need = small_need(mats, n, B, false);
-    if (has_orders(mats, n)) return need;
-    for (int i = 0; i < n; ++i)                                  // (decoded weights: a launch's own, from the workspace's first byte on)
-        if (const int k = vector_decoded(mats + i, n - i, B); k > 0) {
+    const bool orders = has_orders(mats, n);
+    for (int i = 0; i < n; ++i) {
+        if (const int k = orders ? 0 : vector_decoded(mats + i, n - i, B); k > 0) {
             need = std::max(need, decoded_workspace(mats + i, k, B));
             i += k - 1;
+        } else if (const int k = sieve_len(mats + i, n - i, B); k > 0) {
+            need = std::max(need, sieve_workspace(mats + i, k, B));
+            i += k - 1;
         }
+    }
     return need;
 }
 size_t small_workspace_least(const sq_matrix* mats, int n, int B) { return small_need(mats, n, B, true); }
@@ -439,9 +438,9 @@ int launch_small(const sq_matrix* mats, int n, const void* x, int x_dtype, int64
             i += k;
             continue;
         }
-        if (const int k = tight || !x_ok ? 0 : sieve_len(mats + i, n - i, B); k > 0) {
-            if (const int rc = launch_sieve(mats + i, k, x, x_dtype, ldx, y, y_dtype, ldy, B, (char*)ws + ws_off, s)) return rc;
-            ws_off += std::max(sieve_workspace(mats + i, k, B), small_need(mats + i, k, B, false, false));       // (what was counted for them)
+        if (const int k = !x_ok ? 0 : sieve_len(mats + i, n - i, B); k > 0 && sieve_workspace_least(mats + i, k, B) <= ws_bytes) {
+            if (const int rc = launch_sieve(mats + i, k, x, x_dtype, ldx, y, y_dtype, ldy, B, ws, ws_bytes, s)) return rc;
+            ws_off += small_need(mats + i, k, B, tight);         // (what was counted for them)
             i += k;
             continue;
         }

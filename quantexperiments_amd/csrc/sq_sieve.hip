@@ -244,14 +244,14 @@ static int sieve_jobs(const sq_matrix* mats, int n, int tw) {
 
 // The plan of least estimated time, in microseconds: rounds of workgroups over the CUs, each the slice's way to LDS and its steps, and
 // the partial sums, written and read back.  Fitted to 25 plans of the products above (within 10 %); the best of them fill the
-// chip once with the fewest K slices.
-static SievePlan sieve_plan(const sq_matrix* mats, int n, int T, int cus) {
+// chip once with the fewest K slices.  (slices: the number of K slices, if it is given)
+static SievePlan sieve_plan(const sq_matrix* mats, int n, int T, int cus, int slices = 0) {
     const int NP = ((mats[0].C / 64 + 3) / 4 + 1) / 2;                       // pairs of rounds
     int64_t rows = 0;
     for (int i = 0; i < n; ++i) rows += mats[i].R;
     SievePlan best{2, 1, 1e30};
     for (int tw = 2; tw <= SIEVE_TW; ++tw)                                   // (one tile a wave: next to never the best of what pays)
-        for (int ks = 1; ks <= std::min(NP, 8); ++ks) {
+        for (int ks = slices ? slices : 1; ks <= (slices ? slices : std::min(NP, 8)); ++ks) {
             const int64_t jobs = (int64_t)sieve_jobs(mats, n, tw) * ks, rounds = (jobs * SIEVE_SLICES + cus - 1) / cus;
             const int steps = (NP + ks - 1) / ks * 16;
             const double us = 3.2 + rounds * (4.4 + steps * (0.02 + 0.07 * tw)) + 32.0 * ks * T * rows / 2.74e6;
@@ -260,14 +260,15 @@ static SievePlan sieve_plan(const sq_matrix* mats, int n, int T, int cus) {
     return best;
 }
 
-static size_t sieve_part_bytes(const sq_matrix& m, int T, int ks) { return ((size_t)SIEVE_SLICES * ks * T * m.R * 4 + 255) & ~(size_t)255; }
+static size_t sieve_part_bytes(int R, int T, int ks) { return ((size_t)SIEVE_SLICES * ks * T * R * 4 + 255) & ~(size_t)255; }
 
 size_t sieve_workspace(const sq_matrix* mats, int n, int T) {
     const SievePlan pl = sieve_plan(mats, n, T, device_cus());
     size_t need = 0;
-    for (int i = 0; i < n; ++i) need += sieve_part_bytes(mats[i], T, pl.ks);
+    for (int i = 0; i < n; ++i) need += sieve_part_bytes(mats[i].R, T, pl.ks);
     return need;
 }
+size_t sieve_workspace_least(const sq_matrix* mats, int n, int T) { return std::min(sieve_workspace(mats, n, T), SIEVE_ROOM); }
 
 // How many of the n pieces, the first one on, the kernel takes in one launch, 0 where the gathers from L2 are the faster way: they
 // take 4.6 us per million tags and 4 more, 1.1 to 1.3 times that for rows of more than 8192 columns (4096 x 4096 at 9 / 16 rows 15.5 /
@@ -280,7 +281,10 @@ int sieve_group(const sq_matrix* mats, int n, int T) {
     return k && sieve_plan(mats, k, T, device_cus()).us < 0.92 * (4.0 + 4.6 * tags) ? k : 0;
 }
 
-int launch_sieve(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, hipStream_t s) {
+// Rows of all pieces, or, where their partial sums do not fit the workspace, as many at a time as do, evenly cut (2 x 18944 x 3584 at 16
+// rows in two launches 75 us, in one 58, through the gathers from L2 85; 60001 x 4160, which fills the chip anyway, level).  A row's sums depend on the K slices alone, which are those of the whole product: the results are the
+// same bits either way.
+int launch_sieve(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, size_t ws_bytes, hipStream_t s) {
     typedef void (*kernel_t)(SieveArgs);
     static constexpr kernel_t kernels[SIEVE_TW - 1] = {sieve_kernel<2>, sieve_kernel<3>, sieve_kernel<4>, sieve_kernel<5>};
     static const bool raised = [] {
@@ -289,18 +293,40 @@ int launch_sieve(const sq_matrix* mats, int n, const void* x, int x_dtype, int64
         return true;
     }();
     (void)raised;
-    const SievePlan pl = sieve_plan(mats, n, T, device_cus());
-    SieveArgs a{};
-    a.x = (const uint16_t*)x; a.ldx = ldx; a.n = n; a.T = T; a.U = mats[0].C / 64; a.ks = pl.ks; a.bf = x_dtype == SQ_BF16;
-    char* part = (char*)ws;
-    for (int i = 0; i < n; ++i) {
-        a.p[i] = {mats[i], (float*)part, a.jobs};
-        part += sieve_part_bytes(mats[i], T, pl.ks);
-        a.jobs += (mats[i].R + SIEVE_ROWS * pl.tw - 1) / (SIEVE_ROWS * pl.tw) * pl.ks;
+    const SievePlan whole = sieve_plan(mats, n, T, device_cus());
+    int64_t rows = 0;
+    for (int i = 0; i < n; ++i) rows += mats[i].R;
+    int64_t most = rows;                     // rows of a launch
+    if (sieve_workspace(mats, n, T) > ws_bytes) {
+        const int64_t fit = (int64_t)((ws_bytes - std::min(ws_bytes, (size_t)256 * n)) / ((size_t)SIEVE_SLICES * whole.ks * T * 4)) / 16 * 16;
+        const int64_t launches = (rows + fit - 1) / fit;
+        most = std::min(fit, ((rows + launches - 1) / launches + 15) / 16 * 16);
     }
-    hipLaunchKernelGGL(kernels[pl.tw - 2], dim3((unsigned)((a.jobs + 7) / 8 * 64)), dim3(64 * SIEVE_WAVES), (size_t)SIEVE_X + 2 * SIEVE_STAGE, s, a);
-    if (const int rc = check_launch("sq_linear_small(sieve)")) return rc;
-    return launch_slice_sum(a.p, n, SIEVE_SLICES * pl.ks, T, y, y_dtype, ldy, s);
+    for (int i = 0, r0 = 0; i < n;) {
+        sq_matrix part[MID_PIECES];
+        int k = 0;
+        for (int64_t left = most; i < n && left > 0;) {
+            const int R = (int)std::min<int64_t>(mats[i].R - r0, left);
+            sq_matrix& m = part[k++] = mats[i];
+            m.R = R; m.tags += (int64_t)r0 * m.W; m.row_scale += r0; m.y_off += r0;
+            left -= R;
+            r0 += R;
+            if (r0 >= mats[i].R) ++i, r0 = 0;
+        }
+        const SievePlan pl = most == rows ? whole : sieve_plan(part, k, T, device_cus(), whole.ks);
+        SieveArgs a{};
+        a.x = (const uint16_t*)x; a.ldx = ldx; a.n = k; a.T = T; a.U = mats[0].C / 64; a.ks = pl.ks; a.bf = x_dtype == SQ_BF16;
+        char* sums = (char*)ws;
+        for (int j = 0; j < k; ++j) {
+            a.p[j] = {part[j], (float*)sums, a.jobs};
+            sums += sieve_part_bytes(part[j].R, T, pl.ks);
+            a.jobs += (part[j].R + SIEVE_ROWS * pl.tw - 1) / (SIEVE_ROWS * pl.tw) * pl.ks;
+        }
+        hipLaunchKernelGGL(kernels[pl.tw - 2], dim3((unsigned)((a.jobs + 7) / 8 * 64)), dim3(64 * SIEVE_WAVES), (size_t)SIEVE_X + 2 * SIEVE_STAGE, s, a);
+        if (const int rc = check_launch("sq_linear_small(sieve)")) return rc;
+        if (const int rc = launch_slice_sum(a.p, k, SIEVE_SLICES * pl.ks, T, y, y_dtype, ldy, s)) return rc;
+    }
+    return SQ_OK;
 }
 
 }  // namespace sq

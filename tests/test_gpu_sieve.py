@@ -89,3 +89,25 @@ def test_a_codeword_that_is_not_finite():
     ok = torch.isfinite(want)
     assert torch.equal(torch.isfinite(y), ok)
     assert ((y - want).abs()[ok] < 1e-5 * want[ok].abs().max()).all()
+
+
+@pytest.mark.parametrize("rows,C,T", [((18944, 18944), 3584, 16), ((18945, 3, 18946), 3584, 14), ((36000,), 3648, 16), ((60001,), 4160, 13)])
+def test_sums_that_do_not_fit_at_once(rows, C, T):
+    """Rows a part at a time, in the workspace there is: the bits of the whole product, through the entry point that has 16 MB behind its
+    header as well."""
+    lins, w = _pieces(rows, C)
+    mats = _lib.matrix_array([m.descriptor(sum(rows[:i])) for i, m in enumerate(lins)])
+    room = 16 << 20
+    assert _lib.lib().sq_workspace_bytes(mats, len(lins), T, 2) > room
+    x = rand_x(T, C, torch.bfloat16, seed=T)
+    x[2, 5] = float("inf")
+    x = x.cuda()
+    y, z = (torch.full((T, sum(rows)), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    linear_small(lins, x, y)
+    _lib.check(_lib.lib().sq_linear_small_noalloc(mats, len(lins), x.data_ptr(), _lib.SQ_BF16, C, z.data_ptr(), _lib.SQ_BF16, sum(rows), T, _lib.stream_ptr(x.device)))
+    assert torch.equal(y.view(torch.int16), z.view(torch.int16))
+    z.fill_(float("nan"))
+    _call(lins, x, z, torch.empty(room, dtype=torch.uint8, device="cuda"))
+    assert torch.equal(y.view(torch.int16), z.view(torch.int16))
+    ok = [t for t in range(T) if t != 2]
+    assert rel_max_err(y[ok].float().cpu().numpy(), (x[ok].half().double() @ w.T).cpu().numpy()) < 2.0 ** -8 + 1e-5
