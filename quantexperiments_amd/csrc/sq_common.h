@@ -109,13 +109,16 @@ template <int N> __device__ __forceinline__ float row_rotated(float v) {
     const int i = __builtin_bit_cast(int, v);
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, 0x120 + N, 0xF, 0xF, false));
 }
-__device__ __forceinline__ float wave_sum(float v) {
+__device__ __forceinline__ float lane_groups_sum(float v) {        // over lanes 16 apart
     const uint32_t a = __builtin_bit_cast(uint32_t, v);
     const auto h = __builtin_amdgcn_permlane32_swap(a, a, false, false);
     v = __builtin_bit_cast(float, (uint32_t)h[0]) + __builtin_bit_cast(float, (uint32_t)h[1]);
     const uint32_t b = __builtin_bit_cast(uint32_t, v);
     const auto r = __builtin_amdgcn_permlane16_swap(b, b, false, false);
-    v = __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
+    return __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
+}
+__device__ __forceinline__ float wave_sum(float v) {
+    v = lane_groups_sum(v);
     v += row_rotated<8>(v); v += row_rotated<4>(v); v += row_rotated<2>(v);
     return v + row_rotated<1>(v);
 }

@@ -304,6 +304,75 @@ void rows_mfma_kernel(MmaArgs a) {
         stage_table(m.table, a.table_bytes, smem);
     }
     if (BROKEN && tid < 4) reinterpret_cast<uint32_t*>(smem + a.table_bytes)[tid] = 0u;
+    // BROKEN: such rows ran on the vector kernel, which multiplies bf16 in fp32: a token's bf16 activations whose fp16 values would not be
+    // theirs (beyond 65,504), or would lose bits that matter (a mean square below 2^-13, of which values below 2^-17 are no longer a
+    // negligible part), are taken again here, straight into the operands, times a power of two that the sums are divided by.  (The sum of
+    // squares of the fp16 values says which: a dot product per pair of them, while the codebook is on its way; 5120 x 2064 at 2 / 16 / 32 rows
+    // 6.8 / 7.4 / 10.4 us without, 7.0 / 7.6 / 11.0 so.)
+    int xexp[NT];
+    bool scaled = false;
+    if constexpr (BROKEN) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) xexp[nt] = 0;
+        if (a.x_dtype == SQ_BF16) {
+            const float least = (float)min(RW * 4 * UK, m.C - 4 * rbase * UK) * 0x1p-13f;      // (not positive: a wave without columns)
+            bool odd = false;
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                float part[4] = {};                              // (a chain each)
+#pragma unroll
+                for (int n = 0; n < RW; ++n)
+#pragma unroll
+                    for (int s = 0; s < SPU; ++s)
+#pragma unroll
+                        for (int e = 0; e < 8; e += 2) {
+                            const half2v h = {xb[n][s][nt][e], xb[n][s][nt][e + 1]};
+                            part[e >> 1] = __builtin_amdgcn_fdot2(h, h, part[e >> 1], false);
+                        }
+                __builtin_amdgcn_sched_barrier(0);
+                const float sq = lane_groups_sum((part[0] + part[1]) + (part[2] + part[3]));
+                odd = odd || (nt * 16 + li < a.B && least > 0.f && !(sq >= least && sq < __builtin_inff()));
+            }
+            scaled = __any((int)odd) != 0;
+        }
+        if (__builtin_expect(scaled, 0)) {
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                const uint16_t* xr = a.x + (int64_t)min(nt * 16 + li, a.B - 1) * a.ldx;
+                int first = 4 * rbase * UK + lg * UK;
+                auto raw = [&](int n, int s) {
+                    const bool real = live[n] && s * 8 < cols[n] && nt * 16 + li < a.B;
+                    const u32x4 v = *reinterpret_cast<const u32x4*>(xr + (real ? first + 4 * n * UK + s * 8 : 0));
+                    return real ? v : u32x4{0u, 0u, 0u, 0u};
+                };
+                uint32_t top = 0u;                               // the largest magnitude of this token's columns, as bf16 bits
+#pragma unroll
+                for (int n = 0; n < RW; ++n)
+#pragma unroll 1
+                    for (int s = 0; s < SPU; ++s) {
+                        const u32x4 v = raw(n, s);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) top = max(top, max(v[e] & 0x7FFFu, (v[e] >> 16) & 0x7FFFu));
+                    }
+                top = max(top, (uint32_t)__shfl_xor((int)top, 16, 64));
+                top = max(top, (uint32_t)__shfl_xor((int)top, 32, 64));
+                // the largest one to 2^12 .. 2^13 (what is 2^-29 of it and more keeps all its bits); infinities and NaN stay what they are
+                xexp[nt] = max((int)min(top >> 7, 254u) - (127 + 12), -64);
+                const float by = __builtin_bit_cast(float, (uint32_t)(127 - xexp[nt]) << 23);
+#pragma unroll
+                for (int n = 0; n < RW; ++n)
+#pragma unroll
+                    for (int s = 0; s < SPU; ++s) {
+                        const u32x4 v = raw(n, s);
+                        u32x4 h;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) h[e] = f2h_x2(bf2f((uint16_t)(v[e] & 0xFFFFu)) * by, bf2f((uint16_t)(v[e] >> 16)) * by);
+                        xb[n][s][nt] = __builtin_bit_cast(half8v, h);
+                        asm volatile("" : "+v"(first) : "v"(h));  // (one load at a time: there are no registers for more)
+                    }
+            }
+        }
+    }
     SQ_TRACE_POINT(1);
     // every wave has taken its operands out of the staging area (and, with the codebook in LDS, the codebook has landed
     // and the first tile's tags with it)
@@ -358,6 +427,12 @@ void rows_mfma_kernel(MmaArgs a) {
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
                 acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, xb[n][s][nt], acc[nt], 0, 0, 0);
+        }
+        if (BROKEN && __builtin_expect(scaled, 0)) {
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc[nt][v] = __builtin_ldexpf(acc[nt][v], xexp[nt]);
         }
     };
 

@@ -185,3 +185,49 @@ def test_mixed_stacks(d, bits, stream, noalloc):
             alone = torch.empty(B, formats[i][0], device="cuda")
             linear_small([lins[i]], x, alone)
             assert torch.equal(y[:, o:o + formats[i][0]], alone), (B, i)
+
+
+def _wide_activations(B, C, seed):
+    """bf16 rows that fp16 does not hold: far below its normal range, far beyond its largest value, a few of those among ordinary ones, at
+    the row's end alone, one ordinary value among tiny ones, all zero."""
+    x = rand_x(B, C, torch.bfloat16, seed=seed).float()
+    for b in range(B):
+        kind = b % 8
+        if kind == 1: x[b] *= 1e-7
+        if kind == 2: x[b, 5], x[b, C // 2], x[b, C - 9] = 1e5, -3e6, 70000.0
+        if kind == 3: x[b] *= 1e28
+        if kind == 4: x[b] = 0.0
+        if kind == 5: x[b] = 0.0; x[b, C - 1] = 2e5
+        if kind == 6: x[b] *= 2.0 ** -20; x[b, 11] = 1.0
+        if kind == 7: x[b] *= 3e-13; x[b, C // 3] = 4e-12
+    return x.to(torch.bfloat16)
+
+
+def _check_wide_activations(lins, w, C, rows):
+    for B in rows:
+        x = _wide_activations(B, C, seed=B)
+        y = torch.full((B, w.shape[0]), float("nan"), device="cuda")
+        linear_small(lins, x.cuda(), y)
+        y, ref = y.cpu().double().numpy(), x.double().numpy() @ w.T
+        # (sums of products that are exact in 32 bits or below 2^-24 of the largest one: as for ordinary activations)
+        for b in range(B):
+            assert np.abs(y[b] - ref[b]).max() <= 1e-5 * np.abs(ref[b]).max(), (B, b)
+        # what is not finite, beside finite values that fp16 does not hold
+        x[0, 3], x[0, 9] = float("inf"), 1e6
+        x[B - 1, C - 2] = float("nan")
+        y = torch.zeros(B, w.shape[0], device="cuda")
+        linear_small(lins, x.cuda(), y)
+        with np.errstate(invalid="ignore"):
+            ref = x.double().numpy() @ w.T
+        y = y.cpu().double().numpy()
+        for b in {0, B - 1}:
+            assert np.array_equal(np.isnan(y[b]), np.isnan(ref[b])) and np.array_equal(np.isposinf(y[b]), np.isposinf(ref[b])) and \
+                np.array_equal(np.isneginf(y[b]), np.isneginf(ref[b])), (B, b)
+
+
+@pytest.mark.parametrize("rows,C,bits,G", [((100, 7), 2056, 12, 1), ((70,), 904, 8, 1), ((70,), 1000, 10, 4), ((33,), 9224, 12, 1), ((33,), 5672, 12, 4), ((20,), 40, 12, 1)])
+def test_activations_beyond_fp16_of_broken_rows(rows, C, bits, G):
+    """Rows that end within a lane unit: bf16 activations keep their range and their bits."""
+    ss = [synth(R, C, 4, bits, G, 1, seed=R) for R in rows]
+    lins = [to_device(s) for s in ss]
+    _check_wide_activations(lins, np.concatenate([s.decode() for s in ss]).astype(np.float64), C, (1, 2, 7, 9, 16, 17, 32))
