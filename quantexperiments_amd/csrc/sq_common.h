@@ -105,9 +105,11 @@ __device__ __forceinline__ uint32_t tag_at(const uint32_t* __restrict__ row, int
 // Sum over the wave, the same in every lane: v += v of lane ^ 32, then ^ 16, 8, 4, 2, 1.  In registers: swaps of half waves and of
 // rows of 16 lanes, and rotations of a row, whose values repeat every 8, 4, 2 lanes by the time they are rotated by 4, 2, 1 (through
 // __shfl_xor, six LDS round trips one behind the other, an add + norm of 8 x 3584 took 0.3 us more).
+template <int N> __device__ __forceinline__ uint32_t row_rotated_bits(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x120 + N, 0xF, 0xF, false);
+}
 template <int N> __device__ __forceinline__ float row_rotated(float v) {
-    const int i = __builtin_bit_cast(int, v);
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, 0x120 + N, 0xF, 0xF, false));
+    return __builtin_bit_cast(float, row_rotated_bits<N>(__builtin_bit_cast(uint32_t, v)));
 }
 __device__ __forceinline__ float lane_groups_sum(float v) {        // over lanes 16 apart
     const uint32_t a = __builtin_bit_cast(uint32_t, v);
@@ -173,7 +175,9 @@ constexpr int MID_PIECES = 8;          // (kernel arguments of 1 KB)
 bool small_vector(const sq_matrix& m, int B);
 int vector_decoded(const sq_matrix* mats, int n, int B);
 size_t decoded_workspace(const sq_matrix* mats, int n, int T);
-int launch_decoded(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, hipStream_t s);
+// (wide: bf16 activations keep their range and bits, up to 48 rows)
+int launch_decoded(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, hipStream_t s,
+                   bool wide = false);
 // 33 .. a few hundred activation rows in one pass over the tags (sq_mid.h): whether these pieces can take it, and its call
 bool mma_shape(const sq_matrix& m);
 bool mid_ok(const sq_matrix* mats, int n, int T);
@@ -184,7 +188,7 @@ int launch_mid(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t
 bool mid_dense_ok(const sq_matrix* mats, int n, int T);
 size_t mid_dense_workspace(const sq_matrix* mats, int n, int T);
 int launch_mid_decoded(const sq_matrix* mats, int n, const void* const* w, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T,
-                       void* ws, hipStream_t s);
+                       void* ws, hipStream_t s, bool wide);
 // more rows in tiles whose weights are gathered on their way into LDS (sq_fused.h)
 bool fused_route(const sq_matrix* mats, int n, int T);
 size_t fused_workspace(const sq_matrix* mats, int n, int T);

@@ -271,7 +271,7 @@ size_t decoded_workspace(const sq_matrix* mats, int n, int T) {
     return need;
 }
 
-int launch_decoded(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, hipStream_t s) {
+int launch_decoded(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, hipStream_t s, bool wide) {
     int rows = T;                                                // activation rows at a time: all, unless they span 4 GB
     while (rows > 1 && !mid_x_ok(ldx, rows)) rows = (rows + 1) / 2;
     for (int i = 0, r0 = 0; i < n;) {
@@ -285,7 +285,7 @@ int launch_decoded(const sq_matrix* mats, int n, const void* x, int x_dtype, int
         }
         for (int t = 0; d.n && t < T; t += rows)
             if (const int rc = launch_mid_decoded(d.m, d.n, w, (const char*)x + (size_t)t * ldx * 2, x_dtype, rows > 1 ? ldx : mats[0].C,
-                                                  (char*)y + (size_t)t * ldy * (y_dtype == SQ_F32 ? 4 : 2), y_dtype, ldy, std::min(rows, T - t), next, s))
+                                                  (char*)y + (size_t)t * ldy * (y_dtype == SQ_F32 ? 4 : 2), y_dtype, ldy, std::min(rows, T - t), next, s, wide))
                 return rc;
     }
     return SQ_OK;

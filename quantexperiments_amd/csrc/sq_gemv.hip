@@ -434,7 +434,7 @@ int launch_small(const sq_matrix* mats, int n, const void* x, int x_dtype, int64
             continue;
         }
         if (const int k = orders || !x_ok ? 0 : vector_decoded(mats + i, n - i, B); k > 0 && decoded_workspace(mats + i, k, B) <= ws_bytes) {
-            if (const int rc = launch_decoded(mats + i, k, x, x_dtype, ldx, y, y_dtype, ldy, B, ws, s)) return rc;
+            if (const int rc = launch_decoded(mats + i, k, x, x_dtype, ldx, y, y_dtype, ldy, B, ws, s, /*wide=*/true)) return rc;
             i += k;
             continue;
         }

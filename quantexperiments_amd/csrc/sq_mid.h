@@ -27,6 +27,12 @@
 // from there, up to seven steps ahead; step j of lane group g is columns 256 round + 32 j + 8 g .. + 7, so that the four lane groups
 // of a row read 64 neighbouring bytes.
 //
+// WIDE: bf16 activations keep their range and bits, for matrices that come here decoded because the vector kernel, which multiplies in
+// fp32, takes them four rows at a time.  A token's values go to LDS times a power of two chosen by the largest of its columns so far, 1 as long as
+// that is an ordinary one (2^-4 .. 65,504), else what makes it 2^12 .. 2^13; where the power changes the sums so far follow, at the end
+// they are divided by it.  Without branches, on whose account loads would be waited for (18944 x 3584, decode included, at 3 / 32 rows 71.4 / 74.7
+// us without, 72.4 / 75.9 so, 79.5 / 82 with a branch around what ordinary values can do without).
+//
 // An X row of a stage is 4 S pieces of 16 bytes; piece c of row t sits at slot c ^ h(t), with h such that the 16 lanes of an
 // LDS clock (rows 0-3, 12-15 of one lane group with rows 4-11 of the next, and so on) fall into 16 different groups of four
 // banks.
@@ -52,6 +58,7 @@ struct MidArgs {
     int64_t ldy;
     int T, x_dtype, y_dtype;
     int U, ks, table_bytes;
+    int wide;                    // 1: bf16 activations keep their range (WIDE; decoded weights, up to 48 activation rows)
 };
 
 template <int S> __device__ __forceinline__ int mid_swizzle(int t) {
@@ -61,8 +68,9 @@ template <int S> __device__ __forceinline__ int mid_swizzle(int t) {
 }
 
 constexpr int mid_stage_bytes(int NT, int S) { return NT * 16 * S * 64; }
+constexpr int mid_x_bytes(int NT, int S, bool wide) { return 2 * (mid_stage_bytes(NT, S) + (wide ? NT * 64 : 0)); }     // (WIDE: the stages' powers behind)
 
-template <int BITS, int D, int NT, int TW, int S, int NW, bool BF>
+template <int BITS, int D, int NT, int TW, int S, int NW, bool BF, bool WIDE = false>
 __global__ __launch_bounds__(64 * NW, 2) void mid_kernel(MidArgs a) {
     constexpr bool DENSE = D == 0;
     constexpr int UD = DENSE ? 1 : unit_of<DENSE ? 16 : BITS>::UD, TPU = DENSE ? 1 : UD * 32 / (DENSE ? 1 : BITS);
@@ -123,12 +131,31 @@ __global__ __launch_bounds__(64 * NW, 2) void mid_kernel(MidArgs a) {
 #pragma unroll
         for (int k = 0; k < PCS; ++k) px[k] = *reinterpret_cast<const u32x4*>(base + (xo[k] - (uint32_t)(max(xg[k] - left, 0) * (UK * 2))));
     };
+    static_assert(!WIDE || (BF && 4 * S == 16), "a token's pieces of a stage are those of a row of 16 lanes");
+    int* xpow = reinterpret_cast<int*>(xbuf + 2 * STAGE);                    // [2][NT * 16]
+    float top[PCS] = {};                                                     // WIDE: the largest magnitude of the piece's token so far
     auto store_x = [&](const u32x4* px, int buf, int round, int st) {
         const int units = round < r1 ? a.U - UPR * round - st * UPS : 0;
 #pragma unroll
         for (int k = 0; k < PCS; ++k) {
             u32x4 v = px[k];
-            if constexpr (BF) { v.x = bf2h_x2(v.x); v.y = bf2h_x2(v.y); v.z = bf2h_x2(v.z); v.w = bf2h_x2(v.w); }
+            if constexpr (WIDE) {
+                float f[8], mag = 0.f;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (xg[k] >= units) v[e] = 0u;
+                    f[2 * e] = bf2f((uint16_t)(v[e] & 0xFFFFu)); f[2 * e + 1] = bf2f((uint16_t)(v[e] >> 16));
+                    mag = fmaxf(mag, fmaxf(fabsf(f[2 * e]), fabsf(f[2 * e + 1])));
+                }
+                mag = fmaxf(mag, row_rotated<8>(mag)); mag = fmaxf(mag, row_rotated<4>(mag));
+                mag = fmaxf(mag, row_rotated<2>(mag)); mag = fmaxf(mag, row_rotated<1>(mag));
+                top[k] = fmaxf(top[k], mag);
+                const int exponent = (int)min(__builtin_bit_cast(uint32_t, top[k]) >> 23, 254u) - 127, power = exponent >= -4 && exponent <= 15 ? 0 : max(exponent - 12, -64);
+                const float by = __builtin_bit_cast(float, (uint32_t)(127 - power) << 23);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = f2h_x2(f[2 * e] * by, f[2 * e + 1] * by);
+                if ((tid & 15) == 0 && ((NT * 64 * S) % NTH == 0 || tid + NTH * k < NT * 64 * S)) xpow[buf * (NT * 16) + (tid + NTH * k) / 16] = power;
+            } else if constexpr (BF) { v.x = bf2h_x2(v.x); v.y = bf2h_x2(v.y); v.z = bf2h_x2(v.z); v.w = bf2h_x2(v.w); }
             const uint32_t keep = xg[k] < units ? 0xFFFFFFFFu : 0u;
             v.x &= keep; v.y &= keep; v.z &= keep; v.w &= keep;
             if ((NT * 64 * S) % NTH == 0 || tid + NTH * k < NT * 64 * S) *reinterpret_cast<u32x4*>(xbuf + buf * STAGE + xl[k]) = v;
@@ -162,6 +189,13 @@ __global__ __launch_bounds__(64 * NW, 2) void mid_kernel(MidArgs a) {
     for (int i = 0; i < TW; ++i)
 #pragma unroll
         for (int n = 0; n < NT; ++n) acc[i][n] = float4v{0.f, 0.f, 0.f, 0.f};
+    int power[NT] = {};                                                      // WIDE: of this lane's activation rows
+    auto times = [&](int n, int by) {
+#pragma unroll
+        for (int i = 0; i < TW; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[i][n][e] = __builtin_ldexpf(acc[i][n][e], by);
+    };
 
     // Two of everything that is on its way: tags of this round and the next, activations of the next stage and the one after.
     // A pair's members swap by the parity of the round (the loop is unrolled twice), never by moving registers, which would
@@ -190,7 +224,21 @@ __global__ __launch_bounds__(64 * NW, 2) void mid_kernel(MidArgs a) {
 #pragma unroll
                 for (int n = 0; n < NT; ++n) f[n] = *reinterpret_cast<const half8v*>(xs + n * (16 * ROWB));
             };
+            int now[NT] = {};
+            if constexpr (WIDE) {
+#pragma unroll
+                for (int n = 0; n < NT; ++n) now[n] = xpow[q * (NT * 16) + n * 16 + li];
+            }
             if (XB == 2) read_x(xf[0], 0);
+            if constexpr (WIDE) {
+                bool same = true;
+#pragma unroll
+                for (int n = 0; n < NT; ++n) same = same && now[n] == power[n];
+                if (__builtin_expect(!__all((int)same), 0)) {
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) { times(n, power[n] - now[n]); power[n] = now[n]; }
+                }
+            }
 #pragma unroll
             for (int j = 0; j < S; ++j) {
                 const int s = st * S + j;
@@ -218,6 +266,10 @@ __global__ __launch_bounds__(64 * NW, 2) void mid_kernel(MidArgs a) {
     }
 
     // ---- lane: activation row 16 n + li, weight rows 16 tile + 4 lg .. + 3
+    if constexpr (WIDE) {
+#pragma unroll
+        for (int n = 0; n < NT; ++n) times(n, power[n]);
+    }
     const bool vec = m.R % 4 == 0;
 #pragma unroll
     for (int i = 0; i < TW; ++i) {
@@ -254,20 +306,23 @@ __global__ __launch_bounds__(64 * NW, 2) void mid_kernel(MidArgs a) {
     }
 }
 
-template <int BITS, int D, int NT, int TW, int S, int NW, bool BF>
+template <int BITS, int D, int NT, int TW, int S, int NW, bool BF, bool WIDE = false>
 int launch_mid_dtype(const MidArgs& a, int grid, hipStream_t s) {
     static bool raised = false;
     if (!raised) {
-        (void)hipFuncSetAttribute((const void*)mid_kernel<BITS, D, NT, TW, S, NW, BF>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        (void)hipFuncSetAttribute((const void*)mid_kernel<BITS, D, NT, TW, S, NW, BF, WIDE>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         (void)hipGetLastError();
         raised = true;
     }
-    hipLaunchKernelGGL((mid_kernel<BITS, D, NT, TW, S, NW, BF>), dim3((unsigned)grid), dim3(64 * NW), (size_t)a.table_bytes + 2 * mid_stage_bytes(NT, S), s, a);
+    hipLaunchKernelGGL((mid_kernel<BITS, D, NT, TW, S, NW, BF, WIDE>), dim3((unsigned)grid), dim3(64 * NW), (size_t)a.table_bytes + mid_x_bytes(NT, S, WIDE), s, a);
     return check_launch("sq_linear_gemm(mid)");
 }
 
 template <int BITS, int D, int NT, int TW, int S, int NW>
 int launch_mid_as(const MidArgs& a, int grid, hipStream_t s) {
+    if constexpr (D == 0 && NT <= 3 && TW == 1) {
+        if (a.wide && a.x_dtype == SQ_BF16) return launch_mid_dtype<BITS, D, NT, TW, S, NW, true, true>(a, grid, s);
+    }
     return a.x_dtype == SQ_BF16 ? launch_mid_dtype<BITS, D, NT, TW, S, NW, true>(a, grid, s) : launch_mid_dtype<BITS, D, NT, TW, S, NW, false>(a, grid, s);
 }
 

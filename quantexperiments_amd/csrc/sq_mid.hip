@@ -93,12 +93,13 @@ size_t mid_workspace(const sq_matrix* mats, int n, int T) {
 }
 
 static int launch_mid_rows(const sq_matrix* mats, int n, const MidPlan& pl, const void* const* dense, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype,
-                           int64_t ldy, int T, void* ws, hipStream_t s) {
+                           int64_t ldy, int T, void* ws, hipStream_t s, bool wide = false) {
     MidArgs a{};
     const sq_matrix& m0 = mats[0];
     a.n = n;
     a.x = (const uint16_t*)x; a.ldx = ldx; a.y = y; a.ldy = ldy; a.T = T; a.x_dtype = x_dtype; a.y_dtype = y_dtype;
     a.U = dense ? m0.C / 8 : mid_units(m0); a.ks = pl.ks;
+    a.wide = wide;
     a.table_bytes = !dense && m0.d == 4 ? (m0.G << m0.bits) * 8 : 0;
     int wg = 0;
     char* part = (char*)ws;
@@ -151,8 +152,8 @@ size_t mid_dense_workspace(const sq_matrix* mats, int n, int T) {
 }
 
 int launch_mid_decoded(const sq_matrix* mats, int n, const void* const* w, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T,
-                       void* ws, hipStream_t s) {
-    return launch_mid_rows(mats, n, mid_dense_plan(mats, n, T, device_cus()), w, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);
+                       void* ws, hipStream_t s, bool wide) {
+    return launch_mid_rows(mats, n, mid_dense_plan(mats, n, T, device_cus()), w, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s, wide);
 }
 
 int launch_mid(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws,

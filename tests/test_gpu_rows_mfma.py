@@ -231,3 +231,12 @@ def test_activations_beyond_fp16_of_broken_rows(rows, C, bits, G):
     ss = [synth(R, C, 4, bits, G, 1, seed=R) for R in rows]
     lins = [to_device(s) for s in ss]
     _check_wide_activations(lins, np.concatenate([s.decode() for s in ss]).astype(np.float64), C, (1, 2, 7, 9, 16, 17, 32))
+
+
+@pytest.mark.parametrize("rows,C,d,bits,G", [((700, 9), 2080, 8, 16, 1), ((5000,), 5000, 8, 16, 1), ((900,), 1024, 8, 14, 1), ((2000,), 1024, 4, 14, 1), ((600,), 2056, 4, 12, 8),
+                                             ((4000,), 264, 8, 5, 1)])
+def test_activations_beyond_fp16_of_vector_formats(rows, C, d, bits, G):
+    """Formats without a matrix-core kernel, decoded first or not: bf16 activations keep their range and their bits."""
+    ss = [synth(R, C, d, bits, G, 1, seed=R) for R in rows]
+    lins = [to_device(s, stream=False) for s in ss]
+    _check_wide_activations(lins, np.concatenate([s.decode() for s in ss]).astype(np.float64), C, (1, 3, 8, 16, 17, 32))
