@@ -187,7 +187,7 @@ __global__ __launch_bounds__(256, 2) void q8_gemv_kernel(Q8Args a) {
 // l % 16, the same k; D: lane l holds token l % 16, weight rows 4 * (l / 16) .. + 3.  Weights are the A operand and a
 // wave owns 16 rows.  The rows reach the wave through LDS: global_load_lds (no registers in between) fetches them in
 // lane order ALONG the row, one instruction = 8 rows x 128 bytes, whole cache lines with 8 consecutive lanes per
-// line, into a private ring of D steps per wave (a step = 16 rows x 128 columns = 2 KB); the wave reads its
+// line, into a private ring of Q8_RING steps per wave (a step = 16 rows x 128 columns = 2 KB); the wave reads its
 // fragments back in the operand layout (lane (r, g) takes pieces 2 g and 2 g + 1 of row r, 32 bytes per step), so
 // the weights need no barrier, only counted waits.  Rows are XOR-swizzled in 16-byte pieces (piece p of row r at
 // slot p ^ ((r >> 1) & 7), applied through the source addresses of the copy), so the 16 lanes of an LDS read clock
@@ -231,14 +231,14 @@ struct Q8MfmaArgs {
 
 constexpr int q8_vmcnt(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }   // wait on vmcnt only
 
-// weights ring + scales of d - 1 chunks (with a ring of 4 steps the scales of chunk c + 2 are requested while chunk c
-// is still being multiplied)
+constexpr int Q8_RING = 3;                      // steps: one being multiplied, two in flight
+// weights ring + scales of two chunks
 enum { Q8_CHUNKS, Q8_PAIRS, Q8_ODD };       // rows of whole 256-column chunks, of whole pairs of blocks, of an odd number of blocks
 constexpr int q8l_scale_bytes(int rows) { return rows == Q8_ODD ? 512 : 256; }
-constexpr int q8l_wave_bytes(int d, int rows) { return d * 2048 + (d - 1) * q8l_scale_bytes(rows); }
-constexpr int q8l_lds_bytes(int nblk, int waves, int d, int xs, int rows) { return 2 * nblk * 16 * xs * 256 + waves * q8l_wave_bytes(d, rows); }
+constexpr int q8l_wave_bytes(int rows) { return Q8_RING * 2048 + 2 * q8l_scale_bytes(rows); }
+constexpr int q8l_lds_bytes(int nblk, int waves, int xs, int rows) { return 2 * nblk * 16 * xs * 256 + waves * q8l_wave_bytes(rows); }
 
-// NBLK 16-token blocks, WAVES waves per workgroup, ring of D steps per wave (one being multiplied, D - 1 in flight),
+// NBLK 16-token blocks, WAVES waves per workgroup,
 // x chunks of XS steps (128 XS columns; a copy moves 4 / XS tokens, so the first 4 NBLK XS waves make one of every chunk, or all
 // waves XI of them)
 // ROWS: Q8_PAIRS (C % 64 == 0) and Q8_ODD are rows that end within a chunk.  The steps behind the row's end copy its last pieces again and
@@ -266,17 +266,17 @@ __device__ __forceinline__ u32x4 q8_x_take() {
     return u32x4{v[0], v[1], v[2], v[3]};
 }
 constexpr int q8l_x_copies(int nblk, int waves, int xs) { return 4 * nblk * xs > waves ? 4 * nblk * xs / waves : 1; }
-template <int NBLK, int WAVES, int D, int XS, int ROWS, bool CVT, int XI = q8l_x_copies(NBLK, WAVES, XS)>
+template <int NBLK, int WAVES, int XS, int ROWS, bool CVT, int XI = q8l_x_copies(NBLK, WAVES, XS)>
 __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel(Q8MfmaArgs a) {
-    static_assert((D == 3 || (D == 4 && !CVT)) && (XS == 2 || (XS == 1 && D == 3)) && XI <= 4, "wait counts below are written out for these");
+    static_assert(Q8_RING == 3 && (XS == 1 || XS == 2) && XI <= 4, "wait counts below are written out for these");
     constexpr bool ANY_C = ROWS != Q8_CHUNKS;
-    constexpr int Q8L_D = D, Q8L_WAVE_BYTES = q8l_wave_bytes(D, ROWS), SB = q8l_scale_bytes(ROWS), SC = SB / 256;      // SC: copies of a chunk's scales
+    constexpr int Q8L_WAVE_BYTES = q8l_wave_bytes(ROWS), SB = q8l_scale_bytes(ROWS), SC = SB / 256;      // SC: copies of a chunk's scales
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     unsigned char* xs = smem;                                   // [2][16 NBLK tokens][256 XS bytes]
     constexpr int XPITCH = XS * 256, XBUF = NBLK * 16 * XPITCH;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     unsigned char* wl = smem + 2 * XBUF + wave * Q8L_WAVE_BYTES;  // this wave's ring
-    unsigned char* sl_ = wl + Q8L_D * 2048;                        // this wave's scales: [D - 1][16 rows][SB / 16 bytes]
+    unsigned char* sl_ = wl + Q8_RING * 2048;                      // this wave's scales: [2][16 rows][SB / 16 bytes]
     // the workgroups of the same weights are 8 apart: on one die, whose L2 the second finds them in
     const int tgroup = (blockIdx.x >> 3) % a.groups;
     const int task_raw = (int)((blockIdx.x >> 3) / a.groups * 8 + (blockIdx.x & 7)) * (int)(blockDim.x >> 6) + wave;
@@ -342,7 +342,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel
     auto copy_w = [&](int s) {
 #pragma unroll
         for (int n = 0; n < 2; ++n)
-            __builtin_amdgcn_global_load_lds((gptr_t)(wsrc[n] + (ANY_C ? min(s * 128 + wcol[n], C - 16) : s * 128)), (lptr_t)(wl + (s % Q8L_D) * 2048 + n * 1024), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((gptr_t)(wsrc[n] + (ANY_C ? min(s * 128 + wcol[n], C - 16) : s * 128)), (lptr_t)(wl + (s % Q8_RING) * 2048 + n * 1024), 16, 0, 0);
     };
     // scales of chunk c: lane i fetches dword i % 4 of row i / 4 (Q8_ODD: scale i % 8 of rows i / 8 and 8 + i / 8)
     const uint16_t* sodd[2];
@@ -353,10 +353,10 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel
         if constexpr (ROWS == Q8_ODD) {
 #pragma unroll
             for (int n = 0; n < 2; ++n)
-                __builtin_amdgcn_global_load_lds((gptr_t)(sodd[n] + min(c * 8 + (lane & 7), nblk - 1)), (lptr_t)(sl_ + (c % (D - 1)) * SB + n * 256), 2, 0, 0);
+                __builtin_amdgcn_global_load_lds((gptr_t)(sodd[n] + min(c * 8 + (lane & 7), nblk - 1)), (lptr_t)(sl_ + (c % 2) * SB + n * 256), 2, 0, 0);
             return;
         }
-        __builtin_amdgcn_global_load_lds((gptr_t)(ssrc + (ANY_C ? min(c * 16 + (lane & 3) * 4, nblk * 2 - 4) : c * 16)), (lptr_t)(sl_ + (c % (D - 1)) * SB), 4, 0, 0);
+        __builtin_amdgcn_global_load_lds((gptr_t)(ssrc + (ANY_C ? min(c * 16 + (lane & 3) * 4, nblk * 2 - 4) : c * 16)), (lptr_t)(sl_ + (c % 2) * SB), 4, 0, 0);
     };
     const uint32_t xrow = (uint32_t)r * XPITCH, xsw = (uint32_t)r;
     const uint32_t wsw = (uint32_t)((r >> 1) & 7);
@@ -368,9 +368,9 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel
 
     // Issue order per wave (X = this wave's x copy of a chunk, S = scales of a chunk, W = the 2 copies of a step):
     // S(c) goes right before W(2c); step s starts (even s: after the wait and the barrier, then X(s/2 + 1)) with the
-    // refill of step s + D - 1.  Waits count the operations that may stay in flight:
-    //   even s (needs X, S, W of its chunk):  D = 3: W(s+1) -> 2;           D = 4: W(s+1) S W(s+2) -> 4 + SC
-    //   odd s (needs W(s)):  D = 3: X S W(s+1) W(s+2) -> 4 + SC + x;  D = 4: S W(s+1) X W(s+2) S W(s+3) -> 6 + 2 SC + x   (x: this wave's XI copies)
+    // refill of step s + 2.  Waits count the operations that may stay in flight:
+    //   even s (needs X, S, W of its chunk):  W(s+1) -> 2
+    //   odd s (needs W(s)):  X S W(s+1) W(s+2) -> 4 + SC + x   (x: this wave's XI copies)
     // and fall back to "everything" near the end of the row, where refills stop.
     auto refill = [&](int f) {
         if (f < nsteps) {
@@ -380,12 +380,12 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel
     };
     copy_x(0);
 #pragma unroll
-    for (int t = 0; t < D - 1; ++t) refill(t);
+    for (int t = 0; t < Q8_RING - 1; ++t) refill(t);
     if constexpr (CVT) put_x(0, int_c<4 + SC>());
     // CVT: x of the next chunk, before the barrier that opens it.  Behind its load: the refills of the chunk's steps
     auto next_x = [&](int s) __attribute__((always_inline)) {
         if constexpr (CVT) {
-            const int cx = s / XS, f = s + D - 1;               // (f: the step that this one's refill was for)
+            const int cx = s / XS, f = s + Q8_RING - 1;               // (f: the step that this one's refill was for)
             if ((XS == 2 && !(s & 1)) || cx + 1 >= nchunks) return;
             if (f >= nsteps) put_x(cx + 1, int_c<0>());
             else if (XS == 2) put_x(cx + 1, int_c<4 + SC>());
@@ -407,30 +407,30 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel
             __builtin_amdgcn_s_barrier();
             __builtin_amdgcn_sched_barrier(0);
             if (cx + 1 < nchunks) copy_x(cx + 1);
-            refill(s + D - 1);
+            refill(s + Q8_RING - 1);
         } else if (!odd) {
-            if (s + D - 2 < nsteps) ready(int_c<D == 3 ? 2 : 4 + SC>());
+            if (s + 1 < nsteps) ready(int_c<2>());
             else ready(int_c<0>());
             __builtin_amdgcn_s_barrier();
             __builtin_amdgcn_sched_barrier(0);
             if (cx + 1 < nchunks) copy_x(cx + 1);
-            refill(s + D - 1);
+            refill(s + Q8_RING - 1);
         } else {
-            refill(s + D - 1);
-            if (s + D - 1 < nsteps) {
-                if (xo) __builtin_amdgcn_s_waitcnt(q8_vmcnt((D == 3 ? 4 + SC : 6 + 2 * SC) + XI));
-                else __builtin_amdgcn_s_waitcnt(q8_vmcnt(D == 3 ? 4 + SC : 6 + 2 * SC));
+            refill(s + Q8_RING - 1);
+            if (s + Q8_RING - 1 < nsteps) {
+                if (xo) __builtin_amdgcn_s_waitcnt(q8_vmcnt(4 + SC + XI));
+                else __builtin_amdgcn_s_waitcnt(q8_vmcnt(4 + SC));
             } else {
                 __builtin_amdgcn_s_waitcnt(q8_vmcnt(0));
             }
         }
         __builtin_amdgcn_sched_barrier(0);
-        const unsigned char* st = wl + (s % Q8L_D) * 2048;
+        const unsigned char* st = wl + (s % Q8_RING) * 2048;
         if constexpr (ANY_C) {
             typedef std::conditional_t<ROWS == Q8_ODD, u32x4, u32x2> scales_t;
             scales_t sb[4];                                     // the four blocks' scales of this lane's four output rows
 #pragma unroll
-            for (int v = 0; v < 4; ++v) sb[v] = *reinterpret_cast<const scales_t*>(sl_ + (c % (D - 1)) * SB + ((4 * g + v) * 2 + odd) * (SB / 32));
+            for (int v = 0; v < 4; ++v) sb[v] = *reinterpret_cast<const scales_t*>(sl_ + (c % 2) * SB + ((4 * g + v) * 2 + odd) * (SB / 32));
             const unsigned char* xc = xs + (cx & 1) * XBUF + xrow;
 #pragma unroll
             for (int b = 0; b < 4; ++b) {
@@ -460,7 +460,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 2 : 1) void q8_mfma_kernel
             return;
         }
         const u32x4 wq[2] = {*reinterpret_cast<const u32x4*>(st + w0), *reinterpret_cast<const u32x4*>(st + w1)};
-        const half_t sh = __builtin_bit_cast(half_t, *reinterpret_cast<const uint16_t*>(sl_ + (c % (D - 1)) * SB + r * 16 + odd * 8 + g * 2));
+        const half_t sh = __builtin_bit_cast(half_t, *reinterpret_cast<const uint16_t*>(sl_ + (c % 2) * SB + r * 16 + odd * 8 + g * 2));
         const half2v s2 = {sh, sh};
         const unsigned char* xc = xs + (cx & 1) * XBUF + xrow;
 #pragma unroll
@@ -664,19 +664,19 @@ int launch_q8_mid(const int8_t* q, const uint16_t* sc, int V, int C, const void*
         auto go = [&](auto chunks, auto pairs, auto odd, int nblk, int waves, int xs) {
             const int wgs = (tasks + waves - 1) / waves;
             hipLaunchKernelGGL(rows == Q8_CHUNKS ? chunks : rows == Q8_PAIRS ? pairs : odd, dim3((unsigned)(a.groups > 1 ? (wgs + 7) / 8 * 8 * a.groups : wgs)),
-                               dim3((unsigned)waves * 64), q8l_lds_bytes(nblk, waves, 3, xs, rows), s, a);
+                               dim3((unsigned)waves * 64), q8l_lds_bytes(nblk, waves, xs, rows), s, a);
         };
         static bool raised = false;
         if (!raised) {
             auto raise = [](auto... k) { ((void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024), ...); };
-#define SQ_Q8C(CV, N, W, D, X, ...) q8_mfma_kernel<N, W, D, X, Q8_CHUNKS, CV, ##__VA_ARGS__>, q8_mfma_kernel<N, W, D, X, Q8_PAIRS, CV, ##__VA_ARGS__>, q8_mfma_kernel<N, W, D, X, Q8_ODD, CV, ##__VA_ARGS__>
+#define SQ_Q8C(CV, N, W, X, ...) q8_mfma_kernel<N, W, X, Q8_CHUNKS, CV, ##__VA_ARGS__>, q8_mfma_kernel<N, W, X, Q8_PAIRS, CV, ##__VA_ARGS__>, q8_mfma_kernel<N, W, X, Q8_ODD, CV, ##__VA_ARGS__>
 #define SQ_Q8(...) SQ_Q8C(false, __VA_ARGS__), SQ_Q8C(true, __VA_ARGS__)
-            raise(SQ_Q8(1, 8, 3, 2), SQ_Q8(2, 16, 3, 2), SQ_Q8(2, 8, 3, 1), SQ_Q8(4, 16, 3, 1), SQ_Q8(4, 8, 3, 1), SQ_Q8(4, 8, 3, 1, 4));
+            raise(SQ_Q8(1, 8, 2), SQ_Q8(2, 16, 2), SQ_Q8(2, 8, 1), SQ_Q8(4, 16, 1), SQ_Q8(4, 8, 1), SQ_Q8(4, 8, 1, 4));
 #undef SQ_Q8
             (void)hipGetLastError();
             raised = true;
         }
-#define SQ_GO(N, W, X, WAVES, ...) do { if (cvt) go(SQ_Q8C(true, N, W, 3, X, ##__VA_ARGS__), N, WAVES, X); else go(SQ_Q8C(false, N, W, 3, X, ##__VA_ARGS__), N, WAVES, X); } while (0)
+#define SQ_GO(N, W, X, WAVES, ...) do { if (cvt) go(SQ_Q8C(true, N, W, X, ##__VA_ARGS__), N, WAVES, X); else go(SQ_Q8C(false, N, W, X, ##__VA_ARGS__), N, WAVES, X); } while (0)
         // Small heads: half the waves per workgroup, each making twice the copies of x, spread the same waves over twice the CUs (LDS reads,
         // conversions and matrix instructions are what they take).  us, before / so: 16 rows of 9,728 x 3,584 19.7 /
         // 17.8, of 10,000 x 2,048 12.7 / 12.1, of 30,000 x 2,048 14.3 / 14.8; 64 rows of 9,728 x 3,584 44.7 / 30.5, of 32,000 x 3,584 45.9 / 31.9,
