@@ -77,7 +77,17 @@ int sq_dequant_stack(const sq_matrix* mats, int32_t n_mats, void* out, const voi
  * (batched_runs.py:745-771).  Pieces with M > 1 and pieces with a slice stream need a workspace (see
  * sq_workspace_bytes; the latter keep their partial sums in its header); from 3 to 17 activation rows on, depending
  * on the stack (csrc/sq_gemm.hip), one that has column orders (with C % 8 == 0, 16-byte aligned x, ldx % 8 == 0) is decoded
- * to fp16 in the workspace and multiplied from there, which is faster than its decode-time kernel. */
+ * to fp16 in the workspace and multiplied from there, which is faster than its decode-time kernel.
+ * Two kinds of pieces without column orders have a faster kernel that needs workspace, where x is aligned like that; with less than it
+ * needs they run on their other one, whose fp32 additions come in another order:
+ *   - from 3 rows on, where an estimate says that it pays and no piece of the stack has column orders, pieces of formats without a
+ *     matrix-core kernel (tag widths other than 16 at d = 8, and 12, 10 and 8 at d = 4; rows that end within a unit of their tags with
+ *     16-bit tags, codebooks beyond 128 KB or no tile-major copy) are decoded to fp16, at most 192 MB at a time, and multiplied from
+ *     there; bf16 activations keep their range and bits on both ways, as they do on d = 4 rows that end within a unit;
+ *   - up to 16 rows large pieces with d = 8, 16-bit tags, one codebook and C % 64 == 0 that have no slice stream for these rows keep 8
+ *     to 64 partial sums per result (fp32).  Where those are more than 16 MB the rows go a part at a time in 16 MB, with the same bits.
+ * All other kernels, but the one for x of other alignments, multiply activations as fp16.  sq_workspace_bytes(which = 0) accounts for
+ * all of this, which | 4 for the least that the call runs with. */
 #define SQ_SMALL_BMAX 32
 int sq_linear_small(const sq_matrix* mats, int32_t n_mats, const void* x, int x_dtype, int64_t ldx,
                     void* y, int y_dtype, int64_t ldy, int32_t B, void* workspace, size_t ws_bytes,
@@ -105,7 +115,9 @@ int sq_linear_small_noalloc(const sq_matrix* mats, int32_t n_mats, const void* x
  * SQ_SMALL_BMAX + 1 and 256 rows (384 for large matrices with the codebook in LDS) pieces without column
  * orders gather their codewords once for all rows, in one pass over the packed tags, which is cheaper than
  * decoding the matrix first (pieces whose formats differ: passes of SQ_SMALL_BMAX rows).  Rows that are no whole lane units and
- * column orders are decoded up to 256 rows too, into at most 192 MB of workspace at a time.  Up to SQ_SMALL_BMAX rows the call is
+ * column orders are decoded up to 256 rows too, into at most 192 MB of workspace at a time.  Above, pieces are decoded whole (neighbours
+ * in Y together up to 1 GiB), with split-K sums and an fp16 copy of bf16 activations behind them; where C % 64 != 0 a smaller workspace is
+ * taken as well: what 128 x 128 tiles cannot gather themselves (column orders, other tag widths) is all that these need.  Up to SQ_SMALL_BMAX rows the call is
  * sq_linear_small; sq_workspace_bytes(which = 1) accounts for whichever route T takes. */
 int sq_linear_gemm(const sq_matrix* mats, int32_t n_mats, const void* x, int x_dtype, int64_t ldx,
                    void* y, int y_dtype, int64_t ldy, int32_t T, void* workspace, size_t ws_bytes,
@@ -290,8 +302,8 @@ int sq_codebook_rebalance_device(const sq_matrix* mats, int32_t n, void* const* 
  * One or two rows stream q through an exact-product kernel that needs no workspace; 3 .. 320 rows run fp16 MFMA passes of up to 64
  * rows with the block scale folded into the fp16 weight (one rounding) when C % 256 == 0, and, for other widths and as far as
  * they pay, with exact products and the scale on each block's fp32 sum (without a workspace up to SQ_SMALL_BMAX rows run on
- * the exact-product kernel, 4 per pass).  The passes need the workspace sq_q8_workspace_bytes names (an fp16 copy of
- * the activations).  It replaces gemv_q8_batched /
+ * the exact-product kernel, 4 per pass).  The passes need the workspace sq_q8_workspace_bytes names (room for an fp16 copy of
+ * the activations, asked for whatever x is, though aligned fp16 rows and up to 32 aligned bf16 rows are read from where they are).  It replaces gemv_q8_batched /
  * gemv_q8_tile (reference shapequant/kernels/batched_runs.py:826-861, called from vllm_ext/core.py:575-583) and
  * proto_formats.gemv_q8 (shapequant/kernels/proto_formats.py:474-482); it reads the file's natural layout, so
  * there is no counterpart of the reference's tile-major copy.  More rows (from SQ_SMALL_BMAX + 1 on, where no passes are made) decode row chunks to fp16 in

@@ -322,7 +322,7 @@ static double vector_us(const sq_matrix& m, int B) {
 }
 
 // Without orders: how many pieces, the first one on, are decoded and multiplied from there at B rows because the decode-time product would
-// run them on the vector kernel (16-bit tags of rows that end within a lane unit, tags of other widths, codebooks beyond LDS), which
+// run them on the vector kernel (tags of other widths; rows that end within a lane unit with 16-bit tags, codebooks beyond LDS or no tile-major copy), which
 // takes every few rows as long again: from VECTOR_DECODED_B rows, where the decode, a product and a sum of slices take less (vector
 // kernel / decoded, us at 3 / 4 / 5 rows: 5120 x 2080, 16-bit tags, 58 / 66 / 107 and 24 at any; 300 x 2080 21 / 25 / 36, 14; 512 x 1024,
 // 14-bit tags of width 4, 10.8 / 12.5 / 18.2, 17.7; 4864 x 896, 6-bit, 13.8 / 15.8 / 21.5, 20; 2048 x 512, 6-bit, 7.9 / 8.0 / 9.7, 17; 16384 x
