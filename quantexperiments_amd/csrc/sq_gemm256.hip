@@ -743,9 +743,12 @@ struct Gemm256Plan { int mt, main_tiles, tail_tiles, kt; };
 // Tiles of 256 rows read least per product and are the ones for products of many rounds (8192^3: 880 us, 963 with 192 rows,
 // 1019 with 128); where few tiles leave CUs idle, or most of a tile's rows are past the end, smaller ones win.  The plan with the
 // least estimated time is taken.  A slab takes G_SLAB + G_SLAB_BUSY * (share of the CUs at work) microseconds (the chip's power
-// and its L2 set the pace when it is full; fitted to 32 .. 512 tiles of each height at 3584 columns, where one round takes 42 ..
+// and its L2 set the pace when it is full; fitted to 32 .. 512 tiles of each height at 3584 columns, where one round took 42 ..
 // 63 / 55 .. 81 / 70 .. 104 us), a round 5 us at its ends, and a split adds the reduction's launch and the partial tiles written
-// and read back.  Estimated best and measured, tiles of 256 rows unsplit before it (us): 333 x 37888 x 3584 161, now 119;
+// and read back.  All of these times are of a kernel of 32x32x16 instructions with a workgroup per tile.  Today's take less than is estimated,
+// and not by one factor (2048 x 37888 x 3584 481 estimated, 403 - 424 measured; 2048 x 3584 x 18944 258 and 237; 2048 x 4608 x 3584 70 and 66;
+// 2048 x 3584 x 3584 58 and 51; 1024 x 7168 x 5120 81 and 67): what is near another plan in the estimate may not be the best one.
+// Estimated best and measured then, tiles of 256 rows unsplit before it (us): 333 x 37888 x 3584 161, with the plan 119;
 // 1024 x 7168 x 5120 95 (in two 85), now 72; 2048 x 3584 x 3584 66, now 52; 2048 x 4608 x 3584 70, now 64; 512 x 3584 x 18944
 // 104 in four, now 88; 2048 x 3584 x 18944 stays with 256 rows in two, 245 (128 rows: 270).
 // Up to eight parts, for few tiles of long rows (with up to four, now): 333 x 3584 x 18944 83, 71.  Parts of 8 slabs would gain 2

@@ -124,7 +124,7 @@ static_assert(DEAL_STEPS * sizeof(DealStep) <= DEAL_WAVES * 256 * 4, "the steps 
 // it a step took twice as long), then all write the codewords' labels.  The codewords are sorted by count with a stable radix sort, 8 bits
 // a pass, ids in LDS and between two passes in registers (a wave owns a 16th of them); counts below 256, the usual ones, are one pass of
 // as many bits as they have, read from the counts in order, and its digits' places are where the runs of equal counts start.
-// 65,536 codewords: 3584 x 448 evenly spread tags 95 us (sorting 40, 73 steps 42, labels 19), 190 with the sort in general passes, the runs' starts
+// 65,536 codewords: 3584 x 448 evenly spread tags 95 to 102 us (sorting 40, 73 steps 42, labels 19), 190 with the sort in general passes, the runs' starts
 // searched in the sorted counts and every wave at the steps; 1057 x 64 58, 130; 5120 x 640 of a power law 0.89 ms (a load of that matrix 2.62 ms, 3.23).
 // On the host, with the copies and the synchronisation around it, 480 us of a load for every matrix of a stack.
 template <int PER, typename T>               // ids per lane: K / DEAL_NT (0: codebooks of one slice); a slice's tags (less than 2^(bits - 4))
