@@ -128,6 +128,79 @@ template <int N> __device__ __forceinline__ void acc_claim() {                 /
 template <class F, int... I> __device__ __forceinline__ void each(F f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
 template <int N, class F> __device__ __forceinline__ void each(F f) { each(f, std::make_integer_sequence<int, N>{}); }
 
+#define SQ_INLINE __attribute__((always_inline))
+#define SQ_SB() __builtin_amdgcn_sched_barrier(0)
+
+// What both kernels share: the sizes of a tile of 64 MT rows and the rings' waits ...
+template <int MT> struct Gemm256Shape {
+    // XC: copies a wave makes of an X slab (of a W slab: 8); TB: its blocks of 16 tokens; NM: products of a step
+    static constexpr int BM = gemm256_tokens(MT), XC = 2 * MT, X_SLOT = BM * G_BK * 2, TB = 2 * MT, NM = 8 * TB;
+    static constexpr bool XE = gemm256_x_slots(MT) > gemm256_w_slots(MT);        // X is the early operand, the one of E slots; the late one has L
+    static constexpr int E = XE ? gemm256_x_slots(MT) : gemm256_w_slots(MT), L = E - 1, EC = XE ? XC : 8, LC = XE ? 8 : XC;
+    static_assert(L == (XE ? gemm256_w_slots(MT) : gemm256_x_slots(MT)), "the waits count on it");
+    static constexpr int W_AT = gemm256_x_slots(MT) * X_SLOT;
+    static constexpr int ES = XE ? X_SLOT : G_W_SLOT, LS = XE ? G_W_SLOT : X_SLOT;       // the slots' sizes
+    static constexpr int AHEAD = (E - 2) * EC + (L - 2) * LC;                    // copies that may be on their way when slab s + 1 has to be there
+};
+
+// ... copy j of an operand's slab to LDS (four copies share an LDS base: the instruction's own offset, 1024 (j % 4), counts for LDS and memory, so
+// the lanes' offsets hold that much less, and bases that start 3072 bytes early keep them positive); an offset of G_PAST is past the buffer's
+// end and puts zeros there ...
+constexpr uint32_t G_PAST = 0xFFFF0000u;
+__device__ __forceinline__ void gemm256_copy(const char* base, uint32_t off, int at, unsigned char* to, int j) {
+    typedef __attribute__((address_space(3))) void* lptr_t;
+    const __amdgpu_buffer_rsrc_t buf = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, G_PAST, 0x00027000);
+    const lptr_t lds = (lptr_t)to;
+    if ((j & 3) == 0) __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, lds, 16, off, at, 0, 0);
+    if ((j & 3) == 1) __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, lds, 16, off, at, 1024, 0);
+    if ((j & 3) == 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, lds, 16, off, at, 2048, 0);
+    if ((j & 3) == 3) __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, lds, 16, off, at, 3072, 0);
+}
+
+// ... the slots (byte offsets) of the slab being multiplied (early and late operand), of the next one, and the one the early copies go to ...
+template <int MT> struct Gemm256Slots { int ce = 0, cl = 0, ne = 0, nl = 0, to = (Gemm256Shape<MT>::E - 1) * Gemm256Shape<MT>::ES; };
+
+// ... and the schedule of a slab, two steps of 32 columns.  mma(step, n): product n of a step, token block n / 8, weight-row block n % 8, to and
+// fro; read_x(kk, slot, i) and read_w(set, kk, slot, j): fragments of step kk; copy_early, copy_late(slot, j); ready(): the wait for this wave's
+// copies of slab s + 1 (those of later slabs stay in flight) and its reads of slab s; next(): on to the next slab to copy.  The slots are
+// worked out between the products, a little at a time: a scalar instruction in front of them takes four clocks of the matrix core's time.
+template <int MT, class Mma, class ReadX, class ReadW, class Early, class Late, class Ready, class Next>
+__device__ __forceinline__ void gemm256_slab(Gemm256Slots<MT>& p, Mma mma, ReadX read_x, ReadW read_w, Early copy_early, Late copy_late, Ready ready, Next next) {
+    typedef Gemm256Shape<MT> S;
+    constexpr bool XE = S::XE;
+    constexpr int TB = S::TB, NM = S::NM, GAP = MT == 2 ? 2 : 4;
+    // first step: its last X blocks, the second step's fragments, the early copies of slab s + L
+    each<NM>([&](auto nn) SQ_INLINE {
+        constexpr int n = decltype(nn)::value;
+        mma(std::integral_constant<int, 0>{}, nn); SQ_SB();
+        if (n < 2) read_x(0, XE ? p.ce : p.cl, TB - 1 - n);
+        if (n >= 2 && n <= 16 && n % 2 == 0) read_w(1, 1, XE ? p.cl : p.ce, n / 2 - 1);
+        if (n % 8 == 1 && n > 8 && n < NM - 8) read_x(1, XE ? p.ce : p.cl, n / 8 - 1);
+        if (n % 4 == 3 && n / 4 < S::EC) copy_early(p.to, n / 4);
+        if (n == NM - 6) { p.ne = p.ce + S::ES; SQ_SB(); }
+        if (n == NM - 5) { p.ne = p.ne == S::E * S::ES ? 0 : p.ne; SQ_SB(); }
+        if (n == NM - 4) { p.nl = p.cl + S::LS; SQ_SB(); }
+        if (n == NM - 3) { p.nl = p.nl == S::L * S::LS ? 0 : p.nl; SQ_SB(); }
+        if (n == NM - 2) { p.to = p.ce; SQ_SB(); }
+        SQ_SB();
+    });
+    // second step: this wave's copies of slab s + 1 and its reads of slab s, whose slots the copies behind the barrier overwrite, are waited
+    // for; then the barrier: everybody's copies have landed and everybody has read slab s to the end.  (Six products behind the last of
+    // those reads their wait costs little.)
+    each<NM>([&](auto nn) SQ_INLINE {
+        constexpr int n = decltype(nn)::value;
+        mma(std::integral_constant<int, 1>{}, nn); SQ_SB();
+        if (n < 2) read_x(1, XE ? p.ce : p.cl, TB - 1 - n);
+        if (n == 7) { ready(); SQ_SB(); __builtin_amdgcn_s_barrier(); SQ_SB(); }
+        if (n >= 8 && n <= 22 && n % 2 == 0) read_w(0, 0, XE ? p.nl : p.ne, n / 2 - 4);
+        if (n % 8 == 1 && n > 8 && n < NM - 8) read_x(0, XE ? p.ne : p.nl, n / 8 - 1);
+        if (n >= 11 && (n - 11) % GAP == 0 && (n - 11) / GAP < S::LC) copy_late(p.cl, (n - 11) / GAP);
+        if (n == NM - 4) { next(); SQ_SB(); }
+        if (n == NM - 3) { p.ce = p.ne; p.cl = p.nl; SQ_SB(); }
+        SQ_SB();
+    });
+}
+
 // What a workgroup multiplies: a whole tile, or one of the parts of a tail tile.
 struct Gemm256Item { int tile, kz, nparts, t0, r0, k_begin, nk; };
 
@@ -142,8 +215,6 @@ struct Gemm256Item { int tile, kz, nparts, t0, r0, k_begin, nk; };
 // the next tile to get through.  A workgroup per tile spent 9 us a round of tiles beyond its slabs, 4 to 5 of them on the stores;
 // the power limit takes part of that back: gate|up of 2048 rows with its decode (2 x 18944 x 3584, five rounds) 536 -> 523 us, a
 // layer of 2048 rows 980 -> 968, 8192^3 with its decode 809 -> 802, products of one round level.
-#define SQ_INLINE __attribute__((always_inline))
-
 template <int EP, int MT>
 __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -154,7 +225,9 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a)
     const int ntiles = a.tiles_t * a.tiles_r, xcd = (int)(blockIdx.x & 7), stride = (int)(gridDim.x >> 3);
     const int main_per = (a.main_tiles + 7) >> 3, parts = (ntiles - a.main_tiles) * a.kt, parts_per = (parts + 7) >> 3;
     const int main_mine = min(main_per, a.main_tiles - xcd * main_per), items = main_per + max(0, min(parts_per, parts - xcd * parts_per));
-    constexpr int BM = gemm256_tokens(MT), XC = 2 * MT, X_SLOT = BM * G_BK * 2, TB = 2 * MT, NM = 8 * TB;     // XC: copies a wave makes of an X slab (of a W slab: 8); TB: its blocks of 16 tokens; NM: products of a step
+    typedef Gemm256Shape<MT> S;
+    constexpr int BM = S::BM, XC = S::XC, X_SLOT = S::X_SLOT, TB = S::TB, L = S::L, EC = S::EC, LC = S::LC, ES = S::ES, LS = S::LS, W_AT = S::W_AT, AHEAD = S::AHEAD;
+    constexpr bool XE = S::XE;
     const int nk_all = (a.C + G_BK - 1) / G_BK;
     auto valid = [&](int j) SQ_INLINE {                // this item, or the workgroup's next one where the XCD's run of tiles is shorter than others'
         while (j >= main_mine && j < main_per) j += stride;
@@ -196,29 +269,19 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a)
     // last item's last slab that one is read again.  The pieces of a row's last slab that lie past its end (C % 64 != 0) are asked
     // for past the end of the buffer, which puts zeros into LDS, for both operands (global_load_lds instead of the buffers, for whole
     // slabs: level; rows of broken slabs ran in the 128 x 128 kernel: 5120 x 2080 at 400 / 1500 rows 80-120 / 126-194 us, now 38-43 / 47-53).
-    constexpr bool XE = gemm256_x_slots(MT) > gemm256_w_slots(MT);        // X is the early one
-    constexpr int E = XE ? gemm256_x_slots(MT) : gemm256_w_slots(MT), L = E - 1, EC = XE ? XC : 8, LC = XE ? 8 : XC;
-    static_assert(L == (XE ? gemm256_w_slots(MT) : gemm256_x_slots(MT)), "the waits below count on it");
-    constexpr int W_AT = gemm256_x_slots(MT) * X_SLOT;
-    constexpr int ES = XE ? X_SLOT : G_W_SLOT, LS = XE ? G_W_SLOT : X_SLOT;      // the slots' sizes
-    constexpr int AHEAD = (E - 2) * EC + (L - 2) * LC;                    // copies that may be on their way when slab s + 1 has to be there
-    typedef __attribute__((address_space(3))) void* lptr_t;
     const int lrow = lane >> 3, slot = lane & 7;
     bool past[2];                            // this lane's piece of a row's last slab lies past its end, in even and odd copies (whose rows' swizzles differ by 4)
 #pragma unroll
     for (int h = 0; h < 2; ++h) past[h] = (slot ^ (h * 4 + (lrow >> 1))) * 8 >= a.C - (nk_all - 1) * G_BK;
-    // (four copies share an LDS base: the instruction's own offset, 1024 j, counts for LDS and memory, so the lanes' offsets hold that
-    // much less, and bases that start 3072 bytes early keep them positive)
-    constexpr uint32_t PAST = 0xFFFF0000u;
     uint32_t xo[XC], wo[8];
     const char *xt, *wt;
     int at, left, step;                      // the copied slab's first column in bytes, the item's slabs from it on, bytes to the next slab
     int last;                                // 1 in an item that ends with a slab that the row does not fill, until that is the next
     auto row_end = [&]() SQ_INLINE {
 #pragma unroll
-        for (int j = 0; j < XC; ++j) xo[j] = past[j & 1] ? PAST : xo[j];
+        for (int j = 0; j < XC; ++j) xo[j] = past[j & 1] ? G_PAST : xo[j];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) wo[j] = past[j & 1] ? PAST : wo[j];
+        for (int j = 0; j < 8; ++j) wo[j] = past[j & 1] ? G_PAST : wo[j];
     };
     auto copy_from = [&](int j) SQ_INLINE {
         const Gemm256Item it = item(j);
@@ -249,17 +312,9 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a)
         if (jc < items) copy_from(jc);
         else { at -= step; step = 0; left = INT_MAX; }
     };
-    auto copy = [&](const char* base, uint32_t off, int to, int j) SQ_INLINE {
-        const __amdgpu_buffer_rsrc_t buf = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, PAST, 0x00027000);
-        const lptr_t lds = (lptr_t)(smem + to);
-        if ((j & 3) == 0) __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, lds, 16, off, at, 0, 0);
-        if ((j & 3) == 1) __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, lds, 16, off, at, 1024, 0);
-        if ((j & 3) == 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, lds, 16, off, at, 2048, 0);
-        if ((j & 3) == 3) __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, lds, 16, off, at, 3072, 0);
-    };
     // `to`: the slot's offset
-    auto copy_x = [&](int to, int j) SQ_INLINE { copy(xt, xo[j], to + wave * (X_SLOT / 4) + (j & ~3) * 1024, j); };
-    auto copy_w = [&](int to, int j) SQ_INLINE { copy(wt, wo[j], to + W_AT + wave * 8192 + (j & ~3) * 1024, j); };
+    auto copy_x = [&](int to, int j) SQ_INLINE { gemm256_copy(xt, xo[j], at, smem + to + wave * (X_SLOT / 4) + (j & ~3) * 1024, j); };
+    auto copy_w = [&](int to, int j) SQ_INLINE { gemm256_copy(wt, wo[j], at, smem + to + W_AT + wave * 8192 + (j & ~3) * 1024, j); };
     auto copy_early = [&](int to, int j) SQ_INLINE { if constexpr (XE) copy_x(to, j); else copy_w(to, j); };
     auto copy_late = [&](int to, int j) SQ_INLINE { if constexpr (XE) copy_w(to, j); else copy_x(to, j); };
 
@@ -274,10 +329,9 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a)
     auto read_w = [&](int set, int kk, int at, int j) SQ_INLINE {
         fw[set][j] = *reinterpret_cast<const half8v*>(smem + W_AT + at + wn * 128 + j * 2048 + (foff ^ (uint32_t)(kk << 6)));
     };
-    // product n of a step: token block n / 8, weight-row block n % 8, to and fro
     auto mma = [&](auto set, auto n) SQ_INLINE {
-        constexpr int S = decltype(set)::value, N = decltype(n)::value, i = N >> 3, j = i & 1 ? 7 - (N & 7) : N & 7;
-        acc_product<4 * (8 * i + j)>(fw[S][j], fx[i]);
+        constexpr int N = decltype(n)::value, i = N >> 3, j = i & 1 ? 7 - (N & 7) : N & 7;
+        acc_product<4 * (8 * i + j)>(fw[decltype(set)::value][j], fx[i]);
     };
     // (the waits of both directions are written out: the compiler does not know what is in the accumulators)
     auto clear = [&]() SQ_INLINE {
@@ -285,7 +339,6 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a)
         each<2 * TB>([&](auto q) SQ_INLINE { acc_clear16<16 * decltype(q)::value>(half8v{}); });
         asm volatile("s_nop 15\n\ts_nop 15");
     };
-#define SQ_SB() __builtin_amdgcn_sched_barrier(0)
 
     copy_from(jc);
 #pragma unroll 1
@@ -302,9 +355,7 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a)
     for (int i = 0; i < TB - 2; ++i) read_x(0, 0, i);
 #pragma unroll
     for (int j = 0; j < 8; ++j) read_w(0, 0, 0, j);
-    // the slots (byte offsets) of the slab being multiplied, of the next one, and the one the early copies go to.  Worked out between
-    // the products, a little at a time: a scalar instruction in front of them takes four clocks of the matrix core's time.
-    int ce = 0, cl = 0, ne = 0, nl = 0, to = (E - 1) * ES;
+    Gemm256Slots<MT> slots;
     // the 16-byte stores a wave makes of a whole tile's results, which the next tile's first slab need not wait for
     constexpr int STORES = 8 * MT;
     static_assert(AHEAD + STORES < 64, "what the counter holds");
@@ -315,41 +366,13 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a)
     // row's broken end); the others have no branches
     auto slab = [&](auto event) SQ_INLINE {
         constexpr bool EVENT = decltype(event)::value;
-        // first step: its last X blocks, the second step's fragments, the early copies of slab s + L
-        each<NM>([&](auto nn) SQ_INLINE {
-            constexpr int n = decltype(nn)::value;
-            mma(std::integral_constant<int, 0>{}, nn); SQ_SB();
-            if (n < 2) read_x(0, XE ? ce : cl, TB - 1 - n);
-            if (n >= 2 && n <= 16 && n % 2 == 0) read_w(1, 1, XE ? cl : ce, n / 2 - 1);
-            if (n % 8 == 1 && n > 8 && n < NM - 8) read_x(1, XE ? ce : cl, n / 8 - 1);
-            if (n % 4 == 3 && n / 4 < EC) copy_early(to, n / 4);
-            if (n == NM - 6) { ne = ce + ES; SQ_SB(); }
-            if (n == NM - 5) { ne = ne == E * ES ? 0 : ne; SQ_SB(); }
-            if (n == NM - 4) { nl = cl + LS; SQ_SB(); }
-            if (n == NM - 3) { nl = nl == L * LS ? 0 : nl; SQ_SB(); }
-            if (n == NM - 2) { to = ce; SQ_SB(); }
-            SQ_SB();
-        });
-        // second step: this wave's copies of slab s + 1 are waited for (those of later slabs stay in flight, and the stores of the
-        // item before, which went out behind slab s + 1's copies where s is an item's first slab), and its reads of slab
-        // s, whose slots the copies behind the barrier overwrite; then the barrier: everybody's copies have landed and
-        // everybody has read slab s to the end.  (Six products behind the last of those reads their wait costs little.)
-        each<NM>([&](auto nn) SQ_INLINE {
-            constexpr int n = decltype(nn)::value, GAP = MT == 2 ? 2 : 4;
-            mma(std::integral_constant<int, 1>{}, nn); SQ_SB();
-            if (n < 2) read_x(1, XE ? ce : cl, TB - 1 - n);
-            if (n == 7) {
+        gemm256_slab<MT>(slots, mma, read_x, read_w, copy_early, copy_late,
+            // (the stores of the item before went out behind slab s + 1's copies where s is an item's first slab: they stay in flight too)
+            [&]() SQ_INLINE {
                 if (!EVENT || !stores) __builtin_amdgcn_s_waitcnt(vmcnt_and_lds(AHEAD));
                 else __builtin_amdgcn_s_waitcnt(vmcnt_and_lds(AHEAD + STORES));
-                SQ_SB(); __builtin_amdgcn_s_barrier(); SQ_SB();
-            }
-            if (n >= 8 && n <= 22 && n % 2 == 0) read_w(0, 0, XE ? nl : ne, n / 2 - 4);
-            if (n % 8 == 1 && n > 8 && n < NM - 8) read_x(0, XE ? ne : nl, n / 8 - 1);
-            if (n >= 11 && (n - 11) % GAP == 0 && (n - 11) / GAP < LC) copy_late(cl, (n - 11) / GAP);
-            if (n == NM - 4) { if constexpr (EVENT) next_slab(); else at += step; SQ_SB(); }
-            if (n == NM - 3) { ce = ne; cl = nl; SQ_SB(); }
-            SQ_SB();
-        });
+            },
+            [&]() SQ_INLINE { if constexpr (EVENT) next_slab(); else at += step; });
     };
     uint32_t scale[2] = {};                  // of weight rows lane and 64 + lane of this wave's 128, fp16
     clear();
@@ -387,7 +410,7 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a)
             for (int e = 0; e < 4; ++e) sc[j][e] = h2f((uint16_t)__builtin_amdgcn_ds_bpermute(((j & 3) * 16 + 4 * quad + e) * 4, (int)scale[j >> 2]));
         constexpr int TBP = ES / 4 / 4096;
         static_assert(TB % TBP == 0, "whole passes");
-        unsigned char* my = smem + (XE ? 0 : W_AT) + to + wave * (ES / 4);
+        unsigned char* my = smem + (XE ? 0 : W_AT) + slots.to + wave * (ES / 4);
         uint16_t* dst = reinterpret_cast<uint16_t*>(a.y) + (int64_t)(it.t0 + wm) * ldy + a.y_off + it.r0 + wn + (quad * ldy + tok * 8);
         each<TB / TBP>([&](auto pp) SQ_INLINE {
             constexpr int p = decltype(pp)::value;
@@ -458,13 +481,14 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_kernel(Gemm256Args a)
         togo = it.nk;
         clear();
     }
-#undef SQ_SB
     __builtin_amdgcn_s_waitcnt(vmcnt_only(0));       // no copy is on its way into LDS that is another workgroup's by then
 }
 
-#undef SQ_INLINE
-
 constexpr int G_EP_PITCH = 128 * 2 + 16;     // bytes per token row of a wave's 32 MT x 128 output tile in LDS
+
+__device__ __forceinline__ void product(float4v& sums, half8v w, half8v x) {
+    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(sums) : "v"(w), "v"(x));
+}
 
 // The product of at most a tile (or a part of one) per workgroup: what a workgroup needs to go from tile to tile, products that know about events,
 // accumulators it names, addresses in front of every tile, is longer than the slabs of a small product.  us, the kernel above / this one:
@@ -493,7 +517,9 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_one_kernel(Gemm256Arg
     }
     int bt, br;
     gemm256_tile(tile, a.tiles_t, a.tiles_r, gemm256_super(MT), &bt, &br);
-    constexpr int BM = gemm256_tokens(MT), XC = 2 * MT, X_SLOT = BM * G_BK * 2, TB = 2 * MT, NM = 8 * TB;     // XC: copies a wave makes of an X slab (of a W slab: 8); TB: its blocks of 16 tokens; NM: products of a step
+    typedef Gemm256Shape<MT> S;
+    constexpr int BM = S::BM, XC = S::XC, X_SLOT = S::X_SLOT, TB = S::TB, E = S::E, L = S::L, EC = S::EC, LC = S::LC, ES = S::ES, LS = S::LS, W_AT = S::W_AT, AHEAD = S::AHEAD;
+    constexpr bool XE = S::XE;
     const int t0 = bt * BM, r0 = br * G_BN;
     const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * 128;
 
@@ -504,11 +530,6 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_one_kernel(Gemm256Arg
         for (int j = 0; j < 8; ++j) acc[i][j] = float4v{0.f, 0.f, 0.f, 0.f};
 
     // Copies, as above; slabs past the last one re-read the last.
-    constexpr bool XE = gemm256_x_slots(MT) > gemm256_w_slots(MT);        // X is the early one
-    constexpr int E = XE ? gemm256_x_slots(MT) : gemm256_w_slots(MT), L = E - 1, EC = XE ? XC : 8, LC = XE ? 8 : XC;
-    static_assert(L == (XE ? gemm256_w_slots(MT) : gemm256_x_slots(MT)), "the waits below count on it");
-    constexpr int W_AT = gemm256_x_slots(MT) * X_SLOT;
-    constexpr int AHEAD = (E - 2) * EC + (L - 2) * LC;                    // copies that may be on their way when slab s + 1 has to be there
     const int lrow = lane >> 3, slot = lane & 7;
     uint32_t xo[XC], wo[8];
 #pragma unroll
@@ -527,37 +548,26 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_one_kernel(Gemm256Arg
     const int nk = (int)((int64_t)(kz + 1) * nk_all / nparts) - k_begin;
     const char* xt = reinterpret_cast<const char*>(a.x + (int64_t)t0 * a.ldx + (int64_t)k_begin * G_BK) - 3072;
     const char* wt = reinterpret_cast<const char*>(a.w + (int64_t)r0 * a.ldw + (int64_t)k_begin * G_BK) - 3072;
-    typedef __attribute__((address_space(3))) void* lptr_t;
     const int lastk = nk_all - 1 - k_begin;  // the row's last slab, counted from this part's first
     bool past[2];                            // this lane's piece of it lies past the row's end, in even and odd copies (whose rows' swizzles differ by 4)
 #pragma unroll
     for (int h = 0; h < 2; ++h) past[h] = (slot ^ (h * 4 + (lrow >> 1))) * 8 >= a.C - (nk_all - 1) * G_BK;
-    constexpr uint32_t PAST = 0xFFFF0000u;
-    auto copy = [&](const char* base, int at, uint32_t off, int to, int j) {
-        const __amdgpu_buffer_rsrc_t buf = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, PAST, 0x00027000);
-        const lptr_t lds = (lptr_t)(smem + to);
-        if ((j & 3) == 0) __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, lds, 16, off, at, 0, 0);
-        if ((j & 3) == 1) __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, lds, 16, off, at, 1024, 0);
-        if ((j & 3) == 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, lds, 16, off, at, 2048, 0);
-        if ((j & 3) == 3) __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, lds, 16, off, at, 3072, 0);
-    };
     // `at`: the slab's first column in bytes, `to`: its slot's offset
-    auto copy_x = [&](int at, int to, int j) { copy(xt, at, xo[j], to + wave * (X_SLOT / 4) + (j & ~3) * 1024, j); };
-    auto copy_w = [&](int at, int to, int j) { copy(wt, at, wo[j], to + W_AT + wave * 8192 + (j & ~3) * 1024, j); };
+    auto copy_x = [&](int at, int to, int j) { gemm256_copy(xt, xo[j], at, smem + to + wave * (X_SLOT / 4) + (j & ~3) * 1024, j); };
+    auto copy_w = [&](int at, int to, int j) { gemm256_copy(wt, wo[j], at, smem + to + W_AT + wave * 8192 + (j & ~3) * 1024, j); };
     auto copy_early = [&](int at, int to, int j) { if constexpr (XE) copy_x(at, to, j); else copy_w(at, to, j); };
     auto copy_late = [&](int at, int to, int j) { if constexpr (XE) copy_w(at, to, j); else copy_x(at, to, j); };
-    constexpr int ES = XE ? X_SLOT : G_W_SLOT, LS = XE ? G_W_SLOT : X_SLOT;      // their slots' sizes
     // from the row's last slab on the pieces past its end are asked for past the buffer's end
     const int plast = lastk < nk && a.C % G_BK != 0 ? lastk : INT_MAX;
     auto end_early = [&](int q) {
         if (q < plast) return;
 #pragma unroll
-        for (int j = 0; j < EC; ++j) { uint32_t& o = XE ? xo[j] : wo[j]; o = past[j & 1] ? PAST : o; }
+        for (int j = 0; j < EC; ++j) { uint32_t& o = XE ? xo[j] : wo[j]; o = past[j & 1] ? G_PAST : o; }
     };
     auto end_late = [&](int q) {
         if (q < plast) return;
 #pragma unroll
-        for (int j = 0; j < LC; ++j) { uint32_t& o = XE ? wo[j] : xo[j]; o = past[j & 1] ? PAST : o; }
+        for (int j = 0; j < LC; ++j) { uint32_t& o = XE ? wo[j] : xo[j]; o = past[j & 1] ? G_PAST : o; }
     };
     auto column = [&](int q) { return (q < nk ? q : nk - 1) * (G_BK * 2); };
 
@@ -570,15 +580,13 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_one_kernel(Gemm256Arg
     auto read_w = [&](int set, int kk, int at, int j) {
         fw[set][j] = *reinterpret_cast<const half8v*>(smem + W_AT + at + wn * 128 + j * 2048 + (foff ^ (uint32_t)(kk << 6)));
     };
-    // product n of a step: token block n / 8, weight-row block n % 8, to and fro
-    auto mma = [&](int set, int n) {
-        const int i = n >> 3, j = i & 1 ? 7 - (n & 7) : n & 7;
-        asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(fw[set][j]), "v"(fx[i]));
+    auto mma = [&](auto set, auto n) SQ_INLINE {
+        constexpr int N = decltype(n)::value, i = N >> 3, j = i & 1 ? 7 - (N & 7) : N & 7;
+        product(acc[i][j], fw[decltype(set)::value][j], fx[i]);
     };
     // the accumulators stay in their registers before and behind the loop (without this the compiler copies all 256 into the
     // other half of the register file at the loop's end, spills, and a launch that needs scratch memory takes 7 us longer)
 #define SQ_PIN() _Pragma("unroll") for (int i = 0; i < TB; ++i) { asm volatile("" : "+a"(acc[i][0]), "+a"(acc[i][1]), "+a"(acc[i][2]), "+a"(acc[i][3]), "+a"(acc[i][4]), "+a"(acc[i][5]), "+a"(acc[i][6]), "+a"(acc[i][7])); }
-#define SQ_SB() __builtin_amdgcn_sched_barrier(0)
 
 #pragma unroll
     for (int q = 0; q < E - 1; ++q) {
@@ -599,51 +607,18 @@ __global__ __launch_bounds__(G_WAVES * 64, 1) void gemm256_one_kernel(Gemm256Arg
     end_late(L - 1);
 #pragma unroll
     for (int j = 0; j < LC; ++j) copy_late(column(L - 1), (L - 1) * LS, j);
-    // the slots (byte offsets) of the slab being multiplied, of the next one, and the one the early copies go to; the column of the
-    // slab that is copied.  Worked out between the products, a little at a time: a scalar instruction in front of them takes four
-    // clocks of the matrix core's time.
-    int ce = 0, cl = 0, ne = 0, nl = 0, to = (E - 1) * ES, at = column(L);
+    Gemm256Slots<MT> slots;
+    int at = column(L);                      // of the slab that is copied
     SQ_PIN();
     asm volatile("s_nop 7");                 // (no wait of the compiler's between the zeroed accumulators and a written-out product)
 #pragma unroll 1
     for (int s = 0; s < nk; ++s) {
         if (s + L >= plast) { end_early(s + L); end_late(s + L); }
-        // first step: its last X blocks, the second step's fragments, the early copies of slab s + L
-#pragma unroll
-        for (int n = 0; n < NM; ++n) {
-            mma(0, n); SQ_SB();
-            if (n < 2) read_x(0, XE ? ce : cl, TB - 1 - n);
-            if (n >= 2 && n <= 16 && n % 2 == 0) read_w(1, 1, XE ? cl : ce, n / 2 - 1);
-            if (n % 8 == 1 && n > 8 && n < NM - 8) read_x(1, XE ? ce : cl, n / 8 - 1);
-            if (n % 4 == 3 && n / 4 < EC) copy_early(at, to, n / 4);
-            if (n == NM - 6) { ne = ce + ES; SQ_SB(); }
-            if (n == NM - 5) { ne = ne == E * ES ? 0 : ne; SQ_SB(); }
-            if (n == NM - 4) { nl = cl + LS; SQ_SB(); }
-            if (n == NM - 3) { nl = nl == L * LS ? 0 : nl; SQ_SB(); }
-            if (n == NM - 2) { to = ce; SQ_SB(); }
-            SQ_SB();
-        }
-        // second step, with the wait and the barrier as above
-#pragma unroll
-        for (int n = 0; n < NM; ++n) {
-            mma(1, n); SQ_SB();
-            if (n < 2) read_x(1, XE ? ce : cl, TB - 1 - n);
-            if (n == 7) {
-                __builtin_amdgcn_s_waitcnt(vmcnt_and_lds(AHEAD)); SQ_SB();
-                __builtin_amdgcn_s_barrier(); SQ_SB();
-            }
-            if (n >= 8 && n <= 22 && n % 2 == 0) read_w(0, 0, XE ? nl : ne, n / 2 - 4);
-            if (n % 8 == 1 && n > 8 && n < NM - 8) read_x(0, XE ? ne : nl, n / 8 - 1);
-            constexpr int GAP = MT == 2 ? 2 : 4;
-            if (n >= 11 && (n - 11) % GAP == 0 && (n - 11) / GAP < LC) copy_late(at, cl, (n - 11) / GAP);
-            if (n == NM - 4) { at = column(s + 1 + L); SQ_SB(); }
-            if (n == NM - 3) { ce = ne; cl = nl; SQ_SB(); }
-            SQ_SB();
-        }
+        gemm256_slab<MT>(slots, mma, read_x, read_w, [&](int to, int j) SQ_INLINE { copy_early(at, to, j); }, [&](int to, int j) SQ_INLINE { copy_late(at, to, j); },
+                         [&]() SQ_INLINE { __builtin_amdgcn_s_waitcnt(vmcnt_and_lds(AHEAD)); }, [&]() SQ_INLINE { at = column(s + 1 + L); });
     }
     asm volatile("s_nop 15\n\ts_nop 15");    // the last products' results are behind the loop before they are read
     SQ_PIN();
-#undef SQ_SB
 #undef SQ_PIN
     __builtin_amdgcn_s_waitcnt(vmcnt_and_lds(0));
     __syncthreads();                         // every wave is done with the operand ring, and no copy is on its way into it
