@@ -17,7 +17,7 @@
  *     w[r, perms[row_mask[r]][c]] = u[r, c]
  * and the layer computes Y[t, y_off + r] = sum_c X[t, c] * w[r, c] with fp32 accumulation.  A row that names a codeword which is not
  * finite has results that are not finite; an infinity may come out as NaN (idle lanes of the decode-time kernels, and of the d = 4
- * kernel for 33 to 384 rows, multiply codewords of the row with zeros).  Other rows are not touched.
+ * kernel that gathers codewords for 33 and more rows, multiply codewords of the row with zeros).  Other rows are not touched.
  */
 #ifndef SQHIP_H
 #define SQHIP_H
@@ -112,9 +112,9 @@ int sq_linear_small_noalloc(const sq_matrix* mats, int32_t n_mats, const void* x
  * accumulation, row scale applied to the accumulator.  Same argument meaning as sq_linear_small.
  * Replaces runs_gemm.gemm (reference shapequant/kernels/runs_gemm.py:471-514).  Pieces with
  * M > 1 are decoded with their column orders into workspace and multiplied from there.  Between
- * SQ_SMALL_BMAX + 1 and 256 rows (384 for large matrices with the codebook in LDS) pieces without column
- * orders gather their codewords once for all rows, in one pass over the packed tags, which is cheaper than
- * decoding the matrix first (pieces whose formats differ: passes of SQ_SMALL_BMAX rows).  Rows that are no whole lane units and
+ * SQ_SMALL_BMAX + 1 and 256 rows (384 for large matrices with the codebook in LDS), and for more rows of smaller matrices, pieces without column
+ * orders gather their codewords once per block of rows, in one pass over the packed tags, which is cheaper than
+ * decoding the matrix first (as many K slices as the workspace holds the sums of; pieces whose formats differ: passes of SQ_SMALL_BMAX rows).  Rows that are no whole lane units and
  * column orders are decoded up to 256 rows too, into at most 192 MB of workspace at a time.  Above, pieces are decoded whole (neighbours
  * in Y together up to 1 GiB), with split-K sums and an fp16 copy of bf16 activations behind them; where C % 64 != 0 a smaller workspace is
  * taken as well: what 128 x 128 tiles cannot gather themselves (column orders, other tag widths) is all that these need.  Up to SQ_SMALL_BMAX rows the call is

@@ -87,6 +87,20 @@ static FusedPlan fused_plan(const sq_matrix* mats, int n, int T, int cus) {
     return none;
 }
 
+// d = 4 products of the cuts above, in microseconds: a launch of the activations and one of the product, 20 between rounds of workgroups, fitted to
+// 76 of 1700 to 54000 rows at 130 to 768 tokens (9 %).  The kernel of sq_mid.h, in blocks of activation rows, is the faster one for most of
+// them now: 11600 x 3800, 10-bit tags, at 259 rows 68 us here, 42 there; 8300 x 2944 and two of 2093 at 268 62 / 39; 18900 x 1900, 8-bit, at
+// 201 42 / 29; not for 29600 x 2300, 10-bit, at 370 72 / 90, or 15500 x 1200 at 470 37 / 38.  Rows below 512 columns, a launch's length either
+// way, were not measured and stay; a long product runs at a lower clock than both
+// estimates know, hence 85 % and 80 us (26000 x 5600, 10-bit, at 237 rows 95 here, 104 there).
+constexpr int FUSED_MID_C = 512;
+static float fused_us(const FusedPlan& p, const sq_matrix* mats, int n, int cus) {
+    int64_t w = 0;
+    for (int i = 0; i < n; ++i) w += (mats[i].R + 32 * p.tw - 1) / (32 * p.tw);
+    const int64_t rounds = (w * p.ks * p.tbs + cus - 1) / cus;
+    return -4.5f + rounds * (19.6f + mats[0].C * 1e-3f / p.ks * (0.163f * p.tw + 0.809f * p.nw * p.tw + 0.707f * p.nw - 0.217f));
+}
+
 static size_t fused_x_bytes(const sq_matrix* mats, const FusedPlan& p) {
     return (size_t)p.tbs * fused_rounds(mats[0]) * fused_round_steps(mats[0]) * FUSED_TN * p.nw * 1024;
 }
@@ -101,7 +115,10 @@ bool fused_route(const sq_matrix* mats, int n, int T) {
         if (m.d == 8 && ((int64_t)m.G << m.bits) * 16 > ((int64_t)1 << 31)) return false;
         if (m.d == 4 && ((int64_t)m.G << m.bits) * 8 > 128 * 1024) return false;
     }
-    return fused_plan(mats, n, T, device_cus()).nw != 0;
+    const FusedPlan p = fused_plan(mats, n, T, device_cus());
+    if (!p.nw || mats[0].d == 8 || mats[0].C < FUSED_MID_C) return p.nw != 0;
+    const float us = mid_us(mats, n, T);
+    return us > 80.f || us > 0.85f * fused_us(p, mats, n, device_cus());
 }
 
 // For tests: the variant that a stack takes at T rows, as token tiles | weight tiles << 8 | K slices << 16 | token blocks << 24; 0: another kernel.

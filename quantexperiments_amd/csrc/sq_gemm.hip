@@ -148,6 +148,7 @@ int launch_small_generic(const sq_matrix* mats, int n, const void* x, int x_dtyp
 
 bool gemm256_ok(int C, int64_t ldx, int64_t ldw, const void* x, const void* w);
 size_t gemm256_part_bytes(int T, int R, int C, int cus);
+float gemm256_us(int T, int R, int C, int cus);
 int launch_gemm256(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ldw, const Gemm256Scales& sc, void* y,
                    int y_dtype, int64_t ldy, int y_off, int T, int R, int C, float* part, int cus, hipStream_t s);
 int launch_dequant_with_cvt(const sq_matrix& m, void* out, int64_t ld_out, const uint16_t* x, int64_t ldx, int T, int C,
@@ -344,6 +345,20 @@ int vector_decoded(const sq_matrix* mats, int n, int B) {
 
 static size_t gemm_workspace_beyond_small(const sq_matrix* mats, int n, int T);
 
+// Beyond the row counts that always take it, the kernel of sq_mid.h is the faster way for small products: where its estimated
+// time is below 50 us (longer ones run at a lower clock) and 85 % of what decode and tile GEMM take, as fitted to 722 of those (8 %).  There and here, us (700 / 1000 / 1600
+// rows): 1024 x 896, 12-bit tags, 19.9 / 19.6 / 20.2 and 8.2 / 8.5 / 11.0, 3584 x 3584 45.0 / 47.7 / 55.2 and 30.9 / 33.9 / 54.3, 18000 x 1024 43 /
+// 58 / 76 and 45 / 57 / 87; 16-bit, 1024 x 896, 19.2 / 19.1 / 19.8 and 12.5 / 14.9 / 17.9, 3584 x 3584 47 / 51 / 58 and 69 / 80 / 116.
+static bool mid_beyond(const sq_matrix* mats, int n, int T) {
+    float tiles = 11.5f, weights = 0.f;
+    int rows = 0;
+    for (int i = 0; i < n; ++i) weights += (float)mats[i].R * mats[i].C * 1e-6f, rows += mats[i].R;
+    tiles += 0.85f * gemm256_us(T, rows, mats[0].C, device_cus()) + (mats[0].d == 8 ? 0.77f : 0.51f) * weights;
+    const float us = mid_us(mats, n, T);
+    return us < 50.f && us < 0.85f * tiles;
+}
+static bool takes_mid(const sq_matrix* mats, int n, int T) { return mid_ok(mats, n, T) || (T > SQ_SMALL_BMAX && mid_beyond(mats, n, T)); }
+
 size_t gemm_workspace(const sq_matrix* mats, int n, int T) {
     // up to SQ_SMALL_BMAX rows sq_linear_gemm is sq_linear_small, unless the stack goes the other way (see above);
     // which of the two runs then depends on the alignment of x, so the workspace covers both
@@ -357,7 +372,7 @@ static size_t gemm_workspace_beyond_small(const sq_matrix* mats, int n, int T) {
     // decode-time kernel, which the caller adds)
     if (T <= SQ_SMALL_BMAX && decoded_route(mats, n, T)) return decoded_workspace(mats, n, T);
     const size_t rest = std::max(gemm_workspace_without_mid(mats, n, T), fused_route(mats, n, T) ? fused_workspace(mats, n, T) : (size_t)0);
-    if (mid_ok(mats, n, T)) return std::max(rest, mid_workspace(mats, n, T));
+    if (takes_mid(mats, n, T)) return std::max(rest, mid_workspace(mats, n, T));
     return decoded_route(mats, n, T) ? std::max(rest, decoded_workspace(mats, n, T)) : rest;
 }
 
@@ -431,7 +446,7 @@ int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_
         return launch_small(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, ws_bytes, sums, s);
     if (x_vec_ok(x, ldx, mats[0].C) && fused_route(mats, n, T) && fused_workspace(mats, n, T) <= ws_bytes)
         return launch_fused(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);
-    if (mid_ok(mats, n, T) && x_vec_ok(x, ldx, mats[0].C) && mid_x_ok(ldx, T))
+    if (x_vec_ok(x, ldx, mats[0].C) && mid_x_ok(ldx, T) && takes_mid(mats, n, T) && (mid_ok(mats, n, T) || gemm_workspace_without_mid(mats, n, T) <= ws_bytes))
         return launch_mid(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, ws_bytes, s);
     if (T > SQ_SMALL_BMAX && T <= small_pass_limit(mats, n) && x_vec_ok(x, ldx, mats[0].C)) {
         // stacks that cannot go in one pass (pieces of different formats): a few passes of the decode-time kernel read the packed

@@ -713,7 +713,7 @@ __global__ __launch_bounds__(256) void gemm256_reduce_kernel(const float* __rest
 
 // How a T x R output is cut: tiles of 64 mt token rows; whole rounds of whole tiles over the `cus` CUs, and the tiles of
 // the last, partial round split over kt workgroups each (kt = 1: no split) while a part keeps at least 16 slabs.
-struct Gemm256Plan { int mt, main_tiles, tail_tiles, kt; };
+struct Gemm256Plan { int mt, main_tiles, tail_tiles, kt; float us; };
 
 // Tiles of 256 rows read least per product and are the ones for products of many rounds (8192^3: 880 us, 963 with 192 rows,
 // 1019 with 128); where few tiles leave CUs idle, or most of a tile's rows are past the end, smaller ones win.  The plan with the
@@ -734,7 +734,7 @@ static Gemm256Plan gemm256_plan(int T, int R, int C, int cus, bool split) {
     const int slabs = (C + G_BK - 1) / G_BK;
     const bool rounds = cus >= 8 && cus % 8 == 0;
     const int n = rounds ? cus : 256;
-    Gemm256Plan best{4, 0, 0, 1};
+    Gemm256Plan best{4, 0, 0, 1, 0.f};
     double best_t = 1e30;
     for (int mt = 4; mt >= 2; --mt) {
         const int64_t tiles = (int64_t)((T + gemm256_tokens(mt) - 1) / gemm256_tokens(mt)) * ((R + G_BN - 1) / G_BN);
@@ -748,7 +748,7 @@ static Gemm256Plan gemm256_plan(int T, int R, int C, int cus, bool split) {
             if (kt > 1) t += 4.0 + wgs * mt * 0.015;
             if (t < best_t - 1e-9) {
                 best_t = t;
-                best = kt > 1 ? Gemm256Plan{mt, main, tail, kt} : Gemm256Plan{mt, (int)tiles, 0, 1};
+                best = kt > 1 ? Gemm256Plan{mt, main, tail, kt, (float)t} : Gemm256Plan{mt, (int)tiles, 0, 1, (float)t};
             }
         }
     }
@@ -759,6 +759,8 @@ size_t gemm256_part_bytes(int T, int R, int C, int cus) {
     const Gemm256Plan p = gemm256_plan(T, R, C, cus, true);
     return ((size_t)p.tail_tiles * p.kt * gemm256_tokens(p.mt) * G_BN * 4 + 255) & ~(size_t)255;
 }
+
+float gemm256_us(int T, int R, int C, int cus) { return gemm256_plan(T, R, C, cus, true).us; }     // (as estimated, see there)
 
 bool gemm256_ok(int C, int64_t ldx, int64_t ldw, const void* x, const void* w) {
     return C % 8 == 0 && ldx % 8 == 0 && ldw % 8 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0;

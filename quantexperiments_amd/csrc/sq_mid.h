@@ -1,8 +1,10 @@
-// Codebook product for more activation rows than a decode step has and fewer than a prefill: T = 33 .. 256 (384 for large d = 4
-// matrices).
+// Codebook product for more activation rows than a decode step has: T = 33 .. 256 (384 for large d = 4 matrices), and more of them for
+// matrices that are small enough.
 //
 // Decoding the matrix to fp16 first writes and reads eight times its bytes and then multiplies tiles of 256 rows; passes of 32
-// rows through the decode-time kernel gather every codeword once per pass.  Here every codeword is gathered once for all T rows.
+// rows through the decode-time kernel gather every codeword once per pass.  Here every codeword is gathered once for a block of up to 256
+// rows, which are fewer where a launch would leave CUs idle otherwise: what a small product takes is the length of a workgroup's loop (512 x 512
+// at 228 rows 15.7 us in four workgroups, 4.8 in 120; 896 x 896 with 16-bit tags 38 and 8).
 // v_mfma_f32_16x16x32_f16 takes the weights as its A operand (lane l: row l % 16, 8 consecutive k), which are two d = 4
 // codewords (LDS) or one d = 8 codeword (L2), so a lane gathers its operand straight into registers and uses it for all NT
 // tiles of 16 activation rows; the activations are the B operand and come from LDS.
@@ -14,14 +16,16 @@
 // first, at 33 / 77 / 128 / 256 rows: d = 8, 18944 x 2 x 3584: 172 / 205 / 205 / 209 us, here 90 / 96 / 105 / 188 (sq_fused.h: 108);
 // 12-bit: 41 / 68 / 102 / 165, here 27 / 38 / 53 / 105 (82).
 //
-//   workgroup   NW waves, two per SIMD or more so that one gathers while the other multiplies (4 waves: a third slower); each has
-//               TW tiles of 16 weight rows x all NT x 16 activation rows (accumulators TW x NT x 4 registers)
+//   workgroup   NW waves, two per SIMD or more so that one gathers while the other multiplies (4 waves: a third slower, and the choice
+//               where they spread better or a CU takes several); each has TW tiles of 16 weight rows x NT x 16 activation rows
+//               (accumulators TW x NT x 4 registers)
 //   K           in rounds of 4 lane units (UK columns of tags each, as in sq_rows_mfma.h), rounds in stages of S matrix steps;
 //               step j of lane group g is columns (4 round + g) UK + 8 j .. + 7
 //   X           stages of NT x 16 rows x 4 x S x 16 bytes, double buffered in LDS; loaded to registers two stages ahead
 //               (converted bf16 -> fp16 on the way to LDS), one barrier per stage
 //   tags        two rounds ahead; codewords PD steps ahead (one from LDS, three from L2 where the steps are short)
-//   grid        row blocks x ks slices of the rounds; with ks > 1 fp32 partial sums, added by slice_sum_kernel
+//   grid        blocks of weight rows x blocks of activation rows x ks slices of the rounds; with ks > 1 fp32 partial sums, added by
+//               slice_sum_kernel
 //
 // D = 0: weights already decoded to fp16 (column orders, formats whose rows are not whole lane units).  The A operand is loaded
 // from there, up to seven steps ahead; step j of lane group g is columns 256 round + 32 j + 8 g .. + 7, so that the four lane groups
@@ -57,7 +61,7 @@ struct MidArgs {
     void* y;
     int64_t ldy;
     int T, x_dtype, y_dtype;
-    int U, ks, table_bytes;
+    int U, ks, tbs, table_bytes; // tbs: blocks of 16 NT activation rows
     int wide;                    // 1: bf16 activations keep their range (WIDE; decoded weights, up to 48 activation rows)
 };
 
@@ -87,9 +91,11 @@ __global__ __launch_bounds__(64 * NW, 2) void mid_kernel(MidArgs a) {
     while (pi + 1 < a.n && (int)blockIdx.x >= a.p[pi + 1].wg0) ++pi;
     const MidPiece& P = a.p[pi];
     const sq_matrix& m = P.m;
-    const int w = (int)blockIdx.x - P.wg0, slice = w % a.ks, blk = w / a.ks;
+    int blk = (int)blockIdx.x - P.wg0, slice = 0, tok0 = 0;                          // blocks of weight rows, of activation rows in them, slices in those
+    if (a.ks > 1) { const int w = blk; blk = (int)((uint32_t)w / (uint32_t)a.ks); slice = w - blk * a.ks; }
+    if (a.tbs > 1) { const int w = blk; blk = (int)((uint32_t)w / (uint32_t)a.tbs); tok0 = (w - blk * a.tbs) * (16 * NT); }
     const int NR = (a.U + UPR - 1) / UPR, NP = (NR + 1) >> 1;                       // rounds, and pairs of them: slices are whole pairs
-    const int r0 = 2 * (int)((int64_t)NP * slice / a.ks), r1 = min(NR, 2 * (int)((int64_t)NP * (slice + 1) / a.ks));
+    const int r0 = 2 * (int)((uint32_t)(NP * slice) / (uint32_t)a.ks), r1 = min(NR, 2 * (int)((uint32_t)(NP * (slice + 1)) / (uint32_t)a.ks));
     unsigned char* xbuf = smem + a.table_bytes;
 
     // ---- this wave's tiles (tiles past the last row repeat the last one and are not stored)
@@ -119,7 +125,7 @@ __global__ __launch_bounds__(64 * NW, 2) void mid_kernel(MidArgs a) {
     for (int k = 0; k < PCS; ++k) {
         const int q = min(tid + NTH * k, NT * 64 * S - 1), t = q / (4 * S), c = q - t * (4 * S), g = c / S, j = c - g * S;
         xg[k] = DENSE ? j * 4 + g : g;
-        xo[k] = ((uint32_t)min(t, a.T - 1) * (uint32_t)a.ldx + (uint32_t)(g * GC + j * JC)) * 2u;
+        xo[k] = ((uint32_t)min(tok0 + t, a.T - 1) * (uint32_t)a.ldx + (uint32_t)(g * GC + j * JC)) * 2u;
         xl[k] = (uint32_t)(t * ROWB + ((c ^ mid_swizzle<S>(t & 15)) << 4));
     }
     // columns past the row's end (the last round's missing units, rounds past the slice) are zeros; what is read in their
@@ -280,7 +286,7 @@ __global__ __launch_bounds__(64 * NW, 2) void mid_kernel(MidArgs a) {
         for (int e = 0; e < 4; ++e) sc[e] = h2f(m.row_scale[min(r + e, m.R - 1)]);
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
-            const int t = n * 16 + li;
+            const int t = tok0 + n * 16 + li;
             if (t >= a.T) continue;
             if (a.ks > 1) {
                 float* o = P.part + ((int64_t)slice * a.T + t) * m.R + r;
@@ -326,22 +332,21 @@ int launch_mid_as(const MidArgs& a, int grid, hipStream_t s) {
     return a.x_dtype == SQ_BF16 ? launch_mid_dtype<BITS, D, NT, TW, S, NW, true>(a, grid, s) : launch_mid_dtype<BITS, D, NT, TW, S, NW, false>(a, grid, s);
 }
 
-// A variant per number of activation tiles; stages half as deep where many tiles or the codebook leave no room in LDS.
-#define SQ_MID_CASE(NT_, TW_, S_, NW_) if (nt == NT_ && tw == TW_ && st == S_ && nw == NW_) return launch_mid_as<BITS, D, NT_, TW_, S_, NW_>(a, grid, s);
+// Variants: sq_mid.hip
+#define SQ_MID_CASE(NT_, TW_, NW_, S_) if (nt == NT_ && tw == TW_ && nw == NW_ && st == S_) return launch_mid_as<BITS, D, NT_, TW_, S_, NW_>(a, grid, s);
 template <int BITS, int D>
 int launch_mid_format(const MidArgs& a, int nt, int tw, int st, int nw, int grid, hipStream_t s) {
-    if constexpr (D == 0) { SQ_MID_CASE(1, 2, 4, 8) SQ_MID_CASE(1, 1, 4, 8) }
-    SQ_MID_CASE(3, 2, 4, 8) SQ_MID_CASE(3, 1, 4, 8) SQ_MID_CASE(5, 2, 4, 8) SQ_MID_CASE(5, 1, 4, 8) SQ_MID_CASE(8, 2, 4, 8) SQ_MID_CASE(8, 1, 4, 8)
-    SQ_MID_CASE(12, 2, 2, 8) SQ_MID_CASE(12, 1, 2, 8) SQ_MID_CASE(16, 1, 2, 8)
+    SQ_MID_CASE(1, 1, 8, 4) SQ_MID_CASE(3, 1, 8, 4) SQ_MID_CASE(5, 1, 8, 4) SQ_MID_CASE(8, 1, 8, 4)
+    if constexpr (D != 4) { SQ_MID_CASE(12, 1, 8, 2) SQ_MID_CASE(16, 1, 8, 2) }
     if constexpr (D != 0) {
-        SQ_MID_CASE(3, 1, 4, 10) SQ_MID_CASE(3, 1, 4, 12) SQ_MID_CASE(5, 1, 4, 10) SQ_MID_CASE(5, 1, 4, 12) SQ_MID_CASE(12, 1, 2, 12)
+        SQ_MID_CASE(1, 1, 4, 4) SQ_MID_CASE(2, 1, 4, 4) SQ_MID_CASE(3, 1, 4, 4) SQ_MID_CASE(4, 1, 4, 4) SQ_MID_CASE(5, 1, 4, 4)
+        SQ_MID_CASE(4, 1, 8, 4) SQ_MID_CASE(5, 2, 8, 4) SQ_MID_CASE(8, 2, 8, 4)
+        SQ_MID_CASE(3, 1, 10, 4) SQ_MID_CASE(3, 1, 12, 4) SQ_MID_CASE(5, 1, 10, 4) SQ_MID_CASE(5, 1, 12, 4)
     }
-    if constexpr (D == 8) { SQ_MID_CASE(8, 1, 4, 12) }
-    if constexpr (D != 4) {
-        SQ_MID_CASE(16, 2, 2, 8)
-    } else {
-        SQ_MID_CASE(3, 2, 2, 8) SQ_MID_CASE(3, 1, 2, 8) SQ_MID_CASE(5, 2, 2, 8) SQ_MID_CASE(5, 1, 2, 8) SQ_MID_CASE(8, 2, 2, 8) SQ_MID_CASE(8, 1, 2, 8)
-        SQ_MID_CASE(3, 1, 2, 10) SQ_MID_CASE(3, 1, 2, 12) SQ_MID_CASE(5, 1, 2, 10) SQ_MID_CASE(5, 1, 2, 12)
+    if constexpr (D == 8) { SQ_MID_CASE(8, 1, 12, 4) SQ_MID_CASE(12, 1, 12, 2) SQ_MID_CASE(12, 2, 8, 2) SQ_MID_CASE(16, 2, 8, 2) }
+    if constexpr (D == 4) {
+        SQ_MID_CASE(2, 1, 8, 4) SQ_MID_CASE(3, 2, 8, 4) SQ_MID_CASE(4, 2, 8, 4)
+        SQ_MID_CASE(5, 1, 8, 2) SQ_MID_CASE(8, 1, 8, 2) SQ_MID_CASE(5, 2, 8, 2) SQ_MID_CASE(8, 2, 8, 2)
     }
     return SQ_EUNSUPPORTED;
 }

@@ -1,4 +1,4 @@
-// Host side of the product for 33 to 256 (384) activation rows (kernel: sq_mid.h): which stacks it takes, and how the work
+// Host side of the product for 33 and more activation rows (kernel: sq_mid.h): which stacks it takes, and how the work
 // is cut.
 #include <algorithm>
 #include "sq_mid.h"
@@ -12,68 +12,90 @@ int launch_mid_b10d4(const MidArgs&, int, int, int, int, int, hipStream_t);
 int launch_mid_b8d4(const MidArgs&, int, int, int, int, int, hipStream_t);
 int launch_mid_dense(const MidArgs&, int, int, int, int, int, hipStream_t);
 
-struct MidPlan { int nt, tw, st, ks, nw; };
+struct MidPlan { int nt, tw, nw, st, ks; float us; };
 
 static int mid_units(const sq_matrix& m) { return m.W / (m.bits == 12 ? 3 : m.bits == 10 ? 5 : 4); }
 
-// Variants: NT tiles of 16 activation rows (up to 256 rows; a 24-tile variant ran at half the rate), stages of four matrix steps
-// or, where they do not fit beside the codebook, two.  A workgroup is 8 waves of a tile of weight rows, which a CU takes two of no
-// faster than one after the other; where that is more workgroups than CUs, ten or twelve waves if one round is then enough, else
-// two tiles per wave, which halves the activations' way through LDS.  18944 x 2 rows in 148 workgroups of 8 x 2 tiles / 237 of ten
-// (198 of twelve at 128 and 192 activation rows), us, at 40 / 77 / 128 / 192: 10-bit tags 31 / 42 / 55 / 78 and 27 / 37 / 57 (not
-// taken) / 71, 16-bit ones of width 8 100 / 109 / 115 / 142 and 90 / 96 / 105 / 135.  Fewer rows are cut along K until there is about one
-// workgroup per CU, in slices of at least 512 columns (3584 x 3584 at 77 rows, 28 blocks: 28 us whole, 18 in seven).
-static MidPlan mid_plan(const sq_matrix* mats, int n, int T, int cus) {
-    MidPlan p{0, 1, 4, 1, 8};
-    const int sizes[] = {3, 5, 8, 12, 16};
-    for (int nt : sizes) if (T <= nt * 16) { p.nt = nt; break; }
-    if (p.nt == 0) return p;
-    const int tab = mats[0].d == 4 ? (mats[0].G << mats[0].bits) * 8 : 0;
-    if (p.nt > 8 || tab + 2 * mid_stage_bytes(p.nt, 4) > 160 * 1024) p.st = 2;
-    if (tab + 2 * mid_stage_bytes(p.nt, p.st) > 160 * 1024) { p.nt = 0; return p; }
-    int64_t rows = 0;
-    for (int i = 0; i < n; ++i) rows += mats[i].R;
-    auto workgroups = [&](int nw) {
-        int64_t w = 0;
-        for (int i = 0; i < n; ++i) w += (mats[i].R + 16 * nw - 1) / (16 * nw);
-        return w;
-    };
-    if (p.nt == 16 ? rows >= (int64_t)cus / 2 * 32 * 8 : workgroups(8) > cus) {
-        if (p.nt <= 5 && workgroups(10) <= cus) p.nw = 10;
-        else if (p.nt <= 12 && !(p.nt == 8 && mats[0].d == 4) && workgroups(12) <= cus) p.nw = 12;
-        else p.tw = 2;
-    }
-    const int64_t blocks = (rows + 16 * p.nw * p.tw - 1) / (16 * p.nw * p.tw);
-    p.ks = (int)std::max<int64_t>(1, std::min<int64_t>({cus / std::max<int64_t>(blocks, 1), 8, mats[0].C / 512}));
-    return p;
-}
+// The variants: workgroups of NW waves, each with TW tiles of 16 weight rows x NT tiles of 16 activation rows, those of a stack cut into
+// blocks of NT; and K slices, whose sums cost a launch.  Which one is taken is estimated from what a workgroup's matrix steps cost its CU
+// (products, reads of activations by every wave, codewords, activations on their way into LDS) and how long a step takes that waits for nothing
+// but itself, as the constants below say; d = 8 also from the rate at which L2 serves the whole chip's codewords.  They are fitted to 1852 products
+// of 200 .. 30000 rows of 512 .. 18944 columns at 33 .. 2048 activation rows in 10 to 130 cuts each, to 10 %
+// (single tiles take 14 % longer than they say); the cut that is taken then is 2 % slower than the best one in the mean, in one case of ten by 9 % (d = 4),
+// 6 % (d = 8).  In one block of all activation rows and eight waves,
+// the cut of before, and so, us (77 / 228 / 700 activation rows, beyond 256 decoded and in tiles before):
+//   rows x columns   12-bit tags, d = 4                              16-bit tags, d = 8
+//   512 x 512        8.4 / 15.7 / 15.4     4.7 / 4.8 / 5.4           9.0 / 15.6 / 14.7     5.3 / 5.9 / 7.0
+//   1024 x 896      11.2 / 23.6 / 19.9     5.7 / 5.8 / 8.2          12.0 / 23.0 / 19.2     7.3 / 8.3 / 12.5
+//   4096 x 1024     12.3 / 23.4 / 23.6     6.6 / 8.8 / 13.7         13.8 / 24.0 / 25.0    10.0 / 17.2 / 23.7
+//   3584 x 3584     15.8 / 30.5 / 45.0    13.3 / 18.8 / 30.9        21.6 / 36.1 / 46.8    21.8 / 36.3 / 68.6 (not taken)
+//   8000 x 2048     17.6 / 35.1 / 40.4    11.3 / 16.5 / 35.7
+struct MidVariant { int8_t nt, tw, nw, st; };
+static constexpr MidVariant MID4[] = {{1, 1, 4, 4}, {2, 1, 4, 4}, {3, 1, 4, 4}, {4, 1, 4, 4}, {5, 1, 4, 4}, {1, 1, 8, 4}, {2, 1, 8, 4}, {3, 1, 8, 4}, {4, 1, 8, 4},
+                                      {5, 1, 8, 4}, {8, 1, 8, 4}, {3, 2, 8, 4}, {4, 2, 8, 4}, {5, 2, 8, 4}, {8, 2, 8, 4}, {3, 1, 10, 4}, {3, 1, 12, 4}, {5, 1, 10, 4},
+                                      {5, 1, 12, 4}, {5, 1, 8, 2}, {8, 1, 8, 2}, {5, 2, 8, 2}, {8, 2, 8, 2}};
+static constexpr MidVariant MID8[] = {{1, 1, 4, 4}, {2, 1, 4, 4}, {3, 1, 4, 4}, {4, 1, 4, 4}, {5, 1, 4, 4}, {3, 1, 8, 4}, {4, 1, 8, 4}, {5, 1, 8, 4}, {8, 1, 8, 4},
+                                      {12, 1, 8, 2}, {16, 1, 8, 2}, {3, 1, 10, 4}, {3, 1, 12, 4}, {5, 1, 10, 4}, {5, 1, 12, 4}, {8, 1, 12, 4}, {12, 1, 12, 2}, {5, 2, 8, 4},
+                                      {8, 2, 8, 4}, {12, 2, 8, 2}, {16, 2, 8, 2}};
+// us: a launch; staged codebooks per KB and round of workgroups; per matrix step of a workgroup: a wave's product, its read of a tile of
+// activations, a tile of codewords, a tile of activations staged; a step by itself, per tile, and per tile that a wave stages; slices: their launch, and per million sums;
+// per million results; per tile of codewords over the chip
+struct MidCost { float launch, table, product, read, words, stage, wait, wait_tile, wait_stage, slices, sums, results, chip; };
+static constexpr MidCost MID_COST4 = {4.04f, 0.0179f, 0.00132f, 0.00139f, 0.00346f, 0.00832f, 0.0385f, 0.0083f, 0.0362f, 3.14f, 3.16f, 1.86f, 2.1e-5f};
+static constexpr MidCost MID_COST8 = {3.49f, 0.f, 0.00198f, 0.00198f, 0.0168f, 0.0109f, 0.0121f, 0.f, 0.f, 3.38f, 2.87f, 1.09f, 2.74e-4f};
 
-// Activation rows one launch takes: all T, or half of them (whole tiles) where T is more than fits beside the codebook and where
-// sixteen tiles of activations and two of weights need more registers than leave room to fetch ahead (18944 x 2 rows at 256
-// activation rows, 12-bit tags: 133 us at once, 108 us in two; d = 8, bound by its gathers, 188 against 224).
-static int mid_rows(const sq_matrix* mats, int n, int T) {
-    for (int parts = 1; parts <= 2; ++parts) {
-        const int rows = parts == 1 ? T : (T + 31) / 32 * 16;
-        const MidPlan p = mid_plan(mats, n, rows, device_cus());
-        if (p.nt && !(mats[0].d == 4 && p.nt == 16 && p.tw == 2)) return rows;
-    }
-    return 0;
+static int64_t mid_blocks(const sq_matrix* mats, int n, int rows) {       // of `rows` weight rows
+    int64_t w = 0;
+    for (int i = 0; i < n; ++i) w += (mats[i].R + rows - 1) / rows;
+    return w;
 }
-
-// Activation rows up to which this is the faster way.  Decode + tile GEMM costs the decode once and a tile of 256 rows whatever is
-// in it, so it is level at 256 rows (d = 8, 18944 x 2: 188 us here, 205 there) and ahead above, except for large d = 4 matrices,
-// whose decode is the longest part (18944 x 2 rows at 384: 162 us here, 206 there; 3584 x 18944: 109 and 127; 3584 x 3584: 56
-// and 49).
-static int mid_limit(const sq_matrix* mats, int n) {
-    int64_t weights = 0;
-    for (int i = 0; i < n; ++i) weights += (int64_t)mats[i].R * mats[i].C;
-    return mats[0].d == 4 && weights >= (int64_t)1 << 26 ? 384 : 256;
-}
+static int mid_lds(const MidVariant& v, int table) { return table + 2 * mid_stage_bytes(v.nt, v.st); }
 
 static size_t mid_part_bytes(const sq_matrix& m, int T, int ks) { return ks > 1 ? (((size_t)ks * T * m.R * 4) + 255) & ~(size_t)255 : 0; }
+static size_t mid_sums_bytes(const sq_matrix* mats, int n, int T, int ks) {
+    size_t need = 0;
+    for (int i = 0; i < n; ++i) need += mid_part_bytes(mats[i], T, ks);
+    return need;
+}
 
-// the pieces share format, row length and codebook size, and the kernel takes them at T rows
-bool mid_ok(const sq_matrix* mats, int n, int T) {
+// The cut with the least estimated time whose sums of slices take at most `room` bytes
+static MidPlan mid_plan(const sq_matrix* mats, int n, int T, int cus, size_t room) {
+    const bool d4 = mats[0].d == 4;
+    const int table = d4 ? (mats[0].G << mats[0].bits) * 8 : 0, pairs = ((mid_units(mats[0]) + 3) / 4 + 1) / 2;   // of rounds
+    const MidCost& c = d4 ? MID_COST4 : MID_COST8;
+    const MidVariant* vs = d4 ? MID4 : MID8;
+    const int count = d4 ? (int)(sizeof(MID4) / sizeof(MID4[0])) : (int)(sizeof(MID8) / sizeof(MID8[0]));
+    int64_t rows = 0;
+    for (int i = 0; i < n; ++i) rows += mats[i].R;
+    const float results = (float)rows * T * 1e-6f, pair_steps = mats[0].bits == 12 ? 8.f : 16.f;
+    MidPlan best{0, 1, 8, 4, 1, 1e30f};
+    for (int k = 0; k < count; ++k) {
+        const MidVariant& v = vs[k];
+        const int lds = mid_lds(v, table);
+        if (lds > 160 * 1024 || (v.st == 2 && v.nt <= 8 && mid_lds({v.nt, v.tw, v.nw, 4}, table) <= 160 * 1024)) continue;
+        if (v.nt > 1 && v.nt * 16 >= 2 * T) continue;                     // (more than half of it past the last row)
+        // workgroups that a CU runs side by side, by its LDS and registers
+        const int beside = std::max(1, std::min({160 * 1024 / lds, 4 * (512 / (40 + 6 * v.nt + 4 * v.nt * v.tw)) / v.nw, 32 / v.nw}));
+        const int64_t whole = mid_blocks(mats, n, 16 * v.nw * v.tw) * ((T + 16 * v.nt - 1) / (16 * v.nt));
+        if (!d4 && v.tw == 2 && whole < cus) continue;                    // (bound by its codewords, two tiles of which a wave cannot fetch far enough ahead)
+        const int most = (int)std::min<int64_t>({std::max<int64_t>(1, cus / whole), 8, pairs});
+        const float step = (v.nw + 3) / 4 * 4 * v.tw * (c.product * v.nt + c.words) + c.read * v.nw * v.nt + c.stage * v.nt;      // (ten waves: three on a SIMD)
+        for (int cut = 0; cut < 3; ++cut) {
+            const int ks = cut == 0 ? 1 : cut == 1 ? most : most / 2;
+            if (cut && ks < 2) continue;
+            const int64_t wgs = whole * ks, rounds = (wgs + cus - 1) / cus, waits = (rounds + beside - 1) / beside;
+            const float s = pair_steps * ((pairs + ks - 1) / ks);
+            const float work = rounds * s * step, wait = waits * s * (c.wait + c.wait_tile * v.nt * v.tw + c.wait_stage * v.nt / v.nw), chip = wgs * s * v.nw * v.tw * c.chip;
+            const float us = c.launch + c.table * (table >> 10) * waits + (v.nt == 1 ? 1.14f : 1.f) * __builtin_sqrtf(work * work + wait * wait + chip * chip) +
+                             (ks > 1 ? c.slices + c.sums * ks * results : 0.f) + c.results * results;
+            if (us < best.us && (ks == 1 || mid_sums_bytes(mats, n, T, ks) <= room)) best = {v.nt, v.tw, v.nw, v.st, ks, us};
+        }
+    }
+    return best;
+}
+
+// the pieces share format, row length and codebook size, and the kernel takes them
+static bool mid_shape(const sq_matrix* mats, int n, int T) {
     if (n < 1 || n > MID_PIECES || T <= SQ_SMALL_BMAX) return false;
     for (int i = 0; i < n; ++i) {
         const sq_matrix &m = mats[i], &m0 = mats[0];
@@ -82,14 +104,55 @@ bool mid_ok(const sq_matrix* mats, int n, int T) {
         if (((int64_t)m.R + 16) * m.W * 4 >= ((int64_t)1 << 32)) return false;                 // 32-bit offsets
         if (m.d == 8 && ((int64_t)m.G << m.bits) * 16 > ((int64_t)1 << 31)) return false;
     }
-    return T <= mid_limit(mats, n) && mid_rows(mats, n, T) != 0;
+    return true;
+}
+
+// Activation rows that always run here: 256, and 384 of large d = 4 matrices.
+static int mid_limit(const sq_matrix* mats, int n) {
+    int64_t weights = 0;
+    for (int i = 0; i < n; ++i) weights += (int64_t)mats[i].R * mats[i].C;
+    return mats[0].d == 4 && weights >= (int64_t)1 << 26 ? 384 : 256;
+}
+
+bool mid_ok(const sq_matrix* mats, int n, int T) { return mid_shape(mats, n, T) && T <= mid_limit(mats, n); }
+
+// What a workspace has to hold up to there: the sums of as many slices as the kernel took when a launch had one block of all activation
+// rows (or half of them).  Cuts that need more than there is are passed over.
+static size_t mid_least(const sq_matrix* mats, int n, int T) {
+    const int cus = device_cus(), table = mats[0].d == 4 ? (mats[0].G << mats[0].bits) * 8 : 0;
+    int64_t rows = 0;
+    for (int i = 0; i < n; ++i) rows += mats[i].R;
+    for (int parts = 1; parts <= 2; ++parts) {
+        const int t = parts == 1 ? T : (T + 31) / 32 * 16, nt = t <= 48 ? 3 : t <= 80 ? 5 : t <= 128 ? 8 : t <= 192 ? 12 : 16;
+        int nw = 8, tw = 1;
+        if (t > 256 || table + 2 * mid_stage_bytes(nt, 2) > 160 * 1024) continue;
+        if (nt == 16 ? rows >= (int64_t)cus / 2 * 32 * 8 : mid_blocks(mats, n, 16 * 8) > cus) {
+            if (nt <= 5 && mid_blocks(mats, n, 16 * 10) <= cus) nw = 10;
+            else if (nt <= 12 && !(nt == 8 && mats[0].d == 4) && mid_blocks(mats, n, 16 * 12) <= cus) nw = 12;
+            else tw = 2;
+        }
+        if (mats[0].d == 4 && nt == 16 && tw == 2) continue;
+        const int64_t blocks = (rows + 16 * nw * tw - 1) / (16 * nw * tw);
+        const int ks = (int)std::max<int64_t>(1, std::min<int64_t>({cus / std::max<int64_t>(blocks, 1), 8, mats[0].C / 512}));
+        return mid_sums_bytes(mats, n, t, ks);
+    }
+    return 0;
 }
 
 size_t mid_workspace(const sq_matrix* mats, int n, int T) {
-    const MidPlan p = mid_plan(mats, n, mid_rows(mats, n, T), device_cus());
-    size_t need = 0;
-    for (int i = 0; i < n; ++i) need += mid_part_bytes(mats[i], mid_rows(mats, n, T), p.ks);
-    return need;
+    const MidPlan p = mid_plan(mats, n, T, device_cus(), SIZE_MAX);
+    const size_t need = mid_sums_bytes(mats, n, T, p.ks);
+    return T <= mid_limit(mats, n) ? std::max(need, mid_least(mats, n, T)) : need;
+}
+
+// Estimated time at T rows; a very long one where the kernel does not take the pieces
+float mid_us(const sq_matrix* mats, int n, int T) { return mid_shape(mats, n, T) ? mid_plan(mats, n, T, device_cus(), SIZE_MAX).us : 1e30f; }
+
+// For tests: the cut that a stack takes at T rows, as token tiles | weight tiles << 8 | waves << 16 | K slices << 24; 0: the kernel does not take it.
+extern "C" __attribute__((visibility("default"))) int32_t sq_mid_variant_for_tests(const sq_matrix* mats, int32_t n, int32_t T) {
+    if (!mid_shape(mats, n, T)) return 0;
+    const MidPlan p = mid_plan(mats, n, T, device_cus(), SIZE_MAX);
+    return p.nt | p.tw << 8 | p.nw << 16 | p.ks << 24;
 }
 
 static int launch_mid_rows(const sq_matrix* mats, int n, const MidPlan& pl, const void* const* dense, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype,
@@ -98,7 +161,7 @@ static int launch_mid_rows(const sq_matrix* mats, int n, const MidPlan& pl, cons
     const sq_matrix& m0 = mats[0];
     a.n = n;
     a.x = (const uint16_t*)x; a.ldx = ldx; a.y = y; a.ldy = ldy; a.T = T; a.x_dtype = x_dtype; a.y_dtype = y_dtype;
-    a.U = dense ? m0.C / 8 : mid_units(m0); a.ks = pl.ks;
+    a.U = dense ? m0.C / 8 : mid_units(m0); a.ks = pl.ks; a.tbs = (T + 16 * pl.nt - 1) / (16 * pl.nt);
     a.wide = wide;
     a.table_bytes = !dense && m0.d == 4 ? (m0.G << m0.bits) * 8 : 0;
     int wg = 0;
@@ -111,7 +174,7 @@ static int launch_mid_rows(const sq_matrix* mats, int n, const MidPlan& pl, cons
         P.part = (float*)part;
         part += mid_part_bytes(m, T, pl.ks);
         P.wg0 = wg;
-        wg += ((m.R + 16 * pl.nw * pl.tw - 1) / (16 * pl.nw * pl.tw)) * pl.ks;
+        wg += ((m.R + 16 * pl.nw * pl.tw - 1) / (16 * pl.nw * pl.tw)) * pl.ks * a.tbs;
     }
     int rc = SQ_EUNSUPPORTED;
     if (dense) rc = launch_mid_dense(a, pl.nt, pl.tw, pl.st, pl.nw, wg, s);
@@ -127,7 +190,7 @@ static int launch_mid_rows(const sq_matrix* mats, int n, const MidPlan& pl, cons
 // with two), K slices of 256 columns at least, up to eight (3584 x 18944 at 64 rows: 99 us with the decode, 119 in four slices,
 // 111 in nine).
 static MidPlan mid_dense_plan(const sq_matrix* mats, int n, int T, int cus) {
-    MidPlan p{0, 1, 4, 1, 8};
+    MidPlan p{0, 1, 8, 4, 1, 0.f};
     const int sizes[] = {1, 3, 5, 8, 12, 16};
     for (int nt : sizes) if (T <= nt * 16) { p.nt = nt; break; }
     if (p.nt > 8) p.st = 2;
@@ -144,12 +207,7 @@ bool mid_dense_ok(const sq_matrix* mats, int n, int T) {
     return true;
 }
 
-size_t mid_dense_workspace(const sq_matrix* mats, int n, int T) {
-    const MidPlan p = mid_dense_plan(mats, n, T, device_cus());
-    size_t need = 0;
-    for (int i = 0; i < n; ++i) need += mid_part_bytes(mats[i], T, p.ks);
-    return need;
-}
+size_t mid_dense_workspace(const sq_matrix* mats, int n, int T) { return mid_sums_bytes(mats, n, T, mid_dense_plan(mats, n, T, device_cus()).ks); }
 
 int launch_mid_decoded(const sq_matrix* mats, int n, const void* const* w, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T,
                        void* ws, hipStream_t s, bool wide) {
@@ -158,15 +216,8 @@ int launch_mid_decoded(const sq_matrix* mats, int n, const void* const* w, const
 
 int launch_mid(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws,
                size_t ws_bytes, hipStream_t s) {
-    if (mid_workspace(mats, n, T) > ws_bytes) return fail(SQ_EWORKSPACE, "sq_linear_gemm: workspace %zu < %zu", ws_bytes, mid_workspace(mats, n, T));
-    const int rows = mid_rows(mats, n, T);
-    const MidPlan pl = mid_plan(mats, n, rows, device_cus());
-    for (int t = 0; t < T; t += rows) {
-        const int rc = launch_mid_rows(mats, n, pl, nullptr, (const char*)x + (size_t)t * ldx * 2, x_dtype, ldx,
-                                       (char*)y + (size_t)t * ldy * (y_dtype == SQ_F32 ? 4 : 2), y_dtype, ldy, std::min(rows, T - t), ws, s);
-        if (rc) return rc;
-    }
-    return SQ_OK;
+    if (T <= mid_limit(mats, n) && mid_least(mats, n, T) > ws_bytes) return fail(SQ_EWORKSPACE, "sq_linear_gemm: workspace %zu < %zu", ws_bytes, mid_workspace(mats, n, T));
+    return launch_mid_rows(mats, n, mid_plan(mats, n, T, device_cus(), ws_bytes), nullptr, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);
 }
 
 }  // namespace sq

@@ -1,4 +1,4 @@
-"""Products of 33 to 384 activation rows in one pass over the tags: edges of the tiles of rows and activation rows, a last round
+"""Products of 33 to 2048 activation rows whose codewords are gathered once per block of them: edges of the tiles of rows and activation rows, a last round
 with missing units, odd numbers of rounds, K slices, stacks, several codebooks, two tiles of rows per wave, two parts of rows; and
 of 3 to 256 rows with weights decoded first."""
 
@@ -41,6 +41,69 @@ def test_one_pass_matches_oracle(case, dtype, stream):
     linear_gemm(lins, x.cuda(), lowp)
     assert torch.equal(lowp, y.to(dtype))
     assert np.isfinite(lowp.float().cpu().numpy()).all()
+
+
+# rows of the stack's pieces, C, d, bits, G, T, and the cut: tiles of activation rows, tiles of weight rows, waves, K slices.  The last block of
+# activation rows and the last tile of weight rows are broken, products beyond 256 rows among them.
+CUTS = [
+    ((1,), 32, 4, 12, 1, 33, (1, 1, 4, 1)), ((17,), 1600, 4, 10, 1, 34, (1, 1, 4, 4)), ((8218,), 32, 4, 12, 1, 33, (1, 1, 8, 1)),
+    ((5383, 5), 32, 4, 12, 1, 50, (2, 1, 4, 1)), ((8229,), 96, 4, 12, 1, 66, (2, 1, 8, 1)), ((16854,), 32, 4, 12, 1, 35, (3, 1, 8, 1)),
+    ((16647,), 32, 4, 12, 1, 65, (3, 1, 10, 1)), ((41028,), 32, 4, 12, 1, 33, (3, 1, 12, 1)), ((16769,), 32, 4, 12, 1, 99, (3, 2, 8, 1)),
+    ((20862,), 32, 4, 12, 1, 49, (4, 1, 8, 1)), ((41153,), 32, 4, 12, 1, 53, (4, 2, 8, 1)), ((25822,), 32, 4, 12, 1, 66, (5, 1, 8, 1)),
+    ((33221,), 32, 4, 12, 1, 67, (5, 1, 10, 1)), ((41558,), 32, 4, 12, 1, 70, (5, 1, 12, 1)), ((41228,), 32, 4, 12, 1, 206, (5, 2, 8, 1)),
+    ((700,), 512, 4, 12, 1, 1000, (2, 1, 8, 1)), ((3584,), 1024, 4, 8, 1, 385, (3, 1, 8, 1)), ((9000,), 2080, 4, 12, 1, 900, (5, 2, 8, 1)),
+    ((8588,), 32, 4, 12, 4, 33, (1, 1, 8, 1)), ((16934,), 32, 4, 12, 4, 99, (3, 2, 8, 1)), ((25828,), 32, 4, 12, 4, 68, (5, 1, 8, 1)),
+    ((33375,), 32, 4, 12, 4, 67, (5, 2, 8, 1)), ((33294,), 32, 4, 12, 4, 81, (8, 2, 8, 1)), ((3000, 50), 640, 4, 10, 4, 700, (3, 1, 12, 1)),
+    ((1,), 64, 8, 16, 1, 33, (1, 1, 4, 1)), ((1217,), 64, 8, 16, 1, 50, (2, 1, 4, 1)), ((3,), 2112, 8, 16, 1, 250, (2, 1, 4, 5)),
+    ((560, 33), 2112, 8, 16, 1, 33, (3, 1, 4, 5)), ((17153,), 64, 8, 16, 1, 34, (3, 1, 8, 1)), ((33795,), 64, 8, 16, 1, 33, (3, 1, 10, 1)),
+    ((41550,), 64, 8, 16, 1, 37, (3, 1, 12, 1)), ((1091,), 1664, 8, 16, 2, 51, (4, 1, 4, 4)), ((3571,), 2112, 8, 16, 1, 49, (4, 1, 8, 5)),
+    ((4587,), 64, 8, 16, 1, 67, (5, 1, 4, 1)), ((5448,), 64, 8, 16, 1, 194, (5, 1, 8, 1)), ((33034,), 64, 8, 16, 1, 51, (5, 1, 10, 1)),
+    ((41105,), 64, 8, 16, 1, 49, (5, 1, 12, 1)), ((13449,), 64, 8, 16, 1, 83, (8, 1, 8, 1)), ((33589,), 64, 8, 16, 1, 84, (8, 1, 12, 1)),
+    ((16757,), 64, 8, 16, 1, 133, (12, 1, 8, 1)), ((32985,), 64, 8, 16, 1, 138, (12, 1, 12, 1)), ((16805,), 64, 8, 16, 1, 195, (16, 1, 8, 1)),
+    ((600,), 512, 8, 16, 1, 1300, (5, 1, 4, 1)),
+]
+
+
+@pytest.mark.parametrize("case", CUTS, ids=lambda c: "x".join(map(str, c[:-1])))
+@pytest.mark.parametrize("dtype,stream", [(torch.bfloat16, True), (torch.float16, False)], ids=["bf16-tiled", "f16-rows"])
+def test_cuts_match_oracle(case, dtype, stream):
+    rows, C, d, bits, G, T, cut = case
+    ss = [synth(R, C, d, bits, G, 1, seed=R + T) for R in rows]
+    lins = [to_device(s, stream=stream and d == 4) for s in ss]
+    v = _lib.lib().sq_mid_variant_for_tests(_lib.matrix_array([m.descriptor() for m in lins]), len(lins), T)
+    # (the figures of the estimate are for 256 compute units)
+    assert torch.cuda.get_device_properties(0).multi_processor_count != 256 or tuple(v >> k & 255 for k in (0, 8, 16, 24)) == cut
+    x = torch.zeros(T, C + 8, dtype=dtype)
+    x[:, :C] = rand_x(T, C, dtype, seed=T)
+    xd = x.cuda()[:, :C]
+    ref = torch.cat([xd.double() @ torch.from_numpy(s.decode()).cuda().double().T for s in ss], dim=1)
+    y = torch.empty(T, sum(rows), dtype=torch.float32, device="cuda")
+    linear_gemm(lins, xd, y)
+    # products of fp16 values are exact in fp32, whose sums of C terms round at 2^-24 of a partial sum
+    assert rel_max_err(y.cpu().numpy(), ref.cpu().numpy()) < 1e-5
+    lowp = torch.zeros(T, sum(rows) + 8, dtype=dtype, device="cuda")
+    linear_gemm(lins, xd, lowp[:, :sum(rows)])
+    assert torch.equal(lowp[:, :sum(rows)], y.to(dtype)) and not lowp[:, sum(rows):].any()
+
+
+@pytest.mark.parametrize("T", [64, 500])
+def test_least_workspace_is_enough_and_less_is_refused(T):
+    """K slices are as many as the workspace holds; what a call refused for lack of it is refused."""
+    L, R, C = _lib.lib(), 300, 4096
+    s = synth(R, C, 4, 12, seed=T)
+    lin, x = to_device(s), rand_x(T, C, torch.float16, seed=T).cuda()
+    mats = [lin.descriptor(0)]
+    ref = x.double() @ torch.from_numpy(s.decode()).cuda().double().T
+    y = torch.empty(T, R, device="cuda")
+    ws = torch.zeros(L.sq_workspace_bytes(_lib.matrix_array(mats), 1, T, 3), dtype=torch.uint8, device="cuda")
+    # 64 rows: 8 slices of all of them; 500: the decoded matrix, an fp16 copy of x and the sums of the tile GEMM's four parts
+    least = {64: 8 * T * R * 4, 500: R * C * 2 + T * C * 2 + 8 * 4 * 128 * 256 * 4}[T]
+    assert least <= ws.numel()
+    call = lambda n: L.sq_linear_gemm(_lib.matrix_array(mats), 1, x.data_ptr(), _lib.SQ_F16, C, y.data_ptr(), _lib.SQ_F32, R, T, ws.data_ptr(), n, _lib.stream_ptr(x.device))
+    for n in (ws.numel(), least):
+        y.zero_()
+        assert call(n) == 0 and rel_max_err(y.cpu().numpy(), ref.cpu().numpy()) < 1e-5
+    assert call(least - 4096) == _lib.SQ_EWORKSPACE
 
 
 DECODED = [  # rows of the stack's pieces, C, d, bits, G, M, T: column orders, rows of broken lane units, stages past the row's end
