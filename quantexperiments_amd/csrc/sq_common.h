@@ -206,6 +206,11 @@ size_t gemm_workspace_without_mid(const sq_matrix* mats, int n, int T);
 constexpr int GEMM256_PIECES = 8;
 struct Gemm256Scales { const uint16_t* p[GEMM256_PIECES]; int end[GEMM256_PIECES]; int n; };
 int launch_bf16_to_f16(const uint16_t* x, int64_t ldx, int T, int C, uint16_t* out, hipStream_t s);
+// 16-bit tags of width 8 decoded a column of the codebook at a time, results and activations in plane order (sq_planes.hip)
+bool planes_ok(const sq_matrix* mats, int n);
+bool planes_route(const sq_matrix* mats, int n, int T, int x_dtype);      // the tile GEMM's decode goes that way
+size_t planes_bytes(int n);
+int launch_planes(const sq_matrix* mats, int n, uint16_t* out, uint16_t* planes, const void* x, int x_dtype, int64_t ldx, int T, uint16_t* xout, hipStream_t s);
 int launch_dequant_stack(const sq_matrix* mats, int n, void* out, int raw, const uint16_t* x, int64_t ldx, int T, int C, uint16_t* xout, hipStream_t s);
 int launch_gemm_dense(const void* w, int w_dtype, int64_t ldw, int R, int C, const void* x, int x_dtype, int64_t ldx,
                       void* y, int y_dtype, int64_t ldy, int T, hipStream_t s, void* ws = nullptr, size_t ws_bytes = 0);

@@ -101,6 +101,15 @@ static float fused_us(const FusedPlan& p, const sq_matrix* mats, int n, int cus)
     return -4.5f + rounds * (19.6f + mats[0].C * 1e-3f / p.ks * (0.163f * p.tw + 0.809f * p.nw * p.tw + 0.707f * p.nw - 0.217f));
 }
 
+// d = 8: two blocks of tokens in one round of workgroups, where the tile GEMM's decode goes in plane order (sq_planes.hip): there takes less (here and
+// there, us at 450 / 600 / 768 rows: 18944 x 3584 113 / 123 / 128 and 99 / 116 / 117, 15000 x 4992 124 / 145 / 147 and 105 / 126 / 127, 3584 x 18944
+// 141 / 157 / 163 and 122 / 129 / 164, 16000 x 2048 61 / 71 / 73 and 55 / 66 / 66; in two rounds, 37888 x 3584, 205 / 230 / 238 and 206 / 252 / 240).
+static bool tiles_win(const FusedPlan& p, const sq_matrix* mats, int n, int T, int cus) {
+    int64_t w = 0;
+    for (int i = 0; i < n; ++i) w += (mats[i].R + 32 * p.tw - 1) / (32 * p.tw);
+    return p.tbs == 2 && w * p.ks * p.tbs <= cus && planes_route(mats, n, T, SQ_BF16);
+}
+
 static size_t fused_x_bytes(const sq_matrix* mats, const FusedPlan& p) {
     return (size_t)p.tbs * fused_rounds(mats[0]) * fused_round_steps(mats[0]) * FUSED_TN * p.nw * 1024;
 }
@@ -116,7 +125,8 @@ bool fused_route(const sq_matrix* mats, int n, int T) {
         if (m.d == 4 && ((int64_t)m.G << m.bits) * 8 > 128 * 1024) return false;
     }
     const FusedPlan p = fused_plan(mats, n, T, device_cus());
-    if (!p.nw || mats[0].d == 8 || mats[0].C < FUSED_MID_C) return p.nw != 0;
+    if (!p.nw || (mats[0].d == 8 && tiles_win(p, mats, n, T, device_cus()))) return false;
+    if (mats[0].d == 8 || mats[0].C < FUSED_MID_C) return true;
     const float us = mid_us(mats, n, T);
     return us > 80.f || us > 0.85f * fused_us(p, mats, n, device_cus());
 }

@@ -345,6 +345,21 @@ int vector_decoded(const sq_matrix* mats, int n, int B) {
 
 static size_t gemm_workspace_beyond_small(const sq_matrix* mats, int n, int T);
 
+// What decoding in plane order (sq_planes.hip) saves a product in the tile GEMM, in microseconds: 0.24 per million weights, and a launch per
+// piece beyond the first, less a launch that brings the codebooks and the activations into that order, which fp16 activations would otherwise not
+// pay for.  Fitted to 56 products of 3 M to 136 M weights at 1100 and 2048 rows (before / now, us: 2 x 18944 x 3584 at 1024 / 2048 rows 338 / 514 and
+// 301 / 474, 15000 x 4992 at 1100 200 and 183, 3000 + 3000 x 3584 70 and 65; where it is not taken, 3584 x 3584 at 2048 62.2 and 63.3, 3000 x 1024 27 and 32).
+static float planes_gain(const sq_matrix* mats, int n, int T, int x_dtype) {
+    if (n > 1 && !stacked_route(mats, n)) return 0.f;
+    float weights = 0.f;
+    for (int i = 0; i < n; i += GEMM256_PIECES)
+        if (!planes_ok(mats + i, std::min(n - i, GEMM256_PIECES))) return 0.f;
+    for (int i = 0; i < n; ++i) weights += (float)mats[i].R * mats[i].C * 1e-6f;
+    const float x = (float)T * mats[0].C * 1e-6f;
+    return 0.24f * weights + 3.5f * (n - 1) - 5.5f * ((n + GEMM256_PIECES - 1) / GEMM256_PIECES) - (x_dtype == SQ_F16 ? 1.f + 0.35f * x : 0.f);
+}
+bool planes_route(const sq_matrix* mats, int n, int T, int x_dtype) { return big_route(mats, n, T) && planes_gain(mats, n, T, x_dtype) > 0.5f; }
+
 // Beyond the row counts that always take it, the kernel of sq_mid.h is the faster way for small products: where its estimated
 // time is below 50 us (longer ones run at a lower clock) and 85 % of what decode and tile GEMM take, as fitted to 722 of those (8 %).  There and here, us (700 / 1000 / 1600
 // rows): 1024 x 896, 12-bit tags, 19.9 / 19.6 / 20.2 and 8.2 / 8.5 / 11.0, 3584 x 3584 45.0 / 47.7 / 55.2 and 30.9 / 33.9 / 54.3, 18000 x 1024 43 /
@@ -354,6 +369,7 @@ static bool mid_beyond(const sq_matrix* mats, int n, int T) {
     int rows = 0;
     for (int i = 0; i < n; ++i) weights += (float)mats[i].R * mats[i].C * 1e-6f, rows += mats[i].R;
     tiles += 0.85f * gemm256_us(T, rows, mats[0].C, device_cus()) + (mats[0].d == 8 ? 0.77f : 0.51f) * weights;
+    if (mats[0].d == 8) tiles -= 0.6f * std::max(0.f, planes_gain(mats, n, T, SQ_BF16));     // (1500 x 4032 in three pieces: 260 rows 31.3 there, 32.0 decoded, 500 42.0 and 39.9)
     const float us = mid_us(mats, n, T);
     return us < 50.f && us < 0.85f * tiles;
 }
@@ -371,7 +387,8 @@ static size_t gemm_workspace_beyond_small(const sq_matrix* mats, int n, int T) {
     // (covers the other routes too: the size is asked for without knowing x; up to SQ_SMALL_BMAX rows the only one is the
     // decode-time kernel, which the caller adds)
     if (T <= SQ_SMALL_BMAX && decoded_route(mats, n, T)) return decoded_workspace(mats, n, T);
-    const size_t rest = std::max(gemm_workspace_without_mid(mats, n, T), fused_route(mats, n, T) ? fused_workspace(mats, n, T) : (size_t)0);
+    const size_t tiles = gemm_workspace_without_mid(mats, n, T) + (planes_route(mats, n, T, SQ_BF16) ? planes_bytes(std::min(n, GEMM256_PIECES)) : (size_t)0);
+    const size_t rest = std::max(tiles, fused_route(mats, n, T) ? fused_workspace(mats, n, T) : (size_t)0);
     if (takes_mid(mats, n, T)) return std::max(rest, mid_workspace(mats, n, T));
     return decoded_route(mats, n, T) ? std::max(rest, decoded_workspace(mats, n, T)) : rest;
 }
@@ -485,14 +502,22 @@ int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_
         int64_t ldxh = ldx;
         char* wd = (char*)ws;
         // bf16 activations are copied to fp16 once; the copy rides along with the first decode when that takes
-        // the four-chunk kernel (the two overlap in one launch), else it is a launch of its own
-        bool copy_pending = x_dtype == SQ_BF16;
+        // the four-chunk kernel (the two overlap in one launch), else it is a launch of its own.  A decode in plane order
+        // (given the workspace) needs activations of either type in that order.
+        const size_t plane_bytes = planes_route(mats, n, T, x_dtype) ? planes_bytes(std::min(n, GEMM256_PIECES)) : 0;
+        const bool planes = plane_bytes && gemm_workspace_without_mid(mats, n, T) + plane_bytes <= ws_bytes;
+        bool copy_pending = planes || x_dtype == SQ_BF16;
         if (copy_pending) {
             xh = (const uint16_t*)ws;
             ldxh = C;
         }
+        wd += align256((size_t)T * C * 2);
+        uint16_t* plane_tables = (uint16_t*)wd;
+        if (planes) wd += plane_bytes;
         auto decode_stack = [&](const sq_matrix* ms, int k, void* w) -> int {
-            const int rc = launch_dequant_stack(ms, k, w, 1, copy_pending ? (const uint16_t*)x : nullptr, ldx, T, C, (uint16_t*)ws, s);
+            const void* xs = copy_pending ? x : nullptr;
+            const int rc = planes ? launch_planes(ms, k, (uint16_t*)w, plane_tables, xs, x_dtype, ldx, T, (uint16_t*)ws, s)
+                                  : launch_dequant_stack(ms, k, w, 1, (const uint16_t*)xs, ldx, T, C, (uint16_t*)ws, s);
             if (rc == 0) copy_pending = false;
             return rc;
         };
@@ -507,7 +532,6 @@ int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_
             }
             return launch_dequant(m, w, SQ_F16, C, 0, m.R, s, /*raw=*/true);
         };
-        wd += align256((size_t)T * C * 2);
         const int cus0 = device_cus();
         if (stacked_route(mats, n)) {
             for (int i0 = 0; i0 < n; i0 += GEMM256_PIECES) {
