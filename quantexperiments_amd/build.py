@@ -11,7 +11,7 @@ HERE = Path(__file__).resolve().parent
 CSRC = HERE / "csrc"
 LIB = HERE / "libsqhip.so"
 NATIVE = HERE / "_native.so"
-SOURCES = ["sq_api.hip", "sq_dequant.hip", "sq_planes.hip", "sq_small_generic.hip", "sq_gemv.hip", "sq_gemv_b16d8.hip",
+SOURCES = ["sq_api.hip", "sq_dequant.hip", "sq_planes.hip", "sq_plane_product.hip", "sq_small_generic.hip", "sq_gemv.hip", "sq_gemv_b16d8.hip",
            "sq_gemv_b12d4.hip", "sq_gemv_b10d4.hip", "sq_gemv_b8d4.hip", "sq_gemm.hip", "sq_gemm256.hip", "sq_stream.hip", "sq_stream_build.hip", "sq_relabel.hip",
            "sq_q8.hip", "sq_neighbours.hip", "sq_segs.hip", "sq_sieve.hip", "sq_mid.hip", "sq_mid_b16d8.hip", "sq_mid_b12d4.hip", "sq_mid_b10d4.hip", "sq_mid_b8d4.hip",
            "sq_mid_dense.hip", "sq_fused.hip", "sq_fused_b16d8.hip", "sq_fused_b12d4.hip", "sq_fused_b10d4.hip", "sq_fused_b8d4.hip"]

@@ -211,6 +211,11 @@ bool planes_ok(const sq_matrix* mats, int n);
 bool planes_route(const sq_matrix* mats, int n, int T, int x_dtype);      // the tile GEMM's decode goes that way
 size_t planes_bytes(int n);
 int launch_planes(const sq_matrix* mats, int n, uint16_t* out, uint16_t* planes, const void* x, int x_dtype, int64_t ldx, int T, uint16_t* xout, hipStream_t s);
+// 17 to 128 activation rows of 16-bit tags of width 8, a column of the codebook at a time (sq_plane_product.hip): how many of the n pieces, the first
+// one on, it takes in one launch; 0 where the other kernels are the faster way
+int plane_product_group(const sq_matrix* mats, int n, int T);
+size_t plane_product_workspace(const sq_matrix* mats, int n, int T);
+int launch_plane_product(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, hipStream_t s);
 int launch_dequant_stack(const sq_matrix* mats, int n, void* out, int raw, const uint16_t* x, int64_t ldx, int T, int C, uint16_t* xout, hipStream_t s);
 int launch_gemm_dense(const void* w, int w_dtype, int64_t ldw, int R, int C, const void* x, int x_dtype, int64_t ldx,
                       void* y, int y_dtype, int64_t ldy, int T, hipStream_t s, void* ws = nullptr, size_t ws_bytes = 0);

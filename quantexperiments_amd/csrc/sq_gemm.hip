@@ -388,6 +388,7 @@ static size_t gemm_workspace_beyond_small(const sq_matrix* mats, int n, int T) {
     // decode-time kernel, which the caller adds)
     if (T <= SQ_SMALL_BMAX && decoded_route(mats, n, T)) return decoded_workspace(mats, n, T);
     const size_t tiles = gemm_workspace_without_mid(mats, n, T) + (planes_route(mats, n, T, SQ_BF16) ? planes_bytes(std::min(n, GEMM256_PIECES)) : (size_t)0);
+    if (T > SQ_SMALL_BMAX && plane_product_group(mats, n, T) == n) return std::max({tiles, mid_workspace(mats, n, T), plane_product_workspace(mats, n, T)});
     const size_t rest = std::max(tiles, fused_route(mats, n, T) ? fused_workspace(mats, n, T) : (size_t)0);
     if (takes_mid(mats, n, T)) return std::max(rest, mid_workspace(mats, n, T));
     return decoded_route(mats, n, T) ? std::max(rest, decoded_workspace(mats, n, T)) : rest;
@@ -463,6 +464,8 @@ int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_
         return launch_small(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, ws_bytes, sums, s);
     if (x_vec_ok(x, ldx, mats[0].C) && fused_route(mats, n, T) && fused_workspace(mats, n, T) <= ws_bytes)
         return launch_fused(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);
+    if (T > SQ_SMALL_BMAX && x_vec_ok(x, ldx, mats[0].C) && plane_product_group(mats, n, T) == n && plane_product_workspace(mats, n, T) <= ws_bytes)
+        return launch_plane_product(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);
     if (x_vec_ok(x, ldx, mats[0].C) && mid_x_ok(ldx, T) && takes_mid(mats, n, T) && (mid_ok(mats, n, T) || gemm_workspace_without_mid(mats, n, T) <= ws_bytes))
         return launch_mid(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, ws_bytes, s);
     if (T > SQ_SMALL_BMAX && T <= small_pass_limit(mats, n) && x_vec_ok(x, ldx, mats[0].C)) {

@@ -235,6 +235,13 @@ static int sieve_len(const sq_matrix* mats, int n, int B) {
     return sieve_group(mats, k, B);
 }
 
+// The same for the kernel of sq_plane_product.hip
+static int plane_product_len(const sq_matrix* mats, int n, int B) {
+    int k = 0;
+    while (k < n && mma_rows(mats[k]) && !stream_rows(mats[k], B)) ++k;
+    return plane_product_group(mats, k, B);
+}
+
 // What the pieces' kernels keep side by side; not what a launch has from the workspace's first byte on for itself (small_workspace).
 // tight: the pieces that can run without partial sums do
 static size_t small_need(const sq_matrix* mats, int n, int B, bool tight) {
@@ -253,6 +260,9 @@ size_t small_workspace(const sq_matrix* mats, int n, int B) {
     for (int i = 0; i < n; ++i) {
         if (const int k = orders ? 0 : vector_decoded(mats + i, n - i, B); k > 0) {
             need = std::max(need, decoded_workspace(mats + i, k, B));
+            i += k - 1;
+        } else if (const int k = plane_product_len(mats + i, n - i, B); k > 0) {
+            need = std::max(need, plane_product_workspace(mats + i, k, B));
             i += k - 1;
         } else if (const int k = sieve_len(mats + i, n - i, B); k > 0) {
             need = std::max(need, sieve_workspace(mats + i, k, B));
@@ -435,6 +445,12 @@ int launch_small(const sq_matrix* mats, int n, const void* x, int x_dtype, int64
         }
         if (const int k = orders || !x_ok ? 0 : vector_decoded(mats + i, n - i, B); k > 0 && decoded_workspace(mats + i, k, B) <= ws_bytes) {
             if (const int rc = launch_decoded(mats + i, k, x, x_dtype, ldx, y, y_dtype, ldy, B, ws, s, /*wide=*/true)) return rc;
+            i += k;
+            continue;
+        }
+        if (const int k = !x_ok ? 0 : plane_product_len(mats + i, n - i, B); k > 0 && plane_product_workspace(mats + i, k, B) <= ws_bytes) {
+            if (const int rc = launch_plane_product(mats + i, k, x, x_dtype, ldx, y, y_dtype, ldy, B, ws, s)) return rc;
+            ws_off += small_need(mats + i, k, B, tight);
             i += k;
             continue;
         }

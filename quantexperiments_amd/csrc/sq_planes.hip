@@ -7,11 +7,10 @@
 // so whole lines leave.  The activations are copied into the same order of columns and the product does not notice: its sum over
 // columns is the same sum in another order.
 #include <algorithm>
-#include "sq_common.h"
+#include "sq_planes.h"
 
 namespace sq {
 
-constexpr int PLANE = 65536;                 // codewords, and elements of a plane
 constexpr int NT = 512, U = 8;               // planes_kernel's threads, and units of a thread in flight
 
 // Rows of n chunks of 8 elements into plane order, 8 chunks (128 bytes in, a 16-byte piece of each plane out) per thread: the codebooks of
@@ -58,15 +57,7 @@ __global__ __launch_bounds__(256) void plane_order_kernel(PlaneOrderArgs a) {
         for (int i = 0; i < 8; ++i) { v[i].x = bf2h_x2(v[i].x); v[i].y = bf2h_x2(v[i].y); v[i].z = bf2h_x2(v[i].z); v[i].w = bf2h_x2(v[i].w); }
     }
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        u32x4 o;
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const uint32_t lo = v[2 * w][e / 2], hi = v[2 * w + 1][e / 2];
-            o[w] = e & 1 ? (lo >> 16) | (hi & 0xFFFF0000u) : (lo & 0xFFFFu) | (hi << 16);
-        }
-        *reinterpret_cast<u32x4*>(dst + (int64_t)e * n) = o;
-    }
+    for (int e = 0; e < 8; ++e) *reinterpret_cast<u32x4*>(dst + (int64_t)e * n) = plane_of(v, e);
 }
 
 struct PlanesArgs {

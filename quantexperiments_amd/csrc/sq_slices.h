@@ -6,9 +6,9 @@
 namespace sq {
 
 struct SlicePiece {
-    const float* part;           // fp32 [ks, T, R]
+    const float* part;           // fp32 [ks, T, ld]
     const uint16_t* row_scale;
-    int R, y_off;
+    int R, ld, y_off;
     uint32_t end;                // quads of this piece and those before it
 };
 struct SliceArgs {
@@ -31,13 +31,13 @@ static __global__ __launch_bounds__(64) void slice_sum_kernel(SliceArgs a) {
     i -= before;
     const uint32_t q = (uint32_t)(m.R + 3) / 4, t = i / q;
     const int r = (int)(i - t * q) * 4;
-    const float* p = m.part + (int64_t)t * m.R + r;
-    const int64_t step = (int64_t)a.T * m.R, o = (int64_t)t * a.ldy + m.y_off + r;
+    const float* p = m.part + (int64_t)t * m.ld + r;
+    const int64_t step = (int64_t)a.T * m.ld, o = (int64_t)t * a.ldy + m.y_off + r;
     float sc[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) sc[e] = h2f(m.row_scale[min(r + e, m.R - 1)]);
     float4v v = {0.f, 0.f, 0.f, 0.f};
-    if (m.R % 4 == 0 && ((uintptr_t)m.part & 15) == 0) {
+    if (m.ld % 4 == 0 && ((uintptr_t)m.part & 15) == 0) {
         for (int k0 = 0; k0 < a.ks; k0 += 8) {
             float4v s[8];
 #pragma unroll
@@ -45,7 +45,7 @@ static __global__ __launch_bounds__(64) void slice_sum_kernel(SliceArgs a) {
 #pragma unroll
             for (int k = 0; k < 8; ++k) if (k0 + k < a.ks) v += s[k];
         }
-        if (a.y_dtype != SQ_F32 && ((o | (int64_t)((uintptr_t)a.y >> 1)) & 3) == 0) {
+        if (a.y_dtype != SQ_F32 && r + 4 <= m.R && ((o | (int64_t)((uintptr_t)a.y >> 1)) & 3) == 0) {
             *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(a.y) + o) =
                 a.y_dtype == SQ_BF16 ? u32x2{f2bf_x2(v[0] * sc[0], v[1] * sc[1]), f2bf_x2(v[2] * sc[2], v[3] * sc[3])}
                                      : u32x2{f2h_x2(v[0] * sc[0], v[1] * sc[1]), f2h_x2(v[2] * sc[2], v[3] * sc[3])};
@@ -61,16 +61,16 @@ static __global__ __launch_bounds__(64) void slice_sum_kernel(SliceArgs a) {
         if (r + e < m.R) store_y(a.y, a.y_dtype, o + e, v[e] * sc[e]);
 }
 
-// Pieces: {.m, .part}, n of them
+// Pieces: {.m, .part}, n of them; whole_quads: rows of sums are whole quads of them, whatever R is
 template <class Piece>
-int launch_slice_sum(const Piece* pieces, int n, int ks, int T, void* y, int y_dtype, int64_t ldy, hipStream_t s) {
+int launch_slice_sum(const Piece* pieces, int n, int ks, int T, void* y, int y_dtype, int64_t ldy, hipStream_t s, bool whole_quads = false) {
     SliceArgs a{};
     a.y = y; a.ldy = ldy; a.n = n; a.T = T; a.ks = ks; a.y_dtype = y_dtype;
     uint32_t quads = 0;
     for (int i = 0; i < n; ++i) {
         const sq_matrix& m = pieces[i].m;
         quads += (uint32_t)T * (uint32_t)((m.R + 3) / 4);
-        a.p[i] = {pieces[i].part, m.row_scale, m.R, m.y_off, quads};
+        a.p[i] = {pieces[i].part, m.row_scale, m.R, whole_quads ? (m.R + 3) / 4 * 4 : m.R, m.y_off, quads};
     }
     hipLaunchKernelGGL(slice_sum_kernel, dim3((quads + 63) / 64), dim3(64), 0, s, a);
     return check_launch("sum of K slices");
