@@ -17,7 +17,7 @@
  *     w[r, perms[row_mask[r]][c]] = u[r, c]
  * and the layer computes Y[t, y_off + r] = sum_c X[t, c] * w[r, c] with fp32 accumulation.  A row that names a codeword which is not
  * finite has results that are not finite; an infinity may come out as NaN (idle lanes of the decode-time kernels, and of the d = 4
- * kernel that gathers codewords for 33 and more rows, multiply codewords of the row with zeros).  Other rows are not touched.
+ * kernel that gathers codewords for 17 and more rows, multiply codewords of the row with zeros).  Other rows are not touched.
  */
 #ifndef SQHIP_H
 #define SQHIP_H

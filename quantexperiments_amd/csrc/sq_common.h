@@ -181,8 +181,9 @@ int launch_decoded(const sq_matrix* mats, int n, const void* x, int x_dtype, int
 // products in one pass over the tags (sq_mid.h): whether it is the way of these pieces in any case, its estimated time, and its call
 bool mma_shape(const sq_matrix& m);
 bool mid_ok(const sq_matrix* mats, int n, int T);
+inline bool mid_x_ok(int64_t ldx, int T) { return (int64_t)T * ldx * 2 < (int64_t)1 << 32; }     // 32-bit offsets
 size_t mid_workspace(const sq_matrix* mats, int n, int T);
-float mid_us(const sq_matrix* mats, int n, int T);
+float mid_us(const sq_matrix* mats, int n, int T, size_t room = SIZE_MAX);
 int launch_mid(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws,
                size_t ws_bytes, hipStream_t s);
 // the same for weights already decoded to fp16, w[i] = [R, C] of piece i without row scales (1 .. 256 activation rows)

@@ -154,7 +154,6 @@ int launch_gemm256(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ld
 int launch_dequant_with_cvt(const sq_matrix& m, void* out, int64_t ld_out, const uint16_t* x, int64_t ldx, int T, int C,
                             uint16_t* xout, hipStream_t s);
 
-static bool mid_x_ok(int64_t ldx, int T) { return (int64_t)T * ldx * 2 < (int64_t)1 << 32; }     // 32-bit offsets
 static bool x_vec_ok(const void* x, int64_t ldx, int C) { return C % 8 == 0 && ldx % 8 == 0 && ((uintptr_t)x & 15) == 0; }
 // Activation rows from which the large-tile route (decode each piece once into the workspace as raw fp16
 // codewords, then the 256 x 256 tile GEMM with the row scale in its epilogue) replaces the fused 128 x 128

@@ -242,6 +242,58 @@ static int plane_product_len(const sq_matrix* mats, int n, int B) {
     return plane_product_group(mats, k, B);
 }
 
+// SiLU(gate) * up written by the matrix-core kernel: the two pieces' codebooks (one format, one shape) fit LDS side by side next to the
+// accumulators of a group of tiles, the rows are not split over workgroups (same plan, so the same sums, as without), and the product
+// by itself would run on this kernel: two activation rows or more.  us, the two launches / this one, 8 rows: 2 x 18944 x 3584 with 12-bit tags
+// 20.4 / 17.6, 8-bit 18.7 / 15.2; 17408 x 5120, 12-bit 28.7 / 25.0, 10-bit in 4 books 26.3 / 24.0; 8960 x 1536, 12-bit 11.8 / 10.1;
+// 1024 x 512, 8-bit 7.6 / 6.6.  But 4864 x 896 (two waves a workgroup) with 64 KB of codebooks 11.7 / 12.0, with 128 KB 13.7 / 17.5: a
+// workgroup's waves fetch the codebooks, at most 24 KB each here.
+static bool mma_silu_shape(const sq_matrix* mats, int n, int B) {
+    if (n != 2 || B < 2 || B > SQ_SMALL_BMAX) return false;
+    const sq_matrix &g = mats[0], &u = mats[1];
+    if (g.d != 4 || !mma_shape(g) || !mma_shape(u) || g.R <= 0 || g.R != u.R || g.bits != u.bits || g.d != u.d || g.W != u.W || g.G != u.G) return false;
+    if (tiled_piece(g) == nullptr != (tiled_piece(u) == nullptr)) return false;
+    const size_t tab = mma_table_bytes(g);
+    if (tab == 0 || tab > 64 * 1024) return false;               // (beyond 64 KB two rows take the row-segment kernel)
+    const MmaPlan pl = mma_plan(g, B);
+    const int tpu = unit_dwords(g.bits) * 32 / g.bits;
+    return pl.ks == 1 && 2 * tab <= (size_t)pl.KW * 24 * 1024 && 2 * tab + 16 + std::max((size_t)pl.KW * mma_x_stage_bytes(tpu * g.d, mma_x_tokens_min(pl.NT)), (size_t)mma_group(pl.RW, pl.NT, true) * pl.KW * 64 * pl.NT * 16) <= 160 * 1024;
+}
+static bool mma_fuses_silu(const sq_matrix* mats, int n, int B, const void* x, int64_t ldx) {
+    return mma_silu_shape(mats, n, B) && ldx % 8 == 0 && ((uintptr_t)x & 15) == 0 && !small_takes_gemm_route(mats, n, B, x, ldx);
+}
+
+// Estimated microseconds of that kernel for d = 4 pieces that share a launch at 17 to 32 rows, fitted to 400 products (9 %): weights (and more of them
+// where codebooks leave a CU few waves), column slices and their sums, waves and rounds of a wave, results.
+static float mma_us(const sq_matrix* mats, int n, int B) {
+    const MmaPlan pl = mma_plan(mats[0], B);
+    float rows = 0.f;
+    for (int i = 0; i < n; ++i) rows += (float)mats[i].R * 1e-6f;
+    return 4.86f + 0.106f * rows * mats[0].C * (mma_table_bytes(mats[0]) > 64 * 1024 ? 1.43f : 1.f) + (pl.ks > 1 ? 2.8f + 1.58f * pl.ks * B * rows : 0.f) +
+           0.29f * pl.KW + 0.69f * pl.RW + 2.9f * B * rows;
+}
+
+// How many d = 4 pieces, the first one on, take the kernel of sq_mid.h at 17 to SQ_SMALL_BMAX rows; room: bytes for its sums.  With two tiles of activation rows
+// the decode-time kernel's waves are few and add long sums (most where codebooks of 128 KB leave it five, which splits rows); there every wave has its own rows.
+// Taken where it is estimated 8 % faster, as both estimates err by that much: of 400 products of 256 to 19000 rows and 512 to 10000 columns a third, at 0.86 of the
+// time in the mean.  us, decode-time kernel / that one, at 17 / 32 rows: 2 x 18944 x 3584 with four books of 12-bit tags 39.9 / 42.0 and 29.9 / 27.9, 24074 x 1152 so
+// 12.4 / 12.4 and 10.8 / 10.7; 4864 x 896, 8-bit, 7.9 / 8.0 and 5.6 / 5.5; 16546 x 832, 10-bit, 10.1 / 10.4 and 8.1 / 8.3; not 2570 x 2304, 12-bit in two books,
+// 8.9 / 9.1 and 11.3 / 10.5.  At 16 rows it is the slower one for most (18944 x 3584 in four books twice, at 12: 21.5, 32.6).  A gate|up pair that
+// mma_silu_shape takes stays, so that with and without SiLU it has the same sums.
+// (Products below 2 M weights are a launch's length either way, and stay: 464 x 512, 12-bit, 6.4 and 7.4.  Rows below 512 columns were not measured.)
+constexpr int MID_SMALL_T = 17, MID_SMALL_C = 512, MID_SMALL_WEIGHTS = 2 << 20;
+static int mid_len(const sq_matrix* mats, int n, int B, size_t room) {
+    const sq_matrix& m0 = mats[0];
+    if (B < MID_SMALL_T || B > SQ_SMALL_BMAX || m0.d != 4 || m0.C < MID_SMALL_C || mma_silu_shape(mats, n, B)) return 0;
+    int k = 0;
+    int64_t weights = 0;
+    while (k < n && k < MID_PIECES && mma_shape(mats[k]) && mats[k].R > 0 && !stream_rows(mats[k], B) && mats[k].d == 4 && mats[k].bits == m0.bits &&
+           mats[k].W == m0.W && mats[k].G == m0.G) weights += (int64_t)mats[k++].R * m0.C;
+    return weights >= MID_SMALL_WEIGHTS && mma_table_bytes(m0) && mid_us(mats, k, B, room) < 0.92f * mma_us(mats, k, B) ? k : 0;
+}
+// For tests: that number where the workspace holds whatever sums there are.
+extern "C" __attribute__((visibility("default"))) int32_t sq_mid_pieces_for_tests(const sq_matrix* mats, int32_t n, int32_t B) { return mid_len(mats, n, B, SIZE_MAX); }
+
 // What the pieces' kernels keep side by side; not what a launch has from the workspace's first byte on for itself (small_workspace).
 // tight: the pieces that can run without partial sums do
 static size_t small_need(const sq_matrix* mats, int n, int B, bool tight) {
@@ -267,6 +319,9 @@ size_t small_workspace(const sq_matrix* mats, int n, int B) {
         } else if (const int k = sieve_len(mats + i, n - i, B); k > 0) {
             need = std::max(need, sieve_workspace(mats + i, k, B));
             i += k - 1;
+        } else if (const int k = mid_len(mats + i, n - i, B, SIZE_MAX); k > 0) {
+            need = std::max(need, mid_workspace(mats + i, k, B));
+            i += k - 1;
         }
     }
     return need;
@@ -277,24 +332,6 @@ bool small_uses_sums(const sq_matrix* mats, int n) {
     for (int i = 0; i < n; ++i)
         if (mats[i].R > 0 && stream_shape(mats[i])) return true;
     return false;
-}
-
-// SiLU(gate) * up written by the matrix-core kernel: the two pieces' codebooks (one format, one shape) fit LDS side by side next to the
-// accumulators of a group of tiles, the rows are not split over workgroups (same plan, so the same sums, as without), and the product
-// by itself would run on this kernel: two activation rows or more.  us, the two launches / this one, 8 rows: 2 x 18944 x 3584 with 12-bit tags
-// 20.4 / 17.6, 8-bit 18.7 / 15.2; 17408 x 5120, 12-bit 28.7 / 25.0, 10-bit in 4 books 26.3 / 24.0; 8960 x 1536, 12-bit 11.8 / 10.1;
-// 1024 x 512, 8-bit 7.6 / 6.6.  But 4864 x 896 (two waves a workgroup) with 64 KB of codebooks 11.7 / 12.0, with 128 KB 13.7 / 17.5: a
-// workgroup's waves fetch the codebooks, at most 24 KB each here.
-static bool mma_fuses_silu(const sq_matrix* mats, int n, int B, const void* x, int64_t ldx) {
-    if (n != 2 || B < 2 || B > SQ_SMALL_BMAX || ldx % 8 || ((uintptr_t)x & 15)) return false;
-    const sq_matrix &g = mats[0], &u = mats[1];
-    if (g.d != 4 || !mma_shape(g) || !mma_shape(u) || g.R <= 0 || g.R != u.R || g.bits != u.bits || g.d != u.d || g.W != u.W || g.G != u.G) return false;
-    if (small_takes_gemm_route(mats, n, B, x, ldx) || tiled_piece(g) == nullptr != (tiled_piece(u) == nullptr)) return false;
-    const size_t tab = mma_table_bytes(g);
-    if (tab == 0 || tab > 64 * 1024) return false;               // (beyond 64 KB two rows take the row-segment kernel)
-    const MmaPlan pl = mma_plan(g, B);
-    const int tpu = unit_dwords(g.bits) * 32 / g.bits;
-    return pl.ks == 1 && 2 * tab <= (size_t)pl.KW * 24 * 1024 && 2 * tab + 16 + std::max((size_t)pl.KW * mma_x_stage_bytes(tpu * g.d, mma_x_tokens_min(pl.NT)), (size_t)mma_group(pl.RW, pl.NT, true) * pl.KW * 64 * pl.NT * 16) <= 160 * 1024;
 }
 
 // Pieces [0, cnt) share format and row length: one persistent launch (+ one reduction per piece if ks > 1).  act: mma_fuses_silu
@@ -457,6 +494,12 @@ int launch_small(const sq_matrix* mats, int n, const void* x, int x_dtype, int64
         if (const int k = !x_ok ? 0 : sieve_len(mats + i, n - i, B); k > 0 && sieve_workspace_least(mats + i, k, B) <= ws_bytes) {
             if (const int rc = launch_sieve(mats + i, k, x, x_dtype, ldx, y, y_dtype, ldy, B, ws, ws_bytes, s)) return rc;
             ws_off += small_need(mats + i, k, B, tight);         // (what was counted for them)
+            i += k;
+            continue;
+        }
+        if (const int k = !x_ok || !mid_x_ok(ldx, B) ? 0 : mid_len(mats + i, n - i, B, ws_bytes); k > 0) {
+            if (const int rc = launch_mid(mats + i, k, x, x_dtype, ldx, y, y_dtype, ldy, B, ws, ws_bytes, s)) return rc;
+            ws_off += small_need(mats + i, k, B, tight);
             i += k;
             continue;
         }

@@ -1,4 +1,4 @@
-// Host side of the product for 33 and more activation rows (kernel: sq_mid.h): which stacks it takes, and how the work
+// Host side of the product for 33 and more activation rows, and d = 4 from 17 on (kernel: sq_mid.h): which stacks it takes, and how the work
 // is cut.
 #include <algorithm>
 #include "sq_mid.h"
@@ -73,7 +73,7 @@ static MidPlan mid_plan(const sq_matrix* mats, int n, int T, int cus, size_t roo
         const MidVariant& v = vs[k];
         const int lds = mid_lds(v, table);
         if (lds > 160 * 1024 || (v.st == 2 && v.nt <= 8 && mid_lds({v.nt, v.tw, v.nw, 4}, table) <= 160 * 1024)) continue;
-        if (v.nt > 1 && v.nt * 16 >= 2 * T) continue;                     // (more than half of it past the last row)
+        if (v.nt > 3 && v.nt * 16 >= 2 * T) continue;                     // (more than half of it past the last row)
         // workgroups that a CU runs side by side, by its LDS and registers
         const int beside = std::max(1, std::min({160 * 1024 / lds, 4 * (512 / (40 + 6 * v.nt + 4 * v.nt * v.tw)) / v.nw, 32 / v.nw}));
         const int64_t whole = mid_blocks(mats, n, 16 * v.nw * v.tw) * ((T + 16 * v.nt - 1) / (16 * v.nt));
@@ -96,7 +96,7 @@ static MidPlan mid_plan(const sq_matrix* mats, int n, int T, int cus, size_t roo
 
 // the pieces share format, row length and codebook size, and the kernel takes them
 static bool mid_shape(const sq_matrix* mats, int n, int T) {
-    if (n < 1 || n > MID_PIECES || T <= SQ_SMALL_BMAX) return false;
+    if (n < 1 || n > MID_PIECES || T < 1) return false;
     for (int i = 0; i < n; ++i) {
         const sq_matrix &m = mats[i], &m0 = mats[0];
         if (!mma_shape(m) || m.R <= 0 || m.d != m0.d || m.bits != m0.bits || m.W != m0.W || m.G != m0.G) return false;
@@ -114,7 +114,7 @@ static int mid_limit(const sq_matrix* mats, int n) {
     return mats[0].d == 4 && weights >= (int64_t)1 << 26 ? 384 : 256;
 }
 
-bool mid_ok(const sq_matrix* mats, int n, int T) { return mid_shape(mats, n, T) && T <= mid_limit(mats, n); }
+bool mid_ok(const sq_matrix* mats, int n, int T) { return T > SQ_SMALL_BMAX && mid_shape(mats, n, T) && T <= mid_limit(mats, n); }
 
 // What a workspace has to hold up to there: the sums of as many slices as the kernel took when a launch had one block of all activation
 // rows (or half of them).  Cuts that need more than there is are passed over.
@@ -142,11 +142,11 @@ static size_t mid_least(const sq_matrix* mats, int n, int T) {
 size_t mid_workspace(const sq_matrix* mats, int n, int T) {
     const MidPlan p = mid_plan(mats, n, T, device_cus(), SIZE_MAX);
     const size_t need = mid_sums_bytes(mats, n, T, p.ks);
-    return T <= mid_limit(mats, n) ? std::max(need, mid_least(mats, n, T)) : need;
+    return T > SQ_SMALL_BMAX && T <= mid_limit(mats, n) ? std::max(need, mid_least(mats, n, T)) : need;
 }
 
-// Estimated time at T rows; a very long one where the kernel does not take the pieces
-float mid_us(const sq_matrix* mats, int n, int T) { return mid_shape(mats, n, T) ? mid_plan(mats, n, T, device_cus(), SIZE_MAX).us : 1e30f; }
+// Estimated time at T rows with `room` bytes for sums; a very long one where the kernel does not take the pieces
+float mid_us(const sq_matrix* mats, int n, int T, size_t room) { return mid_shape(mats, n, T) ? mid_plan(mats, n, T, device_cus(), room).us : 1e30f; }
 
 // For tests: the cut that a stack takes at T rows, as token tiles | weight tiles << 8 | waves << 16 | K slices << 24; 0: the kernel does not take it.
 extern "C" __attribute__((visibility("default"))) int32_t sq_mid_variant_for_tests(const sq_matrix* mats, int32_t n, int32_t T) {
@@ -216,7 +216,7 @@ int launch_mid_decoded(const sq_matrix* mats, int n, const void* const* w, const
 
 int launch_mid(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws,
                size_t ws_bytes, hipStream_t s) {
-    if (T <= mid_limit(mats, n) && mid_least(mats, n, T) > ws_bytes) return fail(SQ_EWORKSPACE, "sq_linear_gemm: workspace %zu < %zu", ws_bytes, mid_workspace(mats, n, T));
+    if (T > SQ_SMALL_BMAX && T <= mid_limit(mats, n) && mid_least(mats, n, T) > ws_bytes) return fail(SQ_EWORKSPACE, "sq_linear_gemm: workspace %zu < %zu", ws_bytes, mid_workspace(mats, n, T));
     return launch_mid_rows(mats, n, mid_plan(mats, n, T, device_cus(), ws_bytes), nullptr, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);
 }
 

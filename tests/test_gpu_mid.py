@@ -1,13 +1,13 @@
 """Products of 33 to 2048 activation rows whose codewords are gathered once per block of them: edges of the tiles of rows and activation rows, a last round
 with missing units, odd numbers of rounds, K slices, stacks, several codebooks, two tiles of rows per wave, two parts of rows; and
-of 3 to 256 rows with weights decoded first."""
+of 3 to 256 rows with weights decoded first; and decode batches of 17 to 32."""
 
 import numpy as np
 import pytest
 import torch
 
 from quantexperiments_amd import _lib
-from quantexperiments_amd.kernels import linear_gemm
+from quantexperiments_amd.kernels import linear_gemm, linear_small
 from tests.helpers import rand_x, rel_max_err, synth, to_device, with_infinity
 
 pytestmark = pytest.mark.gpu
@@ -83,6 +83,36 @@ def test_cuts_match_oracle(case, dtype, stream):
     assert rel_max_err(y.cpu().numpy(), ref.cpu().numpy()) < 1e-5
     lowp = torch.zeros(T, sum(rows) + 8, dtype=dtype, device="cuda")
     linear_gemm(lins, xd, lowp[:, :sum(rows)])
+    assert torch.equal(lowp[:, :sum(rows)], y.to(dtype)) and not lowp[:, sum(rows):].any()
+
+
+# rows of the stack's pieces, C, bits, G, T, and how many of the pieces (d = 4, up to 32 activation rows) go that way: one and two tiles of activation
+# rows, the last one broken, K slices, several codebooks, more pieces than a launch takes; a pair that SiLU could be fused behind, 16 rows
+DECODE_BATCHES = [
+    ((4863,), 896, 8, 1, 17, 1), ((4864,), 896, 8, 1, 32, 1), ((4864,), 896, 8, 1, 16, 0), ((16546,), 832, 10, 1, 31, 1), ((15002, 9), 512, 10, 4, 24, 2),
+    ((2501,), 9408, 12, 1, 17, 1), ((17000, 17001), 1600, 12, 4, 32, 2), ((9000, 9001), 2080, 12, 4, 17, 0), ((540,) * 9, 512, 8, 4, 20, 8), ((4864, 4864), 1024, 8, 1, 20, 0), ((20000,), 640, 12, 1, 18, 1),
+    ((14570, 3642, 3641), 1088, 12, 1, 32, 3),
+]
+
+
+@pytest.mark.parametrize("case", DECODE_BATCHES, ids=lambda c: "x".join(map(str, c)))
+@pytest.mark.parametrize("dtype,stream", [(torch.bfloat16, True), (torch.float16, False)], ids=["bf16-tiled", "f16-rows"])
+def test_decode_batches_match_oracle(case, dtype, stream):
+    rows, C, bits, G, T, pieces = case
+    ss = [synth(R, C, 4, bits, G, 1, seed=R + T + i) for i, R in enumerate(rows)]
+    lins = [to_device(s, stream=stream) for s in ss]
+    taken = _lib.lib().sq_mid_pieces_for_tests(_lib.matrix_array([m.descriptor() for m in lins]), len(lins), T)
+    assert torch.cuda.get_device_properties(0).multi_processor_count != 256 or taken == pieces
+    x = torch.zeros(T, C + 8, dtype=dtype)
+    x[:, :C] = rand_x(T, C, dtype, seed=T)
+    xd = x.cuda()[:, :C]
+    ref = torch.cat([xd.double() @ torch.from_numpy(s.decode()).cuda().double().T for s in ss], dim=1)
+    y = torch.empty(T, sum(rows), dtype=torch.float32, device="cuda")
+    linear_small(lins, xd, y)
+    # products of fp16 values are exact in fp32, whose sums of C terms round at 2^-24 of a partial sum
+    assert rel_max_err(y.cpu().numpy(), ref.cpu().numpy()) < 1e-5
+    lowp = torch.zeros(T, sum(rows) + 8, dtype=dtype, device="cuda")
+    linear_small(lins, xd, lowp[:, :sum(rows)])
     assert torch.equal(lowp[:, :sum(rows)], y.to(dtype)) and not lowp[:, sum(rows):].any()
 
 
