@@ -360,17 +360,19 @@ static float planes_gain(const sq_matrix* mats, int n, int T, int x_dtype) {
 bool planes_route(const sq_matrix* mats, int n, int T, int x_dtype) { return big_route(mats, n, T) && planes_gain(mats, n, T, x_dtype) > 0.5f; }
 
 // Beyond the row counts that always take it, the kernel of sq_mid.h is the faster way for small products: where its estimated
-// time is below 50 us (longer ones run at a lower clock) and 85 % of what decode and tile GEMM take, as fitted to 722 of those (8 %).  There and here, us (700 / 1000 / 1600
+// time is below 50 us (longer ones run at a lower clock) and 90 % of what decode and tile GEMM take, as fitted to 722 of those (8 %).  There and here, us (700 / 1000 / 1600
 // rows): 1024 x 896, 12-bit tags, 19.9 / 19.6 / 20.2 and 8.2 / 8.5 / 11.0, 3584 x 3584 45.0 / 47.7 / 55.2 and 30.9 / 33.9 / 54.3, 18000 x 1024 43 /
 // 58 / 76 and 45 / 57 / 87; 16-bit, 1024 x 896, 19.2 / 19.1 / 19.8 and 12.5 / 14.9 / 17.9, 3584 x 3584 47 / 51 / 58 and 69 / 80 / 116.
+// With the tile GEMM's estimate as it is now (and 90 % for the 85 that went with the one before) 44 products on whose way the two disagree take 0.94 of the time in the mean,
+// none of them longer (1078 + 1078 x 1408, 16-bit, at 610 rows 37.5 and 24.8, 8310 x 960, 8-bit, at 616 31.6 and 23.4).
 static bool mid_beyond(const sq_matrix* mats, int n, int T) {
-    float tiles = 11.5f, weights = 0.f;
+    float tiles = 3.2f, weights = 0.f;
     int rows = 0;
     for (int i = 0; i < n; ++i) weights += (float)mats[i].R * mats[i].C * 1e-6f, rows += mats[i].R;
-    tiles += 0.85f * gemm256_us(T, rows, mats[0].C, device_cus()) + (mats[0].d == 8 ? 0.77f : 0.51f) * weights;
+    tiles += 1.13f * gemm256_us(T, rows, mats[0].C, device_cus()) + (mats[0].d == 8 ? 0.77f : 0.51f) * weights;
     if (mats[0].d == 8) tiles -= 0.6f * std::max(0.f, planes_gain(mats, n, T, SQ_BF16));     // (1500 x 4032 in three pieces: 260 rows 31.3 there, 32.0 decoded, 500 42.0 and 39.9)
     const float us = mid_us(mats, n, T);
-    return us < 50.f && us < 0.85f * tiles;
+    return us < 50.f && us < 0.9f * tiles;
 }
 static bool takes_mid(const sq_matrix* mats, int n, int T) { return mid_ok(mats, n, T) || (T > SQ_SMALL_BMAX && mid_beyond(mats, n, T)); }
 

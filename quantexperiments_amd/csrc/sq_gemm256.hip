@@ -717,18 +717,14 @@ struct Gemm256Plan { int mt, main_tiles, tail_tiles, kt; float us; };
 
 // Tiles of 256 rows read least per product and are the ones for products of many rounds (8192^3: 880 us, 963 with 192 rows,
 // 1019 with 128); where few tiles leave CUs idle, or most of a tile's rows are past the end, smaller ones win.  The plan with the
-// least estimated time is taken.  A slab takes G_SLAB + G_SLAB_BUSY * (share of the CUs at work) microseconds (the chip's power
-// and its L2 set the pace when it is full; fitted to 32 .. 512 tiles of each height at 3584 columns, where one round took 42 ..
-// 63 / 55 .. 81 / 70 .. 104 us), a round 5 us at its ends, and a split adds the reduction's launch and the partial tiles written
-// and read back.  All of these times are of a kernel of 32x32x16 instructions with a workgroup per tile.  Today's take less than is estimated,
-// and not by one factor (2048 x 37888 x 3584 481 estimated, 403 - 424 measured; 2048 x 3584 x 18944 258 and 237; 2048 x 4608 x 3584 70 and 66;
-// 2048 x 3584 x 3584 58 and 51; 1024 x 7168 x 5120 81 and 67): what is near another plan in the estimate may not be the best one.
-// Estimated best and measured then, tiles of 256 rows unsplit before it (us): 333 x 37888 x 3584 161, with the plan 119;
-// 1024 x 7168 x 5120 95 (in two 85), now 72; 2048 x 3584 x 3584 66, now 52; 2048 x 4608 x 3584 70, now 64; 512 x 3584 x 18944
-// 104 in four, now 88; 2048 x 3584 x 18944 stays with 256 rows in two, 245 (128 rows: 270).
+// least estimated time is taken.  A slab takes G_SLAB + G_SLAB_BUSY * (share of the CUs at work, squared) microseconds (the chip's power
+// and its L2 set the pace when it is full), a round G_ENDS at its ends, and a split adds the partial tiles written and read back.  Fitted to every height in up
+// to eight parts for 153 products of 260 to 2048 x 1500 to 38000 x 512 to 18944 (6 %), and then for the choice: what is taken is 0.4 % slower than the best of them in the
+// mean.  With the times of an earlier kernel it was 1.0 %, up to 23: 902 x 1780 x 4416 36.7 us, now 29.8; 334 x 10325 x 4608 53.3 and 46.2; 372 x 5262 x 5248 39.3, 34.3;
+// 1070 x 7033 x 15488 227, 201; 1382 x 3722 x 4480 60.2, 55.7; none of them slower.
 // Up to eight parts, for few tiles of long rows (with up to four, now): 333 x 3584 x 18944 83, 71.  Parts of 8 slabs would gain 2
 // us on short rows (520 x 1024 x 2048 22.5, 20.6) for twice the workspace.
-constexpr double G_SLAB[5] = {0, 0, 0.58, 0.73, 0.98}, G_SLAB_BUSY[5] = {0, 0, 0.42, 0.56, 0.70};
+constexpr double G_SLAB[5] = {0, 0, 0.449, 0.723, 0.979}, G_SLAB_BUSY[5] = {0, 0, 0.375, 0.404, 0.503}, G_ENDS = 9.8;
 
 static Gemm256Plan gemm256_plan(int T, int R, int C, int cus, bool split) {
     const int slabs = (C + G_BK - 1) / G_BK;
@@ -743,9 +739,10 @@ static Gemm256Plan gemm256_plan(int T, int R, int C, int cus, bool split) {
         for (int kt = 1; kt <= (split && rounds && tail ? 8 : 1); ++kt) {
             if (kt > 1 && slabs / kt < 16) break;
             const int wgs = tail * kt, of = (slabs + kt - 1) / kt;
-            double t = (double)(main / n) * (slabs * slab + 5.0) + (wgs / n) * (of * slab + 5.0);
-            if (wgs % n) t += of * (G_SLAB[mt] + G_SLAB_BUSY[mt] * (wgs % n) / n) + 5.0;
-            if (kt > 1) t += 4.0 + wgs * mt * 0.015;
+            const double share = (double)(wgs % n) / n;
+            double t = 2.5 + (double)(main / n) * (slabs * slab + G_ENDS) + (wgs / n) * (of * slab + G_ENDS);
+            if (wgs % n) t += of * (G_SLAB[mt] + G_SLAB_BUSY[mt] * share * share) + G_ENDS;
+            if (kt > 1) t += 0.1 + wgs * mt * 0.0124;
             if (t < best_t - 1e-9) {
                 best_t = t;
                 best = kt > 1 ? Gemm256Plan{mt, main, tail, kt, (float)t} : Gemm256Plan{mt, (int)tiles, 0, 1, (float)t};
