@@ -36,8 +36,6 @@ __global__ __launch_bounds__(256) void fused_x_kernel(const uint16_t* __restrict
     }
 }
 
-struct FusedPlan { int nw, tw, ks, tbs; };
-
 static int fused_unit_dwords(int bits) { return bits == 12 ? 3 : bits == 10 ? 5 : 4; }
 static int fused_round_steps(const sq_matrix& m) { return fused_unit_dwords(m.bits) * 32 / m.bits / (8 / m.d); }
 static int fused_rounds(const sq_matrix& m) { return (m.W / fused_unit_dwords(m.bits) + 3) / 4; }
@@ -57,7 +55,7 @@ static int fused_rounds(const sq_matrix& m) { return (m.W / fused_unit_dwords(m.
 // is longer than two of them (d = 8 from 193 tokens, d = 4 from 257); and rows of 8192 columns and more are cut into K slices of
 // 2048 at least where there are too few tiles (in shorter rows the slices' sums cost what they gain: 4608 x 3584 at 333 tokens 51 us
 // in three, 53 there).  At 1000 tokens 191 / 225 for 18944 rows, 371 / 353 for 37888.
-static FusedPlan fused_plan(const sq_matrix* mats, int n, int T, int cus) {
+static FusedPlan fused_cut(const sq_matrix* mats, int n, int T, int cus) {
     const FusedPlan none{0, 0, 1, 1};
     if (T < 129 || T > 768) return none;
     const int tbs = T <= 384 ? 1 : 2, per = (T + tbs - 1) / tbs, nw = per <= 192 ? 3 : per <= 256 ? 4 : 6;
@@ -87,27 +85,14 @@ static FusedPlan fused_plan(const sq_matrix* mats, int n, int T, int cus) {
     return none;
 }
 
-// d = 4 products of the cuts above, in microseconds: a launch of the activations and one of the product, 20 between rounds of workgroups, fitted to
-// 76 of 1700 to 54000 rows at 130 to 768 tokens (9 %).  The kernel of sq_mid.h, in blocks of activation rows, is the faster one for most of
-// them now: 11600 x 3800, 10-bit tags, at 259 rows 68 us here, 42 there; 8300 x 2944 and two of 2093 at 268 62 / 39; 18900 x 1900, 8-bit, at
-// 201 42 / 29; not for 29600 x 2300, 10-bit, at 370 72 / 90, or 15500 x 1200 at 470 37 / 38.  Rows below 512 columns, a launch's length either
-// way, were not measured and stay; a long product runs at a lower clock than both
-// estimates know, hence 85 % and 80 us (26000 x 5600, 10-bit, at 237 rows 95 here, 104 there).
-constexpr int FUSED_MID_C = 512;
-static float fused_us(const FusedPlan& p, const sq_matrix* mats, int n, int cus) {
+// What a d = 4 product takes in such a cut, in microseconds: a launch of the activations and one of the product, 20 between rounds of workgroups; fitted to
+// 76 of 1700 to 54000 rows at 130 to 768 tokens (9 %)
+float fused_us(const FusedPlan& p, const sq_matrix* mats, int n) {
     int64_t w = 0;
     for (int i = 0; i < n; ++i) w += (mats[i].R + 32 * p.tw - 1) / (32 * p.tw);
+    const int cus = device_cus();
     const int64_t rounds = (w * p.ks * p.tbs + cus - 1) / cus;
     return -4.5f + rounds * (19.6f + mats[0].C * 1e-3f / p.ks * (0.163f * p.tw + 0.809f * p.nw * p.tw + 0.707f * p.nw - 0.217f));
-}
-
-// d = 8: two blocks of tokens in one round of workgroups, where the tile GEMM's decode goes in plane order (sq_planes.hip): there takes less (here and
-// there, us at 450 / 600 / 768 rows: 18944 x 3584 113 / 123 / 128 and 99 / 116 / 117, 15000 x 4992 124 / 145 / 147 and 105 / 126 / 127, 3584 x 18944
-// 141 / 157 / 163 and 122 / 129 / 164, 16000 x 2048 61 / 71 / 73 and 55 / 66 / 66; in two rounds, 37888 x 3584, 205 / 230 / 238 and 206 / 252 / 240).
-static bool tiles_win(const FusedPlan& p, const sq_matrix* mats, int n, int T, int cus) {
-    int64_t w = 0;
-    for (int i = 0; i < n; ++i) w += (mats[i].R + 32 * p.tw - 1) / (32 * p.tw);
-    return p.tbs == 2 && w * p.ks * p.tbs <= cus && planes_route(mats, n, T, SQ_BF16);
 }
 
 static size_t fused_x_bytes(const sq_matrix* mats, const FusedPlan& p) {
@@ -115,38 +100,35 @@ static size_t fused_x_bytes(const sq_matrix* mats, const FusedPlan& p) {
 }
 static size_t fused_part_bytes(const sq_matrix& m, int T, int ks) { return ks > 1 ? (((size_t)ks * T * m.R * 4) + 255) & ~(size_t)255 : 0; }
 
-bool fused_route(const sq_matrix* mats, int n, int T) {
-    if (n < 1 || n > MID_PIECES) return false;
+FusedPlan fused_plan(const sq_matrix* mats, int n, int T) {
+    const FusedPlan none{0, 0, 1, 1};
+    if (n < 1 || n > MID_PIECES) return none;
     for (int i = 0; i < n; ++i) {
         const sq_matrix &m = mats[i], &m0 = mats[0];
-        if (!mma_shape(m) || m.R <= 0 || m.d != m0.d || m.bits != m0.bits || m.W != m0.W || m.G != m0.G) return false;
-        if (((int64_t)m.R + 16) * m.W * 4 >= ((int64_t)1 << 32)) return false;                 // 32-bit offsets
-        if (m.d == 8 && ((int64_t)m.G << m.bits) * 16 > ((int64_t)1 << 31)) return false;
-        if (m.d == 4 && ((int64_t)m.G << m.bits) * 8 > 128 * 1024) return false;
+        if (!mma_shape(m) || m.R <= 0 || m.d != m0.d || m.bits != m0.bits || m.W != m0.W || m.G != m0.G) return none;
+        if (((int64_t)m.R + 16) * m.W * 4 >= ((int64_t)1 << 32)) return none;                  // 32-bit offsets
+        if (m.d == 8 && ((int64_t)m.G << m.bits) * 16 > ((int64_t)1 << 31)) return none;
+        if (m.d == 4 && ((int64_t)m.G << m.bits) * 8 > 128 * 1024) return none;
     }
-    const FusedPlan p = fused_plan(mats, n, T, device_cus());
-    if (!p.nw || (mats[0].d == 8 && tiles_win(p, mats, n, T, device_cus()))) return false;
-    if (mats[0].d == 8 || mats[0].C < FUSED_MID_C) return true;
-    const float us = mid_us(mats, n, T);
-    return us > 80.f || us > 0.85f * fused_us(p, mats, n, device_cus());
+    return fused_cut(mats, n, T, device_cus());
 }
 
 // For tests: the variant that a stack takes at T rows, as token tiles | weight tiles << 8 | K slices << 16 | token blocks << 24; 0: another kernel.
 extern "C" __attribute__((visibility("default"))) int32_t sq_fused_variant_for_tests(const sq_matrix* mats, int32_t n, int32_t T) {
-    if (!fused_route(mats, n, T)) return 0;
-    const FusedPlan p = fused_plan(mats, n, T, device_cus());
+    if (gemm_kernel(mats, n, T) != GEMM_FUSED) return 0;
+    const FusedPlan p = fused_plan(mats, n, T);
     return p.nw | p.tw << 8 | p.ks << 16 | p.tbs << 24;
 }
 
 size_t fused_workspace(const sq_matrix* mats, int n, int T) {
-    const FusedPlan p = fused_plan(mats, n, T, device_cus());
+    const FusedPlan p = fused_plan(mats, n, T);
     size_t need = fused_x_bytes(mats, p);
     for (int i = 0; i < n; ++i) need += fused_part_bytes(mats[i], T, p.ks);
     return need;
 }
 
 int launch_fused(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, hipStream_t s) {
-    const FusedPlan p = fused_plan(mats, n, T, device_cus());
+    const FusedPlan p = fused_plan(mats, n, T);
     const sq_matrix& m0 = mats[0];
     FusedArgs a{};
     a.n = n; a.y = y; a.ldy = ldy; a.T = T; a.y_dtype = y_dtype; a.ks = p.ks;

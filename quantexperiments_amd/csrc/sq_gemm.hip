@@ -359,22 +359,72 @@ static float planes_gain(const sq_matrix* mats, int n, int T, int x_dtype) {
 }
 bool planes_route(const sq_matrix* mats, int n, int T, int x_dtype) { return big_route(mats, n, T) && planes_gain(mats, n, T, x_dtype) > 0.5f; }
 
-// Beyond the row counts that always take it, the kernel of sq_mid.h is the faster way for small products: where its estimated
-// time is below 50 us (longer ones run at a lower clock) and 90 % of what decode and tile GEMM take, as fitted to 722 of those (8 %).  There and here, us (700 / 1000 / 1600
-// rows): 1024 x 896, 12-bit tags, 19.9 / 19.6 / 20.2 and 8.2 / 8.5 / 11.0, 3584 x 3584 45.0 / 47.7 / 55.2 and 30.9 / 33.9 / 54.3, 18000 x 1024 43 /
-// 58 / 76 and 45 / 57 / 87; 16-bit, 1024 x 896, 19.2 / 19.1 / 19.8 and 12.5 / 14.9 / 17.9, 3584 x 3584 47 / 51 / 58 and 69 / 80 / 116.
-// With the tile GEMM's estimate as it is now (and 90 % for the 85 that went with the one before) 44 products on whose way the two disagree take 0.94 of the time in the mean,
-// none of them longer (1078 + 1078 x 1408, 16-bit, at 610 rows 37.5 and 24.8, 8310 x 960, 8-bit, at 616 31.6 and 23.4).
-static bool mid_beyond(const sq_matrix* mats, int n, int T) {
-    float tiles = 3.2f, weights = 0.f;
+// What decode and tile GEMM take, in microseconds, fitted to 722 products (8 %)
+static float tiles_us(const sq_matrix* mats, int n, int T) {
+    float us = 3.2f, weights = 0.f;
     int rows = 0;
     for (int i = 0; i < n; ++i) weights += (float)mats[i].R * mats[i].C * 1e-6f, rows += mats[i].R;
-    tiles += 1.13f * gemm256_us(T, rows, mats[0].C, device_cus()) + (mats[0].d == 8 ? 0.77f : 0.51f) * weights;
-    if (mats[0].d == 8) tiles -= 0.6f * std::max(0.f, planes_gain(mats, n, T, SQ_BF16));     // (1500 x 4032 in three pieces: 260 rows 31.3 there, 32.0 decoded, 500 42.0 and 39.9)
-    const float us = mid_us(mats, n, T);
-    return us < 50.f && us < 0.9f * tiles;
+    us += 1.13f * gemm256_us(T, rows, mats[0].C, device_cus()) + (mats[0].d == 8 ? 0.77f : 0.51f) * weights;
+    if (mats[0].d == 8) us -= 0.6f * std::max(0.f, planes_gain(mats, n, T, SQ_BF16));     // (1500 x 4032 in three pieces: 260 rows 31.3 there, 32.0 decoded, 500 42.0 and 39.9)
+    return us;
 }
-static bool takes_mid(const sq_matrix* mats, int n, int T) { return mid_ok(mats, n, T) || (T > SQ_SMALL_BMAX && mid_beyond(mats, n, T)); }
+
+// Which kernel takes a product, in one place: what one of them gives up is taken by the one that it was compared with.
+//
+// Products that the fused kernel has a cut for (129 to 768 rows) run there, unless
+//   d = 4   the kernel of sq_mid.h, in blocks of activation rows, is estimated to take at most 85 % of the time and 80 us (a long product runs at a lower clock than both
+//           estimates know: 26000 x 5600, 10-bit tags, at 237 rows 95 us there, 104 here).  It does for most of them: 11600 x 3800, 10-bit, at 259 rows 68 us there, 42
+//           here; 18900 x 1900, 8-bit, at 201 42 / 29; 7704 x 8192 in four books of 10-bit tags at 262 75 / 59, 12257 x 6592, 10-bit, at 391 101 / 78; not for 29600 x
+//           2300, 10-bit, at 370 72 / 90, or 15500 x 1200 at 470 37 / 38.  Rows below 512 columns, a launch's length either way, were not measured and stay.  From 50 us on that
+//           kernel also has to be estimated at 73 % of the tiles, which gain most where the rows are just beyond two of theirs: of 47 products of 50 to 80 us
+//           at 260 to 738 rows those below 73 % took 0.58 to 0.98 of the tiles' time (0.55 to 0.94 of this kernel's), those above 0.88 to 1.12, the
+//           tiles 0.73 to 0.88 of this kernel's (18549 x 1920, 10-bit, at 541 rows 81 here, 69 there, 62 in tiles).
+//   d = 8   they are two blocks of tokens in one round of workgroups and the tile GEMM's decode goes in plane order (sq_planes.hip): the tiles take less (us at 450 / 600 / 768
+//           rows: 18944 x 3584 113 / 123 / 128 and 99 / 116 / 117, 15000 x 4992 124 / 145 / 147 and 105 / 126 / 127, 3584 x 18944 141 / 157 / 163 and 122 / 129 /
+//           164, 16000 x 2048 61 / 71 / 73 and 55 / 66 / 66; in two rounds, 37888 x 3584, 205 / 230 / 238 and 206 / 252 / 240).
+//
+// Without such a cut, beyond the row counts that always take it, the kernel of sq_mid.h is the faster way for small products: where its estimated
+// time is below 50 us (longer ones run at a lower clock) and 90 % of what decode and tile GEMM take.  There and here, us (700 / 1000 / 1600
+// rows): 1024 x 896, 12-bit tags, 19.9 / 19.6 / 20.2 and 8.2 / 8.5 / 11.0, 3584 x 3584 45.0 / 47.7 / 55.2 and 30.9 / 33.9 / 54.3, 18000 x 1024 43 /
+// 58 / 76 and 45 / 57 / 87; 16-bit, 1024 x 896, 19.2 / 19.1 / 19.8 and 12.5 / 14.9 / 17.9, 3584 x 3584 47 / 51 / 58 and 69 / 80 / 116.
+// (44 products on whose way this and an older estimate of the tile GEMM disagree take 0.94 of the time in the mean,
+// none of them longer: 1078 + 1078 x 1408, 16-bit, at 610 rows 37.5 and 24.8, 8310 x 960, 8-bit, at 616 31.6 and 23.4.)
+constexpr int FUSED_MID_C = 512;
+GemmKernel gemm_kernel(const sq_matrix* mats, int n, int T) {
+    const FusedPlan fused = fused_plan(mats, n, T);
+    const bool d8 = mats[0].d == 8;
+    float most = 50.f;                                           // us that the kernel of sq_mid.h may take beyond mid_ok
+    if (fused.nw) {
+        if (d8) {
+            int64_t w = 0;
+            for (int i = 0; i < n; ++i) w += (mats[i].R + 32 * fused.tw - 1) / (32 * fused.tw);
+            if (!(fused.tbs == 2 && w * fused.ks * 2 <= device_cus() && planes_route(mats, n, T, SQ_BF16))) return GEMM_FUSED;
+        } else {
+            most = 80.f;
+            const float us = mats[0].C < FUSED_MID_C ? 1e30f : mid_us(mats, n, T);
+            if (us > most || us > 0.85f * fused_us(fused, mats, n)) return GEMM_FUSED;
+        }
+    }
+    if (T > SQ_SMALL_BMAX) {
+        if (plane_product_group(mats, n, T) == n) return GEMM_COLUMNS;
+        if (mid_ok(mats, n, T)) return GEMM_MID;
+        const float us = mid_us(mats, n, T);
+        if (us < most && us < (us < 50.f ? 0.9f : 0.73f) * tiles_us(mats, n, T)) return GEMM_MID;
+        if (T <= small_pass_limit(mats, n)) return GEMM_PASSES;
+    }
+    return decoded_route(mats, n, T) ? GEMM_DECODED : GEMM_TILES;
+}
+
+// For tests: that kernel (7: the tile GEMM behind a decode in plane order), and what the first one, the kernel of sq_mid.h and the tiles are estimated to take, in
+// microseconds (1e30: not for these pieces).
+extern "C" __attribute__((visibility("default"))) int32_t sq_gemm_kernel_for_tests(const sq_matrix* mats, int32_t n, int32_t T, int32_t x_dtype, float* us) {
+    const FusedPlan fused = fused_plan(mats, n, T);
+    us[0] = fused.nw ? fused_us(fused, mats, n) : 1e30f;
+    us[1] = mid_us(mats, n, T);
+    us[2] = tiles_us(mats, n, T);
+    const GemmKernel k = gemm_kernel(mats, n, T);
+    return k == GEMM_TILES && planes_route(mats, n, T, x_dtype) ? 7 : k;
+}
 
 size_t gemm_workspace(const sq_matrix* mats, int n, int T) {
     // up to SQ_SMALL_BMAX rows sq_linear_gemm is sq_linear_small, unless the stack goes the other way (see above);
@@ -389,10 +439,13 @@ static size_t gemm_workspace_beyond_small(const sq_matrix* mats, int n, int T) {
     // decode-time kernel, which the caller adds)
     if (T <= SQ_SMALL_BMAX && decoded_route(mats, n, T)) return decoded_workspace(mats, n, T);
     const size_t tiles = gemm_workspace_without_mid(mats, n, T) + (planes_route(mats, n, T, SQ_BF16) ? planes_bytes(std::min(n, GEMM256_PIECES)) : (size_t)0);
-    if (T > SQ_SMALL_BMAX && plane_product_group(mats, n, T) == n) return std::max({tiles, mid_workspace(mats, n, T), plane_product_workspace(mats, n, T)});
-    const size_t rest = std::max(tiles, fused_route(mats, n, T) ? fused_workspace(mats, n, T) : (size_t)0);
-    if (takes_mid(mats, n, T)) return std::max(rest, mid_workspace(mats, n, T));
-    return decoded_route(mats, n, T) ? std::max(rest, decoded_workspace(mats, n, T)) : rest;
+    switch (gemm_kernel(mats, n, T)) {
+    case GEMM_FUSED: return std::max({tiles, fused_workspace(mats, n, T), mid_ok(mats, n, T) ? mid_workspace(mats, n, T) : (size_t)0});
+    case GEMM_COLUMNS: return std::max({tiles, mid_workspace(mats, n, T), plane_product_workspace(mats, n, T)});
+    case GEMM_MID: return std::max(tiles, mid_workspace(mats, n, T));
+    case GEMM_DECODED: return std::max(tiles, decoded_workspace(mats, n, T));
+    default: return tiles;
+    }
 }
 
 size_t gemm_workspace_without_mid(const sq_matrix* mats, int n, int T) {
@@ -463,12 +516,17 @@ int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_
                 int64_t ldy, int T, void* ws, size_t ws_bytes, void* sums, hipStream_t s) {
     if (T <= SQ_SMALL_BMAX && !small_takes_gemm_route(mats, n, T, x, ldx))
         return launch_small(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, ws_bytes, sums, s);
-    if (x_vec_ok(x, ldx, mats[0].C) && fused_route(mats, n, T) && fused_workspace(mats, n, T) <= ws_bytes)
-        return launch_fused(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);
-    if (T > SQ_SMALL_BMAX && x_vec_ok(x, ldx, mats[0].C) && plane_product_group(mats, n, T) == n && plane_product_workspace(mats, n, T) <= ws_bytes)
-        return launch_plane_product(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);
-    if (x_vec_ok(x, ldx, mats[0].C) && mid_x_ok(ldx, T) && takes_mid(mats, n, T) && (mid_ok(mats, n, T) || gemm_workspace_without_mid(mats, n, T) <= ws_bytes))
-        return launch_mid(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, ws_bytes, s);
+    if (T > SQ_SMALL_BMAX && x_vec_ok(x, ldx, mats[0].C)) {
+        const GemmKernel k = gemm_kernel(mats, n, T);
+        if (k == GEMM_COLUMNS && plane_product_workspace(mats, n, T) <= ws_bytes) return launch_plane_product(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);
+        // (the fused kernel's cuts also serve where a workspace or the span of x does not let the others in)
+        const bool mid = mid_x_ok(ldx, T) && (mid_ok(mats, n, T) ? mid_least(mats, n, T) <= ws_bytes : k == GEMM_MID && gemm_workspace_without_mid(mats, n, T) <= ws_bytes);
+        if (k == GEMM_FUSED || !mid)
+            if (fused_plan(mats, n, T).nw && fused_workspace(mats, n, T) <= ws_bytes && (k != GEMM_TILES || gemm_workspace_without_mid(mats, n, T) > ws_bytes))
+                return launch_fused(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);
+        if (mid) return launch_mid(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, ws_bytes, s);
+        if (mid_x_ok(ldx, T) && mid_ok(mats, n, T)) return fail(SQ_EWORKSPACE, "sq_linear_gemm: workspace %zu < %zu", ws_bytes, gemm_workspace(mats, n, T));
+    }
     if (T > SQ_SMALL_BMAX && T <= small_pass_limit(mats, n) && x_vec_ok(x, ldx, mats[0].C)) {
         // stacks that cannot go in one pass (pieces of different formats): a few passes of the decode-time kernel read the packed
         // tags a few times; decoding to fp16 first (below) writes and reads 8 to 16 times as many bytes once

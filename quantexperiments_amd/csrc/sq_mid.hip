@@ -118,7 +118,7 @@ bool mid_ok(const sq_matrix* mats, int n, int T) { return T > SQ_SMALL_BMAX && m
 
 // What a workspace has to hold up to there: the sums of as many slices as the kernel took when a launch had one block of all activation
 // rows (or half of them).  Cuts that need more than there is are passed over.
-static size_t mid_least(const sq_matrix* mats, int n, int T) {
+size_t mid_least(const sq_matrix* mats, int n, int T) {
     const int cus = device_cus(), table = mats[0].d == 4 ? (mats[0].G << mats[0].bits) * 8 : 0;
     int64_t rows = 0;
     for (int i = 0; i < n; ++i) rows += mats[i].R;
