@@ -193,9 +193,10 @@ size_t mid_dense_workspace(const sq_matrix* mats, int n, int T);
 int launch_mid_decoded(const sq_matrix* mats, int n, const void* const* w, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T,
                        void* ws, hipStream_t s, bool wide);
 // more rows in tiles whose weights are gathered on their way into LDS (sq_fused.h)
-struct FusedPlan { int nw, tw, ks, tbs; };
+struct FusedPlan { int nw, tw, ks, tbs, t; };      // (t: activation rows)
 FusedPlan fused_plan(const sq_matrix* mats, int n, int T);               // nw = 0: not for these
-float fused_us(const FusedPlan& p, const sq_matrix* mats, int n);
+bool fused_two_blocks(const FusedPlan& p, const sq_matrix* mats, int n);      // of tokens, in one round of workgroups
+float fused_us(const FusedPlan& p, const sq_matrix* mats, int n);        // (d = 8: of those)
 size_t fused_workspace(const sq_matrix* mats, int n, int T);
 int launch_fused(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, hipStream_t s);
 // most activation rows for which passes of SQ_SMALL_BMAX rows through the decode-time kernel beat decode + GEMM
@@ -205,7 +206,7 @@ size_t gemm_workspace(const sq_matrix* mats, int n, int T);
 // The kernel that sq_linear_gemm runs n pieces on at more than SQ_SMALL_BMAX rows of aligned activations, given the workspace: sq_fused.h,
 // sq_plane_product.hip, sq_mid.h, passes of the decode-time kernel, decoded rows on sq_mid.h, the tile GEMM behind a decode (in 128 x 128 tiles: none)
 enum GemmKernel { GEMM_FUSED = 1, GEMM_COLUMNS, GEMM_MID, GEMM_PASSES, GEMM_DECODED, GEMM_TILES };
-GemmKernel gemm_kernel(const sq_matrix* mats, int n, int T);
+GemmKernel gemm_route(const sq_matrix* mats, int n, int T, int x_dtype);
 // what launch_gemm can do with less: the same product without the kernel of sq_mid.h
 size_t gemm_workspace_without_mid(const sq_matrix* mats, int n, int T);
 // Row scales of a product whose R rows are n stacked pieces: rows end[i - 1] .. end[i] - 1 are scaled by p[i]; n = 0: no scales.

@@ -56,7 +56,7 @@ static int fused_rounds(const sq_matrix& m) { return (m.W / fused_unit_dwords(m.
 // 2048 at least where there are too few tiles (in shorter rows the slices' sums cost what they gain: 4608 x 3584 at 333 tokens 51 us
 // in three, 53 there).  At 1000 tokens 191 / 225 for 18944 rows, 371 / 353 for 37888.
 static FusedPlan fused_cut(const sq_matrix* mats, int n, int T, int cus) {
-    const FusedPlan none{0, 0, 1, 1};
+    const FusedPlan none{0, 0, 1, 1, 0};
     if (T < 129 || T > 768) return none;
     const int tbs = T <= 384 ? 1 : 2, per = (T + tbs - 1) / tbs, nw = per <= 192 ? 3 : per <= 256 ? 4 : 6;
     const int table = mats[0].d == 4 ? (mats[0].G << mats[0].bits) * 8 : 0, weight[6] = {0, 0, 17, 21, 27, 32};
@@ -77,22 +77,33 @@ static FusedPlan fused_cut(const sq_matrix* mats, int n, int T, int cus) {
     if (!tw) return none;
     const int64_t used = rows * tbs * 100, room = rounds * cus * 32 * tw;     // percent of the weight rows that the rounds have room for
     const bool whole = tbs == 1 ? used >= 66 * room : used >= 85 * room && tw >= 3;
-    if (whole && (rounds == 1 || (tw == 5 && (tbs == 2 || nw == 6 || (nw == 4 && mats[0].d == 8))))) return {nw, tw, 1, tbs};
-    if (mats[0].d == 8 && nw == 4 && tbs == 1 && tiles(1) <= cus && used >= 70 * cus * 32) return {nw, 1, 1, tbs};   // (6000 x 3584 at 200 tokens: 43 us, 49 there)
+    if (whole && (rounds == 1 || (tw == 5 && (tbs == 2 || nw == 6 || (nw == 4 && mats[0].d == 8))))) return {nw, tw, 1, tbs, T};
+    if (mats[0].d == 8 && nw == 4 && tbs == 1 && tiles(1) <= cus && used >= 70 * cus * 32) return {nw, 1, 1, tbs, T};   // (6000 x 3584 at 200 tokens: 43 us, 49 there)
     const int64_t t3 = tiles(3);
     const int ks = (int)std::min<int64_t>({8, cus / t3, mats[0].C / 2048});
-    if (fits(3) && mats[0].C >= 8192 && ks > 1 && t3 * ks * 4 >= cus * 3) return {nw, 3, ks, tbs};
+    if (fits(3) && mats[0].C >= 8192 && ks > 1 && t3 * ks * 4 >= cus * 3) return {nw, 3, ks, tbs, T};
     return none;
 }
 
-// What a d = 4 product takes in such a cut, in microseconds: a launch of the activations and one of the product, 20 between rounds of workgroups; fitted to
-// 76 of 1700 to 54000 rows at 130 to 768 tokens (9 %)
-float fused_us(const FusedPlan& p, const sq_matrix* mats, int n) {
+static int64_t fused_workgroups(const FusedPlan& p, const sq_matrix* mats, int n) {
     int64_t w = 0;
     for (int i = 0; i < n; ++i) w += (mats[i].R + 32 * p.tw - 1) / (32 * p.tw);
+    return w * p.ks * p.tbs;
+}
+
+bool fused_two_blocks(const FusedPlan& p, const sq_matrix* mats, int n) { return p.tbs == 2 && fused_workgroups(p, mats, n) <= device_cus(); }
+
+// What a product takes in such a cut, in microseconds.  d = 4: a launch of the activations and one of the product, 20 between rounds of workgroups; fitted to
+// 76 of 1700 to 54000 rows at 130 to 768 tokens (9 %).  d = 8, two blocks of tokens in one round (fused_two_blocks): fitted to 226 of 1500 to 23000 rows of 192 to 14000
+// columns (7 %; the more workgroups, the longer L2 takes for each one's codewords), with the sums of K slices per million.
+float fused_us(const FusedPlan& p, const sq_matrix* mats, int n) {
     const int cus = device_cus();
-    const int64_t rounds = (w * p.ks * p.tbs + cus - 1) / cus;
-    return -4.5f + rounds * (19.6f + mats[0].C * 1e-3f / p.ks * (0.163f * p.tw + 0.809f * p.nw * p.tw + 0.707f * p.nw - 0.217f));
+    const int64_t w = fused_workgroups(p, mats, n), rounds = (w + cus - 1) / cus;
+    const float columns = mats[0].C * 1e-3f / p.ks;
+    if (mats[0].d == 4) return -4.5f + rounds * (19.6f + columns * (0.163f * p.tw + 0.809f * p.nw * p.tw + 0.707f * p.nw - 0.217f));
+    float sums = 0.f;
+    for (int i = 0; i < n && p.ks > 1; ++i) sums += (float)mats[i].R * p.t * p.ks * 1e-6f;
+    return 19.7f + columns * (5.89f * p.tw + 2.22f * p.nw + 6.63f * w / cus - 16.1f) + 4.19f * sums;
 }
 
 static size_t fused_x_bytes(const sq_matrix* mats, const FusedPlan& p) {
@@ -101,7 +112,7 @@ static size_t fused_x_bytes(const sq_matrix* mats, const FusedPlan& p) {
 static size_t fused_part_bytes(const sq_matrix& m, int T, int ks) { return ks > 1 ? (((size_t)ks * T * m.R * 4) + 255) & ~(size_t)255 : 0; }
 
 FusedPlan fused_plan(const sq_matrix* mats, int n, int T) {
-    const FusedPlan none{0, 0, 1, 1};
+    const FusedPlan none{0, 0, 1, 1, 0};
     if (n < 1 || n > MID_PIECES) return none;
     for (int i = 0; i < n; ++i) {
         const sq_matrix &m = mats[i], &m0 = mats[0];
@@ -115,7 +126,7 @@ FusedPlan fused_plan(const sq_matrix* mats, int n, int T) {
 
 // For tests: the variant that a stack takes at T rows, as token tiles | weight tiles << 8 | K slices << 16 | token blocks << 24; 0: another kernel.
 extern "C" __attribute__((visibility("default"))) int32_t sq_fused_variant_for_tests(const sq_matrix* mats, int32_t n, int32_t T) {
-    if (gemm_kernel(mats, n, T) != GEMM_FUSED) return 0;
+    if (gemm_route(mats, n, T, SQ_BF16) != GEMM_FUSED) return 0;
     const FusedPlan p = fused_plan(mats, n, T);
     return p.nw | p.tw << 8 | p.ks << 16 | p.tbs << 24;
 }

@@ -360,13 +360,23 @@ static float planes_gain(const sq_matrix* mats, int n, int T, int x_dtype) {
 bool planes_route(const sq_matrix* mats, int n, int T, int x_dtype) { return big_route(mats, n, T) && planes_gain(mats, n, T, x_dtype) > 0.5f; }
 
 // What decode and tile GEMM take, in microseconds, fitted to 722 products (8 %)
-static float tiles_us(const sq_matrix* mats, int n, int T) {
+static float tiles_us(const sq_matrix* mats, int n, int T, int x_dtype) {
     float us = 3.2f, weights = 0.f;
     int rows = 0;
     for (int i = 0; i < n; ++i) weights += (float)mats[i].R * mats[i].C * 1e-6f, rows += mats[i].R;
     us += 1.13f * gemm256_us(T, rows, mats[0].C, device_cus()) + (mats[0].d == 8 ? 0.77f : 0.51f) * weights;
-    if (mats[0].d == 8) us -= 0.6f * std::max(0.f, planes_gain(mats, n, T, SQ_BF16));     // (1500 x 4032 in three pieces: 260 rows 31.3 there, 32.0 decoded, 500 42.0 and 39.9)
+    if (mats[0].d == 8) us -= 0.6f * std::max(0.f, planes_gain(mats, n, T, x_dtype));     // (1500 x 4032 in three pieces: 260 rows 31.3 there, 32.0 decoded, 500 42.0 and 39.9)
     return us;
+}
+
+// The same for the d = 8 products of two blocks of tokens that fused_us knows, fitted to 226 of them with activations of either type (7 %): a million weights costs
+// seven times as much from about where the 256 MB last-level cache no longer holds their fp16 copy beside what the product reads and writes.  (Whether the
+// codebooks go in columns makes no difference beyond that error.)
+static float tiles_us_two_blocks(const sq_matrix* mats, int n, int T) {
+    float weights = 0.f;
+    int rows = 0;
+    for (int i = 0; i < n; ++i) weights += (float)mats[i].R * mats[i].C * 1e-6f, rows += mats[i].R;
+    return 9.4f + 1.225f * gemm256_us(T, rows, mats[0].C, device_cus()) + 0.0765f * weights + 0.51f * std::max(0.f, weights - 90.f);
 }
 
 // Which kernel takes a product, in one place: what one of them gives up is taken by the one that it was compared with.
@@ -379,9 +389,12 @@ static float tiles_us(const sq_matrix* mats, int n, int T) {
 //           kernel also has to be estimated at 73 % of the tiles, which gain most where the rows are just beyond two of theirs: of 47 products of 50 to 80 us
 //           at 260 to 738 rows those below 73 % took 0.58 to 0.98 of the tiles' time (0.55 to 0.94 of this kernel's), those above 0.88 to 1.12, the
 //           tiles 0.73 to 0.88 of this kernel's (18549 x 1920, 10-bit, at 541 rows 81 here, 69 there, 62 in tiles).
-//   d = 8   they are two blocks of tokens in one round of workgroups and the tile GEMM's decode goes in plane order (sq_planes.hip): the tiles take less (us at 450 / 600 / 768
-//           rows: 18944 x 3584 113 / 123 / 128 and 99 / 116 / 117, 15000 x 4992 124 / 145 / 147 and 105 / 126 / 127, 3584 x 18944 141 / 157 / 163 and 122 / 129 /
-//           164, 16000 x 2048 61 / 71 / 73 and 55 / 66 / 66; in two rounds, 37888 x 3584, 205 / 230 / 238 and 206 / 252 / 240).
+//   d = 8   they are two blocks of tokens in one round of workgroups and decode and tiles are estimated to take less.  They do for most of 226 such products
+//           of 192 to 14000 columns, us here and there: 18944 x 3584 at 450 / 700 rows 118 / 135 and 97 / 117, 2 x 9313 x 2048 at 533 90 / 67, 3977 x 8896
+//           at 712 117 / 88; not for short rows (7749 + 2 x 1937 x 448 at 483 25 / 32, 2 x 9394 x 576 at 498 39 / 44) and some long ones whose copy
+//           the last-level cache does not hold (10009 x 13568 twice at 490 382 / 394).  What is taken is 0.6 % slower than the faster one in the mean, by more than 5 % for eight of them
+//           (2 x 6081 x 12992 at 510, in tiles, 244 / 297; 12436 + 2 x 3109 x 576 at 700, here, 49 / 43).  In two rounds, 37888 x 3584 at 450 / 600 / 768, 205 / 230 / 238 here and 206 /
+//           252 / 240.
 //
 // Without such a cut, beyond the row counts that always take it, the kernel of sq_mid.h is the faster way for small products: where its estimated
 // time is below 50 us (longer ones run at a lower clock) and 90 % of what decode and tile GEMM take.  There and here, us (700 / 1000 / 1600
@@ -390,15 +403,13 @@ static float tiles_us(const sq_matrix* mats, int n, int T) {
 // (44 products on whose way this and an older estimate of the tile GEMM disagree take 0.94 of the time in the mean,
 // none of them longer: 1078 + 1078 x 1408, 16-bit, at 610 rows 37.5 and 24.8, 8310 x 960, 8-bit, at 616 31.6 and 23.4.)
 constexpr int FUSED_MID_C = 512;
-GemmKernel gemm_kernel(const sq_matrix* mats, int n, int T) {
+GemmKernel gemm_route(const sq_matrix* mats, int n, int T, int x_dtype) {
     const FusedPlan fused = fused_plan(mats, n, T);
     const bool d8 = mats[0].d == 8;
     float most = 50.f;                                           // us that the kernel of sq_mid.h may take beyond mid_ok
     if (fused.nw) {
         if (d8) {
-            int64_t w = 0;
-            for (int i = 0; i < n; ++i) w += (mats[i].R + 32 * fused.tw - 1) / (32 * fused.tw);
-            if (!(fused.tbs == 2 && w * fused.ks * 2 <= device_cus() && planes_route(mats, n, T, SQ_BF16))) return GEMM_FUSED;
+            if (!fused_two_blocks(fused, mats, n) || tiles_us_two_blocks(mats, n, T) >= fused_us(fused, mats, n)) return GEMM_FUSED;
         } else {
             most = 80.f;
             const float us = mats[0].C < FUSED_MID_C ? 1e30f : mid_us(mats, n, T);
@@ -409,7 +420,7 @@ GemmKernel gemm_kernel(const sq_matrix* mats, int n, int T) {
         if (plane_product_group(mats, n, T) == n) return GEMM_COLUMNS;
         if (mid_ok(mats, n, T)) return GEMM_MID;
         const float us = mid_us(mats, n, T);
-        if (us < most && us < (us < 50.f ? 0.9f : 0.73f) * tiles_us(mats, n, T)) return GEMM_MID;
+        if (us < most && us < (us < 50.f ? 0.9f : 0.73f) * tiles_us(mats, n, T, x_dtype)) return GEMM_MID;
         if (T <= small_pass_limit(mats, n)) return GEMM_PASSES;
     }
     return decoded_route(mats, n, T) ? GEMM_DECODED : GEMM_TILES;
@@ -419,10 +430,11 @@ GemmKernel gemm_kernel(const sq_matrix* mats, int n, int T) {
 // microseconds (1e30: not for these pieces).
 extern "C" __attribute__((visibility("default"))) int32_t sq_gemm_kernel_for_tests(const sq_matrix* mats, int32_t n, int32_t T, int32_t x_dtype, float* us) {
     const FusedPlan fused = fused_plan(mats, n, T);
-    us[0] = fused.nw ? fused_us(fused, mats, n) : 1e30f;
+    const bool two = mats[0].d == 8 && fused.nw && fused_two_blocks(fused, mats, n);
+    us[0] = two || (fused.nw && mats[0].d == 4) ? fused_us(fused, mats, n) : 1e30f;
     us[1] = mid_us(mats, n, T);
-    us[2] = tiles_us(mats, n, T);
-    const GemmKernel k = gemm_kernel(mats, n, T);
+    us[2] = two ? tiles_us_two_blocks(mats, n, T) : tiles_us(mats, n, T, x_dtype);
+    const GemmKernel k = gemm_route(mats, n, T, x_dtype);
     return k == GEMM_TILES && planes_route(mats, n, T, x_dtype) ? 7 : k;
 }
 
@@ -439,13 +451,17 @@ static size_t gemm_workspace_beyond_small(const sq_matrix* mats, int n, int T) {
     // decode-time kernel, which the caller adds)
     if (T <= SQ_SMALL_BMAX && decoded_route(mats, n, T)) return decoded_workspace(mats, n, T);
     const size_t tiles = gemm_workspace_without_mid(mats, n, T) + (planes_route(mats, n, T, SQ_BF16) ? planes_bytes(std::min(n, GEMM256_PIECES)) : (size_t)0);
-    switch (gemm_kernel(mats, n, T)) {
-    case GEMM_FUSED: return std::max({tiles, fused_workspace(mats, n, T), mid_ok(mats, n, T) ? mid_workspace(mats, n, T) : (size_t)0});
-    case GEMM_COLUMNS: return std::max({tiles, mid_workspace(mats, n, T), plane_product_workspace(mats, n, T)});
-    case GEMM_MID: return std::max(tiles, mid_workspace(mats, n, T));
-    case GEMM_DECODED: return std::max(tiles, decoded_workspace(mats, n, T));
-    default: return tiles;
-    }
+    auto of = [&](GemmKernel k) {
+        switch (k) {
+        case GEMM_FUSED: return std::max({tiles, fused_workspace(mats, n, T), mid_ok(mats, n, T) ? mid_workspace(mats, n, T) : (size_t)0});
+        case GEMM_COLUMNS: return std::max({tiles, mid_workspace(mats, n, T), plane_product_workspace(mats, n, T)});
+        case GEMM_MID: return std::max(tiles, mid_workspace(mats, n, T));
+        case GEMM_DECODED: return std::max(tiles, decoded_workspace(mats, n, T));
+        default: return tiles;
+        }
+    };
+    const GemmKernel k = gemm_route(mats, n, T, SQ_BF16), k16 = mats[0].d == 8 ? gemm_route(mats, n, T, SQ_F16) : k;      // (d = 4: whatever x is)
+    return k == k16 ? of(k) : std::max(of(k), of(k16));
 }
 
 size_t gemm_workspace_without_mid(const sq_matrix* mats, int n, int T) {
@@ -517,7 +533,7 @@ int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_
     if (T <= SQ_SMALL_BMAX && !small_takes_gemm_route(mats, n, T, x, ldx))
         return launch_small(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, ws_bytes, sums, s);
     if (T > SQ_SMALL_BMAX && x_vec_ok(x, ldx, mats[0].C)) {
-        const GemmKernel k = gemm_kernel(mats, n, T);
+        const GemmKernel k = gemm_route(mats, n, T, x_dtype);
         if (k == GEMM_COLUMNS && plane_product_workspace(mats, n, T) <= ws_bytes) return launch_plane_product(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);
         // (the fused kernel's cuts also serve where a workspace or the span of x does not let the others in)
         const bool mid = mid_x_ok(ldx, T) && (mid_ok(mats, n, T) ? mid_least(mats, n, T) <= ws_bytes : k == GEMM_MID && gemm_workspace_without_mid(mats, n, T) <= ws_bytes);

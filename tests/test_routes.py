@@ -55,3 +55,24 @@ def test_a_kernel_is_given_up_for_the_one_it_was_compared_with():
     assert seen == {FUSED, MID, TILES}
     for case in (([7704], 8192, 4, 10, 4, 262), ([9792, 9792], 3200, 4, 12, 1, 260), ([6987, 1746, 1746], 4800, 4, 12, 1, 429), ([10752, 10752], 2880, 4, 8, 1, 325)):
         assert _kernel(*case)[0] == MID
+
+
+def test_two_blocks_of_tokens_are_compared_with_the_tiles():
+    """d = 8 at 385 to 768 rows: the fused kernel's one round of two blocks of tokens gives way to a decode and tiles where those are estimated to take less, whatever type x has
+    and whichever order their decode takes, and the kernel of small products is compared with the tiles of x's own type."""
+    for dtype in (_lib.SQ_BF16, _lib.SQ_F16):
+        assert _kernel([18944], 3584, 8, 16, 1, 450, dtype)[0] == TILES_IN_PLANE_ORDER
+        for case in (([9394, 9394], 576, 498), ([7749, 1937, 1937], 448, 483), ([10009, 10009], 13568, 490)):
+            assert _kernel(case[0], case[1], 8, 16, 1, case[2], dtype)[0] == FUSED
+    rng = random.Random(6)
+    seen, types = set(), 0
+    for _ in range(4000):
+        rows, C, T, dtype = _rows(rng), max(192, _log(rng, 192, 14000) // 64 * 64), rng.randint(385, 768), rng.choice((_lib.SQ_BF16, _lib.SQ_F16))
+        k, us = _kernel(rows, C, 8, 16, 1, T, dtype)
+        if us[0] < 1e29:
+            seen.add((k, dtype))
+            assert (k == FUSED) == (us[2] >= us[0]), (rows, C, T, us)
+        elif k in (MID, TILES, TILES_IN_PLANE_ORDER):
+            types += _kernel(rows, C, 8, 16, 1, T, _lib.SQ_BF16)[1][2] != _kernel(rows, C, 8, 16, 1, T, _lib.SQ_F16)[1][2]
+            assert (k == MID) == (us[1] < (0.9 if us[1] < 50 else 0) * us[2]), (rows, C, T, us)
+    assert seen >= {(k, t) for k in (FUSED, TILES, TILES_IN_PLANE_ORDER) for t in (_lib.SQ_BF16, _lib.SQ_F16)} and types
