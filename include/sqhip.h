@@ -78,14 +78,18 @@ int sq_dequant_stack(const sq_matrix* mats, int32_t n_mats, void* out, const voi
  * sq_workspace_bytes; the latter keep their partial sums in its header); from 3 to 17 activation rows on, depending
  * on the stack (csrc/sq_gemm.hip), one that has column orders (with C % 8 == 0, 16-byte aligned x, ldx % 8 == 0) is decoded
  * to fp16 in the workspace and multiplied from there, which is faster than its decode-time kernel.
- * Two kinds of pieces without column orders have a faster kernel that needs workspace, where x is aligned like that; with less than it
+ * Four kinds of pieces without column orders have a faster kernel that needs workspace, where x is aligned like that; with less than it
  * needs they run on their other one, whose fp32 additions come in another order:
  *   - from 3 rows on, where an estimate says that it pays and no piece of the stack has column orders, pieces of formats without a
  *     matrix-core kernel (tag widths other than 16 at d = 8, and 12, 10 and 8 at d = 4; rows that end within a unit of their tags with
  *     16-bit tags, codebooks beyond 128 KB or no tile-major copy) are decoded to fp16, at most 192 MB at a time, and multiplied from
  *     there; bf16 activations keep their range and bits on both ways, as they do on d = 4 rows that end within a unit;
  *   - up to 16 rows large pieces with d = 8, 16-bit tags, one codebook and C % 64 == 0 that have no slice stream for these rows keep 8
- *     to 64 partial sums per result (fp32).  Where those are more than 16 MB the rows go a part at a time in 16 MB, with the same bits.
+ *     to 64 partial sums per result (fp32).  Where those are more than 16 MB the rows go a part at a time in 16 MB, with the same bits;
+ *   - from 17 rows on such pieces keep their codebooks (1 MB each) and the activations in another order and 4 or 8 partial sums per result, and where all of
+ *     that is more than 16 MB the rows go in parts as well, with the same bits;
+ *   - from 17 rows on stacks of d = 4 pieces, where an estimate says that it pays, keep up to 8 partial sums per result, at most 16 MB of them (with less
+ *     workspace, fewer: another order of additions on the same kernel).
  * All other kernels, but the one for x of other alignments, multiply activations as fp16.  sq_workspace_bytes(which = 0) accounts for
  * all of this, which | 4 for the least that the call runs with. */
 #define SQ_SMALL_BMAX 32
@@ -101,7 +105,8 @@ int sq_linear_small(const sq_matrix* mats, int32_t n_mats, const void* x, int x_
  * (sq_workspace_bytes(mats, n_mats, B, 0)) exceeds the array are refused with SQ_EWORKSPACE, except stacks
  * that need so much for their decoded weights only, where they have no column orders, up to 10 rows or C % 64 != 0: those run on the decode-time
  * kernel, whose results may differ from sq_linear_small's in the order of fp32 additions, and d = 4 pieces whose rows one launch
- * takes whole as well, which then differ in the same way (sq_linear_small with too small a workspace too).  Nothing is allocated or freed,
+ * takes whole as well, which then differ in the same way (sq_linear_small with too small a workspace too; the 16 MB behind the array's header are
+ * enough for all of the kinds above but the first).  Nothing is allocated or freed,
  * here or in anything it calls.  All calls on one GPU share that GPU's array: calls that overlap in time on one GPU
  * (two streams, two threads) race; calls on one stream are safe. */
 #define SQ_NOALLOC_SCRATCH_BYTES (48u << 20)

@@ -156,7 +156,7 @@ int sq_linear_small(const sq_matrix* mats, int32_t n_mats, const void* x, int x_
 // In host code `g_static_scratch` is only a handle for hipGetSymbolAddress: the device address it stands for is looked
 // up once per device and kept; kernels are handed that address, never the symbol.
 static_assert(sq::SQ_WS_HEADER == SQ_WS_HEADER_BYTES, "the header size is part of the ABI");
-static_assert(SQ_NOALLOC_SCRATCH_BYTES - sq::SQ_WS_HEADER >= sq::SIEVE_ROOM, "the same kernels as with a workspace of any size");
+static_assert(SQ_NOALLOC_SCRATCH_BYTES - sq::SQ_WS_HEADER >= sq::SMALL_ROOM, "the same kernels as with a workspace of any size");
 static __device__ __align__(256) unsigned char g_static_scratch[SQ_NOALLOC_SCRATCH_BYTES];
 static std::atomic<void*> g_static_scratch_ptr[64];
 // Rows up to which a stack with column orders whose decoded weights the scratch cannot hold runs on the decode-time kernel instead

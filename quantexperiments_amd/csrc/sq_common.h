@@ -151,8 +151,10 @@ int launch_small(const sq_matrix* mats, int n, const void* x, int x_dtype, int64
 // one activation row of these pieces is a single launch of the tag-stream kernel, which can produce its own x
 int sieve_group(const sq_matrix* mats, int n, int T);
 size_t sieve_workspace(const sq_matrix* mats, int n, int T);
-// what launch_sieve can do with, in more launches: SIEVE_ROOM, which sq_linear_small_noalloc has, or less where there is less to keep
-constexpr size_t SIEVE_ROOM = (size_t)16 << 20;
+// What sq_linear_small_noalloc has behind its header.  Kernels that keep sums for up to SQ_SMALL_BMAX rows take the same cuts, and so the same sums, with this much
+// as with more: in parts of the rows, or because they plan with no more than this.  The _least sizes are what they can do with, in more launches: this, or less
+// where there is less to keep
+constexpr size_t SMALL_ROOM = (size_t)16 << 20;
 size_t sieve_workspace_least(const sq_matrix* mats, int n, int T);
 int launch_sieve(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, size_t ws_bytes, hipStream_t s);
 bool small_fuses_producer(const sq_matrix* mats, int n, int B);
@@ -224,7 +226,9 @@ int launch_planes(const sq_matrix* mats, int n, uint16_t* out, uint16_t* planes,
 // one on, it takes in one launch; 0 where the other kernels are the faster way
 int plane_product_group(const sq_matrix* mats, int n, int T);
 size_t plane_product_workspace(const sq_matrix* mats, int n, int T);
-int launch_plane_product(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, hipStream_t s);
+size_t plane_product_workspace_least(const sq_matrix* mats, int n, int T);     // (up to SQ_SMALL_BMAX rows)
+int launch_plane_product(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, size_t ws_bytes,
+                         hipStream_t s);
 int launch_dequant_stack(const sq_matrix* mats, int n, void* out, int raw, const uint16_t* x, int64_t ldx, int T, int C, uint16_t* xout, hipStream_t s);
 int launch_gemm_dense(const void* w, int w_dtype, int64_t ldw, int R, int C, const void* x, int x_dtype, int64_t ldx,
                       void* y, int y_dtype, int64_t ldy, int T, hipStream_t s, void* ws = nullptr, size_t ws_bytes = 0);

@@ -534,7 +534,7 @@ int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_
         return launch_small(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, ws_bytes, sums, s);
     if (T > SQ_SMALL_BMAX && x_vec_ok(x, ldx, mats[0].C)) {
         const GemmKernel k = gemm_route(mats, n, T, x_dtype);
-        if (k == GEMM_COLUMNS && plane_product_workspace(mats, n, T) <= ws_bytes) return launch_plane_product(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);
+        if (k == GEMM_COLUMNS && plane_product_workspace(mats, n, T) <= ws_bytes) return launch_plane_product(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, ws_bytes, s);
         // (the fused kernel's cuts also serve where a workspace or the span of x does not let the others in)
         const bool mid = mid_x_ok(ldx, T) && (mid_ok(mats, n, T) ? mid_least(mats, n, T) <= ws_bytes : k == GEMM_MID && gemm_workspace_without_mid(mats, n, T) <= ws_bytes);
         if (k == GEMM_FUSED || !mid)

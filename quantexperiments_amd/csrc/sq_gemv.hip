@@ -485,8 +485,8 @@ int launch_small(const sq_matrix* mats, int n, const void* x, int x_dtype, int64
             i += k;
             continue;
         }
-        if (const int k = !x_ok ? 0 : plane_product_len(mats + i, n - i, B); k > 0 && plane_product_workspace(mats + i, k, B) <= ws_bytes) {
-            if (const int rc = launch_plane_product(mats + i, k, x, x_dtype, ldx, y, y_dtype, ldy, B, ws, s)) return rc;
+        if (const int k = !x_ok ? 0 : plane_product_len(mats + i, n - i, B); k > 0 && plane_product_workspace_least(mats + i, k, B) <= ws_bytes) {
+            if (const int rc = launch_plane_product(mats + i, k, x, x_dtype, ldx, y, y_dtype, ldy, B, ws, ws_bytes, s)) return rc;
             ws_off += small_need(mats + i, k, B, tight);
             i += k;
             continue;

@@ -139,14 +139,17 @@ size_t mid_least(const sq_matrix* mats, int n, int T) {
     return 0;
 }
 
+// (a decode step's sums are those that sq_linear_small_noalloc has room for)
+static size_t mid_room(int T, size_t room) { return T <= SQ_SMALL_BMAX ? std::min(room, SMALL_ROOM) : room; }
+
 size_t mid_workspace(const sq_matrix* mats, int n, int T) {
-    const MidPlan p = mid_plan(mats, n, T, device_cus(), SIZE_MAX);
+    const MidPlan p = mid_plan(mats, n, T, device_cus(), mid_room(T, SIZE_MAX));
     const size_t need = mid_sums_bytes(mats, n, T, p.ks);
     return T > SQ_SMALL_BMAX && T <= mid_limit(mats, n) ? std::max(need, mid_least(mats, n, T)) : need;
 }
 
 // Estimated time at T rows with `room` bytes for sums; a very long one where the kernel does not take the pieces
-float mid_us(const sq_matrix* mats, int n, int T, size_t room) { return mid_shape(mats, n, T) ? mid_plan(mats, n, T, device_cus(), room).us : 1e30f; }
+float mid_us(const sq_matrix* mats, int n, int T, size_t room) { return mid_shape(mats, n, T) ? mid_plan(mats, n, T, device_cus(), mid_room(T, room)).us : 1e30f; }
 
 // For tests: the cut that a stack takes at T rows, as token tiles | weight tiles << 8 | waves << 16 | K slices << 24; 0: the kernel does not take it.
 extern "C" __attribute__((visibility("default"))) int32_t sq_mid_variant_for_tests(const sq_matrix* mats, int32_t n, int32_t T) {
@@ -217,7 +220,7 @@ int launch_mid_decoded(const sq_matrix* mats, int n, const void* const* w, const
 int launch_mid(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws,
                size_t ws_bytes, hipStream_t s) {
     if (T > SQ_SMALL_BMAX && T <= mid_limit(mats, n) && mid_least(mats, n, T) > ws_bytes) return fail(SQ_EWORKSPACE, "sq_linear_gemm: workspace %zu < %zu", ws_bytes, mid_workspace(mats, n, T));
-    return launch_mid_rows(mats, n, mid_plan(mats, n, T, device_cus(), ws_bytes), nullptr, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);
+    return launch_mid_rows(mats, n, mid_plan(mats, n, T, device_cus(), mid_room(T, ws_bytes)), nullptr, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);
 }
 
 }  // namespace sq

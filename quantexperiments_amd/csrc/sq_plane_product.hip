@@ -74,12 +74,12 @@ __global__ __launch_bounds__(64) void pp_order_kernel(PpOrderArgs a) {
 
 struct PpPiece {
     sq_matrix m;
+    const uint16_t* planes;                  // of its codebook
     float* part;                             // fp32 [8 / pl, T, R rounded up to 4]
     int job0, parts;                         // first job; parts of the rows, a job each
 };
 struct PpArgs {
     PpPiece p[MID_PIECES];
-    const uint16_t* planes;
     const unsigned char* xf;
     int n, T, chunks, pairs, jobs, pl;       // pl: planes of a workgroup, one after the other
 };
@@ -120,7 +120,7 @@ __global__ __launch_bounds__(64 * PP_WAVES) void plane_product_kernel(PpArgs a) 
             const int e = pg * a.pl + q;
             if (round == 0 || a.pl > 1) {
                 if (round > 0 || q > 0) __syncthreads();         // the plane before it has been read
-                const uint16_t* src = a.planes + ((int64_t)pi * 8 + e) * PLANE;
+                const uint16_t* src = P.planes + (int64_t)e * PLANE;
                 const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)src, 0, PLANE * 2, 0x00027000);
 #pragma unroll
                 for (int k = 0; k < PLANE * 2 / (64 * PP_WAVES * 16); ++k)
@@ -209,12 +209,12 @@ struct PpPlan { int tw, nt, pl, parts[MID_PIECES]; double us; };
 
 // Parts of the rows so that every CU has a workgroup, tiles of a wave in as few rounds as registers allow, evenly; one plane a workgroup or
 // two, whichever is estimated to take less.  Microseconds, fitted to 203 products (6 %): launches and activations; staging; look-ups and
-// products; activations to registers; sums.
-static PpPlan pp_plan(const sq_matrix* mats, int n, int T) {
+// products; activations to registers; sums.  (planes: that many a workgroup, if it is given)
+static PpPlan pp_plan(const sq_matrix* mats, int n, int T, int planes = 0) {
     int64_t tiles = 0, rows = 0;
     for (int i = 0; i < n; ++i) tiles += (mats[i].R + 15) / 16, rows += mats[i].R;
     PpPlan best{};
-    for (int pl = 1; pl <= 2; ++pl) {
+    for (int pl = planes ? planes : 1; pl <= (planes ? planes : 2); ++pl) {
         PpPlan p{};
         p.nt = (T + 15) / 16; p.pl = pl;
         int64_t per = 0;                     // most tiles of a part
@@ -227,7 +227,7 @@ static PpPlan pp_plan(const sq_matrix* mats, int n, int T) {
         p.tw = (int)((wave + rounds - 1) / rounds);
         const double steps = (double)((mats[0].C / 8 + 63) / 64) * rounds * pl;
         p.us = 10.3 + 1.3 * n + 5.75e-6 * T * mats[0].C + 1.7 * (pl > 1 ? pl * rounds : 1) + steps * (p.tw * (0.36 + 0.016 * p.nt) + 0.0103 * p.nt) + 11.6e-6 / pl * T * rows;
-        if (pl == 1 || p.us < best.us) best = p;
+        if (!best.pl || p.us < best.us) best = p;
     }
     return best;
 }
@@ -244,22 +244,31 @@ static int pp_fit(const sq_matrix* mats, int n, int T) {
     return k;
 }
 
+// What a launch keeps besides the sums, and the sums of so many rows in n pieces
+static size_t pp_fixed_bytes(const sq_matrix* mats, int n, int nt) { return planes_bytes(n) + pp_x_bytes(mats, nt); }
+static size_t pp_sums_bytes(int64_t rows, int n, int T, int pl) { return (size_t)(8 / pl) * T * 4 * (rows + 4 * n) + 256 * n; }
+
 // The gathers from L2 take 8 us and 4.75 more per million tags up to 32 rows (fitted to 12 products: 10 %), and then what mid_us says; here has
-// to be estimated a seventh faster (8000 x 2048 at 32 / 64 rows 17.3 / 18.7 there, 20.8 / 25 here; 3584 x 3584 16.8 / 19.0, 17.7 / 21.7).
+// to be estimated a seventh faster (8000 x 2048 at 32 / 64 rows 17.3 / 18.7 there, 20.8 / 25 here; 3584 x 3584 16.8 / 19.0, 17.7 / 21.7).  A decode step's
+// products also need room for a fair part of their rows' sums in what sq_linear_small_noalloc has.
+constexpr int PP_PART_ROWS = 4096;
 int plane_product_group(const sq_matrix* mats, int n, int T) {
     const int k = pp_fit(mats, n, T);
     double tags = 0.0;
     for (int i = 0; i < k; ++i) tags += (double)mats[i].R * mats[i].C / 8e6;
     if (tags < 2.0) return 0;                // (no product of that size gains; the estimates cost the host a microsecond)
-    return pp_plan(mats, k, T).us < 0.85 * (T <= SQ_SMALL_BMAX ? 8.0 + 4.75 * tags : (double)mid_us(mats, k, T)) ? k : 0;
+    const PpPlan p = pp_plan(mats, k, T);
+    if (T <= SQ_SMALL_BMAX && pp_fixed_bytes(mats, k, p.nt) + pp_sums_bytes(PP_PART_ROWS, k, T, p.pl) > SMALL_ROOM) return 0;
+    return p.us < 0.85 * (T <= SQ_SMALL_BMAX ? 8.0 + 4.75 * tags : (double)mid_us(mats, k, T)) ? k : 0;
 }
 
 size_t plane_product_workspace(const sq_matrix* mats, int n, int T) {
     const PpPlan p = pp_plan(mats, n, T);
-    size_t need = planes_bytes(n) + pp_x_bytes(mats, p.nt);
+    size_t need = pp_fixed_bytes(mats, n, p.nt);
     for (int i = 0; i < n; ++i) need += pp_part_bytes(mats[i].R, T, p.pl);
     return need;
 }
+size_t plane_product_workspace_least(const sq_matrix* mats, int n, int T) { return std::min(plane_product_workspace(mats, n, T), SMALL_ROOM); }
 
 typedef void (*pp_kernel_t)(PpArgs);
 template <int TW, int NT>
@@ -268,22 +277,28 @@ static constexpr pp_kernel_t pp_kernel() {
     else return nullptr;
 }
 
-int launch_plane_product(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, hipStream_t s) {
-    const PpPlan p = pp_plan(mats, n, T);
+// Rows of all pieces, or, where their sums do not fit the workspace (plane_product_workspace_least: up to SQ_SMALL_BMAX activation rows), as many at a time as do, evenly
+// cut.  A row's sums depend on the planes a workgroup takes alone, which are those of the whole product: the results are the same bits either way.
+int launch_plane_product(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, size_t ws_bytes,
+                         hipStream_t s) {
+    const PpPlan whole = pp_plan(mats, n, T);
+    const size_t fixed = pp_fixed_bytes(mats, n, whole.nt);
+    int64_t rows = 0;
+    for (int i = 0; i < n; ++i) rows += mats[i].R;
+    int64_t most = rows;                     // weight rows of a launch
+    if (plane_product_workspace(mats, n, T) > ws_bytes) {
+        const size_t none = fixed + pp_sums_bytes(0, n, T, whole.pl);
+        const int64_t fit = ws_bytes > none ? (int64_t)((ws_bytes - none) / ((size_t)(8 / whole.pl) * T * 4)) / 16 * 16 : 0;
+        if (fit < 16) return fail(SQ_EWORKSPACE, "plane product: workspace %zu < %zu", ws_bytes, plane_product_workspace(mats, n, T));
+        const int64_t launches = (rows + fit - 1) / fit;
+        most = std::min(fit, ((rows + launches - 1) / launches + 15) / 16 * 16);
+    }
     PpOrderArgs o{};
-    PpArgs a{};
-    o.planes = (uint16_t*)ws; o.x = (const uint16_t*)x; o.ldx = ldx; o.pieces = n; o.T = T; o.NT = p.nt; o.n = mats[0].C / 8; o.pairs = (o.n + 63) / 64;
+    o.planes = (uint16_t*)ws; o.x = (const uint16_t*)x; o.ldx = ldx; o.pieces = n; o.T = T; o.NT = whole.nt; o.n = mats[0].C / 8; o.pairs = (o.n + 63) / 64;
     o.bf = x_dtype == SQ_BF16;
     o.xf = (unsigned char*)ws + planes_bytes(n);
-    char* sums = (char*)o.xf + pp_x_bytes(mats, p.nt);
-    a.planes = o.planes; a.xf = o.xf; a.n = n; a.T = T; a.chunks = o.n; a.pairs = o.pairs; a.pl = p.pl;
-    for (int i = 0; i < n; ++i) {
-        o.table[i] = mats[i].table;
-        a.p[i] = {mats[i], (float*)sums, a.jobs, p.parts[i]};
-        sums += pp_part_bytes(mats[i].R, T, p.pl);
-        a.jobs += p.parts[i];
-    }
-    const int64_t units = (int64_t)n * (PLANE / 8) + (int64_t)p.nt * 16 * o.pairs * 8;
+    for (int i = 0; i < n; ++i) o.table[i] = mats[i].table;
+    const int64_t units = (int64_t)n * (PLANE / 8) + (int64_t)whole.nt * 16 * o.pairs * 8;
     hipLaunchKernelGGL(pp_order_kernel, dim3((unsigned)((units + 63) / 64)), dim3(64), 0, s, o);
     if (const int rc = check_launch("plane order")) return rc;
 #define SQ_NT(NT) {pp_kernel<1, NT>(), pp_kernel<2, NT>(), pp_kernel<3, NT>(), pp_kernel<4, NT>(), pp_kernel<5, NT>()}
@@ -297,10 +312,31 @@ int launch_plane_product(const sq_matrix* mats, int n, const void* x, int x_dtyp
         return true;
     }();
     (void)raised;
-    const pp_kernel_t kernel = kernels[p.nt - 2][p.tw - 1];
-    hipLaunchKernelGGL(kernel, dim3((unsigned)((a.jobs + 7) / 8 * 8 * (8 / p.pl))), dim3(64 * PP_WAVES), PLANE * 2, s, a);
-    if (const int rc = check_launch("plane product")) return rc;
-    return launch_slice_sum(a.p, n, 8 / p.pl, T, y, y_dtype, ldy, s, /*whole_quads=*/true);
+    for (int i = 0, r0 = 0; i < n;) {
+        sq_matrix part[MID_PIECES];
+        PpArgs a{};
+        a.xf = o.xf; a.T = T; a.chunks = o.n; a.pairs = o.pairs; a.pl = whole.pl;
+        for (int64_t left = most; i < n && left > 0;) {
+            const int R = (int)std::min<int64_t>(mats[i].R - r0, left);
+            sq_matrix& m = part[a.n] = mats[i];
+            m.R = R; m.tags += (int64_t)r0 * m.W; m.row_scale += r0; m.y_off += r0;
+            a.p[a.n++].planes = o.planes + (int64_t)i * 8 * PLANE;
+            left -= R;
+            r0 += R;
+            if (r0 >= mats[i].R) ++i, r0 = 0;
+        }
+        const PpPlan p = most == rows ? whole : pp_plan(part, a.n, T, whole.pl);
+        char* sums = (char*)ws + fixed;
+        for (int j = 0; j < a.n; ++j) {
+            a.p[j].m = part[j]; a.p[j].part = (float*)sums; a.p[j].job0 = a.jobs; a.p[j].parts = p.parts[j];
+            sums += pp_part_bytes(part[j].R, T, p.pl);
+            a.jobs += p.parts[j];
+        }
+        hipLaunchKernelGGL(kernels[p.nt - 2][p.tw - 1], dim3((unsigned)((a.jobs + 7) / 8 * 8 * (8 / p.pl))), dim3(64 * PP_WAVES), PLANE * 2, s, a);
+        if (const int rc = check_launch("plane product")) return rc;
+        if (const int rc = launch_slice_sum(a.p, a.n, 8 / p.pl, T, y, y_dtype, ldy, s, /*whole_quads=*/true)) return rc;
+    }
+    return SQ_OK;
 }
 
 }  // namespace sq
@@ -310,5 +346,5 @@ extern "C" __attribute__((visibility("default"))) int64_t sq_plane_product_for_t
                                                                                      int32_t y_dtype, int64_t ldy, int32_t T, void* ws, void* stream) {
     if (n < 1 || sq::pp_fit(mats, n, T) != n) return SQ_EUNSUPPORTED;
     if (!ws) return (int64_t)sq::plane_product_workspace(mats, n, T);
-    return sq::launch_plane_product(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, (hipStream_t)stream);
+    return sq::launch_plane_product(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, sq::plane_product_workspace(mats, n, T), (hipStream_t)stream);
 }

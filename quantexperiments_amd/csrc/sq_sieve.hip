@@ -270,7 +270,7 @@ size_t sieve_workspace(const sq_matrix* mats, int n, int T) {
     for (int i = 0; i < n; ++i) need += sieve_part_bytes(mats[i].R, T, pl.ks);
     return need;
 }
-size_t sieve_workspace_least(const sq_matrix* mats, int n, int T) { return std::min(sieve_workspace(mats, n, T), SIEVE_ROOM); }
+size_t sieve_workspace_least(const sq_matrix* mats, int n, int T) { return std::min(sieve_workspace(mats, n, T), SMALL_ROOM); }
 
 // How many of the n pieces, the first one on, the kernel takes in one launch, 0 where the gathers from L2 are the faster way: they
 // take 4.6 us per million tags and 4 more, 1.1 to 1.3 times that for rows of more than 8192 columns (4096 x 4096 at 9 / 16 rows 15.5 /

@@ -116,6 +116,17 @@ def test_decode_batches_match_oracle(case, dtype, stream):
     assert torch.equal(lowp[:, :sum(rows)], y.to(dtype)) and not lowp[:, sum(rows):].any()
 
 
+@pytest.mark.parametrize("rows,C,bits,G,T", [((17000, 17001), 1600, 12, 4, 32), ((2501,), 9408, 12, 1, 17), ((540,) * 9, 512, 8, 4, 20)], ids=lambda v: str(v))
+def test_decode_batches_have_the_same_sums_without_a_workspace_argument(rows, C, bits, G, T):
+    lins = [to_device(synth(R, C, 4, bits, G, 1, seed=R + T + i)) for i, R in enumerate(rows)]
+    mats = _lib.matrix_array([m.descriptor(o) for m, o in zip(lins, np.cumsum([0] + list(rows)).tolist())])
+    x = rand_x(T, C, torch.bfloat16, seed=T).cuda()
+    y, z = torch.empty(2, T, sum(rows), device="cuda")
+    linear_small(lins, x, y)
+    _lib.check(_lib.lib().sq_linear_small_noalloc(mats, len(lins), x.data_ptr(), _lib.SQ_BF16, C, z.data_ptr(), _lib.SQ_F32, sum(rows), T, _lib.stream_ptr(x.device)))
+    assert torch.equal(z, y)
+
+
 @pytest.mark.parametrize("T", [64, 500])
 def test_least_workspace_is_enough_and_less_is_refused(T):
     """K slices are as many as the workspace holds; what a call refused for lack of it is refused."""

@@ -89,6 +89,32 @@ def test_large_products_take_it(R, C, T):
     assert rel_max_err(y.float().cpu().numpy(), (x.half().double() @ w.T).cpu().numpy()) < 2.0 ** -8 + 1e-5
 
 
+@pytest.mark.parametrize("rows,C,T", [((18944, 18944), 3584, 24), ((18944, 18944), 3584, 32), ((18945, 3, 18950), 3584, 31), ((60001,), 2112, 32), ((7003,) * 8, 3008, 27), ((4000, 50003, 2), 3584, 17)],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_sums_that_do_not_fit_at_once(rows, C, T):
+    """Decode batches: rows a part at a time in the workspace there is are the bits of the whole product, also through the entry point that has 16 MB behind
+    its header, and nothing behind the workspace is touched."""
+    lins = [to_device(synth(R, C, 8, 16, 1, 1, seed=R + T), stream=False) for R in rows]
+    mats, R = _mats(lins), sum(rows)
+    L, room = _lib.lib(), 16 << 20
+    assert L.sq_workspace_bytes(mats, len(lins), T, 2) > room
+    x = rand_x(T, C, torch.bfloat16, seed=T)
+    x[2, 5] = float("inf")
+    x = x.cuda()
+    want, y = (torch.full((T, R), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    _call(lins, x, want)
+    linear_small(lins, x, y)
+    assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+    args = (mats, len(lins), x.data_ptr(), _lib.SQ_BF16, C, y.data_ptr(), _lib.SQ_BF16, R, T)
+    y.fill_(float("nan"))
+    _lib.check(L.sq_linear_small_noalloc(*args, _lib.stream_ptr(x.device)))
+    assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+    ws = torch.full((room + 4096,), 0x5A, dtype=torch.uint8, device="cuda")
+    y.fill_(float("nan"))
+    _lib.check(L.sq_linear_small(*args, ws.data_ptr(), room, _lib.stream_ptr(x.device)))
+    assert torch.equal(y.view(torch.int16), want.view(torch.int16)) and bool((ws[room:] == 0x5A).all())
+
+
 @pytest.mark.parametrize("R,C,d,bits,G,M,T", [(99, 64, 8, 16, 1, 1, 16), (99, 64, 8, 16, 1, 1, 129), (99, 72, 8, 16, 1, 1, 20), (99, 64, 8, 16, 2, 1, 20), (99, 64, 8, 16, 1, 2, 20),
                                               (99, 64, 8, 15, 1, 1, 20), (99, 64, 4, 16, 1, 1, 20)])
 def test_what_it_refuses(R, C, d, bits, G, M, T):
