@@ -49,13 +49,18 @@ def test_decode_is_the_codewords_in_plane_order(rows, C, T, dtype):
     assert bool((out[-guard:] == 7).all()) and bool((xout[-guard:] == 7).all())
 
 
-# the last: too little to gain, decoded a codeword at a time
-@pytest.mark.parametrize("rows,C,T", [((3001, 3000), 3584, 900), ((26003,), 1280, 520), ((1000, 250, 249), 4032, 700), ((18944,), 1600, 1030), ((1100,), 1024, 2000)],
-                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+PRODUCTS = [((3001, 3000), 3584, 900, (7, 7)), ((26003,), 1280, 520, (7, 7)), ((1000, 250, 249), 4032, 700, (7, 7)), ((18944,), 1600, 1030, (7, 6)), ((1100,), 1024, 2000, (6, 6))]
+
+
+# kernels: the one that bf16 and that fp16 activations take, 7 where the codebooks go in columns, 6 a codeword at a time (too little to gain)
+@pytest.mark.parametrize("rows,C,T,kernels", PRODUCTS, ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
-def test_products(rows, C, T, dtype):
+def test_products(rows, C, T, kernels, dtype):
     ss = [synth(R, C, 8, 16, 1, 1, seed=R) for R in rows]
     lins = [to_device(s, stream=False) for s in ss]
+    mats = _lib.matrix_array([m.descriptor(sum(rows[:i])) for i, m in enumerate(lins)])
+    kernel = _lib.lib().sq_gemm_kernel_for_tests(mats, len(lins), T, _lib.DTYPES[dtype], (ctypes.c_float * 3)())
+    assert torch.cuda.get_device_properties(0).multi_processor_count != 256 or kernel == kernels[dtype == torch.float16]
     x = torch.zeros(T, C + 8, dtype=dtype)
     x[:, :C] = rand_x(T, C, dtype, seed=T)
     xd = x.cuda()[:, :C]
