@@ -41,6 +41,8 @@
 // LDS clock (rows 0-3, 12-15 of one lane group with rows 4-11 of the next, and so on) fall into 16 different groups of four
 // banks.
 #pragma once
+#include <iterator>
+#include <utility>
 #include <type_traits>
 #include "sq_rows_mfma.h"
 
@@ -332,23 +334,31 @@ int launch_mid_as(const MidArgs& a, int grid, hipStream_t s) {
     return a.x_dtype == SQ_BF16 ? launch_mid_dtype<BITS, D, NT, TW, S, NW, true>(a, grid, s) : launch_mid_dtype<BITS, D, NT, TW, S, NW, false>(a, grid, s);
 }
 
-// Variants: sq_mid.hip
-#define SQ_MID_CASE(NT_, TW_, NW_, S_) if (nt == NT_ && tw == TW_ && nw == NW_ && st == S_) return launch_mid_as<BITS, D, NT_, TW_, S_, NW_>(a, grid, s);
+// The variants there are, each a kernel per format and type of x: the plans of sq_mid.hip choose among them, the launch finds its kernel in the same list.
+struct MidVariant { int8_t nt, tw, nw, st; };
+inline constexpr MidVariant MID4[] = {{1, 1, 4, 4}, {2, 1, 4, 4}, {3, 1, 4, 4}, {4, 1, 4, 4}, {5, 1, 4, 4}, {1, 1, 8, 4}, {2, 1, 8, 4}, {3, 1, 8, 4}, {4, 1, 8, 4},
+                                      {5, 1, 8, 4}, {8, 1, 8, 4}, {3, 2, 8, 4}, {4, 2, 8, 4}, {5, 2, 8, 4}, {8, 2, 8, 4}, {3, 1, 10, 4}, {3, 1, 12, 4}, {5, 1, 10, 4},
+                                      {5, 1, 12, 4}, {5, 1, 8, 2}, {8, 1, 8, 2}, {5, 2, 8, 2}, {8, 2, 8, 2}};
+inline constexpr MidVariant MID8[] = {{1, 1, 4, 4}, {2, 1, 4, 4}, {3, 1, 4, 4}, {4, 1, 4, 4}, {5, 1, 4, 4}, {3, 1, 8, 4}, {4, 1, 8, 4}, {5, 1, 8, 4}, {8, 1, 8, 4},
+                                      {12, 1, 8, 2}, {16, 1, 8, 2}, {3, 1, 10, 4}, {3, 1, 12, 4}, {5, 1, 10, 4}, {5, 1, 12, 4}, {8, 1, 12, 4}, {12, 1, 12, 2}, {5, 2, 8, 4},
+                                      {8, 2, 8, 4}, {12, 2, 8, 2}, {16, 2, 8, 2}};
+inline constexpr MidVariant MID_DENSE[] = {{1, 1, 8, 4}, {3, 1, 8, 4}, {5, 1, 8, 4}, {8, 1, 8, 4}, {12, 1, 8, 2}, {16, 1, 8, 2}};
+template <int D> constexpr const auto& mid_variants() {
+    if constexpr (D == 4) return MID4;
+    else if constexpr (D == 8) return MID8;
+    else return MID_DENSE;
+}
+
+template <int BITS, int D, size_t... I>
+int launch_mid_variant(std::index_sequence<I...>, const MidArgs& a, int nt, int tw, int st, int nw, int grid, hipStream_t s) {
+    constexpr const auto& v = mid_variants<D>();
+    int rc = SQ_EUNSUPPORTED;
+    (void)((nt == v[I].nt && tw == v[I].tw && nw == v[I].nw && st == v[I].st && (rc = launch_mid_as<BITS, D, v[I].nt, v[I].tw, v[I].st, v[I].nw>(a, grid, s), true)) || ...);
+    return rc;
+}
 template <int BITS, int D>
 int launch_mid_format(const MidArgs& a, int nt, int tw, int st, int nw, int grid, hipStream_t s) {
-    SQ_MID_CASE(1, 1, 8, 4) SQ_MID_CASE(3, 1, 8, 4) SQ_MID_CASE(5, 1, 8, 4) SQ_MID_CASE(8, 1, 8, 4)
-    if constexpr (D != 4) { SQ_MID_CASE(12, 1, 8, 2) SQ_MID_CASE(16, 1, 8, 2) }
-    if constexpr (D != 0) {
-        SQ_MID_CASE(1, 1, 4, 4) SQ_MID_CASE(2, 1, 4, 4) SQ_MID_CASE(3, 1, 4, 4) SQ_MID_CASE(4, 1, 4, 4) SQ_MID_CASE(5, 1, 4, 4)
-        SQ_MID_CASE(4, 1, 8, 4) SQ_MID_CASE(5, 2, 8, 4) SQ_MID_CASE(8, 2, 8, 4)
-        SQ_MID_CASE(3, 1, 10, 4) SQ_MID_CASE(3, 1, 12, 4) SQ_MID_CASE(5, 1, 10, 4) SQ_MID_CASE(5, 1, 12, 4)
-    }
-    if constexpr (D == 8) { SQ_MID_CASE(8, 1, 12, 4) SQ_MID_CASE(12, 1, 12, 2) SQ_MID_CASE(12, 2, 8, 2) SQ_MID_CASE(16, 2, 8, 2) }
-    if constexpr (D == 4) {
-        SQ_MID_CASE(2, 1, 8, 4) SQ_MID_CASE(3, 2, 8, 4) SQ_MID_CASE(4, 2, 8, 4)
-        SQ_MID_CASE(5, 1, 8, 2) SQ_MID_CASE(8, 1, 8, 2) SQ_MID_CASE(5, 2, 8, 2) SQ_MID_CASE(8, 2, 8, 2)
-    }
-    return SQ_EUNSUPPORTED;
+    return launch_mid_variant<BITS, D>(std::make_index_sequence<std::size(mid_variants<D>())>(), a, nt, tw, st, nw, grid, s);
 }
 
 #define SQ_MID_FORMAT(BITS, D)                                                                                             \

@@ -30,13 +30,6 @@ static int mid_units(const sq_matrix& m) { return m.W / (m.bits == 12 ? 3 : m.bi
 //   4096 x 1024     12.3 / 23.4 / 23.6     6.6 / 8.8 / 13.7         13.8 / 24.0 / 25.0    10.0 / 17.2 / 23.7
 //   3584 x 3584     15.8 / 30.5 / 45.0    13.3 / 18.8 / 30.9        21.6 / 36.1 / 46.8    21.8 / 36.3 / 68.6 (not taken)
 //   8000 x 2048     17.6 / 35.1 / 40.4    11.3 / 16.5 / 35.7
-struct MidVariant { int8_t nt, tw, nw, st; };
-static constexpr MidVariant MID4[] = {{1, 1, 4, 4}, {2, 1, 4, 4}, {3, 1, 4, 4}, {4, 1, 4, 4}, {5, 1, 4, 4}, {1, 1, 8, 4}, {2, 1, 8, 4}, {3, 1, 8, 4}, {4, 1, 8, 4},
-                                      {5, 1, 8, 4}, {8, 1, 8, 4}, {3, 2, 8, 4}, {4, 2, 8, 4}, {5, 2, 8, 4}, {8, 2, 8, 4}, {3, 1, 10, 4}, {3, 1, 12, 4}, {5, 1, 10, 4},
-                                      {5, 1, 12, 4}, {5, 1, 8, 2}, {8, 1, 8, 2}, {5, 2, 8, 2}, {8, 2, 8, 2}};
-static constexpr MidVariant MID8[] = {{1, 1, 4, 4}, {2, 1, 4, 4}, {3, 1, 4, 4}, {4, 1, 4, 4}, {5, 1, 4, 4}, {3, 1, 8, 4}, {4, 1, 8, 4}, {5, 1, 8, 4}, {8, 1, 8, 4},
-                                      {12, 1, 8, 2}, {16, 1, 8, 2}, {3, 1, 10, 4}, {3, 1, 12, 4}, {5, 1, 10, 4}, {5, 1, 12, 4}, {8, 1, 12, 4}, {12, 1, 12, 2}, {5, 2, 8, 4},
-                                      {8, 2, 8, 4}, {12, 2, 8, 2}, {16, 2, 8, 2}};
 // us: a launch; staged codebooks per KB and round of workgroups; per matrix step of a workgroup: a wave's product, its read of a tile of
 // activations, a tile of codewords, a tile of activations staged; a step by itself, per tile, and per tile that a wave stages; slices: their launch, and per million sums;
 // per million results; per tile of codewords over the chip
@@ -194,9 +187,7 @@ static int launch_mid_rows(const sq_matrix* mats, int n, const MidPlan& pl, cons
 // 111 in nine).
 static MidPlan mid_dense_plan(const sq_matrix* mats, int n, int T, int cus) {
     MidPlan p{0, 1, 8, 4, 1, 0.f};
-    const int sizes[] = {1, 3, 5, 8, 12, 16};
-    for (int nt : sizes) if (T <= nt * 16) { p.nt = nt; break; }
-    if (p.nt > 8) p.st = 2;
+    for (const MidVariant& v : MID_DENSE) if (T <= v.nt * 16) { p.nt = v.nt; p.st = v.st; break; }
     int64_t blocks = 0;
     for (int i = 0; i < n; ++i) blocks += (mats[i].R + 16 * 8 - 1) / (16 * 8);
     p.ks = (int)std::max<int64_t>(1, std::min<int64_t>({cus / std::max<int64_t>(blocks, 1), 8, mats[0].C / 256}));
