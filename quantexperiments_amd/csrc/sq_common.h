@@ -180,15 +180,17 @@ size_t decoded_workspace(const sq_matrix* mats, int n, int T);
 // (wide: bf16 activations keep their range and bits, up to 48 rows)
 int launch_decoded(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, hipStream_t s,
                    bool wide = false);
-// products in one pass over the tags (sq_mid.h): whether it is the way of these pieces in any case, its estimated time, and its call
+// products in one pass over the tags (sq_mid.h): whether it is the way of these pieces in any case, its cut with the estimated time (with `room` bytes for sums; nt = 0
+// and a very long time: not for these), and its call, with the cut that mid_plan gave for a workspace of any size or without it
+struct MidPlan { int nt, tw, nw, st, ks; float us; };
+MidPlan mid_plan(const sq_matrix* mats, int n, int T, size_t room = SIZE_MAX);
 bool mma_shape(const sq_matrix& m);
 bool mid_ok(const sq_matrix* mats, int n, int T);
 inline bool mid_x_ok(int64_t ldx, int T) { return (int64_t)T * ldx * 2 < (int64_t)1 << 32; }     // 32-bit offsets
-size_t mid_workspace(const sq_matrix* mats, int n, int T);
+size_t mid_workspace(const sq_matrix* mats, int n, int T, const MidPlan* planned = nullptr);
 size_t mid_least(const sq_matrix* mats, int n, int T);                   // (where mid_ok)
-float mid_us(const sq_matrix* mats, int n, int T, size_t room = SIZE_MAX);
 int launch_mid(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws,
-               size_t ws_bytes, hipStream_t s);
+               size_t ws_bytes, hipStream_t s, const MidPlan* planned = nullptr);
 // the same for weights already decoded to fp16, w[i] = [R, C] of piece i without row scales (1 .. 256 activation rows)
 bool mid_dense_ok(const sq_matrix* mats, int n, int T);
 size_t mid_dense_workspace(const sq_matrix* mats, int n, int T);
@@ -199,16 +201,19 @@ struct FusedPlan { int nw, tw, ks, tbs, t; };      // (t: activation rows)
 FusedPlan fused_plan(const sq_matrix* mats, int n, int T);               // nw = 0: not for these
 bool fused_two_blocks(const FusedPlan& p, const sq_matrix* mats, int n);      // of tokens, in one round of workgroups
 float fused_us(const FusedPlan& p, const sq_matrix* mats, int n);        // (d = 8: of those)
-size_t fused_workspace(const sq_matrix* mats, int n, int T);
-int launch_fused(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, hipStream_t s);
+size_t fused_workspace(const FusedPlan& p, const sq_matrix* mats, int n, int T);
+int launch_fused(const FusedPlan& p, const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, hipStream_t s);
 // most activation rows for which passes of SQ_SMALL_BMAX rows through the decode-time kernel beat decode + GEMM
 // for these pieces (0: never), where they cannot share a pass
 int small_pass_limit(const sq_matrix* mats, int n);
 size_t gemm_workspace(const sq_matrix* mats, int n, int T);
+constexpr int PLANE_PRODUCT_MIN_T = 17;
+struct PlanePlan { int tw, nt, pl, parts[MID_PIECES]; double us; };
 // The kernel that sq_linear_gemm runs n pieces on at more than SQ_SMALL_BMAX rows of aligned activations, given the workspace: sq_fused.h,
 // sq_plane_product.hip, sq_mid.h, passes of the decode-time kernel, decoded rows on sq_mid.h, the tile GEMM behind a decode (in 128 x 128 tiles: none)
 enum GemmKernel { GEMM_FUSED = 1, GEMM_COLUMNS, GEMM_MID, GEMM_PASSES, GEMM_DECODED, GEMM_TILES };
-GemmKernel gemm_route(const sq_matrix* mats, int n, int T, int x_dtype);
+struct GemmRoute { GemmKernel kernel; FusedPlan fused; MidPlan mid; PlanePlan columns; };      // and the cuts that were planned on the way (nw = 0, nt = 0: none)
+GemmRoute gemm_route(const sq_matrix* mats, int n, int T, int x_dtype);
 // what launch_gemm can do with less: the same product without the kernel of sq_mid.h
 size_t gemm_workspace_without_mid(const sq_matrix* mats, int n, int T);
 // Row scales of a product whose R rows are n stacked pieces: rows end[i - 1] .. end[i] - 1 are scaled by p[i]; n = 0: no scales.
@@ -224,11 +229,11 @@ size_t planes_bytes(int n);
 int launch_planes(const sq_matrix* mats, int n, uint16_t* out, uint16_t* planes, const void* x, int x_dtype, int64_t ldx, int T, uint16_t* xout, hipStream_t s);
 // 17 to 128 activation rows of 16-bit tags of width 8, a column of the codebook at a time (sq_plane_product.hip): how many of the n pieces, the first
 // one on, it takes in one launch; 0 where the other kernels are the faster way
-int plane_product_group(const sq_matrix* mats, int n, int T);
-size_t plane_product_workspace(const sq_matrix* mats, int n, int T);
-size_t plane_product_workspace_least(const sq_matrix* mats, int n, int T);     // (up to SQ_SMALL_BMAX rows)
+int plane_product_group(const sq_matrix* mats, int n, int T, PlanePlan& planned, const MidPlan* mid = nullptr);      // (mid: mid_plan of all n, where it is known)
+size_t plane_product_workspace(const sq_matrix* mats, int n, int T, const PlanePlan* planned = nullptr);
+size_t plane_product_workspace_least(const sq_matrix* mats, int n, int T, const PlanePlan* planned);     // (up to SQ_SMALL_BMAX rows)
 int launch_plane_product(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, size_t ws_bytes,
-                         hipStream_t s);
+                         hipStream_t s, const PlanePlan* planned = nullptr);
 int launch_dequant_stack(const sq_matrix* mats, int n, void* out, int raw, const uint16_t* x, int64_t ldx, int T, int C, uint16_t* xout, hipStream_t s);
 int launch_gemm_dense(const void* w, int w_dtype, int64_t ldw, int R, int C, const void* x, int x_dtype, int64_t ldx,
                       void* y, int y_dtype, int64_t ldy, int T, hipStream_t s, void* ws = nullptr, size_t ws_bytes = 0);

@@ -126,20 +126,19 @@ FusedPlan fused_plan(const sq_matrix* mats, int n, int T) {
 
 // For tests: the variant that a stack takes at T rows, as token tiles | weight tiles << 8 | K slices << 16 | token blocks << 24; 0: another kernel.
 extern "C" __attribute__((visibility("default"))) int32_t sq_fused_variant_for_tests(const sq_matrix* mats, int32_t n, int32_t T) {
-    if (gemm_route(mats, n, T, SQ_BF16) != GEMM_FUSED) return 0;
-    const FusedPlan p = fused_plan(mats, n, T);
+    const GemmRoute r = gemm_route(mats, n, T, SQ_BF16);
+    if (r.kernel != GEMM_FUSED) return 0;
+    const FusedPlan& p = r.fused;
     return p.nw | p.tw << 8 | p.ks << 16 | p.tbs << 24;
 }
 
-size_t fused_workspace(const sq_matrix* mats, int n, int T) {
-    const FusedPlan p = fused_plan(mats, n, T);
+size_t fused_workspace(const FusedPlan& p, const sq_matrix* mats, int n, int T) {
     size_t need = fused_x_bytes(mats, p);
     for (int i = 0; i < n; ++i) need += fused_part_bytes(mats[i], T, p.ks);
     return need;
 }
 
-int launch_fused(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, hipStream_t s) {
-    const FusedPlan p = fused_plan(mats, n, T);
+int launch_fused(const FusedPlan& p, const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, hipStream_t s) {
     const sq_matrix& m0 = mats[0];
     FusedArgs a{};
     a.n = n; a.y = y; a.ldy = ldy; a.T = T; a.y_dtype = y_dtype; a.ks = p.ks;

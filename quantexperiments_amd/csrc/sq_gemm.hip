@@ -403,27 +403,25 @@ static float tiles_us_two_blocks(const sq_matrix* mats, int n, int T) {
 // (44 products on whose way this and an older estimate of the tile GEMM disagree take 0.94 of the time in the mean,
 // none of them longer: 1078 + 1078 x 1408, 16-bit, at 610 rows 37.5 and 24.8, 8310 x 960, 8-bit, at 616 31.6 and 23.4.)
 constexpr int FUSED_MID_C = 512;
-GemmKernel gemm_route(const sq_matrix* mats, int n, int T, int x_dtype) {
-    const FusedPlan fused = fused_plan(mats, n, T);
-    const bool d8 = mats[0].d == 8;
+GemmRoute gemm_route(const sq_matrix* mats, int n, int T, int x_dtype) {
+    GemmRoute r{GEMM_FUSED, fused_plan(mats, n, T), {}, {}};
     float most = 50.f;                                           // us that the kernel of sq_mid.h may take beyond mid_ok
-    if (fused.nw) {
-        if (d8) {
-            if (!fused_two_blocks(fused, mats, n) || tiles_us_two_blocks(mats, n, T) >= fused_us(fused, mats, n)) return GEMM_FUSED;
-        } else {
-            most = 80.f;
-            const float us = mats[0].C < FUSED_MID_C ? 1e30f : mid_us(mats, n, T);
-            if (us > most || us > 0.85f * fused_us(fused, mats, n)) return GEMM_FUSED;
-        }
+    if (r.fused.nw && mats[0].d == 8) {
+        if (!fused_two_blocks(r.fused, mats, n) || tiles_us_two_blocks(mats, n, T) >= fused_us(r.fused, mats, n)) return r;
+    } else if (r.fused.nw) {
+        if (mats[0].C < FUSED_MID_C) return r;
+        most = 80.f;
+        r.mid = mid_plan(mats, n, T);
+        if (r.mid.us > most || r.mid.us > 0.85f * fused_us(r.fused, mats, n)) return r;
     }
     if (T > SQ_SMALL_BMAX) {
-        if (plane_product_group(mats, n, T) == n) return GEMM_COLUMNS;
-        if (mid_ok(mats, n, T)) return GEMM_MID;
-        const float us = mid_us(mats, n, T);
-        if (us < most && us < (us < 50.f ? 0.9f : 0.73f) * tiles_us(mats, n, T, x_dtype)) return GEMM_MID;
-        if (T <= small_pass_limit(mats, n)) return GEMM_PASSES;
+        if (!r.mid.nt) r.mid = mid_plan(mats, n, T);
+        if (plane_product_group(mats, n, T, r.columns, &r.mid) == n) { r.kernel = GEMM_COLUMNS; return r; }
+        if (r.mid.nt && (mid_ok(mats, n, T) || (r.mid.us < most && r.mid.us < (r.mid.us < 50.f ? 0.9f : 0.73f) * tiles_us(mats, n, T, x_dtype)))) { r.kernel = GEMM_MID; return r; }
+        if (T <= small_pass_limit(mats, n)) { r.kernel = GEMM_PASSES; return r; }
     }
-    return decoded_route(mats, n, T) ? GEMM_DECODED : GEMM_TILES;
+    r.kernel = decoded_route(mats, n, T) ? GEMM_DECODED : GEMM_TILES;
+    return r;
 }
 
 // For tests: that kernel (7: the tile GEMM behind a decode in plane order), and what the first one, the kernel of sq_mid.h and the tiles are estimated to take, in
@@ -432,9 +430,9 @@ extern "C" __attribute__((visibility("default"))) int32_t sq_gemm_kernel_for_tes
     const FusedPlan fused = fused_plan(mats, n, T);
     const bool two = mats[0].d == 8 && fused.nw && fused_two_blocks(fused, mats, n);
     us[0] = two || (fused.nw && mats[0].d == 4) ? fused_us(fused, mats, n) : 1e30f;
-    us[1] = mid_us(mats, n, T);
+    us[1] = mid_plan(mats, n, T).us;
     us[2] = two ? tiles_us_two_blocks(mats, n, T) : tiles_us(mats, n, T, x_dtype);
-    const GemmKernel k = gemm_route(mats, n, T, x_dtype);
+    const GemmKernel k = gemm_route(mats, n, T, x_dtype).kernel;
     return k == GEMM_TILES && planes_route(mats, n, T, x_dtype) ? 7 : k;
 }
 
@@ -451,17 +449,15 @@ static size_t gemm_workspace_beyond_small(const sq_matrix* mats, int n, int T) {
     // decode-time kernel, which the caller adds)
     if (T <= SQ_SMALL_BMAX && decoded_route(mats, n, T)) return decoded_workspace(mats, n, T);
     const size_t tiles = gemm_workspace_without_mid(mats, n, T) + (planes_route(mats, n, T, SQ_BF16) ? planes_bytes(std::min(n, GEMM256_PIECES)) : (size_t)0);
-    auto of = [&](GemmKernel k) {
-        switch (k) {
-        case GEMM_FUSED: return std::max({tiles, fused_workspace(mats, n, T), mid_ok(mats, n, T) ? mid_workspace(mats, n, T) : (size_t)0});
-        case GEMM_COLUMNS: return std::max({tiles, mid_workspace(mats, n, T), plane_product_workspace(mats, n, T)});
-        case GEMM_MID: return std::max(tiles, mid_workspace(mats, n, T));
-        case GEMM_DECODED: return std::max(tiles, decoded_workspace(mats, n, T));
-        default: return tiles;
-        }
-    };
-    const GemmKernel k = gemm_route(mats, n, T, SQ_BF16), k16 = mats[0].d == 8 ? gemm_route(mats, n, T, SQ_F16) : k;      // (d = 4: whatever x is)
-    return k == k16 ? of(k) : std::max(of(k), of(k16));
+    // (the kernel of small products takes some with fp16 activations that go through the tiles, which are counted above, with bf16 ones; else x's type makes no difference)
+    const GemmRoute r = gemm_route(mats, n, T, SQ_F16);
+    switch (r.kernel) {
+    case GEMM_FUSED: return std::max({tiles, fused_workspace(r.fused, mats, n, T), mid_ok(mats, n, T) ? mid_workspace(mats, n, T, &r.mid) : (size_t)0});
+    case GEMM_COLUMNS: return std::max({tiles, mid_workspace(mats, n, T, &r.mid), plane_product_workspace(mats, n, T, &r.columns)});
+    case GEMM_MID: return std::max(tiles, mid_workspace(mats, n, T, &r.mid));
+    case GEMM_DECODED: return std::max(tiles, decoded_workspace(mats, n, T));
+    default: return tiles;
+    }
 }
 
 size_t gemm_workspace_without_mid(const sq_matrix* mats, int n, int T) {
@@ -533,14 +529,14 @@ int launch_gemm(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_
     if (T <= SQ_SMALL_BMAX && !small_takes_gemm_route(mats, n, T, x, ldx))
         return launch_small(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, ws_bytes, sums, s);
     if (T > SQ_SMALL_BMAX && x_vec_ok(x, ldx, mats[0].C)) {
-        const GemmKernel k = gemm_route(mats, n, T, x_dtype);
-        if (k == GEMM_COLUMNS && plane_product_workspace(mats, n, T) <= ws_bytes) return launch_plane_product(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, ws_bytes, s);
+        const GemmRoute r = gemm_route(mats, n, T, x_dtype);
+        if (r.kernel == GEMM_COLUMNS && plane_product_workspace(mats, n, T, &r.columns) <= ws_bytes)
+            return launch_plane_product(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, ws_bytes, s, &r.columns);
         // (the fused kernel's cuts also serve where a workspace or the span of x does not let the others in)
-        const bool mid = mid_x_ok(ldx, T) && (mid_ok(mats, n, T) ? mid_least(mats, n, T) <= ws_bytes : k == GEMM_MID && gemm_workspace_without_mid(mats, n, T) <= ws_bytes);
-        if (k == GEMM_FUSED || !mid)
-            if (fused_plan(mats, n, T).nw && fused_workspace(mats, n, T) <= ws_bytes && (k != GEMM_TILES || gemm_workspace_without_mid(mats, n, T) > ws_bytes))
-                return launch_fused(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);
-        if (mid) return launch_mid(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, ws_bytes, s);
+        const bool mid = mid_x_ok(ldx, T) && (mid_ok(mats, n, T) ? mid_least(mats, n, T) <= ws_bytes : r.kernel == GEMM_MID && gemm_workspace_without_mid(mats, n, T) <= ws_bytes);
+        if (r.fused.nw && (r.kernel == GEMM_FUSED || !mid) && fused_workspace(r.fused, mats, n, T) <= ws_bytes && (r.kernel != GEMM_TILES || gemm_workspace_without_mid(mats, n, T) > ws_bytes))
+            return launch_fused(r.fused, mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);
+        if (mid) return launch_mid(mats, n, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, ws_bytes, s, &r.mid);
         if (mid_x_ok(ldx, T) && mid_ok(mats, n, T)) return fail(SQ_EWORKSPACE, "sq_linear_gemm: workspace %zu < %zu", ws_bytes, gemm_workspace(mats, n, T));
     }
     if (T > SQ_SMALL_BMAX && T <= small_pass_limit(mats, n) && x_vec_ok(x, ldx, mats[0].C)) {

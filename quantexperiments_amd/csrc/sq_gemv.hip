@@ -236,10 +236,11 @@ static int sieve_len(const sq_matrix* mats, int n, int B) {
 }
 
 // The same for the kernel of sq_plane_product.hip
-static int plane_product_len(const sq_matrix* mats, int n, int B) {
+static int plane_product_len(const sq_matrix* mats, int n, int B, PlanePlan& planned) {
+    if (B < PLANE_PRODUCT_MIN_T) return 0;
     int k = 0;
     while (k < n && mma_rows(mats[k]) && !stream_rows(mats[k], B)) ++k;
-    return plane_product_group(mats, k, B);
+    return plane_product_group(mats, k, B, planned);
 }
 
 // SiLU(gate) * up written by the matrix-core kernel: the two pieces' codebooks (one format, one shape) fit LDS side by side next to the
@@ -282,17 +283,22 @@ static float mma_us(const sq_matrix* mats, int n, int B) {
 // mma_silu_shape takes stays, so that with and without SiLU it has the same sums.
 // (Products below 2 M weights are a launch's length either way, and stay: 464 x 512, 12-bit, 6.4 and 7.4.  Rows below 512 columns were not measured.)
 constexpr int MID_SMALL_T = 17, MID_SMALL_C = 512, MID_SMALL_WEIGHTS = 2 << 20;
-static int mid_len(const sq_matrix* mats, int n, int B, size_t room) {
+static int mid_len(const sq_matrix* mats, int n, int B, size_t room, MidPlan& planned) {
     const sq_matrix& m0 = mats[0];
     if (B < MID_SMALL_T || B > SQ_SMALL_BMAX || m0.d != 4 || m0.C < MID_SMALL_C || mma_silu_shape(mats, n, B)) return 0;
     int k = 0;
     int64_t weights = 0;
     while (k < n && k < MID_PIECES && mma_shape(mats[k]) && mats[k].R > 0 && !stream_rows(mats[k], B) && mats[k].d == 4 && mats[k].bits == m0.bits &&
            mats[k].W == m0.W && mats[k].G == m0.G) weights += (int64_t)mats[k++].R * m0.C;
-    return weights >= MID_SMALL_WEIGHTS && mma_table_bytes(m0) && mid_us(mats, k, B, room) < 0.92f * mma_us(mats, k, B) ? k : 0;
+    if (weights < MID_SMALL_WEIGHTS || !mma_table_bytes(m0)) return 0;
+    planned = mid_plan(mats, k, B, room);
+    return planned.us < 0.92f * mma_us(mats, k, B) ? k : 0;
 }
 // For tests: that number where the workspace holds whatever sums there are.
-extern "C" __attribute__((visibility("default"))) int32_t sq_mid_pieces_for_tests(const sq_matrix* mats, int32_t n, int32_t B) { return mid_len(mats, n, B, SIZE_MAX); }
+extern "C" __attribute__((visibility("default"))) int32_t sq_mid_pieces_for_tests(const sq_matrix* mats, int32_t n, int32_t B) {
+    MidPlan planned;
+    return mid_len(mats, n, B, SIZE_MAX, planned);
+}
 
 // What the pieces' kernels keep side by side; not what a launch has from the workspace's first byte on for itself (small_workspace).
 // tight: the pieces that can run without partial sums do
@@ -309,18 +315,20 @@ static size_t small_need(const sq_matrix* mats, int n, int B, bool tight) {
 size_t small_workspace(const sq_matrix* mats, int n, int B) {
     size_t need = small_need(mats, n, B, false);
     const bool orders = has_orders(mats, n);
+    PlanePlan plane;
+    MidPlan mid;
     for (int i = 0; i < n; ++i) {
         if (const int k = orders ? 0 : vector_decoded(mats + i, n - i, B); k > 0) {
             need = std::max(need, decoded_workspace(mats + i, k, B));
             i += k - 1;
-        } else if (const int k = plane_product_len(mats + i, n - i, B); k > 0) {
-            need = std::max(need, plane_product_workspace(mats + i, k, B));
+        } else if (const int k = plane_product_len(mats + i, n - i, B, plane); k > 0) {
+            need = std::max(need, plane_product_workspace(mats + i, k, B, &plane));
             i += k - 1;
         } else if (const int k = sieve_len(mats + i, n - i, B); k > 0) {
             need = std::max(need, sieve_workspace(mats + i, k, B));
             i += k - 1;
-        } else if (const int k = mid_len(mats + i, n - i, B, SIZE_MAX); k > 0) {
-            need = std::max(need, mid_workspace(mats + i, k, B));
+        } else if (const int k = mid_len(mats + i, n - i, B, SIZE_MAX, mid); k > 0) {
+            need = std::max(need, mid_workspace(mats + i, k, B, &mid));
             i += k - 1;
         }
     }
@@ -465,6 +473,8 @@ int launch_small(const sq_matrix* mats, int n, const void* x, int x_dtype, int64
     const int cus = device_cus();
     const bool x_ok = (B == 1 || ldx % 8 == 0) && (((uintptr_t)x & 15) == 0);   // 16-byte activation loads
     size_t ws_off = 0;
+    PlanePlan plane;
+    MidPlan mid;
     int i = 0;
     while (i < n) {
         const sq_matrix& m0 = mats[i];
@@ -485,8 +495,8 @@ int launch_small(const sq_matrix* mats, int n, const void* x, int x_dtype, int64
             i += k;
             continue;
         }
-        if (const int k = !x_ok ? 0 : plane_product_len(mats + i, n - i, B); k > 0 && plane_product_workspace_least(mats + i, k, B) <= ws_bytes) {
-            if (const int rc = launch_plane_product(mats + i, k, x, x_dtype, ldx, y, y_dtype, ldy, B, ws, ws_bytes, s)) return rc;
+        if (const int k = !x_ok ? 0 : plane_product_len(mats + i, n - i, B, plane); k > 0 && plane_product_workspace_least(mats + i, k, B, &plane) <= ws_bytes) {
+            if (const int rc = launch_plane_product(mats + i, k, x, x_dtype, ldx, y, y_dtype, ldy, B, ws, ws_bytes, s, &plane)) return rc;
             ws_off += small_need(mats + i, k, B, tight);
             i += k;
             continue;
@@ -497,8 +507,8 @@ int launch_small(const sq_matrix* mats, int n, const void* x, int x_dtype, int64
             i += k;
             continue;
         }
-        if (const int k = !x_ok || !mid_x_ok(ldx, B) ? 0 : mid_len(mats + i, n - i, B, ws_bytes); k > 0) {
-            if (const int rc = launch_mid(mats + i, k, x, x_dtype, ldx, y, y_dtype, ldy, B, ws, ws_bytes, s)) return rc;
+        if (const int k = !x_ok || !mid_x_ok(ldx, B) ? 0 : mid_len(mats + i, n - i, B, ws_bytes, mid); k > 0) {
+            if (const int rc = launch_mid(mats + i, k, x, x_dtype, ldx, y, y_dtype, ldy, B, ws, ws_bytes, s, &mid)) return rc;
             ws_off += small_need(mats + i, k, B, tight);
             i += k;
             continue;

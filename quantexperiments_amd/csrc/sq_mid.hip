@@ -12,8 +12,6 @@ int launch_mid_b10d4(const MidArgs&, int, int, int, int, int, hipStream_t);
 int launch_mid_b8d4(const MidArgs&, int, int, int, int, int, hipStream_t);
 int launch_mid_dense(const MidArgs&, int, int, int, int, int, hipStream_t);
 
-struct MidPlan { int nt, tw, nw, st, ks; float us; };
-
 static int mid_units(const sq_matrix& m) { return m.W / (m.bits == 12 ? 3 : m.bits == 10 ? 5 : 4); }
 
 // The variants: workgroups of NW waves, each with TW tiles of 16 weight rows x NT tiles of 16 activation rows, those of a stack cut into
@@ -39,7 +37,7 @@ static constexpr MidCost MID_COST8 = {3.49f, 0.f, 0.00198f, 0.00198f, 0.0168f, 0
 
 static int64_t mid_blocks(const sq_matrix* mats, int n, int rows) {       // of `rows` weight rows
     int64_t w = 0;
-    for (int i = 0; i < n; ++i) w += (mats[i].R + rows - 1) / rows;
+    for (int i = 0; i < n; ++i) w += (uint32_t)(mats[i].R + rows - 1) / (uint32_t)rows;
     return w;
 }
 static int mid_lds(const MidVariant& v, int table) { return table + 2 * mid_stage_bytes(v.nt, v.st); }
@@ -51,36 +49,61 @@ static size_t mid_sums_bytes(const sq_matrix* mats, int n, int T, int ks) {
     return need;
 }
 
-// The cut with the least estimated time whose sums of slices take at most `room` bytes
-static MidPlan mid_plan(const sq_matrix* mats, int n, int T, int cus, size_t room) {
+// What the estimate needs of a variant alone
+struct MidTerms { float step, wait, chip; int beside, rows; };          // rows: of a workgroup's weights, as a place in mid_cut's list of blocks
+template <size_t N> struct MidTermsOf { MidTerms t[N]; };
+template <size_t N>
+static constexpr MidTermsOf<N> mid_terms(const MidVariant (&vs)[N], const MidCost& c) {
+    MidTermsOf<N> r{};
+    for (size_t k = 0; k < N; ++k) {
+        const MidVariant v = vs[k];
+        r.t[k].step = (v.nw + 3) / 4 * 4 * v.tw * (c.product * v.nt + c.words) + c.read * v.nw * v.nt + c.stage * v.nt;      // (ten waves: three on a SIMD)
+        r.t[k].wait = c.wait + c.wait_tile * v.nt * v.tw + c.wait_stage * v.nt / v.nw;
+        r.t[k].chip = v.nw * v.tw * c.chip;
+        r.t[k].beside = std::max(1, std::min(4 * (512 / (40 + 6 * v.nt + 4 * v.nt * v.tw)) / v.nw, 32 / v.nw));              // workgroups that a CU's registers hold side by side
+        r.t[k].rows = v.tw == 2 ? 4 : v.nw == 4 ? 0 : v.nw == 8 ? 1 : v.nw == 10 ? 2 : 3;
+    }
+    return r;
+}
+static constexpr auto MID_TERMS4 = mid_terms(MID4, MID_COST4);
+static constexpr auto MID_TERMS8 = mid_terms(MID8, MID_COST8);
+
+// The cut with the least estimated time whose sums of slices take at most `room` bytes.  (Every call plans; what the matrix steps alone, spread evenly, rule
+// out is not looked at any further.)
+static MidPlan mid_cut(const sq_matrix* mats, int n, int T, size_t room) {
     const bool d4 = mats[0].d == 4;
-    const int table = d4 ? (mats[0].G << mats[0].bits) * 8 : 0, pairs = ((mid_units(mats[0]) + 3) / 4 + 1) / 2;   // of rounds
+    const int cus = device_cus(), table = d4 ? (mats[0].G << mats[0].bits) * 8 : 0, pairs = ((mid_units(mats[0]) + 3) / 4 + 1) / 2;   // of rounds
     const MidCost& c = d4 ? MID_COST4 : MID_COST8;
     const MidVariant* vs = d4 ? MID4 : MID8;
-    const int count = d4 ? (int)(sizeof(MID4) / sizeof(MID4[0])) : (int)(sizeof(MID8) / sizeof(MID8[0]));
+    const MidTerms* terms = d4 ? MID_TERMS4.t : MID_TERMS8.t;
+    const int count = d4 ? (int)std::size(MID4) : (int)std::size(MID8);
     int64_t rows = 0;
     for (int i = 0; i < n; ++i) rows += mats[i].R;
-    const float results = (float)rows * T * 1e-6f, pair_steps = mats[0].bits == 12 ? 8.f : 16.f;
+    const float results = (float)rows * T * 1e-6f, pair_steps = mats[0].bits == 12 ? 8.f : 16.f, fixed = c.launch + c.results * results;
+    const float even = pair_steps * pairs / cus;                          // matrix steps of a workgroup whose row is one slice, per CU
+    // blocks of weight rows, and of activation rows by tiles
+    const int64_t blocks[5] = {mid_blocks(mats, n, 64), mid_blocks(mats, n, 128), mid_blocks(mats, n, 160), mid_blocks(mats, n, 192), mid_blocks(mats, n, 256)};
+    auto over = [](int64_t a, int b) { return a >> 32 ? a / b : (int64_t)((uint32_t)a / (uint32_t)b); };
     MidPlan best{0, 1, 8, 4, 1, 1e30f};
     for (int k = 0; k < count; ++k) {
         const MidVariant& v = vs[k];
+        const MidTerms& t = terms[k];
+        const int64_t whole = blocks[t.rows] * (int64_t)((uint32_t)(T + 16 * v.nt - 1) / (uint32_t)(16 * v.nt));
+        if (fixed + whole * even * t.step * 0.9999f >= best.us) continue;
         const int lds = mid_lds(v, table);
         if (lds > 160 * 1024 || (v.st == 2 && v.nt <= 8 && mid_lds({v.nt, v.tw, v.nw, 4}, table) <= 160 * 1024)) continue;
         if (v.nt > 3 && v.nt * 16 >= 2 * T) continue;                     // (more than half of it past the last row)
-        // workgroups that a CU runs side by side, by its LDS and registers
-        const int beside = std::max(1, std::min({160 * 1024 / lds, 4 * (512 / (40 + 6 * v.nt + 4 * v.nt * v.tw)) / v.nw, 32 / v.nw}));
-        const int64_t whole = mid_blocks(mats, n, 16 * v.nw * v.tw) * ((T + 16 * v.nt - 1) / (16 * v.nt));
         if (!d4 && v.tw == 2 && whole < cus) continue;                    // (bound by its codewords, two tiles of which a wave cannot fetch far enough ahead)
-        const int most = (int)std::min<int64_t>({std::max<int64_t>(1, cus / whole), 8, pairs});
-        const float step = (v.nw + 3) / 4 * 4 * v.tw * (c.product * v.nt + c.words) + c.read * v.nw * v.nt + c.stage * v.nt;      // (ten waves: three on a SIMD)
+        const int beside = std::max(1, std::min(160 * 1024 / lds, t.beside)), most = whole > cus ? 1 : std::min({cus / (int)whole, 8, pairs});
         for (int cut = 0; cut < 3; ++cut) {
             const int ks = cut == 0 ? 1 : cut == 1 ? most : most / 2;
             if (cut && ks < 2) continue;
-            const int64_t wgs = whole * ks, rounds = (wgs + cus - 1) / cus, waits = (rounds + beside - 1) / beside;
-            const float s = pair_steps * ((pairs + ks - 1) / ks);
-            const float work = rounds * s * step, wait = waits * s * (c.wait + c.wait_tile * v.nt * v.tw + c.wait_stage * v.nt / v.nw), chip = wgs * s * v.nw * v.tw * c.chip;
-            const float us = c.launch + c.table * (table >> 10) * waits + (v.nt == 1 ? 1.14f : 1.f) * __builtin_sqrtf(work * work + wait * wait + chip * chip) +
-                             (ks > 1 ? c.slices + c.sums * ks * results : 0.f) + c.results * results;
+            const int64_t wgs = whole * ks, rounds = over(wgs + cus - 1, cus);
+            const float s = pair_steps * ((pairs + ks - 1) / ks), work = rounds * s * t.step, sums = ks > 1 ? c.slices + c.sums * ks * results : 0.f;
+            if (fixed + work + sums >= best.us) continue;
+            const int64_t waits = over(rounds + beside - 1, beside);
+            const float wait = waits * s * t.wait, chip = wgs * s * t.chip;
+            const float us = fixed + c.table * (table >> 10) * waits + (v.nt == 1 ? 1.14f : 1.f) * __builtin_sqrtf(work * work + wait * wait + chip * chip) + sums;
             if (us < best.us && (ks == 1 || mid_sums_bytes(mats, n, T, ks) <= room)) best = {v.nt, v.tw, v.nw, v.st, ks, us};
         }
     }
@@ -135,20 +158,19 @@ size_t mid_least(const sq_matrix* mats, int n, int T) {
 // (a decode step's sums are those that sq_linear_small_noalloc has room for)
 static size_t mid_room(int T, size_t room) { return T <= SQ_SMALL_BMAX ? std::min(room, SMALL_ROOM) : room; }
 
-size_t mid_workspace(const sq_matrix* mats, int n, int T) {
-    const MidPlan p = mid_plan(mats, n, T, device_cus(), mid_room(T, SIZE_MAX));
-    const size_t need = mid_sums_bytes(mats, n, T, p.ks);
+MidPlan mid_plan(const sq_matrix* mats, int n, int T, size_t room) {
+    return mid_shape(mats, n, T) ? mid_cut(mats, n, T, mid_room(T, room)) : MidPlan{0, 1, 8, 4, 1, 1e30f};
+}
+
+size_t mid_workspace(const sq_matrix* mats, int n, int T, const MidPlan* planned) {
+    const size_t need = mid_sums_bytes(mats, n, T, planned && planned->nt ? planned->ks : mid_plan(mats, n, T).ks);
     return T > SQ_SMALL_BMAX && T <= mid_limit(mats, n) ? std::max(need, mid_least(mats, n, T)) : need;
 }
 
-// Estimated time at T rows with `room` bytes for sums; a very long one where the kernel does not take the pieces
-float mid_us(const sq_matrix* mats, int n, int T, size_t room) { return mid_shape(mats, n, T) ? mid_plan(mats, n, T, device_cus(), mid_room(T, room)).us : 1e30f; }
-
 // For tests: the cut that a stack takes at T rows, as token tiles | weight tiles << 8 | waves << 16 | K slices << 24; 0: the kernel does not take it.
 extern "C" __attribute__((visibility("default"))) int32_t sq_mid_variant_for_tests(const sq_matrix* mats, int32_t n, int32_t T) {
-    if (!mid_shape(mats, n, T)) return 0;
-    const MidPlan p = mid_plan(mats, n, T, device_cus(), SIZE_MAX);
-    return p.nt | p.tw << 8 | p.nw << 16 | p.ks << 24;
+    const MidPlan p = mid_plan(mats, n, T);
+    return p.nt ? p.nt | p.tw << 8 | p.nw << 16 | p.ks << 24 : 0;
 }
 
 static int launch_mid_rows(const sq_matrix* mats, int n, const MidPlan& pl, const void* const* dense, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype,
@@ -209,9 +231,9 @@ int launch_mid_decoded(const sq_matrix* mats, int n, const void* const* w, const
 }
 
 int launch_mid(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws,
-               size_t ws_bytes, hipStream_t s) {
-    if (T > SQ_SMALL_BMAX && T <= mid_limit(mats, n) && mid_least(mats, n, T) > ws_bytes) return fail(SQ_EWORKSPACE, "sq_linear_gemm: workspace %zu < %zu", ws_bytes, mid_workspace(mats, n, T));
-    return launch_mid_rows(mats, n, mid_plan(mats, n, T, device_cus(), mid_room(T, ws_bytes)), nullptr, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);
+               size_t ws_bytes, hipStream_t s, const MidPlan* planned) {
+    const bool kept = planned && planned->nt && (planned->ks == 1 || mid_sums_bytes(mats, n, T, planned->ks) <= ws_bytes);
+    return launch_mid_rows(mats, n, kept ? *planned : mid_plan(mats, n, T, ws_bytes), nullptr, x, x_dtype, ldx, y, y_dtype, ldy, T, ws, s);
 }
 
 }  // namespace sq

@@ -22,7 +22,7 @@
 
 namespace sq {
 
-constexpr int PP_WAVES = 8, PP_MIN_T = 17, PP_MAX_NT = 8;
+constexpr int PP_WAVES = 8, PP_MAX_NT = 8;
 constexpr int PP_TILES[PP_MAX_NT + 1] = {0, 0, 5, 5, 5, 4, 3, 2, 2};     // most tiles of a wave at once, by token tiles: what 256 registers hold
 typedef __attribute__((address_space(3))) void* pp_lptr_t;
 
@@ -205,22 +205,21 @@ static bool pp_shape(const sq_matrix& m) {
            (((uintptr_t)m.tags | (uintptr_t)m.table) & 15) == 0 && (int64_t)m.R * m.W < ((int64_t)1 << 30);
 }
 
-struct PpPlan { int tw, nt, pl, parts[MID_PIECES]; double us; };
-
 // Parts of the rows so that every CU has a workgroup, tiles of a wave in as few rounds as registers allow, evenly; one plane a workgroup or
 // two, whichever is estimated to take less.  Microseconds, fitted to 203 products (6 %): launches and activations; staging; look-ups and
 // products; activations to registers; sums.  (planes: that many a workgroup, if it is given)
-static PpPlan pp_plan(const sq_matrix* mats, int n, int T, int planes = 0) {
+static PlanePlan pp_plan(const sq_matrix* mats, int n, int T, int planes = 0) {
+    const int cus = device_cus();
     int64_t tiles = 0, rows = 0;
     for (int i = 0; i < n; ++i) tiles += (mats[i].R + 15) / 16, rows += mats[i].R;
-    PpPlan best{};
+    PlanePlan best{};
     for (int pl = planes ? planes : 1; pl <= (planes ? planes : 2); ++pl) {
-        PpPlan p{};
+        PlanePlan p{};
         p.nt = (T + 15) / 16; p.pl = pl;
         int64_t per = 0;                     // most tiles of a part
         for (int i = 0; i < n; ++i) {
             const int64_t mine = (mats[i].R + 15) / 16;
-            p.parts[i] = (int)std::max<int64_t>(1, std::min<int64_t>(mine, device_cus() * pl / 8 * mine / tiles));
+            p.parts[i] = (int)std::max<int64_t>(1, std::min<int64_t>(mine, cus * pl / 8 * mine / tiles));
             per = std::max(per, (mine + p.parts[i] - 1) / p.parts[i]);
         }
         const int64_t wave = (per + PP_WAVES - 1) / PP_WAVES, rounds = (wave + PP_TILES[p.nt] - 1) / PP_TILES[p.nt];
@@ -238,7 +237,7 @@ static size_t pp_part_bytes(int R, int T, int pl) { return pp_align((size_t)(8 /
 
 // how many of the pieces, the first one on, have a shape that the kernel takes
 static int pp_fit(const sq_matrix* mats, int n, int T) {
-    if (T < PP_MIN_T || T > 16 * PP_MAX_NT || device_cus() < 64) return 0;
+    if (T < PLANE_PRODUCT_MIN_T || T > 16 * PP_MAX_NT || device_cus() < 64) return 0;
     int k = 0;
     while (k < n && k < MID_PIECES && pp_shape(mats[k]) && mats[k].C == mats[0].C) ++k;
     return k;
@@ -248,27 +247,27 @@ static int pp_fit(const sq_matrix* mats, int n, int T) {
 static size_t pp_fixed_bytes(const sq_matrix* mats, int n, int nt) { return planes_bytes(n) + pp_x_bytes(mats, nt); }
 static size_t pp_sums_bytes(int64_t rows, int n, int T, int pl) { return (size_t)(8 / pl) * T * 4 * (rows + 4 * n) + 256 * n; }
 
-// The gathers from L2 take 8 us and 4.75 more per million tags up to 32 rows (fitted to 12 products: 10 %), and then what mid_us says; here has
+// The gathers from L2 take 8 us and 4.75 more per million tags up to 32 rows (fitted to 12 products: 10 %), and then what mid_plan says; here has
 // to be estimated a seventh faster (8000 x 2048 at 32 / 64 rows 17.3 / 18.7 there, 20.8 / 25 here; 3584 x 3584 16.8 / 19.0, 17.7 / 21.7).  A decode step's
 // products also need room for a fair part of their rows' sums in what sq_linear_small_noalloc has.
 constexpr int PP_PART_ROWS = 4096;
-int plane_product_group(const sq_matrix* mats, int n, int T) {
+int plane_product_group(const sq_matrix* mats, int n, int T, PlanePlan& p, const MidPlan* mid) {
     const int k = pp_fit(mats, n, T);
     double tags = 0.0;
     for (int i = 0; i < k; ++i) tags += (double)mats[i].R * mats[i].C / 8e6;
     if (tags < 2.0) return 0;                // (no product of that size gains; the estimates cost the host a microsecond)
-    const PpPlan p = pp_plan(mats, k, T);
+    p = pp_plan(mats, k, T);
     if (T <= SQ_SMALL_BMAX && pp_fixed_bytes(mats, k, p.nt) + pp_sums_bytes(PP_PART_ROWS, k, T, p.pl) > SMALL_ROOM) return 0;
-    return p.us < 0.85 * (T <= SQ_SMALL_BMAX ? 8.0 + 4.75 * tags : (double)mid_us(mats, k, T)) ? k : 0;
+    return p.us < 0.85 * (T <= SQ_SMALL_BMAX ? 8.0 + 4.75 * tags : (double)(mid && k == n ? *mid : mid_plan(mats, k, T)).us) ? k : 0;
 }
 
-size_t plane_product_workspace(const sq_matrix* mats, int n, int T) {
-    const PpPlan p = pp_plan(mats, n, T);
+size_t plane_product_workspace(const sq_matrix* mats, int n, int T, const PlanePlan* planned) {
+    const PlanePlan p = planned ? *planned : pp_plan(mats, n, T);
     size_t need = pp_fixed_bytes(mats, n, p.nt);
     for (int i = 0; i < n; ++i) need += pp_part_bytes(mats[i].R, T, p.pl);
     return need;
 }
-size_t plane_product_workspace_least(const sq_matrix* mats, int n, int T) { return std::min(plane_product_workspace(mats, n, T), SMALL_ROOM); }
+size_t plane_product_workspace_least(const sq_matrix* mats, int n, int T, const PlanePlan* planned) { return std::min(plane_product_workspace(mats, n, T, planned), SMALL_ROOM); }
 
 typedef void (*pp_kernel_t)(PpArgs);
 template <int TW, int NT>
@@ -280,13 +279,13 @@ static constexpr pp_kernel_t pp_kernel() {
 // Rows of all pieces, or, where their sums do not fit the workspace (plane_product_workspace_least: up to SQ_SMALL_BMAX activation rows), as many at a time as do, evenly
 // cut.  A row's sums depend on the planes a workgroup takes alone, which are those of the whole product: the results are the same bits either way.
 int launch_plane_product(const sq_matrix* mats, int n, const void* x, int x_dtype, int64_t ldx, void* y, int y_dtype, int64_t ldy, int T, void* ws, size_t ws_bytes,
-                         hipStream_t s) {
-    const PpPlan whole = pp_plan(mats, n, T);
+                         hipStream_t s, const PlanePlan* planned) {
+    const PlanePlan whole = planned ? *planned : pp_plan(mats, n, T);
     const size_t fixed = pp_fixed_bytes(mats, n, whole.nt);
     int64_t rows = 0;
     for (int i = 0; i < n; ++i) rows += mats[i].R;
     int64_t most = rows;                     // weight rows of a launch
-    if (plane_product_workspace(mats, n, T) > ws_bytes) {
+    if (plane_product_workspace(mats, n, T, &whole) > ws_bytes) {
         const size_t none = fixed + pp_sums_bytes(0, n, T, whole.pl);
         const int64_t fit = ws_bytes > none ? (int64_t)((ws_bytes - none) / ((size_t)(8 / whole.pl) * T * 4)) / 16 * 16 : 0;
         if (fit < 16) return fail(SQ_EWORKSPACE, "plane product: workspace %zu < %zu", ws_bytes, plane_product_workspace(mats, n, T));
@@ -325,7 +324,7 @@ int launch_plane_product(const sq_matrix* mats, int n, const void* x, int x_dtyp
             r0 += R;
             if (r0 >= mats[i].R) ++i, r0 = 0;
         }
-        const PpPlan p = most == rows ? whole : pp_plan(part, a.n, T, whole.pl);
+        const PlanePlan p = most == rows ? whole : pp_plan(part, a.n, T, whole.pl);
         char* sums = (char*)ws + fixed;
         for (int j = 0; j < a.n; ++j) {
             a.p[j].m = part[j]; a.p[j].part = (float*)sums; a.p[j].job0 = a.jobs; a.p[j].parts = p.parts[j];
