@@ -40,7 +40,7 @@ static int fused_unit_dwords(int bits) { return bits == 12 ? 3 : bits == 10 ? 5 
 static int fused_round_steps(const sq_matrix& m) { return fused_unit_dwords(m.bits) * 32 / m.bits / (8 / m.d); }
 static int fused_rounds(const sq_matrix& m) { return (m.W / fused_unit_dwords(m.bits) + 3) / 4; }
 
-// How a product is cut, nw = 0 where the other kernels are the faster ones.  Up to 768 rows, in blocks of up to 384 tokens; rows of
+// How a product is cut, nw = 0 where the others were the faster ones when this kernel was cut (which products with a cut run here: gemm_route, sq_gemm.hip).  Up to 768 rows, in blocks of up to 384 tokens; rows of
 // the weights in tiles of 32 tw, where a launch should fill the CUs once: what a workgroup takes hardly depends on how many run
 // beside it.  A tile of 64 / 96 / 128 / 160 rows x 333 tokens x 3584 columns takes 66 / 83 / 104 / 123 us with 16-bit tags of
 // width 8 (the weights below), 62 / 73 / 85 / 103 with 10-bit ones of width 4.  Decoded and multiplied in tiles, or in one pass over the tags where

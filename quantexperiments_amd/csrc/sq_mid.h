@@ -13,8 +13,8 @@
 // 18944 x 2 x 3584 at 77 rows, which take 96 us; the matrix cores are busy 15 % of the time).  d = 4 by no pipe
 // alone: with 12-bit tags at 128 rows the matrix cores are busy 47 % of a CU's time and LDS 51 % (every wave reads all the
 // activations for its 32 weight rows; 29 % of it bank conflicts of the codeword reads), taking turns.  In passes of 32 rows or decoded
-// first, at 33 / 77 / 128 / 256 rows: d = 8, 18944 x 2 x 3584: 172 / 205 / 205 / 209 us, here 90 / 96 / 105 / 188 (sq_fused.h: 108);
-// 12-bit: 41 / 68 / 102 / 165, here 27 / 38 / 53 / 105 (82).
+// first, at 33 / 77 / 128 / 256 rows: d = 8, 18944 x 2 x 3584: 172 / 205 / 205 / 209 us, here 86 / 91 / 103 / 188 (sq_plane_product.hip, which takes it up to 96 rows:
+// 54 / 78; sq_fused.h: 103 at 256); 12-bit: 41 / 68 / 102 / 165, here 25 / 34 / 53 / 105 (sq_fused.h: 80).
 //
 //   workgroup   NW waves, two per SIMD or more so that one gathers while the other multiplies (4 waves: a third slower, and the choice
 //               where they spread better or a CU takes several); each has TW tiles of 16 weight rows x NT x 16 activation rows

@@ -13,8 +13,9 @@
 //               halves (55 -> 48 us at 16 rows, 75 -> 67 at 64).  A tile's tags are asked for as soon as the last ones have been used
 //   X           in the order of the operands (pp_order_kernel), 1 KB a step and token tile, straight to registers
 //
-// Bound: LDS look-ups (27 us of 2 x 18944 x 3584) and the tags' way, eight times 34 MB out of L2, side by side; then the sums (8 T R fp32 written and read:
-// 14 us of 67 at 64 rows).  us at 24 / 48 / 64 / 96 rows before and now: 2 x 18944 x 3584 89 / 88 / 91 / 99 -> 53 / 56 / 60 / 82, 18944 x 3584 49 / 54 / 56 / 60 ->
+// Bound: LDS look-ups, two thirds of a CU's time (2 x 18944 x 3584 at 24 / 64 rows 69 and 64 %, 72 % of that bank conflicts of 64 random two-byte elements),
+// then the way of tags, activations and columns, which a workgroup that fills a CU does not overlap; and the sums (4 or 8 T R fp32 written and read: the
+// launch that adds them takes 9 us of 60 at 64 rows).  us at 24 / 48 / 64 / 96 rows before and now: 2 x 18944 x 3584 89 / 88 / 91 / 99 -> 53 / 56 / 60 / 82, 18944 x 3584 49 / 54 / 56 / 60 ->
 // 34 / 38 / 41 / 47, 3584 x 18944 54 / 56 / 58 / 63 -> 34 / 37 / 40 / 48, q|k|v of 7168 x 5120 35 / 33 / 36 / 45 -> 28 / 30 / 31 / 36.
 #include <algorithm>
 #include "sq_planes.h"

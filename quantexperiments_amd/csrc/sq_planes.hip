@@ -4,7 +4,7 @@
 // columns is 128 KB, which LDS holds.  A workgroup stages plane e and looks up element e of every tag of its rows; chunks that are
 // neighbours in a row then have neighbouring results in plane order,
 //     out[r, e * n + j] = table[tag[r, j]][e]        (n = C / 8 chunks)
-// so whole lines leave.  The activations are copied into the same order of columns and the product does not notice: its sum over
+// so stretches of C / 4 bytes leave, whole lines where C is a multiple of 512.  The activations are copied into the same order of columns and the product does not notice: its sum over
 // columns is the same sum in another order.
 #include <algorithm>
 #include "sq_planes.h"
@@ -71,8 +71,8 @@ struct PlanesArgs {
 
 // A group of eight workgroups, one per plane, shares the tags of its rows; it sits on one XCD, whose L2 then reads them once.
 // A thread has eight tags (16 bytes) in, eight look-ups and 16 bytes out per unit, U units at a time with the next U's tags on their way.
-// What bounds it is the write of the dense copy: 37888 x 3584 (272 MB) in 66 us, 27 without the stores, 74 without the look-ups.  1024 threads with 4 units
-// 76, with 8 69; 512 with 6 or 12 71 and 75.  Stores that bypass the caches take 52, but the product that reads them next then takes as much
+// 37888 x 3584 (272 MB written) takes 66 us, 27 without the stores: look-ups keep the LDS busy half of the time, 70 % of that bank conflicts, the stores
+// reach 4.1 TB/s (kernels that write whole rows 5.5), and with one workgroup per CU the two take turns in part.  1024 threads with 4 units 76, with 8 69; 512 with 6 or 12 71 and 75.  Stores that bypass the caches take 52, but the product that reads them next then takes as much
 // longer, and with small matrices more: 3584 x 3584 at 2048 rows 63 us in all and 73.
 // A codeword at a time out of L2 (sq_dequant.hip) the decode takes 122 us: product of 2048 rows 514, now 474 with the 10 us of plane_order_kernel.
 __global__ __launch_bounds__(NT) void planes_kernel(PlanesArgs a) {

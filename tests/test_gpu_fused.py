@@ -2,6 +2,8 @@
 workgroup takes, edges of tiles, pieces and token blocks, rounds with missing units, odd numbers of rounds, K slices, several
 codebooks, results that allow no 16-byte stores."""
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -78,3 +80,35 @@ def test_missing_units_meet_no_codeword(R, C, d, bits, G, T):
     ref[5] = 0
     y[:, 5] = 0
     assert rel_max_err(y.cpu().numpy(), (x.cuda().double() @ ref.T).cpu().numpy()) < 1e-5       # (exact products, fp32 sums)
+
+
+# products that other kernels are the faster ones for, and the kernel that takes them (3: small products, 6 and 7: decode and tiles)
+GIVEN_UP = [(10843, 512, 4, 10, 263, (6, 1), 3), (10527, 2432, 4, 8, 578, (6, 2), 6), (10538, 768, 8, 16, 583, (6, 2), 6), (10858, 2304, 8, 16, 387, (4, 2), 7)]
+
+
+@pytest.mark.parametrize("R,C,d,bits,T,cut,kernel", GIVEN_UP)
+def test_runs_where_the_workspace_lets_no_other_in(R, C, d, bits, T, cut, kernel):
+    """With room for no more than the activations in fragment order a product still runs here; with less it is refused."""
+    L = _lib.lib()
+    s = synth(R, C, d, bits, seed=R)
+    lin, x = to_device(s, stream=False), rand_x(T, C, torch.float16, seed=T).cuda()
+    mats = _lib.matrix_array([lin.descriptor(0)])
+    assert torch.cuda.get_device_properties(0).multi_processor_count != 256 or L.sq_gemm_kernel_for_tests(mats, 1, T, _lib.SQ_BF16, (ctypes.c_float * 3)()) == kernel
+    ref = x.double() @ torch.from_numpy(s.decode()).cuda().double().T
+    need = cut[1] * 64 * cut[0] * ((C + 255) // 256 * 256) * 2                     # blocks of tokens, 64 tokens per `cut[0]`, whole rounds of 256 columns
+    ws, y = torch.full((need + 4096,), 0x5A, dtype=torch.uint8, device="cuda"), torch.empty(T, R, device="cuda")
+    call = lambda n: L.sq_linear_gemm(mats, 1, x.data_ptr(), _lib.SQ_F16, C, y.data_ptr(), _lib.SQ_F32, R, T, ws.data_ptr(), n, _lib.stream_ptr(x.device))
+    assert call(need) == 0 and rel_max_err(y.cpu().numpy(), ref.cpu().numpy()) < 1e-5 and bool((ws[need:] == 0x5A).all())      # (as above)
+    assert call(need - 256) == _lib.SQ_EWORKSPACE
+
+
+def test_runs_where_x_spans_more_than_the_others_address():
+    R, C, T, ld = 11028, 512, 134, 1 << 24                                         # 4.5 GB from the first row of x to the last
+    s = synth(R, C, 4, 12, seed=R)
+    lin = to_device(s)
+    x = torch.empty(T, ld, dtype=torch.float16, device="cuda")[:, :C]
+    x.copy_(rand_x(T, C, torch.float16, seed=T))
+    y = torch.empty(T, R, device="cuda")
+    linear_gemm([lin], x, y)
+    ref = x.double() @ torch.from_numpy(s.decode()).cuda().double().T
+    assert rel_max_err(y.cpu().numpy(), ref.cpu().numpy()) < 1e-5
